@@ -5,25 +5,41 @@ cross-compiles, so no GPU is needed to build.
 """
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import re
 import shutil
 import subprocess
-import sys
+import tempfile
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _ROOT = os.path.dirname(_HERE)
-SOURCES = [os.path.join(_HERE, "csrc", "hbsa_fwd.hip")]
+CSRC = os.path.join(_HERE, "csrc")
+API_SOURCE = os.path.join(CSRC, "hbsa_fwd.hip")     # the C ABI and the kernels that are no templates over the head dim
+INST_SOURCE = os.path.join(CSRC, "hbsa_inst.hip")   # the attention kernels of one head dim and element type
 OUTPUT = os.path.join(_HERE, "libhbsattn_amd.so")
-HAND_ISSUED_READS = "hbsa_fwd_kernel"   # substring of the mangled names of the kernels with hand-issued LDS reads ...
+# substrings of the mangled names of the kernels with hand-issued LDS reads ...
+HAND_ISSUED_READS = ("hbsa_fwd_kernel", "hbsa_bwd_dq_kernel", "hbsa_bwd_dkv8_kernel")
 COMPILER_ISSUED = "hbsa_fwd_kernelILi256E"   # ... except the head dim 256 instantiations, whose reads the compiler issues
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32 out of scalar float code.
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility-inlines-hidden",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-I" + os.path.join(_ROOT, "include"),
+    "-I" + os.path.join(_ROOT, "include"), "-I" + CSRC,
 ]
+
+
+def units() -> list:
+    """``(name, source, extra flags)`` of every translation unit of the library, the ones that take longest first."""
+    def inst(d, elem, part):
+        return (f"{elem}_{d}_{part}", INST_SOURCE, [f"-DHBSA_D={d}", f"-DHBSA_E={elem}", f"-DHBSA_PART={part}"])
+
+    out = [inst(d, e, 1) for d in (128, 64, 256, 32) for e in ("ElemBF16", "ElemF16")]
+    out += [inst(d, e, 3) for d in (128, 64, 32) for e in ("ElemBF16", "ElemF16")]
+    out += [inst(d, "ElemF16", 2) for d in (128, 64, 256, 32)]
+    out += [inst(d, "ElemF16", 4) for d in (256, 128, 64, 32)]
+    return out + [("api", API_SOURCE, [])]
 
 
 def _vgpr_spills(remarks: str) -> dict:
@@ -39,28 +55,49 @@ def _vgpr_spills(remarks: str) -> dict:
     return spills
 
 
-def build(verbose: bool = False) -> str:
+def compile_unit(unit, objdir: str):
+    """Compiles one unit into ``objdir``; returns (object file, compiler remarks)."""
+    name, source, flags = unit
+    obj = os.path.join(objdir, name + ".o")
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    cmd = [hipcc] + HIPCC_FLAGS + ["-Rpass-analysis=kernel-resource-usage"] + SOURCES + ["-o", OUTPUT]
+    cmd = [hipcc] + HIPCC_FLAGS + flags + ["-Rpass-analysis=kernel-resource-usage", "-c", source, "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed: " + " ".join(cmd))
-    # The forward attention kernel issues its LDS reads by hand and waits for them by count.  The
+        raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+    return obj, res.stderr
+
+
+def link(objects, output: str) -> None:
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + list(objects) + ["-o", output]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+
+
+def build(verbose: bool = False) -> str:
+    jobs = max(1, min(8, os.cpu_count() or 1))
+    with tempfile.TemporaryDirectory() as objdir, concurrent.futures.ThreadPoolExecutor(jobs) as pool:
+        done = list(pool.map(lambda u: compile_unit(u, objdir), units()))
+        check_spills("".join(remarks for _, remarks in done), verbose)
+        link([obj for obj, _ in done], OUTPUT)
+    if verbose:
+        print(f"{OUTPUT}: {len(done)} units")
+    return OUTPUT
+
+
+def check_spills(remarks: str, verbose: bool = False) -> None:
+    # The attention kernels named above issue their LDS reads by hand and wait for them by count.  The
     # compiler does not know that such a register has a read in flight; if it spills one, it saves the
     # register before the data has arrived and the result is wrong now and then.  So a build in which
-    # that kernel spills vector registers is refused.  (The other kernels leave every wait to the
+    # such a kernel spills vector registers is refused.  (The other kernels leave every wait to the
     # compiler; a spill there only costs time and is reported.)
-    spills = _vgpr_spills(res.stderr)
-    fatal = {k: v for k, v in spills.items() if HAND_ISSUED_READS in k and COMPILER_ISSUED not in k}
+    spills = _vgpr_spills(remarks)
+    fatal = {k: v for k, v in spills.items() if any(n in k for n in HAND_ISSUED_READS) and COMPILER_ISSUED not in k}
     if fatal:
-        os.remove(OUTPUT)
         raise RuntimeError(f"vector-register spills in {fatal}: reduce register pressure (see the comment here)")
     if spills and verbose:
         print(f"note: vector-register spills in {spills}")
-    if verbose:
-        print(" ".join(cmd))
-    return OUTPUT
 
 
 EXAMPLE_SOURCE = os.path.join(_HERE, "csrc", "cabi_example.cpp")
@@ -75,8 +112,7 @@ def build_example(verbose: bool = False) -> str:
            "-L" + _HERE, "-lhbsattn_amd", "-Wl,-rpath,$ORIGIN", "-o", EXAMPLE_OUTPUT]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed: " + " ".join(cmd))
+        raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + res.stdout + res.stderr)
     if verbose:
         print(" ".join(cmd))
     return EXAMPLE_OUTPUT

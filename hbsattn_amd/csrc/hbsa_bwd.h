@@ -1,5 +1,5 @@
 // Block-sparse attention backward for gfx950: dQ, dK, dV from dO, the forward's output and its
-// log-sum-exp.  Part of the translation unit hbsa_fwd.hip (included after the forward's helpers).
+// log-sum-exp.
 //
 // The reference stops at the forward (reference hbsattn/hbsa_interface.py:31-32 raises
 // NotImplementedError in backward), so this follows the mathematics of that forward
@@ -32,25 +32,11 @@
 // scheduling is not applied here: the grids already start their heaviest workgroups first, and what bounds
 // both kernels at long sequences is the stream of tiles from memory next to the matrix work, not the tail.
 
-namespace {
+#pragma once
 
-struct BwdParams {
-  const char *q, *k, *v, *out, *dout;
-  char *dq, *dk, *dv;
-  const float *lse;           // [total_q, nhead_q], contiguous
-  float *delta;               // [total_q, nhead_q], contiguous: rowsum(dO * O), written by the dQ kernel, read by the dK/dV kernels
-  float *lse2;                // [total_q, nhead_q]: lse * log2(e), +inf where lse is -inf; written by the dQ kernel for the D = 128 dK/dV kernel
-  const QBlockInfo *info;
-  const uint32_t *bits;
-  const int32_t *cu_k, *cu_num_q_block, *cu_num_k_block;
-  int64_t q_s, q_h, k_s, k_h, v_s, v_h, o_s, o_h, do_s, do_h, dq_s, dq_h, dk_s, dk_h, dv_s, dv_h;   // bytes
-  int32_t nqb, nkb, xcd_heads, batch, ratio, nhead_q, qbs, kbs, wpr, causal;   // xcd_heads: see the dK/dV kernels
-  int32_t total_k;
-  int32_t wps, nsub;     // q side: wave slots per q head and workgroups per (kv head, q block), as in the forward
-  int32_t nsub_k;        // k side: workgroups per (kv head, k block) = ceil(k_block_size / 128)
-  float c;               // softmax_scale * log2(e), signed
-  float scale;
-};
+#include "hbsa_common.h"
+
+namespace hbsa {
 
 // ---- shared pieces of the two main kernels ---------------------------------------------------------
 template <int D>
@@ -1091,4 +1077,4 @@ int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t st
   return e == hipSuccess ? 0 : (int)e;
 }
 
-}  // namespace
+}  // namespace hbsa

@@ -1,0 +1,335 @@
+// Types, element policies and device helpers shared by the kernels of the library, the kernel parameter blocks,
+// and the declarations of the launch functions.  The attention kernels are templates over head dim and element type;
+// each (head dim, element type) is a translation unit of its own (hbsa_inst.hip), so that they compile side by side.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstdarg>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <mutex>
+#include <type_traits>
+
+#include "hbsattn_amd.h"
+
+namespace hbsa {
+
+typedef short short4v __attribute__((ext_vector_type(4)));
+typedef short short8v __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+#define HBSA_AS1(p) ((const __attribute__((address_space(1))) void *)(p))
+#define HBSA_AS3(p) ((__attribute__((address_space(3))) void *)(p))
+
+constexpr int kThreads = 256;   // 4 wavefronts
+constexpr int kWaveRows = 32;   // query rows per wavefront (the MFMA N dimension)
+constexpr int kTileKeys = 64;   // keys per main-loop step
+constexpr int kWalkReportTiles = 8;   // an item adds its progress to its walk clock every so many tiles (a power of two)
+constexpr float kLog2e = 1.4426950408889634f;
+// One-launch form: sequences whose boundaries the scheduler keeps in LDS (batch + 1 entries of four arrays)
+constexpr int kSeqCap = 128;
+constexpr int kMaxDevices = 64;            // devices of one process the launch caches cover
+constexpr float kLazyRescaleLog2 = 8.0f;  // running max may lag the true max by 2^8
+
+// Geometry of one q block, written by the pre-pass (48 bytes).
+struct QBlockInfo {
+  int32_t row_begin;   // token row of the block's first query
+  int32_t rows;        // queries in the block (ragged last block of a sequence)
+  int32_t key_begin;   // token row of the sequence's first key
+  int32_t klen;        // keys in the sequence
+  int32_t q_pos;       // in-sequence position of the block's first query
+  int32_t shift;       // k_len - q_len: bottom-right causal alignment
+  int32_t nkblk;       // k blocks in the sequence
+  int32_t kmax;        // exclusive in-sequence bound of keys any row of the block may see
+  int32_t seq;         // first q block of the block's sequence: identifies the sequence by a number below num_q_block
+                       // (the batch index can exceed it when the batch holds sequences without queries)
+  int32_t flags;       // 1: the block's sequence did not fit the tensors; it has no keys (and perhaps no rows)
+  int32_t pad[2];
+};
+static_assert(sizeof(QBlockInfo) == 48, "QBlockInfo is read as twelve 32-bit words");
+
+struct Sched;
+
+struct PrepParams {
+  const int32_t *cu_q, *cu_k, *q_block_to_batch, *cu_num_q_block, *cu_num_k_block;
+  const uint8_t *mask;
+  int64_t ms_h, ms_q, ms_k;
+  QBlockInfo *info;
+  uint32_t *bits;
+  struct Sched *sched;
+  unsigned long long *clock;
+  int32_t nqb, qbs, kbs, wpr, causal;
+  int32_t batch, nkb, total_q, total_k;   // bounds the sequences' boundaries are checked against
+};
+
+// Division by a launch constant d, exact for 0 <= n < 2^31: n / d == (n * m) >> s with
+// s = 31 + ceil(log2 d), m = ceil(2^s / d) (which fits 32 bits).  Three scalar instructions where
+// a hardware-less integer division takes about forty.
+struct FastDiv {
+  uint32_t m, s;
+};
+__host__ __device__ inline uint32_t fast_div(uint32_t n, FastDiv f) { return (uint32_t)(((uint64_t)n * f.m) >> f.s); }
+inline FastDiv make_fast_div(uint32_t d) {
+  uint32_t l = 0;
+  while (((uint64_t)1 << l) < d) ++l;
+  FastDiv f;
+  f.s = 31 + l;
+  f.m = (uint32_t)((((uint64_t)1 << f.s) + d - 1) / d);
+  return f;
+}
+
+// (Fields are appended at the end, never inserted: the compiler fetches the kernel arguments in aligned groups,
+// and a layout that splits the fields the tile loop uses makes it fetch some of them again inside that loop,
+// where a scalar load's wait also waits for every hand-issued LDS read; measured, 0.8 % of T for one such shift.)
+struct FwdParams {
+  const char *q, *k, *v;
+  char *out;
+  const QBlockInfo *info;
+  const uint32_t *bits;
+  int64_t q_s, q_h, k_s, k_h, v_s, v_h, o_s, o_h;  // bytes
+  int32_t nqb, ratio, kbs, wpr, causal;
+  int32_t wps;    // wave slots per q head = ceil(q_block_size / 32)
+  int32_t nw;     // wavefronts per workgroup (4 or 8)
+  int32_t nsub;   // workgroups per (kv head, q block) = ceil(ratio * wps / nw)
+  uint32_t q_sign;  // 0x80008000 when softmax_scale < 0 (Q is negated, |scale| used)
+  float c;        // |softmax_scale| * log2(e)
+  float lag;      // kLazyRescaleLog2 / c: how far the running max may lag, in raw score units
+  FastDiv div_nsub, div_nqb, div_kbs;   // divisions on the scheduler's path
+  int32_t f32;    // fp32 inputs staged as fp16: the softmax constants come from the launch record, where
+                  // the setup kernel derived them from the tensors' maxima
+  int32_t nhead_k;
+  int32_t one_each;   // > 0: the number of work items, handed out without queues: workgroup i of G takes items i, 2G - 1 - i, 2G + i, ...
+  struct Sched *sched;
+  // Walk order of the kept k blocks (see the kernel's comment).  walk != 0: the workgroups that work on
+  // one (kv head, sequence) keep near each other in key space through a shared clock, so that they find
+  // each other's K/V blocks in the L2; the summation order, and with it the last bits of the result,
+  // then depend on timing.  walk == 0: every item walks its blocks in ascending order (deterministic).
+  unsigned long long *clock;   // [nhead_k, num_q_block]: clock of (kv head, first q block of the sequence)
+  int32_t walk;
+  float *lse;             // optional [total_q, nhead_q] log-sum-exp output (nullptr: none)
+  int64_t lse_s, lse_h;   // its strides in elements
+  // Split over key blocks (few, long work items): every (kv head, q block, slot group) becomes
+  // nparts items, part i sees the bit row copy i (its share of the k blocks) and stores a
+  // normalised fp32 partial result and its log-sum-exp; hbsa_merge_kernel combines them.
+  int32_t nparts;         // 1: no split
+  FastDiv div_nparts;
+  float *part_out;        // [nparts, total_q, nhead_q, D]
+  float *part_lse;        // [nparts, total_q, nhead_q]
+  int32_t total_q, nhead_q;
+  // One-launch form (the kernel instantiated with FUSED): no pre-pass has run, `info` and `bits` are unused,
+  // and the scheduler derives every item's geometry and bit row itself from the caller's arrays.
+  const int32_t *cu_q, *cu_k, *cu_nqb, *cu_nkb;   // int32[batch + 1] each
+  const uint8_t *mask;                            // block_mask bytes, innermost (k block) stride 1
+  int64_t ms_h, ms_q;                             // its head and q block strides
+  int32_t batch, nkb_total, total_k, qbs;
+  int32_t pack;   // host side only: the launch uses the kernel whose wave slots are packed across the q heads of a GQA group
+  FastDiv div_nhk;   // division by nhead_k (items handed out without queues)
+};
+
+// Boundaries of one sequence of the packed batch, as read from the caller's device arrays.
+struct SeqBounds {
+  int32_t q0, q1;     // cu_q_seqlens[b], [b + 1]
+  int32_t k0, k1;     // cu_k_seqlens[b], [b + 1]
+  int32_t kb0, kb1;   // cu_num_k_block[b], [b + 1]
+  int32_t qb0;        // cu_num_q_block[b]
+};
+
+// Geometry record of q block g.  The sequence boundaries are device data the host cannot check, so they
+// are checked here against the token counts of q and k/v and the block counts.  A sequence that does
+// not fit (a wrong cu_seqlens, q/k/v shorter than it says, inconsistent block metadata) gets no keys:
+// nothing of k, v or the mask is read for it, and those of its query rows that lie inside q and out are
+// written as zeros, like any row that sees no key (flags = 1 marks such a block).  When not even the
+// query side makes sense (have == false: the block's sequence index is outside the batch) the block
+// has no rows and nothing is written for it.  kb0: first global k block of the sequence.
+__host__ __device__ inline QBlockInfo q_block_geometry(int g, bool have, SeqBounds s, int qbs, int kbs, int causal,
+                                                      int nkb_total, int total_q, int total_k, int &kb0) {
+  const int qlen = s.q1 - s.q0, klen_in = s.k1 - s.k0, nkb_in = s.kb1 - s.kb0;
+  const int q_pos = (g - s.qb0) * qbs;
+  const bool q_ok = have && s.q0 >= 0 && qlen > 0 && s.qb0 >= 0 && g >= s.qb0 && q_pos >= 0 && q_pos < qlen &&
+                    (int64_t)s.q0 + q_pos < total_q;
+  const bool ok = q_ok && (int64_t)s.q0 + qlen <= total_q && s.k0 >= 0 && klen_in >= 0 && (int64_t)s.k0 + klen_in <= total_k &&
+                  s.kb0 >= 0 && nkb_in >= 0 && (int64_t)s.kb0 + nkb_in <= nkb_total && (int64_t)nkb_in * kbs >= klen_in;
+  QBlockInfo r;
+  r.row_begin = q_ok ? s.q0 + q_pos : 0;
+  int rows = 0;
+  if (q_ok) {
+    rows = qlen - q_pos < qbs ? qlen - q_pos : qbs;
+    if (rows > total_q - r.row_begin) rows = total_q - r.row_begin;
+  }
+  r.rows = rows;
+  r.key_begin = ok ? s.k0 : 0;
+  r.klen = ok ? klen_in : 0;
+  r.q_pos = q_ok ? q_pos : 0;
+  r.shift = ok ? klen_in - qlen : 0;
+  r.nkblk = ok ? nkb_in : 0;
+  int kmax = 0;
+  if (ok) {
+    kmax = klen_in;
+    if (causal && q_pos + rows + r.shift < kmax) kmax = q_pos + rows + r.shift;
+    if (kmax < 0) kmax = 0;
+  }
+  r.kmax = kmax;
+  r.seq = q_ok ? s.qb0 : 0;
+  r.flags = ok ? 0 : 1;
+  r.pad[0] = r.pad[1] = 0;
+  kb0 = ok ? s.kb0 : 0;
+  return r;
+}
+
+// --------------------------------------------------------------------------------------
+// Element-type policies.
+// --------------------------------------------------------------------------------------
+struct ElemBF16 {
+  static __device__ __forceinline__ f32x16 mfma(short8v a, short8v b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+    bf16x2 v = {(__bf16)lo, (__bf16)hi};
+    return __builtin_bit_cast(uint32_t, v);
+  }
+  static __device__ __forceinline__ float lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
+  static __device__ __forceinline__ float hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+  static __device__ __forceinline__ uint32_t scale_packed(uint32_t w, float f) { return pack2(lo(w) * f, hi(w) * f); }
+  // acc + lo + hi of a packed pair (v_dot2c_f32_bf16 with a vector of ones)
+  static __device__ __forceinline__ float dot2_ones(uint32_t packed, float acc) {
+    const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), ones, acc, false);
+  }
+};
+struct ElemF16 {
+  static __device__ __forceinline__ f32x16 mfma(short8v a, short8v b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+    f16x2 v = {(_Float16)lo, (_Float16)hi};
+    return __builtin_bit_cast(uint32_t, v);
+  }
+  static __device__ __forceinline__ float lo(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w).x; }
+  static __device__ __forceinline__ float hi(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w).y; }
+  static __device__ __forceinline__ uint32_t scale_packed(uint32_t w, float f) { return pack2(lo(w) * f, hi(w) * f); }
+  static __device__ __forceinline__ float dot2_ones(uint32_t packed, float acc) {
+    const f16x2 ones = {(_Float16)1.0f, (_Float16)1.0f};
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, packed), ones, acc, false);
+  }
+};
+
+// exchange-and-combine between lane i and lane i^32
+__device__ __forceinline__ float half_max(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+__device__ __forceinline__ float half_sum(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+
+struct Sched {
+  uint32_t qnext[8];   // next unclaimed entry of each queue
+  uint32_t done;       // workgroups of the running attention launch that have made their last claim
+  // fp32 inputs staged as fp16 only (written by hbsa_setup_kernel, read by the attention kernel at its start):
+  float c;             // |softmax_scale| * log2(e), divided by the q and k staging multipliers
+  float lag;           // kLazyRescaleLog2 / c, in raw score units
+  float out_mul;       // 1 / (v staging multiplier)
+  // bit patterns of max|x| over q, k, v and the power-of-two staging multipliers
+  uint32_t amax[3];
+  float in_mul[3];
+  uint32_t pad[46];
+};
+static_assert(sizeof(Sched) == 256, "Sched is one 256-byte slot of the workspace");
+
+// ---- LDS reads issued by hand.  The compiler neither waits for these nor knows they touch LDS,
+// so each result must pass through lds_wait<N>() before it is used: LDS operations of a
+// wavefront complete in order, and lds_wait<N> returns once at most N of them are outstanding.
+// (The transposing read is issued this way because the compiler otherwise waits for every
+// outstanding global->LDS load before it; the K reads so that their issue distance is fixed.)
+// HAND = false gives the same reads as ordinary loads the compiler schedules and waits for itself (the
+// lds_wait calls then do nothing): the form for instantiations that spill registers, where a register with
+// a hand-issued read in flight could be saved before its data arrives.
+template <int OFF, bool HAND = true>
+__device__ __forceinline__ short8v lds_read_b128(uint32_t addr) {
+  if constexpr (HAND) {
+    short8v r;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(r) : "v"(addr), "n"(OFF));
+    return r;
+  } else {
+    return *(const __attribute__((address_space(3))) short8v *)(uintptr_t)(addr + (uint32_t)OFF);
+  }
+}
+template <int OFF, bool HAND = true>
+__device__ __forceinline__ short4v lds_read_tr16_b64(uint32_t addr) {
+  if constexpr (HAND) {
+    short4v r;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=&v"(r) : "v"(addr), "n"(OFF));
+    return r;
+  } else {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)(uintptr_t)(addr + (uint32_t)OFF));
+  }
+}
+template <int N>
+__device__ __forceinline__ void lds_wait1(short8v &a) {
+  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(a) : "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void lds_wait(short8v &a, short8v &b) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void lds_wait(short4v &a, short4v &b, short4v &c, short4v &d, short4v &e, short4v &f, short4v &g,
+                                         short4v &h) {
+  asm volatile("s_waitcnt lgkmcnt(%8)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f), "+v"(g), "+v"(h) : "n"(N));
+}
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+// Arguments of the backward kernels (hbsa_bwd.h).
+struct BwdParams {
+  const char *q, *k, *v, *out, *dout;
+  char *dq, *dk, *dv;
+  const float *lse;           // [total_q, nhead_q], contiguous
+  float *delta;               // [total_q, nhead_q], contiguous: rowsum(dO * O), written by the dQ kernel, read by the dK/dV kernels
+  float *lse2;                // [total_q, nhead_q]: lse * log2(e), +inf where lse is -inf; written by the dQ kernel for the D = 128 dK/dV kernel
+  const QBlockInfo *info;
+  const uint32_t *bits;
+  const int32_t *cu_k, *cu_num_q_block, *cu_num_k_block;
+  int64_t q_s, q_h, k_s, k_h, v_s, v_h, o_s, o_h, do_s, do_h, dq_s, dq_h, dk_s, dk_h, dv_s, dv_h;   // bytes
+  int32_t nqb, nkb, xcd_heads, batch, ratio, nhead_q, qbs, kbs, wpr, causal;   // xcd_heads: see the dK/dV kernels
+  int32_t total_k;
+  int32_t wps, nsub;     // q side: wave slots per q head and workgroups per (kv head, q block), as in the forward
+  int32_t nsub_k;        // k side: workgroups per (kv head, k block) = ceil(k_block_size / 128)
+  float c;               // softmax_scale * log2(e), signed
+  float scale;
+};
+
+// Keeps the message hbsa_last_error() returns and gives back `code` (defined in hbsa_fwd.hip).
+int fail(int code, const char *fmt, ...);
+
+// Launches, defined in hbsa_fwd_kernel.h, hbsa_fwd_f32.h and hbsa_bwd.h, instantiated by hbsa_inst.hip.
+template <int D, typename E, bool OUT32>
+int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
+int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D>
+int launch_fwd_f32(const FwdParams &fp, float c_signed, long long items, hipStream_t stream);
+template <int D, typename E>
+int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream);
+
+}  // namespace hbsa
