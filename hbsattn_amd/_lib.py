@@ -6,7 +6,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libhbsattn_amd.so")
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 DTYPE_BF16 = 0
 DTYPE_F16 = 1
@@ -16,6 +16,7 @@ ERR_WORKSPACE_TOO_SMALL = -3
 STATIC_SCRATCH_BYTES = 32 << 20   # HBSA_STATIC_SCRATCH_BYTES of include/hbsattn_amd.h
 
 _lib = None
+_host = None
 
 
 class HBSAttnLibraryError(RuntimeError):
@@ -55,8 +56,8 @@ def load() -> ctypes.CDLL:
     lib.hbsa_fwd.argtypes = ([vp] * 11 + [ctypes.c_size_t] + [ctypes.c_int32] * 12 + [ctypes.c_float]
                              + [ctypes.POINTER(ctypes.c_int64), vp])
     i64p = ctypes.POINTER(ctypes.c_int64)
-    # hbsa_fwd_v through a handle that keeps the interpreter lock during the call: its argument arrays are
-    # kept per shape and refilled per call, so no other Python thread may refill them while the library reads them
+    # hbsa_fwd_v through a handle that keeps the interpreter lock during the call, for callers that keep its argument
+    # arrays and refill them: no other Python thread may do so while the library reads them
     locked = ctypes.PyDLL(LIB_PATH)
     lib.hbsa_fwd_v_locked = locked.hbsa_fwd_v
     lib.hbsa_fwd_v_locked.restype = ctypes.c_int
@@ -74,6 +75,11 @@ def load() -> ctypes.CDLL:
     lib.hbsa_fwd_split_workspace_bytes.argtypes = [ctypes.c_int32] * 7
     lib.hbsa_calculate_blocks.restype = ctypes.c_int
     lib.hbsa_calculate_blocks.argtypes = [vp, ctypes.c_int32, ctypes.c_int32, vp, vp, vp, vp, ctypes.c_int32]
+    i32 = ctypes.c_int32
+    lib.hbsa_block_counts.restype = ctypes.c_int
+    lib.hbsa_block_counts.argtypes = [vp, i32, i32, vp, vp, i32, i32, vp, i32, vp, i32, vp]
+    lib.hbsa_block_arrays.restype = ctypes.c_int
+    lib.hbsa_block_arrays.argtypes = [vp, vp, i32, i32, i32, vp, vp, vp]
     lib.hbsa_bwd_workspace_bytes.restype = ctypes.c_size_t
     lib.hbsa_bwd_workspace_bytes.argtypes = [ctypes.c_int32] * 2
     lib.hbsa_bwd.restype = ctypes.c_int
@@ -81,6 +87,20 @@ def load() -> ctypes.CDLL:
                              + [ctypes.c_float, i64p, vp])
     _lib = lib
     return lib
+
+
+def host():
+    """The compiled host path (``csrc/torch_host.cpp``), which links ``libhbsattn_amd.so``."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _torch_host
+        except ImportError as e:
+            raise HBSAttnLibraryError(f"hbsattn_amd/_torch_host.so cannot be loaded ({e}): build it with "
+                                      "`python -m hbsattn_amd.build`") from e
+        _host = _torch_host
+    return _host
 
 
 def last_error() -> str:

@@ -10,6 +10,7 @@ import os
 import re
 import shutil
 import subprocess
+import sysconfig
 import tempfile
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -78,12 +79,47 @@ def link(objects, output: str) -> None:
 def build(verbose: bool = False) -> str:
     jobs = max(1, min(8, os.cpu_count() or 1))
     with tempfile.TemporaryDirectory() as objdir, concurrent.futures.ThreadPoolExecutor(jobs) as pool:
+        host = pool.submit(compile_host, objdir)
         done = list(pool.map(lambda u: compile_unit(u, objdir), units()))
         check_spills("".join(remarks for _, remarks in done), verbose)
         link([obj for obj, _ in done], OUTPUT)
+        link_host(host.result())
     if verbose:
         print(f"{OUTPUT}: {len(done)} units")
     return OUTPUT
+
+
+HOST_SOURCE = os.path.join(CSRC, "torch_host.cpp")
+HOST_OUTPUT = os.path.join(_HERE, "_torch_host.so")
+
+
+def compile_host(objdir: str) -> str:
+    """Compiles the host path (plain C++ on torch's headers, no device code)."""
+    import torch
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(objdir, "torch_host.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + os.path.join(_ROOT, "include"),
+           "-I" + sysconfig.get_paths()["include"]]
+    for path in cpp_extension.include_paths("cuda"):
+        cmd += ["-isystem", path]
+    res = subprocess.run(cmd + ["-c", HOST_SOURCE, "-o", obj], capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed: " + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+    return obj
+
+
+def link_host(obj: str) -> None:
+    """Links the host path against torch and the library built beside it."""
+    import torch
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-shared", obj, "-o", HOST_OUTPUT, "-L" + lib, "-L" + _HERE, "-lhbsattn_amd", "-ltorch_python", "-ltorch_cpu",
+           "-ltorch_hip", "-lc10", "-lc10_hip", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed: " + " ".join(cmd) + "\n" + res.stdout + res.stderr)
 
 
 def check_spills(remarks: str, verbose: bool = False) -> None:

@@ -38,7 +38,18 @@ __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 9) ((uint32_t *)p.sched)[threadIdx.x] = 0;
   if (g >= p.nqb) return;
   const int hk = blockIdx.y;
-  const int b = p.q_block_to_batch[g];
+  int b;
+  if (p.q_block_to_batch != nullptr) {
+    b = p.q_block_to_batch[g];
+  } else {   // the last sequence that starts at or before g
+    int lo = 0, hi = p.batch;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (p.cu_num_q_block[mid] <= g) lo = mid;
+      else hi = mid;
+    }
+    b = lo;
+  }
   SeqBounds sb = {0, 0, 0, 0, 0, 0, 0};
   const bool have = b >= 0 && b < p.batch;
   if (have) {
@@ -62,6 +73,92 @@ __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
     const uint64_t bal = __ballot(keep);
     if (lane < 2) row[2 * w + lane] = lane ? (uint32_t)(bal >> 32) : (uint32_t)bal;
   }
+}
+
+// Block counts of a packed batch, for up to two sides (queries and keys): first[b] = blocks before sequence b, and
+// counts = {total of side a, total of side b, 1 if both are usable, ticket} in host memory, the ticket last.  A side is
+// usable when no length is negative and its total is the expected one; otherwise every first[] is zero, which leaves
+// empty sequences (nothing is read or written for them).  One workgroup: the batch is a few hundred numbers at most, and the
+// launch itself is the cost (in place of some twenty torch launches a side).
+struct CountSide {
+  const int32_t *cu;   // nullptr: no such side
+  int32_t *first;
+  int32_t block_size, expect;   // expect < 0: any total
+};
+__global__ __launch_bounds__(kThreads) void hbsa_block_counts_kernel(CountSide sa, CountSide sb, int batch, int32_t *counts, int32_t ticket) {
+  __shared__ int wave_sum[kThreads / 64];
+  __shared__ int bad;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) bad = 0;
+  __syncthreads();
+  int totals[2] = {0, 0};
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const CountSide s = side == 0 ? sa : sb;
+    if (s.cu == nullptr) continue;
+    int before = 0;
+    for (int base = 0; base < batch; base += kThreads) {
+      const int b = base + (int)threadIdx.x;
+      int n = 0;
+      if (b < batch) {
+        const int64_t len = (int64_t)s.cu[b + 1] - s.cu[b];
+        if (len < 0) bad = 1;
+        else n = (int)((len + s.block_size - 1) / s.block_size);
+      }
+      int incl = n;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int x = __shfl_up(incl, off);
+        if (lane >= off) incl += x;
+      }
+      if (lane == 63) wave_sum[wave] = incl;
+      __syncthreads();
+      int all = 0, lower = 0;
+#pragma unroll
+      for (int w = 0; w < kThreads / 64; ++w) {
+        if (w < wave) lower += wave_sum[w];
+        all += wave_sum[w];
+      }
+      if (b < batch) s.first[b] = before + lower + incl - n;
+      before += all;
+      __syncthreads();
+    }
+    totals[side] = before;
+    if (threadIdx.x == 0) {
+      s.first[batch] = before;
+      if (s.expect >= 0 && before != s.expect) bad = 1;
+    }
+  }
+  __syncthreads();
+  if (bad)
+    for (int b = threadIdx.x; b <= batch; b += kThreads) {
+      if (sa.cu != nullptr) sa.first[b] = 0;
+      if (sb.cu != nullptr) sb.first[b] = 0;
+    }
+  if (threadIdx.x == 0) {
+    counts[0] = totals[0];
+    counts[1] = totals[1];
+    counts[2] = bad ? 0 : 1;
+    __threadfence_system();
+    __hip_atomic_store(counts + 3, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// Token boundaries and sequences of the blocks counted by hbsa_block_counts_kernel, one thread per block.
+__global__ __launch_bounds__(kThreads) void hbsa_block_arrays_kernel(const int32_t *cu, const int32_t *first, int batch, int block_size, int num_block,
+                                                                     int32_t *cu_block, int32_t *block_to_batch) {
+  const int j = blockIdx.x * kThreads + threadIdx.x;
+  if (j == 0) cu_block[0] = 0;
+  if (j >= num_block) return;
+  int lo = 0, hi = batch;   // the last sequence with first[] <= j (sequences without blocks share their successor's first[])
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (first[mid] <= j) lo = mid;
+    else hi = mid;
+  }
+  block_to_batch[j] = lo;
+  const int64_t end = (int64_t)cu[lo] + (int64_t)(j - first[lo] + 1) * block_size;
+  cu_block[j + 1] = (int32_t)(end < cu[lo + 1] ? end : (int64_t)cu[lo + 1]);
 }
 
 // Softmax constants of an attention launch on fp32 inputs staged as fp16: they follow from the maxima
@@ -542,6 +639,30 @@ int hbsa_calculate_blocks(const int32_t *cu_seqlen, int32_t batch, int32_t block
   return 0;
 }
 
+int hbsa_block_counts(const int32_t *cu_a, int32_t block_size_a, int32_t expect_a, int32_t *first_a, const int32_t *cu_b,
+                      int32_t block_size_b, int32_t expect_b, int32_t *first_b, int32_t batch, int32_t *counts, int32_t ticket,
+                      void *stream) {
+  g_err[0] = 0;
+  if (!counts || (cu_a && !first_a) || (cu_b && !first_b)) return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if (batch < 0 || (cu_a && block_size_a <= 0) || (cu_b && block_size_b <= 0))
+    return fail(HBSA_ERR_INVALID_ARGUMENT, "negative batch, or block_size not positive");
+  const CountSide a = {cu_a, first_a, block_size_a, expect_a}, b = {cu_b, first_b, block_size_b, expect_b};
+  hipLaunchKernelGGL(hbsa_block_counts_kernel, dim3(1), dim3(kThreads), 0, (hipStream_t)stream, a, b, batch, counts, ticket);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : fail((int)e, "hbsa_block_counts_kernel launch: %s", hipGetErrorString(e));
+}
+
+int hbsa_block_arrays(const int32_t *cu_seqlen, const int32_t *first, int32_t batch, int32_t block_size, int32_t num_block,
+                      int32_t *cu_block, int32_t *block_to_batch, void *stream) {
+  g_err[0] = 0;
+  if (!cu_seqlen || !first || !cu_block || (!block_to_batch && num_block > 0)) return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if (batch <= 0 || block_size <= 0 || num_block < 0) return fail(HBSA_ERR_INVALID_ARGUMENT, "batch and block_size must be positive");
+  hipLaunchKernelGGL(hbsa_block_arrays_kernel, dim3((unsigned)(num_block / kThreads + 1)), dim3(kThreads), 0, (hipStream_t)stream, cu_seqlen,
+                     first, batch, block_size, num_block, cu_block, block_to_batch);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : fail((int)e, "hbsa_block_arrays_kernel launch: %s", hipGetErrorString(e));
+}
+
 size_t hbsa_fwd_workspace_bytes(int32_t nhead_k, int32_t num_q_block, int32_t num_k_block) {
   if (nhead_k <= 0 || num_q_block <= 0 || num_k_block <= 0) return 256;
   const size_t bits = align_up((size_t)nhead_k * num_q_block * words_per_row(num_k_block) * sizeof(uint32_t), 256);
@@ -575,8 +696,8 @@ int hbsa_fwd_prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, c
   if (batch < 0 || num_q_block < 0 || num_k_block < 0 || total_q < 0 || total_k < 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
   if (num_q_block == 0) return 0;
-  if (!cu_q_seqlens || !cu_k_seqlens || !block_mask || !q_block_to_batch || !cu_num_q_block || !cu_num_k_block ||
-      !workspace || !mask_strides)
+  if (!cu_q_seqlens || !cu_k_seqlens || !block_mask || !cu_num_q_block || !cu_num_k_block || !workspace ||
+      !mask_strides)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
   if (nhead_k <= 0) return fail(HBSA_ERR_INVALID_ARGUMENT, "nhead_k must be positive");
   if (q_block_size <= 0 || k_block_size <= 0 || q_block_size % 16 || k_block_size % 16)
@@ -766,7 +887,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   if (int rc = check_strides(strides, dtype == HBSA_DTYPE_F32 || dtype == HBSA_DTYPE_F32_STAGED16)) return rc;
   if (batch < 0 || num_q_block < 0 || num_k_block < 0 || total_q < 0 || total_k < 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
-  if (!cu_q_seqlens || !cu_k_seqlens || !block_mask || !q_block_to_batch || !cu_num_q_block || !cu_num_k_block)
+  if (!cu_q_seqlens || !cu_k_seqlens || !block_mask || !cu_num_q_block || !cu_num_k_block)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
   if (q_block_size <= 0 || k_block_size <= 0 || q_block_size % 16 || k_block_size % 16)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "q_block_size (%d) and k_block_size (%d) must be positive multiples of 16",

@@ -10,6 +10,8 @@ from typing import Tuple
 
 import torch
 
+from . import _lib
+
 
 def calculate_blocks(cu_seqlen: torch.Tensor, block_size: int) -> Tuple[int, torch.Tensor, torch.Tensor, torch.Tensor]:
     """``cu_seqlen`` int tensor ``[B+1]`` (any device), ``block_size`` int.
@@ -21,6 +23,10 @@ def calculate_blocks(cu_seqlen: torch.Tensor, block_size: int) -> Tuple[int, tor
     * ``block_to_batch`` int32 ``[num_block]``: sequence index of each block
     * ``cu_num_block``   ``cu_seqlen.dtype`` ``[B+1]``: first global block index of each sequence
     """
+    if cu_seqlen.is_cuda:   # two small kernels instead of some twenty torch launches; None: not an int32 vector
+        got = _lib.host().blocks(cu_seqlen, block_size)
+        if got is not None:
+            return got
     dev = cu_seqlen.device
     lengths = cu_seqlen[1:] - cu_seqlen[:-1]
     per_seq = torch.div(lengths + (block_size - 1), block_size, rounding_mode="floor")

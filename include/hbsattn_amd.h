@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define HBSA_ABI_VERSION 6
+#define HBSA_ABI_VERSION 7
 
 /* element types of q/k/v/out (reference: dtype follows the input tensors,
  * hbsattn/fwd_triton_auto_tile_size.py:272) */
@@ -94,6 +94,23 @@ int hbsa_calculate_blocks(const int32_t *cu_seqlen, int32_t batch, int32_t block
                           int32_t *cu_block, int32_t *block_to_batch, int32_t capacity);
 
 /*
+ * The same on the DEVICE, in two launches with the counts in between (their sizes are what the arrays are
+ * allocated by).  hbsa_block_counts takes up to two sides (queries and keys; cu_x = NULL: no such side)
+ * of one batch: first_x[b] = blocks before sequence b (first_x[batch] = the total, what the other entry points call
+ * cu_num_q_block / cu_num_k_block), and writes counts[0], counts[1] = the two totals, counts[2] = 1 when
+ * no length is negative and every total is the expected one (expect_x < 0: any), and counts[3] = ticket, last.
+ * `counts` is four int32 of host memory the device can write (hipHostMalloc), so that a caller can watch
+ * counts[3] instead of waiting for the stream.  When counts[2] is 0 every first_x is zero: the attention
+ * entry points find empty sequences there.  hbsa_block_arrays writes cu_block[num_block + 1] and
+ * block_to_batch[num_block] for one side.
+ */
+int hbsa_block_counts(const int32_t *cu_a, int32_t block_size_a, int32_t expect_a, int32_t *first_a,
+                      const int32_t *cu_b, int32_t block_size_b, int32_t expect_b, int32_t *first_b,
+                      int32_t batch, int32_t *counts, int32_t ticket, void *stream);
+int hbsa_block_arrays(const int32_t *cu_seqlen, const int32_t *first, int32_t batch, int32_t block_size,
+                      int32_t num_block, int32_t *cu_block, int32_t *block_to_batch, void *stream);
+
+/*
  * Bytes of device scratch hbsa_fwd needs for this problem.  Replaces the launcher's
  * own scratch allocations (reference hbsattn/fwd_triton_auto_tile_size.py:273-274:
  * `lse`, `tmp`); here the scratch holds the compacted work description the pre-pass
@@ -145,7 +162,8 @@ size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t 
  *   cu_q_seqlens, cu_k_seqlens  int32[batch+1]  packed-sequence boundaries
  *   block_mask  bytes (0 / non-0) [nhead_k, num_q_block, num_k_block] over GLOBAL block
  *               indices; entries pairing blocks of different sequences are ignored
- *   q_block_to_batch int32[num_q_block], cu_num_q_block / cu_num_k_block int32[batch+1]
+ *   q_block_to_batch int32[num_q_block] (may be NULL: the pre-pass then finds a block's sequence in
+ *   cu_num_q_block), cu_num_q_block / cu_num_k_block int32[batch+1]
  *               exactly as hbsattn.utils.calculate_blocks returns them
  *               (reference hbsattn/utils.py:7-50)
  *   causal      bottom-right aligned: in-sequence key j visible to in-sequence query i
