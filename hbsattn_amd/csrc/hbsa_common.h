@@ -135,6 +135,7 @@ struct FwdParams {
   int32_t batch, nkb_total, total_k, qbs;
   int32_t pack;   // host side only: the launch uses the kernel whose wave slots are packed across the q heads of a GQA group
   FastDiv div_nhk;   // division by nhead_k (items handed out without queues)
+  int32_t ncol;      // 16-byte chunks of a row (the COLS form of the kernel)
 };
 
 // Boundaries of one sequence of the packed batch, as read from the caller's device arrays.
@@ -327,6 +328,8 @@ template <int D, typename E, bool OUT32>
 int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
+int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D>
 int launch_fwd_f32(const FwdParams &fp, float c_signed, long long items, hipStream_t stream);
 template <int D, typename E>

@@ -392,14 +392,15 @@ inline size_t split_bytes(int parts, int total_q, int nhead_q, int nhead_k, int 
 
 // The fields of FwdParams that follow from the call's shape and softmax_scale alone.
 void fill_shape(FwdParams &fp, int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size,
-                int k_block_size, int causal, float softmax_scale, bool f32_exact, bool may_pack = false) {
+                int k_block_size, int causal, float softmax_scale, bool f32_exact, bool may_pack = false, bool cols = false) {
   fp.nhead_k = nhead_k;
   fp.nqb = num_q_block; fp.ratio = nhead_q / nhead_k; fp.kbs = k_block_size; fp.wpr = words_per_row(num_k_block);
   fp.causal = causal ? 1 : 0;
   fp.wps = (q_block_size + kWaveRows - 1) / kWaveRows;
-  fp.pack = may_pack && fwd_packs(fp.ratio, q_block_size) ? 1 : 0;
+  fp.pack = cols || (may_pack && fwd_packs(fp.ratio, q_block_size)) ? 1 : 0;
   const int slots = fwd_slots(fp.ratio, q_block_size, fp.pack != 0);
-  fp.nw = fwd_wavefronts(slots, headdim, f32_exact);
+  fp.nw = cols ? 4 : fwd_wavefronts(slots, headdim, f32_exact);
+  fp.ncol = headdim / 8;
   fp.nsub = (slots + fp.nw - 1) / fp.nw;
   fp.div_nsub = make_fast_div((uint32_t)fp.nsub);
   fp.div_nqb = make_fast_div((uint32_t)num_q_block);
@@ -547,8 +548,9 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
                 int32_t k_block_size, int32_t causal, float softmax_scale, const int64_t *strides, hipStream_t st) {
   FwdParams fp;
   std::memset(&fp, 0, sizeof(fp));
+  const bool cols = headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256;
   fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, false,
-             true);
+             true, cols);
   const long long items = (long long)nhead_k * num_q_block * fp.nsub;
   Sched *sched = onepass_record(dtype, batch, total_k, headdim, num_k_block, k_block_size, strides[10], items, st);
   if (sched == nullptr) return kNotOnePass;
@@ -564,6 +566,15 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   fp.mask = block_mask; fp.ms_h = strides[8]; fp.ms_q = strides[9];
   fp.batch = batch; fp.nkb_total = num_k_block; fp.total_k = total_k; fp.qbs = q_block_size;
   const bool bf = dtype == HBSA_DTYPE_BF16;
+  if (cols) {   // a head dim without a kernel of its own runs in the next one up, its missing columns zero on the chip
+    if (headdim < 32) return bf ? launch_fwd_cols<32, ElemBF16>(fp, items, st) : launch_fwd_cols<32, ElemF16>(fp, items, st);
+    if (headdim < 64) return bf ? launch_fwd_cols<64, ElemBF16>(fp, items, st) : launch_fwd_cols<64, ElemF16>(fp, items, st);
+    if (headdim <= 96) return bf ? launch_fwd_cols<96, ElemBF16>(fp, items, st) : launch_fwd_cols<96, ElemF16>(fp, items, st);
+    if (headdim < 128) return bf ? launch_fwd_cols<128, ElemBF16>(fp, items, st) : launch_fwd_cols<128, ElemF16>(fp, items, st);
+    if (headdim <= 160) return bf ? launch_fwd_cols<160, ElemBF16>(fp, items, st) : launch_fwd_cols<160, ElemF16>(fp, items, st);
+    if (headdim <= 192) return bf ? launch_fwd_cols<192, ElemBF16>(fp, items, st) : launch_fwd_cols<192, ElemF16>(fp, items, st);
+    return bf ? launch_fwd_cols<256, ElemBF16>(fp, items, st) : launch_fwd_cols<256, ElemF16>(fp, items, st);
+  }
   switch (headdim) {
     case 32: return bf ? launch_fwd_fused<32, ElemBF16>(fp, items, st) : launch_fwd_fused<32, ElemF16>(fp, items, st);
     case 64: return bf ? launch_fwd_fused<64, ElemBF16>(fp, items, st) : launch_fwd_fused<64, ElemF16>(fp, items, st);
@@ -869,7 +880,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
              size_t workspace_bytes, int32_t dtype, int32_t batch, int32_t total_q, int32_t total_k,
              int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block, int32_t num_k_block,
              int32_t q_block_size, int32_t k_block_size, int32_t causal, float softmax_scale,
-             const int64_t *strides, void *stream, bool allow_onepass) {
+             const int64_t *strides, void *stream, bool allow_onepass, bool any_dim = false) {
   g_err[0] = 0;
   if (total_q == 0 || num_q_block == 0 || nhead_q == 0) return 0;
   if (!strides) return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
@@ -877,8 +888,8 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   if (!q || !k || !v || !out) return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
   if (nhead_k <= 0 || nhead_q % nhead_k != 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "nhead_q (%d) must be divisible by nhead_k (%d)", nhead_q, nhead_k);
-  if (headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256)
-    return fail(HBSA_ERR_UNSUPPORTED, "headdim %d not in {32, 64, 128, 256}", headdim);
+  if (any_dim ? headdim <= 0 || headdim > 256 || headdim % 8 != 0 : headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256)
+    return fail(HBSA_ERR_UNSUPPORTED, any_dim ? "headdim %d is no multiple of 8 up to 256" : "headdim %d not in {32, 64, 128, 256}", headdim);
   if (dtype < HBSA_DTYPE_BF16 || dtype > HBSA_DTYPE_F32_STAGED16)
     return fail(HBSA_ERR_UNSUPPORTED, "dtype code %d not supported", dtype);
   if (!std::isfinite(softmax_scale)) return fail(HBSA_ERR_INVALID_ARGUMENT, "softmax_scale is not finite");
@@ -900,6 +911,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
                                 k_block_size, causal, softmax_scale, strides, (hipStream_t)stream);
     if (one != kNotOnePass) return one;
   }
+  if (any_dim) return fail(HBSA_ERR_WORKSPACE_TOO_SMALL, "the call is not one launch: use hbsa_fwd with a workspace");
   {
     const size_t need = hbsa_fwd_workspace_bytes_dtype(dtype, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block,
                                                        num_k_block);
@@ -938,6 +950,17 @@ int hbsa_fwd_v(const void *const *ptrs, size_t workspace_bytes, const int32_t *s
                   (const uint8_t *)ptrs[6], (const int32_t *)ptrs[7], (const int32_t *)ptrs[8], (const int32_t *)ptrs[9],
                   (void *)ptrs[10], workspace_bytes, sizes[0], sizes[1], sizes[2], sizes[3], sizes[4], sizes[5], sizes[6], sizes[7],
                   sizes[8], sizes[9], sizes[10], sizes[11], softmax_scale, strides, stream, true);
+}
+
+int hbsa_fwd_one(const void *const *ptrs, const int32_t *sizes, float softmax_scale, const int64_t *strides, void *stream) {
+  if (!ptrs || !sizes) {
+    g_err[0] = 0;
+    return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
+  }
+  return fwd_call(ptrs[0], ptrs[1], ptrs[2], (void *)ptrs[3], (const int32_t *)ptrs[4], (const int32_t *)ptrs[5],
+                  (const uint8_t *)ptrs[6], (const int32_t *)ptrs[7], (const int32_t *)ptrs[8], (const int32_t *)ptrs[9],
+                  nullptr, 0, sizes[0], sizes[1], sizes[2], sizes[3], sizes[4], sizes[5], sizes[6], sizes[7],
+                  sizes[8], sizes[9], sizes[10], sizes[11], softmax_scale, strides, stream, true, true);
 }
 
 int hbsa_fwd_static(const void *q, const void *k, const void *v, void *out, const int32_t *cu_q_seqlens,

@@ -66,17 +66,19 @@ __device__ __forceinline__ int pack_tile(int pos, int valid) { return ((pos >> 4
 // Executed by one whole wavefront; `first_words`: lane i holds bit word i of the row.  Rows longer than
 // 2048 blocks ask `more_words(window)` for the words window * 64 + lane (lane i: word window * 64 + i, zero
 // past the row's end), arrived and ready to use.
-template <typename MoreWords>
+template <int KT, typename MoreWords>
 __device__ __forceinline__ int build_tile_list(int *list, int chunk_base, MoreWords &&more_words, int nwords, int kbs,
                                                 FastDiv div_kbs, int kmax, uint32_t first_words, int lane) {
   if (kmax <= 0 || nwords <= 0) return 0;
   int total = 0;
-  if ((kbs & 63) == 0) {
-    // Blocks are whole tiles: every kept block yields kbs/64 tiles (those starting at or past
+  if ((kbs & (KT - 1)) == 0) {
+    // Blocks are whole tiles: every kept block yields kbs / KT tiles (those starting at or past
     // kmax are dropped; they would be the last of the list).  Two bit words are expanded per
     // step: lane l looks at bit (l & 31) of word 2*step + (l >> 5), and its tiles go right after
     // the tiles of the kept blocks below it.
-    const int tpb = kbs >> 6;
+    constexpr int kShift = KT == 64 ? 6 : 5;
+    static_assert(1 << kShift == KT, "tiles of 64 or 32 keys");
+    const int tpb = kbs >> kShift;
     const int half = lane >> 5, bit = lane & 31;
     const int j_last = (int)fast_div((uint32_t)(kmax - 1), div_kbs);   // no bit above this block is set
     int window = 0;
@@ -95,14 +97,14 @@ __device__ __forceinline__ int build_tile_list(int *list, int chunk_base, MoreWo
         const int j = (w2 + half) * 32 + bit;
         int off = total + below * tpb - chunk_base;
         for (int t = 0; t < tpb; ++t, ++off) {
-          const int pos = j * kbs + 64 * t;
-          if (pos < kmax && off >= 0 && off < kListCap) list[off] = pack_tile(pos, min(kTileKeys, kmax - pos));
+          const int pos = j * kbs + KT * t;
+          if (pos < kmax && off >= 0 && off < kListCap) list[off] = pack_tile(pos, min(KT, kmax - pos));
         }
       }
       total += (__builtin_popcount(lo) + __builtin_popcount(hi)) * tpb;
       if ((j_last >> 6) == (w2 >> 1)) {   // tiles dropped at the end of the last visible block
         const uint32_t wsel = (j_last & 32) ? hi : lo;
-        if ((wsel >> (j_last & 31)) & 1u) total -= tpb - ((kmax - j_last * kbs + 63) >> 6);
+        if ((wsel >> (j_last & 31)) & 1u) total -= tpb - ((kmax - j_last * kbs + KT - 1) >> kShift);
       }
     }
   } else {
@@ -135,9 +137,9 @@ __device__ __forceinline__ int build_tile_list(int *list, int chunk_base, MoreWo
       const int stop = (w >= nwords) ? nwords * 32 : w * 32 + __builtin_ctz(inv);
       blk = stop;
       const int end = min(stop * kbs, kmax);
-      for (int pos = first * kbs; pos < end; pos += kTileKeys) {
+      for (int pos = first * kbs; pos < end; pos += KT) {
         const int off = total - chunk_base;
-        if (lane == 0 && off >= 0 && off < kListCap) list[off] = pack_tile(pos, min(kTileKeys, end - pos));
+        if (lane == 0 && off >= 0 && off < kListCap) list[off] = pack_tile(pos, min(KT, end - pos));
         ++total;
       }
       if (end >= kmax) break;
@@ -146,8 +148,24 @@ __device__ __forceinline__ int build_tile_list(int *list, int chunk_base, MoreWo
   return total;
 }
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK>
-__global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel(FwdParams p) {
+// Placement of a K / V tile's rows in LDS: 16-byte chunk c of row r sits at chunk position c ^ k(r) (K), c ^ v(r) (V).
+// Rows by 16 consecutive ones (K, one chunk column at a time) then start at 16 different 16-byte slots of the 256-byte
+// bank sweep, and the 4 rows x 64 bytes of a transposing V read cover it once.  With a row of 4, 8, 16 or 32 chunks
+// that takes an exclusive or over all chunk bits; rows of 12, 20 and 24 chunks already step by 12, 4 and 8 slots, so
+// that the low two or three bits are enough (and the exchange stays inside the row).
+template <int D>
+struct FwdSwizzle {
+  static constexpr int CPR = D / 8;
+  static constexpr int RPG = 16 / CPR > 0 ? 16 / CPR : 1;   // rows per 256-byte bank sweep
+  static constexpr bool POW2 = (CPR & (CPR - 1)) == 0;
+  static __device__ __forceinline__ int k(int r) { return POW2 ? (r / RPG) % CPR : CPR % 8 == 0 ? (r >> 1) & 7 : (r >> 2) & 3; }
+  static __device__ __forceinline__ int v(int r) {
+    return POW2 ? (CPR >= 8 ? ((r / RPG) % (CPR / 4)) << 2 : 0) : CPR % 8 == 0 ? ((r >> 1) & 1) << 2 : 0;
+  }
+};
+
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS>
+__global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel(FwdParams p) {
   // OUT32: fp32 output (the fp32-input path; q/k/v are then fp16 staging copies)
   // EXTRAS: the clocked walk, the split over key blocks and the log-sum-exp output are compiled in.  The
   // plain call uses none of them, and its kernel is a tenth shorter without them (1-2 % faster: eight
@@ -157,18 +175,25 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // fetches into an LDS staging area one item ahead, where the other form fetches the prepared records.
   // PACK: wave slots packed across the q heads of a GQA group (see slot_of below); instantiated for the
   // one-launch form only, since either placement of the queries gives the same results bit for bit.
+  // COLS: the tensors' rows hold p.ncol <= D / 8 chunks of eight elements (a head dim that is no D of its own).  The
+  // columns past them are zero in LDS (cleared once, never loaded) and in the Q operand, and not stored: in place of
+  // zero-padded copies of q, k, v and a copy of the output.
   // NW: wavefronts (wave slots) of a workgroup, 4 or 8.  Eight are used when the q heads of a GQA group
   // and the 32-row slices of a q block give an item more than four wave slots: one workgroup per CU then
   // stages every K/V tile once for all of them instead of two workgroups staging it each.
   constexpr int RB = D * 2;            // row bytes
   constexpr int CPR = RB / 16;         // 16-byte chunks per row
-  constexpr int RPG = 16 / CPR > 0 ? 16 / CPR : 1;  // rows per 256-byte bank sweep
-  constexpr int TILE_BYTES = kTileKeys * RB;
-  constexpr int LOADS = CPR / NW;      // 16-byte loads per thread per tile per operand
-  static_assert(LOADS >= 1, "a tile row has fewer 16-byte chunks than the workgroup has wavefronts");
+  // Keys per tile.  At head dims 160 and 192 tiles of 32 keys let two workgroups share a CU (their LDS, and the
+  // registers of a wavefront with one half tile in the making): 8 x ~2000 tokens, 16 heads of 192, fp16, keep 0.3: see
+  // launch_fwd_cols for the measurement.
+  constexpr int KT = D > 128 && D <= 192 ? 32 : 64;
+  constexpr int TILE_BYTES = KT * RB;
+  constexpr int LOADS = (CPR * KT + 64 * NW - 1) / (64 * NW);   // 16-byte loads per thread per tile per operand
+  constexpr bool LAST_PART = CPR * KT % (64 * NW) != 0;         // the last round is for the first wavefronts only
+  using SW = FwdSwizzle<D>;
   constexpr int KSTEPS = D / 16;       // MFMA k-steps of Q.K^T
   constexpr int DT = D / 32;           // 32-row tiles of O^T
-  constexpr bool HAND = D <= 128;      // operand reads from LDS issued and waited for by hand (see lds_read_b128)
+  constexpr bool HAND = D <= 192;      // operand reads from LDS issued and waited for by hand (see lds_read_b128)
 
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   char *lds_k = lds;
@@ -402,11 +427,11 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
       if constexpr (FUSED) {
         // the staged bytes arrived with the wait of a tile (or of the kernel's first lines) since stage()
         st_bits = st_nvis > 0 ? staged_words(st_ms, min(st_nvis, kMaskWindow)) : 0u;
-        total = build_tile_list(lds_list + c * kListCap, 0, fused_more_words(st_mrow, st_nvis), 2 * ((st_nvis + 63) >> 6),
+        total = build_tile_list<KT>(lds_list + c * kListCap, 0, fused_more_words(st_mrow, st_nvis), 2 * ((st_nvis + 63) >> 6),
                                 p.kbs, p.div_kbs, kmax, st_bits, lane);
       } else {
         const int nwords = 2 * ((nkblk + 63) >> 6);
-        total = build_tile_list(lds_list + c * kListCap, 0,
+        total = build_tile_list<KT>(lds_list + c * kListCap, 0,
                                 prepared_more_words(p.bits + (((size_t)st_part * p.nhead_k + st_hk) * p.nqb + st_qb) * p.wpr, nwords),
                                 nwords, p.kbs, p.div_kbs, kmax, st_bits, lane);
       }
@@ -512,6 +537,9 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
     w_ptr = nullptr;
   };
 
+  if constexpr (COLS) {
+    for (int i = threadIdx.x; i < 4 * TILE_BYTES / 16; i += NW * 64) *(u32x4 *)(lds_k + i * 16) = u32x4{0u, 0u, 0u, 0u};
+  }
   if (wave == 0) {
     if constexpr (FUSED) {   // the sequences' boundaries, for fused_geometry()
       for (int i = lane; i <= p.batch; i += 64) {
@@ -535,13 +563,14 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // ------------------------------------------------------------------ per-thread constants
   // tile loads: thread -> (row, 16-byte chunk) of the tile, same for every tile
   uint32_t ld_koff[LOADS], ld_voff[LOADS];   // byte offset of the thread's chunk from the tile's first row
+  bool ld_kin[LOADS], ld_vin[LOADS];         // COLS: the chunk is one of the row's
   const uint32_t ks32 = (uint32_t)p.k_s, vs32 = (uint32_t)p.v_s;   // row strides in bytes (the host checks they fit)
   auto ld_place = [&](int i, int &r, uint32_t &kchunk, uint32_t &vchunk) {
     const int c = (i * NW + wave) * 64 + lane;
     const int pc = c % CPR;
     r = c / CPR;
-    kchunk = (uint32_t)((pc ^ ((r / RPG) % CPR)) * 16);
-    vchunk = (uint32_t)((pc ^ ((CPR >= 8) ? (((r / RPG) % (CPR / 4)) << 2) : 0)) * 16);
+    kchunk = (uint32_t)((pc ^ SW::k(r)) * 16);
+    vchunk = (uint32_t)((pc ^ SW::v(r)) * 16);
   };
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
@@ -549,6 +578,8 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
     ld_place(i, r, kc, vc);
     ld_koff[i] = (uint32_t)r * ks32 + kc;
     ld_voff[i] = (uint32_t)r * vs32 + vc;
+    ld_kin[i] = !COLS || kc < (uint32_t)p.ncol * 16u;
+    ld_vin[i] = !COLS || vc < (uint32_t)p.ncol * 16u;
   }
   const uint32_t lds_k_addr = (uint32_t)(uintptr_t)HBSA_AS3(lds_k);
   // kbase / vbase: wavefront-uniform address of the tile's first key row (for this kv head).
@@ -569,9 +600,10 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
     constexpr bool V_PART = decltype(v_part_)::value;
     constexpr int lds_off = V_PART ? 2 * TILE_BYTES : 0;
     const uint32_t l0 = lds_k_addr + (uint32_t)(buf * TILE_BYTES) + (uint32_t)wave * 1024u;
-    if (valid == kTileKeys) {
+    if (valid == KT) {
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
+        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))   // (a lane that loads nothing leaves its 16 bytes of LDS alone)
         dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, V_PART ? ld_voff[i] : ld_koff[i], l0);
       });
     } else {   // ragged tail of a run: rows past the end re-read the last valid row (masked later)
@@ -580,6 +612,7 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
         int r; uint32_t kc, vc;
         ld_place(i, r, kc, vc);
         r = min(r, valid - 1);
+        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))
         dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, (uint32_t)r * (V_PART ? vs32 : ks32) + (V_PART ? vc : kc), l0);
       });
     }
@@ -593,34 +626,34 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
 
   // per-lane LDS read addresses
   // K (A operand of S^T): row l32 (+32), chunk (2*ks + g32) ^ swz(row)
-  const int k_rd = l32 * RB + ((g32 ^ ((l32 / RPG) % CPR)) << 4);
   // V^T (A operand of O^T) through ds_read_b64_tr_b16: within a group of 16 lanes, lane r
   // supplies the address of key (r / 4), dims 4*(r % 4) .. +3 and receives dim r of 4 keys.
   const int v_key = 4 * g32 + ((lane & 15) >> 2);
   const int v_lc = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-  const int v_swz = (CPR >= 8) ? (((v_key / RPG) % (CPR / 4)) << 2) : 0;
-  const int v_rd = v_key * RB + ((v_lc | v_swz) << 4) + 8 * (lane & 1);
+  const int v_rd = v_key * RB + 8 * (lane & 1);
 
   // Absolute LDS addresses of this lane's operand reads in the CURRENT tile buffer: one per k-step
   // for K, one per 32-dim block for V.  flip_buffers() moves them to the other buffer with one add
   // each (the two buffers of K, and of V, are TILE_BYTES apart), so the per-tile path has no
   // address arithmetic besides that.
-  uint32_t k_addr[KSTEPS], v_addr[DT];
+  // (Where the swizzle touches the low chunk bits only, k-steps and blocks further on are immediate offsets.)
+  constexpr int KADDR = SW::POW2 ? KSTEPS : CPR % 8 == 0 ? 4 : 2, VADDR = SW::POW2 ? DT : CPR % 8 == 0 ? 2 : 1;
+  uint32_t k_addr[KADDR], v_addr[VADDR];
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) k_addr[ks] = lds_k_addr + (uint32_t)(k_rd ^ (ks * 32));
+  for (int ks = 0; ks < KADDR; ++ks) k_addr[ks] = lds_k_addr + (uint32_t)(l32 * RB + (((2 * ks + g32) ^ SW::k(l32)) << 4));
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) v_addr[dt] = lds_k_addr + 2 * TILE_BYTES + (uint32_t)(v_rd ^ (dt * 64));
+  for (int dt = 0; dt < VADDR; ++dt) v_addr[dt] = lds_k_addr + 2 * TILE_BYTES + (uint32_t)(v_rd + (((4 * dt + v_lc) ^ SW::v(v_key)) << 4));
   int buf = 0;
   auto flip_buffers = [&]() {
     buf ^= 1;
     const uint32_t step = buf ? (uint32_t)TILE_BYTES : (uint32_t)-TILE_BYTES;
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
+    for (int ks = 0; ks < KADDR; ++ks) {
       k_addr[ks] += step;
       asm volatile("" : "+v"(k_addr[ks]));   // keep it in its register instead of recomputing it per read
     }
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
+    for (int dt = 0; dt < VADDR; ++dt) {
       v_addr[dt] += step;
       asm volatile("" : "+v"(v_addr[dt]));
     }
@@ -703,7 +736,11 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
     if constexpr (KSTEPS >= 2) {
 #pragma unroll
       for (int k = 0; k < KSTEPS / 2; ++k) {
-        u32x4 a = *(const u32x4 *)(ra + 64 * k), b = *(const u32x4 *)(rb + 64 * k);
+        u32x4 a = {0u, 0u, 0u, 0u}, b = a;
+        if (!COLS || 4 * k + ((lane >> 4) & 1) * 2 + g32 < p.ncol) {
+          a = *(const u32x4 *)(ra + 64 * k);
+          b = *(const u32x4 *)(rb + 64 * k);
+        }
         a ^= p.q_sign;
         b ^= p.q_sign;
 #pragma unroll
@@ -844,7 +881,7 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
           // The tile is processed as two halves of 32 keys so that, inside one wavefront, the
           // matrix cores always have work queued while the vector ALU does the softmax of the
           // other half:   S0, max(S0) | S1 + exp(S0) | PV0 + max(S1), exp(S1) | PV1.
-          const bool edge = valid < kTileKeys || (p.causal && kpos + valid - 1 > wave_kvis_min);
+          const bool edge = valid < KT || (p.causal && kpos + valid - 1 > wave_kvis_min);
           int lim = valid;                      // keys (of this lane's query) below lim are visible
           if (p.causal) lim = min(lim, lane_kvis - kpos + 1);
           lim -= 4 * g32;
@@ -856,13 +893,14 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
           // ---- K operand reads: 2 * KSTEPS reads (all k-steps of the first 32 keys, then of the
           // second 32), PF of them in flight, each consumed by one MFMA
           constexpr int PF = 4;
-          constexpr int NK = 2 * KSTEPS;
+          constexpr int NK = KT / 32 * KSTEPS;
           short8v kb[PF];
           auto read_k = [&](auto i_) {
             constexpr int i = decltype(i_)::value;
             constexpr int ks = i % KSTEPS;
-            if constexpr (i < KSTEPS) kb[i % PF] = lds_read_b128<0, HAND>(k_addr[ks]);
-            else kb[i % PF] = lds_read_b128<32 * RB, HAND>(k_addr[ks]);
+            constexpr int off = ks / KADDR * KADDR * 32;
+            if constexpr (i < KSTEPS) kb[i % PF] = lds_read_b128<off, HAND>(k_addr[ks % KADDR]);
+            else kb[i % PF] = lds_read_b128<off + 32 * RB, HAND>(k_addr[ks % KADDR]);
           };
           static_for<0, PF>(read_k);
           // the next tile's K is requested while this tile's first operands are on their way from LDS
@@ -927,8 +965,9 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
             constexpr int g = decltype(g_)::value;
             static_for<0, DT>([&](auto dt_) {
               constexpr int dt = decltype(dt_)::value;
-              dst[2 * dt] = lds_read_tr16_b64<g * 16 * RB, HAND>(v_addr[dt]);
-              dst[2 * dt + 1] = lds_read_tr16_b64<g * 16 * RB + 8 * RB, HAND>(v_addr[dt]);
+              constexpr int off = g * 16 * RB + dt / VADDR * VADDR * 64;
+              dst[2 * dt] = lds_read_tr16_b64<off, HAND>(v_addr[dt % VADDR]);
+              dst[2 * dt + 1] = lds_read_tr16_b64<off + 8 * RB, HAND>(v_addr[dt % VADDR]);
             });
           };
           auto wait_vgroup = [&](auto n_, short4v *v) {
@@ -937,6 +976,12 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
               (void)v;   // the compiler waits for its own reads
             } else if constexpr (DT == 4) {
               lds_wait<n>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
+            } else if constexpr (DT > 4) {
+              asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(v[0]), "+v"(v[1]) : "n"(n));
+#pragma unroll
+              for (int i = 2; i < 2 * DT; i += 2) asm volatile("" : "+v"(v[i]), "+v"(v[i + 1]));
+            } else if constexpr (DT == 3) {
+              asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]) : "n"(n));
             } else if constexpr (DT == 2) {
               asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : "n"(n));
             } else {
@@ -951,6 +996,19 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
             }
           };
 
+          if constexpr (KT == 32) {
+            // one half: its V operands are on their way while the vector ALU does the softmax
+            short8v p0a, p0b;
+            short4v vb[2 * DT];
+            read_vgroup(std::integral_constant<int, 0>{}, vb);
+            half_rowmax(s0, 0);
+            half_exp(s0, p0a, p0b);
+            wait_vgroup(std::integral_constant<int, 0>{}, vb);
+            pv_group(p0a, vb);
+            read_vgroup(std::integral_constant<int, 1>{}, vb);
+            wait_vgroup(std::integral_constant<int, 0>{}, vb);
+            pv_group(p0b, vb);
+          } else {
           half_rowmax(s0, 0);
 
           // ---- S1 = K[32:64] . Q^T   interleaved with   P0 = exp(S0)
@@ -1014,6 +1072,7 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
           pv_group(p1a, vb[0]);
           wait_vgroup(std::integral_constant<int, 0>{}, vb[1]);
           pv_group(p1b, vb[1]);
+          }
         }
         if (last && nxt_hk >= 0) {
           // Q of this item is no longer needed: fetch the next item's rows while the last MFMAs
@@ -1035,7 +1094,7 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
           const int nvis = min(inf.nkblk, (int)fast_div((uint32_t)(inf.kmax + p.kbs - 1), p.div_kbs));
           auto more = fused_more_words(p.mask + (int64_t)cur_hk * p.ms_h + (int64_t)qb * p.ms_q + kb0, nvis);
           const uint32_t first = more(0);
-          (void)build_tile_list(lds_list + c * kListCap, chunk_base, more, 2 * ((nvis + 63) >> 6), p.kbs, p.div_kbs, inf.kmax,
+          (void)build_tile_list<KT>(lds_list + c * kListCap, chunk_base, more, 2 * ((nvis + 63) >> 6), p.kbs, p.div_kbs, inf.kmax,
                                 first, lane);
           // the staging area held the staged item's bytes: request them again (they arrive with the next tile's wait)
           if (st_hk >= 0 && st_nvis > 0) st_ms = mask_dma(st_mrow, 0, min(st_nvis, kMaskWindow));
@@ -1043,7 +1102,7 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
           const QBlockInfo inf = p.info[qb];
           const uint32_t *row = p.bits + (((size_t)cur_part * p.nhead_k + cur_hk) * p.nqb + qb) * p.wpr;
           const int nwords = 2 * ((inf.nkblk + 63) >> 6);
-          (void)build_tile_list(lds_list + c * kListCap, chunk_base, prepared_more_words(row, nwords), nwords, p.kbs, p.div_kbs,
+          (void)build_tile_list<KT>(lds_list + c * kListCap, chunk_base, prepared_more_words(row, nwords), nwords, p.kbs, p.div_kbs,
                                 inf.kmax, lane < nwords ? row[lane] : 0u, lane);
         }
       }
@@ -1128,8 +1187,9 @@ __global__ __launch_bounds__(NW * 64, D > 128 ? 1 : 8 / NW) void hbsa_fwd_kernel
             w[0][j] = r[0];
             w[1][j] = r[1];
           }
-          if (st_x) *(u32x4 *)(row_x + dt * 64) = w[0];
-          if (st_y) *(u32x4 *)(row_y + dt * 64) = w[1];
+          const bool in = !COLS || 4 * dt + ((lane >> 4) & 1) * 2 + g32 < p.ncol;
+          if (st_x && in) *(u32x4 *)(row_x + dt * 64) = w[0];
+          if (st_y && in) *(u32x4 *)(row_y + dt * 64) = w[1];
         }
       }
       }
@@ -1170,10 +1230,10 @@ inline int persistent_grid(const void *kernel, int lds_bytes, int threads) {
   return cus * per_cu;
 }
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false>
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false, bool COLS = false>
 int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
-  constexpr int lds_bytes = 4 * kTileKeys * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
-  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK>);
+  constexpr int lds_bytes = 4 * (D > 128 && D <= 192 ? 32 : 64) * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
+  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS>);
   // workgroups that fit the current device at once; the attribute and the occupancy are per device
   static thread_local int resident_of[kMaxDevices] = {};
   int dev = 0;
@@ -1191,7 +1251,7 @@ int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   // Few items per workgroup: a fixed order instead of the per-XCD queues, whose round trips (and, with few kv
   // heads, the crowd at few counters) would be a good part of such a launch.
   launch.one_each = items <= (long long)kStaticShare * resident ? (int)items : 0;
-  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
+  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, "hbsa_fwd_kernel launch: %s", hipGetErrorString(e));
   return 0;
@@ -1215,6 +1275,12 @@ int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream) {
   }
   return fp.pack ? launch_fwd_nw<D, E, false, 4, false, true, true>(fp, items, stream)
                  : launch_fwd_nw<D, E, false, 4, false, true, false>(fp, items, stream);
+}
+
+// the one-launch form for tensors whose head dim (fp.ncol chunks of eight elements) is D or less
+template <int D, typename E>
+int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream) {
+  return launch_fwd_nw<D, E, false, 4, false, true, true, true>(fp, items, stream);
 }
 
 }  // namespace hbsa

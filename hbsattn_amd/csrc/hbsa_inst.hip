@@ -2,6 +2,7 @@
 // once for each value of HBSA_D (32, 64, 128, 256), HBSA_E (ElemBF16, ElemF16) and HBSA_PART:
 //   1  forward with 16-bit output (both forms)     2  forward with fp32 output (fp32 tensors staged as fp16)
 //   3  backward                                    4  forward on fp32 operands
+//   5  forward, head dims up to HBSA_D (also 96, 160 and 192)
 #if HBSA_PART == 1
 #include "hbsa_fwd_kernel.h"
 template int hbsa::launch_fwd<HBSA_D, hbsa::HBSA_E, false>(const FwdParams &, long long, hipStream_t);
@@ -15,6 +16,9 @@ template int hbsa::launch_bwd<HBSA_D, hbsa::HBSA_E>(const BwdParams &, int, int,
 #elif HBSA_PART == 4
 #include "hbsa_fwd_f32.h"
 template int hbsa::launch_fwd_f32<HBSA_D>(const FwdParams &, float, long long, hipStream_t);
+#elif HBSA_PART == 5
+#include "hbsa_fwd_kernel.h"
+template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
 #else
-#error "HBSA_PART is 1, 2, 3 or 4"
+#error "HBSA_PART is 1 to 5"
 #endif

@@ -122,6 +122,9 @@ size_t workspace_bytes(const Problem &p) {
 
 at::Tensor bytes_like(const at::Tensor &t, size_t n) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
 
+bool native_dim(int64_t d) { return d == 32 || d == 64 || d == 128 || d == 256; }
+
+// The output; undefined when the head dim has to be padded first.
 at::Tensor plain_forward(const Problem &p, hipStream_t stream) {
   at::Tensor out = at::empty(p.q.sizes(), p.q.options());
   const int64_t strides[11] = {p.q.stride(0), p.q.stride(1), p.k.stride(0), p.k.stride(1), p.v.stride(0), p.v.stride(1),
@@ -133,6 +136,12 @@ at::Tensor plain_forward(const Problem &p, hipStream_t stream) {
                           p.cu_q.const_data_ptr(), p.cu_k.const_data_ptr(), p.mask.const_data_ptr(),
                           p.qb2b.defined() ? p.qb2b.const_data_ptr() : nullptr, p.cu_nqb.const_data_ptr(), p.cu_nkb.const_data_ptr(),
                           nullptr};
+  if (!native_dim(p.q.size(2))) {
+    const int rc = hbsa_fwd_one(ptrs, sizes, (float)p.scale, strides, stream);
+    if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) return at::Tensor();   // no single launch: the caller pads
+    if (rc != 0) raise("hbsa_fwd_one", rc);
+    return out;
+  }
   int rc = hbsa_fwd_v(ptrs, 0, sizes, (float)p.scale, strides, stream);
   if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) {   // nothing was launched: this call is no single launch
     const size_t n = workspace_bytes(p);
@@ -252,7 +261,7 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
   if (p.q.dim() != 3 || p.k.dim() != 3 || p.v.dim() != 3 || p.mask.dim() != 3 || p.cu_q.dim() != 1) Py_RETURN_NONE;
   const int64_t tq = p.q.size(0), tk = p.k.size(0), hq = p.q.size(1), hk = p.k.size(1), d = p.q.size(2);
   if (tq <= 0 || tk <= 0 || tq > 0x7fffffff || tk > 0x7fffffff || hq <= 0 || hk <= 0 || hq % hk != 0) Py_RETURN_NONE;
-  if (d != 32 && d != 64 && d != 128 && d != 256) Py_RETURN_NONE;
+  if (d <= 0 || d > 256 || (!native_dim(d) && (d % 8 != 0 || st == at::kFloat))) Py_RETURN_NONE;
   if (p.k.size(2) != d || p.v.sizes() != p.k.sizes()) Py_RETURN_NONE;
   if (!rows_ok(p.q) || !rows_ok(p.k) || !rows_ok(p.v)) Py_RETURN_NONE;
   if (!to_int(a[A_QBS], p.qbs) || !to_int(a[A_KBS], p.kbs) || p.qbs <= 0 || p.kbs <= 0 || p.qbs % 16 || p.kbs % 16 ||
@@ -273,7 +282,7 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     Py_RETURN_NONE;
 
   const bool wants_grad = at::GradMode::is_enabled() && (p.q.requires_grad() || p.k.requires_grad() || p.v.requires_grad());
-  if (wants_grad && (st == at::kFloat || d > 128)) Py_RETURN_NONE;
+  if (wants_grad && (st == at::kFloat || d > 128 || !native_dim(d))) Py_RETURN_NONE;
 
   // Block metadata is all-or-recompute per side.
   const bool q_given = a[A_NQB] != Py_None && a[A_CUQB] != Py_None && a[A_QB2B] != Py_None && a[A_CUNQB] != Py_None;
@@ -342,7 +351,7 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     Py_END_ALLOW_THREADS
     g_slots.give_back(slot);
   }
-  if (!counts_fit) Py_RETURN_NONE;
+  if (!counts_fit || !out.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }

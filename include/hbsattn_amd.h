@@ -223,6 +223,14 @@ int hbsa_fwd_v(const void *const *ptrs, size_t workspace_bytes, const int32_t *s
                const int64_t *strides, void *stream);
 
 /*
+ * hbsa_fwd_v without a workspace: the one-launch form alone, for any head dim that is a multiple of 8 up to 256 (a
+ * head dim other than 32, 64, 128 and 256 runs in the next larger kernel with its missing columns zero on the chip;
+ * 96, 160 and 192 have kernels of their own).  ptrs[10] is not looked at.  HBSA_ERR_WORKSPACE_TOO_SMALL, and nothing
+ * launched, when the one-launch form does not apply to the call.
+ */
+int hbsa_fwd_one(const void *const *ptrs, const int32_t *sizes, float softmax_scale, const int64_t *strides, void *stream);
+
+/*
  * hbsa_fwd for callers that cannot allocate device memory or pass a workspace: code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
  * reference (whose launcher allocates its scratch with torch on every call, reference
