@@ -75,6 +75,8 @@ def load() -> ctypes.CDLL:
                                      + [ctypes.c_float, i64p, vp])
     lib.hbsa_fwd_split_workspace_bytes.restype = ctypes.c_size_t
     lib.hbsa_fwd_split_workspace_bytes.argtypes = [ctypes.c_int32] * 7
+    lib.hbsa_fwd_parts_bytes.restype = ctypes.c_size_t
+    lib.hbsa_fwd_parts_bytes.argtypes = [ctypes.c_int32] * 8
     lib.hbsa_calculate_blocks.restype = ctypes.c_int
     lib.hbsa_calculate_blocks.argtypes = [vp, ctypes.c_int32, ctypes.c_int32, vp, vp, vp, vp, ctypes.c_int32]
     i32 = ctypes.c_int32

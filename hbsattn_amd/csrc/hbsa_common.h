@@ -39,6 +39,7 @@ constexpr int kWalkReportTiles = 8;   // an item adds its progress to its walk c
 constexpr float kLog2e = 1.4426950408889634f;
 // One-launch form: sequences whose boundaries the scheduler keeps in LDS (batch + 1 entries of four arrays)
 constexpr int kSeqCap = 128;
+constexpr int kMaxPartItems = 4096;   // items of a launch that may be cut into parts (its arrival counters)
 constexpr int kMaxDevices = 64;            // devices of one process the launch caches cover
 constexpr float kLazyRescaleLog2 = 8.0f;  // running max may lag the true max by 2^8
 
@@ -136,6 +137,14 @@ struct FwdParams {
   int32_t pack;   // host side only: the launch uses the kernel whose wave slots are packed across the q heads of a GQA group
   FastDiv div_nhk;   // division by nhead_k (items handed out without queues)
   int32_t ncol;      // 16-byte chunks of a row (the COLS form of the kernel)
+  // Kernels that cut an item's k blocks into parts, one workgroup each, and combine them themselves (see ItemParts)
+  int64_t ms_k;          // stride of the mask's innermost dimension
+  int32_t max_parts;     // parts of an item at most (1: items are whole)
+  int32_t min_blocks;    // k blocks of a part at least
+  float *parts;          // partial results
+  FastDiv div_items;     // division by the number of items
+  int32_t parts_last;    // workgroups are numbered by part first (else: the parts of an item are neighbours)
+  uint32_t *arrivals;    // one counter per item, zero before and after every launch
 };
 
 // Boundaries of one sequence of the packed batch, as read from the caller's device arrays.
@@ -319,6 +328,78 @@ struct BwdParams {
   float c;               // softmax_scale * log2(e), signed
   float scale;
 };
+
+// ---- Items of the kernels without a scheduler: geometry and kept blocks straight from the caller's arrays (bits == nullptr)
+// or from a prepared workspace.  Everything here is uniform over the calling wavefront.
+__device__ __forceinline__ QBlockInfo item_geometry(const FwdParams &p, int qb, int lane, int &kb0) {
+  if (p.bits != nullptr) {
+    const uint32_t w = lane < 12 ? ((const uint32_t *)(p.info + qb))[lane] : 0u;
+    QBlockInfo r;
+    int32_t *f = (int32_t *)&r;
+#pragma unroll
+    for (int i = 0; i < 12; ++i) f[i] = __builtin_amdgcn_readlane((int)w, i);
+    kb0 = 0;
+    return r;
+  }
+  int b = 0;   // sequences that start at or before qb, minus one
+  for (int base = 0; base < p.batch; base += 64) {
+    const int i = base + lane + 1;
+    const int first_qb = i <= p.batch ? p.cu_nqb[i] : 0x7fffffff;
+    b += __builtin_popcountll(__builtin_amdgcn_ballot_w64(first_qb <= qb));
+  }
+  const bool have = b < p.batch;
+  SeqBounds s = {0, 0, 0, 0, 0, 0, 0};
+  if (have) {   // seven numbers, one load
+    const int32_t *at = lane < 2 ? p.cu_q + b + lane : lane < 4 ? p.cu_k + b + lane - 2 : lane < 6 ? p.cu_nkb + b + lane - 4 : p.cu_nqb + b;
+    const int v = lane < 7 ? *at : 0;
+    s.q0 = __builtin_amdgcn_readlane(v, 0); s.q1 = __builtin_amdgcn_readlane(v, 1);
+    s.k0 = __builtin_amdgcn_readlane(v, 2); s.k1 = __builtin_amdgcn_readlane(v, 3);
+    s.kb0 = __builtin_amdgcn_readlane(v, 4); s.kb1 = __builtin_amdgcn_readlane(v, 5);
+    s.qb0 = __builtin_amdgcn_readlane(v, 6);
+  }
+  return q_block_geometry(qb, have, s, p.qbs, p.kbs, p.causal, p.nkb_total, p.total_q, p.total_k, kb0);
+}
+
+// Kept k blocks among blocks first .. first + 63 of the q block's own sequence, those below `end` only.  The load and the
+// vote are apart, so that the load can be on its way while something else is done.
+struct KeptWindow {
+  const FwdParams &p;
+  const uint32_t *row;     // prepared bit row, or
+  const uint8_t *mrow;     // mask byte of the sequence's first k block
+  int lane;
+  __device__ __forceinline__ KeptWindow(const FwdParams &p_, int hk, int qb, int kb0, int lane_) : p(p_), lane(lane_) {
+    row = p.bits != nullptr ? p.bits + ((size_t)hk * p.nqb + qb) * p.wpr : nullptr;
+    mrow = p.mask + (int64_t)hk * p.ms_h + (int64_t)qb * p.ms_q + (int64_t)kb0 * p.ms_k;
+  }
+  __device__ __forceinline__ uint32_t load(int first, int end) const {
+    const int j = first + lane;
+    if (j >= end) return 0u;
+    return row != nullptr ? (row[j >> 5] >> (j & 31)) & 1u : (uint32_t)mrow[(int64_t)j * p.ms_k];
+  }
+  static __device__ __forceinline__ uint64_t vote(uint32_t loaded) { return __builtin_amdgcn_ballot_w64(loaded != 0); }
+};
+
+// An item's visible k blocks [0, nvis) cut into parts of `per` blocks: as few as keep a part at min_blocks or more, at most
+// max_parts.  Every part is one workgroup; the one that arrives last combines the others' partial results with its own, in
+// the order of the parts, so the result does not depend on the order of arrival.
+struct ItemParts {
+  int per, count;
+  __device__ __forceinline__ ItemParts(const FwdParams &p, int nvis) {
+    const int even = (nvis + p.max_parts - 1) / p.max_parts;
+    per = even > p.min_blocks ? even : p.min_blocks;
+    count = (nvis + per - 1) / per;
+    if (count < 1) count = 1;
+  }
+};
+
+// Partial results travel between workgroups (and the chip's eight dies) with accesses of agent scope, which bypass the
+// caches that are not shared: a store has reached the common memory once its wavefront has waited for it.
+__device__ __forceinline__ void part_store(float *at, float v) {
+  __hip_atomic_store((uint32_t *)at, __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float part_load(const float *at) {
+  return __builtin_bit_cast(float, __hip_atomic_load((const uint32_t *)at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
 
 // Keeps the message hbsa_last_error() returns and gives back `code` (defined in hbsa_fwd.hip).
 int fail(int code, const char *fmt, ...);

@@ -390,6 +390,34 @@ inline size_t split_bytes(int parts, int total_q, int nhead_q, int nhead_k, int 
          align_up((size_t)parts * total_q * nhead_q * 4, 256);
 }
 
+int device_cus() {
+  static thread_local int cus_of[kMaxDevices] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  if (cus_of[dev] == 0 && hipDeviceGetAttribute(&cus_of[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus_of[dev] = 0;
+  return cus_of[dev];
+}
+
+// Parts an item of the fp32 kernel may be cut into, kPartKeys keys each at least.  With up to two items per CU (all resident
+// at once, the longest several times the average) enough parts for eight per CU, no more than all k blocks can fill, 32,
+// and kMaxPartBytes of partial results.  Measured, 4 sequences of 1279 .. 2697 tokens, 8 / 4 heads, keep 0.5: whole items
+// 153 us, parts of at least 512 / 256 / 128 keys 158 / 121 / 117 us at D = 64; 87 / 86 / 67 / 63 us at D = 32.
+constexpr int kPartKeys = 128;
+constexpr size_t kMaxPartBytes = 96ull << 20;
+inline size_t f32_part_bytes(int headdim) { return (size_t)4 * (headdim / 2 + 2) * 64 * sizeof(float); }   // of one part
+int f32_max_parts(long long items, int headdim, int num_k_block) {
+  const int cus = device_cus();
+  if (items <= 0 || items > 2ll * cus || items > kMaxPartItems) return 1;
+  long long parts = std::min<long long>(32, 8ll * cus / items);
+  parts = std::min<long long>(parts, num_k_block);
+  parts = std::min<long long>(parts, (long long)(kMaxPartBytes / (f32_part_bytes(headdim) * (size_t)items)));
+  return parts < 2 ? 1 : (int)parts;
+}
+inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_block_size) {
+  const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, true);
+  return (long long)nhead_k * num_q_block * ((slots + 3) / 4);
+}
+
 // The fields of FwdParams that follow from the call's shape and softmax_scale alone.
 void fill_shape(FwdParams &fp, int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size,
                 int k_block_size, int causal, float softmax_scale, bool f32_exact, bool may_pack = false, bool cols = false) {
@@ -397,12 +425,20 @@ void fill_shape(FwdParams &fp, int nhead_q, int nhead_k, int headdim, int num_q_
   fp.nqb = num_q_block; fp.ratio = nhead_q / nhead_k; fp.kbs = k_block_size; fp.wpr = words_per_row(num_k_block);
   fp.causal = causal ? 1 : 0;
   fp.wps = (q_block_size + kWaveRows - 1) / kWaveRows;
-  fp.pack = cols || (may_pack && fwd_packs(fp.ratio, q_block_size)) ? 1 : 0;
+  fp.pack = cols || f32_exact || (may_pack && fwd_packs(fp.ratio, q_block_size)) ? 1 : 0;
   const int slots = fwd_slots(fp.ratio, q_block_size, fp.pack != 0);
   fp.nw = cols ? 4 : fwd_wavefronts(slots, headdim, f32_exact);
   fp.ncol = headdim / 8;
+  fp.max_parts = 1;
+  fp.min_blocks = 1;
+  fp.parts = nullptr;
+  fp.arrivals = nullptr;
+  fp.parts_last = 0;
+  fp.nparts = 1;
+  fp.div_nparts = make_fast_div(1u);
   fp.nsub = (slots + fp.nw - 1) / fp.nw;
   fp.div_nsub = make_fast_div((uint32_t)fp.nsub);
+  fp.div_items = make_fast_div((uint32_t)(nhead_k * num_q_block * fp.nsub));
   fp.div_nqb = make_fast_div((uint32_t)num_q_block);
   fp.div_nhk = make_fast_div((uint32_t)nhead_k);
   fp.div_kbs = make_fast_div((uint32_t)k_block_size);
@@ -461,6 +497,8 @@ int run_fwd(FwdParams &fp, long long items, hipStream_t stream, char *split_area
 static __device__ __align__(256) unsigned char scratch[HBSA_STATIC_SCRATCH_BYTES];
 constexpr int kStreamSlots = 64;
 static __device__ __align__(256) unsigned char stream_sched[kStreamSlots * sizeof(hbsa::Sched)];
+// stream_arrivals: the counters of launches whose items are cut into parts (ItemParts), likewise one set per stream.
+static __device__ __align__(256) uint32_t stream_arrivals[kStreamSlots * hbsa::kMaxPartItems];
 namespace hbsa {
 std::mutex g_scratch_mutex;
 void *g_scratch_ptr[kMaxDevices] = {};
@@ -481,26 +519,29 @@ int static_scratch(void **ptr) {
   return 0;
 }
 
-// The launch record of `stream` on the current device, nullptr when there is none to give (no device, the
-// lookup failed, or kStreamSlots other streams of this device have taken the records).
+// The launch record and the arrival counters of `stream` on the current device; nullptr when there are none to give (no
+// device, the lookup failed, or kStreamSlots other streams of this device have taken them).
 struct StreamSlots {
   char *base;
+  uint32_t *arrivals;
   int used;
   hipStream_t stream[kStreamSlots];
 };
 StreamSlots g_stream_slots[kMaxDevices] = {};
-Sched *stream_sched_of(hipStream_t stream) {
+Sched *stream_sched_of(hipStream_t stream, uint32_t **arrivals = nullptr) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
   StreamSlots &t = g_stream_slots[dev];
   if (t.base == nullptr) {
-    void *p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(stream_sched)) != hipSuccess || p == nullptr) {
+    void *p = nullptr, *a = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(stream_sched)) != hipSuccess || p == nullptr ||
+        hipGetSymbolAddress(&a, HIP_SYMBOL(stream_arrivals)) != hipSuccess || a == nullptr) {
       (void)hipGetLastError();
       return nullptr;
     }
     t.base = (char *)p;
+    t.arrivals = (uint32_t *)a;
   }
   int i = 0;
   while (i < t.used && t.stream[i] != stream) ++i;
@@ -508,7 +549,16 @@ Sched *stream_sched_of(hipStream_t stream) {
     if (t.used == kStreamSlots) return nullptr;
     t.stream[t.used++] = stream;
   }
+  if (arrivals != nullptr) *arrivals = t.arrivals + (size_t)i * kMaxPartItems;
   return (Sched *)(t.base + (size_t)i * sizeof(Sched));
+}
+bool is_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return capturing != hipStreamCaptureStatusNone;
 }
 
 // The one-launch form of the forward is used when it applies (see hbsa_set_onepass in the header).
@@ -525,13 +575,7 @@ Sched *onepass_record(int32_t dtype, int32_t batch, int32_t total_k, int32_t hea
   if (items <= 0 || items > 0x7fffffffLL) return nullptr;
   if (split_parts(items, num_k_block) > 1) return nullptr;
   if (!g_deterministic && k_block_size % kTileKeys == 0 && 2ll * total_k * headdim * 2 >= g_walk_min_bytes) return nullptr;
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  if (capturing != hipStreamCaptureStatusNone) return nullptr;
-  return stream_sched_of(st);
+  return is_capturing(st) ? nullptr : stream_sched_of(st);
 }
 
 constexpr int kNotOnePass = 0x7fffffff;   // try_onepass: the call has to take the two-launch path
@@ -580,6 +624,25 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
     case 64: return bf ? launch_fwd_fused<64, ElemBF16>(fp, items, st) : launch_fwd_fused<64, ElemF16>(fp, items, st);
     case 128: return bf ? launch_fwd_fused<128, ElemBF16>(fp, items, st) : launch_fwd_fused<128, ElemF16>(fp, items, st);
     default: return bf ? launch_fwd_fused<256, ElemBF16>(fp, items, st) : launch_fwd_fused<256, ElemF16>(fp, items, st);
+  }
+}
+
+// The fp32 kernel on a filled-in parameter block, with `room` bytes at `area` for partial results.
+int run_f32(FwdParams &fp, float softmax_scale, int headdim, int num_k_block, long long items, char *area, size_t room, hipStream_t st) {
+  const int parts = std::min(f32_max_parts(items, headdim, num_k_block), (int)std::min<size_t>(32, room / (f32_part_bytes(headdim) * (size_t)items)));
+  if (parts > 1 && !is_capturing(st) && stream_sched_of(st, &fp.arrivals) != nullptr) {
+    fp.max_parts = parts;
+    fp.min_blocks = std::max(1, kPartKeys / fp.kbs);
+    fp.parts = (float *)area;
+    fp.parts_last = items * parts < 4ll * device_cus();
+    fp.div_nparts = make_fast_div((uint32_t)parts);
+  }
+  const float c_signed = softmax_scale * kLog2e;
+  switch (headdim) {
+    case 32: return launch_fwd_f32<32>(fp, c_signed, items, st);
+    case 64: return launch_fwd_f32<64>(fp, c_signed, items, st);
+    case 128: return launch_fwd_f32<128>(fp, c_signed, items, st);
+    default: return launch_fwd_f32<256>(fp, c_signed, items, st);
   }
 }
 }  // namespace hbsa
@@ -688,14 +751,25 @@ size_t hbsa_fwd_workspace_bytes_dtype(int32_t dtype, int32_t total_q, int32_t to
   return n;
 }
 
-size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim,
-                                      int32_t num_q_block, int32_t num_k_block, int32_t q_block_size) {
-  if (total_q <= 0 || nhead_q <= 0 || nhead_k <= 0 || headdim <= 0 || num_q_block <= 0 || num_k_block <= 0 || q_block_size <= 0)
-    return 0;
+size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block,
+                            int32_t num_k_block, int32_t q_block_size) {
+  if (total_q <= 0 || nhead_q <= 0 || nhead_k <= 0 || headdim <= 0 || num_q_block <= 0 || num_k_block <= 0 || q_block_size <= 0) return 0;
+  if (dtype == HBSA_DTYPE_F32) {
+    const long long items = f32_items(nhead_q, nhead_k, num_q_block, q_block_size);
+    const int parts = f32_max_parts(items, headdim, num_k_block);
+    return parts < 2 ? 0 : (size_t)items * parts * f32_part_bytes(headdim);
+  }
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, false);
   const int nw = fwd_wavefronts(slots, headdim, false);
   const long long items = (long long)nhead_k * num_q_block * ((slots + nw - 1) / nw);
   return split_bytes(split_parts(items, num_k_block), total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
+}
+
+size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim,
+                                      int32_t num_q_block, int32_t num_k_block, int32_t q_block_size) {
+  const size_t b16 = hbsa_fwd_parts_bytes(HBSA_DTYPE_BF16, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size);
+  const size_t f32 = hbsa_fwd_parts_bytes(HBSA_DTYPE_F32, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size);
+  return b16 > f32 ? b16 : f32;
 }
 
 int hbsa_fwd_prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
@@ -782,6 +856,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
 
   hipStream_t st = (hipStream_t)stream;
   FwdParams fp;
+  std::memset(&fp, 0, sizeof(fp));
   fp.q = (const char *)q; fp.k = (const char *)k; fp.v = (const char *)v; fp.out = (char *)out;
   fp.info = (const QBlockInfo *)workspace;
   fp.bits = (const uint32_t *)((const char *)workspace + bits_offset(nhead_k, num_q_block));
@@ -832,15 +907,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
   fp.walk = (!g_deterministic && fp.nparts == 1 && k_block_size % kTileKeys == 0 &&
              2ll * total_k * headdim * 2 >= g_walk_min_bytes) ? 1 : 0;
 
-  if (f32_exact) {
-    const float c_signed = softmax_scale * kLog2e;
-    switch (headdim) {
-      case 32: return launch_fwd_f32<32>(fp, c_signed, items, st);
-      case 64: return launch_fwd_f32<64>(fp, c_signed, items, st);
-      case 128: return launch_fwd_f32<128>(fp, c_signed, items, st);
-      default: return launch_fwd_f32<256>(fp, c_signed, items, st);
-    }
-  }
+  if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, split_area, workspace_bytes - need, st);
   if (f32) {
     // setup (multipliers from the maxima), staging, attention: the launch order on the stream is the
     // dependency order
@@ -912,11 +979,24 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
     if (one != kNotOnePass) return one;
   }
   if (any_dim) return fail(HBSA_ERR_WORKSPACE_TOO_SMALL, "the call is not one launch: use hbsa_fwd with a workspace");
-  {
-    const size_t need = hbsa_fwd_workspace_bytes_dtype(dtype, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block,
-                                                       num_k_block);
-    if (!workspace || workspace_bytes < need)
-      return fail(HBSA_ERR_WORKSPACE_TOO_SMALL, "workspace %zu bytes < required %zu", workspace ? workspace_bytes : (size_t)0, need);
+  const size_t need = hbsa_fwd_workspace_bytes_dtype(dtype, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
+  if (!workspace || workspace_bytes < need)
+    return fail(HBSA_ERR_WORKSPACE_TOO_SMALL, "workspace %zu bytes < required %zu", workspace ? workspace_bytes : (size_t)0, need);
+  if (dtype == HBSA_DTYPE_F32 && allow_onepass) {   // the fp32 kernel reads boundaries and mask itself: no pre-pass
+    if ((uintptr_t)workspace & 255) return fail(HBSA_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");
+    FwdParams fp;
+    std::memset(&fp, 0, sizeof(fp));
+    fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, true);
+    const long long items = (long long)nhead_k * num_q_block * fp.nsub;
+    if (items > 0x7fffffffLL) return fail(HBSA_ERR_UNSUPPORTED, "too many work items (%lld)", items);
+    fp.q = (const char *)q; fp.k = (const char *)k; fp.v = (const char *)v; fp.out = (char *)out;
+    fp.q_s = strides[0] * 4; fp.q_h = strides[1] * 4; fp.k_s = strides[2] * 4; fp.k_h = strides[3] * 4;
+    fp.v_s = strides[4] * 4; fp.v_h = strides[5] * 4; fp.o_s = strides[6] * 4; fp.o_h = strides[7] * 4;
+    fp.total_q = total_q; fp.nhead_q = nhead_q;
+    fp.cu_q = cu_q_seqlens; fp.cu_k = cu_k_seqlens; fp.cu_nqb = cu_num_q_block; fp.cu_nkb = cu_num_k_block;
+    fp.mask = block_mask; fp.ms_h = strides[8]; fp.ms_q = strides[9]; fp.ms_k = strides[10];
+    fp.batch = batch; fp.nkb_total = num_k_block; fp.total_k = total_k; fp.qbs = q_block_size;
+    return run_f32(fp, softmax_scale, headdim, num_k_block, items, (char *)workspace, workspace_bytes, (hipStream_t)stream);
   }
   int rc = hbsa_fwd_prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block,
                             workspace, workspace_bytes, batch, nhead_k, num_q_block, num_k_block, q_block_size,

@@ -116,7 +116,7 @@ bool rows_ok(const at::Tensor &t) {
 size_t workspace_bytes(const Problem &p) {
   return hbsa_fwd_workspace_bytes_dtype(p.dtype, (int)p.q.size(0), (int)p.k.size(0), (int)p.q.size(1), (int)p.k.size(1),
                                         (int)p.q.size(2), (int)p.nqb, (int)p.nkb) +
-         hbsa_fwd_split_workspace_bytes((int)p.q.size(0), (int)p.q.size(1), (int)p.k.size(1), (int)p.q.size(2), (int)p.nqb,
+         hbsa_fwd_parts_bytes(p.dtype, (int)p.q.size(0), (int)p.q.size(1), (int)p.k.size(1), (int)p.q.size(2), (int)p.nqb,
                                         (int)p.nkb, (int)p.qbs);
 }
 

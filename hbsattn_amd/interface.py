@@ -136,8 +136,8 @@ def _run_workspace_bytes(lib, device, code, total_q, total_k, nhead_q, nhead_k, 
         need = int(lib.hbsa_fwd_workspace_bytes_dtype(code, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block,
                                                       num_k_block))
         with torch.cuda.device(device):
-            need += int(lib.hbsa_fwd_split_workspace_bytes(total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block,
-                                                           q_block_size))
+            need += int(lib.hbsa_fwd_parts_bytes(code, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block,
+                                                 q_block_size))
         if len(_ws_bytes_cache) > 4096:
             _ws_bytes_cache.clear()
         _ws_bytes_cache[key] = need

@@ -70,7 +70,8 @@ int hbsa_set_deterministic(int on);
 int hbsa_set_onepass(int on);   /* see hbsa_fwd */
 
 /* Launches an hbsa_fwd call with these sizes would make on `stream` right now: 1 when its one-launch form
- * applies (the call then needs no workspace), else 2 (pre-pass and attention kernel; more for
+ * applies (the call then needs no workspace), else 2 (pre-pass and attention kernel; for HBSA_DTYPE_F32 the
+ * attention kernel alone, on a workspace; more for
  * HBSA_DTYPE_F32_STAGED16 and for work split over key blocks).  Host-side only, nothing is launched. */
 int hbsa_fwd_launches(int32_t dtype, int32_t batch, int32_t total_k, int32_t nhead_q, int32_t nhead_k,
                       int32_t headdim, int32_t num_q_block, int32_t num_k_block,
@@ -152,6 +153,12 @@ size_t hbsa_fwd_workspace_bytes_dtype(int32_t dtype, int32_t total_q, int32_t to
  */
 size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim,
                                       int32_t num_q_block, int32_t num_k_block, int32_t q_block_size);
+
+/*
+ * The same for a given element type (hbsa_fwd_split_workspace_bytes is the most any type can use).
+ */
+size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim,
+                            int32_t num_q_block, int32_t num_k_block, int32_t q_block_size);
 
 /*
  * Block-sparse attention forward.  Replaces `_forward_auto_tile_size` and
