@@ -39,6 +39,7 @@ constexpr int kWalkReportTiles = 8;   // an item adds its progress to its walk c
 constexpr float kLog2e = 1.4426950408889634f;
 // One-launch form: sequences whose boundaries the scheduler keeps in LDS (batch + 1 entries of four arrays)
 constexpr int kSeqCap = 128;
+constexpr int kDecodeMaxParts = 32;    // parts of an item of the decode kernel
 constexpr int kMaxPartItems = 4096;   // items of a launch that may be cut into parts (its arrival counters)
 constexpr int kMaxDevices = 64;            // devices of one process the launch caches cover
 constexpr float kLazyRescaleLog2 = 8.0f;  // running max may lag the true max by 2^8
@@ -392,14 +393,19 @@ struct ItemParts {
   }
 };
 
-// Partial results travel between workgroups (and the chip's eight dies) with accesses of agent scope, which bypass the
-// caches that are not shared: a store has reached the common memory once its wavefront has waited for it.
+// Partial results travel between workgroups, and so between the chip's eight dies, whose L2 caches know nothing of each
+// other.  They are stored through to the memory all dies share (agent scope, as an atomic store of that scope is done): such
+// a store has arrived once its wavefront has waited for it.  The workgroup that combines them first drops what its own
+// caches hold (an acquire of that scope) and may then load plainly, many at a time: with loads of agent scope, each waited
+// for by itself, combining 32 parts took longer (50 us) than everything before it.
 __device__ __forceinline__ void part_store(float *at, float v) {
   __hip_atomic_store((uint32_t *)at, __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ float part_load(const float *at) {
-  return __builtin_bit_cast(float, __hip_atomic_load((const uint32_t *)at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+__device__ __forceinline__ void part_store4(float *at, f32x4 v) {   // 16-byte aligned
+  asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(at), "v"(v) : "memory");
 }
+__device__ __forceinline__ void parts_arrived() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
+__device__ __forceinline__ void parts_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 
 // Keeps the message hbsa_last_error() returns and gives back `code` (defined in hbsa_fwd.hip).
 int fail(int code, const char *fmt, ...);
@@ -411,6 +417,8 @@ template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
+int launch_fwd_decode(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D>
 int launch_fwd_f32(const FwdParams &fp, float c_signed, long long items, hipStream_t stream);
 template <int D, typename E>

@@ -398,8 +398,10 @@ int device_cus() {
   return cus_of[dev];
 }
 
+// An odd number of parts (see decode_max_parts for why)
+inline int odd_parts(long long parts) { return parts < 2 ? 1 : parts % 2 ? (int)parts : (int)parts - 1; }
 // Parts an item of the fp32 kernel may be cut into, kPartKeys keys each at least.  With up to two items per CU (all resident
-// at once, the longest several times the average) enough parts for eight per CU, no more than all k blocks can fill, 32,
+// at once, the longest several times the average) enough parts for nine per CU, no more than all k blocks can fill, 32,
 // and kMaxPartBytes of partial results.  Measured, 4 sequences of 1279 .. 2697 tokens, 8 / 4 heads, keep 0.5: whole items
 // 153 us, parts of at least 512 / 256 / 128 keys 158 / 121 / 117 us at D = 64; 87 / 86 / 67 / 63 us at D = 32.
 constexpr int kPartKeys = 128;
@@ -408,10 +410,32 @@ inline size_t f32_part_bytes(int headdim) { return (size_t)4 * (headdim / 2 + 2)
 int f32_max_parts(long long items, int headdim, int num_k_block) {
   const int cus = device_cus();
   if (items <= 0 || items > 2ll * cus || items > kMaxPartItems) return 1;
-  long long parts = std::min<long long>(32, 8ll * cus / items);
+  long long parts = std::min<long long>(32, 9ll * cus / items);
   parts = std::min<long long>(parts, num_k_block);
   parts = std::min<long long>(parts, (long long)(kMaxPartBytes / (f32_part_bytes(headdim) * (size_t)items)));
-  return parts < 2 ? 1 : (int)parts;
+  return odd_parts(parts);
+}
+// ---- The decode kernel (hbsa_fwd_decode.h): at most 16 (q head, row) entries per kv head and q block on average, so that
+// the 32-query slots and four-wavefront workgroups of the other kernel would be mostly empty.
+inline bool decode_shape(int32_t dtype, int nhead_q, int nhead_k, int num_q_block, int total_q) {
+  return (dtype == HBSA_DTYPE_BF16 || dtype == HBSA_DTYPE_F16) && (long long)(nhead_q / nhead_k) * total_q <= 16ll * num_q_block;
+}
+inline size_t decode_part_bytes(int total_q, int nhead_q, int headdim) { return (size_t)total_q * nhead_q * (headdim + 2) * sizeof(float); }
+// Parts of about the same size for all items, kDecodePartKeys keys each at least, twelve per CU in all; an item of more than
+// two and a half times the mean length gets longer ones.  Measured at 32 x 2000 .. 32000 keys, 32 / 8 heads of 128, keep
+// 0.25: 8, 10, 12, 14 per CU 126-131, 126, 126-128, 127 us; 64 x 10000 .. 40000 keys, 32 heads 1530, 1450, 1417, 1520 us.
+// The number of parts is odd: workgroups go to the eight dies by their number, and with an even number of parts the
+// later parts, which short items do not have, would all meet on the same dies (with 32 in place of 30 168 and 2045 us).
+constexpr int kDecodePartKeys = 256;
+int decode_part_blocks(int nhead_k, int num_k_block, int k_block_size) {
+  const long long target = std::max(1, 12 * device_cus());
+  const long long even = ((long long)nhead_k * num_k_block + target - 1) / target;
+  return (int)std::max<long long>(even, std::max(1, kDecodePartKeys / k_block_size));
+}
+int decode_max_parts(long long items, int num_k_block) {
+  if (items <= 0 || items > kMaxPartItems) return 1;
+  long long parts = std::min<long long>(kDecodeMaxParts, 30ll * device_cus() / items);
+  return odd_parts(std::min<long long>(parts, num_k_block));
 }
 inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_block_size) {
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, true);
@@ -627,22 +651,63 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   }
 }
 
+__global__ void hbsa_zero_kernel(uint32_t *x, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) x[i] = 0u;
+}
+
+// Sets up `fp` for up to `parts` parts per item of `part_bytes` bytes of partial results each, with `room` bytes at `area`.  The
+// arrival counters are the stream's own; a captured launch may be replayed on any stream, and more streams than there are
+// sets of counters may be in use: then they lie behind the partial results and are cleared by a launch of their own.
+int set_parts(FwdParams &fp, int parts, int min_keys, size_t part_bytes, long long items, char *area, size_t room, hipStream_t st) {
+  const size_t counters = align_up((size_t)items * sizeof(uint32_t), 256);
+  if (parts < 2 || area == nullptr || room <= counters) return 0;
+  parts = odd_parts(std::min<long long>(parts, (long long)((room - counters) / part_bytes)));
+  if (parts < 2) return 0;
+  if (is_capturing(st) || stream_sched_of(st, &fp.arrivals) == nullptr) {
+    fp.arrivals = (uint32_t *)(area + align_up(part_bytes * parts, 256));
+    if ((char *)fp.arrivals + counters > area + room) return 0;
+    hipLaunchKernelGGL(hbsa_zero_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, fp.arrivals, (int)items);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail((int)e, "hbsa_zero_kernel launch: %s", hipGetErrorString(e));
+  }
+  fp.max_parts = parts;
+  fp.min_blocks = std::max(1, min_keys / fp.kbs);
+  fp.parts = (float *)area;
+  fp.parts_last = items * parts < 4ll * device_cus();
+  fp.div_nparts = make_fast_div((uint32_t)parts);
+  return 0;
+}
+inline size_t parts_room(int parts, size_t part_bytes, long long items) {
+  return parts < 2 ? 0 : align_up(part_bytes * parts, 256) + align_up((size_t)items * sizeof(uint32_t), 256);
+}
+
 // The fp32 kernel on a filled-in parameter block, with `room` bytes at `area` for partial results.
 int run_f32(FwdParams &fp, float softmax_scale, int headdim, int num_k_block, long long items, char *area, size_t room, hipStream_t st) {
-  const int parts = std::min(f32_max_parts(items, headdim, num_k_block), (int)std::min<size_t>(32, room / (f32_part_bytes(headdim) * (size_t)items)));
-  if (parts > 1 && !is_capturing(st) && stream_sched_of(st, &fp.arrivals) != nullptr) {
-    fp.max_parts = parts;
-    fp.min_blocks = std::max(1, kPartKeys / fp.kbs);
-    fp.parts = (float *)area;
-    fp.parts_last = items * parts < 4ll * device_cus();
-    fp.div_nparts = make_fast_div((uint32_t)parts);
-  }
+  if (int rc = set_parts(fp, f32_max_parts(items, headdim, num_k_block), kPartKeys, f32_part_bytes(headdim) * (size_t)items, items, area, room, st))
+    return rc;
   const float c_signed = softmax_scale * kLog2e;
   switch (headdim) {
     case 32: return launch_fwd_f32<32>(fp, c_signed, items, st);
     case 64: return launch_fwd_f32<64>(fp, c_signed, items, st);
     case 128: return launch_fwd_f32<128>(fp, c_signed, items, st);
     default: return launch_fwd_f32<256>(fp, c_signed, items, st);
+  }
+}
+
+// The decode kernel likewise.
+int run_decode(FwdParams &fp, bool bf, int headdim, int num_k_block, char *area, size_t room, hipStream_t st) {
+  const long long items = (long long)fp.nhead_k * fp.nqb;
+  fp.div_items = make_fast_div((uint32_t)items);
+  fp.div_nparts = make_fast_div(1u);
+  if (int rc = set_parts(fp, decode_max_parts(items, num_k_block), decode_part_blocks(fp.nhead_k, num_k_block, fp.kbs) * fp.kbs, decode_part_bytes(fp.total_q, fp.nhead_q, headdim), items,
+                         area, room, st))
+    return rc;
+  switch (headdim) {
+    case 32: return bf ? launch_fwd_decode<32, ElemBF16>(fp, items, st) : launch_fwd_decode<32, ElemF16>(fp, items, st);
+    case 64: return bf ? launch_fwd_decode<64, ElemBF16>(fp, items, st) : launch_fwd_decode<64, ElemF16>(fp, items, st);
+    case 128: return bf ? launch_fwd_decode<128, ElemBF16>(fp, items, st) : launch_fwd_decode<128, ElemF16>(fp, items, st);
+    default: return bf ? launch_fwd_decode<256, ElemBF16>(fp, items, st) : launch_fwd_decode<256, ElemF16>(fp, items, st);
   }
 }
 }  // namespace hbsa
@@ -756,8 +821,11 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
   if (total_q <= 0 || nhead_q <= 0 || nhead_k <= 0 || headdim <= 0 || num_q_block <= 0 || num_k_block <= 0 || q_block_size <= 0) return 0;
   if (dtype == HBSA_DTYPE_F32) {
     const long long items = f32_items(nhead_q, nhead_k, num_q_block, q_block_size);
-    const int parts = f32_max_parts(items, headdim, num_k_block);
-    return parts < 2 ? 0 : (size_t)items * parts * f32_part_bytes(headdim);
+    return parts_room(f32_max_parts(items, headdim, num_k_block), f32_part_bytes(headdim) * (size_t)items, items);
+  }
+  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q)) {
+    const long long items = (long long)nhead_k * num_q_block;
+    return parts_room(decode_max_parts(items, num_k_block), decode_part_bytes(total_q, nhead_q, headdim), items);
   }
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, false);
   const int nw = fwd_wavefronts(slots, headdim, false);
@@ -907,6 +975,8 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
   fp.walk = (!g_deterministic && fp.nparts == 1 && k_block_size % kTileKeys == 0 &&
              2ll * total_k * headdim * 2 >= g_walk_min_bytes) ? 1 : 0;
 
+  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q))
+    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, split_area, workspace_bytes - need, st);
   if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, split_area, workspace_bytes - need, st);
   if (f32) {
     // setup (multipliers from the maxima), staging, attention: the launch order on the stream is the
@@ -972,7 +1042,10 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
                 q_block_size, k_block_size);
   if (num_k_block <= 0 || total_k <= 0) return fail(HBSA_ERR_INVALID_ARGUMENT, "no keys");
   if (nhead_k > 65535) return fail(HBSA_ERR_UNSUPPORTED, "nhead_k %d > 65535", nhead_k);
-  if (allow_onepass) {
+  const bool f32_exact = dtype == HBSA_DTYPE_F32;
+  const bool decode = !any_dim && decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q);
+  const bool direct = allow_onepass && g_onepass && (f32_exact || decode);   // a kernel that reads boundaries and mask itself
+  if (allow_onepass && !direct) {
     const int one = try_onepass(q, k, v, out, cu_q_seqlens, cu_k_seqlens, block_mask, cu_num_q_block, cu_num_k_block, dtype,
                                 batch, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size,
                                 k_block_size, causal, softmax_scale, strides, (hipStream_t)stream);
@@ -980,23 +1053,29 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   }
   if (any_dim) return fail(HBSA_ERR_WORKSPACE_TOO_SMALL, "the call is not one launch: use hbsa_fwd with a workspace");
   const size_t need = hbsa_fwd_workspace_bytes_dtype(dtype, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
-  if (!workspace || workspace_bytes < need)
+  const bool roomy = workspace != nullptr && workspace_bytes >= need;
+  if (!roomy && !(direct && decode))   // (the decode kernel needs none; without one its items stay whole)
     return fail(HBSA_ERR_WORKSPACE_TOO_SMALL, "workspace %zu bytes < required %zu", workspace ? workspace_bytes : (size_t)0, need);
-  if (dtype == HBSA_DTYPE_F32 && allow_onepass) {   // the fp32 kernel reads boundaries and mask itself: no pre-pass
-    if ((uintptr_t)workspace & 255) return fail(HBSA_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");
+  if (direct) {
+    if (roomy && ((uintptr_t)workspace & 255)) return fail(HBSA_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");
     FwdParams fp;
     std::memset(&fp, 0, sizeof(fp));
-    fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, true);
+    fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
     const long long items = (long long)nhead_k * num_q_block * fp.nsub;
     if (items > 0x7fffffffLL) return fail(HBSA_ERR_UNSUPPORTED, "too many work items (%lld)", items);
+    const int64_t es = f32_exact ? 4 : 2;
     fp.q = (const char *)q; fp.k = (const char *)k; fp.v = (const char *)v; fp.out = (char *)out;
-    fp.q_s = strides[0] * 4; fp.q_h = strides[1] * 4; fp.k_s = strides[2] * 4; fp.k_h = strides[3] * 4;
-    fp.v_s = strides[4] * 4; fp.v_h = strides[5] * 4; fp.o_s = strides[6] * 4; fp.o_h = strides[7] * 4;
+    fp.q_s = strides[0] * es; fp.q_h = strides[1] * es; fp.k_s = strides[2] * es; fp.k_h = strides[3] * es;
+    fp.v_s = strides[4] * es; fp.v_h = strides[5] * es; fp.o_s = strides[6] * es; fp.o_h = strides[7] * es;
     fp.total_q = total_q; fp.nhead_q = nhead_q;
     fp.cu_q = cu_q_seqlens; fp.cu_k = cu_k_seqlens; fp.cu_nqb = cu_num_q_block; fp.cu_nkb = cu_num_k_block;
     fp.mask = block_mask; fp.ms_h = strides[8]; fp.ms_q = strides[9]; fp.ms_k = strides[10];
     fp.batch = batch; fp.nkb_total = num_k_block; fp.total_k = total_k; fp.qbs = q_block_size;
-    return run_f32(fp, softmax_scale, headdim, num_k_block, items, (char *)workspace, workspace_bytes, (hipStream_t)stream);
+    // (behind the work description, as in the prepared form: both forms then have the same room and make the same parts)
+    char *area = roomy ? (char *)workspace + need : nullptr;
+    const size_t room = roomy ? workspace_bytes - need : 0;
+    if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, area, room, (hipStream_t)stream);
+    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, area, room, (hipStream_t)stream);
   }
   int rc = hbsa_fwd_prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block,
                             workspace, workspace_bytes, batch, nhead_k, num_q_block, num_k_block, q_block_size,

@@ -289,7 +289,7 @@ __global__ __launch_bounds__(kThreads, F32Tile<D>::WG_PER_CU) void hbsa_fwd_f32_
       part_store(mine + DT * 16 * 64, m_run);
       part_store(mine + (DT * 16 + 1) * 64, l_tot);
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): ... it has reached memory
+    parts_arrived();
     __syncthreads();
     if (threadIdx.x == 0) {
       const uint32_t before = __hip_atomic_fetch_add(p.arrivals + item, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -298,24 +298,27 @@ __global__ __launch_bounds__(kThreads, F32Tile<D>::WG_PER_CU) void hbsa_fwd_f32_
     }
     __syncthreads();
     if (!last_flag) return;
+    parts_acquire();
     if (active && l32 < n) {
       const float *all = p.parts + ((size_t)item * p.max_parts * 4 + wave) * stride + lane;
       float m_all = -INFINITY;
-      for (int pt = 0; pt < parts.count; ++pt) m_all = fmaxf(m_all, part_load(all + (size_t)pt * 4 * stride + DT * 16 * 64));
+#pragma unroll 8
+      for (int pt = 0; pt < parts.count; ++pt) m_all = fmaxf(m_all, all[(size_t)pt * 4 * stride + DT * 16 * 64]);
       const float m_ref = m_all == -INFINITY ? 0.f : m_all;
       l_tot = 0.f;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+#pragma unroll 2
       for (int pt = 0; pt < parts.count; ++pt) {
         const float *q = all + (size_t)pt * 4 * stride;
-        const float f = __builtin_amdgcn_exp2f(part_load(q + DT * 16 * 64) - m_ref);
-        l_tot += f * part_load(q + (DT * 16 + 1) * 64);
+        const float f = __builtin_amdgcn_exp2f(q[DT * 16 * 64] - m_ref);
+        l_tot += f * q[(DT * 16 + 1) * 64];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) o[dt][i] += f * part_load(q + (dt * 16 + i) * 64);
+          for (int i = 0; i < 16; ++i) o[dt][i] += f * q[(dt * 16 + i) * 64];
       }
       m_run = m_all;
     }

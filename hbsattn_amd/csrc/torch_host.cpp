@@ -113,11 +113,14 @@ bool rows_ok(const at::Tensor &t) {
   __builtin_unreachable();
 }
 
+// Room for partial results of work that is cut over its key blocks (0: it is not), and the whole workspace
+size_t parts_bytes(const Problem &p) {
+  return hbsa_fwd_parts_bytes(p.dtype, (int)p.q.size(0), (int)p.q.size(1), (int)p.k.size(1), (int)p.q.size(2), (int)p.nqb, (int)p.nkb,
+                              (int)p.qbs);
+}
 size_t workspace_bytes(const Problem &p) {
   return hbsa_fwd_workspace_bytes_dtype(p.dtype, (int)p.q.size(0), (int)p.k.size(0), (int)p.q.size(1), (int)p.k.size(1),
-                                        (int)p.q.size(2), (int)p.nqb, (int)p.nkb) +
-         hbsa_fwd_parts_bytes(p.dtype, (int)p.q.size(0), (int)p.q.size(1), (int)p.k.size(1), (int)p.q.size(2), (int)p.nqb,
-                                        (int)p.nkb, (int)p.qbs);
+                                        (int)p.q.size(2), (int)p.nqb, (int)p.nkb) + parts_bytes(p);
 }
 
 at::Tensor bytes_like(const at::Tensor &t, size_t n) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
@@ -142,8 +145,9 @@ at::Tensor plain_forward(const Problem &p, hipStream_t stream) {
     if (rc != 0) raise("hbsa_fwd_one", rc);
     return out;
   }
-  int rc = hbsa_fwd_v(ptrs, 0, sizes, (float)p.scale, strides, stream);
-  if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) {   // nothing was launched: this call is no single launch
+  int rc = HBSA_ERR_WORKSPACE_TOO_SMALL;
+  if (p.dtype < HBSA_DTYPE_F32 && parts_bytes(p) == 0) rc = hbsa_fwd_v(ptrs, 0, sizes, (float)p.scale, strides, stream);
+  if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) {   // nothing was launched: this call needs a workspace
     const size_t n = workspace_bytes(p);
     at::Tensor ws = bytes_like(p.q, n);
     ptrs[10] = ws.mutable_data_ptr();
