@@ -86,6 +86,8 @@ def load() -> ctypes.CDLL:
     lib.hbsa_block_arrays.argtypes = [vp, vp, i32, i32, i32, vp, vp, vp]
     lib.hbsa_bwd_workspace_bytes.restype = ctypes.c_size_t
     lib.hbsa_bwd_workspace_bytes.argtypes = [ctypes.c_int32] * 2
+    lib.hbsa_bwd_workspace_bytes_parts.restype = ctypes.c_size_t
+    lib.hbsa_bwd_workspace_bytes_parts.argtypes = [ctypes.c_int32] * 8
     lib.hbsa_bwd.restype = ctypes.c_int
     lib.hbsa_bwd.argtypes = ([vp] * 13 + [ctypes.c_size_t, vp, ctypes.c_size_t] + [ctypes.c_int32] * 12
                              + [ctypes.c_float, i64p, vp])

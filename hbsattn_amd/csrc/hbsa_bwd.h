@@ -218,8 +218,92 @@ __device__ __forceinline__ bool bwd_sequence_skipped(const BwdParams &p, int b, 
   return true;
 }
 
+// ---- Items cut into parts (PARTS instantiations) -------------------------------------------------------
+// One workgroup per item leaves the chip idle when there are few items, and under a causal mask over ragged sequences
+// the longest item is several times the average.  An item's range of blocks is then cut into parts, one workgroup
+// each; all leave their fp32 accumulators in the workspace and the one that arrives last adds them up in the order of
+// the parts, so the result does not depend on the order of arrival (the stores and the counter as in ItemParts).
+// Accumulators of a wavefront at `at` (+ 4 * lane): NT blocks of 16 registers, [register / 4][lane][4].
+template <int NT>
+__device__ __forceinline__ void bwd_leave_part(const f32x16 *acc, float *at) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4)
+      part_store4(at + (t * 4 + i4) * 256, f32x4{acc[t][4 * i4], acc[t][4 * i4 + 1], acc[t][4 * i4 + 2], acc[t][4 * i4 + 3]});
+}
+// whether this workgroup is the last of the item's `count` to arrive; `flag` is a word of LDS nobody reads any more
+// after the barrier at the start
+__device__ __forceinline__ bool bwd_last_part(uint32_t *counter, int count, int *flag) {
+  parts_arrived();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const bool last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (uint32_t)count;
+    if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = last;
+  }
+  __syncthreads();
+  if (!*flag) return false;
+  parts_acquire();
+  return true;
+}
+template <int NT>
+__device__ __forceinline__ void bwd_sum_parts(f32x16 *acc, const float *first, size_t stride, int count) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
+#pragma unroll 2
+  for (int pt = 0; pt < count; ++pt) {
+    const float *at = first + (size_t)pt * stride;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const f32x4 v = *(const f32x4 *)(at + (t * 4 + i4) * 256);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[t][4 * i4 + j] += v[j];
+      }
+  }
+}
+// Cut of n blocks into at most max_parts parts of at least min_len (part i: blocks i * per .. )
+struct BwdCut {
+  int per, count;
+  __device__ __forceinline__ BwdCut(int n, int max_parts, int min_len) {
+    const int even = (n + max_parts - 1) / max_parts;
+    per = even > min_len ? even : min_len;
+    count = (n + per - 1) / per;
+    if (count < 1) count = 1;
+  }
+};
+// What a workgroup of the D = 128 dK/dV kernel keeps of its part in LDS, where no registers are left for it.
+struct BwdPartRecord {
+  float *first;        // partial accumulators of the item's first part
+  uint32_t *counter;
+  int part, count, qb_first, r_first, r_last_end, unused;
+};
+// The dK/dV kernels' share of a k block: the (q block, q head of the group) pairs, q block by q block, from the first
+// q block with a row that sees a key of the workgroup (causal) to the sequence's last; one part's are [u0, u1) of them.
+struct BwdKeyPart {
+  int qb_first, r_first, qb_last, r_last_end;   // q blocks qb_first .. qb_last, heads r_first .. of the first, .. r_last_end - 1 of the last
+  int count;
+  __device__ __forceinline__ BwdKeyPart(const BwdParams &p, int qb_begin, int qb_end, int shift, int wg_first_key, int part) {
+    int skip = 0;
+    if (p.causal) skip = min(max(0, wg_first_key - shift) / p.qbs, qb_end - qb_begin);
+    const int units = (qb_end - qb_begin - skip) * p.ratio;
+    const BwdCut cut(units, p.parts_k, p.min_units_k);
+    count = cut.count;
+    const int u0 = min(part * cut.per, units), u1 = min(u0 + cut.per, units);
+    const int first = u0 / p.ratio, last = (u1 - 1) / p.ratio;
+    qb_first = qb_begin + skip + first;
+    r_first = u0 - first * p.ratio;
+    qb_last = u1 > u0 ? qb_begin + skip + last : qb_first - 1;
+    r_last_end = u1 - last * p.ratio;
+  }
+};
+
 // ---- dQ ----------------------------------------------------------------------------------------------
-template <int D, typename E>
+template <int D, typename E, bool PARTS>
 __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   using T = BwdTile<D>;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -232,15 +316,29 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   // (grid decoding by XCD: see hbsa_bwd_dkv_kernel)
   int hk = blockIdx.y, bx = blockIdx.x;
   if (p.xcd_heads) {
-    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nqb * p.nsub);
+    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nqb * p.nsub) * (PARTS ? (unsigned)p.parts_q : 1u);
     hk = (int)(blockIdx.x & 7u) + 8 * (int)(t / per_head);
     bx = (int)(t % per_head);
+  }
+  int part = 0, nparts = 1;
+  const int per_part = p.nqb * p.nsub;
+  if constexpr (PARTS) {
+    part = bx / per_part;
+    bx -= part * per_part;
   }
   // last q blocks first: under a causal mask they are the long ones, and the grid should not end on them
   const int qb_rev = bx / p.nsub, sub = bx - qb_rev * p.nsub;
   const int qb = p.nqb - 1 - qb_rev;
   const QBlockInfo inf = p.info[qb];
   if (inf.rows <= 0) return;   // a q block with no row inside the tensors (its sequence did not fit them)
+  int blk_begin = 0, blk_end = inf.nkblk;   // k blocks of this part
+  if constexpr (PARTS) {
+    const BwdCut cut(min(inf.nkblk, (inf.kmax + p.kbs - 1) / p.kbs), p.parts_q, p.min_blocks_q);
+    nparts = cut.count;
+    if (part >= nparts) return;
+    blk_begin = part * cut.per;
+    blk_end = min(inf.nkblk, blk_begin + cut.per);
+  }
 
   const int slot = sub * 4 + wave;
   const int head_in_group = slot / p.wps;
@@ -275,7 +373,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
       }
     }
     dlt = half_sum(dlt);
-    if (g32 == 0 && l32 < nrows) {
+    if (g32 == 0 && l32 < nrows && (!PARTS || part == 0)) {
       p.delta[(int64_t)my_row * p.nhead_q + hq] = dlt;
       p.lse2[(int64_t)my_row * p.nhead_q + hq] = lse2;
     }
@@ -297,12 +395,13 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
 
   // the tile sequence: 64-key tiles of the kept k blocks, cut at the last key any row of the block sees
   int j = -1, kpos = 0;
-  int word_base = -32;      // k block of bit 0 of the word being walked
+  int word_base = (PARTS ? blk_begin & ~31 : 0) - 32;      // k block of bit 0 of the word being walked
   uint32_t word_left = 0;   // its kept blocks not visited yet
   // The bit row is read once, a word per lane (64 words = 2048 k blocks at a time), so that no load and its wait
   // stand between two tiles.
-  const int last_word = (inf.nkblk - 1) >> 5;
-  uint32_t row_words = lane <= last_word ? bits[lane] : 0u;
+  const int last_word = (blk_end - 1) >> 5;
+  const int word_at = PARTS ? ((blk_begin >> 5) & ~63) + lane : lane;
+  uint32_t row_words = word_at <= last_word ? bits[word_at] : 0u;
   auto next_tile = [&]() -> bool {
     if (j >= 0) {
       kpos += kTileKeys;
@@ -310,13 +409,17 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
     }
     while (word_left == 0) {   // next word of the bit row: 32 k blocks, kept or not
       word_base += 32;
-      if (word_base >= inf.nkblk) return false;
+      if (word_base >= blk_end) return false;
       const int w = word_base >> 5;
       if (w >= 64 && (w & 63) == 0) {   // beyond 2048 k blocks: the next 64 words, waited for here so that no other path waits
         row_words = w + lane <= last_word ? bits[w + lane] : 0u;
         __builtin_amdgcn_s_waitcnt(0x0F70);
       }
       word_left = (uint32_t)__builtin_amdgcn_readlane((int)row_words, w & 63);
+      if constexpr (PARTS) {
+        if (word_base < blk_begin) word_left &= ~0u << (blk_begin - word_base);
+        if (word_base + 32 > blk_end) word_left &= ~0u >> (word_base + 32 - blk_end);
+      }
     }
     j = word_base + __builtin_ctz(word_left);
     word_left &= word_left - 1;
@@ -475,6 +578,16 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
     half(std::integral_constant<int, 0>{});
     half(std::integral_constant<int, 1>{});
   }
+  if constexpr (PARTS) {
+    if (nparts > 1) {
+      constexpr size_t kWaveFloats = (size_t)T::DT * 1024;   // of one wavefront's accumulators
+      const uint32_t item = (uint32_t)hk * (uint32_t)per_part + (uint32_t)bx;
+      float *first = p.parts + ((size_t)item * p.parts_q * 4 + wave) * kWaveFloats + lane * 4;
+      if (active) bwd_leave_part<T::DT>(acc, first + (size_t)part * 4 * kWaveFloats);
+      if (!bwd_last_part(p.arrivals + item, nparts, (int *)lds)) return;
+      if (active) bwd_sum_parts<T::DT>(acc, first, 4 * kWaveFloats, nparts);
+    }
+  }
   if (active && l32 < nrows)
     bwd_store_rows<D, E>(p.dq + (int64_t)(inf.row_begin + row0 + l32) * p.dq_s + (int64_t)hq * p.dq_h, acc, p.scale, g32);
 }
@@ -485,7 +598,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
 // fill at most two 32-key slots (k blocks of up to 64 keys, or the narrow rest of a wider block), two
 // wavefronts share a slot and take the upper and lower 32 rows of every tile; their partial sums are added
 // through LDS at the end, as in the D = 128 kernel below.
-template <int D, typename E>
+template <int D, typename E, bool PARTS>
 __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) {
   static_assert(D <= 64, "head dim 128 has its own kernel");
   using T = BwdTile<D>;
@@ -502,9 +615,15 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   // one sequence at a time, and every XCD has the same amount of work whatever the sequence lengths.
   int hk = blockIdx.y, bx = blockIdx.x;
   if (p.xcd_heads) {
-    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nkb * p.nsub_k);
+    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u);
     hk = (int)(blockIdx.x & 7u) + 8 * (int)(t / per_head);
     bx = (int)(t % per_head);
+  }
+  int part = 0;
+  const int per_part = p.nkb * p.nsub_k;
+  if constexpr (PARTS) {
+    part = bx / per_part;
+    bx -= part * per_part;
   }
   const int kb = bx / p.nsub_k, sub = bx - kb * p.nsub_k;
 
@@ -517,7 +636,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   const int wg_keys = min(4 * kWaveRows, p.kbs - sub * 4 * kWaveRows);   // by the block size: the same for every k block
   const bool shared_slots = wg_keys <= 2 * kWaveRows;                    // two wavefronts per 32-key slot
   const int slot = shared_slots ? (wave & 1) : wave;
-  const int part = shared_slots ? (wave >> 1) : 0;                       // which 32 rows of a tile (shared slots)
+  const int rows_half = shared_slots ? (wave >> 1) : 0;                  // which 32 rows of a tile (shared slots)
   const int row0 = (sub * 4 + slot) * kWaveRows;
   const int nrows = min(kWaveRows, krows - row0);
   const bool active = nrows > 0;
@@ -547,9 +666,10 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   // the group, the block's rows in 64-row tiles (under a causal mask only those with a row that sees a
   // key of this workgroup)
   int qb = p.cu_num_q_block[b] - 1, r = 0, qoff = 0;
-  const int qb_end = p.cu_num_q_block[b + 1];
+  int qb_end = p.cu_num_q_block[b + 1];
   const int qb_begin = p.cu_num_q_block[b];
   int kept_base = qb_begin - 64;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
+  int qb_first = qb_begin, r_first = 0, r_last_end = p.ratio, nparts = 1;   // the part's share (BwdKeyPart)
   uint64_t kept = 0;
   QBlockInfo inf = {};
   int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
@@ -559,6 +679,16 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
     seq_qlen = klen - first.shift;
     inf.shift = first.shift;
   }
+  if constexpr (PARTS) {
+    const BwdKeyPart share(p, qb_begin, qb_end, inf.shift, wg_first_key, part);
+    nparts = share.count;
+    if (part >= nparts) return;
+    qb_first = share.qb_first;
+    r_first = share.r_first;
+    r_last_end = share.r_last_end;
+    qb_end = share.qb_last + 1;
+    kept_base = qb_first - 64;
+  }
   auto tile_reaches = [&]() {
     return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
   };
@@ -567,7 +697,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       if (qb >= qb_begin) {   // inside a kept q block: next tile, then next head
         qoff += 64;
         if (qoff >= inf.rows) { qoff = 0; ++r; }
-        if (r < p.ratio) {
+        if (r < (PARTS && qb == qb_end - 1 ? r_last_end : p.ratio)) {
           if (tile_reaches()) return true;
           continue;
         }
@@ -585,7 +715,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       inf.q_pos = (qb - qb_begin) * p.qbs;
       inf.row_begin = seq_row0 + inf.q_pos;
       inf.rows = min(p.qbs, seq_qlen - inf.q_pos);
-      r = 0;
+      r = PARTS && qb == qb_first ? r_first : 0;
       qoff = -64;   // the step above moves to the block's first tile
     }
   };
@@ -640,7 +770,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
     if (l32 >= nrows) first_vis = 64;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      if (shared_slots && h != part) continue;   // the slot's other wavefront takes these rows
+      if (shared_slots && h != rows_half) continue;   // the slot's other wavefront takes these rows
       const f32x16 s = bwd_rows_times_frag<D, E>(q_t, h, kf, lane);
       const f32x16 dp = bwd_rows_times_frag<D, E>(g_t, h, vf, lane);
       float ep[16], ed[16];
@@ -669,7 +799,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   if (shared_slots) {   // the wavefronts of the lower rows hand their sums to those of the upper rows: [slot][register][lane] floats
     __syncthreads();
     float *xch = (float *)lds + (size_t)slot * (2 * T::DT * 16) * 64 + lane;
-    if (part == 1) {
+    if (rows_half == 1) {
 #pragma unroll
       for (int dt = 0; dt < T::DT; ++dt)
 #pragma unroll
@@ -679,7 +809,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
         }
     }
     __syncthreads();
-    if (part == 0) {
+    if (rows_half == 0) {
 #pragma unroll
       for (int dt = 0; dt < T::DT; ++dt)
 #pragma unroll
@@ -689,7 +819,23 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
         }
     }
   }
-  if (part == 0 && active && l32 < nrows) {
+  if constexpr (PARTS) {
+    if (nparts > 1) {
+      constexpr size_t kWaveFloats = (size_t)2 * T::DT * 1024;   // of one slot's accumulators
+      const uint32_t item = (uint32_t)hk * (uint32_t)per_part + (uint32_t)bx;
+      float *at = p.parts + ((size_t)item * p.parts_k * 4 + slot) * kWaveFloats + lane * 4;
+      if (rows_half == 0 && active) {
+        bwd_leave_part<T::DT>(acc_k, at + (size_t)part * 4 * kWaveFloats);
+        bwd_leave_part<T::DT>(acc_v, at + (size_t)part * 4 * kWaveFloats + kWaveFloats / 2);
+      }
+      if (!bwd_last_part(p.arrivals + item, nparts, (int *)lds)) return;
+      if (rows_half == 0 && active) {
+        bwd_sum_parts<T::DT>(acc_k, at, 4 * kWaveFloats, nparts);
+        bwd_sum_parts<T::DT>(acc_v, at + kWaveFloats / 2, 4 * kWaveFloats, nparts);
+      }
+    }
+  }
+  if (rows_half == 0 && active && l32 < nrows) {
     const int64_t row = k0 + kbl * p.kbs + row0 + l32;
     bwd_store_rows<D, E>(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h, acc_k, p.scale, g32);
     bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, acc_v, 1.f, g32);
@@ -709,7 +855,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
 // and two tiles ahead (one workgroup per CU has nobody else to cover its waits for memory): four Q buffers
 // (tile t - 1 is still read while tile t + 2 arrives), three for dO, and with them three and four sets of the
 // rows' log-sum-exp and delta, which wavefront 0 loads into LDS the same way.
-template <typename E>
+template <typename E, bool PARTS>
 __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   constexpr int D = 128;
   using T = BwdTile<D>;
@@ -719,6 +865,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   char *p_buf = lds + 7 * T::TILE_BYTES;               // [2 tile parities][4 slots][2 halves][2][64 lanes] eight 16-bit values
   float *lse_s = (float *)(lds + 9 * T::TILE_BYTES);   // [3][64] log2-domain log-sum-exp of the tile's rows (index: the dO buffer's)
   float *dlt_s = lse_s + 192;                          // [4][64] their delta (index: the Q buffer's)
+  BwdPartRecord *part_s = (BwdPartRecord *)(dlt_s + 256);   // PARTS
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -730,9 +877,15 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   // one sequence at a time, and every XCD has the same amount of work whatever the sequence lengths.
   int hk = blockIdx.y, bx = blockIdx.x;
   if (p.xcd_heads) {
-    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nkb * p.nsub_k);
+    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u);
     hk = (int)(blockIdx.x & 7u) + 8 * (int)(t / per_head);
     bx = (int)(t % per_head);
+  }
+  int part = 0;
+  const int per_part = p.nkb * p.nsub_k;
+  if constexpr (PARTS) {
+    part = bx / per_part;
+    bx -= part * per_part;
   }
   const int kb = bx / p.nsub_k, sub = bx - kb * p.nsub_k;
 
@@ -769,9 +922,10 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
 
   int qb = p.cu_num_q_block[b] - 1, r = 0, qoff = 0;
-  const int qb_end = p.cu_num_q_block[b + 1];
+  int qb_end = p.cu_num_q_block[b + 1];
   const int qb_begin = p.cu_num_q_block[b];
   int kept_base = qb_begin - 64;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
+  int r_end = p.ratio;   // heads of the q block that are the part's
   uint64_t kept = 0;
   QBlockInfo inf = {};
   int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
@@ -781,6 +935,18 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     seq_qlen = klen - first.shift;
     inf.shift = first.shift;
   }
+  if constexpr (PARTS) {
+    const BwdKeyPart share(p, qb_begin, qb_end, inf.shift, wg_first_key, part);
+    if (part >= share.count) return;
+    if (threadIdx.x == 0) {
+      const size_t item = (size_t)hk * per_part + bx;
+      *part_s = BwdPartRecord{p.parts + item * p.parts_k * 8 * (T::DT * 1024), p.arrivals + item, part, share.count,
+                              share.qb_first, share.r_first, share.r_last_end, 0};
+    }
+    __syncthreads();
+    qb_end = share.qb_last + 1;
+    kept_base = share.qb_first - 64;
+  }
   auto tile_reaches = [&]() {
     return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
   };
@@ -789,7 +955,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       if (qb >= qb_begin) {
         qoff += 64;
         if (qoff >= inf.rows) { qoff = 0; ++r; }
-        if (r < p.ratio) {
+        if (r < (PARTS ? r_end : p.ratio)) {
           if (tile_reaches()) return true;
           continue;
         }
@@ -809,6 +975,10 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       inf.row_begin = seq_row0 + inf.q_pos;
       inf.rows = min(p.qbs, seq_qlen - inf.q_pos);
       r = 0;
+      if constexpr (PARTS) {
+        if (qb == __builtin_amdgcn_readfirstlane(part_s->qb_first)) r = __builtin_amdgcn_readfirstlane(part_s->r_first);
+        r_end = qb == qb_end - 1 ? __builtin_amdgcn_readfirstlane(part_s->r_last_end) : p.ratio;
+      }
       qoff = -64;
     }
   };
@@ -1030,6 +1200,17 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     gi = gi == 2 ? 0 : gi + 1;
     par ^= 1;
   }
+  if constexpr (PARTS) {
+    const BwdPartRecord rec = *part_s;
+    const int count = __builtin_amdgcn_readfirstlane(rec.count);
+    if (count > 1) {
+      constexpr size_t kWaveFloats = (size_t)T::DT * 1024;   // of one wavefront's accumulators
+      float *at = rec.first + (size_t)wave * kWaveFloats + lane * 4;
+      if (active) bwd_leave_part<T::DT>(acc, at + (size_t)rec.part * 8 * kWaveFloats);
+      if (!bwd_last_part(rec.counter, count, (int *)lds)) return;
+      if (active) bwd_sum_parts<T::DT>(acc, at, 8 * kWaveFloats, count);
+    }
+  }
   if (active && l32 < nrows) {
     const int64_t row = k0 + kbl * p.kbs + row0 + l32;
     if constexpr (ROLE == 0) bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, acc, 1.f, g32);
@@ -1040,41 +1221,46 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   else run(std::integral_constant<int, 1>{});
 }
 
-template <int D, typename E>
-int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
+template <int D, typename E, bool PARTS_Q, bool PARTS_K>
+int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   using T = BwdTile<D>;
   // LDS: the dQ kernel's three K and two V tiles; the dK/dV kernels' tile buffers, P records and row values
-  const int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? 9 * T::TILE_BYTES + 2048 : 4 * T::TILE_BYTES + 1024;
-  if (lds_dkv > 48 * 1024) {
+  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? 9 * T::TILE_BYTES + 2048 : 4 * T::TILE_BYTES + 1024;
+  if constexpr (lds_dkv > 48 * 1024) {
     static thread_local bool raised[kMaxDevices] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
       return fail(HBSA_ERR_UNSUPPORTED, "no current device, or device index above %d", kMaxDevices - 1);
     if (!raised[dev]) {
       const void *dkv = nullptr;
-      if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E>);
-      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E>);
+      if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E, PARTS_K>);
+      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K>);
       hipError_t e = hipFuncSetAttribute(dkv, hipFuncAttributeMaxDynamicSharedMemorySize, lds_dkv);
       if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&hbsa_bwd_dq_kernel<D, E>),
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&hbsa_bwd_dq_kernel<D, E, PARTS_Q>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_dq);
       if (e != hipSuccess) return (int)e;
       raised[dev] = true;
     }
   }
-  const dim3 q_grid = bp.xcd_heads ? dim3((unsigned)(bp.nqb * bp.nsub * nhead_k)) : dim3((unsigned)(bp.nqb * bp.nsub), (unsigned)nhead_k);
-  hipLaunchKernelGGL((hbsa_bwd_dq_kernel<D, E>), q_grid, dim3(kThreads), lds_dq, stream, bp);
-  const dim3 kv_grid = bp.xcd_heads ? dim3((unsigned)(num_k_block * bp.nsub_k * nhead_k))
-                                    : dim3((unsigned)(num_k_block * bp.nsub_k), (unsigned)nhead_k);
-  if constexpr (D == 128) {
-    hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E>), kv_grid, dim3(512),
-                       lds_dkv, stream, bp);
-  } else {
-    hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E>), kv_grid,
-                       dim3(kThreads), lds_dkv, stream, bp);
-  }
+  const unsigned q_wgs = (unsigned)(bp.nqb * bp.nsub * (PARTS_Q ? bp.parts_q : 1));
+  const unsigned k_wgs = (unsigned)(num_k_block * bp.nsub_k * (PARTS_K ? bp.parts_k : 1));
+  const dim3 q_grid = bp.xcd_heads ? dim3(q_wgs * (unsigned)nhead_k) : dim3(q_wgs, (unsigned)nhead_k);
+  const dim3 kv_grid = bp.xcd_heads ? dim3(k_wgs * (unsigned)nhead_k) : dim3(k_wgs, (unsigned)nhead_k);
+  hipLaunchKernelGGL((hbsa_bwd_dq_kernel<D, E, PARTS_Q>), q_grid, dim3(kThreads), lds_dq, stream, bp);
+  if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K>), kv_grid, dim3(512), lds_dkv, stream, bp);
+  else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
+}
+
+template <int D, typename E>
+int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
+  const bool pq = bp.parts_q > 1, pk = bp.parts_k > 1;
+  if (pq && pk) return launch_bwd_kernels<D, E, true, true>(bp, nhead_k, num_k_block, stream);
+  if (pq) return launch_bwd_kernels<D, E, true, false>(bp, nhead_k, num_k_block, stream);
+  if (pk) return launch_bwd_kernels<D, E, false, true>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_kernels<D, E, false, false>(bp, nhead_k, num_k_block, stream);
 }
 
 }  // namespace hbsa

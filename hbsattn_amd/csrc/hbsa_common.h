@@ -328,6 +328,11 @@ struct BwdParams {
   int32_t nsub_k;        // k side: workgroups per (kv head, k block) = ceil(k_block_size / 128)
   float c;               // softmax_scale * log2(e), signed
   float scale;
+  // Items cut into parts (see BwdCut): at most parts_q k block ranges a dQ item, of min_blocks_q k blocks at least, and parts_k
+  // ranges of (q block, q head) pairs a dK/dV item, of min_units_k pairs at least; 1: whole
+  int32_t parts_q, min_blocks_q, parts_k, min_units_k;
+  float *parts;          // partial accumulators, shared by the two launches
+  uint32_t *arrivals;    // one counter per item, zero before and after every launch
 };
 
 // ---- Items of the kernels without a scheduler: geometry and kept blocks straight from the caller's arrays (bits == nullptr)

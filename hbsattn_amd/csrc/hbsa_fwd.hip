@@ -437,6 +437,37 @@ int decode_max_parts(long long items, int num_k_block) {
   long long parts = std::min<long long>(kDecodeMaxParts, 30ll * device_cus() / items);
   return odd_parts(std::min<long long>(parts, num_k_block));
 }
+// ---- Parts of the backward's items (BwdCut), when the items leave places of the device empty (`resident` workgroups a CU):
+// as many as fill the places `rounds` times, of kBwdPartKeys keys or query rows at least.  Partial sums cost a write
+// through to memory and a read back (128 KB a part of the D = 128 dK/dV kernel), so more items than that stay whole.
+// Measured (forward not included, whole items -> parts): 1 x 3000 tokens, 8 / 2 heads of 128, 48 dK/dV items, 262 us -> 2, 4, 6, 8,
+// 12 parts 171, 136, 125, 134, 147; 1 x 8000, 32 / 1 heads of 64, 63 items, 2068 -> 4, 8, 16, 32 parts 827, 648, 535, 490;
+// 6 x 300 .. 4000, 16 / 4 heads of 64, 708 items, 253 -> 2, 4, 8 parts 250, 250, 276; 512 items of 128 542 -> 556, 650, 945.
+constexpr int kBwdPartKeys = 512, kBwdPartRows = 512;
+struct BwdPartPlan {
+  long long q_items, k_items;
+  int parts_q, parts_k;
+  size_t bytes;   // of the partial accumulators, shared by the two launches
+};
+inline int bwd_parts(long long items, int resident, int rounds, int pieces, size_t item_bytes) {
+  const long long places = (long long)device_cus() * resident;
+  if (items <= 0 || items > kMaxPartItems || 4 * items > 3 * places) return 1;
+  long long parts = std::min<long long>(std::min<long long>(32, (rounds * places + items - 1) / items), pieces);
+  parts = std::min<long long>(parts, (long long)(kMaxPartBytes / (item_bytes * (size_t)items)));
+  return parts < 2 ? 1 : (int)parts;
+}
+BwdPartPlan bwd_part_plan(int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size, int k_block_size) {
+  const int ratio = nhead_q / nhead_k, wps = (q_block_size + kWaveRows - 1) / kWaveRows;
+  BwdPartPlan r;
+  r.q_items = (long long)nhead_k * num_q_block * ((ratio * wps + 3) / 4);
+  r.k_items = (long long)nhead_k * num_k_block * ((k_block_size + 4 * kWaveRows - 1) / (4 * kWaveRows));
+  const size_t q_bytes = (size_t)4 * kWaveRows * headdim * sizeof(float), k_bytes = 2 * q_bytes;
+  r.parts_q = bwd_parts(r.q_items, headdim == 128 ? 2 : 3, 1, num_k_block, q_bytes);
+  r.parts_k = bwd_parts(r.k_items, headdim == 128 ? 1 : 3, headdim == 128 ? 1 : 2, (int)std::min<long long>((long long)num_q_block * ratio, 1 << 20), k_bytes);
+  const size_t bq = r.parts_q > 1 ? q_bytes * r.parts_q * (size_t)r.q_items : 0, bk = r.parts_k > 1 ? k_bytes * r.parts_k * (size_t)r.k_items : 0;
+  r.bytes = align_up(std::max(bq, bk), 256);
+  return r;
+}
 inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_block_size) {
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, true);
   return (long long)nhead_k * num_q_block * ((slots + 3) / 4);
@@ -1149,6 +1180,17 @@ size_t hbsa_bwd_workspace_bytes(int32_t total_q, int32_t nhead_q) {
   return 2 * align_up((size_t)total_q * nhead_q * sizeof(float), 256);   // delta and the scaled log-sum-exp of every (row, q head)
 }
 
+size_t hbsa_bwd_workspace_bytes_parts(int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block,
+                                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size) {
+  const size_t base = hbsa_bwd_workspace_bytes(total_q, nhead_q);
+  if (nhead_k <= 0 || nhead_q <= 0 || nhead_q % nhead_k || num_q_block <= 0 || num_k_block <= 0 || q_block_size <= 0 || k_block_size <= 0 ||
+      (headdim != 32 && headdim != 64 && headdim != 128))
+    return base;
+  const BwdPartPlan plan = bwd_part_plan(nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size);
+  if (plan.bytes == 0) return base;
+  return align_up(base, 256) + 256 + plan.bytes + align_up((size_t)std::max(plan.q_items, plan.k_items) * sizeof(uint32_t), 256);
+}
+
 int hbsa_bwd(const void *q, const void *k, const void *v, const void *out, const void *dout, const float *lse, void *dq,
              void *dk, void *dv, const int32_t *cu_k_seqlens, const int32_t *cu_num_q_block, const int32_t *cu_num_k_block,
              const void *workspace, size_t workspace_bytes, void *bwd_workspace, size_t bwd_workspace_bytes, int32_t dtype,
@@ -1216,6 +1258,26 @@ int hbsa_bwd(const void *q, const void *k, const void *v, const void *out, const
   bp.c = softmax_scale * kLog2e;
   bp.scale = softmax_scale;
   hipStream_t st = (hipStream_t)stream;
+  bp.parts_q = bp.parts_k = 1;
+  const size_t with_parts = hbsa_bwd_workspace_bytes_parts(total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size);
+  const size_t base = hbsa_bwd_workspace_bytes(total_q, nhead_q);
+  if (with_parts > base && bwd_workspace_bytes >= with_parts) {
+    const BwdPartPlan plan = bwd_part_plan(nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size);
+    char *area = (char *)(((uintptr_t)bwd_workspace + base + 255) & ~(uintptr_t)255);
+    // (counters of a captured launch, or of a stream without counters of its own: as in set_parts)
+    if (is_capturing(st) || stream_sched_of(st, &bp.arrivals) == nullptr) {
+      bp.arrivals = (uint32_t *)(area + plan.bytes);
+      const int n = (int)std::max(plan.parts_q > 1 ? plan.q_items : 0, plan.parts_k > 1 ? plan.k_items : 0);
+      hipLaunchKernelGGL(hbsa_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, bp.arrivals, n);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return fail((int)e, "hbsa_zero_kernel launch: %s", hipGetErrorString(e));
+    }
+    bp.parts = (float *)area;
+    bp.parts_q = plan.parts_q;
+    bp.parts_k = plan.parts_k;
+    bp.min_blocks_q = std::max(1, kBwdPartKeys / k_block_size);
+    bp.min_units_k = std::max(1, kBwdPartRows / q_block_size);
+  }
   const bool bf = dtype == HBSA_DTYPE_BF16;
   switch (headdim) {
     case 32: return bf ? launch_bwd<32, ElemBF16>(bp, nhead_k, num_k_block, st) : launch_bwd<32, ElemF16>(bp, nhead_k, num_k_block, st);

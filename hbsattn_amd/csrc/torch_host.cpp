@@ -201,7 +201,7 @@ struct Attention : public torch::autograd::Function<Attention> {
     const hipStream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)q.get_device()).stream();
     at::Tensor dq = at::empty(q.sizes(), q.options()), dk = at::empty(k.sizes(), k.options()), dv = at::empty(v.sizes(), v.options());
     const int tq = (int)q.size(0), tk = (int)k.size(0), hq = (int)q.size(1), hk = (int)k.size(1), d = (int)q.size(2);
-    const size_t n = hbsa_bwd_workspace_bytes(tq, hq);
+    const size_t n = hbsa_bwd_workspace_bytes_parts(tq, hq, hk, d, (int)shape[0], (int)shape[1], (int)shape[2], (int)shape[3]);
     at::Tensor bws = bytes_like(q, n);
     const int64_t strides[16] = {q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), out.stride(0), out.stride(1),
                                  dout.stride(0), dout.stride(1), dq.stride(0), dq.stride(1), dk.stride(0), dk.stride(1), dv.stride(0),

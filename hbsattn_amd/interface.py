@@ -301,7 +301,8 @@ def hbsa_backward(q, k, v, out, dout, lse, prepared: PreparedMask, softmax_scale
         dout = dout if _rows_ok(dout) else dout.contiguous()
     lse = lse.contiguous()
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    bws_bytes = int(lib.hbsa_bwd_workspace_bytes(total_q, nhead_q))
+    bws_bytes = int(lib.hbsa_bwd_workspace_bytes_parts(total_q, nhead_q, nhead_k, d_run, prepared.num_q_block, prepared.num_k_block,
+                                                       prepared.q_block_size, prepared.k_block_size))
     bws = torch.empty(bws_bytes, dtype=torch.uint8, device=q.device)
     strides = (ctypes.c_int64 * 16)(q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
                                     out.stride(0), out.stride(1), dout.stride(0), dout.stride(1), dq.stride(0),

@@ -349,7 +349,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out,
  *                             dout_tok, dout_head, dq_tok, dq_head, dk_tok, dk_head, dv_tok, dv_head }
  *
  * Supported: HBSA_DTYPE_BF16 and HBSA_DTYPE_F16, headdim in {32, 64, 128}.  Every element of dq, dk
- * and dv is written (zeros where no gradient flows); no atomics, so results are deterministic.
+ * and dv is written (zeros where no gradient flows), sums are taken in a fixed order: results are deterministic.
  * There are no fp32 backward kernels: the fp32 matrix rate is a sixteenth of the 16-bit one and a backward
  * is 2.5 forwards of matrix work.  A caller with fp32 tensors passes bf16 copies of q, k, v, out and dout
  * (bf16 keeps fp32's range), with out and lse from a forward on those copies, and widens the gradients, which
@@ -358,6 +358,12 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out,
  * in registers, 254 of 256 at headdim 128.
  */
 size_t hbsa_bwd_workspace_bytes(int32_t total_q, int32_t nhead_q);
+
+/* The bwd_workspace with which problems of few blocks are cut into parts that fill the device: with that many bytes or more
+ * hbsa_bwd adds partial dq, dk and dv up in fp32, in a fixed order; with fewer every block is one workgroup's, and the last
+ * bits of the results may differ.  Never less than hbsa_bwd_workspace_bytes; follows the current device's number of CUs. */
+size_t hbsa_bwd_workspace_bytes_parts(int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block,
+                                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size);
 
 int hbsa_bwd(const void *q, const void *k, const void *v, const void *out, const void *dout,
              const float *lse, void *dq, void *dk, void *dv,
