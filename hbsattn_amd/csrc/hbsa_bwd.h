@@ -8,7 +8,8 @@
 //     dV = P^T dO      dP = dO V^T      dS = P * (dP - delta)
 //     dQ = scale * dS K                 dK = scale * dS^T Q
 //
-// Two launches per call, no atomics, every output element written by exactly one workgroup:
+// Two launches per call, every output element written by exactly one workgroup, sums in a fixed order (few items are cut
+// into parts that combine themselves, see bwd_last_part):
 //   hbsa_bwd_dq_kernel    : one workgroup per (kv head, q block, group of four 32-row wave slots), the
 //                           forward's decomposition; walks the kept k blocks of the q block's bit row.
 //                           Per 64-key tile  S^T = K Q^T,  dP^T = V dO^T  (A = tile rows from LDS,
@@ -24,8 +25,10 @@
 //                           S = Q K^T,  dP = dO V^T,  dV^T += dO^T P,  dK^T += Q^T dS.
 // Both recompute S.  The kept blocks of a mask row or column are found with one load per 32 or 64
 // blocks, not one per block.  Tiles go from global memory straight into LDS (global_load_lds_dwordx4),
-// two buffers: tile t + 1 travels while tile t is computed on, one barrier per tile (the D = 128 dK/dV kernel
-// has four Q and three dO buffers and fetches two tiles ahead).  A tile that is
+// two tiles ahead (V tiles of the dQ kernel one): tiles t + 1 and t + 2 travel while tile t is computed on, one barrier per
+// tile.  The dK/dV kernels walk the q blocks from the last to the first, so that the workgroups of a sequence, each of which
+// a causal mask lets begin at another q block, start with the same tiles; the delta and the log-sum-exp of a tile's rows are
+// consecutive floats of one q head.  A tile that is
 // read both by rows and transposed is stored once, in a layout without bank conflicts for either
 // (BwdTile::swz_both).  In the dQ kernel and the D = 128 dK/dV kernel the operand reads from LDS are issued by
 // hand, a fixed number ahead of the products that use them (BwdOperandOffsets).  The forward's persistent
@@ -33,6 +36,7 @@
 // both kernels at long sequences is the stream of tiles from memory next to the matrix work, not the tail.
 
 #pragma once
+
 
 #include "hbsa_common.h"
 
@@ -302,6 +306,26 @@ struct BwdKeyPart {
   }
 };
 
+// The kv head and the workgroup of that head (of per_head).  Workgroup ids go round the eight XCDs, each with its own L2.
+// With a multiple of eight kv heads XCD x works on the heads x, x + 8, ..., one after the other: the workgroups that share an
+// L2 then read one head of one sequence at a time, and every XCD has the same amount of work whatever the sequence lengths.
+// Any other number of heads goes round with the ids: with 1, 2 or 4 of them an XCD still sees one head only, and the
+// heaviest workgroups of all heads start before the light ones of any (4 heads: 228 -> 195 and 533 -> 456 us backward).
+__device__ __forceinline__ void bwd_decode_grid(const BwdParams &p, unsigned per_head, int &hk, int &bx) {
+  const unsigned nhk = gridDim.x / per_head;
+  if (p.xcd_heads) {
+    const unsigned t = blockIdx.x >> 3;
+    hk = (int)(blockIdx.x & 7u) + 8 * (int)(t / per_head);
+    bx = (int)(t % per_head);
+  } else if (nhk > 1) {
+    hk = (int)(blockIdx.x % nhk);
+    bx = (int)(blockIdx.x / nhk);
+  } else {
+    hk = blockIdx.y;
+    bx = blockIdx.x;
+  }
+}
+
 // ---- dQ ----------------------------------------------------------------------------------------------
 template <int D, typename E, bool PARTS>
 __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
@@ -313,13 +337,8 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g32 = lane >> 5, l32 = lane & 31;
-  // (grid decoding by XCD: see hbsa_bwd_dkv_kernel)
-  int hk = blockIdx.y, bx = blockIdx.x;
-  if (p.xcd_heads) {
-    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nqb * p.nsub) * (PARTS ? (unsigned)p.parts_q : 1u);
-    hk = (int)(blockIdx.x & 7u) + 8 * (int)(t / per_head);
-    bx = (int)(t % per_head);
-  }
+  int hk, bx;
+  bwd_decode_grid(p, (unsigned)(p.nqb * p.nsub) * (PARTS ? (unsigned)p.parts_q : 1u), hk, bx);
   int part = 0, nparts = 1;
   const int per_part = p.nqb * p.nsub;
   if constexpr (PARTS) {
@@ -374,8 +393,8 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
     }
     dlt = half_sum(dlt);
     if (g32 == 0 && l32 < nrows && (!PARTS || part == 0)) {
-      p.delta[(int64_t)my_row * p.nhead_q + hq] = dlt;
-      p.lse2[(int64_t)my_row * p.nhead_q + hq] = lse2;
+      p.delta[(int64_t)hq * p.total_q + my_row] = dlt;
+      p.lse2[(int64_t)hq * p.total_q + my_row] = lse2;
     }
   } else {
 #pragma unroll
@@ -594,31 +613,28 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
 
 // ---- dK, dV (head dims up to 64) ---------------------------------------------------------------------
 // Four wavefronts; K^T and V^T of a wavefront's 32 keys stay in registers.  The Q and dO tiles go straight
-// into LDS like the dQ kernel's (two buffers, one layout, one barrier per tile).  When the workgroup's keys
+// into LDS like the dQ kernel's (three buffers, one layout, one barrier per tile).  When the workgroup's keys
 // fill at most two 32-key slots (k blocks of up to 64 keys, or the narrow rest of a wider block), two
 // wavefronts share a slot and take the upper and lower 32 rows of every tile; their partial sums are added
-// through LDS at the end, as in the D = 128 kernel below.
+// through LDS at the end.
+// What bounds it: instruction issue, with two wavefronts per SIMD (226 registers when P, dS and both accumulators were in
+// flight together, 207 now; at three wavefronts, 168 registers, 50 of them spill).  Hence no comparisons where all rows see
+// all keys and none for keys past the block's end (their columns are not stored).  Operand reads issued by hand as in the
+// dQ kernel were measured and are no faster.  dQ + dK/dV, 6 x 300 .. 4000 tokens, 16 / 4 heads, 64-key blocks, keep 0.4:
+// 250 -> 227 us with the loads two tiles ahead, 195 with the heads going round the grid (bwd_decode_grid).
 template <int D, typename E, bool PARTS>
 __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) {
   static_assert(D <= 64, "head dim 128 has its own kernel");
   using T = BwdTile<D>;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  // buffer s of the tiles: Q rows at s * 2 * TILE_BYTES, dO rows one tile further
-  float *rowv = (float *)(lds + 4 * T::TILE_BYTES);    // buffer s: [64] log2-domain log-sum-exp of the tile's rows, [64] their delta
+  // buffer s of the tiles (three of them): Q rows at s * 2 * TILE_BYTES, dO rows one tile further
+  float *rowv = (float *)(lds + 6 * T::TILE_BYTES);    // buffer s: [64] log2-domain log-sum-exp of the tile's rows, [64] their delta
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g32 = lane >> 5, l32 = lane & 31;
-  // With a multiple of eight kv heads the grid is one-dimensional and workgroup ids, which go round the
-  // eight XCDs (each with its own L2), are decoded so that XCD x works on the heads x, x + 8, ...: the
-  // workgroups that share an L2 then walk the k blocks of one head in order and read the Q and dO rows of
-  // one sequence at a time, and every XCD has the same amount of work whatever the sequence lengths.
-  int hk = blockIdx.y, bx = blockIdx.x;
-  if (p.xcd_heads) {
-    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u);
-    hk = (int)(blockIdx.x & 7u) + 8 * (int)(t / per_head);
-    bx = (int)(t % per_head);
-  }
+  int hk, bx;
+  bwd_decode_grid(p, (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u), hk, bx);
   int part = 0;
   const int per_part = p.nkb * p.nsub_k;
   if constexpr (PARTS) {
@@ -642,6 +658,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   const bool active = nrows > 0;
   const int key_pos = kbl * p.kbs + min(row0 + l32, krows - 1);   // in-sequence position of this lane's key
   const int wg_first_key = kbl * p.kbs + sub * 4 * kWaveRows;     // of the workgroup's first key
+  const int wave_key_max = kbl * p.kbs + min(row0 + kWaveRows - 1, krows - 1);   // position of the wavefront's last key
 
   short8v kf[T::KSTEPS], vf[T::KSTEPS];   // K^T and V^T fragments: lane holds key l32, d = 16*ks + 8*g32 .. +7
   if (active) {
@@ -668,7 +685,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   int qb = p.cu_num_q_block[b] - 1, r = 0, qoff = 0;
   int qb_end = p.cu_num_q_block[b + 1];
   const int qb_begin = p.cu_num_q_block[b];
-  int kept_base = qb_begin - 64;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
+  int kept_base = qb_end;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
   int qb_first = qb_begin, r_first = 0, r_last_end = p.ratio, nparts = 1;   // the part's share (BwdKeyPart)
   uint64_t kept = 0;
   QBlockInfo inf = {};
@@ -687,7 +704,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
     r_first = share.r_first;
     r_last_end = share.r_last_end;
     qb_end = share.qb_last + 1;
-    kept_base = qb_first - 64;
+    kept_base = qb_end;
   }
   auto tile_reaches = [&]() {
     return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
@@ -703,14 +720,16 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
         }
       }
       while (kept == 0) {   // one load per 64 q blocks: lane i looks at q block kept_base + i
-        kept_base += 64;
-        if (kept_base >= qb_end) return false;
+        kept_base -= 64;
+        if (kept_base + 63 < qb_first) return false;
         uint32_t word = 0;
-        if (kept_base + lane < qb_end) word = p.bits[((size_t)hk * p.nqb + kept_base + lane) * p.wpr + (kbl >> 5)];
+        if (kept_base + lane >= qb_first && kept_base + lane < qb_end) word = p.bits[((size_t)hk * p.nqb + kept_base + lane) * p.wpr + (kbl >> 5)];
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // (waited for here so that no other path waits)
         kept = __ballot((word >> (kbl & 31)) & 1u);
       }
-      qb = kept_base + __builtin_ctzll(kept);
-      kept &= kept - 1;
+      const int at = 63 - __builtin_clzll(kept);
+      qb = kept_base + at;
+      kept &= ~(1ull << at);
       // the q block's geometry follows from the sequence's (no load on this path)
       inf.q_pos = (qb - qb_begin) * p.qbs;
       inf.row_begin = seq_row0 + inf.q_pos;
@@ -725,8 +744,9 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   const uint32_t ld_chunk = (uint32_t)(((lane % T::CPR) ^ T::swz_both(ld_row)) * 16);
   const uint32_t q_s32 = (uint32_t)p.q_s, do_s32 = (uint32_t)p.do_s;   // the host checks that they fit
   const uint32_t tiles_addr = (uint32_t)(uintptr_t)HBSA_AS3(lds) + (uint32_t)wave * 1024u;
-  float l2_next = INFINITY, dl_next = 0.f;   // threads 0-63: log2-domain log-sum-exp and delta of the tile's row
-  auto fetch = [&](int buf) {
+  const uint32_t row_addr = (uint32_t)(uintptr_t)HBSA_AS3(rowv);
+  // Loads of one tile per wavefront: LOADS of Q and of dO, and in wavefront 0 the two of the rows' values
+  auto fetch = [&](int buf) {   // the tile next_tile() has moved to
     const int valid = min(64, inf.rows - qoff);
     const int64_t row_first = inf.row_begin + qoff;
     const int hq = hk * p.ratio + r;
@@ -739,61 +759,90 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       bwd_dma16(dst + (uint32_t)(i * 4 * 1024), qsrc, rr * q_s32 + ld_chunk);
       bwd_dma16(dst + (uint32_t)(T::TILE_BYTES + i * 4 * 1024), gsrc, rr * do_s32 + ld_chunk);
     }
-    l2_next = INFINITY;   // rows past the block's end take no part: P = exp2(-inf) = 0
-    dl_next = 0.f;
-    if (threadIdx.x < valid) {
-      const float l = p.lse[(row_first + threadIdx.x) * p.nhead_q + hq];
-      l2_next = l == -INFINITY ? INFINITY : l * kLog2e;
-      dl_next = p.delta[(row_first + threadIdx.x) * p.nhead_q + hq];
+    if (wave == 0) {
+      const uint32_t rvoff = (uint32_t)min(lane, valid - 1) * 4u;
+      bwd_dma4(row_addr + (uint32_t)(buf * 512), p.lse2 + (int64_t)hq * p.total_q + row_first, rvoff);
+      bwd_dma4(row_addr + (uint32_t)(buf * 512 + 256), p.delta + (int64_t)hq * p.total_q + row_first, rvoff);
     }
   };
-  bool have = next_tile();
-  int buf = 0;
-  if (have) fetch(0);
-  while (have) {
-    const int first_q_pos = inf.q_pos + qoff, shift = inf.shift;
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wavefront's part of the tile has landed (and its lse, delta)
-    if (threadIdx.x < 64) {
-      rowv[buf * 128 + threadIdx.x] = l2_next;
-      rowv[buf * 128 + 64 + threadIdx.x] = dl_next;
+  // Everything loaded so far has arrived before the first tile is requested (see hbsa_bwd_dkv8_kernel).
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+  int n_ahead = 0;                               // tiles fetched and not computed on yet
+  int buf_f = 0, buf = 0;                        // buffer of the next fetch, and of the current tile
+  int fq_a = 0, fq_b = 0, va_a = 64, va_b = 64;  // first query position and row count of those tiles (a: the older)
+  bool more = next_tile();
+  auto issue = [&]() {   // fetches the tile next_tile() stands on and moves on
+    const int fq = inf.q_pos + qoff, va = min(64, inf.rows - qoff);
+    if (n_ahead == 0) { fq_a = fq; va_a = va; } else { fq_b = fq; va_b = va; }
+    fetch(buf_f);
+    buf_f = buf_f == 2 ? 0 : buf_f + 1;
+    ++n_ahead;
+    more = next_tile();
+  };
+  if (more) issue();
+  if (more) issue();
+  const int shift = inf.shift;
+  const int h_begin = shared_slots ? rows_half : 0, h_end = shared_slots ? rows_half + 1 : 2;   // 32-row halves of a tile
+  while (n_ahead > 0) {
+    const int first_q_pos = fq_a, valid = va_a;
+    // This wavefront's part of the tile has landed; the loads of the tile after it (a wavefront's loads return in
+    // order) may still be under way.
+    if (n_ahead >= 2) {
+      if (wave == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * LOADS + 2));
+      else __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * LOADS));
+    } else {
+      __builtin_amdgcn_s_waitcnt(0x0F70);
     }
-    __syncthreads();   // ... every wavefront's, and the other buffer has been read by all
+    __syncthreads();   // ... every wavefront's, and the buffer of the tile before has been read by all
     const char *q_t = lds + buf * 2 * T::TILE_BYTES, *g_t = q_t + T::TILE_BYTES;
     const float *lse_s = rowv + buf * 128, *dlt_s = lse_s + 64;
-    have = next_tile();
-    if (have) fetch(buf ^ 1);   // on its way while this tile is computed on
-    buf ^= 1;
+    buf = buf == 2 ? 0 : buf + 1;
+    fq_a = fq_b;
+    va_a = va_b;
+    --n_ahead;
+    if (more) issue();   // two tiles ahead
     if (!active) continue;
-    // rows of the tile from first_vis on see this lane's key (causal); lanes past the block's keys see nothing
+    // rows first_vis .. valid - 1 of the tile see this lane's key (what lanes without a key sum up is not stored);
+    // comparisons and selects are left out where all 64 rows see all of the wavefront's keys
     int first_vis = 0;
     if (p.causal) first_vis = max(0, key_pos - shift - first_q_pos);
-    if (l32 >= nrows) first_vis = 64;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (shared_slots && h != rows_half) continue;   // the slot's other wavefront takes these rows
+    const bool diagonal = p.causal && wave_key_max - shift - first_q_pos > 0;
+#pragma unroll 1
+    for (int h = h_begin; h < h_end; ++h) {
+      // P first, its product with dO next, then dP: half as many values are alive at a time as with both at once
       const f32x16 s = bwd_rows_times_frag<D, E>(q_t, h, kf, lane);
+      float e[16];
+      auto form_p = [&](auto short_, auto diagonal_) {
+        const int left = valid - 32 * h - 4 * g32, before = first_vis - 32 * h - 4 * g32;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          const f32x4 l4 = *(const f32x4 *)(lse_s + 32 * h + 8 * a + 4 * g32);
+#pragma unroll
+          for (int bq = 0; bq < 4; ++bq) {
+            float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * a + bq], p.c, -l4[bq]));
+            if constexpr (decltype(short_)::value) pv = 8 * a + bq < left ? pv : 0.f;   // (rows past the end repeat the last one)
+            if constexpr (decltype(diagonal_)::value) pv = 8 * a + bq >= before ? pv : 0.f;
+            e[4 * a + bq] = pv;
+          }
+        }
+      };
+      if (diagonal) form_p(std::true_type{}, std::true_type{});
+      else if (valid < 64) form_p(std::true_type{}, std::false_type{});
+      else form_p(std::false_type{}, std::false_type{});
+      short8v lo, hi;
+      bwd_pack<E>(e, lo, hi);
       const f32x16 dp = bwd_rows_times_frag<D, E>(g_t, h, vf, lane);
-      float ep[16], ed[16];
+      bwd_transposed_times_packed<D, E>(g_t, 2 * h, lo, lane, acc_v);
+      bwd_transposed_times_packed<D, E>(g_t, 2 * h + 1, hi, lane, acc_v);
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
-        const int rr0 = 32 * h + 8 * a + 4 * g32;
-        const f32x4 l4 = *(const f32x4 *)(lse_s + rr0), d4 = *(const f32x4 *)(dlt_s + rr0);
+        const f32x4 d4 = *(const f32x4 *)(dlt_s + 32 * h + 8 * a + 4 * g32);
 #pragma unroll
-        for (int bq = 0; bq < 4; ++bq) {
-          const int i = 4 * a + bq;
-          const bool vis = rr0 + bq >= first_vis;   // rows past the block's end carry lse = +inf, hence P = 0
-          const float pv = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], p.c, -l4[bq])) : 0.f;
-          ep[i] = pv;
-          ed[i] = pv * (dp[i] - d4[bq]);
-        }
+        for (int bq = 0; bq < 4; ++bq) e[4 * a + bq] *= dp[4 * a + bq] - d4[bq];
       }
-      short8v plo, phi, dlo, dhi;
-      bwd_pack<E>(ep, plo, phi);
-      bwd_pack<E>(ed, dlo, dhi);
-      bwd_transposed_times_packed<D, E>(g_t, 2 * h, plo, lane, acc_v);
-      bwd_transposed_times_packed<D, E>(g_t, 2 * h + 1, phi, lane, acc_v);
-      bwd_transposed_times_packed<D, E>(q_t, 2 * h, dlo, lane, acc_k);
-      bwd_transposed_times_packed<D, E>(q_t, 2 * h + 1, dhi, lane, acc_k);
+      bwd_pack<E>(e, lo, hi);
+      bwd_transposed_times_packed<D, E>(q_t, 2 * h, lo, lane, acc_k);
+      bwd_transposed_times_packed<D, E>(q_t, 2 * h + 1, hi, lane, acc_k);
     }
   }
   if (shared_slots) {   // the wavefronts of the lower rows hand their sums to those of the upper rows: [slot][register][lane] floats
@@ -871,16 +920,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = wave & 3, role = wave >> 2;   // 32-key slot of the workgroup; 0: the P wavefront, 1: the dS wavefront
   const int g32 = lane >> 5, l32 = lane & 31;
-  // With a multiple of eight kv heads the grid is one-dimensional and workgroup ids, which go round the
-  // eight XCDs (each with its own L2), are decoded so that XCD x works on the heads x, x + 8, ...: the
-  // workgroups that share an L2 then walk the k blocks of one head in order and read the Q and dO rows of
-  // one sequence at a time, and every XCD has the same amount of work whatever the sequence lengths.
-  int hk = blockIdx.y, bx = blockIdx.x;
-  if (p.xcd_heads) {
-    const unsigned t = blockIdx.x >> 3, per_head = (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u);
-    hk = (int)(blockIdx.x & 7u) + 8 * (int)(t / per_head);
-    bx = (int)(t % per_head);
-  }
+  int hk, bx;
+  bwd_decode_grid(p, (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u), hk, bx);
   int part = 0;
   const int per_part = p.nkb * p.nsub_k;
   if constexpr (PARTS) {
@@ -924,8 +965,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   int qb = p.cu_num_q_block[b] - 1, r = 0, qoff = 0;
   int qb_end = p.cu_num_q_block[b + 1];
   const int qb_begin = p.cu_num_q_block[b];
-  int kept_base = qb_begin - 64;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
-  int r_end = p.ratio;   // heads of the q block that are the part's
+  int kept_base = qb_end;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
+  int qb_low = qb_begin, r_end = p.ratio;   // the part's first q block, and the q block's heads that are the part's
   uint64_t kept = 0;
   QBlockInfo inf = {};
   int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
@@ -944,8 +985,9 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
                               share.qb_first, share.r_first, share.r_last_end, 0};
     }
     __syncthreads();
+    qb_low = share.qb_first;
     qb_end = share.qb_last + 1;
-    kept_base = share.qb_first - 64;
+    kept_base = qb_end;
   }
   auto tile_reaches = [&]() {
     return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
@@ -961,15 +1003,16 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
         }
       }
       while (kept == 0) {   // one load per 64 q blocks: lane i looks at q block kept_base + i; waited for here so that no other path waits
-        kept_base += 64;
-        if (kept_base >= qb_end) return false;
+        kept_base -= 64;
+        if (kept_base + 63 < qb_low) return false;
         uint32_t word = 0;
-        if (kept_base + lane < qb_end) word = p.bits[((size_t)hk * p.nqb + kept_base + lane) * p.wpr + (kbl >> 5)];
+        if (kept_base + lane >= qb_low && kept_base + lane < qb_end) word = p.bits[((size_t)hk * p.nqb + kept_base + lane) * p.wpr + (kbl >> 5)];
         __builtin_amdgcn_s_waitcnt(0x0F70);
         kept = __ballot((word >> (kbl & 31)) & 1u);
       }
-      qb = kept_base + __builtin_ctzll(kept);
-      kept &= kept - 1;
+      const int at = 63 - __builtin_clzll(kept);
+      qb = kept_base + at;
+      kept &= ~(1ull << at);
       // the q block's geometry follows from the sequence's (no load on this path)
       inf.q_pos = (qb - qb_begin) * p.qbs;
       inf.row_begin = seq_row0 + inf.q_pos;
@@ -1014,9 +1057,9 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       }
     }
     if (wave == 0) {   // the rows' log-sum-exp and delta, one row per lane (rows past the block's end repeat its last row)
-      const uint32_t rvoff = (uint32_t)min(lane, valid - 1) * (uint32_t)(p.nhead_q * 4);
-      bwd_dma4(row_addr + (uint32_t)(gi * 256), p.lse2 + row_first * p.nhead_q + hq, rvoff);
-      bwd_dma4(row_addr + (uint32_t)(768 + qi * 256), p.delta + row_first * p.nhead_q + hq, rvoff);
+      const uint32_t rvoff = (uint32_t)min(lane, valid - 1) * 4u;
+      bwd_dma4(row_addr + (uint32_t)(gi * 256), p.lse2 + (int64_t)hq * p.total_q + row_first, rvoff);
+      bwd_dma4(row_addr + (uint32_t)(768 + qi * 256), p.delta + (int64_t)hq * p.total_q + row_first, rvoff);
     }
   };
   // this lane's 2 x 16 bytes of a (tile parity, slot, half) record of P
@@ -1089,7 +1132,6 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
           const uint32_t q_t = lds_base + (uint32_t)(q_now * T::TILE_BYTES), g_t = lds_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
           int first_vis = 0;   // rows of the tile from first_vis on see this lane's key (causal)
           if (p.causal) first_vis = max(0, key_pos - shift - first_q_pos);
-          if (l32 >= nrows) first_vis = 64;
           // S = Q K^T of both halves of the tile, their steps in turn (read i: half i % 2, step i / 2)
           auto chain_read = [&](auto i_) {
             constexpr int i = decltype(i_)::value;
@@ -1111,7 +1153,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
           // edge: some row of the tile does not see some key of the wavefront (the causal diagonal, a slot with
           // fewer than 32 keys, a tile with fewer than 64 rows); elsewhere the per-element comparison and select
           // are left out.
-          const bool edge = nrows < kWaveRows || valid < 64 || (p.causal && wave_key_max - shift - first_q_pos > 0);
+          const bool edge = valid < 64 || (p.causal && wave_key_max - shift - first_q_pos > 0);
           auto half = [&](auto h_) {
             constexpr int h = decltype(h_)::value;
             float ep[16];
@@ -1225,7 +1267,7 @@ template <int D, typename E, bool PARTS_Q, bool PARTS_K>
 int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   using T = BwdTile<D>;
   // LDS: the dQ kernel's three K and two V tiles; the dK/dV kernels' tile buffers, P records and row values
-  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? 9 * T::TILE_BYTES + 2048 : 4 * T::TILE_BYTES + 1024;
+  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? 9 * T::TILE_BYTES + 2048 : 6 * T::TILE_BYTES + 1536;
   if constexpr (lds_dkv > 48 * 1024) {
     static thread_local bool raised[kMaxDevices] = {};
     int dev = 0;
@@ -1245,8 +1287,8 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
   }
   const unsigned q_wgs = (unsigned)(bp.nqb * bp.nsub * (PARTS_Q ? bp.parts_q : 1));
   const unsigned k_wgs = (unsigned)(num_k_block * bp.nsub_k * (PARTS_K ? bp.parts_k : 1));
-  const dim3 q_grid = bp.xcd_heads ? dim3(q_wgs * (unsigned)nhead_k) : dim3(q_wgs, (unsigned)nhead_k);
-  const dim3 kv_grid = bp.xcd_heads ? dim3(k_wgs * (unsigned)nhead_k) : dim3(k_wgs, (unsigned)nhead_k);
+  const dim3 q_grid = bp.flat_grid ? dim3(q_wgs * (unsigned)nhead_k) : dim3(q_wgs, (unsigned)nhead_k);
+  const dim3 kv_grid = bp.flat_grid ? dim3(k_wgs * (unsigned)nhead_k) : dim3(k_wgs, (unsigned)nhead_k);
   hipLaunchKernelGGL((hbsa_bwd_dq_kernel<D, E, PARTS_Q>), q_grid, dim3(kThreads), lds_dq, stream, bp);
   if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K>), kv_grid, dim3(512), lds_dkv, stream, bp);
   else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);

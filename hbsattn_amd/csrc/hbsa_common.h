@@ -316,8 +316,9 @@ struct BwdParams {
   const char *q, *k, *v, *out, *dout;
   char *dq, *dk, *dv;
   const float *lse;           // [total_q, nhead_q], contiguous
-  float *delta;               // [total_q, nhead_q], contiguous: rowsum(dO * O), written by the dQ kernel, read by the dK/dV kernels
-  float *lse2;                // [total_q, nhead_q]: lse * log2(e), +inf where lse is -inf; written by the dQ kernel for the D = 128 dK/dV kernel
+  // [nhead_q, total_q]: what the dQ kernel leaves for the dK/dV kernels, whose tiles are consecutive rows of one q head
+  float *delta;               // rowsum(dO * O)
+  float *lse2;                // lse * log2(e), +inf where lse is -inf
   const QBlockInfo *info;
   const uint32_t *bits;
   const int32_t *cu_k, *cu_num_q_block, *cu_num_k_block;
@@ -331,6 +332,8 @@ struct BwdParams {
   // Items cut into parts (see BwdCut): at most parts_q k block ranges a dQ item, of min_blocks_q k blocks at least, and parts_k
   // ranges of (q block, q head) pairs a dK/dV item, of min_units_k pairs at least; 1: whole
   int32_t parts_q, min_blocks_q, parts_k, min_units_k;
+  int32_t total_q;
+  int32_t flat_grid;     // one-dimensional grids (bwd_decode_grid)
   float *parts;          // partial accumulators, shared by the two launches
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
 };
