@@ -146,6 +146,7 @@ struct FwdParams {
   FastDiv div_items;     // division by the number of items
   int32_t parts_last;    // workgroups are numbered by part first (else: the parts of an item are neighbours)
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
+  int32_t split;         // host side only: parts of the split over key blocks that pay (fwd_split)
 };
 
 // Boundaries of one sequence of the packed batch, as read from the caller's device arrays.

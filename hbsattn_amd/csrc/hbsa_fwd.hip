@@ -353,29 +353,64 @@ inline bool fwd_packs(int ratio, int q_block_size) { return ratio > 1 && q_block
 inline int fwd_slots(int ratio, int q_block_size, bool packed) {
   return packed ? (ratio * q_block_size + kWaveRows - 1) / kWaveRows : ratio * ((q_block_size + kWaveRows - 1) / kWaveRows);
 }
-// Wavefronts per workgroup of the 16-bit attention kernel for an item of `slots` wave slots: eight when the
-// item has more than four slots, so that one workgroup stages its K/V tiles once (head dims 64 and 128; the
-// fp32 kernel always has four), unless the item's last workgroup of eight would be at most half full: then
-// workgroups of four, none of them with idle wavefronts (measured at 20 slots, head dim 64: 0.365 -> 0.33 ms).
-inline int fwd_wavefronts(int slots, int headdim, bool f32_exact) {
-  if (f32_exact || slots <= 4 || headdim < 64 || headdim > 128) return 4;
-  const int in_last = slots % 8;
-  return (in_last >= 1 && in_last <= 4) ? 4 : 8;
-}
-
-// Split over key blocks pays when the work items cannot fill the device: fewer than one per CU.
-// Returns the number of parts (1 = no split) for the current device.
-int split_parts(long long items, int num_k_block) {
+int device_cus() {
   static thread_local int cus_of[kMaxDevices] = {};
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 1;
-  if (cus_of[dev] == 0 && hipDeviceGetAttribute(&cus_of[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 1;
-  const int cus = cus_of[dev];
-  if (items <= 0 || items > cus) return 1;
-  long long parts = std::min<long long>(32, (2LL * cus) / items);
-  parts = std::min<long long>(parts, num_k_block / 8);     // a part should still have a few k blocks
-  return parts < 2 ? 1 : (int)parts;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  if (cus_of[dev] == 0 && hipDeviceGetAttribute(&cus_of[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus_of[dev] = 0;
+  return cus_of[dev];
+}
+
+// Split of `items` equal items over key blocks where `places` workgroups run at once: the number of parts with the fewest
+// rounds of the device, counted in whole items, plus what a part costs (its fp32 partial results are written and merged;
+// and the split is four launches in place of one).  A problem of chunks, its keys many times its queries, has items of
+// about one weight, so the count is right and parts of 2048 keys pay; elsewhere the causal order evens the rounds out and
+// only a problem that leaves places empty is split, into parts of 8192 keys.  Measured, us, with the split as it was before
+// (2 * CUs / items parts) and as here: chunks of 512 on 32000 keys, 32 / 8 heads of 128, 143 -> 122; 2 x 300 .. 512 on 65000
+// 285 -> 258; 4 x 700 .. 1500 on 30000 .. 60000, 16 / 2 heads, 487 -> 394; 2 x 64 .. 128 on 8000 .. 16000 69 -> 51; sequences by
+// themselves, 32 / 8 heads, 1 x 1024 33 -> 27, 1 x 2048 67 -> 40; 1 x 4096, 8 / 1 heads, 59 -> 45.
+// (At most five items for eight places of workgroups of four: beyond that they stay one launch.)
+int split_parts(long long items, int nw, int headdim, int num_k_block, long long keys, long long queries) {
+  const bool chunks = keys >= 4 * queries;
+  const long long cus = device_cus(), places = nw == 8 || headdim > 192 ? cus : 2 * cus;
+  if (items <= 0 || cus <= 0 || items > (nw == 8 ? (chunks ? 2 * cus : cus) : 5 * cus / 4)) return 1;
+  const long long most = std::min<long long>(std::min<long long>(32, num_k_block / 8), keys / (chunks ? 2048 : 8192));
+  const double part = 0.05 * std::max<double>((double)items, 1.0) / (double)places;
+  double best = (double)((items + places - 1) / places) + part;
+  int parts = 1;
+  for (int n = 2; n <= most; ++n) {
+    const double cost = (double)((items * n + places - 1) / places) / n + part * n;
+    if (cost < best) {
+      best = cost;
+      parts = n;
+    }
+  }
+  return parts;
+}
+
+// Wavefronts per workgroup of the 16-bit attention kernel for an item of `slots` wave slots, and its split over key blocks.
+// `keys` and `queries` are the problem's, up to whole blocks.
+// Eight wavefronts stage an item's K/V tiles once where workgroups of four stage them twice, but only one such workgroup
+// fits a CU, and it waits for its own barriers and items.  At head dim 64 three workgroups of four do fit and are faster
+// everywhere (16 / 4 heads of 64, 6 x 300 .. 4000 tokens 78 -> 74 us; 32 / 8 heads, 4 x 500 .. 3000 81 -> 61, 8 x 2048 .. 8000 670 ->
+// 591; 32 / 4 heads, 4 x 8000 322 -> 292).  At head dim 128 eight are faster by 3 to 8 % when the items fill the CUs an even
+// number of times (the order of the items pairs rounds), or are many: 8 x 500 .. 3000, 8 items a CU, 198 against 206.
+// Few items that do not come out at whole pairs of rounds take four: 1.9 items a CU 62 -> 59, 2.5 40.7 -> 37.9, 3.0 145 ->
+// 134, 3.7 101 -> 99, 3.8 110 -> 95, 4.8 98 -> 87, 5.1 140 -> 124; at 2.0 82 -> 83, at 4.0 205 -> 220, which stay at eight.
+// An item whose last workgroup of eight would be at most half full has none with idle wavefronts as fours.
+struct FwdSplit {
+  int nw, parts;
+};
+FwdSplit fwd_split(int slots, int headdim, bool f32_exact, long long item_groups, int num_k_block, long long keys, long long queries) {
+  const long long cus = device_cus(), fours = item_groups * ((slots + 3) / 4), eights = item_groups * ((slots + 7) / 8);
+  if (f32_exact) return {4, 1};
+  const int in_last = slots % 8;
+  if (headdim == 128 && slots > 4 && !(in_last >= 1 && in_last <= 4)) {
+    const int parts = split_parts(eights, 8, headdim, num_k_block, keys, queries);
+    const long long room = 2 * cus * ((eights + 2 * cus - 1) / std::max(1ll, 2 * cus));
+    if (parts > 1 || cus == 0 || eights >= 6 * cus || 32 * eights >= 31 * room) return {8, parts};
+  }
+  return {4, split_parts(fours, 4, headdim, num_k_block, keys, queries)};
 }
 // split area: nparts bit row copies | nparts partial outputs | nparts partial log-sum-exps, each array packed
 inline size_t split_bits_bytes(int parts, int nhead_k, int num_q_block, int num_k_block) {
@@ -388,14 +423,6 @@ inline size_t split_bytes(int parts, int total_q, int nhead_q, int nhead_k, int 
   if (parts < 2) return 0;
   return split_bits_bytes(parts, nhead_k, num_q_block, num_k_block) + split_out_bytes(parts, total_q, nhead_q, headdim) +
          align_up((size_t)parts * total_q * nhead_q * 4, 256);
-}
-
-int device_cus() {
-  static thread_local int cus_of[kMaxDevices] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
-  if (cus_of[dev] == 0 && hipDeviceGetAttribute(&cus_of[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus_of[dev] = 0;
-  return cus_of[dev];
 }
 
 // An odd number of parts (see decode_max_parts for why)
@@ -482,7 +509,10 @@ void fill_shape(FwdParams &fp, int nhead_q, int nhead_k, int headdim, int num_q_
   fp.wps = (q_block_size + kWaveRows - 1) / kWaveRows;
   fp.pack = cols || f32_exact || (may_pack && fwd_packs(fp.ratio, q_block_size)) ? 1 : 0;
   const int slots = fwd_slots(fp.ratio, q_block_size, fp.pack != 0);
-  fp.nw = cols ? 4 : fwd_wavefronts(slots, headdim, f32_exact);
+  const FwdSplit split = fwd_split(slots, headdim, f32_exact, (long long)nhead_k * num_q_block, num_k_block,
+                                   (long long)num_k_block * k_block_size, (long long)num_q_block * q_block_size);
+  fp.nw = split.nw;
+  fp.split = split.parts;
   fp.ncol = headdim / 8;
   fp.max_parts = 1;
   fp.min_blocks = 1;
@@ -623,12 +653,12 @@ int g_onepass = [] {
 }();
 
 // The launch record a call would use in the one-launch form, nullptr when the form does not apply to it.
-Sched *onepass_record(int32_t dtype, int32_t batch, int32_t total_k, int32_t headdim, int32_t num_k_block, int32_t k_block_size,
-                      int64_t mask_kblk_stride, long long items, hipStream_t st) {
+Sched *onepass_record(int32_t dtype, int32_t batch, int32_t total_k, int32_t headdim, int32_t k_block_size,
+                      int64_t mask_kblk_stride, long long items, int split, hipStream_t st) {
   if (!g_onepass || (dtype != HBSA_DTYPE_BF16 && dtype != HBSA_DTYPE_F16)) return nullptr;
   if (mask_kblk_stride != 1 || batch < 1 || batch >= kSeqCap) return nullptr;
   if (items <= 0 || items > 0x7fffffffLL) return nullptr;
-  if (split_parts(items, num_k_block) > 1) return nullptr;
+  if (split > 1) return nullptr;
   if (!g_deterministic && k_block_size % kTileKeys == 0 && 2ll * total_k * headdim * 2 >= g_walk_min_bytes) return nullptr;
   return is_capturing(st) ? nullptr : stream_sched_of(st);
 }
@@ -651,7 +681,7 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, false,
              true, cols);
   const long long items = (long long)nhead_k * num_q_block * fp.nsub;
-  Sched *sched = onepass_record(dtype, batch, total_k, headdim, num_k_block, k_block_size, strides[10], items, st);
+  Sched *sched = onepass_record(dtype, batch, total_k, headdim, k_block_size, strides[10], items, fp.split, st);
   if (sched == nullptr) return kNotOnePass;
 
   fp.q = (const char *)q; fp.k = (const char *)k; fp.v = (const char *)v; fp.out = (char *)out;
@@ -762,10 +792,10 @@ int hbsa_fwd_launches(int32_t dtype, int32_t batch, int32_t total_k, int32_t nhe
       k_block_size <= 0 || (headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256))
     return 2;
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, fwd_packs(nhead_q / nhead_k, q_block_size));   // as try_onepass
-  const int nw = fwd_wavefronts(slots, headdim, false);
-  const long long items = (long long)nhead_k * num_q_block * ((slots + nw - 1) / nw);
-  return onepass_record(dtype, batch, total_k, headdim, num_k_block, k_block_size, mask_kblk_stride, items,
-                        (hipStream_t)stream) != nullptr ? 1 : 2;
+  const FwdSplit split = fwd_split(slots, headdim, false, (long long)nhead_k * num_q_block, num_k_block,
+                                   (long long)num_k_block * k_block_size, (long long)num_q_block * q_block_size);
+  const long long items = (long long)nhead_k * num_q_block * ((slots + split.nw - 1) / split.nw);
+  return onepass_record(dtype, batch, total_k, headdim, k_block_size, mask_kblk_stride, items, split.parts, (hipStream_t)stream) != nullptr ? 1 : 2;
 }
 
 int hbsa_set_onepass(int on) {
@@ -859,9 +889,12 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
     return parts_room(decode_max_parts(items, num_k_block), decode_part_bytes(total_q, nhead_q, headdim), items);
   }
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, false);
-  const int nw = fwd_wavefronts(slots, headdim, false);
-  const long long items = (long long)nhead_k * num_q_block * ((slots + nw - 1) / nw);
-  return split_bytes(split_parts(items, num_k_block), total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
+  // (without the k block size the keys are not known: the room for the most parts any size can get)
+  int parts = 1;
+  for (int kbs = 16; kbs <= 2048; kbs *= 2)
+    parts = std::max(parts, fwd_split(slots, headdim, false, (long long)nhead_k * num_q_block, num_k_block, (long long)num_k_block * kbs,
+                                      (long long)num_q_block * q_block_size).parts);
+  return split_bytes(parts, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
 }
 
 size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t headdim,
@@ -997,7 +1030,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
   fp.total_q = total_q; fp.nhead_q = nhead_q;
   char *split_area = (char *)workspace + need;
   if (!f32_exact) {
-    const int parts = split_parts(items, num_k_block);
+    const int parts = fp.split;
     if (parts > 1 && workspace_bytes >= need + split_bytes(parts, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block))
       fp.nparts = parts;
   }

@@ -180,7 +180,8 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // zero-padded copies of q, k, v and a copy of the output.
   // NW: wavefronts (wave slots) of a workgroup, 4 or 8.  Eight are used when the q heads of a GQA group
   // and the 32-row slices of a q block give an item more than four wave slots: one workgroup per CU then
-  // stages every K/V tile once for all of them instead of two workgroups staging it each.
+  // stages every K/V tile once for all of them instead of two workgroups staging it each (D = 128 only, and
+  // where the items fill the device: see fwd_split).
   constexpr int RB = D * 2;            // row bytes
   constexpr int CPR = RB / 16;         // 16-byte chunks per row
   // Keys per tile.  At head dims 160 and 192 tiles of 32 keys let two workgroups share a CU (their LDS, and the
@@ -1259,7 +1260,7 @@ int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
 template <int D, typename E, bool OUT32>
 int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream) {
   const bool extras = fp.walk != 0 || fp.nparts > 1 || fp.lse != nullptr;
-  if constexpr (D >= 64 && D <= 128) {
+  if constexpr (D == 128) {
     if (fp.nw == 8)
       return extras ? launch_fwd_nw<D, E, OUT32, 8, true>(fp, items, stream) : launch_fwd_nw<D, E, OUT32, 8, false>(fp, items, stream);
   }
@@ -1268,7 +1269,7 @@ int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream) {
 // the one-launch form (16-bit tensors, none of the extras)
 template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream) {
-  if constexpr (D >= 64 && D <= 128) {
+  if constexpr (D == 128) {
     if (fp.nw == 8)
       return fp.pack ? launch_fwd_nw<D, E, false, 8, false, true, true>(fp, items, stream)
                      : launch_fwd_nw<D, E, false, 8, false, true, false>(fp, items, stream);
