@@ -410,8 +410,11 @@ struct ItemParts {
 __device__ __forceinline__ void part_store(float *at, float v) {
   __hip_atomic_store((uint32_t *)at, __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void part_store4(float *at, f32x4 v) {   // 16-byte aligned
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(at), "v"(v) : "memory");
+// 16-byte aligned.  The two wait states belong to the store: it still reads its data registers when the next instruction is
+// issued, and the compiler, which keeps vector instructions from writing them too early after its own wide stores, does not
+// know this one (measured without them: the first registers of a part, lanes 12-15 of every 16, replaced by what came next).
+__device__ __forceinline__ void part_store4(float *at, f32x4 v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(at), "v"(v) : "memory");
 }
 __device__ __forceinline__ void parts_arrived() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 __device__ __forceinline__ void parts_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }

@@ -1,0 +1,22 @@
+"""What the compiler cannot check in the kernels' inline assembly."""
+import glob
+import os
+import re
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hbsattn_amd", "csrc")
+
+
+def test_wide_stores_keep_their_data_registers_for_two_wait_states():
+    """A store of more than 64 bits reads its data registers after it was issued; a vector instruction may write them two
+    wait states later at the earliest, and the compiler counts those for its own stores only."""
+    found = 0
+    for path in sorted(glob.glob(os.path.join(CSRC, "*"))):
+        if not path.endswith((".h", ".hip")):
+            continue
+        with open(path) as f:
+            for asm in re.findall(r'asm volatile\((.*?)\);', f.read(), re.S):
+                for store in re.finditer(r"(?:global|buffer|flat)_store_dwordx[34][^\\\"]*((?:\\n\\t[^\\\"]*)?)", asm):
+                    found += 1
+                    wait = re.search(r"s_nop (\d+)", store.group(1))
+                    assert wait and int(wait.group(1)) >= 1, f"{os.path.basename(path)}: {store.group(0)}"
+    assert found   # (the partial results of items cut into parts)
