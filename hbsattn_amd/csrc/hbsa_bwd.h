@@ -904,7 +904,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
 // and two tiles ahead (one workgroup per CU has nobody else to cover its waits for memory): four Q buffers
 // (tile t - 1 is still read while tile t + 2 arrives), three for dO, and with them three and four sets of the
 // rows' log-sum-exp and delta, which wavefront 0 loads into LDS the same way.
-template <typename E, bool PARTS>
+template <typename E, bool PARTS, bool SHARED>
 __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   constexpr int D = 128;
   using T = BwdTile<D>;
@@ -918,7 +918,16 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int slot = wave & 3, role = wave >> 2;   // 32-key slot of the workgroup; 0: the P wavefront, 1: the dS wavefront
+  const int slot = wave & 3, role = wave >> 2;   // pair of wavefronts; 0: the P wavefront, 1: the dS wavefront
+  // SHARED (k blocks of up to 64 keys): pairs 0 and 2, 1 and 3 work on the same 32 keys, the first ones on the upper 32 rows
+  // of every tile and the others on the lower ones, whose sums are added through LDS at the end.  Otherwise pair i has keys
+  // 32 i .. 32 i + 31 and both halves of the tile.
+  // (with four of eight wavefronts idle, dQ + dK/dV, 64-key blocks: 6 x 1500 .. 4000 tokens, 32 / 8 heads, 801 -> 678 us;
+  // 4 x 4096, 32 heads, 1013 -> 954; 48-key blocks, 4 x 2000 .. 6000, 16 heads, 848 -> 770.  With the chain in two accumulators
+  // 692, 971 and 785.)
+  constexpr int NH = SHARED ? 1 : 2;                 // halves of a tile a wavefront works on
+  const int key_slot = SHARED ? slot & 1 : slot;
+  const int first_row = SHARED ? 32 * (slot >> 1) : 0;   // ... from this row on
   const int g32 = lane >> 5, l32 = lane & 31;
   int hk, bx;
   bwd_decode_grid(p, (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u), hk, bx);
@@ -937,7 +946,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   const int k0 = p.cu_k[b], klen = p.cu_k[b + 1] - k0;
   const int krows = min(p.kbs, klen - kbl * p.kbs);
   const int wg_row0 = sub * 4 * kWaveRows;                 // first key of the workgroup inside the block
-  const int row0 = wg_row0 + slot * kWaveRows;
+  const int row0 = wg_row0 + key_slot * kWaveRows;
   const int nrows = min(kWaveRows, krows - row0);
   const bool active = nrows > 0;
   const int key_pos = kbl * p.kbs + min(row0 + l32, krows - 1);
@@ -1095,9 +1104,9 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   if (more) issue();
   bool prev = false;        // the tile before the current one exists: its dK part is still due
   int qi = 0, gi = 0, par = 0;   // Q buffer, dO buffer and parity of the current tile
-  f32x16 dp_prev[2];        // dS wavefront: dP of the previous tile, both halves
+  f32x16 dp_prev[NH];       // dS wavefront: dP of the previous tile
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < NH; ++h)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dp_prev[h][i] = 0.f;
   const int shift = inf.shift;
@@ -1124,28 +1133,29 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       // Operand reads are issued by hand (BwdOperandOffsets): PF reads of a pair of chains under way ahead of
       // their products, the transposing reads of a key group before the vector ALU work that precedes their
       // products.  The counts in the waits name only reads that every path issues.
-      constexpr int PF = 4, NC = 2 * T::KSTEPS;
+      constexpr int PF = 4, NC = NH * T::KSTEPS;
+      const uint32_t half_base = lds_base + (uint32_t)(first_row * T::RB);
       short8v rb[PF];
       short4v tb[2][2 * T::DT];
       if constexpr (ROLE == 0) {
         if (had) {   // ---- P wavefront, current tile
-          const uint32_t q_t = lds_base + (uint32_t)(q_now * T::TILE_BYTES), g_t = lds_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
+          const uint32_t q_t = half_base + (uint32_t)(q_now * T::TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
           int first_vis = 0;   // rows of the tile from first_vis on see this lane's key (causal)
           if (p.causal) first_vis = max(0, key_pos - shift - first_q_pos);
-          // S = Q K^T of both halves of the tile, their steps in turn (read i: half i % 2, step i / 2)
+          // S = Q K^T, the steps of the halves in turn (read i: half i % NH, step i / NH)
           auto chain_read = [&](auto i_) {
             constexpr int i = decltype(i_)::value;
-            rb[i % PF] = lds_read_b128<(i & 1) * 32 * T::RB>(off.rows[i >> 1] + q_t);
+            rb[i % PF] = lds_read_b128<(i % NH) * 32 * T::RB>(off.rows[i / NH] + q_t);
           };
           static_for<0, PF>(chain_read);
-          f32x16 sv[2];
+          f32x16 sv[NH];
 #pragma unroll
-          for (int i = 0; i < 16; ++i) { sv[0][i] = 0.f; sv[1][i] = 0.f; }
+          for (int i = 0; i < 16; ++i) { sv[0][i] = 0.f; sv[NH - 1][i] = 0.f; }
           static_for<0, NC>([&](auto i_) {
             constexpr int i = decltype(i_)::value;
             constexpr int ahead = (NC - 1 - i) < (PF - 1) ? (NC - 1 - i) : (PF - 1);
             lds_wait1<ahead>(rb[i % PF]);
-            sv[i & 1] = E::mfma(rb[i % PF], frag[i >> 1], sv[i & 1]);
+            sv[i % NH] = E::mfma(rb[i % PF], frag[i / NH], sv[i % NH]);
             if constexpr (i + PF < NC) chain_read(std::integral_constant<int, i + PF>{});
           });
           bwd_issue_transposed<D, 0>(off, g_t, tb[0]);
@@ -1160,7 +1170,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
             auto form_p = [&](auto edge_) {
 #pragma unroll
               for (int a = 0; a < 4; ++a) {
-                const int rr0 = 32 * h + 8 * a + 4 * g32;
+                const int rr0 = first_row + 32 * h + 8 * a + 4 * g32;
                 const f32x4 l4 = *(const f32x4 *)(lse_s + gi * 64 + rr0);
 #pragma unroll
                 for (int bq = 0; bq < 4; ++bq) {
@@ -1178,19 +1188,18 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
             *(short8v *)(p_mine + par * 16384 + h * 2048 + 1024) = phi;
             bwd_wait_transposed<D, 2 * T::DT>(tb[0]);
             bwd_transposed_products<D, E>(tb[0], plo, acc);
-            if constexpr (h == 0) bwd_issue_transposed<D, 2>(off, g_t, tb[0]);
-            bwd_wait_transposed<D, (h == 0 ? 2 * T::DT : 0)>(tb[1]);
+            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 2>(off, g_t, tb[0]);
+            bwd_wait_transposed<D, (h + 1 < NH ? 2 * T::DT : 0)>(tb[1]);
             bwd_transposed_products<D, E>(tb[1], phi, acc);
-            if constexpr (h == 0) bwd_issue_transposed<D, 3>(off, g_t, tb[1]);
+            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 3>(off, g_t, tb[1]);
           };
-          half(std::integral_constant<int, 0>{});
-          half(std::integral_constant<int, 1>{});
+          static_for<0, NH>(half);
         }
       } else {
-        const uint32_t q_t = lds_base + (uint32_t)(q_before * T::TILE_BYTES), g_t = lds_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
+        const uint32_t q_t = half_base + (uint32_t)(q_before * T::TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
         auto chain_read = [&](auto i_) {   // dP = dO V^T of both halves of the current tile, as above
           constexpr int i = decltype(i_)::value;
-          rb[i % PF] = lds_read_b128<(i & 1) * 32 * T::RB>(off.rows[i >> 1] + g_t);
+          rb[i % PF] = lds_read_b128<(i % NH) * 32 * T::RB>(off.rows[i / NH] + g_t);
         };
         if (prev) {   // ---- dS wavefront, the tile before: dS = P * (dP - delta), dK^T += Q^T dS
           bwd_issue_transposed<D, 0>(off, q_t, tb[0]);
@@ -1202,7 +1211,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
                                  *(const u32x4 *)(p_mine + (par ^ 1) * 16384 + h * 2048 + 1024)};
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
-              const int rr0 = 32 * h + 8 * a + 4 * g32;
+              const int rr0 = first_row + 32 * h + 8 * a + 4 * g32;
               const f32x4 d4 = *(const f32x4 *)(dlt_s + q_before * 64 + rr0);
 #pragma unroll
               for (int bq = 0; bq < 4; ++bq) {
@@ -1215,23 +1224,22 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
             bwd_pack<E>(ed, dlo, dhi);
             bwd_wait_transposed<D, 2 * T::DT>(tb[0]);
             bwd_transposed_products<D, E>(tb[0], dlo, acc);
-            if constexpr (h == 0) bwd_issue_transposed<D, 2>(off, q_t, tb[0]);
-            bwd_wait_transposed<D, (h == 0 ? 2 * T::DT : 0)>(tb[1]);
+            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 2>(off, q_t, tb[0]);
+            bwd_wait_transposed<D, (h + 1 < NH ? 2 * T::DT : 0)>(tb[1]);
             bwd_transposed_products<D, E>(tb[1], dhi, acc);
-            if constexpr (h == 0) bwd_issue_transposed<D, 3>(off, q_t, tb[1]);
+            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 3>(off, q_t, tb[1]);
           };
-          half(std::integral_constant<int, 0>{});
-          half(std::integral_constant<int, 1>{});
+          static_for<0, NH>(half);
         }
         if (had) {   // ---- dS wavefront, current tile: dP = dO V^T, kept for the next iteration
           static_for<0, PF>(chain_read);
 #pragma unroll
-          for (int i = 0; i < 16; ++i) { dp_prev[0][i] = 0.f; dp_prev[1][i] = 0.f; }
+          for (int i = 0; i < 16; ++i) { dp_prev[0][i] = 0.f; dp_prev[NH - 1][i] = 0.f; }
           static_for<0, NC>([&](auto i_) {
             constexpr int i = decltype(i_)::value;
             constexpr int ahead = (NC - 1 - i) < (PF - 1) ? (NC - 1 - i) : (PF - 1);
             lds_wait1<ahead>(rb[i % PF]);
-            dp_prev[i & 1] = E::mfma(rb[i % PF], frag[i >> 1], dp_prev[i & 1]);
+            dp_prev[i % NH] = E::mfma(rb[i % PF], frag[i / NH], dp_prev[i % NH]);
             if constexpr (i + PF < NC) chain_read(std::integral_constant<int, i + PF>{});
           });
         }
@@ -1242,18 +1250,37 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     gi = gi == 2 ? 0 : gi + 1;
     par ^= 1;
   }
+  if constexpr (SHARED) {   // the lower rows' sums go to the pair with the upper rows: [pair % 2][role][register][lane] floats
+    // (the record of the part lies behind what this overwrites)
+    __syncthreads();
+    float *xch = (float *)lds + (size_t)(key_slot * 2 + ROLE) * (T::DT * 16) * 64 + lane;
+    if (slot >= 2) {
+#pragma unroll
+      for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) xch[(dt * 16 + i) * 64] = acc[dt][i];
+    }
+    __syncthreads();
+    if (slot < 2) {
+#pragma unroll
+      for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[dt][i] += xch[(dt * 16 + i) * 64];
+    }
+  }
+  const bool owner = active && (!SHARED || slot < 2);   // of the sums of 32 keys
   if constexpr (PARTS) {
     const BwdPartRecord rec = *part_s;
     const int count = __builtin_amdgcn_readfirstlane(rec.count);
     if (count > 1) {
       constexpr size_t kWaveFloats = (size_t)T::DT * 1024;   // of one wavefront's accumulators
       float *at = rec.first + (size_t)wave * kWaveFloats + lane * 4;
-      if (active) bwd_leave_part<T::DT>(acc, at + (size_t)rec.part * 8 * kWaveFloats);
+      if (owner) bwd_leave_part<T::DT>(acc, at + (size_t)rec.part * 8 * kWaveFloats);
       if (!bwd_last_part(rec.counter, count, (int *)lds)) return;
-      if (active) bwd_sum_parts<T::DT>(acc, at, 8 * kWaveFloats, count);
+      if (owner) bwd_sum_parts<T::DT>(acc, at, 8 * kWaveFloats, count);
     }
   }
-  if (active && l32 < nrows) {
+  if (owner && l32 < nrows) {
     const int64_t row = k0 + kbl * p.kbs + row0 + l32;
     if constexpr (ROLE == 0) bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, acc, 1.f, g32);
     else bwd_store_rows<D, E>(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h, acc, p.scale, g32);
@@ -1263,7 +1290,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   else run(std::integral_constant<int, 1>{});
 }
 
-template <int D, typename E, bool PARTS_Q, bool PARTS_K>
+template <int D, typename E, bool PARTS_Q, bool PARTS_K, bool SHARED>
 int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   using T = BwdTile<D>;
   // LDS: the dQ kernel's three K and two V tiles; the dK/dV kernels' tile buffers, P records and row values
@@ -1275,7 +1302,7 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
       return fail(HBSA_ERR_UNSUPPORTED, "no current device, or device index above %d", kMaxDevices - 1);
     if (!raised[dev]) {
       const void *dkv = nullptr;
-      if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E, PARTS_K>);
+      if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>);
       else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K>);
       hipError_t e = hipFuncSetAttribute(dkv, hipFuncAttributeMaxDynamicSharedMemorySize, lds_dkv);
       if (e == hipSuccess)
@@ -1290,19 +1317,25 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
   const dim3 q_grid = bp.flat_grid ? dim3(q_wgs * (unsigned)nhead_k) : dim3(q_wgs, (unsigned)nhead_k);
   const dim3 kv_grid = bp.flat_grid ? dim3(k_wgs * (unsigned)nhead_k) : dim3(k_wgs, (unsigned)nhead_k);
   hipLaunchKernelGGL((hbsa_bwd_dq_kernel<D, E, PARTS_Q>), q_grid, dim3(kThreads), lds_dq, stream, bp);
-  if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K>), kv_grid, dim3(512), lds_dkv, stream, bp);
+  if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>), kv_grid, dim3(512), lds_dkv, stream, bp);
   else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
 
+template <int D, typename E, bool SHARED>
+int launch_bwd_parts(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
+  const bool pq = bp.parts_q > 1, pk = bp.parts_k > 1;
+  if (pq && pk) return launch_bwd_kernels<D, E, true, true, SHARED>(bp, nhead_k, num_k_block, stream);
+  if (pq) return launch_bwd_kernels<D, E, true, false, SHARED>(bp, nhead_k, num_k_block, stream);
+  if (pk) return launch_bwd_kernels<D, E, false, true, SHARED>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_kernels<D, E, false, false, SHARED>(bp, nhead_k, num_k_block, stream);
+}
 template <int D, typename E>
 int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
-  const bool pq = bp.parts_q > 1, pk = bp.parts_k > 1;
-  if (pq && pk) return launch_bwd_kernels<D, E, true, true>(bp, nhead_k, num_k_block, stream);
-  if (pq) return launch_bwd_kernels<D, E, true, false>(bp, nhead_k, num_k_block, stream);
-  if (pk) return launch_bwd_kernels<D, E, false, true>(bp, nhead_k, num_k_block, stream);
-  return launch_bwd_kernels<D, E, false, false>(bp, nhead_k, num_k_block, stream);
+  // (the kernel for smaller head dims decides for itself whether wavefronts share a slot)
+  if (D == 128 && bp.kbs <= 2 * kWaveRows) return launch_bwd_parts<D, E, D == 128>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_parts<D, E, false>(bp, nhead_k, num_k_block, stream);
 }
 
 }  // namespace hbsa

@@ -82,3 +82,17 @@ def test_a_workspace_without_room_for_parts_is_served_whole():
     for got in results:
         for x, ref, name in zip(got, refs, ("dq", "dk", "dv")):
             _check(x, ref, name)
+
+
+@pytest.mark.parametrize("kbs", [16, 32, 48, 64, 80])
+@pytest.mark.parametrize("hq,hk", [(16, 16), (2, 1)], ids=["whole", "parts"])
+def test_key_blocks_of_up_to_64_keys_at_head_dim_128(kbs, hq, hk):
+    """Two pairs of wavefronts share 32 keys there (up to 80: the size above); ragged tiles, a last block of one key."""
+    q, k, v, do, cu_q, cu_k, cq, ck, mask = _problem(kbs, [333, 97], [321, 129], hq, hk, 128, 80, kbs, 0.6, torch.bfloat16)
+    qd, kd, vd, dod = (t.cuda() for t in (q, k, v, do))
+    prepared = _prepare(cq, ck, mask, 80, kbs, True)
+    out, lse = hbsa_run(qd, kd, vd, prepared, None, return_lse=True)
+    got = hbsa_backward(qd, kd, vd, out, dod, lse, prepared, None)
+    for x, ref, name in zip(got, hbsa_oracle_grads(q, k, v, do, cu_q, cu_k, mask, 80, kbs, True, None), ("dq", "dk", "dv")):
+        _check(x, ref, name)
+    assert all(torch.equal(a, b) for a, b in zip(got, hbsa_backward(qd, kd, vd, out, dod, lse, prepared, None)))
