@@ -21,8 +21,8 @@
 
 #include <atomic>
 #include <cmath>
-#include <mutex>
 
+#include "count_slots.h"
 #include "hbsattn_amd.h"
 
 namespace {
@@ -39,54 +39,32 @@ struct OnDevice {
   }
 };
 
-// ---- Small pinned buffers the device writes block counts to, one per call in flight.  One page for the life of the
-// process; a call that finds every slot taken goes the long way round.
-constexpr int kSlots = 64, kSlotInts = 16;
-struct CountSlots {
-  std::mutex m;
-  int32_t *page = nullptr;
-  uint64_t taken = 0;
-  int32_t *take() {
-    std::lock_guard<std::mutex> lock(m);
-    if (page == nullptr) {
-      void *p = nullptr;
-      if (hipHostMalloc(&p, kSlots * kSlotInts * sizeof(int32_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-      }
-      page = (int32_t *)p;
-      for (int i = 0; i < kSlots * kSlotInts; ++i) page[i] = 0;
-    }
-    if (taken == ~0ull) return nullptr;
-    const int i = __builtin_ctzll(~taken);
-    taken |= 1ull << i;
-    return page + i * kSlotInts;
-  }
-  void give_back(int32_t *slot) {
-    std::lock_guard<std::mutex> lock(m);
-    taken &= ~(1ull << ((slot - page) / kSlotInts));
-  }
-};
-CountSlots g_slots;
+// ---- Pinned slots the device writes block counts to (count_slots.h).  A call that finds none free goes the long way round.
+hbsa_host::CountSlots g_slots;
 std::atomic<int32_t> g_ticket{0};
 
-// Waits until the device has written `ticket` behind the counts.  Looks at memory instead of waiting for an event: the
-// answer arrives while later launches of the same stream are already running.  False: the stream went idle (or failed)
-// without writing it.
-bool wait_for_ticket(const int32_t *slot, int32_t ticket, hipStream_t stream) {
-  const auto arrived = [&]() { return __atomic_load_n(slot + 3, __ATOMIC_ACQUIRE) == ticket; };
-  for (unsigned spins = 1;; ++spins) {
-    if (arrived()) return true;
-    __builtin_ia32_pause();
-    if ((spins & 0xfffu) == 0) {
-      const hipError_t e = hipStreamQuery(stream);
-      if (e != hipErrorNotReady) {
-        (void)hipGetLastError();
-        return arrived();
-      }
-    }
+int32_t *count_page() {
+  void *p = nullptr;
+  constexpr size_t n = hbsa_host::kSlots * hbsa_host::kSlotInts;
+  if (hipHostMalloc(&p, n * sizeof(int32_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
   }
+  for (size_t i = 0; i < n; ++i) ((int32_t *)p)[i] = 0;
+  return (int32_t *)p;
 }
+
+struct StateOf {
+  hipStream_t stream;
+  hbsa_host::StreamState operator()() const {
+    const hipError_t e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) return hbsa_host::StreamState::kBusy;
+    if (e == hipSuccess) return hbsa_host::StreamState::kIdle;
+    (void)hipGetLastError();
+    return hbsa_host::StreamState::kUnknown;
+  }
+};
+using CountTicket = hbsa_host::CountTicket<StateOf>;
 
 struct Problem {
   at::Tensor q, k, v, mask;
@@ -305,28 +283,28 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
 
   const OnDevice on(index);
   const hipStream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)index).stream();
-  int32_t *slot = nullptr, ticket = 0;
-  if (!q_given || !k_given) {
-    // Counts and first blocks of the sequences in one small launch.  The device checks the counts against the mask's
-    // shape and leaves empty sequences when they differ, so the attention launch can follow at once; the host reads
-    // the counts while it runs, and a call whose mask does not fit is reported by the caller.
+  const bool counting = !q_given || !k_given;
+  if (counting) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
       (void)hipGetLastError();
       Py_RETURN_NONE;
     }
-    slot = g_slots.take();
-    if (slot == nullptr) Py_RETURN_NONE;
-    ticket = g_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
+  }
+  CountTicket counts(g_slots, counting ? g_slots.take(count_page) : nullptr, StateOf{stream});
+  if (counting) {
+    // Counts and first blocks of the sequences in one small launch.  The device checks the counts against the mask's
+    // shape and leaves empty sequences when they differ, so the attention launch can follow at once; the host reads
+    // the counts while it runs, and a call whose mask does not fit is reported by the caller.
+    if (counts.slot == nullptr) Py_RETURN_NONE;
+    counts.ticket = g_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
     at::Tensor firsts = at::empty({2, n_seq}, p.cu_q.options());
     int32_t *first = firsts.mutable_data_ptr<int32_t>();
+    counts.launched = true;
     const int rc = hbsa_block_counts(q_given ? nullptr : p.cu_q.const_data_ptr<int32_t>(), (int)p.qbs, (int)p.mask.size(1), first,
                                      k_given ? nullptr : p.cu_k.const_data_ptr<int32_t>(), (int)p.kbs, (int)p.mask.size(2),
-                                     first + n_seq, (int)n_seq - 1, slot, ticket, stream);
-    if (rc != 0) {
-      g_slots.give_back(slot);
-      Py_RETURN_NONE;
-    }
+                                     first + n_seq, (int)n_seq - 1, counts.slot, counts.ticket, stream);
+    if (rc != 0) Py_RETURN_NONE;
     if (!q_given) {
       p.cu_nqb = firsts.select(0, 0);
       p.nqb = p.mask.size(1);
@@ -337,26 +315,15 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     }
   }
 
-  at::Tensor out;
+  const at::Tensor out = wants_grad ? Attention::apply(p.q, p.k, p.v, p) : plain_forward(p, stream);
   bool counts_fit = true;
-  try {
-    if (wants_grad) out = Attention::apply(p.q, p.k, p.v, p);
-    else out = plain_forward(p, stream);
-  } catch (...) {
-    if (slot != nullptr) {
-      (void)wait_for_ticket(slot, ticket, stream);
-      g_slots.give_back(slot);
-    }
-    throw;
-  }
-  if (slot != nullptr) {
+  if (counting) {
     Py_BEGIN_ALLOW_THREADS
-    counts_fit = wait_for_ticket(slot, ticket, stream) && slot[2] == 1;
+    counts_fit = counts.wait() && counts.slot[2] == 1;
     Py_END_ALLOW_THREADS
-    g_slots.give_back(slot);
   }
   if (!counts_fit || !out.defined()) Py_RETURN_NONE;
-  return THPVariable_Wrap(std::move(out));
+  return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }
 
@@ -374,23 +341,21 @@ PyObject *blocks(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     (void)hipGetLastError();
     Py_RETURN_NONE;
   }
-  int32_t *slot = g_slots.take();
-  if (slot == nullptr) Py_RETURN_NONE;
-  const int32_t ticket = g_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
+  CountTicket counts(g_slots, g_slots.take(count_page), StateOf{stream});
+  if (counts.slot == nullptr) Py_RETURN_NONE;
+  counts.ticket = g_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
   at::Tensor first = at::empty({cu.numel()}, cu.options());
   const int batch = (int)cu.numel() - 1;
-  const int rc = hbsa_block_counts(cu.const_data_ptr<int32_t>(), (int)block_size, -1, first.mutable_data_ptr<int32_t>(), nullptr, 1, -1,
-                                   nullptr, batch, slot, ticket, stream);
-  bool good = rc == 0;
-  int64_t num = 0;
-  if (good) {
-    Py_BEGIN_ALLOW_THREADS
-    good = wait_for_ticket(slot, ticket, stream) && slot[2] == 1;
-    Py_END_ALLOW_THREADS
-    num = slot[0];
-  }
-  g_slots.give_back(slot);
+  counts.launched = true;
+  if (hbsa_block_counts(cu.const_data_ptr<int32_t>(), (int)block_size, -1, first.mutable_data_ptr<int32_t>(), nullptr, 1, -1, nullptr,
+                        batch, counts.slot, counts.ticket, stream) != 0)
+    Py_RETURN_NONE;
+  bool good;
+  Py_BEGIN_ALLOW_THREADS
+  good = counts.wait() && counts.slot[2] == 1;
+  Py_END_ALLOW_THREADS
   if (!good) Py_RETURN_NONE;
+  const int64_t num = counts.slot[0];
   at::Tensor cu_block = at::empty({num + 1}, cu.options()), to_batch = at::empty({num}, cu.options());
   const int rc2 = hbsa_block_arrays(cu.const_data_ptr<int32_t>(), first.const_data_ptr<int32_t>(), batch, (int)block_size, (int)num,
                                     cu_block.mutable_data_ptr<int32_t>(), to_batch.mutable_data_ptr<int32_t>(), stream);
