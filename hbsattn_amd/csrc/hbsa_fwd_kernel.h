@@ -977,15 +977,18 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
               (void)v;   // the compiler waits for its own reads
             } else if constexpr (DT == 4) {
               lds_wait<n>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
-            } else if constexpr (DT > 4) {
-              asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(v[0]), "+v"(v[1]) : "n"(n));
-#pragma unroll
-              for (int i = 2; i < 2 * DT; i += 2) asm volatile("" : "+v"(v[i]), "+v"(v[i + 1]));
+            } else if constexpr (DT == 6) {
+              asm volatile("s_waitcnt lgkmcnt(%12)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]),
+                           "+v"(v[6]), "+v"(v[7]), "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]) : "n"(n));
+            } else if constexpr (DT == 5) {
+              asm volatile("s_waitcnt lgkmcnt(%10)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]),
+                           "+v"(v[6]), "+v"(v[7]), "+v"(v[8]), "+v"(v[9]) : "n"(n));
             } else if constexpr (DT == 3) {
               asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]) : "n"(n));
             } else if constexpr (DT == 2) {
               asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : "n"(n));
             } else {
+              static_assert(DT == 1, "one statement waits and names every register of the reads it waits for");
               asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(v[0]), "+v"(v[1]) : "n"(n));
             }
           };
