@@ -160,7 +160,13 @@ struct Attention : public torch::autograd::Function<Attention> {
                           lse_strides, ws.mutable_data_ptr(), n, p.dtype, tq, tk, hq, hk, d, nqb, nkb, (int)p.qbs, (int)p.kbs,
                           p.causal ? 1 : 0, (float)p.scale, strides, stream);
     if (rc != 0) raise("hbsa_fwd_run_lse", rc);
-    ctx->save_for_backward({q, k, v, out, lse, ws, p.cu_k, p.cu_nqb, p.cu_nkb});
+    ctx->save_for_backward({q, k, v, out, lse});
+    // The work description and the boundaries go beside the saved tensors: they may be inference tensors (made by a data
+    // loader or scheduler), their versions are the caller's business, and they are nothing for saved-tensor hooks.
+    ctx->saved_data["workspace"] = ws;
+    ctx->saved_data["cu_k"] = p.cu_k;
+    ctx->saved_data["cu_num_q_block"] = p.cu_nqb;
+    ctx->saved_data["cu_num_k_block"] = p.cu_nkb;
     ctx->saved_data["shape"] = std::vector<int64_t>{p.nqb, p.nkb, p.qbs, p.kbs, p.causal ? 1 : 0, p.dtype};
     ctx->saved_data["scale"] = p.scale;
     return out;
@@ -168,7 +174,9 @@ struct Attention : public torch::autograd::Function<Attention> {
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const at::Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &ws = saved[5];
+    const at::Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
+    const at::Tensor ws = ctx->saved_data["workspace"].toTensor(), cu_k = ctx->saved_data["cu_k"].toTensor();
+    const at::Tensor cu_nqb = ctx->saved_data["cu_num_q_block"].toTensor(), cu_nkb = ctx->saved_data["cu_num_k_block"].toTensor();
     const auto shape = ctx->saved_data["shape"].toIntVector();
     const float scale = (float)ctx->saved_data["scale"].toDouble();
     at::NoGradGuard no_grad;
@@ -186,9 +194,9 @@ struct Attention : public torch::autograd::Function<Attention> {
                                  dv.stride(1)};
     const int rc = hbsa_bwd(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), out.const_data_ptr(), dout.const_data_ptr(),
                             lse.const_data_ptr<float>(), dq.mutable_data_ptr(), dk.mutable_data_ptr(), dv.mutable_data_ptr(),
-                            saved[6].const_data_ptr<int32_t>(), saved[7].const_data_ptr<int32_t>(), saved[8].const_data_ptr<int32_t>(),
+                            cu_k.const_data_ptr<int32_t>(), cu_nqb.const_data_ptr<int32_t>(), cu_nkb.const_data_ptr<int32_t>(),
                             ws.const_data_ptr(), (size_t)ws.numel(), bws.mutable_data_ptr(), n, (int)shape[5],
-                            (int)saved[6].numel() - 1, tq, tk, hq, hk, d, (int)shape[0], (int)shape[1], (int)shape[2], (int)shape[3],
+                            (int)cu_k.numel() - 1, tq, tk, hq, hk, d, (int)shape[0], (int)shape[1], (int)shape[2], (int)shape[3],
                             (int)shape[4], scale, strides, stream);
     if (rc != 0) raise("hbsa_bwd", rc);
     return {dq, dk, dv, at::Tensor()};
