@@ -79,11 +79,16 @@ bool int32_on(const at::Tensor &t, int index, int64_t n) {
   return t.scalar_type() == at::kInt && t.is_cuda() && t.get_device() == index && t.numel() == n && t.is_contiguous();
 }
 
+// Token and head stride of [tokens, heads, head dim].  The stride of a dimension of one element means nothing (torch leaves
+// any number there, in a tensor it calls contiguous too): the shape's stands in for it.
+int64_t tok_stride(const at::Tensor &t) { return t.size(0) == 1 ? t.size(1) * t.size(2) : t.stride(0); }
+int64_t head_stride(const at::Tensor &t) { return t.size(1) == 1 ? t.size(2) : t.stride(1); }
+
 // 16-byte rows with a unit head-dim stride, and token strides the kernels' 32-bit tile offsets can hold
 bool rows_ok(const at::Tensor &t) {
-  const int64_t unit = 16 / t.element_size();
-  return t.stride(2) == 1 && t.stride(0) % unit == 0 && t.stride(1) % unit == 0 && (uintptr_t)t.const_data_ptr() % 16 == 0 &&
-         t.stride(0) >= 0 && t.stride(0) <= (1 << 24);
+  const int64_t unit = 16 / t.element_size(), tok = tok_stride(t);
+  return t.stride(2) == 1 && tok % unit == 0 && head_stride(t) % unit == 0 && (uintptr_t)t.const_data_ptr() % 16 == 0 && tok >= 0 &&
+         tok <= (1 << 24);
 }
 
 [[noreturn]] void raise(const char *what, int rc) {
@@ -108,8 +113,9 @@ bool native_dim(int64_t d) { return d == 32 || d == 64 || d == 128 || d == 256; 
 // The output; undefined when the head dim has to be padded first.
 at::Tensor plain_forward(const Problem &p, hipStream_t stream) {
   at::Tensor out = at::empty(p.q.sizes(), p.q.options());
-  const int64_t strides[11] = {p.q.stride(0), p.q.stride(1), p.k.stride(0), p.k.stride(1), p.v.stride(0), p.v.stride(1),
-                               out.stride(0), out.stride(1), p.mask.stride(0), p.mask.stride(1), p.mask.stride(2)};
+  const int64_t strides[11] = {tok_stride(p.q), head_stride(p.q), tok_stride(p.k), head_stride(p.k), tok_stride(p.v), head_stride(p.v),
+                               tok_stride(out), head_stride(out), p.mask.stride(0), p.mask.stride(1),
+                               p.mask.size(2) == 1 ? 1 : p.mask.stride(2)};
   const int32_t sizes[12] = {p.dtype, (int32_t)(p.cu_q.numel() - 1), (int32_t)p.q.size(0), (int32_t)p.k.size(0),
                              (int32_t)p.q.size(1), (int32_t)p.k.size(1), (int32_t)p.q.size(2), (int32_t)p.nqb, (int32_t)p.nkb,
                              (int32_t)p.qbs, (int32_t)p.kbs, p.causal ? 1 : 0};
@@ -154,7 +160,8 @@ struct Attention : public torch::autograd::Function<Attention> {
     if (rc != 0) raise("hbsa_fwd_prepare", rc);
     at::Tensor out = at::empty(q.sizes(), q.options());
     at::Tensor lse = at::empty({q.size(0), q.size(1)}, q.options().dtype(at::kFloat));
-    const int64_t strides[8] = {q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), out.stride(0), out.stride(1)};
+    const int64_t strides[8] = {tok_stride(q), head_stride(q), tok_stride(k), head_stride(k), tok_stride(v), head_stride(v),
+                                tok_stride(out), head_stride(out)};
     const int64_t lse_strides[2] = {lse.stride(0), lse.stride(1)};
     rc = hbsa_fwd_run_lse(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), out.mutable_data_ptr(), lse.mutable_data_ptr<float>(),
                           lse_strides, ws.mutable_data_ptr(), n, p.dtype, tq, tk, hq, hk, d, nqb, nkb, (int)p.qbs, (int)p.kbs,
@@ -189,9 +196,9 @@ struct Attention : public torch::autograd::Function<Attention> {
     const int tq = (int)q.size(0), tk = (int)k.size(0), hq = (int)q.size(1), hk = (int)k.size(1), d = (int)q.size(2);
     const size_t n = hbsa_bwd_workspace_bytes_parts(tq, hq, hk, d, (int)shape[0], (int)shape[1], (int)shape[2], (int)shape[3]);
     at::Tensor bws = bytes_like(q, n);
-    const int64_t strides[16] = {q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), out.stride(0), out.stride(1),
-                                 dout.stride(0), dout.stride(1), dq.stride(0), dq.stride(1), dk.stride(0), dk.stride(1), dv.stride(0),
-                                 dv.stride(1)};
+    const int64_t strides[16] = {tok_stride(q), head_stride(q), tok_stride(k), head_stride(k), tok_stride(v), head_stride(v),
+                                 tok_stride(out), head_stride(out), tok_stride(dout), head_stride(dout), tok_stride(dq), head_stride(dq),
+                                 tok_stride(dk), head_stride(dk), tok_stride(dv), head_stride(dv)};
     const int rc = hbsa_bwd(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), out.const_data_ptr(), dout.const_data_ptr(),
                             lse.const_data_ptr<float>(), dq.mutable_data_ptr(), dk.mutable_data_ptr(), dv.mutable_data_ptr(),
                             cu_k.const_data_ptr<int32_t>(), cu_nqb.const_data_ptr<int32_t>(), cu_nkb.const_data_ptr<int32_t>(),

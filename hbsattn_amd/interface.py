@@ -64,11 +64,17 @@ def _as_int32(t: torch.Tensor) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
+def _row_strides(t: torch.Tensor):
+    """Token and head stride of ``[tokens, heads, headdim]``.  The stride of a dimension of one element means nothing
+    (torch leaves any number there, in a tensor it calls contiguous too): the shape's stands in for it."""
+    return (t.shape[1] * t.shape[2] if t.shape[0] == 1 else t.stride(0), t.shape[2] if t.shape[1] == 1 else t.stride(1))
+
+
 def _rows_ok(t: torch.Tensor) -> bool:
     """16-byte aligned rows with a unit head-dim stride are what the kernels load."""
     unit = 16 // t.element_size()
-    return (t.stride(2) == 1 and t.stride(0) % unit == 0 and t.stride(1) % unit == 0 and t.data_ptr() % 16 == 0
-            and 0 <= t.stride(0) <= 1 << 24)
+    tok, head = _row_strides(t)
+    return t.stride(2) == 1 and tok % unit == 0 and head % unit == 0 and t.data_ptr() % 16 == 0 and 0 <= tok <= 1 << 24
 
 
 def _pad_headdim(t: torch.Tensor, d_pad: int) -> torch.Tensor:
@@ -232,8 +238,7 @@ def hbsa_run(q, k, v, prepared: PreparedMask, softmax_scale, return_lse: bool = 
         k = k if _rows_ok(k) else k.contiguous()
         v = v if _rows_ok(v) else v.contiguous()
         out_run = out
-    strides = (ctypes.c_int64 * 8)(q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                                   out_run.stride(0), out_run.stride(1))
+    strides = (ctypes.c_int64 * 8)(*(n for t in (q, k, v, out_run) for n in _row_strides(t)))
     ws = prepared.workspace
     code = _dtype_code(q.dtype)
     need = _run_workspace_bytes(lib, q.device, code, total_q, total_k, nhead_q, nhead_k, d_run, prepared.num_q_block,
@@ -304,9 +309,7 @@ def hbsa_backward(q, k, v, out, dout, lse, prepared: PreparedMask, softmax_scale
     bws_bytes = int(lib.hbsa_bwd_workspace_bytes_parts(total_q, nhead_q, nhead_k, d_run, prepared.num_q_block, prepared.num_k_block,
                                                        prepared.q_block_size, prepared.k_block_size))
     bws = torch.empty(bws_bytes, dtype=torch.uint8, device=q.device)
-    strides = (ctypes.c_int64 * 16)(q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                                    out.stride(0), out.stride(1), dout.stride(0), dout.stride(1), dq.stride(0),
-                                    dq.stride(1), dk.stride(0), dk.stride(1), dv.stride(0), dv.stride(1))
+    strides = (ctypes.c_int64 * 16)(*(n for t in (q, k, v, out, dout, dq, dk, dv) for n in _row_strides(t)))
     ws = prepared.workspace
     with torch.cuda.device(q.device):
         rc = lib.hbsa_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dout.data_ptr(), lse.data_ptr(),
