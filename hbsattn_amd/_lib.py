@@ -6,7 +6,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libhbsattn_amd.so")
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 DTYPE_BF16 = 0
 DTYPE_F16 = 1
@@ -43,6 +43,8 @@ def load() -> ctypes.CDLL:
     lib.hbsa_set_deterministic.argtypes = [ctypes.c_int]
     lib.hbsa_fwd_launches.restype = ctypes.c_int
     lib.hbsa_fwd_launches.argtypes = [ctypes.c_int32] * 10 + [ctypes.c_int64, ctypes.c_void_p]
+    lib.hbsa_fwd_decodes.restype = ctypes.c_int
+    lib.hbsa_fwd_decodes.argtypes = [ctypes.c_int32] * 8
     lib.hbsa_set_onepass.restype = ctypes.c_int
     lib.hbsa_set_onepass.argtypes = [ctypes.c_int]
     lib.hbsa_set_walk_min_bytes.restype = ctypes.c_longlong

@@ -40,6 +40,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 // One-launch form: sequences whose boundaries the scheduler keeps in LDS (batch + 1 entries of four arrays)
 constexpr int kSeqCap = 128;
 constexpr int kDecodeMaxParts = 32;    // parts of an item of the decode kernel
+constexpr int kDecodeEntries = 64;     // (q head, row) entries of an item of the decode kernel, as the host bounds them
 constexpr int kMaxPartItems = 4096;   // items of a launch that may be cut into parts (its arrival counters)
 constexpr int kMaxDevices = 64;            // devices of one process the launch caches cover
 constexpr float kLazyRescaleLog2 = 8.0f;  // running max may lag the true max by 2^8
@@ -430,7 +431,7 @@ int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
-int launch_fwd_decode(const FwdParams &fp, long long items, hipStream_t stream);
+int launch_fwd_decode(const FwdParams &fp, int most, long long items, hipStream_t stream);
 template <int D>
 int launch_fwd_f32(const FwdParams &fp, float c_signed, long long items, hipStream_t stream);
 template <int D, typename E>

@@ -442,10 +442,19 @@ int f32_max_parts(long long items, int headdim, int num_k_block) {
   parts = std::min<long long>(parts, (long long)(kMaxPartBytes / (f32_part_bytes(headdim) * (size_t)items)));
   return odd_parts(parts);
 }
-// ---- The decode kernel (hbsa_fwd_decode.h): at most 16 (q head, row) entries per kv head and q block on average, so that
-// the 32-query slots and four-wavefront workgroups of the other kernel would be mostly empty.
-inline bool decode_shape(int32_t dtype, int nhead_q, int nhead_k, int num_q_block, int total_q) {
-  return (dtype == HBSA_DTYPE_BF16 || dtype == HBSA_DTYPE_F16) && (long long)(nhead_q / nhead_k) * total_q <= 16ll * num_q_block;
+// ---- The decode kernel (hbsa_fwd_decode.h): up to 16 (q head, row) entries per kv head and q block on average, so that
+// the 32-query slots and four-wavefront workgroups of the other kernel would be mostly empty, and up to kDecodeEntries in any
+// item, which a single wavefront works on: one longer item (a chunk among decode steps) would keep the whole batch waiting.
+// The host does not know the longest q block; with a row at least in every block it has no more entries than entries_most.
+// 60 single queries and a chunk of 128, 32 / 8 heads of 128, blocks of 32, 64 and 128 rows: 449, 780 and 1447 us here, 262,
+// 401 and 778 in the other kernel.
+inline long long entries_most(int ratio, int num_q_block, int total_q, int q_block_size) {
+  return ratio * std::max(1ll, std::min<long long>(q_block_size, (long long)total_q - num_q_block + 1));
+}
+inline bool decode_shape(int32_t dtype, int nhead_q, int nhead_k, int num_q_block, int total_q, int q_block_size) {
+  const int ratio = nhead_q / nhead_k;
+  return (dtype == HBSA_DTYPE_BF16 || dtype == HBSA_DTYPE_F16) && (long long)ratio * total_q <= 16ll * num_q_block &&
+         entries_most(ratio, num_q_block, total_q, q_block_size) <= kDecodeEntries;
 }
 inline size_t decode_part_bytes(int total_q, int nhead_q, int headdim) { return (size_t)total_q * nhead_q * (headdim + 2) * sizeof(float); }
 // Parts of about the same size for all items, kDecodePartKeys keys each at least, twelve per CU in all; an item of more than
@@ -757,18 +766,19 @@ int run_f32(FwdParams &fp, float softmax_scale, int headdim, int num_k_block, lo
 }
 
 // The decode kernel likewise.
-int run_decode(FwdParams &fp, bool bf, int headdim, int num_k_block, char *area, size_t room, hipStream_t st) {
+int run_decode(FwdParams &fp, bool bf, int headdim, int num_k_block, int q_block_size, char *area, size_t room, hipStream_t st) {
   const long long items = (long long)fp.nhead_k * fp.nqb;
   fp.div_items = make_fast_div((uint32_t)items);
   fp.div_nparts = make_fast_div(1u);
   if (int rc = set_parts(fp, decode_max_parts(items, num_k_block), decode_part_blocks(fp.nhead_k, num_k_block, fp.kbs) * fp.kbs, decode_part_bytes(fp.total_q, fp.nhead_q, headdim), items,
                          area, room, st))
     return rc;
+  const int most = (int)entries_most(fp.ratio, fp.nqb, fp.total_q, q_block_size);
   switch (headdim) {
-    case 32: return bf ? launch_fwd_decode<32, ElemBF16>(fp, items, st) : launch_fwd_decode<32, ElemF16>(fp, items, st);
-    case 64: return bf ? launch_fwd_decode<64, ElemBF16>(fp, items, st) : launch_fwd_decode<64, ElemF16>(fp, items, st);
-    case 128: return bf ? launch_fwd_decode<128, ElemBF16>(fp, items, st) : launch_fwd_decode<128, ElemF16>(fp, items, st);
-    default: return bf ? launch_fwd_decode<256, ElemBF16>(fp, items, st) : launch_fwd_decode<256, ElemF16>(fp, items, st);
+    case 32: return bf ? launch_fwd_decode<32, ElemBF16>(fp, most, items, st) : launch_fwd_decode<32, ElemF16>(fp, most, items, st);
+    case 64: return bf ? launch_fwd_decode<64, ElemBF16>(fp, most, items, st) : launch_fwd_decode<64, ElemF16>(fp, most, items, st);
+    case 128: return bf ? launch_fwd_decode<128, ElemBF16>(fp, most, items, st) : launch_fwd_decode<128, ElemF16>(fp, most, items, st);
+    default: return bf ? launch_fwd_decode<256, ElemBF16>(fp, most, items, st) : launch_fwd_decode<256, ElemF16>(fp, most, items, st);
   }
 }
 }  // namespace hbsa
@@ -796,6 +806,14 @@ int hbsa_fwd_launches(int32_t dtype, int32_t batch, int32_t total_k, int32_t nhe
                                    (long long)num_k_block * k_block_size, (long long)num_q_block * q_block_size);
   const long long items = (long long)nhead_k * num_q_block * ((slots + split.nw - 1) / split.nw);
   return onepass_record(dtype, batch, total_k, headdim, k_block_size, mask_kblk_stride, items, split.parts, (hipStream_t)stream) != nullptr ? 1 : 2;
+}
+
+int hbsa_fwd_decodes(int32_t dtype, int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t num_q_block, int32_t num_k_block,
+                     int32_t q_block_size, int32_t k_block_size) {
+  if (nhead_k <= 0 || nhead_q <= 0 || nhead_q % nhead_k != 0 || num_q_block <= 0 || num_k_block <= 0 || q_block_size <= 0 ||
+      k_block_size <= 0 || total_q <= 0)
+    return 0;
+  return decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size) ? 1 : 0;
 }
 
 int hbsa_set_onepass(int on) {
@@ -884,7 +902,7 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
     const long long items = f32_items(nhead_q, nhead_k, num_q_block, q_block_size);
     return parts_room(f32_max_parts(items, headdim, num_k_block), f32_part_bytes(headdim) * (size_t)items, items);
   }
-  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q)) {
+  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size)) {
     const long long items = (long long)nhead_k * num_q_block;
     return parts_room(decode_max_parts(items, num_k_block), decode_part_bytes(total_q, nhead_q, headdim), items);
   }
@@ -1039,8 +1057,8 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
   fp.walk = (!g_deterministic && fp.nparts == 1 && k_block_size % kTileKeys == 0 &&
              2ll * total_k * headdim * 2 >= g_walk_min_bytes) ? 1 : 0;
 
-  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q))
-    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, split_area, workspace_bytes - need, st);
+  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size))
+    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, q_block_size, split_area, workspace_bytes - need, st);
   if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, split_area, workspace_bytes - need, st);
   if (f32) {
     // setup (multipliers from the maxima), staging, attention: the launch order on the stream is the
@@ -1107,7 +1125,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   if (num_k_block <= 0 || total_k <= 0) return fail(HBSA_ERR_INVALID_ARGUMENT, "no keys");
   if (nhead_k > 65535) return fail(HBSA_ERR_UNSUPPORTED, "nhead_k %d > 65535", nhead_k);
   const bool f32_exact = dtype == HBSA_DTYPE_F32;
-  const bool decode = !any_dim && decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q);
+  const bool decode = !any_dim && decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size);
   const bool direct = allow_onepass && g_onepass && (f32_exact || decode);   // a kernel that reads boundaries and mask itself
   if (allow_onepass && !direct) {
     const int one = try_onepass(q, k, v, out, cu_q_seqlens, cu_k_seqlens, block_mask, cu_num_q_block, cu_num_k_block, dtype,
@@ -1139,7 +1157,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
     char *area = roomy ? (char *)workspace + need : nullptr;
     const size_t room = roomy ? workspace_bytes - need : 0;
     if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, area, room, (hipStream_t)stream);
-    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, area, room, (hipStream_t)stream);
+    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, q_block_size, area, room, (hipStream_t)stream);
   }
   int rc = hbsa_fwd_prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block,
                             workspace, workspace_bytes, batch, nhead_k, num_q_block, num_k_block, q_block_size,

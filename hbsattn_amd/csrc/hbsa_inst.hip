@@ -22,7 +22,7 @@ template int hbsa::launch_fwd_f32<HBSA_D>(const FwdParams &, float, long long, h
 template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
 #elif HBSA_PART == 6
 #include "hbsa_fwd_decode.h"
-template int hbsa::launch_fwd_decode<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
+template int hbsa::launch_fwd_decode<HBSA_D, hbsa::HBSA_E>(const FwdParams &, int, long long, hipStream_t);
 #else
 #error "HBSA_PART is 1 to 6"
 #endif

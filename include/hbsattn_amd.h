@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define HBSA_ABI_VERSION 7
+#define HBSA_ABI_VERSION 8
 
 /* element types of q/k/v/out (reference: dtype follows the input tensors,
  * hbsattn/fwd_triton_auto_tile_size.py:272) */
@@ -76,6 +76,12 @@ int hbsa_set_onepass(int on);   /* see hbsa_fwd */
 int hbsa_fwd_launches(int32_t dtype, int32_t batch, int32_t total_k, int32_t nhead_q, int32_t nhead_k,
                       int32_t headdim, int32_t num_q_block, int32_t num_k_block,
                       int32_t q_block_size, int32_t k_block_size, int64_t mask_kblk_stride, void *stream);
+
+/* 1 when calls of these sizes go to the kernel for few queries per q block (decode steps, drafts; bf16 / fp16, head dims
+ * 32, 64, 128 and 256).  Such a call of hbsa_fwd needs no workspace, whatever hbsa_fwd_launches says; with one it cuts its
+ * items into parts over their k blocks and writes their partial results there.  Host-side only. */
+int hbsa_fwd_decodes(int32_t dtype, int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t num_q_block,
+                     int32_t num_k_block, int32_t q_block_size, int32_t k_block_size);
 
 /* Size (K + V bytes of one kv head) from which the clocked walk above is used; a negative value only
  * reads the setting.  Returns the previous value. */
