@@ -119,7 +119,7 @@ __device__ __forceinline__ void decode_combine(const FwdParams &p, const QBlockI
 #pragma unroll
         for (int i = 0; i < CHUNK / 4; ++i) f[i] = *(const f32x4 *)(weight + e * kMaxParts + base + 4 * i);
 #pragma unroll
-        for (int i = 0; i < CHUNK; ++i) acc += f[i / 4][i % 4] * v[i];   // (weight zero past the last part)
+        for (int i = 0; i < CHUNK; ++i) acc += f[i / 4][i % 4] * (base + i < count ? v[i] : f32x4{0.f, 0.f, 0.f, 0.f});   // (no 0 * inf)
       }
       const float l_tot = sum[e], inv = l_tot > 0.f ? __builtin_amdgcn_rcpf(l_tot) : 0.f;
       if (p.lse != nullptr && dq == 0)

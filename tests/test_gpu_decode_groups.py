@@ -64,3 +64,17 @@ def test_groups_can_be_captured_and_replayed():
         torch.cuda.synchronize()
         assert torch.equal(captured, HBSAttention(*args)), f"replay {step}"
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("q_lens,hq", [([1, 1, 1], 2), ([1] * 9 + [16], 8)])
+def test_an_infinite_value_stays_infinite(q_lens, hq):
+    """Parts that are combined sixteen at a time: what fills the last sixteen up is not multiplied in."""
+    w = _problem(64, q_lens, [5000] * len(q_lens), hq, 2, 64, causal=False)
+    w.block_mask.fill_(True)
+    token = w.cu_k[-1] - 2   # in the last part of the last sequence, inside a whole tile
+    w.v[token, :, 5] = float("inf")
+    out = HBSAttention(*w.args()).float()
+    last = w.cu_q[-2]
+    assert torch.isinf(out[last:, :, 5]).all()
+    out[last:, :, 5] = 0.0
+    assert torch.isfinite(out).all()
