@@ -353,6 +353,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
       if (count <= 0) return 0u;
       const int sh = mask_dma(mrow, first, count);
       __builtin_amdgcn_s_waitcnt(0x0F70);
+      asm volatile("" : : : "memory");
       return staged_words(sh, count);
     };
   };
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
       const int nkblk = __builtin_amdgcn_readlane((int)st_info, 6);
       const int kmax = __builtin_amdgcn_readlane((int)st_info, 7);
       if constexpr (FUSED) {
-        // the staged bytes arrived with the wait of a tile (or of the kernel's first lines) since stage()
+        // the staged bytes arrived with the wait of a tile, or one of the waits before the first item, since stage()
         st_bits = st_nvis > 0 ? staged_words(st_ms, min(st_nvis, kMaskWindow)) : 0u;
         total = build_tile_list<KT>(lds_list + c * kListCap, 0, fused_more_words(st_mrow, st_nvis), 2 * ((st_nvis + 63) >> 6),
                                 p.kbs, p.div_kbs, kmax, st_bits, lane);
@@ -552,7 +553,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     }
     pending = claim();
     stage();
-    if constexpr (FUSED) __builtin_amdgcn_s_waitcnt(0x0F70);   // the first item's mask bytes
+    if constexpr (FUSED) {   // the first item's mask bytes
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      asm volatile("" : : : "memory");
+    }
     build(0);
     note_item(0, hdr_word(0, H_TOTAL));
     pending = claim();
@@ -772,6 +776,12 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     }
   }
   load_q(hdr_word(0, H_HK), hdr_word(0, H_SUB), hdr_word(0, H_ROW_BEGIN), hdr_word(0, H_ROWS));
+  if (FUSED && wave == 0) {
+    // The second item's mask bytes: its list is built below, before any tile has been waited for.  (load_q waits for its
+    // rows, and so for what was requested before them, but a wavefront that has no rows of the first item loads none.)
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    asm volatile("" : : : "memory");
+  }
 
   for (;;) {   // ------------------------------------------------------ one iteration per work item
     const int cur_hk = hdr_word(c, H_HK);
