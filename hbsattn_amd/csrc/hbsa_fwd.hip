@@ -451,10 +451,32 @@ int f32_max_parts(long long items, int headdim, int num_k_block) {
 inline long long entries_most(int ratio, int num_q_block, int total_q, int q_block_size) {
   return ratio * std::max(1ll, std::min<long long>(q_block_size, (long long)total_q - num_q_block + 1));
 }
-inline bool decode_shape(int32_t dtype, int nhead_q, int nhead_k, int num_q_block, int total_q, int q_block_size) {
+// Blocks at most half full on average are decode steps and drafts, alone or beside a chunk: their items are cut into parts.
+// Fuller ones are a prefill in small blocks (of 16 rows, one q head per kv head).  Parts do not pay there, with 16 entries of partial
+// results each (4 heads of 128, 1 x 4096 tokens, blocks of 64 keys: 105 us in parts, 59 whole, 53 in the other kernel), and
+// whole items are better than the other kernel's (us there and here; heads of 128, blocks of 64 keys where nothing else is said):
+// - with k blocks smaller than its tiles of 64 keys: blocks of 16, 1 x 2790 tokens, 1 head 97 and 36, 7 x 1250 on 10000 keys, 16
+//   heads 4138 and 1276; not for a few items of many keys: blocks of 32, 3 x 540 on 4300, 1 head of 32, 36 and 53;
+// - where they are many: 4 heads, 4 x 2048 tokens 65 and 48, 1 x 4096 53 and 59; 16 heads, 16 x 1000 391 and 214;
+// - but no chunks (8 x 160 on 9000 keys, 32 heads of 32: 153 and 171), and not where the K and V that the items share
+//   overflow the caches (1 x 32768 tokens, 8 heads 1330 and 1142, 16 heads 2646 and 3039);
+// - for short sequences: 4 x 100 tokens 10.6 and 8.1, 1 x 300 13.7 and 12.2, 1 x 1000 24 and 28 (8 heads).  The number of
+//   sequences is not known here, only that each leaves less than a block's rows empty.
+struct DecodePlan {
+  bool use, parts;
+};
+DecodePlan decode_plan(int32_t dtype, int nhead_q, int nhead_k, int num_q_block, int total_q, int q_block_size, int num_k_block, int k_block_size) {
   const int ratio = nhead_q / nhead_k;
-  return (dtype == HBSA_DTYPE_BF16 || dtype == HBSA_DTYPE_F16) && (long long)ratio * total_q <= 16ll * num_q_block &&
-         entries_most(ratio, num_q_block, total_q, q_block_size) <= kDecodeEntries;
+  const long long blocks = num_q_block, rows = total_q, keys = (long long)num_k_block * k_block_size;
+  const long long most = entries_most(ratio, num_q_block, total_q, q_block_size);
+  if ((dtype != HBSA_DTYPE_BF16 && dtype != HBSA_DTYPE_F16) || ratio * rows > 16 * blocks || most > kDecodeEntries) return {false, false};
+  if (2 * rows <= blocks * q_block_size) return {true, true};
+  if (most > 16) return {false, false};
+  const long long items = nhead_k * blocks, empty_rows = std::max(0ll, blocks * q_block_size - rows);
+  const long long sequences = std::max(1ll, (empty_rows + q_block_size - 2) / (q_block_size - 1));
+  if (keys <= 512 * sequences && keys <= 4 * rows) return {true, false};
+  if (k_block_size < kTileKeys) return {items >= 256 || keys <= 2 * rows, false};
+  return {items >= 2048 && keys <= 8 * rows && keys * nhead_k < (1ll << 19), false};
 }
 inline size_t decode_part_bytes(int total_q, int nhead_q, int headdim) { return (size_t)total_q * nhead_q * (headdim + 2) * sizeof(float); }
 // Parts of about the same size for all items, kDecodePartKeys keys each at least, twelve per CU in all; an item of more than
@@ -766,11 +788,11 @@ int run_f32(FwdParams &fp, float softmax_scale, int headdim, int num_k_block, lo
 }
 
 // The decode kernel likewise.
-int run_decode(FwdParams &fp, bool bf, int headdim, int num_k_block, int q_block_size, char *area, size_t room, hipStream_t st) {
+int run_decode(FwdParams &fp, bool cut, bool bf, int headdim, int num_k_block, int q_block_size, char *area, size_t room, hipStream_t st) {
   const long long items = (long long)fp.nhead_k * fp.nqb;
   fp.div_items = make_fast_div((uint32_t)items);
   fp.div_nparts = make_fast_div(1u);
-  if (int rc = set_parts(fp, decode_max_parts(items, num_k_block), decode_part_blocks(fp.nhead_k, num_k_block, fp.kbs) * fp.kbs, decode_part_bytes(fp.total_q, fp.nhead_q, headdim), items,
+  if (int rc = set_parts(fp, cut ? decode_max_parts(items, num_k_block) : 1, decode_part_blocks(fp.nhead_k, num_k_block, fp.kbs) * fp.kbs, decode_part_bytes(fp.total_q, fp.nhead_q, headdim), items,
                          area, room, st))
     return rc;
   const int most = (int)entries_most(fp.ratio, fp.nqb, fp.total_q, q_block_size);
@@ -813,7 +835,7 @@ int hbsa_fwd_decodes(int32_t dtype, int32_t total_q, int32_t nhead_q, int32_t nh
   if (nhead_k <= 0 || nhead_q <= 0 || nhead_q % nhead_k != 0 || num_q_block <= 0 || num_k_block <= 0 || q_block_size <= 0 ||
       k_block_size <= 0 || total_q <= 0)
     return 0;
-  return decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size) ? 1 : 0;
+  return decode_plan(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size, num_k_block, k_block_size).use ? 1 : 0;
 }
 
 int hbsa_set_onepass(int on) {
@@ -902,7 +924,8 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
     const long long items = f32_items(nhead_q, nhead_k, num_q_block, q_block_size);
     return parts_room(f32_max_parts(items, headdim, num_k_block), f32_part_bytes(headdim) * (size_t)items, items);
   }
-  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size)) {
+  const DecodePlan plan = decode_plan(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size, num_k_block, 16);   // (parts: whatever the k block size)
+  if (plan.use && plan.parts) {
     const long long items = (long long)nhead_k * num_q_block;
     return parts_room(decode_max_parts(items, num_k_block), decode_part_bytes(total_q, nhead_q, headdim), items);
   }
@@ -1057,8 +1080,9 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
   fp.walk = (!g_deterministic && fp.nparts == 1 && k_block_size % kTileKeys == 0 &&
              2ll * total_k * headdim * 2 >= g_walk_min_bytes) ? 1 : 0;
 
-  if (decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size))
-    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, q_block_size, split_area, workspace_bytes - need, st);
+  const DecodePlan decode = decode_plan(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size, num_k_block, k_block_size);
+  if (decode.use)
+    return run_decode(fp, decode.parts, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, q_block_size, split_area, workspace_bytes - need, st);
   if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, split_area, workspace_bytes - need, st);
   if (f32) {
     // setup (multipliers from the maxima), staging, attention: the launch order on the stream is the
@@ -1125,7 +1149,8 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   if (num_k_block <= 0 || total_k <= 0) return fail(HBSA_ERR_INVALID_ARGUMENT, "no keys");
   if (nhead_k > 65535) return fail(HBSA_ERR_UNSUPPORTED, "nhead_k %d > 65535", nhead_k);
   const bool f32_exact = dtype == HBSA_DTYPE_F32;
-  const bool decode = !any_dim && decode_shape(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size);
+  const DecodePlan plan = decode_plan(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size, num_k_block, k_block_size);
+  const bool decode = !any_dim && plan.use;
   const bool direct = allow_onepass && g_onepass && (f32_exact || decode);   // a kernel that reads boundaries and mask itself
   if (allow_onepass && !direct) {
     const int one = try_onepass(q, k, v, out, cu_q_seqlens, cu_k_seqlens, block_mask, cu_num_q_block, cu_num_k_block, dtype,
@@ -1157,7 +1182,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
     char *area = roomy ? (char *)workspace + need : nullptr;
     const size_t room = roomy ? workspace_bytes - need : 0;
     if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, area, room, (hipStream_t)stream);
-    return run_decode(fp, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, q_block_size, area, room, (hipStream_t)stream);
+    return run_decode(fp, plan.parts, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, q_block_size, area, room, (hipStream_t)stream);
   }
   int rc = hbsa_fwd_prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block,
                             workspace, workspace_bytes, batch, nhead_k, num_q_block, num_k_block, q_block_size,

@@ -29,6 +29,25 @@ def test_by_the_longest_block(rows, hq, hk, qbs, expected):
         assert _decodes(rows, hq, hk, qbs, [4000] * len(rows), dtype=dtype) == 0
 
 
+@pytest.mark.parametrize("rows,k_lens,hk,kbs,expected", [
+    ([2048] * 4, None, 4, 64, 1),            # 2048 items
+    ([4096], None, 4, 64, 0),                # 1024 of long sequences
+    ([4096], None, 4, 48, 1),                # k blocks smaller than the other kernel's tiles
+    ([540] * 3, [4300] * 3, 1, 32, 0),       # ... but few items of many keys
+    ([540] * 3, [4300] * 3, 4, 32, 1),
+    ([160] * 8, [9000] * 8, 32, 64, 0),      # chunks
+    ([32768], None, 8, 64, 1),
+    ([32768], None, 16, 64, 0),              # more K and V than the caches hold
+    ([300], None, 8, 64, 1),                 # short
+    ([1000], None, 8, 64, 0),
+    ([100] * 16, None, 2, 64, 1),            # short, as the rows missing in the last blocks tell
+    ([16] * 32, [40000] * 32, 8, 64, 0),     # whole blocks of queries on long caches: no parts, too few items
+])
+def test_full_blocks(rows, k_lens, hk, kbs, expected):
+    """16-row blocks, one q head per kv head: every prefill and training call has items of at most 16 entries."""
+    assert _decodes(rows, hk, hk, 16, k_lens or rows, kbs) == expected
+
+
 def test_sizes_that_make_no_call():
     lib = _lib.load()
     good = [_lib.DTYPE_BF16, 32, 32, 8, 32, 2000, 16, 64]
