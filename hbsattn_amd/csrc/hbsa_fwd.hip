@@ -361,20 +361,29 @@ int device_cus() {
   return cus_of[dev];
 }
 
-// Split of `items` equal items over key blocks where `places` workgroups run at once: the number of parts with the fewest
+// Split of `items` items over key blocks where `places` workgroups run at once: the number of parts with the fewest
 // rounds of the device, counted in whole items, plus what a part costs (its fp32 partial results are written and merged;
 // and the split is four launches in place of one).  A problem of chunks, its keys many times its queries, has items of
-// about one weight, so the count is right and parts of 2048 keys pay; elsewhere the causal order evens the rounds out and
-// only a problem that leaves places empty is split, into parts of 8192 keys.  Measured, us, with the split as it was before
-// (2 * CUs / items parts) and as here: chunks of 512 on 32000 keys, 32 / 8 heads of 128, 143 -> 122; 2 x 300 .. 512 on 65000
-// 285 -> 258; 4 x 700 .. 1500 on 30000 .. 60000, 16 / 2 heads, 487 -> 394; 2 x 64 .. 128 on 8000 .. 16000 69 -> 51; sequences by
-// themselves, 32 / 8 heads, 1 x 1024 33 -> 27, 1 x 2048 67 -> 40; 1 x 4096, 8 / 1 heads, 59 -> 45.
-// (At most five items for eight places of workgroups of four: beyond that they stay one launch.)
-int split_parts(long long items, int nw, int headdim, int num_k_block, long long keys, long long queries) {
-  const bool chunks = keys >= 4 * queries;
+// about one weight, so the count is right and parts of kChunkPartTiles tiles pay; elsewhere the causal order evens the rounds out and
+// only a problem that leaves places empty is split, into parts of kPartTiles.  (Tiles and not keys: a k block smaller than a
+// tile has one to itself.  All tiles of the problem stand in for an item's.)  Where a CU has one place and the parts fill a
+// single round, nothing follows that could even out unequal items: twice the parts then, if they stay long (but not for two
+// parts, which few items do not need: 2 x 300 .. 512 on 65000 keys 269, with four 277).
+// Measured, us, before any of this (2 * CUs / items parts) and as here: chunks of 512 on 32000 keys, 32 / 8 heads of 128, 143 ->
+// 122; 4 x 700 .. 1500 on 30000 .. 60000, 16 / 2 heads, 487 -> 394; 2 x 64 .. 128 on 8000 .. 16000 69 -> 51; sequences by
+// themselves, 32 / 8 heads, 1 x 1024 33 -> 27, 1 x 2048 67 -> 40; 1 x 4096, 8 / 1 heads, 59 -> 45.  With keys
+// counted in place of tiles (2048 a part, 8192 outside chunks): 2 x 560 on 12000 keys in blocks of 16, 8 / 1 heads of 256, 641, here
+// 359; 1 x 3318 tokens in k blocks of 16, 4 heads of 128, 118 and 85; without the second round: 4 x 440 on 24000 keys, 8 / 4 heads of
+// 128, 238 and 177.  (Shorter parts cost a little where few blocks are kept: 1 .. 4 queries on 2000 .. 32000 keys, 8 / 1 heads, 59 and 67.)
+// (At most five items for eight places of workgroups of four: beyond that they stay one launch.  10 x 32 items of 256 dims on
+// 21000 keys, a place for 256 of them: split 1428, whole 932.)
+constexpr int kChunkPartTiles = 20, kPartTiles = 64, kLongPartTiles = 128;
+int split_parts(long long items, int nw, int headdim, int num_k_block, int k_block_size, long long queries) {
+  const long long tiles = (long long)num_k_block * ((k_block_size + kTileKeys - 1) / kTileKeys);
+  const bool chunks = (long long)num_k_block * k_block_size >= 4 * queries;
   const long long cus = device_cus(), places = nw == 8 || headdim > 192 ? cus : 2 * cus;
-  if (items <= 0 || cus <= 0 || items > (nw == 8 ? (chunks ? 2 * cus : cus) : 5 * cus / 4)) return 1;
-  const long long most = std::min<long long>(std::min<long long>(32, num_k_block / 8), keys / (chunks ? 2048 : 8192));
+  if (items <= 0 || cus <= 0 || items > (nw == 8 ? (chunks ? 2 * cus : cus) : 5 * places / 8)) return 1;
+  const long long most = std::min<long long>(std::min<long long>(32, num_k_block / 8), tiles / (chunks ? kChunkPartTiles : kPartTiles));
   const double part = 0.05 * std::max<double>((double)items, 1.0) / (double)places;
   double best = (double)((items + places - 1) / places) + part;
   int parts = 1;
@@ -385,11 +394,12 @@ int split_parts(long long items, int nw, int headdim, int num_k_block, long long
       parts = n;
     }
   }
+  if (parts > 2 && parts <= 16 && places == cus && items * parts <= places && tiles >= 2 * parts * kLongPartTiles) parts *= 2;
   return parts;
 }
 
 // Wavefronts per workgroup of the 16-bit attention kernel for an item of `slots` wave slots, and its split over key blocks.
-// `keys` and `queries` are the problem's, up to whole blocks.
+// `queries` are the problem's, up to whole blocks, `rows` its query rows.
 // Eight wavefronts stage an item's K/V tiles once where workgroups of four stage them twice, but only one such workgroup
 // fits a CU, and it waits for its own barriers and items.  At head dim 64 three workgroups of four do fit and are faster
 // everywhere (16 / 4 heads of 64, 6 x 300 .. 4000 tokens 78 -> 74 us; 32 / 8 heads, 4 x 500 .. 3000 81 -> 61, 8 x 2048 .. 8000 670 ->
@@ -398,19 +408,21 @@ int split_parts(long long items, int nw, int headdim, int num_k_block, long long
 // Few items that do not come out at whole pairs of rounds take four: 1.9 items a CU 62 -> 59, 2.5 40.7 -> 37.9, 3.0 145 ->
 // 134, 3.7 101 -> 99, 3.8 110 -> 95, 4.8 98 -> 87, 5.1 140 -> 124; at 2.0 82 -> 83, at 4.0 205 -> 220, which stay at eight.
 // An item whose last workgroup of eight would be at most half full has none with idle wavefronts as fours.
+// Where the blocks are at most half full (decode steps beside a chunk) every workgroup of an item stages the tiles for a row
+// or two: eights, half as many (60 single queries and a chunk of 128 in 128-row blocks 778 -> 742).
 struct FwdSplit {
   int nw, parts;
 };
-FwdSplit fwd_split(int slots, int headdim, bool f32_exact, long long item_groups, int num_k_block, long long keys, long long queries) {
+FwdSplit fwd_split(int slots, int headdim, bool f32_exact, long long item_groups, int num_k_block, int k_block_size, long long queries, long long rows) {
   const long long cus = device_cus(), fours = item_groups * ((slots + 3) / 4), eights = item_groups * ((slots + 7) / 8);
   if (f32_exact) return {4, 1};
   const int in_last = slots % 8;
   if (headdim == 128 && slots > 4 && !(in_last >= 1 && in_last <= 4)) {
-    const int parts = split_parts(eights, 8, headdim, num_k_block, keys, queries);
+    const int parts = split_parts(eights, 8, headdim, num_k_block, k_block_size, queries);
     const long long room = 2 * cus * ((eights + 2 * cus - 1) / std::max(1ll, 2 * cus));
-    if (parts > 1 || cus == 0 || eights >= 6 * cus || 32 * eights >= 31 * room) return {8, parts};
+    if (parts > 1 || cus == 0 || eights >= 6 * cus || 32 * eights >= 31 * room || 2 * rows <= queries) return {8, parts};
   }
-  return {4, split_parts(fours, 4, headdim, num_k_block, keys, queries)};
+  return {4, split_parts(fours, 4, headdim, num_k_block, k_block_size, queries)};
 }
 // split area: nparts bit row copies | nparts partial outputs | nparts partial log-sum-exps, each array packed
 inline size_t split_bits_bytes(int parts, int nhead_k, int num_q_block, int num_k_block) {
@@ -532,7 +544,7 @@ inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_bloc
 }
 
 // The fields of FwdParams that follow from the call's shape and softmax_scale alone.
-void fill_shape(FwdParams &fp, int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size,
+void fill_shape(FwdParams &fp, int total_q, int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size,
                 int k_block_size, int causal, float softmax_scale, bool f32_exact, bool may_pack = false, bool cols = false) {
   fp.nhead_k = nhead_k;
   fp.nqb = num_q_block; fp.ratio = nhead_q / nhead_k; fp.kbs = k_block_size; fp.wpr = words_per_row(num_k_block);
@@ -540,8 +552,8 @@ void fill_shape(FwdParams &fp, int nhead_q, int nhead_k, int headdim, int num_q_
   fp.wps = (q_block_size + kWaveRows - 1) / kWaveRows;
   fp.pack = cols || f32_exact || (may_pack && fwd_packs(fp.ratio, q_block_size)) ? 1 : 0;
   const int slots = fwd_slots(fp.ratio, q_block_size, fp.pack != 0);
-  const FwdSplit split = fwd_split(slots, headdim, f32_exact, (long long)nhead_k * num_q_block, num_k_block,
-                                   (long long)num_k_block * k_block_size, (long long)num_q_block * q_block_size);
+  const FwdSplit split = fwd_split(slots, headdim, f32_exact, (long long)nhead_k * num_q_block, num_k_block, k_block_size,
+                                   (long long)num_q_block * q_block_size, total_q);
   fp.nw = split.nw;
   fp.split = split.parts;
   fp.ncol = headdim / 8;
@@ -709,7 +721,7 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   FwdParams fp;
   std::memset(&fp, 0, sizeof(fp));
   const bool cols = headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256;
-  fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, false,
+  fill_shape(fp, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, false,
              true, cols);
   const long long items = (long long)nhead_k * num_q_block * fp.nsub;
   Sched *sched = onepass_record(dtype, batch, total_k, headdim, k_block_size, strides[10], items, fp.split, st);
@@ -824,8 +836,8 @@ int hbsa_fwd_launches(int32_t dtype, int32_t batch, int32_t total_k, int32_t nhe
       k_block_size <= 0 || (headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256))
     return 2;
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, fwd_packs(nhead_q / nhead_k, q_block_size));   // as try_onepass
-  const FwdSplit split = fwd_split(slots, headdim, false, (long long)nhead_k * num_q_block, num_k_block,
-                                   (long long)num_k_block * k_block_size, (long long)num_q_block * q_block_size);
+  const long long queries = (long long)num_q_block * q_block_size;   // (as if the q blocks were full)
+  const FwdSplit split = fwd_split(slots, headdim, false, (long long)nhead_k * num_q_block, num_k_block, k_block_size, queries, queries);
   const long long items = (long long)nhead_k * num_q_block * ((slots + split.nw - 1) / split.nw);
   return onepass_record(dtype, batch, total_k, headdim, k_block_size, mask_kblk_stride, items, split.parts, (hipStream_t)stream) != nullptr ? 1 : 2;
 }
@@ -930,11 +942,9 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
     return parts_room(decode_max_parts(items, num_k_block), decode_part_bytes(total_q, nhead_q, headdim), items);
   }
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, false);
-  // (without the k block size the keys are not known: the room for the most parts any size can get)
-  int parts = 1;
-  for (int kbs = 16; kbs <= 2048; kbs *= 2)
-    parts = std::max(parts, fwd_split(slots, headdim, false, (long long)nhead_k * num_q_block, num_k_block, (long long)num_k_block * kbs,
-                                      (long long)num_q_block * q_block_size).parts);
+  // (without the k block size the tiles are not known: the room for the most parts, which grow with it)
+  const int parts = fwd_split(slots, headdim, false, (long long)nhead_k * num_q_block, num_k_block, 2048, (long long)num_q_block * q_block_size,
+                              total_q).parts;
   return split_bytes(parts, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
 }
 
@@ -1061,7 +1071,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
     fp.q_s = strides[0] * es; fp.q_h = strides[1] * es; fp.k_s = strides[2] * es; fp.k_h = strides[3] * es;
     fp.v_s = strides[4] * es; fp.v_h = strides[5] * es; fp.o_s = strides[6] * es; fp.o_h = strides[7] * es;
   }
-  fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale,
+  fill_shape(fp, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale,
              f32_exact);
   const long long items = (long long)nhead_k * num_q_block * fp.nsub;
   if (items > 0x7fffffffLL) return fail(HBSA_ERR_UNSUPPORTED, "too many work items (%lld)", items);
@@ -1167,7 +1177,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
     if (roomy && ((uintptr_t)workspace & 255)) return fail(HBSA_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");
     FwdParams fp;
     std::memset(&fp, 0, sizeof(fp));
-    fill_shape(fp, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
+    fill_shape(fp, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
     const long long items = (long long)nhead_k * num_q_block * fp.nsub;
     if (items > 0x7fffffffLL) return fail(HBSA_ERR_UNSUPPORTED, "too many work items (%lld)", items);
     const int64_t es = f32_exact ? 4 : 2;
