@@ -502,9 +502,15 @@ int decode_part_blocks(int nhead_k, int num_k_block, int k_block_size) {
   const long long even = ((long long)nhead_k * num_k_block + target - 1) / target;
   return (int)std::max<long long>(even, std::max(1, kDecodePartKeys / k_block_size));
 }
-int decode_max_parts(long long items, int num_k_block) {
+// The launch has this many workgroups for every item, and those without a part of it are not free (2.7 ns each at head dim 128): no
+// more than items of eight times the mean length can use, six times with two items a CU.  64 sequences of 10 .. 60 and of 100 ..
+// 600 keys, 32 / 8 heads of 128, 14.9 -> 6.9 and 27.3 -> 23.9 us (10.4 and 20.1 in the other kernel); one of 32000 keys among 64 of 100
+// .. 600, 4 heads, 34.5 -> 36.4 (342), with four times 54; among 128, where six times are allowed, 51.2 -> 50.6, with four times 69.
+int decode_max_parts(int nhead_k, int num_q_block, int num_k_block, int part_blocks) {
+  const long long items = (long long)nhead_k * num_q_block;
   if (items <= 0 || items > kMaxPartItems) return 1;
-  long long parts = std::min<long long>(kDecodeMaxParts, 30ll * device_cus() / items);
+  const long long times = items >= 2 * device_cus() ? 6 : 8, even = (long long)num_q_block * part_blocks;
+  const long long parts = std::min<long long>(std::min<long long>(kDecodeMaxParts, 30ll * device_cus() / items), (times * num_k_block + even - 1) / even);
   return odd_parts(std::min<long long>(parts, num_k_block));
 }
 // ---- Parts of the backward's items (BwdCut), when the items leave places of the device empty (`resident` workgroups a CU):
@@ -804,8 +810,9 @@ int run_decode(FwdParams &fp, bool cut, bool bf, int headdim, int num_k_block, i
   const long long items = (long long)fp.nhead_k * fp.nqb;
   fp.div_items = make_fast_div((uint32_t)items);
   fp.div_nparts = make_fast_div(1u);
-  if (int rc = set_parts(fp, cut ? decode_max_parts(items, num_k_block) : 1, decode_part_blocks(fp.nhead_k, num_k_block, fp.kbs) * fp.kbs, decode_part_bytes(fp.total_q, fp.nhead_q, headdim), items,
-                         area, room, st))
+  const int part_blocks = decode_part_blocks(fp.nhead_k, num_k_block, fp.kbs);
+  if (int rc = set_parts(fp, cut ? decode_max_parts(fp.nhead_k, fp.nqb, num_k_block, part_blocks) : 1, part_blocks * fp.kbs,
+                         decode_part_bytes(fp.total_q, fp.nhead_q, headdim), items, area, room, st))
     return rc;
   const int most = (int)entries_most(fp.ratio, fp.nqb, fp.total_q, q_block_size);
   switch (headdim) {
@@ -938,8 +945,9 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
   }
   const DecodePlan plan = decode_plan(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size, num_k_block, 16);   // (parts: whatever the k block size)
   if (plan.use && plan.parts) {
-    const long long items = (long long)nhead_k * num_q_block;
-    return parts_room(decode_max_parts(items, num_k_block), decode_part_bytes(total_q, nhead_q, headdim), items);
+    // (a part's blocks, for k blocks of any size: the room for the most parts)
+    const int parts = decode_max_parts(nhead_k, num_q_block, num_k_block, decode_part_blocks(nhead_k, num_k_block, kDecodePartKeys));
+    return parts_room(parts, decode_part_bytes(total_q, nhead_q, headdim), (long long)nhead_k * num_q_block);
   }
   const int slots = fwd_slots(nhead_q / nhead_k, q_block_size, false);
   // (without the k block size the tiles are not known: the room for the most parts, which grow with it)

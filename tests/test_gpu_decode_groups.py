@@ -78,3 +78,12 @@ def test_an_infinite_value_stays_infinite(q_lens, hq):
     assert torch.isinf(out[last:, :, 5]).all()
     out[last:, :, 5] = 0.0
     assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("blocks_each", [1, 6, 40])
+def test_parts_follow_the_mean_length(blocks_each):
+    """64 single queries, 32 / 8 heads of 128: no more room, and so no more workgroups, for parts than items of six times
+    the mean number of k blocks (eight times with less than two items a compute unit) can have."""
+    part_bytes = 64 * 32 * (128 + 2) * 4
+    room = _lib.load().hbsa_fwd_parts_bytes(_lib.DTYPE_BF16, 64, 32, 8, 128, 64, 64 * blocks_each, 16)
+    assert part_bytes < room <= min(32, 8 * blocks_each) * part_bytes + 8192
