@@ -214,11 +214,6 @@ struct ElemBF16 {
   static __device__ __forceinline__ float lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
   static __device__ __forceinline__ float hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
   static __device__ __forceinline__ uint32_t scale_packed(uint32_t w, float f) { return pack2(lo(w) * f, hi(w) * f); }
-  // acc + lo + hi of a packed pair (v_dot2c_f32_bf16 with a vector of ones)
-  static __device__ __forceinline__ float dot2_ones(uint32_t packed, float acc) {
-    const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), ones, acc, false);
-  }
 };
 struct ElemF16 {
   static __device__ __forceinline__ f32x16 mfma(short8v a, short8v b, f32x16 c) {
@@ -231,10 +226,6 @@ struct ElemF16 {
   static __device__ __forceinline__ float lo(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w).x; }
   static __device__ __forceinline__ float hi(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w).y; }
   static __device__ __forceinline__ uint32_t scale_packed(uint32_t w, float f) { return pack2(lo(w) * f, hi(w) * f); }
-  static __device__ __forceinline__ float dot2_ones(uint32_t packed, float acc) {
-    const f16x2 ones = {(_Float16)1.0f, (_Float16)1.0f};
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, packed), ones, acc, false);
-  }
 };
 
 // exchange-and-combine between lane i and lane i^32
@@ -294,10 +285,6 @@ __device__ __forceinline__ short4v lds_read_tr16_b64(uint32_t addr) {
 template <int N>
 __device__ __forceinline__ void lds_wait1(short8v &a) {
   asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(a) : "n"(N));
-}
-template <int N>
-__device__ __forceinline__ void lds_wait(short8v &a, short8v &b) {
-  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N));
 }
 template <int N>
 __device__ __forceinline__ void lds_wait(short4v &a, short4v &b, short4v &c, short4v &d, short4v &e, short4v &f, short4v &g,
