@@ -366,18 +366,19 @@ int device_cus() {
 // and the split is four launches in place of one).  A problem of chunks, its keys many times its queries, has items of
 // about one weight, so the count is right and parts of kChunkPartTiles tiles pay; elsewhere the causal order evens the rounds out and
 // only a problem that leaves places empty is split, into parts of kPartTiles.  (Tiles and not keys: a k block smaller than a
-// tile has one to itself.  All tiles of the problem stand in for an item's.)  Where a CU has one place and the parts fill a
-// single round, nothing follows that could even out unequal items: twice the parts then, if they stay long (but not for two
-// parts, which few items do not need: 2 x 300 .. 512 on 65000 keys 269, with four 277).
+// tile has one to itself.  All tiles of the problem stand in for an item's.)
 // Measured, us, before any of this (2 * CUs / items parts) and as here: chunks of 512 on 32000 keys, 32 / 8 heads of 128, 143 ->
-// 122; 4 x 700 .. 1500 on 30000 .. 60000, 16 / 2 heads, 487 -> 394; 2 x 64 .. 128 on 8000 .. 16000 69 -> 51; sequences by
-// themselves, 32 / 8 heads, 1 x 1024 33 -> 27, 1 x 2048 67 -> 40; 1 x 4096, 8 / 1 heads, 59 -> 45.  With keys
-// counted in place of tiles (2048 a part, 8192 outside chunks): 2 x 560 on 12000 keys in blocks of 16, 8 / 1 heads of 256, 641, here
-// 359; 1 x 3318 tokens in k blocks of 16, 4 heads of 128, 118 and 85; without the second round: 4 x 440 on 24000 keys, 8 / 4 heads of
-// 128, 238 and 177.  (Shorter parts cost a little where few blocks are kept: 1 .. 4 queries on 2000 .. 32000 keys, 8 / 1 heads, 59 and 67.)
+// 122; 2 x 300 .. 512 on 65000 285 -> 258; 4 x 700 .. 1500 on 30000 .. 60000, 16 / 2 heads, 487 -> 394; 2 x 64 .. 128 on 8000 .. 16000
+// 69 -> 51; sequences by themselves, 32 / 8 heads, 1 x 1024 33 -> 27, 1 x 2048 67 -> 40; 1 x 4096, 8 / 1 heads, 59 -> 45.  With keys counted in
+// place of tiles (2048 and 8192 a part): 1 x 3318 tokens in k blocks of 16, 4 heads of 128, 118, here 84; 2 x 100 on 22000 keys in
+// such blocks, 2 heads, 109 and 94.
+// At head dim 256 a CU has one place, and parts that fill a single round have nothing behind them that could even out items of
+// unequal sequences: twice the parts, if they stay long (2 x 560 on 12000 keys on average, in blocks of 16, 8 / 1 heads, 641 ->
+// 359; 8 x 6 on 2000 .. 14000, 32 / 4 heads, 341 -> 246).  At 128, where chunks of about one length lose by it (3 x 80 .. 161 on
+// 80000 keys, 32 / 8 heads, 260 and 278), it is left alone.
 // (At most five items for eight places of workgroups of four: beyond that they stay one launch.  10 x 32 items of 256 dims on
 // 21000 keys, a place for 256 of them: split 1428, whole 932.)
-constexpr int kChunkPartTiles = 20, kPartTiles = 64, kLongPartTiles = 128;
+constexpr int kChunkPartTiles = 32, kPartTiles = 96, kLongPartTiles = 128;
 int split_parts(long long items, int nw, int headdim, int num_k_block, int k_block_size, long long queries) {
   const long long tiles = (long long)num_k_block * ((k_block_size + kTileKeys - 1) / kTileKeys);
   const bool chunks = (long long)num_k_block * k_block_size >= 4 * queries;
@@ -394,7 +395,7 @@ int split_parts(long long items, int nw, int headdim, int num_k_block, int k_blo
       parts = n;
     }
   }
-  if (parts > 2 && parts <= 16 && places == cus && items * parts <= places && tiles >= 2 * parts * kLongPartTiles) parts *= 2;
+  if (headdim > 192 && parts > 2 && parts <= 16 && items * parts <= places && tiles >= 2 * parts * kLongPartTiles) parts *= 2;
   return parts;
 }
 
