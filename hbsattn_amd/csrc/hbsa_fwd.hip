@@ -367,11 +367,11 @@ int device_cus() {
 // about one weight, so the count is right and parts of kChunkPartTiles tiles pay; elsewhere the causal order evens the rounds out and
 // only a problem that leaves places empty is split, into parts of kPartTiles.  (Tiles and not keys: a k block smaller than a
 // tile has one to itself.  All tiles of the problem stand in for an item's.)
-// Measured, us, before any of this (2 * CUs / items parts) and as here: chunks of 512 on 32000 keys, 32 / 8 heads of 128, 143 ->
-// 122; 2 x 300 .. 512 on 65000 285 -> 258; 4 x 700 .. 1500 on 30000 .. 60000, 16 / 2 heads, 487 -> 394; 2 x 64 .. 128 on 8000 .. 16000
-// 69 -> 51; sequences by themselves, 32 / 8 heads, 1 x 1024 33 -> 27, 1 x 2048 67 -> 40; 1 x 4096, 8 / 1 heads, 59 -> 45.  With keys counted in
-// place of tiles (2048 and 8192 a part): 1 x 3318 tokens in k blocks of 16, 4 heads of 128, 118, here 84; 2 x 100 on 22000 keys in
-// such blocks, 2 heads, 109 and 94.
+// Measured, us, before any of this (2 * CUs / items parts) and as here: chunks of 512 on 32000 keys, 32 / 8 heads of 128, one 113 ->
+// 100, four 294 -> 270; 2 x 300 .. 512 on 65000 271 -> 266 (keep 0.2, blocks of 128); 4 x 700 .. 1500 on 30000 .. 60000, 16 / 2 heads, 460 ->
+// 419; 2 x 64 .. 128 on 8000 .. 16000 59 -> 48; sequences by themselves, 32 / 8 heads, 1 x 1024 33 -> 27, 1 x 2048 67 -> 39; 1 x 4096,
+// 8 / 1 heads, 62 -> 52.  With keys counted in place of tiles (2048 and 8192 a part): 1 x 3318 tokens in k blocks of 16, 4 heads of
+// 128, 118, here 84; 2 x 100 on 22000 keys in such blocks, 2 heads, 109 and 94.
 // At head dim 256 a CU has one place, and parts that fill a single round have nothing behind them that could even out items of
 // unequal sequences: twice the parts, if they stay long (2 x 560 on 12000 keys on average, in blocks of 16, 8 / 1 heads, 641 ->
 // 359; 8 x 6 on 2000 .. 14000, 32 / 4 heads, 341 -> 246).  At 128, where chunks of about one length lose by it (3 x 80 .. 161 on

@@ -7,11 +7,11 @@
 namespace hbsa {
 
 // --------------------------------------------------------------------------------------
-// What bounds it: the stream of K and V rows, each used by at most 16 queries (a 32-query wave slot of the other kernel
-// would be mostly empty, and three of its four wavefronts idle).  So a workgroup is ONE wavefront with its own two tile
+// What bounds it: the stream of K and V rows, each used by a few queries (16 on average and 64 at most; the 32-query wave slots
+// of the other kernel would be mostly empty, and three of its four wavefronts idle).  So a workgroup is ONE wavefront with its own two tile
 // buffers in LDS: no barriers, nothing shared, five of them on a CU at D = 128, each with up to two tiles of 32 keys
 // (16 KB) on their way.  An item (kv head, q block) is cut into parts over its k blocks (ItemParts) whatever the lengths of the
-// sequences; the part that arrives last combines them.  32 sequences of 2000 .. 32000 keys, 32 / 8 heads of 128, bf16, keep
+// sequences; the part that arrives last combines them, or a second launch where items may have more than 16 queries.  32 sequences of 2000 .. 32000 keys, 32 / 8 heads of 128, bf16, keep
 // 0.25: 151 us in the other kernel with a pre-pass, a split and a merge launch, 125 here (4.5 TB/s of K and V); 2 sequences
 // of 3400 .. 8400 keys, 16 / 4 heads of 64: 35 and 12 us; 64 x 10000 .. 40000 keys, 32 heads: 5.7 TB/s.
 //

@@ -20,7 +20,7 @@ import torch
 from . import _lib
 from .utils import calculate_blocks
 
-_NATIVE_HEADDIMS = (32, 64, 128, 256)      # head dims the forward kernels are instantiated for; others run zero-padded
+_NATIVE_HEADDIMS = (32, 64, 128, 256)      # head dims every form of the forward has kernels for; others run zero-padded here
 _BWD_MAX_HEADDIM = 128                      # the backward kernels stop here
 _DTYPE_CODES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16, torch.float32: _lib.DTYPE_F32}
 

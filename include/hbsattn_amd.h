@@ -72,14 +72,18 @@ int hbsa_set_onepass(int on);   /* see hbsa_fwd */
 /* Launches an hbsa_fwd call with these sizes would make on `stream` right now: 1 when its one-launch form
  * applies (the call then needs no workspace), else 2 (pre-pass and attention kernel; for HBSA_DTYPE_F32 the
  * attention kernel alone, on a workspace; more for
- * HBSA_DTYPE_F32_STAGED16 and for work split over key blocks).  Host-side only, nothing is launched. */
+ * HBSA_DTYPE_F32_STAGED16 and for work split over key blocks).  It knows no total_q and takes every q block as full;
+ * calls that hbsa_fwd_decodes says 1 to are not its subject.  Host-side only, nothing is launched. */
 int hbsa_fwd_launches(int32_t dtype, int32_t batch, int32_t total_k, int32_t nhead_q, int32_t nhead_k,
                       int32_t headdim, int32_t num_q_block, int32_t num_k_block,
                       int32_t q_block_size, int32_t k_block_size, int64_t mask_kblk_stride, void *stream);
 
 /* 1 when calls of these sizes go to the kernel for few queries per q block (decode steps, drafts; bf16 / fp16, head dims
- * 32, 64, 128 and 256).  Such a call of hbsa_fwd needs no workspace, whatever hbsa_fwd_launches says; with one it cuts its
- * items into parts over their k blocks and writes their partial results there.  Host-side only. */
+ * 32, 64, 128 and 256).  Such a call of hbsa_fwd needs no workspace, whatever hbsa_fwd_launches says; with one of
+ * hbsa_fwd_workspace_bytes_dtype(...) + hbsa_fwd_parts_bytes(...) bytes it cuts its items into parts over their k blocks and
+ * writes their partial results there.  One launch; where items are cut one more when an item may have more than 16 (q head of
+ * its group, row) entries (the combination), and one more, which clears counters, on a stream that is being captured or has
+ * no launch record.  Host-side only. */
 int hbsa_fwd_decodes(int32_t dtype, int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t num_q_block,
                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size);
 
@@ -193,7 +197,9 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
  * read the boundaries and the mask bytes itself: mask_kblk stride 1, at most 127 sequences, work that
  * would neither be split over key blocks (hbsa_fwd_split_workspace_bytes) nor use the clocked walk,
  * `stream` not being captured into a graph, and fewer than 64 other streams of the device having made such
- * calls.  The launch record (work-queue counters) of that form lives in device memory inside the library,
+ * calls.  (A call with few queries per q block, see hbsa_fwd_decodes, goes to a kernel of its own that reads boundaries and
+ * mask itself under none of these conditions, and writes partial results to `workspace` where it is large enough.)  The
+ * launch record (work-queue counters) of that form lives in device memory inside the library,
  * one record per stream, so calls on different streams may overlap; it replaces the reference kernel's
  * per-program scan of the mask (reference hbsattn/fwd_triton_auto_tile_size.py:153-164) and the
  * launcher's two host synchronisations (:276-277) with nothing at all.  Results are bitwise those of the
@@ -205,8 +211,8 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
  * Supported: headdim in {32, 64, 128, 256} (the reference pads any head dim to the next power of two,
  * reference hbsattn/fwd_triton_auto_tile_size.py:269; callers do the same with zero columns up to one of
  * these); q_block_size, k_block_size positive multiples of 16; nhead_q % nhead_k == 0; every sequence
- * length >= 1.  At headdim 256 a CU runs one workgroup of four wavefronts whose operand reads the compiler
- * schedules: it works, at about two thirds of the efficiency of headdim 128.  Query rows with no
+ * length >= 1; hbsa_fwd_one takes other head dims too.  At headdim 256 a CU runs one workgroup of four wavefronts whose
+ * operand reads the compiler schedules: it works, at about two thirds of the efficiency of headdim 128.  Query rows with no
  * visible key produce exactly 0 (reference hbsattn/reference.py:97-98).
  */
 int hbsa_fwd(const void *q, const void *k, const void *v, void *out,
