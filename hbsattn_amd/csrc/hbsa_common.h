@@ -43,7 +43,7 @@ constexpr int kDecodeMaxParts = 32;    // parts of an item of the decode kernel
 constexpr int kDecodeEntries = 64;     // (q head, row) entries of an item of the decode kernel, as the host bounds them
 constexpr int kMaxPartItems = 4096;   // items of a launch that may be cut into parts (its arrival counters)
 constexpr int kMaxDevices = 64;            // devices of one process the launch caches cover
-constexpr float kLazyRescaleLog2 = 8.0f;  // running max may lag the true max by 2^8
+constexpr float kLazyRescaleLog2 = 8.0f;  // the reference of a row's exponentials may lag the true maximum by 2^8
 
 // Geometry of one q block, written by the pre-pass (48 bytes).
 struct QBlockInfo {
@@ -245,12 +245,11 @@ struct Sched {
   uint32_t done;       // workgroups of the running attention launch that have made their last claim
   // fp32 inputs staged as fp16 only (written by hbsa_setup_kernel, read by the attention kernel at its start):
   float c;             // |softmax_scale| * log2(e), divided by the q and k staging multipliers
-  float lag;           // kLazyRescaleLog2 / c, in raw score units
   float out_mul;       // 1 / (v staging multiplier)
   // bit patterns of max|x| over q, k, v and the power-of-two staging multipliers
   uint32_t amax[3];
   float in_mul[3];
-  uint32_t pad[46];
+  uint32_t pad[47];
 };
 static_assert(sizeof(Sched) == 256, "Sched is one 256-byte slot of the workspace");
 

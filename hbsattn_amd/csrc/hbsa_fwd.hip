@@ -185,7 +185,6 @@ __global__ void hbsa_setup_kernel(Sched *s, float c, int f32) {
     out_mul = 1.f / mul[2];
   }
   s->c = c;
-  s->lag = kLazyRescaleLog2 / c;
   s->out_mul = out_mul;
 }
 

@@ -47,6 +47,8 @@ constexpr int kStaticShare = 8;
 // Bytes of the one-launch form's staging area for one row of block_mask bytes (2048 blocks and the alignment slack)
 constexpr int kMaskWindow = 2048;
 constexpr int kMaskStage = kMaskWindow + 256;
+constexpr float kMostSum = 256.f;   // 2^kLazyRescaleLog2
+static_assert(kLazyRescaleLog2 == 8.0f, "kMostSum");
 
 // Item header in LDS (16 ints).
 enum { H_HK = 0, H_QB, H_SUB, H_TOTAL, H_ROW_BEGIN, H_ROWS, H_KEY_BEGIN, H_Q_POS, H_SHIFT, H_PART, H_T0, H_SEQ, H_NKBLK, H_WORDS = 16 };
@@ -211,10 +213,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
 
   // softmax constants of this launch (uniform): kernel arguments, or for fp32 inputs staged as fp16 what
   // the setup kernel that precedes this launch derived on the device
-  float sm_c = p.c, sm_lag = p.lag, sm_out_mul = 1.f;
+  float sm_c = p.c, sm_out_mul = 1.f;
   if (p.f32) {
     sm_c = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, p.sched->c)));
-    sm_lag = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, p.sched->lag)));
     sm_out_mul = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, p.sched->out_mul)));
   }
   // Leaving: wavefront 0 makes every claim of its workgroup.  Once its last claim has been performed it
@@ -822,7 +823,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
-    float m_run = -INFINITY;  // running reference max, raw (unscaled) score units
+    float m_ref = -INFINITY;  // reference the row's exponentials are formed against, times c (log2 units)
     float l_run = 0.f;        // this lane's share of the row sum
 
     const char *kg = p.k + (int64_t)cur_hk * p.k_h + (int64_t)key_begin * p.k_s;
@@ -893,6 +894,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
           // The tile is processed as two halves of 32 keys so that, inside one wavefront, the
           // matrix cores always have work queued while the vector ALU does the softmax of the
           // other half:   S0, max(S0) | S1 + exp(S0) | PV0 + max(S1), exp(S1) | PV1.
+          const bool first = chunk_base + t == 0;   // the item's first tile gives the reference
           const bool edge = valid < KT || (p.causal && kpos + valid - 1 > wave_kvis_min);
           int lim = valid;                      // keys (of this lane's query) below lim are visible
           if (p.causal) lim = min(lim, lane_kvis - kpos + 1);
@@ -928,50 +930,64 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
 
           if (nx_valid > 0) issue_v(buf ^ 1, nx_vbase, nx_valid);
 
-          // row max of one half, merged into the running max; O and l are rescaled (rarely:
-          // the running max may lag the true one by 2^kLazyRescaleLog2)
-          auto half_rowmax = [&](f32x16 &sh, int key0) {
+          // Largest score of one half in log2 units.  The first reduction step is an instruction the compiler knows, so
+          // that it inserts the wait states an MFMA result needs before the vector ALU may read it; the
+          // hand-written v_max3 steps all depend on that first result.
+          auto half_rowmax = [&](const f32x16 &sh) {
+            float mx = __builtin_amdgcn_fmed3f(sh[0], sh[1], INFINITY);   // = max(sh[0], sh[1])
+#pragma unroll
+            for (int i = 2; i < 16; i += 2) mx = max3(mx, sh[i], sh[i + 1]);
+            return half_max(mx) * sm_c;
+          };
+          auto hide = [&](f32x16 &sh, int key0) {   // keys this lane's query does not see
             if (edge) {
 #pragma unroll
               for (int i = 0; i < 16; ++i)
                 if (key0 + 8 * (i >> 2) + (i & 3) >= lim) sh[i] = -INFINITY;
             }
-            // The first reduction step is an instruction the compiler knows, so that it inserts
-            // the wait states an MFMA result needs before the vector ALU may read it; the
-            // hand-written v_max3 steps all depend on that first result.
-            float mx = __builtin_amdgcn_fmed3f(sh[0], sh[1], INFINITY);   // = max(sh[0], sh[1])
+          };
+          // exponentials of one half against reference m, packed to the element type (two groups of 16 keys); their sum
+          auto half_exp = [&](const f32x16 &sh, float m, short8v &p_lo, short8v &p_hi) {
+            u32x4 w[2];
+            float sum = 0.f;
 #pragma unroll
-            for (int i = 2; i < 16; i += 2) mx = max3(mx, sh[i], sh[i + 1]);
-            mx = half_max(mx);
-            const bool grow = mx > m_run + sm_lag;
-            if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-              const float m_new = grow ? mx : m_run;
-              const float alpha = grow ? __builtin_amdgcn_exp2f((m_run - m_new) * sm_c) : 1.f;
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+              for (int q4 = 0; q4 < 4; ++q4) {
+                const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sh[8 * j + 2 * q4], sm_c, -m));
+                const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sh[8 * j + 2 * q4 + 1], sm_c, -m));
+                w[j][q4] = E::pack2(e0, e1);
+                // fp32 adds, not v_dot2c: the dot instructions share the matrix pipeline and would
+                // stall the MFMAs of the wavefront's neighbour on the SIMD
+                sum += e0 + e1;
+              }
+              asm volatile("" : "+v"(w[j]));   // packed here, or the 32-bit exponentials stay alive until their sum has been looked at
+            }
+            p_lo = __builtin_bit_cast(short8v, w[0]);
+            p_hi = __builtin_bit_cast(short8v, w[1]);
+            return sum;
+          };
+          // Whether the reference was good enough for a half, and if not (rarely, or with a NaN) a better one.  No maximum
+          // is formed: the exponentials are taken against the reference of the halves before, and only a sum (which
+          // has to be formed anyway) above 2^kLazyRescaleLog2 can hide an exponential above it.  Then the maximum is looked
+          // for, the reference moved, O and l rescaled and the exponentials formed again.
+          // In place of a maximum of every half (eight v_max3 in a chain, an exchange between half wavefronts, a rescaled P),
+          // which the exponentials had to wait for.
+          auto settle_half = [&](const f32x16 &sh, float sum, short8v &p_lo, short8v &p_hi) {
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= kMostSum)) != 0, 0)) {
+              const float mx = half_rowmax(sh);
+              const bool grow = mx > m_ref + kLazyRescaleLog2;
+              const float m_new = grow ? mx : m_ref;
+              const float alpha = grow ? __builtin_amdgcn_exp2f(m_ref - m_new) : 1.f;
               l_run *= alpha;
 #pragma unroll
               for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-              m_run = m_new;
+              m_ref = m_new;
+              sum = half_exp(sh, m_ref == -INFINITY ? 0.f : m_ref, p_lo, p_hi);   // (a row that has seen no key yet)
             }
-          };
-          // exponentials of one half, packed to the element type (two groups of 16 keys), row sum
-          auto half_exp = [&](const f32x16 &sh, short8v &p_lo, short8v &p_hi) {
-            const float mc = (m_run == -INFINITY) ? 0.f : m_run * sm_c;
-            u32x4 w[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-              for (int q4 = 0; q4 < 4; ++q4) {
-                const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sh[8 * j + 2 * q4], sm_c, -mc));
-                const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sh[8 * j + 2 * q4 + 1], sm_c, -mc));
-                w[j][q4] = E::pack2(e0, e1);
-                // fp32 adds, not v_dot2c: the dot instructions share the matrix pipeline and would
-                // stall the MFMAs of the wavefront's neighbour on the SIMD
-                l_run += e0 + e1;
-              }
-            p_lo = __builtin_bit_cast(short8v, w[0]);
-            p_hi = __builtin_bit_cast(short8v, w[1]);
+            l_run += sum;
           };
           auto read_vgroup = [&](auto g_, short4v *dst) {   // V^T operands of keys 16*g .. 16*g+15
             constexpr int g = decltype(g_)::value;
@@ -1016,15 +1032,17 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
             short8v p0a, p0b;
             short4v vb[2 * DT];
             read_vgroup(std::integral_constant<int, 0>{}, vb);
-            half_rowmax(s0, 0);
-            half_exp(s0, p0a, p0b);
+            hide(s0, 0);
+            if (first) m_ref = half_rowmax(s0);
+            settle_half(s0, half_exp(s0, m_ref, p0a, p0b), p0a, p0b);
             wait_vgroup(std::integral_constant<int, 0>{}, vb);
             pv_group(p0a, vb);
             read_vgroup(std::integral_constant<int, 1>{}, vb);
             wait_vgroup(std::integral_constant<int, 0>{}, vb);
             pv_group(p0b, vb);
           } else {
-          half_rowmax(s0, 0);
+          hide(s0, 0);
+          if (first) m_ref = half_rowmax(s0);
 
           // ---- S1 = K[32:64] . Q^T   interleaved with   P0 = exp(S0)
           short8v p0a, p0b, p1a, p1b;
@@ -1038,40 +1056,8 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
           short4v vb[2][2 * DT];
           read_vgroup(std::integral_constant<int, 0>{}, vb[0]);
           read_vgroup(std::integral_constant<int, 1>{}, vb[1]);
-          half_exp(s0, p0a, p0b);
-
-          // ---- row max of S1.  P0 was formed under the running max as it stood after S0 and is not
-          // accumulated yet, so if that max has to move now (rare), P0 is rescaled along with O and l.
-          {
-            if (edge) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i)
-                if (32 + 8 * (i >> 2) + (i & 3) >= lim) s1[i] = -INFINITY;
-            }
-            float mx = __builtin_amdgcn_fmed3f(s1[0], s1[1], INFINITY);
-#pragma unroll
-            for (int i = 2; i < 16; i += 2) mx = max3(mx, s1[i], s1[i + 1]);
-            mx = half_max(mx);
-            const bool grow = mx > m_run + sm_lag;
-            if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-              const float m_new = grow ? mx : m_run;
-              const float alpha = grow ? __builtin_amdgcn_exp2f((m_run - m_new) * sm_c) : 1.f;
-              l_run *= alpha;
-#pragma unroll
-              for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-              u32x4 wa = __builtin_bit_cast(u32x4, p0a), wb = __builtin_bit_cast(u32x4, p0b);
-#pragma unroll
-              for (int q4 = 0; q4 < 4; ++q4) {
-                wa[q4] = E::scale_packed(wa[q4], alpha);
-                wb[q4] = E::scale_packed(wb[q4], alpha);
-              }
-              p0a = __builtin_bit_cast(short8v, wa);
-              p0b = __builtin_bit_cast(short8v, wb);
-              m_run = m_new;
-            }
-          }
+          settle_half(s0, half_exp(s0, m_ref, p0a, p0b), p0a, p0b);
+          hide(s1, 32);
 
           // ---- O^T += V^T[:, 0:32] . P0   interleaved with   P1 = exp(S1)
           wait_vgroup(std::integral_constant<int, 2 * DT>{}, vb[0]);
@@ -1080,7 +1066,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
           wait_vgroup(std::integral_constant<int, 2 * DT>{}, vb[1]);
           pv_group(p0b, vb[1]);
           read_vgroup(std::integral_constant<int, 3>{}, vb[1]);
-          half_exp(s1, p1a, p1b);
+          settle_half(s1, half_exp(s1, m_ref, p1a, p1b), p1a, p1b);
 
           // ---- O^T += V^T[:, 32:64] . P1
           wait_vgroup(std::integral_constant<int, 2 * DT>{}, vb[0]);
@@ -1140,7 +1126,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
         if (l32 < nrows) {
           const int64_t rh = ((int64_t)cur_part * p.total_q + (row_begin + my_r)) * p.nhead_q + hq;
           if (g32 == 0)
-            p.part_lse[rh] = l_tot > 0.f ? (m_run * sm_c + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
+            p.part_lse[rh] = l_tot > 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
           float *dst = p.part_out + rh * D;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
@@ -1152,9 +1138,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
         }
       } else {
       if (EXTRAS && p.lse != nullptr && g32 == 0 && l32 < nrows) {
-        // natural-log sum over the row's visible keys of exp(scale * q.k); m_run is the (possibly
+        // natural-log sum over the row's visible keys of exp(scale * q.k); m_ref is the (possibly
         // lagging) reference maximum the row sum was accumulated under, which makes this exact
-        const float lse = l_tot > 0.f ? (m_run * sm_c + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
+        const float lse = l_tot > 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
         p.lse[(int64_t)(row_begin + my_r) * p.lse_s + (int64_t)hq * p.lse_h] = lse;
       }
       if constexpr (OUT32) {
