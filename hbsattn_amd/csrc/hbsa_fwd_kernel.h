@@ -728,8 +728,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // the lane, load A_k takes row (lane % 16), load B_k row 16 + (lane % 16), both at bytes
   // 64*k + 32*h + 16*g32; then the h = 1 lanes of A_k and the h = 0 lanes of B_k trade places
   // (v_permlane16_swap), which leaves k-step 2k in A_k and k-step 2k+1 in B_k.
+  // The loads go out when the item before has formed its last scores; place_q() waits for them when the item begins.
   short8v qf[KSTEPS];
-  auto load_q = [&](int hk, int sub, int row_begin, int rows) {
+  static_assert(KSTEPS % 2 == 0, "the loads come in pairs of k-steps");
+  auto request_q = [&](int hk, int sub, int row_begin, int rows) {
     const Slot sl = slot_of(hk, sub, rows);
     if (sl.n <= 0) return;   // this wavefront has no rows: qf is never used
     const int l16 = lane & 15;
@@ -739,25 +741,29 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     const char *base = p.q + (lane & 16) * 2 + g32 * 16;
     const char *ra = base + (int64_t)(row_begin + r_a) * p.q_s + (int64_t)hq_a * p.q_h;
     const char *rb = base + (int64_t)(row_begin + r_b) * p.q_s + (int64_t)hq_b * p.q_h;
-    if constexpr (KSTEPS >= 2) {
 #pragma unroll
-      for (int k = 0; k < KSTEPS / 2; ++k) {
-        u32x4 a = {0u, 0u, 0u, 0u}, b = a;
-        if (!COLS || 4 * k + ((lane >> 4) & 1) * 2 + g32 < p.ncol) {
-          a = *(const u32x4 *)(ra + 64 * k);
-          b = *(const u32x4 *)(rb + 64 * k);
-        }
-        a ^= p.q_sign;
-        b ^= p.q_sign;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const auto r = __builtin_amdgcn_permlane16_swap(a[j], b[j], false, false);
-          a[j] = r[0];
-          b[j] = r[1];
-        }
-        qf[2 * k] = __builtin_bit_cast(short8v, a);
-        qf[2 * k + 1] = __builtin_bit_cast(short8v, b);
+    for (int k = 0; k < KSTEPS / 2; ++k) {
+      u32x4 a = {0u, 0u, 0u, 0u}, b = a;
+      if (!COLS || 4 * k + ((lane >> 4) & 1) * 2 + g32 < p.ncol) {
+        a = *(const u32x4 *)(ra + 64 * k);
+        b = *(const u32x4 *)(rb + 64 * k);
       }
+      qf[2 * k] = __builtin_bit_cast(short8v, a);
+      qf[2 * k + 1] = __builtin_bit_cast(short8v, b);
+    }
+  };
+  auto place_q = [&]() {
+#pragma unroll
+    for (int k = 0; k < KSTEPS / 2; ++k) {
+      u32x4 a = __builtin_bit_cast(u32x4, qf[2 * k]) ^ p.q_sign, b = __builtin_bit_cast(u32x4, qf[2 * k + 1]) ^ p.q_sign;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const auto r = __builtin_amdgcn_permlane16_swap(a[j], b[j], false, false);
+        a[j] = r[0];
+        b[j] = r[1];
+      }
+      qf[2 * k] = __builtin_bit_cast(short8v, a);
+      qf[2 * k + 1] = __builtin_bit_cast(short8v, b);
     }
   };
 
@@ -776,14 +782,15 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
       issue_loads(0, tile_ptr(p.k + (int64_t)hk * p.k_h, tok, ks32), tile_ptr(p.v + (int64_t)hk * p.v_h, tok, vs32), (e & 63) + 1);
     }
   }
-  load_q(hdr_word(0, H_HK), hdr_word(0, H_SUB), hdr_word(0, H_ROW_BEGIN), hdr_word(0, H_ROWS));
-  if constexpr (FUSED) {
-    // The second item's mask bytes: wavefront 0 builds its list below, before any tile has been waited for.  (load_q waits for
-    // its rows, and so for what was requested before them, but a wavefront that has no rows of the first item loads none.
-    // All wavefronts wait: as a branch of wavefront 0 this costs the 96- and 192-dim kernels 1 to 4 %.)
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    asm volatile("" : : : "memory");
-  }
+  request_q(hdr_word(0, H_HK), hdr_word(0, H_SUB), hdr_word(0, H_ROW_BEGIN), hdr_word(0, H_ROWS));
+  // What this wavefront asked for so far has arrived, the scheduler's records included: the compiler is told here, or it
+  // waits for ALL outstanding memory traffic where they are first read.
+  bool settled = false;   // ... since the scheduler last asked for something
+  auto settle = [&]() {
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+    asm volatile("" : "+v"(st_info), "+v"(st_bits), "+v"(pending), "+v"(w_clk));
+    settled = true;
+  };
 
   for (;;) {   // ------------------------------------------------------ one iteration per work item
     const int cur_hk = hdr_word(c, H_HK);
@@ -796,11 +803,17 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     const int q_pos = hdr_word(c, H_Q_POS);
     const int shift = hdr_word(c, H_SHIFT);
 
+    // The q rows were requested after the item's first tile, and a wavefront's loads return in order: once it has put them in
+    // place its part of that tile is there as well.  What the scheduler asks for below then has the first tile's time to arrive.
+    // (In every wavefront: the compiler then knows that these loads have arrived.)
+    place_q();
     if (wave == 0) {   // stay one item ahead: expand the staged item, stage the one after it
+      if (!settled) settle();   // (the staged item's mask bytes among what it waits for: no tile of the item before may have been waited for)
       build(c ^ 1);
       if (EXTRAS && p.walk) note_item(c ^ 1, hdr_word(c ^ 1, H_TOTAL));
       stage();
       pending = claim();
+      settled = false;
     }
 
     const Slot slot = slot_of(cur_hk, cur_sub, rows);
@@ -842,10 +855,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
         const int e = __builtin_amdgcn_readlane(held, t & 63);
         const int kpos = (e >> 6) << 4, valid = (e & 63) + 1;
 
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the current tile has landed in LDS
-        // Everything fetched so far has arrived, the scheduler's records included: tell the
-        // compiler here, or it waits for ALL outstanding memory traffic where they are first read.
-        asm volatile("" : "+v"(st_info), "+v"(st_bits), "+v"(pending), "+v"(w_clk));
+        if (t > 0 || chunk_base > 0 || !active) settle();   // the current tile has landed in LDS
         __syncthreads();                     // ... for every wave, and the other buffers are free
 
         const bool last = chunk_base + t + 1 == total;
@@ -1075,11 +1085,6 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
           pv_group(p1b, vb[1]);
           }
         }
-        if (last && nxt_hk >= 0) {
-          // Q of this item is no longer needed: fetch the next item's rows while the last MFMAs
-          // drain and the epilogue runs
-          load_q(nxt_hk, hdr_word(c ^ 1, H_SUB), hdr_word(c ^ 1, H_ROW_BEGIN), hdr_word(c ^ 1, H_ROWS));
-        }
         flip_buffers();
       }
       chunk_base += n;
@@ -1114,6 +1119,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
         issue_loads(buf, tile_ptr(kg, tok, ks32), tile_ptr(vg, tok, vs32), (e & 63) + 1);
       }
     }
+
+    // Q of this item is no longer needed: the next item's rows are requested while the last MFMAs drain and the epilogue runs
+    // (outside of the tile loop, or the compiler waits for them inside it)
+    if (nxt_hk >= 0) request_q(nxt_hk, hdr_word(c ^ 1, H_SUB), hdr_word(c ^ 1, H_ROW_BEGIN), hdr_word(c ^ 1, H_ROWS));
 
     // ---- epilogue: normalise, convert, store (rows with no visible key store exact zeros)
     if (active) {
@@ -1201,7 +1210,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
       // No tile, hence no barrier since this item began: the next list may still be being written,
       // and nothing of the next item has been requested yet.
       w_next_lap = -1;   // (nor has its walk been given a start: it takes no part in the clock)
-      __builtin_amdgcn_s_waitcnt(0x0F70);   // keeps "every fetch has arrived" true on every path
+      settle();
       __syncthreads();
       nxt_hk = hdr_word(c ^ 1, H_HK);
       if (nxt_hk >= 0) {
@@ -1211,7 +1220,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
           issue_loads(buf, tile_ptr(p.k + (int64_t)nxt_hk * p.k_h, tok, ks32), tile_ptr(p.v + (int64_t)nxt_hk * p.v_h, tok, vs32),
                       (e1 & 63) + 1);
         }
-        load_q(nxt_hk, hdr_word(c ^ 1, H_SUB), hdr_word(c ^ 1, H_ROW_BEGIN), hdr_word(c ^ 1, H_ROWS));
+        request_q(nxt_hk, hdr_word(c ^ 1, H_SUB), hdr_word(c ^ 1, H_ROW_BEGIN), hdr_word(c ^ 1, H_ROWS));
       }
       __syncthreads();   // wave 0 rewrites this item's list next; every wave has read its header by now
     }
