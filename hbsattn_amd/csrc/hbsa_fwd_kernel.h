@@ -160,6 +160,7 @@ struct FwdSwizzle {
   static constexpr int CPR = D / 8;
   static constexpr int RPG = 16 / CPR > 0 ? 16 / CPR : 1;   // rows per 256-byte bank sweep
   static constexpr bool POW2 = (CPR & (CPR - 1)) == 0;
+  static constexpr int PERIOD = RPG * CPR;   // rows after which the placement repeats (POW2)
   static __device__ __forceinline__ int k(int r) { return POW2 ? (r / RPG) % CPR : CPR % 8 == 0 ? (r >> 1) & 7 : (r >> 2) & 3; }
   static __device__ __forceinline__ int v(int r) {
     return POW2 ? (CPR >= 8 ? ((r / RPG) % (CPR / 4)) << 2 : 0) : CPR % 8 == 0 ? ((r >> 1) & 1) << 2 : 0;
@@ -167,7 +168,7 @@ struct FwdSwizzle {
 };
 
 template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS>
-__global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel(FwdParams p) {
+__global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3 : 4) void hbsa_fwd_kernel(FwdParams p) {
   // OUT32: fp32 output (the fp32-input path; q/k/v are then fp16 staging copies)
   // EXTRAS: the clocked walk, the split over key blocks and the log-sum-exp output are compiled in.  The
   // plain call uses none of them, and its kernel is a tenth shorter without them (1-2 % faster: eight
@@ -211,6 +212,14 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   const int g32 = lane >> 5;   // which half of the wavefront
   const int l32 = lane & 31;   // query within the wave slot / key row within a sub-tile
 
+  // The launch's arguments, for what is done once an item: read again (scalar loads) each time.  Held in scalar registers over
+  // the tile loop they do not fit: 100 to 240 of them went to lanes of vector registers.
+  auto fresh_args = [&]() -> const FwdParams & {
+    auto at = (const __attribute__((address_space(4))) FwdParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(at));
+    return *(const FwdParams *)at;
+  };
+
   // softmax constants of this launch (uniform): kernel arguments, or for fp32 inputs staged as fp16 what
   // the setup kernel that precedes this launch derived on the device
   float sm_c = p.c, sm_out_mul = 1.f;
@@ -244,6 +253,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   uint32_t st_info = 0, st_bits = 0;       // lane i: word i of its QBlockInfo / of its bit row
 
   auto queue_len = [&](int v) -> uint32_t {
+    const FwdParams &p = fresh_args();
     const int heads = v < p.nhead_k ? (p.nhead_k - v + 7) / 8 : 0;
     return (uint32_t)heads * (uint32_t)p.nqb * (uint32_t)p.nsub * (uint32_t)p.nparts;
   };
@@ -255,6 +265,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // counter for the later rounds, 8 x 1024 tokens 106 -> 99 us and C5 0.258 -> 0.241 ms.
   int own_claims = 0;
   auto claim = [&]() -> uint32_t {   // the value is looked at an item later, so its latency is hidden
+    const FwdParams &p = fresh_args();
     uint32_t r = 0xffffffffu;
     if (p.one_each) {
       r = (own_claims & 1) ? (uint32_t)(own_claims + 1) * gridDim.x - 1u - blockIdx.x : (uint32_t)own_claims * gridDim.x + blockIdx.x;
@@ -267,6 +278,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // (kv head, q block, slot group, part) of entry `claimed` of a head-major list that starts at kv head
   // `head0` and holds every `head_step`-th head
   auto decode_entry = [&](uint32_t claimed, int head0, int head_step) {
+    const FwdParams &p = fresh_args();
     const uint32_t whole = fast_div(claimed, p.div_nparts);   // parts of one item are neighbours
     st_part = (int)(claimed - whole * (uint32_t)p.nparts);
     const uint32_t t = fast_div(whole, p.div_nsub);
@@ -278,6 +290,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // (kv head, q block, slot group, part) of item `claimed` of the numbering without queues: parts, slot groups and
   // kv heads of a q block are neighbours, the last q block comes first
   auto decode_free_entry = [&](uint32_t claimed) {
+    const FwdParams &p = fresh_args();
     const uint32_t whole = fast_div(claimed, p.div_nparts);
     st_part = (int)(claimed - whole * (uint32_t)p.nparts);
     const uint32_t t = fast_div(whole, p.div_nsub);
@@ -295,6 +308,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   int seq_qb_end = -1;      // q blocks [seq_sb.qb0, seq_qb_end) belong to the kept sequence (none at first)
   bool seq_have = false;
   auto fused_geometry = [&](int qb, int &kb0) -> QBlockInfo {
+    const FwdParams &p = fresh_args();
     if (!(qb >= seq_sb.qb0 && qb < seq_qb_end)) {
       int b = 0;   // sequences that start at or before qb, minus one
       for (int base = 0; base < p.batch; base += 64) {
@@ -372,6 +386,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   // turn `pending` into the staged item (claiming again from the next queues when the one it
   // came from is exhausted) and start fetching the item's records
   auto stage = [&]() {
+    const FwdParams &p = fresh_args();
     uint32_t claimed = (uint32_t)__builtin_amdgcn_readfirstlane((int)pending);
     st_hk = -1;
     if (p.one_each) {
@@ -422,6 +437,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   };
   // expand the staged item into list `c` and write its header
   auto build = [&](int c) {
+    const FwdParams &p = fresh_args();
     int *hdr = lds_hdr + c * H_WORDS;
     int total = 0;
     if (st_hk >= 0) {
@@ -472,6 +488,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   int w_tiles_of[2] = {1, 1};
   bool w_part_of[2] = {false, false};
   auto note_item = [&](int c_, int total_) {   // right after build(c_), from the staged records
+    const FwdParams &p = fresh_args();
     const int nkblk = __builtin_amdgcn_readlane((int)st_info, 6);
     const int seq = __builtin_amdgcn_readlane((int)st_info, 8);
     w_part_of[c_] = EXTRAS && p.walk != 0 && st_hk >= 0 && total_ >= 3 && total_ <= kListCap;
@@ -568,8 +585,12 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
 
   // ------------------------------------------------------------------ per-thread constants
   // tile loads: thread -> (row, 16-byte chunk) of the tile, same for every tile
-  uint32_t ld_koff[LOADS], ld_voff[LOADS];   // byte offset of the thread's chunk from the tile's first row
-  bool ld_kin[LOADS], ld_vin[LOADS];         // COLS: the chunk is one of the row's
+  // Where a round of the workgroup's loads is a whole number of rows after which the chunk placement repeats, the rounds
+  // differ in their scalar base only; elsewhere every load has its offset in a register.
+  constexpr bool UNIFORM = (64 * NW) % CPR == 0 && SW::POW2 && (64 * NW / CPR) % SW::PERIOD == 0;
+  constexpr int ROUND_ROWS = UNIFORM ? 64 * NW / CPR : 0, OFFSETS = UNIFORM ? 1 : LOADS;
+  uint32_t ld_koff[OFFSETS], ld_voff[OFFSETS];   // byte offset of the thread's chunk from the tile's first row
+  bool ld_kin[LOADS], ld_vin[LOADS];             // COLS: the chunk is one of the row's
   const uint32_t ks32 = (uint32_t)p.k_s, vs32 = (uint32_t)p.v_s;   // row strides in bytes (the host checks they fit)
   auto ld_place = [&](int i, int &r, uint32_t &kchunk, uint32_t &vchunk) {
     const int c = (i * NW + wave) * 64 + lane;
@@ -582,8 +603,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   for (int i = 0; i < LOADS; ++i) {
     int r; uint32_t kc, vc;
     ld_place(i, r, kc, vc);
-    ld_koff[i] = (uint32_t)r * ks32 + kc;
-    ld_voff[i] = (uint32_t)r * vs32 + vc;
+    if (i < OFFSETS) {
+      ld_koff[i] = (uint32_t)r * ks32 + kc;
+      ld_voff[i] = (uint32_t)r * vs32 + vc;
+    }
     ld_kin[i] = !COLS || kc < (uint32_t)p.ncol * 16u;
     ld_vin[i] = !COLS || vc < (uint32_t)p.ncol * 16u;
   }
@@ -610,16 +633,17 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
         if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))   // (a lane that loads nothing leaves its 16 bytes of LDS alone)
-        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, V_PART ? ld_voff[i] : ld_koff[i], l0);
+        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base + (uint64_t)(uint32_t)(i * ROUND_ROWS) * (V_PART ? vs32 : ks32),
+              V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i], l0);
       });
     } else {   // ragged tail of a run: rows past the end re-read the last valid row (masked later)
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
-        int r; uint32_t kc, vc;
-        ld_place(i, r, kc, vc);
-        r = min(r, valid - 1);
+        const int r0 = ((UNIFORM ? 0 : i * NW) * 64 + wave * 64 + lane) / CPR;
+        uint32_t step = (uint32_t)(min(r0 + i * ROUND_ROWS, valid - 1) - r0) * (V_PART ? vs32 : ks32);
+        asm volatile("" : "+v"(step));   // (or a 64-bit multiply-add is formed, and its 64-bit addend kept in registers)
         if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))
-        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, (uint32_t)r * (V_PART ? vs32 : ks32) + (V_PART ? vc : kc), l0);
+        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, (V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i]) + step, l0);
       });
     }
   };
@@ -682,6 +706,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
   };
   auto slot_of = [&](int hk, int sub, int rows) -> Slot {
+    const FwdParams &p = fresh_args();
     const int slot = sub * NW + wave;
     Slot sl;
     if constexpr (PACK) {
@@ -732,6 +757,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
   short8v qf[KSTEPS];
   static_assert(KSTEPS % 2 == 0, "the loads come in pairs of k-steps");
   auto request_q = [&](int hk, int sub, int row_begin, int rows) {
+    const FwdParams &p = fresh_args();
     const Slot sl = slot_of(hk, sub, rows);
     if (sl.n <= 0) return;   // this wavefront has no rows: qf is never used
     const int l16 = lane & 15;
@@ -753,6 +779,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     }
   };
   auto place_q = [&]() {
+    const FwdParams &p = fresh_args();
 #pragma unroll
     for (int k = 0; k < KSTEPS / 2; ++k) {
       u32x4 a = __builtin_bit_cast(u32x4, qf[2 * k]) ^ p.q_sign, b = __builtin_bit_cast(u32x4, qf[2 * k + 1]) ^ p.q_sign;
@@ -839,8 +866,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
     float m_ref = -INFINITY;  // reference the row's exponentials are formed against, times c (log2 units)
     float l_run = 0.f;        // this lane's share of the row sum
 
-    const char *kg = p.k + (int64_t)cur_hk * p.k_h + (int64_t)key_begin * p.k_s;
-    const char *vg = p.v + (int64_t)cur_hk * p.v_h + (int64_t)key_begin * p.v_s;
+    const FwdParams &pi = fresh_args();
+    const char *kg = pi.k + (int64_t)cur_hk * pi.k_h + (int64_t)key_begin * pi.k_s;
+    const char *vg = pi.v + (int64_t)cur_hk * pi.v_h + (int64_t)key_begin * pi.v_s;
 
     int nxt_hk = -1;          // known once the last tile is reached
     int chunk_base = 0;
@@ -888,8 +916,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
             const int e1 = __builtin_amdgcn_readfirstlane(lds_list[(c ^ 1) * kListCap + hdr_word(c ^ 1, H_T0)]);
             const int tok = hdr_word(c ^ 1, H_KEY_BEGIN) + ((e1 >> 6) << 4);
             nx_valid = (e1 & 63) + 1;
-            nx_vbase = tile_ptr(p.v + (int64_t)nxt_hk * p.v_h, tok, vs32);
-            nx_kbase = tile_ptr(p.k + (int64_t)nxt_hk * p.k_h, tok, ks32);
+            const FwdParams &pn = fresh_args();
+            nx_vbase = tile_ptr(pn.v + (int64_t)nxt_hk * pn.v_h, tok, vs32);
+            nx_kbase = tile_ptr(pn.k + (int64_t)nxt_hk * pn.k_h, tok, ks32);
           }
         }
         // The next tile's K is requested right after this tile's first operand reads, its V only after
@@ -1093,6 +1122,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
       __syncthreads();
       if (wave == 0) {
         // (the staged records now belong to a later item, so this item's are fetched again)
+        const FwdParams &p = fresh_args();
         const int qb = hdr_word(c, H_QB);
         if constexpr (FUSED) {
           int kb0;
@@ -1126,6 +1156,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : 8 / NW) void hbsa_fwd_kernel
 
     // ---- epilogue: normalise, convert, store (rows with no visible key store exact zeros)
     if (active) {
+      const FwdParams &p = fresh_args();
       int hq, my_r;   // this lane's query (lanes l32 >= nrows repeat the last one and store nothing)
       slot_entry(slot, l32, rows, hq, my_r);
       const float l_tot = half_sum(l_run);
