@@ -196,17 +196,46 @@ __device__ __forceinline__ void bwd_store_rows(char *row_ptr, const f32x16 *acc,
     }
 }
 
-// The dK/dV kernels' check of the sequence b their k block belongs to.  A sequence the pre-pass found not to
-// fit the tensors (flagged q block records, no bit rows) takes no part: its keys get zero gradients where they
-// lie inside dk and dv, and the workgroup is done.
+// The sequence a k block belongs to: what the dK/dV kernels need of it from the caller's arrays.  All three arrays are asked
+// for at once, a sequence per lane (one wait in place of one per sequence passed and two more behind it).
+struct BwdSequence {
+  int k0, k1, kb0, qb0, qb1;   // keys [k0, k1), first k block, q blocks [qb0, qb1)
+  __device__ __forceinline__ BwdSequence(const BwdParams &p, int kb, int lane) {
+    if (p.batch < 64) {
+      const int i = min(lane, p.batch);
+      const int nkb = p.cu_num_k_block[i], k = p.cu_k[i], nqb = p.cu_num_q_block[i];
+      // the last sequence reached from the first one by steps to a sequence that starts at or before kb
+      const uint64_t starts = __builtin_amdgcn_ballot_w64(lane >= 1 && lane < p.batch && nkb <= kb);
+      const int b = __builtin_ctzll(~(starts >> 1));
+      k0 = __builtin_amdgcn_readlane(k, b);
+      k1 = __builtin_amdgcn_readlane(k, b + 1);
+      kb0 = __builtin_amdgcn_readlane(nkb, b);
+      qb0 = __builtin_amdgcn_readlane(nqb, b);
+      qb1 = __builtin_amdgcn_readlane(nqb, b + 1);
+    } else {
+      int b = 0;
+      while (b + 1 < p.batch && p.cu_num_k_block[b + 1] <= kb) ++b;
+      k0 = p.cu_k[b];
+      k1 = p.cu_k[b + 1];
+      kb0 = p.cu_num_k_block[b];
+      qb0 = p.cu_num_q_block[b];
+      qb1 = p.cu_num_q_block[b + 1];
+    }
+  }
+  // the sequence's keys lie inside the tensors, and the k block inside the sequence's numbering
+  __device__ __forceinline__ bool fits(const BwdParams &p, int kb) const { return k0 >= 0 && k1 >= k0 && k1 <= p.total_k && kb >= kb0; }
+};
+// The record of the sequence's first q block, a word per lane (nullptr words: no q blocks).
+__device__ __forceinline__ uint32_t bwd_first_record(const BwdParams &p, const BwdSequence &s, int lane) {
+  return s.qb0 < s.qb1 && lane < 12 ? ((const uint32_t *)(p.info + s.qb0))[lane] : 0u;
+}
+// A sequence the pre-pass found not to fit the tensors (flagged q block records, no bit rows) takes no part: its keys get zero
+// gradients where they lie inside dk and dv.
 template <int D>
-__device__ __forceinline__ bool bwd_sequence_skipped(const BwdParams &p, int b, int kb, int sub, int hk) {
-  const int first_qb = p.cu_num_q_block[b];
-  if (first_qb < 0 || first_qb >= p.nqb) return true;
-  if (first_qb >= p.cu_num_q_block[b + 1] || p.info[first_qb].flags == 0) return false;
-  const int64_t k0 = p.cu_k[b], k1 = p.cu_k[b + 1];
-  const int kbl = kb - p.cu_num_k_block[b];
-  if (k0 < 0 || k1 <= k0 || kbl < 0) return true;
+__device__ __forceinline__ void bwd_zero_keys(const BwdParams &p, const BwdSequence &s, int kb, int sub, int hk) {
+  const int64_t k0 = s.k0, k1 = s.k1;
+  const int kbl = kb - s.kb0;
+  if (k0 < 0 || k1 <= k0 || kbl < 0) return;
   const int64_t first = k0 + (int64_t)kbl * p.kbs + (int64_t)sub * 4 * kWaveRows;
   int64_t stop = k0 + (int64_t)(kbl + 1) * p.kbs;
   stop = stop < k1 ? stop : k1;
@@ -219,7 +248,6 @@ __device__ __forceinline__ bool bwd_sequence_skipped(const BwdParams &p, int b, 
     *(u32x4 *)(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h + c * 16) = zero;
     *(u32x4 *)(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h + c * 16) = zero;
   }
-  return true;
 }
 
 // ---- Items cut into parts (PARTS instantiations) -------------------------------------------------------
@@ -348,6 +376,8 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   // last q blocks first: under a causal mask they are the long ones, and the grid should not end on them
   const int qb_rev = bx / p.nsub, sub = bx - qb_rev * p.nsub;
   const int qb = p.nqb - 1 - qb_rev;
+  const uint32_t *bits = p.bits + ((size_t)hk * p.nqb + qb) * p.wpr;
+  const uint32_t first_words = !PARTS && lane < p.wpr ? bits[lane] : 0u;
   const QBlockInfo inf = p.info[qb];
   if (inf.rows <= 0) return;   // a q block with no row inside the tensors (its sequence did not fit them)
   int blk_begin = 0, blk_end = inf.nkblk;   // k blocks of this part
@@ -366,49 +396,28 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   const bool active = head_in_group < p.ratio && nrows > 0;
   const int hq = hk * p.ratio + head_in_group;
 
-  short8v qf[T::KSTEPS], dof[T::KSTEPS];   // Q^T and dO^T fragments: lane holds row l32, d = 16*ks + 8*g32 .. +7
-  float lse2 = INFINITY, dlt = 0.f;         // a row that takes no part gets P = exp2(-inf) = 0
+  // Asked for together: the rows of Q, dO and O, and below the first tiles.  (One after the other they cost every workgroup two
+  // waits for memory before its first product.)
+  short8v qf[T::KSTEPS], dof[T::KSTEPS], of[T::KSTEPS];   // Q^T, dO^T and O^T fragments: lane holds row l32, d = 16*ks + 8*g32 .. +7
+  float row_lse = 0.f;
   const int my_row = inf.row_begin + min(row0 + l32, inf.rows - 1);
   if (active) {
     const char *qrow = p.q + (int64_t)my_row * p.q_s + (int64_t)hq * p.q_h + g32 * 16;
     const char *grow = p.dout + (int64_t)my_row * p.do_s + (int64_t)hq * p.do_h + g32 * 16;
-#pragma unroll
-    for (int ks = 0; ks < T::KSTEPS; ++ks) {
-      qf[ks] = *(const short8v *)(qrow + ks * 32);
-      dof[ks] = *(const short8v *)(grow + ks * 32);
-    }
-    const float l = p.lse[(int64_t)my_row * p.nhead_q + hq];
-    lse2 = l == -INFINITY ? INFINITY : l * kLog2e;
-    // delta = sum over d of dO * O of the row: this lane's half of the head dim, then the other half's from lane + 32.
-    // Every (row, q head) belongs to exactly one wavefront of this grid, which also leaves it for the dK/dV kernel.
     const char *orow = p.out + (int64_t)my_row * p.o_s + (int64_t)hq * p.o_h + g32 * 16;
+    row_lse = p.lse[(int64_t)my_row * p.nhead_q + hq];
 #pragma unroll
     for (int ks = 0; ks < T::KSTEPS; ++ks) {
-      const u32x4 a = __builtin_bit_cast(u32x4, dof[ks]), b = *(const u32x4 *)(orow + ks * 32);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        dlt += E::lo(a[j]) * E::lo(b[j]);
-        dlt += E::hi(a[j]) * E::hi(b[j]);
-      }
-    }
-    dlt = half_sum(dlt);
-    if (g32 == 0 && l32 < nrows && (!PARTS || part == 0)) {
-      p.delta[(int64_t)hq * p.total_q + my_row] = dlt;
-      p.lse2[(int64_t)hq * p.total_q + my_row] = lse2;
+      dof[ks] = *(const short8v *)(grow + ks * 32);
+      of[ks] = *(const short8v *)(orow + ks * 32);
+      qf[ks] = *(const short8v *)(qrow + ks * 32);
     }
   } else {
 #pragma unroll
-    for (int ks = 0; ks < T::KSTEPS; ++ks) { qf[ks] = short8v{0, 0, 0, 0, 0, 0, 0, 0}; dof[ks] = qf[ks]; }
+    for (int ks = 0; ks < T::KSTEPS; ++ks) { qf[ks] = short8v{0, 0, 0, 0, 0, 0, 0, 0}; dof[ks] = of[ks] = qf[ks]; }
   }
-  f32x16 acc[T::DT];
-#pragma unroll
-  for (int dt = 0; dt < T::DT; ++dt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
-
   const int lane_kvis = inf.q_pos + min(row0 + l32, inf.rows - 1) + inf.shift;   // last key position the row sees (causal)
   const int wave_kvis_min = inf.q_pos + min(row0, inf.rows - 1) + inf.shift;      // ... the wavefront's first row sees
-  const uint32_t *bits = p.bits + ((size_t)hk * p.nqb + qb) * p.wpr;
   const char *kg = p.k + (int64_t)hk * p.k_h + (int64_t)inf.key_begin * p.k_s;
   const char *vg = p.v + (int64_t)hk * p.v_h + (int64_t)inf.key_begin * p.v_s;
 
@@ -420,7 +429,8 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   // stand between two tiles.
   const int last_word = (blk_end - 1) >> 5;
   const int word_at = PARTS ? ((blk_begin >> 5) & ~63) + lane : lane;
-  uint32_t row_words = word_at <= last_word ? bits[word_at] : 0u;
+  uint32_t row_words = PARTS ? (word_at <= last_word ? bits[word_at] : 0u) : first_words;
+  if (word_at > last_word) row_words = 0u;   // (only the words of the sequence's blocks have been written)
   auto next_tile = [&]() -> bool {
     if (j >= 0) {
       kpos += kTileKeys;
@@ -475,6 +485,47 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   auto fetch_v = [&](int vb, int at, int valid) {
     fetch_one(tiles_addr + (uint32_t)((3 + vb) * T::TILE_BYTES), vg + (int64_t)at * p.v_s, p.v_s, v_s32, v_voff, valid);
   };
+  bool have_c = next_tile(), have_n = false;   // the current tile exists; the one after it exists (its K is requested)
+  int kpos_c = 0, valid_c = 0, kpos_n = 0, valid_n = 0;
+  int kb = 0, vb = 0;   // K and V buffer of the current tile
+  if (have_c) {
+    kpos_c = kpos;
+    valid_c = tile_valid();
+    fetch_k(0, kpos_c, valid_c);
+    fetch_v(0, kpos_c, valid_c);
+    have_n = next_tile();
+    if (have_n) {
+      kpos_n = kpos;
+      valid_n = tile_valid();
+      fetch_k(1, kpos_n, valid_n);
+    }
+  }
+  float lse2 = INFINITY, dlt = 0.f;         // a row that takes no part gets P = exp2(-inf) = 0
+  if (active) {
+    lse2 = row_lse == -INFINITY ? INFINITY : row_lse * kLog2e;
+    // delta = sum over d of dO * O of the row: this lane's half of the head dim, then the other half's from lane + 32.
+    // Every (row, q head) belongs to exactly one wavefront of this grid, which also leaves it for the dK/dV kernel.
+#pragma unroll
+    for (int ks = 0; ks < T::KSTEPS; ++ks) {
+      const u32x4 a = __builtin_bit_cast(u32x4, dof[ks]), b = __builtin_bit_cast(u32x4, of[ks]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        dlt += E::lo(a[j]) * E::lo(b[j]);
+        dlt += E::hi(a[j]) * E::hi(b[j]);
+      }
+    }
+    dlt = half_sum(dlt);
+    if (g32 == 0 && l32 < nrows && (!PARTS || part == 0)) {
+      p.delta[(int64_t)hq * p.total_q + my_row] = dlt;
+      p.lse2[(int64_t)hq * p.total_q + my_row] = lse2;
+    }
+  }
+  f32x16 acc[T::DT];
+#pragma unroll
+  for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
+
   // Operand addresses of the K tile in use: they move to the next buffer with one addition per tile instead of
   // one per read (the V tile's reads add the distance between the two buffers in use).
   BwdOperandOffsets<D> off;
@@ -491,25 +542,10 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   constexpr int PF = 4, NC = 2 * T::KSTEPS;
   static_assert(NC >= PF, "the first reads of a half are issued as one group");
   static_assert(LOADS <= 15, "vmcnt immediate");
-  // What was loaded so far (the rows' Q above all, first used in the loop) has arrived before the first tile is
-  // requested: the compiler counts only the loads it knows, and a wait of its own for them inside the loop would
+  // What was loaded so far (the rows' Q above all, first used in the loop) has arrived before the loop begins, and with it the
+  // tiles requested behind it: the compiler counts only the loads it knows, and a wait of its own for them inside the loop would
   // also wait for every tile under way.
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-  bool have_c = next_tile(), have_n = false;   // the current tile exists; the one after it exists (its K is requested)
-  int kpos_c = 0, valid_c = 0, kpos_n = 0, valid_n = 0;
-  int kb = 0, vb = 0;   // K and V buffer of the current tile
-  if (have_c) {
-    kpos_c = kpos;
-    valid_c = tile_valid();
-    fetch_k(0, kpos_c, valid_c);
-    fetch_v(0, kpos_c, valid_c);
-    have_n = next_tile();
-    if (have_n) {
-      kpos_n = kpos;
-      valid_n = tile_valid();
-      fetch_k(1, kpos_n, valid_n);
-    }
-  }
   while (have_c) {
     const int cur_kpos = kpos_c, valid = valid_c, cur_kb = kb, cur_vb = vb;
     // This wavefront's part of the tile has landed; the K loads of the tile after it (requested last; a
@@ -643,11 +679,18 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   }
   const int kb = bx / p.nsub_k, sub = bx - kb * p.nsub_k;
 
-  int b = 0;   // the sequence the k block belongs to
-  while (b + 1 < p.batch && p.cu_num_k_block[b + 1] <= kb) ++b;
-  if (bwd_sequence_skipped<D>(p, b, kb, sub, hk)) return;
-  const int kbl = kb - p.cu_num_k_block[b];          // in-sequence index of the k block
-  const int k0 = p.cu_k[b], klen = p.cu_k[b + 1] - k0;
+  const BwdSequence seq(p, kb, lane);
+  if (seq.qb0 < 0 || seq.qb0 >= p.nqb) return;
+  // asked for together: the sequence's record, the mask column's first 64 words, the resident operands
+  const uint32_t record = bwd_first_record(p, seq, lane);
+  const int kbl = kb - seq.kb0;                      // in-sequence index of the k block
+  const int k0 = seq.k0, klen = seq.k1 - k0;
+  const bool fits = seq.fits(p, kb);
+  auto column_word = [&](int first, int low, int end) -> uint32_t {   // lane i: the word of q block first + i, if low <= first + i < end
+    const int g = first + lane;
+    return g >= low && g < end ? p.bits[((size_t)hk * p.nqb + g) * p.wpr + (kbl >> 5)] : 0u;
+  };
+  const uint32_t first_word = !PARTS && fits ? column_word(seq.qb1 - 64, seq.qb0, seq.qb1) : 0u;
   const int krows = min(p.kbs, klen - kbl * p.kbs);  // keys in the block
   const int wg_keys = min(4 * kWaveRows, p.kbs - sub * 4 * kWaveRows);   // by the block size: the same for every k block
   const bool shared_slots = wg_keys <= 2 * kWaveRows;                    // two wavefronts per 32-key slot
@@ -661,7 +704,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   const int wave_key_max = kbl * p.kbs + min(row0 + kWaveRows - 1, krows - 1);   // position of the wavefront's last key
 
   short8v kf[T::KSTEPS], vf[T::KSTEPS];   // K^T and V^T fragments: lane holds key l32, d = 16*ks + 8*g32 .. +7
-  if (active) {
+  if (active && fits) {
     const char *krow = p.k + (int64_t)(k0 + key_pos) * p.k_s + (int64_t)hk * p.k_h + g32 * 16;
     const char *vrow = p.v + (int64_t)(k0 + key_pos) * p.v_s + (int64_t)hk * p.v_h + g32 * 16;
 #pragma unroll
@@ -682,20 +725,23 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   // the tile sequence: for every q block of the sequence that keeps this k block, for every q head of
   // the group, the block's rows in 64-row tiles (under a causal mask only those with a row that sees a
   // key of this workgroup)
-  int qb = p.cu_num_q_block[b] - 1, r = 0, qoff = 0;
-  int qb_end = p.cu_num_q_block[b + 1];
-  const int qb_begin = p.cu_num_q_block[b];
+  const int qb_begin = seq.qb0;
+  int qb = qb_begin - 1, r = 0, qoff = 0, qb_end = seq.qb1;
   int kept_base = qb_end;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
   int qb_first = qb_begin, r_first = 0, r_last_end = p.ratio, nparts = 1;   // the part's share (BwdKeyPart)
   uint64_t kept = 0;
   QBlockInfo inf = {};
   int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
   if (qb_begin < qb_end) {
-    const QBlockInfo first = p.info[qb_begin];
-    seq_row0 = first.row_begin;
-    seq_qlen = klen - first.shift;
-    inf.shift = first.shift;
+    if (__builtin_amdgcn_readlane((int)record, 9) != 0) {   // flags
+      bwd_zero_keys<D>(p, seq, kb, sub, hk);
+      return;
+    }
+    inf.shift = __builtin_amdgcn_readlane((int)record, 5);
+    seq_row0 = __builtin_amdgcn_readlane((int)record, 0);
+    seq_qlen = klen - inf.shift;
   }
+  if (!fits) return;   // (a sequence without queries that lies outside of the tensors)
   if constexpr (PARTS) {
     const BwdKeyPart share(p, qb_begin, qb_end, inf.shift, wg_first_key, part);
     nparts = share.count;
@@ -706,6 +752,8 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
     qb_end = share.qb_last + 1;
     kept_base = qb_end;
   }
+  kept_base -= 64;
+  kept = __ballot(((PARTS ? column_word(kept_base, qb_first, qb_end) : first_word) >> (kbl & 31)) & 1u);
   auto tile_reaches = [&]() {
     return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
   };
@@ -722,8 +770,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       while (kept == 0) {   // one load per 64 q blocks: lane i looks at q block kept_base + i
         kept_base -= 64;
         if (kept_base + 63 < qb_first) return false;
-        uint32_t word = 0;
-        if (kept_base + lane >= qb_first && kept_base + lane < qb_end) word = p.bits[((size_t)hk * p.nqb + kept_base + lane) * p.wpr + (kbl >> 5)];
+        const uint32_t word = column_word(kept_base, qb_first, qb_end);
         __builtin_amdgcn_s_waitcnt(0x0F70);   // (waited for here so that no other path waits)
         kept = __ballot((word >> (kbl & 31)) & 1u);
       }
@@ -765,8 +812,6 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       bwd_dma4(row_addr + (uint32_t)(buf * 512 + 256), p.delta + (int64_t)hq * p.total_q + row_first, rvoff);
     }
   };
-  // Everything loaded so far has arrived before the first tile is requested (see hbsa_bwd_dkv8_kernel).
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
   int n_ahead = 0;                               // tiles fetched and not computed on yet
   int buf_f = 0, buf = 0;                        // buffer of the next fetch, and of the current tile
   int fq_a = 0, fq_b = 0, va_a = 64, va_b = 64;  // first query position and row count of those tiles (a: the older)
@@ -781,6 +826,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   };
   if (more) issue();
   if (more) issue();
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the resident operands have arrived, and the tiles (see hbsa_bwd_dkv8_kernel)
   const int shift = inf.shift;
   const int h_begin = shared_slots ? rows_half : 0, h_end = shared_slots ? rows_half + 1 : 2;   // 32-row halves of a tile
   while (n_ahead > 0) {
@@ -939,11 +985,19 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   }
   const int kb = bx / p.nsub_k, sub = bx - kb * p.nsub_k;
 
-  int b = 0;   // the sequence the k block belongs to
-  while (b + 1 < p.batch && p.cu_num_k_block[b + 1] <= kb) ++b;
-  if (bwd_sequence_skipped<D>(p, b, kb, sub, hk)) return;
-  const int kbl = kb - p.cu_num_k_block[b];
-  const int k0 = p.cu_k[b], klen = p.cu_k[b + 1] - k0;
+  const BwdSequence seq(p, kb, lane);
+  if (seq.qb0 < 0 || seq.qb0 >= p.nqb) return;
+  // Asked for together: the sequence's record, the mask column's first 64 words, the resident operand.  With one workgroup
+  // per CU nothing covers the loads a workgroup begins with, and it has some eight tiles where 8K sequences keep a tenth.
+  const uint32_t record = bwd_first_record(p, seq, lane);
+  const int kbl = kb - seq.kb0;
+  const int k0 = seq.k0, klen = seq.k1 - k0;
+  const bool fits = seq.fits(p, kb);
+  auto column_word = [&](int first, int low, int end) -> uint32_t {   // lane i: the word of q block first + i, if low <= first + i < end
+    const int g = first + lane;
+    return g >= low && g < end ? p.bits[((size_t)hk * p.nqb + g) * p.wpr + (kbl >> 5)] : 0u;
+  };
+  const uint32_t first_word = !PARTS && fits ? column_word(seq.qb1 - 64, seq.qb0, seq.qb1) : 0u;
   const int krows = min(p.kbs, klen - kbl * p.kbs);
   const int wg_row0 = sub * 4 * kWaveRows;                 // first key of the workgroup inside the block
   const int row0 = wg_row0 + key_slot * kWaveRows;
@@ -956,7 +1010,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   // this wavefront's resident operand: K^T (P wavefront) or V^T (dS wavefront) of its 32 keys; lane holds
   // key l32, d = 16 * ks + 8 * g32 .. + 7
   short8v frag[T::KSTEPS];
-  if (active) {
+  if (active && fits) {
     const char *src = role == 0 ? p.k + (int64_t)(k0 + key_pos) * p.k_s + (int64_t)hk * p.k_h
                                 : p.v + (int64_t)(k0 + key_pos) * p.v_s + (int64_t)hk * p.v_h;
 #pragma unroll
@@ -971,20 +1025,23 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
 
-  int qb = p.cu_num_q_block[b] - 1, r = 0, qoff = 0;
-  int qb_end = p.cu_num_q_block[b + 1];
-  const int qb_begin = p.cu_num_q_block[b];
+  const int qb_begin = seq.qb0;
+  int qb = qb_begin - 1, r = 0, qoff = 0, qb_end = seq.qb1;
   int kept_base = qb_end;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
   int qb_low = qb_begin, r_end = p.ratio;   // the part's first q block, and the q block's heads that are the part's
   uint64_t kept = 0;
   QBlockInfo inf = {};
   int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
   if (qb_begin < qb_end) {
-    const QBlockInfo first = p.info[qb_begin];
-    seq_row0 = first.row_begin;
-    seq_qlen = klen - first.shift;
-    inf.shift = first.shift;
+    if (__builtin_amdgcn_readlane((int)record, 9) != 0) {   // flags
+      bwd_zero_keys<D>(p, seq, kb, sub, hk);
+      return;
+    }
+    inf.shift = __builtin_amdgcn_readlane((int)record, 5);
+    seq_row0 = __builtin_amdgcn_readlane((int)record, 0);
+    seq_qlen = klen - inf.shift;
   }
+  if (!fits) return;   // (a sequence without queries that lies outside of the tensors)
   if constexpr (PARTS) {
     const BwdKeyPart share(p, qb_begin, qb_end, inf.shift, wg_first_key, part);
     if (part >= share.count) return;
@@ -998,6 +1055,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     qb_end = share.qb_last + 1;
     kept_base = qb_end;
   }
+  kept_base -= 64;
+  kept = __ballot(((PARTS ? column_word(kept_base, qb_low, qb_end) : first_word) >> (kbl & 31)) & 1u);
   auto tile_reaches = [&]() {
     return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
   };
@@ -1014,8 +1073,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       while (kept == 0) {   // one load per 64 q blocks: lane i looks at q block kept_base + i; waited for here so that no other path waits
         kept_base -= 64;
         if (kept_base + 63 < qb_low) return false;
-        uint32_t word = 0;
-        if (kept_base + lane >= qb_low && kept_base + lane < qb_end) word = p.bits[((size_t)hk * p.nqb + kept_base + lane) * p.wpr + (kbl >> 5)];
+        const uint32_t word = column_word(kept_base, qb_low, qb_end);
         __builtin_amdgcn_s_waitcnt(0x0F70);
         kept = __ballot((word >> (kbl & 31)) & 1u);
       }
@@ -1086,10 +1144,6 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   int n_ahead = 0;                               // tiles fetched and not computed on yet
   int qi_f = 0, gi_f = 0;                        // buffers of the next fetch
   int fq_a = 0, fq_b = 0, va_a = 64, va_b = 64;  // first query position and row count of those tiles (a: the older)
-  // Everything loaded so far (the resident operand above all) has arrived before the first tile is requested: the
-  // compiler counts only the loads it knows, and a wait of its own for them inside the loop would also wait for
-  // every tile under way.
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
   bool more = next_tile();
   auto issue = [&]() {   // fetches the tile next_tile() stands on and moves on
     const int fq = inf.q_pos + qoff, va = min(64, inf.rows - qoff);
@@ -1102,6 +1156,9 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   };
   if (more) issue();
   if (more) issue();
+  // The resident operand has arrived before the loop begins (and with it the first two tiles, requested behind it): the
+  // compiler counts only the loads it knows, and a wait of its own for it inside the loop would also wait for every tile under way.
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
   bool prev = false;        // the tile before the current one exists: its dK part is still due
   int qi = 0, gi = 0, par = 0;   // Q buffer, dO buffer and parity of the current tile
   f32x16 dp_prev[NH];       // dS wavefront: dP of the previous tile
