@@ -74,6 +74,9 @@ struct PrepParams {
   unsigned long long *clock;
   int32_t nqb, qbs, kbs, wpr, causal;
   int32_t batch, nkb, total_q, total_k;   // bounds the sequences' boundaries are checked against
+  uint32_t *order;         // order of the items (see OrderRoom), nullptr: not wanted
+  struct OrderRoom *room;  // the stream's room for making it, nullptr: the order without weights is written
+  int32_t nhead_k, weight_shift;
 };
 
 // Division by a launch constant d, exact for 0 <= n < 2^31: n / d == (n * m) >> s with
@@ -148,6 +151,8 @@ struct FwdParams {
   int32_t parts_last;    // workgroups are numbered by part first (else: the parts of an item are neighbours)
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
   int32_t split;         // host side only: parts of the split over key blocks that pay (fwd_split)
+  // Items handed out without queues in the order of their weights (see OrderRoom), nullptr: last q blocks first
+  const uint32_t *order;         // [num_q_block * nhead_k]: q block << 16 | kv head, heaviest first
 };
 
 // Boundaries of one sequence of the packed batch, as read from the caller's device arrays.
@@ -405,6 +410,89 @@ __device__ __forceinline__ void part_store4(float *at, f32x4 v) {
 }
 __device__ __forceinline__ void parts_arrived() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 __device__ __forceinline__ void parts_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
+
+// ---- Items in the order of their weights.  A launch whose workgroups take two to eight items each in a fixed order ends when
+// the unluckiest workgroup does: a Bernoulli mask, ragged sequences and a causal mask make items differ by factors.  So the
+// (q block, kv head) pairs are counted (their kept keys) and sorted, heaviest first; the fixed order (forwards, then backwards
+// through the list) then gives every workgroup about the same.  One wavefront counts each pair, the workgroup that arrives last
+// sorts by counting; the order among equals is left to chance, and no result depends on it.
+// Measured, forward kernels: 6 x 300 .. 4000 tokens, 16 / 4 heads of 64, 1.8 items a place, 67 -> 48 us, the pre-pass 4.7 -> 7.7.
+// In the one-launch form, which has no pre-pass, a launch for the order alone (8 to 11 us) takes back what it gives: 8 x 2050
+// tokens, 16 heads of 192, not causal, 221 -> 199 + 11; C5's shape 276 -> 262 + 8.
+constexpr int kMaxOrderItems = 4096;   // pairs (of 8192, 4 x 8192 tokens with 32 heads, no launch takes the order, and sorting them costs 10 us)
+constexpr int kOrderBins = 2 * kThreads;   // weights told apart
+constexpr int kOrderCopies = 4;            // counters of one weight, by lane: equal weights otherwise queue at one word of LDS
+struct OrderRoom {   // a stream's
+  uint32_t order[kMaxOrderItems], weight[kMaxOrderItems];
+  uint32_t arrived, pad[63];   // zero before and after every launch
+};
+struct OrderLds {
+  uint32_t count[kOrderCopies][kOrderBins];
+  uint16_t bin[kMaxOrderItems];
+  uint32_t sums[kThreads / 64], last;
+};
+__device__ __forceinline__ void order_note(OrderRoom *room, int pair, int keys, int shift) {
+  __hip_atomic_store(&room->weight[pair], (uint32_t)min(kOrderBins - 1, (keys + (1 << shift) - 1) >> shift), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+// Behind the notes: every workgroup of kThreads threads arrives, the last of `workgroups` sorts.
+__device__ __forceinline__ void order_arrive(OrderRoom *room, uint32_t *order, int pairs, int nhead_k, uint32_t workgroups, OrderLds &lds) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const bool last = __hip_atomic_fetch_add(&room->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == workgroups;
+    if (last) __hip_atomic_store(&room->arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    lds.last = last;
+  }
+  for (int i = threadIdx.x; i < kOrderCopies * kOrderBins; i += kThreads) (&lds.count[0][0])[i] = 0;
+  __syncthreads();
+  if (!lds.last) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  const int copy = lane & (kOrderCopies - 1);   // (pair i is always thread i % kThreads's)
+  for (int base = threadIdx.x; base < pairs; base += 8 * kThreads) {   // (eight loads under way: each comes from beyond the L2)
+    uint32_t w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = room->weight[min(base + j * kThreads, pairs - 1)];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int i = base + j * kThreads, bin = kOrderBins - 1 - (int)w[j];
+      if (i < pairs) {
+        lds.bin[i] = (uint16_t)bin;
+        atomicAdd(&lds.count[copy][bin], 1u);
+      }
+    }
+  }
+  __syncthreads();
+  // places of the first of every (weight, copy): two weights a thread
+  uint32_t n[2][kOrderCopies], sum = 0;
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int c = 0; c < kOrderCopies; ++c) sum += n[x][c] = lds.count[c][2 * threadIdx.x + x];
+  uint32_t incl = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(incl, off);
+    if (lane >= off) incl += y;
+  }
+  if (lane == 63) lds.sums[wave] = incl;
+  __syncthreads();
+  uint32_t before = incl - sum;
+  for (int w = 0; w < wave; ++w) before += lds.sums[w];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int c = 0; c < kOrderCopies; ++c) {
+      lds.count[c][2 * threadIdx.x + x] = before;
+      before += n[x][c];
+    }
+  __syncthreads();
+  for (int i = threadIdx.x; i < pairs; i += kThreads) {
+    const int qb = i / nhead_k;
+    order[atomicAdd(&lds.count[copy][lds.bin[i]], 1u)] = (uint32_t)qb << 16 | (uint32_t)(i - qb * nhead_k);
+  }
+}
 
 // Keeps the message hbsa_last_error() returns and gives back `code` (defined in hbsa_fwd.hip).
 int fail(int code, const char *fmt, ...);

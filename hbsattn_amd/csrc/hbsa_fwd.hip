@@ -31,13 +31,16 @@ namespace hbsa {
 // --------------------------------------------------------------------------------------
 // Pre-pass: one wavefront per (kv head, q block).
 // --------------------------------------------------------------------------------------
+// ORDER: the order of the items (see OrderRoom) is made, too.
+template <bool ORDER>
 __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
   const int lane = threadIdx.x & 63;
   const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int hk = blockIdx.y;
+  int kept_keys = 0;
   // the work-queue counters of the launch record start at zero; every attention launch leaves them so
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 9) ((uint32_t *)p.sched)[threadIdx.x] = 0;
-  if (g >= p.nqb) return;
-  const int hk = blockIdx.y;
+  if (g < p.nqb) {
   int b;
   if (p.q_block_to_batch != nullptr) {
     b = p.q_block_to_batch[g];
@@ -72,6 +75,16 @@ __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
     const bool keep = j < nvis && m[j * p.ms_k] != 0;
     const uint64_t bal = __ballot(keep);
     if (lane < 2) row[2 * w + lane] = lane ? (uint32_t)(bal >> 32) : (uint32_t)bal;
+    kept_keys += __builtin_popcountll(bal) * p.kbs;
+  }
+  if (ORDER && lane == 0) {
+    if (p.room == nullptr) p.order[(size_t)(p.nqb - 1 - g) * p.nhead_k + hk] = (uint32_t)g << 16 | (uint32_t)hk;   // last q blocks first
+    else order_note(p.room, g * p.nhead_k + hk, kept_keys, p.weight_shift);
+  }
+  }
+  if constexpr (ORDER) {
+    __shared__ OrderLds lds;
+    if (p.room != nullptr) order_arrive(p.room, p.order, p.nqb * p.nhead_k, p.nhead_k, gridDim.x * gridDim.y, lds);
   }
 }
 
@@ -297,13 +310,27 @@ int fail(int code, const char *fmt, ...) {
   return code;
 }
 
+// Weights are counted in 2^shift keys, so that even all keys of the batch in one row stay below the number of bins where they can
+inline int weight_shift(long long keys) {
+  int s = 4;
+  while (s < 16 && (keys >> s) >= kOrderBins) ++s;
+  return s;
+}
+
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 inline int words_per_row(int num_k_block) { return 2 * ((num_k_block + 63) / 64); }
-// workspace layout: QBlockInfo[num_q_block] | Sched | walk clocks [nhead_k, num_q_block] | bit words
+// workspace layout: QBlockInfo[num_q_block] | Sched | walk clocks [nhead_k, num_q_block] | bit words | order of the items
 inline size_t sched_offset(int num_q_block) { return align_up((size_t)num_q_block * sizeof(QBlockInfo), 256); }
 inline size_t clock_offset(int num_q_block) { return sched_offset(num_q_block) + align_up(sizeof(Sched), 256); }
 inline size_t bits_offset(int nhead_k, int num_q_block) {
   return clock_offset(num_q_block) + align_up((size_t)nhead_k * num_q_block * sizeof(unsigned long long), 256);
+}
+inline size_t order_offset(int nhead_k, int num_q_block, int num_k_block) {
+  return bits_offset(nhead_k, num_q_block) + align_up((size_t)nhead_k * num_q_block * words_per_row(num_k_block) * sizeof(uint32_t), 256);
+}
+inline size_t order_bytes(int nhead_k, int num_q_block) {   // 0: too many items for an order
+  const long long pairs = (long long)nhead_k * num_q_block;
+  return pairs > kMaxOrderItems ? 0 : align_up((size_t)pairs * sizeof(uint32_t), 256);
 }
 
 // Deterministic mode (the default, like the reference's ascending scan): every item walks its tiles in
@@ -633,6 +660,8 @@ constexpr int kStreamSlots = 64;
 static __device__ __align__(256) unsigned char stream_sched[kStreamSlots * sizeof(hbsa::Sched)];
 // stream_arrivals: the counters of launches whose items are cut into parts (ItemParts), likewise one set per stream.
 static __device__ __align__(256) uint32_t stream_arrivals[kStreamSlots * hbsa::kMaxPartItems];
+// stream_order: room for making the order of a launch's items (see OrderRoom), likewise one per stream.
+static __device__ __align__(256) hbsa::OrderRoom stream_order[kStreamSlots];
 namespace hbsa {
 std::mutex g_scratch_mutex;
 void *g_scratch_ptr[kMaxDevices] = {};
@@ -658,24 +687,27 @@ int static_scratch(void **ptr) {
 struct StreamSlots {
   char *base;
   uint32_t *arrivals;
+  OrderRoom *order;
   int used;
   hipStream_t stream[kStreamSlots];
 };
 StreamSlots g_stream_slots[kMaxDevices] = {};
-Sched *stream_sched_of(hipStream_t stream, uint32_t **arrivals = nullptr) {
+Sched *stream_sched_of(hipStream_t stream, uint32_t **arrivals = nullptr, OrderRoom **order = nullptr) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
   StreamSlots &t = g_stream_slots[dev];
   if (t.base == nullptr) {
-    void *p = nullptr, *a = nullptr;
+    void *p = nullptr, *a = nullptr, *o = nullptr;
     if (hipGetSymbolAddress(&p, HIP_SYMBOL(stream_sched)) != hipSuccess || p == nullptr ||
-        hipGetSymbolAddress(&a, HIP_SYMBOL(stream_arrivals)) != hipSuccess || a == nullptr) {
+        hipGetSymbolAddress(&a, HIP_SYMBOL(stream_arrivals)) != hipSuccess || a == nullptr ||
+        hipGetSymbolAddress(&o, HIP_SYMBOL(stream_order)) != hipSuccess || o == nullptr) {
       (void)hipGetLastError();
       return nullptr;
     }
     t.base = (char *)p;
     t.arrivals = (uint32_t *)a;
+    t.order = (OrderRoom *)o;
   }
   int i = 0;
   while (i < t.used && t.stream[i] != stream) ++i;
@@ -683,6 +715,8 @@ Sched *stream_sched_of(hipStream_t stream, uint32_t **arrivals = nullptr) {
     if (t.used == kStreamSlots) return nullptr;
     t.stream[t.used++] = stream;
   }
+  // (hipStreamPerThread is one handle for every thread's own stream: two of them would share the room)
+  if (order != nullptr) *order = stream == hipStreamPerThread ? nullptr : t.order + i;
   if (arrivals != nullptr) *arrivals = t.arrivals + (size_t)i * kMaxPartItems;
   return (Sched *)(t.base + (size_t)i * sizeof(Sched));
 }
@@ -924,8 +958,7 @@ int hbsa_block_arrays(const int32_t *cu_seqlen, const int32_t *first, int32_t ba
 
 size_t hbsa_fwd_workspace_bytes(int32_t nhead_k, int32_t num_q_block, int32_t num_k_block) {
   if (nhead_k <= 0 || num_q_block <= 0 || num_k_block <= 0) return 256;
-  const size_t bits = align_up((size_t)nhead_k * num_q_block * words_per_row(num_k_block) * sizeof(uint32_t), 256);
-  return bits_offset(nhead_k, num_q_block) + bits;
+  return order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block);
 }
 
 size_t hbsa_fwd_workspace_bytes_dtype(int32_t dtype, int32_t total_q, int32_t total_k, int32_t nhead_q,
@@ -963,11 +996,14 @@ size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t 
   return b16 > f32 ? b16 : f32;
 }
 
-int hbsa_fwd_prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
+}  // extern "C"
+namespace {
+// ordered: the order of the items is made, too (see OrderRoom); only a run that is split over key blocks can do without
+int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
                      const int32_t *q_block_to_batch, const int32_t *cu_num_q_block, const int32_t *cu_num_k_block,
                      void *workspace, size_t workspace_bytes, int32_t batch, int32_t nhead_k, int32_t num_q_block,
                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size, int32_t causal,
-                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream) {
+                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream, bool ordered) {
   g_err[0] = 0;
   if (batch < 0 || num_q_block < 0 || num_k_block < 0 || total_q < 0 || total_k < 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
@@ -997,10 +1033,34 @@ int hbsa_fwd_prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, c
   pp.nqb = num_q_block; pp.qbs = q_block_size; pp.kbs = k_block_size; pp.wpr = words_per_row(num_k_block);
   pp.causal = causal ? 1 : 0;
   pp.batch = batch; pp.nkb = num_k_block; pp.total_q = total_q; pp.total_k = total_k;
-  hipLaunchKernelGGL(hbsa_prep_kernel, dim3((num_q_block + 3) / 4, nhead_k), dim3(kThreads), 0, (hipStream_t)stream, pp);
+  pp.nhead_k = nhead_k;
+  pp.weight_shift = weight_shift((long long)num_k_block * k_block_size);
+  pp.order = nullptr;
+  pp.room = nullptr;
+  const dim3 grid((num_q_block + 3) / 4, nhead_k);
+  if (ordered && order_bytes(nhead_k, num_q_block) != 0) {
+    pp.order = (uint32_t *)((char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
+    // (a captured launch may be replayed on any stream, while the room belongs to this one)
+    if (!is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
+    hipLaunchKernelGGL((hbsa_prep_kernel<true>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
+  } else {
+    hipLaunchKernelGGL((hbsa_prep_kernel<false>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, "hbsa_prep_kernel launch: %s", hipGetErrorString(e));
   return 0;
+}
+}  // namespace
+extern "C" {
+
+int hbsa_fwd_prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
+                     const int32_t *q_block_to_batch, const int32_t *cu_num_q_block, const int32_t *cu_num_k_block,
+                     void *workspace, size_t workspace_bytes, int32_t batch, int32_t nhead_k, int32_t num_q_block,
+                     int32_t num_k_block, int32_t q_block_size, int32_t k_block_size, int32_t causal,
+                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream) {
+  return prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block, workspace,
+                 workspace_bytes, batch, nhead_k, num_q_block, num_k_block, q_block_size, k_block_size,
+                 causal, total_q, total_k, mask_strides, stream, true);
 }
 
 int hbsa_fwd_run(const void *q, const void *k, const void *v, void *out, void *workspace, size_t workspace_bytes,
@@ -1095,6 +1155,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
   }
   fp.div_nparts = make_fast_div((uint32_t)fp.nparts);
   // the clocked walk: block sizes that are whole tiles, work that is not split, K/V of a head beyond what an L2 holds
+  if (order_bytes(nhead_k, num_q_block) != 0) fp.order = (const uint32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
   fp.walk = (!g_deterministic && fp.nparts == 1 && k_block_size % kTileKeys == 0 &&
              2ll * total_k * headdim * 2 >= g_walk_min_bytes) ? 1 : 0;
 
@@ -1202,9 +1263,13 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
     if (f32_exact) return run_f32(fp, softmax_scale, headdim, num_k_block, items, area, room, (hipStream_t)stream);
     return run_decode(fp, plan.parts, dtype == HBSA_DTYPE_BF16, headdim, num_k_block, q_block_size, area, room, (hipStream_t)stream);
   }
-  int rc = hbsa_fwd_prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block,
-                            workspace, workspace_bytes, batch, nhead_k, num_q_block, num_k_block, q_block_size,
-                            k_block_size, causal, total_q, total_k, strides + 8, stream);
+  FwdParams shape;
+  std::memset(&shape, 0, sizeof(shape));
+  fill_shape(shape, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
+  const bool split = shape.split > 1 && workspace_bytes >= need + split_bytes(shape.split, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
+  int rc = prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block, workspace, workspace_bytes,
+                   batch, nhead_k, num_q_block, num_k_block, q_block_size, k_block_size, causal, total_q, total_k, strides + 8, stream,
+                   !split);
   if (rc != 0) return rc;
   return hbsa_fwd_run(q, k, v, out, workspace, workspace_bytes, dtype, total_q, total_k, nhead_q, nhead_k, headdim,
                       num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, strides, stream);

@@ -263,13 +263,18 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   // lightest item of a round goes to the workgroup that got the heaviest of the round before, and the
   // workgroups (those of one CU, too) end at about the same time.  Nothing is claimed: measured against a shared
   // counter for the later rounds, 8 x 1024 tokens 106 -> 99 us and C5 0.258 -> 0.241 ms.
-  int own_claims = 0;
+  int own_claims = 0, pending_sub = 0;
   auto claim = [&]() -> uint32_t {   // the value is looked at an item later, so its latency is hidden
     const FwdParams &p = fresh_args();
     uint32_t r = 0xffffffffu;
     if (p.one_each) {
       r = (own_claims & 1) ? (uint32_t)(own_claims + 1) * gridDim.x - 1u - blockIdx.x : (uint32_t)own_claims * gridDim.x + blockIdx.x;
       ++own_claims;
+      if (p.order != nullptr) {   // the place in the order -> the item; a load that is waited for when the value is looked at
+        const uint32_t whole = fast_div(r, p.div_nsub);
+        pending_sub = (int)(r - whole * (uint32_t)p.nsub);
+        r = r < (uint32_t)p.one_each ? p.order[whole] : 0xffffffffu;
+      }
     } else if (tries < 8) {
       if (lane == 0) r = atomicAdd(&p.sched->qnext[(first_queue + tries) & 7], 1u);
     }
@@ -390,7 +395,16 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     uint32_t claimed = (uint32_t)__builtin_amdgcn_readfirstlane((int)pending);
     st_hk = -1;
     if (p.one_each) {
-      if (claimed < (uint32_t)p.one_each) decode_free_entry(claimed);
+      if (p.order != nullptr) {
+        if (claimed != 0xffffffffu) {
+          st_hk = (int)(claimed & 0xffffu);
+          st_qb = (int)(claimed >> 16);
+          st_sub = pending_sub;
+          st_part = 0;
+        }
+      } else if (claimed < (uint32_t)p.one_each) {
+        decode_free_entry(claimed);
+      }
     } else {
       while (tries < 8) {
         const int v = (first_queue + tries) & 7;
@@ -1292,6 +1306,7 @@ int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   // Few items per workgroup: a fixed order instead of the per-XCD queues, whose round trips (and, with few kv
   // heads, the crowd at few counters) would be a good part of such a launch.
   launch.one_each = items <= (long long)kStaticShare * resident ? (int)items : 0;
+  if (launch.one_each == 0 || launch.nparts != 1 || items <= resident) launch.order = nullptr;
   hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, "hbsa_fwd_kernel launch: %s", hipGetErrorString(e));
