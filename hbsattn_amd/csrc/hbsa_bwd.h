@@ -658,7 +658,11 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
 // all keys and none for keys past the block's end (their columns are not stored).  Operand reads issued by hand as in the
 // dQ kernel were measured and are no faster.  dQ + dK/dV, 6 x 300 .. 4000 tokens, 16 / 4 heads, 64-key blocks, keep 0.4:
 // 250 -> 227 us with the loads two tiles ahead, 195 with the heads going round the grid (bwd_decode_grid).
-template <int D, typename E, bool PARTS>
+// MANY: the form with 165 registers a wavefront, three workgroups to a CU (head dim 32: 127, four), for many rounds of items.
+// Two workgroups of 209 registers are better where there are few rounds and the longest item sets the time: dQ + dK/dV, 64-key blocks, at 1.4 rounds of two (6 x 300 ..
+// 4000 tokens, 16 / 4 heads) 205 and 215 us, at 2.0 (128-key blocks, 8 x 500 .. 3000, 32 / 8) 310 and 337, at 2.3 (2 x 600 .. 1500,
+// 32) 73 and 71, at 3.0 (6 x 4000, 16 / 4) 419 and 401, at 8 (4 x 8192, 16) 400 and 371.
+template <int D, typename E, bool PARTS, bool MANY>
 __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) {
   static_assert(D <= 64, "head dim 128 has its own kernel");
   using T = BwdTile<D>;
@@ -667,7 +671,9 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   float *rowv = (float *)(lds + 6 * T::TILE_BYTES);    // buffer s: [64] log2-domain log-sum-exp of the tile's rows, [64] their delta
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // ("& 3": the compiler then sees the two values rows_half can take, and does less of the loop over the halves at once.
+  // A launch bound of three workgroups in its place makes 46 registers spill.)
+  const int wave = __builtin_amdgcn_readfirstlane(MANY ? (threadIdx.x >> 6) & 3 : threadIdx.x >> 6);
   const int g32 = lane >> 5, l32 = lane & 31;
   int hk, bx;
   bwd_decode_grid(p, (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u), hk, bx);
@@ -677,7 +683,8 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
     part = bx / per_part;
     bx -= part * per_part;
   }
-  const int kb = bx / p.nsub_k, sub = bx - kb * p.nsub_k;
+  const int kb_at = bx / p.nsub_k, sub = bx - kb_at * p.nsub_k;
+  const int kb = p.order_k != nullptr ? p.order_k[kb_at] : kb_at;
 
   const BwdSequence seq(p, kb, lane);
   if (seq.qb0 < 0 || seq.qb0 >= p.nqb) return;
@@ -983,7 +990,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     part = bx / per_part;
     bx -= part * per_part;
   }
-  const int kb = bx / p.nsub_k, sub = bx - kb * p.nsub_k;
+  const int kb_at = bx / p.nsub_k, sub = bx - kb_at * p.nsub_k;
+  const int kb = p.order_k != nullptr ? p.order_k[kb_at] : kb_at;
 
   const BwdSequence seq(p, kb, lane);
   if (seq.qb0 < 0 || seq.qb0 >= p.nqb) return;
@@ -1347,7 +1355,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   else run(std::integral_constant<int, 1>{});
 }
 
-template <int D, typename E, bool PARTS_Q, bool PARTS_K, bool SHARED>
+// MANY: of the dK/dV kernel for head dims up to 64; SHARED: of the one for 128
+template <int D, typename E, bool PARTS_Q, bool PARTS_K, bool SHARED, bool MANY>
 int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   using T = BwdTile<D>;
   // LDS: the dQ kernel's three K and two V tiles; the dK/dV kernels' tile buffers, P records and row values
@@ -1360,7 +1369,7 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
     if (!raised[dev]) {
       const void *dkv = nullptr;
       if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>);
-      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K>);
+      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K, MANY>);
       hipError_t e = hipFuncSetAttribute(dkv, hipFuncAttributeMaxDynamicSharedMemorySize, lds_dkv);
       if (e == hipSuccess)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&hbsa_bwd_dq_kernel<D, E, PARTS_Q>),
@@ -1375,24 +1384,29 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
   const dim3 kv_grid = bp.flat_grid ? dim3(k_wgs * (unsigned)nhead_k) : dim3(k_wgs, (unsigned)nhead_k);
   hipLaunchKernelGGL((hbsa_bwd_dq_kernel<D, E, PARTS_Q>), q_grid, dim3(kThreads), lds_dq, stream, bp);
   if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>), kv_grid, dim3(512), lds_dkv, stream, bp);
-  else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
+  else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K, MANY>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
 
-template <int D, typename E, bool SHARED>
+template <int D, typename E, bool SHARED, bool MANY>
 int launch_bwd_parts(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   const bool pq = bp.parts_q > 1, pk = bp.parts_k > 1;
-  if (pq && pk) return launch_bwd_kernels<D, E, true, true, SHARED>(bp, nhead_k, num_k_block, stream);
-  if (pq) return launch_bwd_kernels<D, E, true, false, SHARED>(bp, nhead_k, num_k_block, stream);
-  if (pk) return launch_bwd_kernels<D, E, false, true, SHARED>(bp, nhead_k, num_k_block, stream);
-  return launch_bwd_kernels<D, E, false, false, SHARED>(bp, nhead_k, num_k_block, stream);
+  if (pq && pk) return launch_bwd_kernels<D, E, true, true, SHARED, false>(bp, nhead_k, num_k_block, stream);
+  if (pk) return launch_bwd_kernels<D, E, false, true, SHARED, false>(bp, nhead_k, num_k_block, stream);
+  if (pq) return launch_bwd_kernels<D, E, true, false, SHARED, MANY>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_kernels<D, E, false, false, SHARED, MANY>(bp, nhead_k, num_k_block, stream);
 }
 template <int D, typename E>
 int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
-  // (the kernel for smaller head dims decides for itself whether wavefronts share a slot)
-  if (D == 128 && bp.kbs <= 2 * kWaveRows) return launch_bwd_parts<D, E, D == 128>(bp, nhead_k, num_k_block, stream);
-  return launch_bwd_parts<D, E, false>(bp, nhead_k, num_k_block, stream);
+  if constexpr (D == 128) {
+    if (bp.kbs <= 2 * kWaveRows) return launch_bwd_parts<D, E, true, false>(bp, nhead_k, num_k_block, stream);
+    return launch_bwd_parts<D, E, false, false>(bp, nhead_k, num_k_block, stream);
+  } else {
+    // (the kernel for smaller head dims decides for itself whether wavefronts share a slot)
+    if (D == 32 || bp.many) return launch_bwd_parts<D, E, false, true>(bp, nhead_k, num_k_block, stream);
+    return launch_bwd_parts<D, E, false, false>(bp, nhead_k, num_k_block, stream);
+  }
 }
 
 }  // namespace hbsa

@@ -77,6 +77,7 @@ struct PrepParams {
   uint32_t *order;         // order of the items (see OrderRoom), nullptr: not wanted
   struct OrderRoom *room;  // the stream's room for making it, nullptr: the order without weights is written
   int32_t nhead_k, weight_shift;
+  int32_t *order_k;        // [nkb]: the k blocks by falling number of query rows that can see them
 };
 
 // Division by a launch constant d, exact for 0 <= n < 2^31: n / d == (n * m) >> s with
@@ -329,6 +330,8 @@ struct BwdParams {
   int32_t flat_grid;     // one-dimensional grids (bwd_decode_grid)
   float *parts;          // partial accumulators, shared by the two launches
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
+  const int32_t *order_k;   // k blocks by falling number of query rows that can see them, nullptr: in their own order
+  int32_t many;          // host side only: more than two rounds of dK/dV items (head dim 64)
 };
 
 // ---- Items of the kernels without a scheduler: geometry and kept blocks straight from the caller's arrays (bits == nullptr)

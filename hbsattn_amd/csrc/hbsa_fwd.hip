@@ -31,6 +31,33 @@ namespace hbsa {
 // --------------------------------------------------------------------------------------
 // Pre-pass: one wavefront per (kv head, q block).
 // --------------------------------------------------------------------------------------
+// The place of k block kb among all k blocks of the batch, by falling number of query rows that can see a key of it (equals in
+// their own order).  That number falls along a sequence, so how many blocks of another sequence come first is a division.
+// Boundaries that do not fit each other, or a long batch: its own number.
+__device__ __forceinline__ int k_block_place(const PrepParams &p, int kb) {
+  if (p.batch > 256 || p.cu_num_k_block[0] != 0 || p.cu_num_k_block[p.batch] != p.nkb) return kb;
+  auto qlen_of = [&](int s) { return p.cu_q[s + 1] - p.cu_q[s]; };
+  auto klen_of = [&](int s) { return p.cu_k[s + 1] - p.cu_k[s]; };
+  int b = 0;
+  bool good = true;
+  for (int s = 0; s < p.batch; ++s) {
+    const int qlen = qlen_of(s), klen = klen_of(s), first = p.cu_num_k_block[s];
+    good = good && qlen >= 0 && klen >= 0 && p.cu_num_k_block[s + 1] - first == (int)(((int64_t)klen + p.kbs - 1) / p.kbs);
+    if (first <= kb) b = s;
+  }
+  if (!good) return kb;
+  const int j = kb - p.cu_num_k_block[b];
+  const int rows = qlen_of(b), weight = p.causal ? min(rows, klen_of(b) - j * p.kbs) : rows;
+  auto at_least = [&](int s, int w) {   // blocks of sequence s that w rows or more can see
+    const int klen = klen_of(s), n = p.cu_num_k_block[s + 1] - p.cu_num_k_block[s];
+    if (w <= 0) return n;
+    if (w > qlen_of(s)) return 0;
+    return !p.causal ? n : klen < w ? 0 : min(n, (klen - w) / p.kbs + 1);
+  };
+  int place = 0;
+  for (int s = 0; s < p.batch; ++s) place += s == b ? j : at_least(s, s < b ? weight : weight + 1);
+  return place;
+}
 // ORDER: the order of the items (see OrderRoom) is made, too.
 template <bool ORDER>
 __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
@@ -81,6 +108,9 @@ __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
     if (p.room == nullptr) p.order[(size_t)(p.nqb - 1 - g) * p.nhead_k + hk] = (uint32_t)g << 16 | (uint32_t)hk;   // last q blocks first
     else order_note(p.room, g * p.nhead_k + hk, kept_keys, p.weight_shift);
   }
+  }
+  if (ORDER && hk == 0 && p.order_k != nullptr) {
+    for (int kb = blockIdx.x * kThreads + threadIdx.x; kb < p.nkb; kb += gridDim.x * kThreads) p.order_k[k_block_place(p, kb)] = kb;
   }
   if constexpr (ORDER) {
     __shared__ OrderLds lds;
@@ -319,7 +349,7 @@ inline int weight_shift(long long keys) {
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 inline int words_per_row(int num_k_block) { return 2 * ((num_k_block + 63) / 64); }
-// workspace layout: QBlockInfo[num_q_block] | Sched | walk clocks [nhead_k, num_q_block] | bit words | order of the items
+// workspace layout: QBlockInfo[num_q_block] | Sched | walk clocks [nhead_k, num_q_block] | bit words | order of the items | order of the k blocks
 inline size_t sched_offset(int num_q_block) { return align_up((size_t)num_q_block * sizeof(QBlockInfo), 256); }
 inline size_t clock_offset(int num_q_block) { return sched_offset(num_q_block) + align_up(sizeof(Sched), 256); }
 inline size_t bits_offset(int nhead_k, int num_q_block) {
@@ -328,9 +358,12 @@ inline size_t bits_offset(int nhead_k, int num_q_block) {
 inline size_t order_offset(int nhead_k, int num_q_block, int num_k_block) {
   return bits_offset(nhead_k, num_q_block) + align_up((size_t)nhead_k * num_q_block * words_per_row(num_k_block) * sizeof(uint32_t), 256);
 }
-inline size_t order_bytes(int nhead_k, int num_q_block) {   // 0: too many items for an order
+inline size_t order_bytes(int nhead_k, int num_q_block) {   // of the items; 0: too many of them, and no orders at all
   const long long pairs = (long long)nhead_k * num_q_block;
   return pairs > kMaxOrderItems ? 0 : align_up((size_t)pairs * sizeof(uint32_t), 256);
+}
+inline size_t order_k_bytes(int nhead_k, int num_q_block, int num_k_block) {
+  return order_bytes(nhead_k, num_q_block) == 0 ? 0 : align_up((size_t)num_k_block * sizeof(int32_t), 256);
 }
 
 // Deterministic mode (the default, like the reference's ascending scan): every item walks its tiles in
@@ -958,7 +991,7 @@ int hbsa_block_arrays(const int32_t *cu_seqlen, const int32_t *first, int32_t ba
 
 size_t hbsa_fwd_workspace_bytes(int32_t nhead_k, int32_t num_q_block, int32_t num_k_block) {
   if (nhead_k <= 0 || num_q_block <= 0 || num_k_block <= 0) return 256;
-  return order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block);
+  return order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block) + order_k_bytes(nhead_k, num_q_block, num_k_block);
 }
 
 size_t hbsa_fwd_workspace_bytes_dtype(int32_t dtype, int32_t total_q, int32_t total_k, int32_t nhead_q,
@@ -1036,10 +1069,12 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
   pp.nhead_k = nhead_k;
   pp.weight_shift = weight_shift((long long)num_k_block * k_block_size);
   pp.order = nullptr;
+  pp.order_k = nullptr;
   pp.room = nullptr;
   const dim3 grid((num_q_block + 3) / 4, nhead_k);
   if (ordered && order_bytes(nhead_k, num_q_block) != 0) {
     pp.order = (uint32_t *)((char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
+    pp.order_k = (int32_t *)((char *)pp.order + order_bytes(nhead_k, num_q_block));
     // (a captured launch may be replayed on any stream, while the room belongs to this one)
     if (!is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
     hipLaunchKernelGGL((hbsa_prep_kernel<true>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
@@ -1414,6 +1449,9 @@ int hbsa_bwd(const void *q, const void *k, const void *v, const void *out, const
   bp.nsub_k = (k_block_size + 4 * kWaveRows - 1) / (4 * kWaveRows);
   bp.flat_grid = ((long long)num_k_block * bp.nsub_k * nhead_k < (1LL << 31) && (long long)num_q_block * bp.nsub * nhead_k < (1LL << 31)) ? 1 : 0;
   bp.xcd_heads = bp.flat_grid && nhead_k % 8 == 0 ? 1 : 0;
+  if (order_bytes(nhead_k, num_q_block) != 0)
+    bp.order_k = (const int32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block));
+  bp.many = 2ll * num_k_block * bp.nsub_k * nhead_k > 9ll * device_cus();
   bp.c = softmax_scale * kLog2e;
   bp.scale = softmax_scale;
   hipStream_t st = (hipStream_t)stream;
