@@ -609,6 +609,18 @@ inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_bloc
   return (long long)nhead_k * num_q_block * ((slots + 3) / 4);
 }
 
+// Tiles of 16-key groups, for key block sizes that are no multiple of the tile: a tile of consecutive keys ends with its run of
+// kept blocks, and is then partly empty and masked.  The shorter the blocks, the more of that: 4 x 777 .. 5120 queries, 4100 ..
+// 8192 keys, 16 / 4 heads, half of the blocks kept, head dim 64, blocks of 16 / 48 / 112 / 208 keys 444 / 257 / 218 / 218 -> 177 /
+// 181 / 183 / 192 us; head dim 128, a fifth kept, 16 / 48 keys 420 / 209 -> 146 / 155; head dim 192 and 48 keys 273 -> 236; head dim
+// 256 1206 / 557 -> 391 / 405.  Whatever is kept the groups cost more address work a tile, and their list is longer: 464 and 976 keys
+// were even (239 -> 227, 261 -> 243, as much as runs gave), 2032 lost (151 -> 155 with a twentieth kept).
+// A group is numbered in 16 bits.  The rule is the same for the one-launch and the prepared form, so they compute the same bits.
+constexpr int kMostGroupedBlock = 256;
+inline bool fwd_grouped(int num_k_block, int k_block_size) {
+  return k_block_size % kTileKeys != 0 && k_block_size < kMostGroupedBlock && (long long)num_k_block * k_block_size <= 16 * 65535ll;
+}
+
 // The fields of FwdParams that follow from the call's shape and softmax_scale alone.
 void fill_shape(FwdParams &fp, int total_q, int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size,
                 int k_block_size, int causal, float softmax_scale, bool f32_exact, bool may_pack = false, bool cols = false) {
@@ -621,6 +633,7 @@ void fill_shape(FwdParams &fp, int total_q, int nhead_q, int nhead_k, int headdi
   const FwdSplit split = fwd_split(slots, headdim, f32_exact, (long long)nhead_k * num_q_block, num_k_block, k_block_size,
                                    (long long)num_q_block * q_block_size, total_q);
   fp.nw = split.nw;
+  fp.grouped = fwd_grouped(num_k_block, k_block_size) ? 1 : 0;
   fp.split = split.parts;
   fp.ncol = headdim / 8;
   fp.max_parts = 1;

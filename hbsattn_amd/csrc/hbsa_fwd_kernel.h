@@ -39,6 +39,7 @@ namespace hbsa {
 // item headers and two tile lists.
 // --------------------------------------------------------------------------------------
 constexpr int kListCap = 1024;   // tile entries per list; longer items are expanded in chunks
+constexpr int kGroupCap = 2 * kListCap;   // GROUPED: 16-bit entries of a list, one per 16 keys
 // Up to this many items per resident workgroup are handed out without the per-XCD work queues, in a fixed order
 // (see claim() in the kernel).  Measured against the queues: 8 x 512 tokens 71 -> 45 us, 8 x 1024 113 -> 99,
 // 8 x 2048 causal 200 -> 189, C5 0.33 -> 0.245 ms; at sixteen per workgroup 8 x 4096 tokens lose 5 % and at 64
@@ -51,7 +52,7 @@ constexpr float kMostSum = 256.f;   // 2^kLazyRescaleLog2
 static_assert(kLazyRescaleLog2 == 8.0f, "kMostSum");
 
 // Item header in LDS (16 ints).
-enum { H_HK = 0, H_QB, H_SUB, H_TOTAL, H_ROW_BEGIN, H_ROWS, H_KEY_BEGIN, H_Q_POS, H_SHIFT, H_PART, H_T0, H_SEQ, H_NKBLK, H_WORDS = 16 };
+enum { H_HK = 0, H_QB, H_SUB, H_TOTAL, H_ROW_BEGIN, H_ROWS, H_KEY_BEGIN, H_Q_POS, H_SHIFT, H_PART, H_T0, H_SEQ, H_NKBLK, H_GROUPS, H_KMAX, H_WORDS = 16 };
 
 __device__ __forceinline__ float max3(float a, float b, float c) {
   float r;
@@ -150,6 +151,43 @@ __device__ __forceinline__ int build_tile_list(int *list, int chunk_base, MoreWo
   return total;
 }
 
+// The same for tiles of 16-key groups: the kept blocks' groups (their in-sequence position / 16) one after another, entries
+// [chunk_base, chunk_base + kGroupCap) of them to list[0..); returns the item's number of groups.  Whole wavefront; block sizes
+// that are any multiple of 16.
+template <typename MoreWords>
+__device__ __forceinline__ int build_group_list(uint16_t *list, int chunk_base, MoreWords &&more_words, int nwords, int kbs,
+                                                FastDiv div_kbs, int kmax, uint32_t first_words, int lane) {
+  if (kmax <= 0 || nwords <= 0) return 0;
+  const int gpb = kbs >> 4;
+  const int half = lane >> 5, bit = lane & 31;
+  const int j_last = (int)fast_div((uint32_t)(kmax - 1), div_kbs);   // no bit above this block is set
+  int total = 0, window = 0;
+  uint32_t held = lane < nwords ? first_words : 0u;
+  for (int w2 = 0; w2 < nwords; w2 += 2) {   // 64 blocks a step, as above
+    if ((w2 >> 6) != window) {
+      window = w2 >> 6;
+      held = more_words(window);
+    }
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)held, w2 & 63);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)held, (w2 + 1) & 63);
+    if ((lo | hi) == 0) continue;
+    const uint32_t mine = half ? hi : lo;
+    if ((mine >> bit) & 1u) {
+      const int below = __builtin_popcount(mine & ((1u << bit) - 1u)) + (half ? __builtin_popcount(lo) : 0);
+      const int first = ((w2 + half) * 32 + bit) * gpb;
+      int off = total + below * gpb - chunk_base;
+      for (int g = 0; g < gpb; ++g, ++off)
+        if ((first + g) * 16 < kmax && off >= 0 && off < kGroupCap) list[off] = (uint16_t)(first + g);
+    }
+    total += (__builtin_popcount(lo) + __builtin_popcount(hi)) * gpb;
+    if ((j_last >> 6) == (w2 >> 1)) {   // groups dropped at the end of the last visible block
+      const uint32_t wsel = (j_last & 32) ? hi : lo;
+      if ((wsel >> (j_last & 31)) & 1u) total -= gpb - ((kmax - j_last * kbs + 15) >> 4);
+    }
+  }
+  return total;
+}
+
 // Placement of a K / V tile's rows in LDS: 16-byte chunk c of row r sits at chunk position c ^ k(r) (K), c ^ v(r) (V).
 // Rows by 16 consecutive ones (K, one chunk column at a time) then start at 16 different 16-byte slots of the 256-byte
 // bank sweep, and the 4 rows x 64 bytes of a transposing V read cover it once.  With a row of 4, 8, 16 or 32 chunks
@@ -167,7 +205,7 @@ struct FwdSwizzle {
   }
 };
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS>
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED>
 __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3 : 4) void hbsa_fwd_kernel(FwdParams p) {
   // OUT32: fp32 output (the fp32-input path; q/k/v are then fp16 staging copies)
   // EXTRAS: the clocked walk, the split over key blocks and the log-sum-exp output are compiled in.  The
@@ -181,6 +219,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   // COLS: the tensors' rows hold p.ncol <= D / 8 chunks of eight elements (a head dim that is no D of its own).  The
   // columns past them are zero in LDS (cleared once, never loaded) and in the Q operand, and not stored: in place of
   // zero-padded copies of q, k, v and a copy of the output.
+  // GROUPED: tiles are made of groups of 16 keys from any places, for block sizes that are no multiple of the tile.  Otherwise a
+  // tile is consecutive keys of one run of kept blocks, and the end of every run is a tile that is partly empty and has to be
+  // masked (blocks of 48 keys, half of them kept: 120 keys' worth of tiles for 96, half of the tiles masked).
   // NW: wavefronts (wave slots) of a workgroup, 4 or 8.  Eight are used when the q heads of a GQA group
   // and the 32-row slices of a q block give an item more than four wave slots: one workgroup per CU then
   // stages every K/V tile once for all of them instead of two workgroups staging it each (D = 128 only, and
@@ -449,6 +490,14 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       }
     }
   };
+  // the tiles (GROUPED: groups) [chunk_base, ..) of an item into list `c`; returns how many the item has
+  auto list_of = [&](int c, int chunk_base, auto &&more_words, int nwords, int kmax, uint32_t first_words) -> int {
+    const FwdParams &p = fresh_args();
+    if constexpr (GROUPED)
+      return build_group_list((uint16_t *)(lds_list + c * kListCap), chunk_base * (KT / 16), more_words, nwords, p.kbs, p.div_kbs, kmax, first_words, lane);
+    else
+      return build_tile_list<KT>(lds_list + c * kListCap, chunk_base, more_words, nwords, p.kbs, p.div_kbs, kmax, first_words, lane);
+  };
   // expand the staged item into list `c` and write its header
   auto build = [&](int c) {
     const FwdParams &p = fresh_args();
@@ -460,22 +509,22 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       if constexpr (FUSED) {
         // the staged bytes arrived with the wait of a tile, or one of the waits before the first item, since stage()
         st_bits = st_nvis > 0 ? staged_words(st_ms, min(st_nvis, kMaskWindow)) : 0u;
-        total = build_tile_list<KT>(lds_list + c * kListCap, 0, fused_more_words(st_mrow, st_nvis), 2 * ((st_nvis + 63) >> 6),
-                                p.kbs, p.div_kbs, kmax, st_bits, lane);
+        total = list_of(c, 0, fused_more_words(st_mrow, st_nvis), 2 * ((st_nvis + 63) >> 6), kmax, st_bits);
       } else {
         const int nwords = 2 * ((nkblk + 63) >> 6);
-        total = build_tile_list<KT>(lds_list + c * kListCap, 0,
-                                prepared_more_words(p.bits + (((size_t)st_part * p.nhead_k + st_hk) * p.nqb + st_qb) * p.wpr, nwords),
-                                nwords, p.kbs, p.div_kbs, kmax, st_bits, lane);
+        total = list_of(c, 0, prepared_more_words(p.bits + (((size_t)st_part * p.nhead_k + st_hk) * p.nqb + st_qb) * p.wpr, nwords),
+                        nwords, kmax, st_bits);
       }
     }
     if (lane == 0) {
-      hdr[H_HK] = st_hk; hdr[H_QB] = st_qb; hdr[H_SUB] = st_sub; hdr[H_TOTAL] = total; hdr[H_PART] = st_part;
+      hdr[H_HK] = st_hk; hdr[H_QB] = st_qb; hdr[H_SUB] = st_sub; hdr[H_PART] = st_part;
+      hdr[H_TOTAL] = GROUPED ? (total + KT / 16 - 1) / (KT / 16) : total;
+      if (GROUPED) hdr[H_GROUPS] = total;
       hdr[H_T0] = 0;   // the item's walk starts at its first tile unless next_start() decides otherwise
     }
     if (lane < 9) {   // QBlockInfo words: row_begin, rows, key_begin, klen, q_pos, shift, nkblk, kmax, seq
       const int dst = lane == 0 ? H_ROW_BEGIN : lane == 1 ? H_ROWS : lane == 2 ? H_KEY_BEGIN : lane == 4 ? H_Q_POS
-                      : lane == 5 ? H_SHIFT : lane == 6 ? H_NKBLK : lane == 8 ? H_SEQ : -1;
+                      : lane == 5 ? H_SHIFT : lane == 6 ? H_NKBLK : lane == 7 ? H_KMAX : lane == 8 ? H_SEQ : -1;
       if (dst >= 0) hdr[dst] = (int)st_info;
     }
   };
@@ -603,7 +652,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   // differ in their scalar base only; elsewhere every load has its offset in a register.
   constexpr bool UNIFORM = (64 * NW) % CPR == 0 && SW::POW2 && (64 * NW / CPR) % SW::PERIOD == 0;
   constexpr int ROUND_ROWS = UNIFORM ? 64 * NW / CPR : 0, OFFSETS = UNIFORM ? 1 : LOADS;
-  uint32_t ld_koff[OFFSETS], ld_voff[OFFSETS];   // byte offset of the thread's chunk from the tile's first row
+  uint32_t ld_koff[OFFSETS], ld_voff[OFFSETS];   // byte offset of the thread's chunk from the tile's (GROUPED: the group's) first row
   bool ld_kin[LOADS], ld_vin[LOADS];             // COLS: the chunk is one of the row's
   const uint32_t ks32 = (uint32_t)p.k_s, vs32 = (uint32_t)p.v_s;   // row strides in bytes (the host checks they fit)
   auto ld_place = [&](int i, int &r, uint32_t &kchunk, uint32_t &vchunk) {
@@ -618,8 +667,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     int r; uint32_t kc, vc;
     ld_place(i, r, kc, vc);
     if (i < OFFSETS) {
-      ld_koff[i] = (uint32_t)r * ks32 + kc;
-      ld_voff[i] = (uint32_t)r * vs32 + vc;
+      const uint32_t from = GROUPED ? (uint32_t)r & 15u : (uint32_t)r;
+      ld_koff[i] = from * ks32 + kc;
+      ld_voff[i] = from * vs32 + vc;
     }
     ld_kin[i] = !COLS || kc < (uint32_t)p.ncol * 16u;
     ld_vin[i] = !COLS || vc < (uint32_t)p.ncol * 16u;
@@ -638,11 +688,112 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   auto tile_ptr = [&](const char *base, int tok, uint32_t stride) {   // tok >= 0
     return base + (uint64_t)(uint32_t)tok * (uint64_t)stride;
   };
+  // A tile as the wavefronts know it: keys 0 .. valid - 1 of it exist, key x is the sequence's key pos(x / 16) + x % 16.
+  // Plain: consecutive keys from `first` on.  GROUPED: sixteen bits per group of 16 keys, their position / 16.
+  struct TileRef {
+    int first, valid;
+    uint32_t lo, hi;
+    __device__ __forceinline__ int pos(int g) const {
+      if constexpr (GROUPED) return (int)(((g < 2 ? lo : hi) >> (16 * (g & 1))) & 0xffffu) << 4;
+      else return first + 16 * g;
+    }
+  };
+  // step `at` (of all steps) of the item with header c_, from its list entry (GROUPED: 64 bits, four groups; 32 with two)
+  auto tile_ref = [&](uint32_t lo, uint32_t hi, int c_, int at, int total) -> TileRef {
+    TileRef r;
+    if constexpr (GROUPED) {
+      r.lo = lo;
+      r.hi = hi;
+      r.valid = KT;
+      r.first = r.pos(0);
+      if (at + 1 >= total) {   // the item's last tile: groups may be missing, and keys of the last group
+        const int n = hdr_word(c_, H_GROUPS) - at * (KT / 16);
+        int last = r.pos(0);
+#pragma unroll
+        for (int g = 1; g < KT / 16; ++g) last = n > g ? r.pos(g) : last;
+        r.valid = 16 * (n - 1) + min(16, hdr_word(c_, H_KMAX) - last);
+      }
+    } else {
+      r.first = (int)(lo >> 6) << 4;
+      r.valid = (int)(lo & 63u) + 1;
+      r.lo = r.hi = 0;
+    }
+    return r;
+  };
+  auto group_entry = [&](int c_, int at) -> u32x2 {   // GROUPED: entry `at` of list c_, the tile's groups
+    const int *list = lds_list + c_ * kListCap + at * (KT / 32);
+    if constexpr (KT == 64) return *(const u32x2 *)list;
+    else return u32x2{(uint32_t)*list, 0u};
+  };
+  // the tile of list entry `at` (of the list's chunk, which starts at step chunk_base)
+  auto listed_tile = [&](int c_, int at, int chunk_base) -> TileRef {
+    const int total = GROUPED ? hdr_word(c_, H_TOTAL) : 0;
+    if constexpr (GROUPED) {
+      const u32x2 w = group_entry(c_, at);
+      return tile_ref((uint32_t)__builtin_amdgcn_readfirstlane((int)w.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)w.y), c_, chunk_base + at, total);
+    } else {
+      return tile_ref((uint32_t)__builtin_amdgcn_readfirstlane(lds_list[c_ * kListCap + at]), 0u, c_, chunk_base + at, total);
+    }
+  };
+  static_assert(!GROUPED || 1024 % RB != 0 || NW * 64 / CPR % 16 == 0 || 16 % (NW * 64 / CPR) == 0, "no load is rows of two groups");
   // One operand's half of a tile's loads.  V_PART selects the V buffers (which follow the K buffers).
-  auto issue_part = [&](auto v_part_, int buf, const char *base, int valid) {
+  // base: of the sequence's first key (for this kv head)
+  auto issue_part = [&](auto v_part_, int buf, const char *base, const TileRef &tile) {
     constexpr bool V_PART = decltype(v_part_)::value;
     constexpr int lds_off = V_PART ? 2 * TILE_BYTES : 0;
     const uint32_t l0 = lds_k_addr + (uint32_t)(buf * TILE_BYTES) + (uint32_t)wave * 1024u;
+    const int valid = tile.valid;
+    const uint32_t stride = V_PART ? vs32 : ks32;
+    if constexpr (GROUPED) {
+      // Load i of this wavefront is rows of one group (g), or of two where a row is no power of two long.  The lane offsets
+      // count from the row's group.  Rows past the tile's end re-read the last valid row (masked later).
+      const uint64_t groups = (uint64_t)tile.hi << 32 | tile.lo;
+      int wave_ = wave;
+      if constexpr (KT == 32) asm volatile("" : "+s"(wave_));   // (or what follows from it is kept in registers for every load)
+      auto group_at = [&](int g) -> uint32_t { return ((uint32_t)(groups >> (16 * g)) & 0xffffu) << 4; };
+      if constexpr (KT == 32) {   // two groups: one scalar base, and the second group's lanes go on by the distance
+        const uint32_t apart = valid > 16 ? (uint32_t)(tile.pos(1) - tile.pos(0)) * stride : 0u;
+        base += (uint64_t)(uint32_t)tile.pos(0) * (uint64_t)stride;
+        static_for<0, LOADS>([&](auto i_) {
+          constexpr int i = decltype(i_)::value;
+          uint32_t voff = (V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i]) +
+                          (lane >= 16 * CPR - (i * NW + wave_) * 64 ? apart : 0u);
+          if (valid < KT) {
+            const int row = ((i * NW + wave_) * 64 + lane) / CPR;
+            uint32_t step = (uint32_t)((min(row, valid - 1) & 15) - (row & 15)) * stride;
+            asm volatile("" : "+v"(step));
+            voff += step;
+          }
+          if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))
+            dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, voff, l0);
+        });
+        return;
+      }
+      static_for<0, LOADS>([&](auto i_) {
+        constexpr int i = decltype(i_)::value;
+        constexpr bool ONE = 1024 % RB == 0;
+        constexpr int ROUND = NW * 64 / CPR;   // rows between two loads
+        const int row = ((i * NW + wave_) * 64 + lane) / CPR;
+        int g = ONE ? ((wave_ * 64 / CPR) >> 4) + i * ROUND / 16 : ((i * NW + wave_) * 64 / CPR) >> 4;
+        uint32_t voff = V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i];
+        if (valid < KT) {
+          g = min(g, (valid - 1) >> 4);
+          uint32_t step = (uint32_t)((min(row, valid - 1) & 15) - (row & 15)) * stride;
+          asm volatile("" : "+v"(step));   // (or a 64-bit multiply-add is formed, and its 64-bit addend kept in registers)
+          voff += step;
+        }
+        const uint32_t pos = group_at(g);
+        if constexpr (!ONE) {
+          const int second = 16 * (g + 1) * CPR - (i * NW + wave_) * 64;   // first lane of the second group, if one of them is
+          voff += lane >= second ? (group_at(min(g + 1, (valid - 1) >> 4)) - pos) * stride : 0u;
+        }
+        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))
+          dma16(std::integral_constant<int, lds_off + i * NW * 1024>{},
+                base + (uint64_t)(pos + (UNIFORM ? (uint32_t)(i * ROUND) & 15u : 0u)) * (uint64_t)stride, voff, l0);
+      });
+      return;
+    }
+    base = tile_ptr(base, tile.first, stride);
     if (valid == KT) {
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
@@ -661,11 +812,21 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       });
     }
   };
-  auto issue_k = [&](int buf, const char *kbase, int valid) { issue_part(std::false_type{}, buf, kbase, valid); };
-  auto issue_v = [&](int buf, const char *vbase, int valid) { issue_part(std::true_type{}, buf, vbase, valid); };
-  auto issue_loads = [&](int buf, const char *kbase, const char *vbase, int valid) {
-    issue_k(buf, kbase, valid);
-    issue_v(buf, vbase, valid);
+  auto issue_k = [&](int buf, const char *kbase, const TileRef &tile) { issue_part(std::false_type{}, buf, kbase, tile); };
+  auto issue_v = [&](int buf, const char *vbase, const TileRef &tile) { issue_part(std::true_type{}, buf, vbase, tile); };
+  // the first keys of the sequence of the item with header c_
+  auto item_k = [&](int c_) -> const char * {
+    const FwdParams &pn = fresh_args();
+    return tile_ptr(pn.k + (int64_t)hdr_word(c_, H_HK) * pn.k_h, hdr_word(c_, H_KEY_BEGIN), ks32);
+  };
+  auto item_v = [&](int c_) -> const char * {
+    const FwdParams &pn = fresh_args();
+    return tile_ptr(pn.v + (int64_t)hdr_word(c_, H_HK) * pn.v_h, hdr_word(c_, H_KEY_BEGIN), vs32);
+  };
+  auto issue_first = [&](int buf, int c_) {   // the first tile of an item that starts at its list's first entry
+    const TileRef tile = listed_tile(c_, 0, 0);
+    issue_k(buf, item_k(c_), tile);
+    issue_v(buf, item_v(c_), tile);
   };
 
   // per-lane LDS read addresses
@@ -814,15 +975,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     leave();
     return;
   }
-  {
-    const int total0 = hdr_word(0, H_TOTAL);
-    if (total0 > 0) {
-      const int e = __builtin_amdgcn_readfirstlane(lds_list[0]);
-      const int tok = hdr_word(0, H_KEY_BEGIN) + ((e >> 6) << 4);
-      const int hk = hdr_word(0, H_HK);
-      issue_loads(0, tile_ptr(p.k + (int64_t)hk * p.k_h, tok, ks32), tile_ptr(p.v + (int64_t)hk * p.v_h, tok, vs32), (e & 63) + 1);
-    }
-  }
+  if (hdr_word(0, H_TOTAL) > 0) issue_first(0, 0);
   request_q(hdr_word(0, H_HK), hdr_word(0, H_SUB), hdr_word(0, H_ROW_BEGIN), hdr_word(0, H_ROWS));
   // What this wavefront asked for so far has arrived, the scheduler's records included: the compiler is told here, or it
   // waits for ALL outstanding memory traffic where they are first read.
@@ -887,15 +1040,28 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     int nxt_hk = -1;          // known once the last tile is reached
     int chunk_base = 0;
     // the walk starts at entry t0 of the (ascending) list and wraps: step t takes entry rot(t)
-    const int t0 = total <= kListCap ? hdr_word(c, H_T0) : 0;
+    constexpr int kCap = GROUPED ? kGroupCap / (KT / 16) : kListCap;   // tiles of a list
+    const int t0 = !GROUPED && total <= kListCap ? hdr_word(c, H_T0) : 0;
     for (;;) {   // ---------------------------------------------------- chunks of the tile list (usually one)
-      const int n = min(kListCap, total - chunk_base);
+      const int n = min(kCap, total - chunk_base);
       auto rot = [&](int x) { return x + t0 >= n ? x + t0 - n : x + t0; };   // x < n
-      int held = 0;           // lane i: entry of step (window * 64 + i) of the current chunk
+      u32x2 held = {0u, 0u};  // lane i: entry of step (window * 64 + i) of the current chunk
+      auto entry_of = [&](int x) -> u32x2 {   // lane i: that of step x + i
+        u32x2 w = {0u, 0u};
+        if (x + lane < n) {
+          if constexpr (GROUPED) w = group_entry(c, x + lane);
+          else w.x = (uint32_t)lds_list[c * kListCap + rot(x + lane)];
+        }
+        return w;
+      };
+      auto held_tile = [&](const u32x2 &from, int lane_at, int x) -> TileRef {
+        return tile_ref((uint32_t)__builtin_amdgcn_readlane((int)from.x, lane_at),
+                        GROUPED ? (uint32_t)__builtin_amdgcn_readlane((int)from.y, lane_at) : 0u, c, chunk_base + x, total);
+      };
       for (int t = 0; t < n; ++t) {   // ---------------------------------- one iteration per 64-key tile
-        if ((t & 63) == 0) held = (t + lane < n) ? lds_list[c * kListCap + rot(t + lane)] : 0;
-        const int e = __builtin_amdgcn_readlane(held, t & 63);
-        const int kpos = (e >> 6) << 4, valid = (e & 63) + 1;
+        if ((t & 63) == 0) held = entry_of(t);
+        const TileRef tile = held_tile(held, t & 63, t);
+        const int kpos = tile.first, valid = tile.valid;
 
         if (t > 0 || chunk_base > 0 || !active) settle();   // the current tile has landed in LDS
         __syncthreads();                     // ... for every wave, and the other buffers are free
@@ -910,48 +1076,35 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           if (chunk_base + t + 2 == total) next_start(c ^ 1);
           if (last) leave_clock();
         }
-        int nx_valid = 0;                 // > 0: a next tile exists and its loads go out during this tile
-        const char *nx_vbase = nullptr, *nx_kbase = nullptr;
+        TileRef nx = {0, 0, 0u, 0u};      // valid > 0: a next tile exists and its loads go out during this tile
+        const char *nx_k = kg, *nx_v = vg;
         if (t + 1 < n) {
-          int e1;
-          if (((t + 1) & 63) == 0) {
-            const int h1 = (t + 1 + lane < n) ? lds_list[c * kListCap + rot(t + 1 + lane)] : 0;
-            e1 = __builtin_amdgcn_readlane(h1, 0);
-          } else {
-            e1 = __builtin_amdgcn_readlane(held, (t + 1) & 63);
-          }
-          const int tok = (e1 >> 6) << 4;
-          nx_valid = (e1 & 63) + 1;
-          nx_vbase = tile_ptr(vg, tok, vs32);
-          nx_kbase = tile_ptr(kg, tok, ks32);
+          if (((t + 1) & 63) == 0) nx = held_tile(entry_of(t + 1), 0, t + 1);
+          else nx = held_tile(held, (t + 1) & 63, t + 1);
         } else if (last) {
           nxt_hk = hdr_word(c ^ 1, H_HK);
           if (nxt_hk >= 0 && hdr_word(c ^ 1, H_TOTAL) > 0) {
-            const int e1 = __builtin_amdgcn_readfirstlane(lds_list[(c ^ 1) * kListCap + hdr_word(c ^ 1, H_T0)]);
-            const int tok = hdr_word(c ^ 1, H_KEY_BEGIN) + ((e1 >> 6) << 4);
-            nx_valid = (e1 & 63) + 1;
-            const FwdParams &pn = fresh_args();
-            nx_vbase = tile_ptr(pn.v + (int64_t)nxt_hk * pn.v_h, tok, vs32);
-            nx_kbase = tile_ptr(pn.k + (int64_t)nxt_hk * pn.k_h, tok, ks32);
+            nx = listed_tile(c ^ 1, GROUPED ? 0 : hdr_word(c ^ 1, H_T0), 0);
+            nx_k = item_k(c ^ 1);
+            nx_v = item_v(c ^ 1);
           }
         }
         // The next tile's K is requested right after this tile's first operand reads, its V only after
         // the first MFMA block: the wavefronts then do not all queue at the load unit at once.
 
         const bool compute = active && (!p.causal || kpos <= wave_kvis_max);
-        if (!compute && nx_valid > 0) {
-          issue_k(buf ^ 1, nx_kbase, nx_valid);
-          issue_v(buf ^ 1, nx_vbase, nx_valid);
+        if (!compute && nx.valid > 0) {
+          issue_k(buf ^ 1, nx_k, nx);
+          issue_v(buf ^ 1, nx_v, nx);
         }
         if (compute) {
           // The tile is processed as two halves of 32 keys so that, inside one wavefront, the
           // matrix cores always have work queued while the vector ALU does the softmax of the
           // other half:   S0, max(S0) | S1 + exp(S0) | PV0 + max(S1), exp(S1) | PV1.
           const bool first = chunk_base + t == 0;   // the item's first tile gives the reference
-          const bool edge = valid < KT || (p.causal && kpos + valid - 1 > wave_kvis_min);
-          int lim = valid;                      // keys (of this lane's query) below lim are visible
-          if (p.causal) lim = min(lim, lane_kvis - kpos + 1);
-          lim -= 4 * g32;
+          // keys that are missing, or (causal) a last key that some lane's query does not see
+          const bool edge = valid < KT || (p.causal && tile.pos(KT / 16 - 1) + 15 > wave_kvis_min);
+
 
           f32x16 s0, s1;
 #pragma unroll
@@ -971,7 +1124,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           };
           static_for<0, PF>(read_k);
           // the next tile's K is requested while this tile's first operands are on their way from LDS
-          if (nx_valid > 0) issue_k(buf ^ 1, nx_kbase, nx_valid);
+          if (nx.valid > 0) issue_k(buf ^ 1, nx_k, nx);
           // ---- S0 = K[0:32] . Q^T
           static_for<0, KSTEPS>([&](auto i_) {
             constexpr int i = decltype(i_)::value;
@@ -981,7 +1134,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
             if constexpr (i + PF < NK) read_k(std::integral_constant<int, i + PF>{});
           });
 
-          if (nx_valid > 0) issue_v(buf ^ 1, nx_vbase, nx_valid);
+          if (nx.valid > 0) issue_v(buf ^ 1, nx_v, nx);
 
           // Largest score of one half in log2 units.  The first reduction step is an instruction the compiler knows, so
           // that it inserts the wait states an MFMA result needs before the vector ALU may read it; the
@@ -992,11 +1145,18 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
             for (int i = 2; i < 16; i += 2) mx = max3(mx, sh[i], sh[i + 1]);
             return half_max(mx) * sm_c;
           };
-          auto hide = [&](f32x16 &sh, int key0) {   // keys this lane's query does not see
+          auto hide = [&](f32x16 &sh, int half) {   // keys this lane's query does not see
             if (edge) {
+              int lim[2];   // keys of the half's two groups below lim are visible
+#pragma unroll
+              for (int g = 0; g < 2; ++g) {
+                lim[g] = valid - 32 * half - 16 * g;
+                if (p.causal) lim[g] = min(lim[g], lane_kvis - tile.pos(2 * half + g) + 1);
+                lim[g] -= 4 * g32;
+              }
 #pragma unroll
               for (int i = 0; i < 16; ++i)
-                if (key0 + 8 * (i >> 2) + (i & 3) >= lim) sh[i] = -INFINITY;
+                if (8 * ((i >> 2) & 1) + (i & 3) >= lim[i >> 3]) sh[i] = -INFINITY;
             }
           };
           // exponentials of one half against reference m, packed to the element type (two groups of 16 keys); their sum
@@ -1110,7 +1270,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           read_vgroup(std::integral_constant<int, 0>{}, vb[0]);
           read_vgroup(std::integral_constant<int, 1>{}, vb[1]);
           settle_half(s0, half_exp(s0, m_ref, p0a, p0b), p0a, p0b);
-          hide(s1, 32);
+          hide(s1, 1);
 
           // ---- O^T += V^T[:, 0:32] . P0   interleaved with   P1 = exp(S1)
           wait_vgroup(std::integral_constant<int, 2 * DT>{}, vb[0]);
@@ -1144,23 +1304,21 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           const int nvis = min(inf.nkblk, (int)fast_div((uint32_t)(inf.kmax + p.kbs - 1), p.div_kbs));
           auto more = fused_more_words(p.mask + (int64_t)cur_hk * p.ms_h + (int64_t)qb * p.ms_q + kb0, nvis);
           const uint32_t first = more(0);
-          (void)build_tile_list<KT>(lds_list + c * kListCap, chunk_base, more, 2 * ((nvis + 63) >> 6), p.kbs, p.div_kbs, inf.kmax,
-                                first, lane);
+          (void)list_of(c, chunk_base, more, 2 * ((nvis + 63) >> 6), inf.kmax, first);
           // the staging area held the staged item's bytes: request them again (they arrive with the next tile's wait)
           if (st_hk >= 0 && st_nvis > 0) st_ms = mask_dma(st_mrow, 0, min(st_nvis, kMaskWindow));
         } else {
           const QBlockInfo inf = p.info[qb];
           const uint32_t *row = p.bits + (((size_t)cur_part * p.nhead_k + cur_hk) * p.nqb + qb) * p.wpr;
           const int nwords = 2 * ((inf.nkblk + 63) >> 6);
-          (void)build_tile_list<KT>(lds_list + c * kListCap, chunk_base, prepared_more_words(row, nwords), nwords, p.kbs, p.div_kbs,
-                                inf.kmax, lane < nwords ? row[lane] : 0u, lane);
+          (void)list_of(c, chunk_base, prepared_more_words(row, nwords), nwords, inf.kmax, lane < nwords ? row[lane] : 0u);
         }
       }
       __syncthreads();
       {   // nothing is in flight here: fetch the chunk's first tile
-        const int e = __builtin_amdgcn_readfirstlane(lds_list[c * kListCap]);
-        const int tok = (e >> 6) << 4;
-        issue_loads(buf, tile_ptr(kg, tok, ks32), tile_ptr(vg, tok, vs32), (e & 63) + 1);
+        const TileRef tile = listed_tile(c, 0, chunk_base);
+        issue_k(buf, kg, tile);
+        issue_v(buf, vg, tile);
       }
     }
 
@@ -1259,12 +1417,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       __syncthreads();
       nxt_hk = hdr_word(c ^ 1, H_HK);
       if (nxt_hk >= 0) {
-        if (hdr_word(c ^ 1, H_TOTAL) > 0) {
-          const int e1 = __builtin_amdgcn_readfirstlane(lds_list[(c ^ 1) * kListCap]);
-          const int tok = hdr_word(c ^ 1, H_KEY_BEGIN) + ((e1 >> 6) << 4);
-          issue_loads(buf, tile_ptr(p.k + (int64_t)nxt_hk * p.k_h, tok, ks32), tile_ptr(p.v + (int64_t)nxt_hk * p.v_h, tok, vs32),
-                      (e1 & 63) + 1);
-        }
+        if (hdr_word(c ^ 1, H_TOTAL) > 0) issue_first(buf, c ^ 1);
         request_q(nxt_hk, hdr_word(c ^ 1, H_SUB), hdr_word(c ^ 1, H_ROW_BEGIN), hdr_word(c ^ 1, H_ROWS));
       }
       __syncthreads();   // wave 0 rewrites this item's list next; every wave has read its header by now
@@ -1285,10 +1438,10 @@ inline int persistent_grid(const void *kernel, int lds_bytes, int threads) {
   return cus * per_cu;
 }
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false, bool COLS = false>
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false, bool COLS = false, bool GROUPED = false>
 int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   constexpr int lds_bytes = 4 * (D > 128 && D <= 192 ? 32 : 64) * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
-  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS>);
+  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED>);
   // workgroups that fit the current device at once; the attribute and the occupancy are per device
   static thread_local int resident_of[kMaxDevices] = {};
   int dev = 0;
@@ -1307,35 +1460,48 @@ int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   // heads, the crowd at few counters) would be a good part of such a launch.
   launch.one_each = items <= (long long)kStaticShare * resident ? (int)items : 0;
   if (launch.one_each == 0 || launch.nparts != 1 || items <= resident) launch.order = nullptr;
-  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
+  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, "hbsa_fwd_kernel launch: %s", hipGetErrorString(e));
   return 0;
 }
-template <int D, typename E, bool OUT32>
-int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream) {
+template <int D, typename E, bool OUT32, bool GROUPED>
+int launch_fwd_tiles(const FwdParams &fp, long long items, hipStream_t stream) {
   const bool extras = fp.walk != 0 || fp.nparts > 1 || fp.lse != nullptr;
   if constexpr (D == 128) {
     if (fp.nw == 8)
-      return extras ? launch_fwd_nw<D, E, OUT32, 8, true>(fp, items, stream) : launch_fwd_nw<D, E, OUT32, 8, false>(fp, items, stream);
+      return extras ? launch_fwd_nw<D, E, OUT32, 8, true, false, false, false, GROUPED>(fp, items, stream)
+                    : launch_fwd_nw<D, E, OUT32, 8, false, false, false, false, GROUPED>(fp, items, stream);
   }
-  return extras ? launch_fwd_nw<D, E, OUT32, 4, true>(fp, items, stream) : launch_fwd_nw<D, E, OUT32, 4, false>(fp, items, stream);
+  return extras ? launch_fwd_nw<D, E, OUT32, 4, true, false, false, false, GROUPED>(fp, items, stream)
+                : launch_fwd_nw<D, E, OUT32, 4, false, false, false, false, GROUPED>(fp, items, stream);
+}
+template <int D, typename E, bool OUT32>
+int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream) {
+  return fp.grouped ? launch_fwd_tiles<D, E, OUT32, true>(fp, items, stream) : launch_fwd_tiles<D, E, OUT32, false>(fp, items, stream);
 }
 // the one-launch form (16-bit tensors, none of the extras)
-template <int D, typename E>
-int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream) {
+template <int D, typename E, bool GROUPED>
+int launch_fused_tiles(const FwdParams &fp, long long items, hipStream_t stream) {
   if constexpr (D == 128) {
     if (fp.nw == 8)
-      return fp.pack ? launch_fwd_nw<D, E, false, 8, false, true, true>(fp, items, stream)
-                     : launch_fwd_nw<D, E, false, 8, false, true, false>(fp, items, stream);
+      return fp.pack ? launch_fwd_nw<D, E, false, 8, false, true, true, false, GROUPED>(fp, items, stream)
+                     : launch_fwd_nw<D, E, false, 8, false, true, false, false, GROUPED>(fp, items, stream);
   }
-  return fp.pack ? launch_fwd_nw<D, E, false, 4, false, true, true>(fp, items, stream)
-                 : launch_fwd_nw<D, E, false, 4, false, true, false>(fp, items, stream);
+  return fp.pack ? launch_fwd_nw<D, E, false, 4, false, true, true, false, GROUPED>(fp, items, stream)
+                 : launch_fwd_nw<D, E, false, 4, false, true, false, false, GROUPED>(fp, items, stream);
+}
+template <int D, typename E>
+int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream) {
+  return fp.grouped ? launch_fused_tiles<D, E, true>(fp, items, stream) : launch_fused_tiles<D, E, false>(fp, items, stream);
 }
 
 // the one-launch form for tensors whose head dim (fp.ncol chunks of eight elements) is D or less
 template <int D, typename E>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream) {
+  // (a load of rows whose length is no power of two can span two groups: the lanes' offsets have to reach from one to the other)
+  const bool reaches = 1024 % (2 * D) == 0 || (uint64_t)fp.wpr * 32u * (uint64_t)fp.kbs * (uint64_t)std::max(fp.k_s, fp.v_s) < (1ull << 32);
+  if (fp.grouped && reaches) return launch_fwd_nw<D, E, false, 4, false, true, true, true, true>(fp, items, stream);
   return launch_fwd_nw<D, E, false, 4, false, true, true, true>(fp, items, stream);
 }
 

@@ -1,0 +1,47 @@
+"""Key block sizes that are no multiple of the forward kernel's tile: tiles made of 16-key groups of any kept blocks."""
+import pytest
+import torch
+
+from hbsattn_amd import HBSAttention, set_onepass
+from hbsattn_amd.workloads import make_problem
+from helpers import assert_close_to_oracle, oracle_for
+
+pytestmark = pytest.mark.gpu
+
+
+def check(w, what, same_bits=True):
+    """Against the oracle, in the one-launch form and in the prepared form, which compute the same bits."""
+    ref, outs = oracle_for(w), []
+    for one in (True, False):
+        previous = set_onepass(one)
+        try:
+            outs.append(HBSAttention(*w.args()))
+        finally:
+            set_onepass(previous)
+        assert_close_to_oracle(outs[-1], ref, f"{what} one={one}")
+    assert not same_bits or torch.equal(*outs)
+
+
+@pytest.mark.parametrize("kbs", [16, 48, 80, 240, 272])   # 256 and more keep to runs of consecutive keys
+@pytest.mark.parametrize("d", [32, 40, 64, 96, 128, 160, 192, 224, 256])
+def test_blocks_and_tails_of_every_remainder(d, kbs):
+    # key lengths of 1, 15, 16, 17, 63, 64, 65 past whole blocks, more and fewer keys than queries, whole and missing last groups
+    for causal, gqa, k_lens in ((True, 1, [kbs + 1, 2 * kbs + 15, 3 * kbs + 16, 700]), (False, 4, [17, 4 * kbs + 63, 64, 65 + kbs])):
+        w = make_problem(seed=kbs + d, q_lens=[130, 77, 300, 64], k_lens=k_lens, hq=4, hk=4 // gqa, d=d, qbs=64, kbs=kbs, keep=0.6,
+                         diag=True, causal=causal, scale=None)
+        check(w, f"d={d} kbs={kbs} causal={causal}")
+
+
+@pytest.mark.parametrize("d", [64, 96, 192, 256])
+def test_items_longer_than_a_list(d):
+    # about 38000 kept keys an item, a list holds 32768; more items than are split over their key blocks
+    w = make_problem(seed=5, q_lens=[350], k_lens=[40003], hq=16, hk=16, d=d, qbs=16, kbs=48, keep=0.95, diag=False, causal=False, scale=None)
+    check(w, f"d={d}", same_bits=d in (64, 256))   # (padded head dims may be cut into parts differently)
+
+
+@pytest.mark.parametrize("blocks", [65535, 65536], ids=lambda n: f"{n}blocks")
+def test_the_last_group_that_can_be_numbered(blocks):
+    # a group's number has 16 bits: one key block more and the kernel for runs is taken
+    w = make_problem(seed=6, q_lens=[64], k_lens=[16 * blocks - 3], hq=1, hk=1, d=32, qbs=64, kbs=16, keep=0.01, diag=False, causal=False, scale=None)
+    w.block_mask[..., -40:] = True   # (half of the kept keys' weight is where numbers are largest)
+    check(w, f"{blocks} blocks")
