@@ -1044,12 +1044,13 @@ size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t 
 
 }  // extern "C"
 namespace {
-// ordered: the order of the items is made, too (see OrderRoom); only a run that is split over key blocks can do without
+// weighted: the items' order is made by their weights (see OrderRoom), which only a run that is split over key blocks can do
+// without.  The k blocks' order is there in any case: a backward may follow on the workspace.
 int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
                      const int32_t *q_block_to_batch, const int32_t *cu_num_q_block, const int32_t *cu_num_k_block,
                      void *workspace, size_t workspace_bytes, int32_t batch, int32_t nhead_k, int32_t num_q_block,
                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size, int32_t causal,
-                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream, bool ordered) {
+                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream, bool weighted) {
   g_err[0] = 0;
   if (batch < 0 || num_q_block < 0 || num_k_block < 0 || total_q < 0 || total_k < 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
@@ -1085,11 +1086,11 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
   pp.order_k = nullptr;
   pp.room = nullptr;
   const dim3 grid((num_q_block + 3) / 4, nhead_k);
-  if (ordered && order_bytes(nhead_k, num_q_block) != 0) {
+  if (order_bytes(nhead_k, num_q_block) != 0) {
     pp.order = (uint32_t *)((char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
     pp.order_k = (int32_t *)((char *)pp.order + order_bytes(nhead_k, num_q_block));
     // (a captured launch may be replayed on any stream, while the room belongs to this one)
-    if (!is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
+    if (weighted && !is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
     hipLaunchKernelGGL((hbsa_prep_kernel<true>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
   } else {
     hipLaunchKernelGGL((hbsa_prep_kernel<false>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);

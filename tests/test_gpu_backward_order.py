@@ -1,9 +1,11 @@
 """dK/dV items taken in the order of the rows that can see them, and the form of the kernel for many of them."""
+import ctypes
+
 import pytest
 import torch
 
-from hbsattn_amd import calculate_blocks
-from hbsattn_amd.interface import hbsa_backward, hbsa_prepare, hbsa_run
+from hbsattn_amd import _lib, calculate_blocks
+from hbsattn_amd.interface import PreparedMask, hbsa_backward, hbsa_prepare, hbsa_run
 from oracle.grads import hbsa_oracle_grads
 from test_gpu_backward import _check, _problem
 
@@ -48,3 +50,29 @@ def test_gradients_in_the_order_of_the_weights(case, dtype):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out2, out) and all(torch.equal(a, b) for a, b in zip(got, grads))
+
+
+def test_gradients_on_the_workspace_of_a_forward_split_over_key_blocks():
+    # such a forward takes its items in no order of weights; the backward's order of the k blocks has to be there all the same
+    q_lens, k_lens, hq, hk, d, qbs, kbs, causal = [200, 130], [9000, 7001], 4, 4, 64, 64, 64, True
+    q, k, v, do, cu_q, cu_k, cq, ck, mask = _problem(12, q_lens, k_lens, hq, hk, d, qbs, kbs, 0.5, torch.bfloat16)
+    print("backward on a split forward's workspace", flush=True)
+    lib = _lib.load()
+    qd, kd, vd, dod, maskd = (t.cuda() for t in (q, k, v, do, mask))
+    (nq, _, q2b, cu_nq), (nk, _, _, cu_nk) = calculate_blocks(cq, qbs), calculate_blocks(ck, kbs)
+    need = lib.hbsa_fwd_workspace_bytes(hk, nq, nk)
+    split = lib.hbsa_fwd_split_workspace_bytes(q.shape[0], hq, hk, d, nq, nk, qbs)
+    assert split > 0
+    ws = torch.zeros(need + split, dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(qd)
+    meta = [t.to(torch.int32).contiguous() for t in (q2b, cu_nq, cu_nk)]
+    strides = (ctypes.c_int64 * 11)(*(n for t in (qd, kd, vd, out) for n in t.stride()[:2]), *maskd.stride())
+    rc = lib.hbsa_fwd(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), cq.data_ptr(), ck.data_ptr(), maskd.data_ptr(),
+                      *(t.data_ptr() for t in meta), ws.data_ptr(), ws.numel(), _lib.DTYPE_BF16, len(q_lens), q.shape[0], k.shape[0],
+                      hq, hk, d, nq, nk, qbs, kbs, int(causal), d ** -0.5, strides, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    prepared = PreparedMask(ws, hk, nq, nk, qbs, kbs, causal, ck, meta[1], meta[2])
+    out, lse = hbsa_run(qd, kd, vd, prepared, None, return_lse=True)
+    got = hbsa_backward(qd, kd, vd, out, dod, lse, prepared, None)
+    for x, ref, name in zip(got, hbsa_oracle_grads(q, k, v, do, cu_q, cu_k, mask, qbs, kbs, causal, None), ("dq", "dk", "dv")):
+        _check(x, ref, name)
