@@ -358,12 +358,16 @@ inline size_t bits_offset(int nhead_k, int num_q_block) {
 inline size_t order_offset(int nhead_k, int num_q_block, int num_k_block) {
   return bits_offset(nhead_k, num_q_block) + align_up((size_t)nhead_k * num_q_block * words_per_row(num_k_block) * sizeof(uint32_t), 256);
 }
-inline size_t order_bytes(int nhead_k, int num_q_block) {   // of the items; 0: too many of them, and no orders at all
+constexpr int kMaxOrderKBlocks = 65536;   // (hbsa_fwd_static's array has room for the orders beside what it holds without them)
+inline size_t order_bytes(int nhead_k, int num_q_block, int num_k_block) {   // of the items; 0: too many of them, and no orders at all
   const long long pairs = (long long)nhead_k * num_q_block;
-  return pairs > kMaxOrderItems ? 0 : align_up((size_t)pairs * sizeof(uint32_t), 256);
+  return pairs > kMaxOrderItems || num_k_block > kMaxOrderKBlocks ? 0 : align_up((size_t)pairs * sizeof(uint32_t), 256);
 }
 inline size_t order_k_bytes(int nhead_k, int num_q_block, int num_k_block) {
-  return order_bytes(nhead_k, num_q_block) == 0 ? 0 : align_up((size_t)num_k_block * sizeof(int32_t), 256);
+  return order_bytes(nhead_k, num_q_block, num_k_block) == 0 ? 0 : align_up((size_t)num_k_block * sizeof(int32_t), 256);
+}
+inline size_t orders_bytes(int nhead_k, int num_q_block, int num_k_block) {
+  return order_bytes(nhead_k, num_q_block, num_k_block) + order_k_bytes(nhead_k, num_q_block, num_k_block);
 }
 
 // Deterministic mode (the default, like the reference's ascending scan): every item walks its tiles in
@@ -701,7 +705,8 @@ int run_fwd(FwdParams &fp, long long items, hipStream_t stream, char *split_area
 // stream_sched: launch records (work-queue counters) of the one-launch form of hbsa_fwd, one per stream.  They
 // are zero when the library is loaded and every attention launch leaves its record at zero, so a call needs
 // no launch of its own to prepare one; calls on different streams use different records and may overlap.
-static __device__ __align__(256) unsigned char scratch[HBSA_STATIC_SCRATCH_BYTES];
+// Behind HBSA_STATIC_SCRATCH_BYTES there is room for the orders of the items and k blocks.
+static __device__ __align__(256) unsigned char scratch[HBSA_STATIC_SCRATCH_BYTES + 4 * hbsa::kMaxOrderItems + 4 * hbsa::kMaxOrderKBlocks];
 constexpr int kStreamSlots = 64;
 static __device__ __align__(256) unsigned char stream_sched[kStreamSlots * sizeof(hbsa::Sched)];
 // stream_arrivals: the counters of launches whose items are cut into parts (ItemParts), likewise one set per stream.
@@ -1004,7 +1009,7 @@ int hbsa_block_arrays(const int32_t *cu_seqlen, const int32_t *first, int32_t ba
 
 size_t hbsa_fwd_workspace_bytes(int32_t nhead_k, int32_t num_q_block, int32_t num_k_block) {
   if (nhead_k <= 0 || num_q_block <= 0 || num_k_block <= 0) return 256;
-  return order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block) + order_k_bytes(nhead_k, num_q_block, num_k_block);
+  return order_offset(nhead_k, num_q_block, num_k_block) + orders_bytes(nhead_k, num_q_block, num_k_block);
 }
 
 size_t hbsa_fwd_workspace_bytes_dtype(int32_t dtype, int32_t total_q, int32_t total_k, int32_t nhead_q,
@@ -1086,9 +1091,9 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
   pp.order_k = nullptr;
   pp.room = nullptr;
   const dim3 grid((num_q_block + 3) / 4, nhead_k);
-  if (order_bytes(nhead_k, num_q_block) != 0) {
+  if (order_bytes(nhead_k, num_q_block, num_k_block) != 0) {
     pp.order = (uint32_t *)((char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
-    pp.order_k = (int32_t *)((char *)pp.order + order_bytes(nhead_k, num_q_block));
+    pp.order_k = (int32_t *)((char *)pp.order + order_bytes(nhead_k, num_q_block, num_k_block));
     // (a captured launch may be replayed on any stream, while the room belongs to this one)
     if (weighted && !is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
     hipLaunchKernelGGL((hbsa_prep_kernel<true>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
@@ -1204,7 +1209,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
   }
   fp.div_nparts = make_fast_div((uint32_t)fp.nparts);
   // the clocked walk: block sizes that are whole tiles, work that is not split, K/V of a head beyond what an L2 holds
-  if (order_bytes(nhead_k, num_q_block) != 0) fp.order = (const uint32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
+  if (order_bytes(nhead_k, num_q_block, num_k_block) != 0) fp.order = (const uint32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
   fp.walk = (!g_deterministic && fp.nparts == 1 && k_block_size % kTileKeys == 0 &&
              2ll * total_k * headdim * 2 >= g_walk_min_bytes) ? 1 : 0;
 
@@ -1371,15 +1376,16 @@ int hbsa_fwd_static(const void *q, const void *k, const void *v, void *out, cons
   if (total_q == 0 || num_q_block == 0 || nhead_q == 0) return 0;
   const size_t need = hbsa_fwd_workspace_bytes_dtype(dtype, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block,
                                                      num_k_block);
-  if (need > (size_t)HBSA_STATIC_SCRATCH_BYTES)
+  // (nhead_k <= 0 is refused by the call)
+  const size_t holds = (size_t)HBSA_STATIC_SCRATCH_BYTES + (nhead_k > 0 && num_k_block > 0 ? orders_bytes(nhead_k, num_q_block, num_k_block) : 0);
+  if (need > holds)
     return fail(HBSA_ERR_WORKSPACE_TOO_SMALL,
-                "this problem needs %zu bytes of scratch, hbsa_fwd_static holds %zu: use hbsa_fwd with a workspace", need,
-                (size_t)HBSA_STATIC_SCRATCH_BYTES);
+                "this problem needs %zu bytes of scratch, hbsa_fwd_static holds %zu: use hbsa_fwd with a workspace", need, holds);
   void *ws = nullptr;
   if (int rc = static_scratch(&ws)) return rc;
   // (always the pre-pass and the attention kernel on the static array: this form may be captured into a graph)
   return fwd_call(q, k, v, out, cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block, ws,
-                  (size_t)HBSA_STATIC_SCRATCH_BYTES, dtype, batch, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block,
+                  holds, dtype, batch, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block,
                   num_k_block, q_block_size, k_block_size, causal, softmax_scale, strides, stream, false);
 }
 
@@ -1463,8 +1469,8 @@ int hbsa_bwd(const void *q, const void *k, const void *v, const void *out, const
   bp.nsub_k = (k_block_size + 4 * kWaveRows - 1) / (4 * kWaveRows);
   bp.flat_grid = ((long long)num_k_block * bp.nsub_k * nhead_k < (1LL << 31) && (long long)num_q_block * bp.nsub * nhead_k < (1LL << 31)) ? 1 : 0;
   bp.xcd_heads = bp.flat_grid && nhead_k % 8 == 0 ? 1 : 0;
-  if (order_bytes(nhead_k, num_q_block) != 0)
-    bp.order_k = (const int32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block));
+  if (order_bytes(nhead_k, num_q_block, num_k_block) != 0)
+    bp.order_k = (const int32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block, num_k_block));
   bp.many = 2ll * num_k_block * bp.nsub_k * nhead_k > 9ll * device_cus();
   bp.c = softmax_scale * kLog2e;
   bp.scale = softmax_scale;

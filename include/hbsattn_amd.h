@@ -257,7 +257,8 @@ int hbsa_fwd_one(const void *const *ptrs, const int32_t *sizes, float softmax_sc
  * `workspace` / `workspace_bytes`: the work description lives in a device array of
  * HBSA_STATIC_SCRATCH_BYTES inside the library, which every GPU the library runs on holds until the
  * process ends.  The call allocates and frees nothing.  A problem whose
- * hbsa_fwd_workspace_bytes_dtype(...) exceeds HBSA_STATIC_SCRATCH_BYTES is refused with
+ * hbsa_fwd_workspace_bytes_dtype(...) exceeds HBSA_STATIC_SCRATCH_BYTES (not counting the orders of its q and
+ * k blocks, at most 272 KiB, which lie behind them) is refused with
  * HBSA_ERR_WORKSPACE_TOO_SMALL before anything is launched.  All calls on one GPU share that GPU's
  * array: calls on one stream are ordered and safe; calls that overlap on one GPU (different streams
  * or host threads) race on it and must be serialised by the caller.  The first call on a device looks

@@ -72,6 +72,18 @@ def test_static_entry_point_matches_hbsa_fwd_on_two_calls_in_a_row():
         assert_close_to_oracle(got, oracle_for(w), name)
 
 
+def test_static_entry_point_takes_what_fills_its_array():
+    # 4096 q blocks x 65,000 k blocks: 31.97 MiB without the orders of the blocks, which come on top
+    lib = _lib.load()
+    w = make_problem(seed=33, q_lens=[64 * 4096 - 5], k_lens=[16 * 65000 - 3], hq=1, hk=1, d=32, qbs=64, kbs=16, keep=0.0005, diag=False,
+                     causal=False, scale=None, device="cuda", gen_device="device")
+    need = lib.hbsa_fwd_workspace_bytes(1, 4096, 65000)
+    assert _lib.STATIC_SCRATCH_BYTES < need <= _lib.STATIC_SCRATCH_BYTES + (272 << 10)
+    rc, got = _fwd_static(w)
+    assert rc == 0, _lib.last_error()
+    assert torch.equal(got, _fwd_with_workspace(w))
+
+
 def test_static_entry_point_refuses_problems_beyond_its_array():
     # 64 kv heads x 4096 q blocks x 4096 k blocks: the bit rows alone need 128 MiB
     lib = _lib.load()
