@@ -42,6 +42,11 @@ constexpr int kSeqCap = 128;
 constexpr int kDecodeMaxParts = 32;    // parts of an item of the decode kernel
 constexpr int kDecodeEntries = 64;     // (q head, row) entries of an item of the decode kernel, as the host bounds them
 constexpr int kMaxPartItems = 4096;   // items of a launch that may be cut into parts (its arrival counters)
+// Up to this many items per resident workgroup are handed out without the per-XCD work queues, in a fixed order
+// (see claim() in hbsa_fwd_kernel).  Measured against the queues: 8 x 512 tokens 71 -> 45 us, 8 x 1024 113 -> 99,
+// 8 x 2048 causal 200 -> 189, C5 0.33 -> 0.245 ms; at sixteen per workgroup 8 x 4096 tokens lose 5 % and at 64
+// C2 and C3 lose 5-8 % (the queues keep one head's K/V in one XCD's L2).
+constexpr int kStaticShare = 8;
 constexpr int kMaxDevices = 64;            // devices of one process the launch caches cover
 constexpr float kLazyRescaleLog2 = 8.0f;  // the reference of a row's exponentials may lag the true maximum by 2^8
 
@@ -78,6 +83,7 @@ struct PrepParams {
   struct OrderRoom *room;  // the stream's room for making it, nullptr: the order without weights is written
   int32_t nhead_k, weight_shift;
   int32_t *order_k;        // [nkb]: the k blocks by falling number of query rows that can see them
+  int32_t weigh_k;         // 0: in their own order
 };
 
 // Division by a launch constant d, exact for 0 <= n < 2^31: n / d == (n * m) >> s with

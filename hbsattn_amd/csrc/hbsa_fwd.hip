@@ -31,32 +31,63 @@ namespace hbsa {
 // --------------------------------------------------------------------------------------
 // Pre-pass: one wavefront per (kv head, q block).
 // --------------------------------------------------------------------------------------
-// The place of k block kb among all k blocks of the batch, by falling number of query rows that can see a key of it (equals in
-// their own order).  That number falls along a sequence, so how many blocks of another sequence come first is a division.
-// Boundaries that do not fit each other, or a long batch: its own number.
-__device__ __forceinline__ int k_block_place(const PrepParams &p, int kb) {
-  if (p.batch > 256 || p.cu_num_k_block[0] != 0 || p.cu_num_k_block[p.batch] != p.nkb) return kb;
-  auto qlen_of = [&](int s) { return p.cu_q[s + 1] - p.cu_q[s]; };
-  auto klen_of = [&](int s) { return p.cu_k[s + 1] - p.cu_k[s]; };
-  int b = 0;
-  bool good = true;
-  for (int s = 0; s < p.batch; ++s) {
-    const int qlen = qlen_of(s), klen = klen_of(s), first = p.cu_num_k_block[s];
-    good = good && qlen >= 0 && klen >= 0 && p.cu_num_k_block[s + 1] - first == (int)(((int64_t)klen + p.kbs - 1) / p.kbs);
-    if (first <= kb) b = s;
+// The k blocks of the batch by falling number of query rows that can see a key of them (equals in their own order), for a
+// backward.  That number falls along a sequence, so how many blocks of another sequence come before a block is a division.  A
+// wavefront works on one block at a time, a lane on a sequence in 64.  (A lane per block that went through the sequences took
+// 110 us with 250 of them and 40 with 64.)  Boundaries that do not fit each other, a long batch, a
+// call that no backward need follow (weigh_k 0): the blocks' own order.
+constexpr int kWeighedSequences = 256;
+__device__ __forceinline__ void order_k_blocks(const PrepParams &p, int wave, int waves, int lane) {
+  constexpr int N = kWeighedSequences / 64;
+  int qlen[N], klen[N], first[N], n[N];
+  bool weigh = p.weigh_k != 0 && p.batch <= kWeighedSequences;
+  if (weigh) {
+    bool good = p.cu_num_k_block[0] == 0 && p.cu_num_k_block[p.batch] == p.nkb;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int s = i * 64 + lane;
+      qlen[i] = klen[i] = n[i] = 0;
+      first[i] = p.nkb;
+      if (s < p.batch) {
+        qlen[i] = p.cu_q[s + 1] - p.cu_q[s];
+        klen[i] = p.cu_k[s + 1] - p.cu_k[s];
+        first[i] = p.cu_num_k_block[s];
+        n[i] = p.cu_num_k_block[s + 1] - first[i];
+        good = good && qlen[i] >= 0 && klen[i] >= 0 && n[i] == (int)(((int64_t)klen[i] + p.kbs - 1) / p.kbs);
+      }
+    }
+    weigh = __ballot(!good) == 0;
   }
-  if (!good) return kb;
-  const int j = kb - p.cu_num_k_block[b];
-  const int rows = qlen_of(b), weight = p.causal ? min(rows, klen_of(b) - j * p.kbs) : rows;
-  auto at_least = [&](int s, int w) {   // blocks of sequence s that w rows or more can see
-    const int klen = klen_of(s), n = p.cu_num_k_block[s + 1] - p.cu_num_k_block[s];
-    if (w <= 0) return n;
-    if (w > qlen_of(s)) return 0;
-    return !p.causal ? n : klen < w ? 0 : min(n, (klen - w) / p.kbs + 1);
-  };
-  int place = 0;
-  for (int s = 0; s < p.batch; ++s) place += s == b ? j : at_least(s, s < b ? weight : weight + 1);
-  return place;
+  if (!weigh) {
+    for (int kb = wave * 64 + lane; kb < p.nkb; kb += waves * 64) p.order_k[kb] = kb;
+    return;
+  }
+  for (int kb = wave; kb < p.nkb; kb += waves) {
+    int b = -1;   // the last sequence that starts at or before the block
+#pragma unroll
+    for (int i = 0; i < N; ++i) b += __builtin_popcountll(__ballot(first[i] <= kb));
+    int rows = 0, keys = 0, j = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (b >> 6 == i) {
+        rows = __builtin_amdgcn_readlane(qlen[i], b & 63);
+        keys = __builtin_amdgcn_readlane(klen[i], b & 63);
+        j = kb - __builtin_amdgcn_readlane(first[i], b & 63);
+      }
+    const int weight = p.causal ? min(rows, keys - j * p.kbs) : rows;
+    int before = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      if (i * 64 >= p.batch) break;
+      const int s = i * 64 + lane, w = s < b ? weight : weight + 1;   // blocks of sequence s that w rows or more can see
+      int c = n[i];
+      if (w > 0) c = w > qlen[i] ? 0 : !p.causal ? c : klen[i] < w ? 0 : min(c, (int)((unsigned)(klen[i] - w) / (unsigned)p.kbs) + 1);
+      before += s == b ? j : c;
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) before += __shfl_xor(before, off);
+    if (lane == 0) p.order_k[before] = kb;
+  }
 }
 // ORDER: the order of the items (see OrderRoom) is made, too.
 template <bool ORDER>
@@ -109,10 +140,8 @@ __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
     else order_note(p.room, g * p.nhead_k + hk, kept_keys, p.weight_shift);
   }
   }
-  if (ORDER && hk == 0 && p.order_k != nullptr) {
-    for (int kb = blockIdx.x * kThreads + threadIdx.x; kb < p.nkb; kb += gridDim.x * kThreads) p.order_k[k_block_place(p, kb)] = kb;
-  }
   if constexpr (ORDER) {
+    order_k_blocks(p, (int)(blockIdx.y * gridDim.x + blockIdx.x) * 4 + (int)(threadIdx.x >> 6), (int)(gridDim.y * gridDim.x) * 4, lane);
     __shared__ OrderLds lds;
     if (p.room != nullptr) order_arrive(p.room, p.order, p.nqb * p.nhead_k, p.nhead_k, gridDim.x * gridDim.y, lds);
   }
@@ -1049,13 +1078,14 @@ size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t 
 
 }  // extern "C"
 namespace {
-// weighted: the items' order is made by their weights (see OrderRoom), which only a run that is split over key blocks can do
-// without.  The k blocks' order is there in any case: a backward may follow on the workspace.
+constexpr long long kWeighedKeys = 384;   // keys of a sequence, on average, from which on items are weighed
+// weigh_items, weigh_k_blocks: the orders are made by weight.  Without, they are there, too (last q blocks first, k blocks in their
+// own order): a run or a backward may follow on the workspace.
 int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
                      const int32_t *q_block_to_batch, const int32_t *cu_num_q_block, const int32_t *cu_num_k_block,
                      void *workspace, size_t workspace_bytes, int32_t batch, int32_t nhead_k, int32_t num_q_block,
                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size, int32_t causal,
-                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream, bool weighted) {
+                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream, bool weigh_items, bool weigh_k_blocks) {
   g_err[0] = 0;
   if (batch < 0 || num_q_block < 0 || num_k_block < 0 || total_q < 0 || total_k < 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
@@ -1087,6 +1117,7 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
   pp.batch = batch; pp.nkb = num_k_block; pp.total_q = total_q; pp.total_k = total_k;
   pp.nhead_k = nhead_k;
   pp.weight_shift = weight_shift((long long)num_k_block * k_block_size);
+  pp.weigh_k = weigh_k_blocks ? 1 : 0;
   pp.order = nullptr;
   pp.order_k = nullptr;
   pp.room = nullptr;
@@ -1095,7 +1126,12 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
     pp.order = (uint32_t *)((char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
     pp.order_k = (int32_t *)((char *)pp.order + order_bytes(nhead_k, num_q_block, num_k_block));
     // (a captured launch may be replayed on any stream, while the room belongs to this one)
-    if (weighted && !is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
+    // Counting and sorting takes 3 to 5 us, and gives what unequal items leave of a launch's end: nothing where the device has no
+    // second round of them, and too little where they are a few tiles long (250 x 20 .. 128 tokens, 16 / 4 heads of 64: 39.4 ->
+    // 44.6 us with the order, 2 x 700 tokens, 8 heads, in training 51.8 -> 55.0; 24 x 100 .. 900 in training 134 -> 114).
+    const long long keys = std::min<long long>(total_k, (long long)num_k_block * k_block_size);
+    weigh_items = weigh_items && (long long)nhead_k * num_q_block >= device_cus() && keys >= kWeighedKeys * batch;
+    if (weigh_items && !is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
     hipLaunchKernelGGL((hbsa_prep_kernel<true>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
   } else {
     hipLaunchKernelGGL((hbsa_prep_kernel<false>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
@@ -1114,7 +1150,7 @@ int hbsa_fwd_prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, c
                      int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream) {
   return prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block, workspace,
                  workspace_bytes, batch, nhead_k, num_q_block, num_k_block, q_block_size, k_block_size,
-                 causal, total_q, total_k, mask_strides, stream, true);
+                 causal, total_q, total_k, mask_strides, stream, true, true);
 }
 
 int hbsa_fwd_run(const void *q, const void *k, const void *v, void *out, void *workspace, size_t workspace_bytes,
@@ -1321,9 +1357,11 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   std::memset(&shape, 0, sizeof(shape));
   fill_shape(shape, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
   const bool split = shape.split > 1 && workspace_bytes >= need + split_bytes(shape.split, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
+  // Of the orders only what this call's own launch takes (see launch_fwd_nw) is worth its time: 3 us for the items' weights.
+  const long long places = (long long)device_cus() * (shape.nw == 8 || headdim > 192 ? 1 : 2), items = (long long)nhead_k * num_q_block * shape.nsub;
   int rc = prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block, workspace, workspace_bytes,
                    batch, nhead_k, num_q_block, num_k_block, q_block_size, k_block_size, causal, total_q, total_k, strides + 8, stream,
-                   !split);
+                   !split && !f32_exact && items > places && items <= 2ll * kStaticShare * places, false);
   if (rc != 0) return rc;
   return hbsa_fwd_run(q, k, v, out, workspace, workspace_bytes, dtype, total_q, total_k, nhead_q, nhead_k, headdim,
                       num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, strides, stream);

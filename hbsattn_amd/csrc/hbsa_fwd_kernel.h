@@ -40,11 +40,6 @@ namespace hbsa {
 // --------------------------------------------------------------------------------------
 constexpr int kListCap = 1024;   // tile entries per list; longer items are expanded in chunks
 constexpr int kGroupCap = 2 * kListCap;   // GROUPED: 16-bit entries of a list, one per 16 keys
-// Up to this many items per resident workgroup are handed out without the per-XCD work queues, in a fixed order
-// (see claim() in the kernel).  Measured against the queues: 8 x 512 tokens 71 -> 45 us, 8 x 1024 113 -> 99,
-// 8 x 2048 causal 200 -> 189, C5 0.33 -> 0.245 ms; at sixteen per workgroup 8 x 4096 tokens lose 5 % and at 64
-// C2 and C3 lose 5-8 % (the queues keep one head's K/V in one XCD's L2).
-constexpr int kStaticShare = 8;
 // Bytes of the one-launch form's staging area for one row of block_mask bytes (2048 blocks and the alignment slack)
 constexpr int kMaskWindow = 2048;
 constexpr int kMaskStage = kMaskWindow + 256;

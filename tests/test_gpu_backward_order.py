@@ -19,6 +19,10 @@ CASES = [
     ([200, 333], [1000, 333], 32, 32, 64, 128, 96, False),
     ([90, 260], [260, 90], 36, 36, 32, 16, 16, True),
     ([129, 400, 64], [129, 400, 64], 16, 8, 128, 64, 64, True),
+    # sequences of two rounds of a wavefront's lanes, the last of those that are ordered (256), one more; empty ones among them
+    ([i % 40 for i in range(65)], [i % 50 for i in range(65)], 4, 4, 64, 16, 16, True),
+    ([i % 23 for i in range(256)], [i % 37 for i in range(256)], 4, 2, 32, 16, 16, True),
+    ([1 + i % 23 for i in range(257)], [1 + i % 37 for i in range(257)], 2, 2, 32, 16, 16, False),
 ]
 
 

@@ -24,6 +24,7 @@ SPECS = [
     dict(q_lens=[2048, 2049], k_lens=[2048, 2049], hq=16, hk=16, d=64, qbs=16, kbs=128, keep=0.3, causal=True),          # 4112
     dict(q_lens=[900, 1300], k_lens=[900, 1300], hq=16, hk=16, d=128, qbs=64, kbs=64, keep=0.0, causal=True),
     dict(q_lens=[3000], k_lens=[90000], hq=16, hk=16, d=64, qbs=64, kbs=64, keep=0.9, causal=False),
+    dict(q_lens=[3300, 2025, 0, 498, 3205], k_lens=[3300, 2025, 77, 498, 3205], hq=16, hk=4, d=64, qbs=64, kbs=64, keep=0.4, causal=True),
 ]
 
 
@@ -54,7 +55,7 @@ def test_a_captured_preparation_takes_the_order_without_weights_and_can_be_repla
 
 
 def test_two_streams_prepare_at_once(two_launches):
-    a, b = (make_problem(seed=33 + i, diag=True, scale=None, **SPECS[i]) for i in range(2))
+    a, b = (make_problem(seed=33 + i, diag=True, scale=None, **SPECS[i]) for i in (2, 6))   # both weighed, several rounds of items
     want = [HBSAttention(*a.args()), HBSAttention(*b.args())]
     torch.cuda.synchronize()
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
