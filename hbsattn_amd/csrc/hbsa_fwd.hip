@@ -648,14 +648,19 @@ inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_bloc
 // 181 / 183 / 192 us; head dim 128, a fifth kept, 16 / 48 keys 420 / 209 -> 146 / 155; head dim 192 and 48 keys 273 -> 236; head dim
 // 256 1206 / 557 -> 391 / 405.  Whatever is kept the groups cost more address work a tile, and their list is longer: 464 and 976 keys
 // were even (239 -> 227, 261 -> 243, as much as runs gave), 2032 lost (151 -> 155 with a twentieth kept).
+// An item's first tile is under way 0.2 to 0.8 us later, though, which is what shows where there is little to be saved: a kept block
+// leaves `empty` keys of its tiles, and a sequence has no more blocks than there are to each that ends in part of one (there are at
+// least that many sequences).  Up to two tiles saved a sequence: 2 x 12 .. 40 tokens, 8 heads of 32, 48-key blocks 8.0 (runs) and 8.3 us;
+// 9 x 135 .. 272, 2 heads of 128, 112-key blocks 14.4 and 15.0; above, 8 x 40 .. 70, 8 / 2 heads of 64, 16-key blocks 10.0 -> 9.4.
 // A group is numbered in 16 bits.  The rule is the same for the one-launch and the prepared form, so they compute the same bits.
 constexpr int kMostGroupedBlock = 256;
-inline bool fwd_grouped(int num_k_block, int k_block_size) {
-  return k_block_size % kTileKeys != 0 && k_block_size < kMostGroupedBlock && (long long)num_k_block * k_block_size <= 16 * 65535ll;
+inline bool fwd_grouped(int total_k, int num_k_block, int k_block_size) {
+  const long long empty = (kTileKeys - k_block_size % kTileKeys) % kTileKeys, parts = std::max<long long>(1, num_k_block - total_k / k_block_size);
+  return num_k_block * empty > 2 * kTileKeys * parts && k_block_size % kTileKeys != 0 && k_block_size < kMostGroupedBlock && (long long)num_k_block * k_block_size <= 16 * 65535ll;
 }
 
 // The fields of FwdParams that follow from the call's shape and softmax_scale alone.
-void fill_shape(FwdParams &fp, int total_q, int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size,
+void fill_shape(FwdParams &fp, int total_q, int total_k, int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size,
                 int k_block_size, int causal, float softmax_scale, bool f32_exact, bool may_pack = false, bool cols = false) {
   fp.nhead_k = nhead_k;
   fp.nqb = num_q_block; fp.ratio = nhead_q / nhead_k; fp.kbs = k_block_size; fp.wpr = words_per_row(num_k_block);
@@ -666,7 +671,7 @@ void fill_shape(FwdParams &fp, int total_q, int nhead_q, int nhead_k, int headdi
   const FwdSplit split = fwd_split(slots, headdim, f32_exact, (long long)nhead_k * num_q_block, num_k_block, k_block_size,
                                    (long long)num_q_block * q_block_size, total_q);
   fp.nw = split.nw;
-  fp.grouped = fwd_grouped(num_k_block, k_block_size) ? 1 : 0;
+  fp.grouped = fwd_grouped(total_k, num_k_block, k_block_size) ? 1 : 0;
   fp.split = split.parts;
   fp.ncol = headdim / 8;
   fp.max_parts = 1;
@@ -841,7 +846,7 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   FwdParams fp;
   std::memset(&fp, 0, sizeof(fp));
   const bool cols = headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256;
-  fill_shape(fp, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, false,
+  fill_shape(fp, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, false,
              true, cols);
   const long long items = (long long)nhead_k * num_q_block * fp.nsub;
   Sched *sched = onepass_record(dtype, batch, total_k, headdim, k_block_size, strides[10], items, fp.split, st);
@@ -1229,7 +1234,7 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
     fp.q_s = strides[0] * es; fp.q_h = strides[1] * es; fp.k_s = strides[2] * es; fp.k_h = strides[3] * es;
     fp.v_s = strides[4] * es; fp.v_h = strides[5] * es; fp.o_s = strides[6] * es; fp.o_h = strides[7] * es;
   }
-  fill_shape(fp, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale,
+  fill_shape(fp, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale,
              f32_exact);
   const long long items = (long long)nhead_k * num_q_block * fp.nsub;
   if (items > 0x7fffffffLL) return fail(HBSA_ERR_UNSUPPORTED, "too many work items (%lld)", items);
@@ -1336,7 +1341,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
     if (roomy && ((uintptr_t)workspace & 255)) return fail(HBSA_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");
     FwdParams fp;
     std::memset(&fp, 0, sizeof(fp));
-    fill_shape(fp, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
+    fill_shape(fp, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
     const long long items = (long long)nhead_k * num_q_block * fp.nsub;
     if (items > 0x7fffffffLL) return fail(HBSA_ERR_UNSUPPORTED, "too many work items (%lld)", items);
     const int64_t es = f32_exact ? 4 : 2;
@@ -1355,7 +1360,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   }
   FwdParams shape;
   std::memset(&shape, 0, sizeof(shape));
-  fill_shape(shape, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
+  fill_shape(shape, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, f32_exact);
   const bool split = shape.split > 1 && workspace_bytes >= need + split_bytes(shape.split, total_q, nhead_q, nhead_k, headdim, num_q_block, num_k_block);
   // Of the orders only what this call's own launch takes (see launch_fwd_nw) is worth its time: 3 us for the items' weights.
   const long long places = (long long)device_cus() * (shape.nw == 8 || headdim > 192 ? 1 : 2), items = (long long)nhead_k * num_q_block * shape.nsub;

@@ -25,8 +25,9 @@ def check(w, what, same_bits=True):
 @pytest.mark.parametrize("kbs", [16, 48, 80, 240, 272])   # 256 and more keep to runs of consecutive keys
 @pytest.mark.parametrize("d", [32, 40, 64, 96, 128, 160, 192, 224, 256])
 def test_blocks_and_tails_of_every_remainder(d, kbs):
-    # key lengths of 1, 15, 16, 17, 63, 64, 65 past whole blocks, more and fewer keys than queries, whole and missing last groups
-    for causal, gqa, k_lens in ((True, 1, [kbs + 1, 2 * kbs + 15, 3 * kbs + 16, 700]), (False, 4, [17, 4 * kbs + 63, 64, 65 + kbs])):
+    # key lengths of 1, 15, 16, 17, 63, 64, 65 past whole blocks, more and fewer keys than queries, whole and missing last groups;
+    # the last sequence is long, since groups are for sequences of several blocks
+    for causal, gqa, k_lens in ((True, 1, [kbs + 1, 2 * kbs + 15, 3 * kbs + 16, 40 * kbs + 700]), (False, 4, [17, 4 * kbs + 63, 64, 65 + 40 * kbs])):
         w = make_problem(seed=kbs + d, q_lens=[130, 77, 300, 64], k_lens=k_lens, hq=4, hk=4 // gqa, d=d, qbs=64, kbs=kbs, keep=0.6,
                          diag=True, causal=causal, scale=None)
         check(w, f"d={d} kbs={kbs} causal={causal}")
@@ -37,6 +38,13 @@ def test_items_longer_than_a_list(d):
     # about 38000 kept keys an item, a list holds 32768; more items than are split over their key blocks
     w = make_problem(seed=5, q_lens=[350], k_lens=[40003], hq=16, hk=16, d=d, qbs=16, kbs=48, keep=0.95, diag=False, causal=False, scale=None)
     check(w, f"d={d}", same_bits=d in (64, 256))   # (padded head dims may be cut into parts differently)
+
+
+@pytest.mark.parametrize("k_lens", [[8 * 48 + 1], [8 * 48 - 48 + 1], [48] * 8, [49] * 8], ids=str)
+def test_sequences_on_both_sides_of_the_line(k_lens):
+    # nine blocks of one sequence can save more than two tiles, eight cannot; eight sequences of a block each are not told from one
+    w = make_problem(seed=7, q_lens=[40] * len(k_lens), k_lens=k_lens, hq=4, hk=2, d=64, qbs=32, kbs=48, keep=0.7, diag=True, causal=True, scale=None)
+    check(w, str(k_lens))
 
 
 @pytest.mark.parametrize("blocks", [65535, 65536], ids=lambda n: f"{n}blocks")
