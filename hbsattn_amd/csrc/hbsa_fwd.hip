@@ -650,13 +650,14 @@ inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_bloc
 // were even (239 -> 227, 261 -> 243, as much as runs gave), 2032 lost (151 -> 155 with a twentieth kept).
 // An item's first tile is under way 0.2 to 0.8 us later, though, which is what shows where there is little to be saved: a kept block
 // leaves `empty` keys of its tiles, and a sequence has no more blocks than there are to each that ends in part of one (there are at
-// least that many sequences).  Up to two tiles saved a sequence: 2 x 12 .. 40 tokens, 8 heads of 32, 48-key blocks 8.0 (runs) and 8.3 us;
-// 9 x 135 .. 272, 2 heads of 128, 112-key blocks 14.4 and 15.0; above, 8 x 40 .. 70, 8 / 2 heads of 64, 16-key blocks 10.0 -> 9.4.
+// least that many sequences).  Up to four tiles saved a sequence, runs and groups: 13 x 92 .. 176 tokens, 8 heads of 128, 80-key blocks
+// 11.9 and 12.7 us; 4 x 200 .. 400, 8 of 64, 96-key blocks 13.2 and 13.9, but 48-key blocks 14.4 and 13.8; 9 x 135 .. 272, 2 of 128, 112-key
+// blocks 14.4 and 15.0.  Above: 8 x 40 .. 70, 8 / 2 heads of 64, 16-key blocks 10.2 and 9.2; 8 x 300 .. 500, 16 of 128, 80-key blocks 33.8 and 32.4.
 // A group is numbered in 16 bits.  The rule is the same for the one-launch and the prepared form, so they compute the same bits.
 constexpr int kMostGroupedBlock = 256;
 inline bool fwd_grouped(int total_k, int num_k_block, int k_block_size) {
   const long long empty = (kTileKeys - k_block_size % kTileKeys) % kTileKeys, parts = std::max<long long>(1, num_k_block - total_k / k_block_size);
-  return num_k_block * empty > 2 * kTileKeys * parts && k_block_size % kTileKeys != 0 && k_block_size < kMostGroupedBlock && (long long)num_k_block * k_block_size <= 16 * 65535ll;
+  return num_k_block * empty > 4 * kTileKeys * parts && k_block_size % kTileKeys != 0 && k_block_size < kMostGroupedBlock && (long long)num_k_block * k_block_size <= 16 * 65535ll;
 }
 
 // The fields of FwdParams that follow from the call's shape and softmax_scale alone.

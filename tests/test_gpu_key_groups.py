@@ -27,7 +27,7 @@ def check(w, what, same_bits=True):
 def test_blocks_and_tails_of_every_remainder(d, kbs):
     # key lengths of 1, 15, 16, 17, 63, 64, 65 past whole blocks, more and fewer keys than queries, whole and missing last groups;
     # the last sequence is long, since groups are for sequences of several blocks
-    for causal, gqa, k_lens in ((True, 1, [kbs + 1, 2 * kbs + 15, 3 * kbs + 16, 40 * kbs + 700]), (False, 4, [17, 4 * kbs + 63, 64, 65 + 40 * kbs])):
+    for causal, gqa, k_lens in ((True, 1, [kbs + 1, 2 * kbs + 15, 3 * kbs + 16, 60 * kbs + 700]), (False, 4, [17, 4 * kbs + 63, 64, 65 + 60 * kbs])):
         w = make_problem(seed=kbs + d, q_lens=[130, 77, 300, 64], k_lens=k_lens, hq=4, hk=4 // gqa, d=d, qbs=64, kbs=kbs, keep=0.6,
                          diag=True, causal=causal, scale=None)
         check(w, f"d={d} kbs={kbs} causal={causal}")
@@ -40,9 +40,9 @@ def test_items_longer_than_a_list(d):
     check(w, f"d={d}", same_bits=d in (64, 256))   # (padded head dims may be cut into parts differently)
 
 
-@pytest.mark.parametrize("k_lens", [[8 * 48 + 1], [8 * 48 - 48 + 1], [48] * 8, [49] * 8], ids=str)
+@pytest.mark.parametrize("k_lens", [[16 * 48 + 1], [16 * 48 - 48 + 1], [48] * 17, [49] * 8], ids=str)
 def test_sequences_on_both_sides_of_the_line(k_lens):
-    # nine blocks of one sequence can save more than two tiles, eight cannot; eight sequences of a block each are not told from one
+    # 17 blocks that can be one sequence's save more than four tiles, 16 do not; sequences that end in part of a block count as such
     w = make_problem(seed=7, q_lens=[40] * len(k_lens), k_lens=k_lens, hq=4, hk=2, d=64, qbs=32, kbs=48, keep=0.7, diag=True, causal=True, scale=None)
     check(w, str(k_lens))
 
