@@ -687,7 +687,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   const int kb = p.order_k != nullptr ? p.order_k[kb_at] : kb_at;
 
   const BwdSequence seq(p, kb, lane);
-  if (seq.qb0 < 0 || seq.qb0 >= p.nqb) return;
+  if (seq.qb0 < 0 || seq.qb0 > p.nqb) return;   // (== nqb: sequences without queries at the batch's end, whose keys get zeros)
   // asked for together: the sequence's record, the mask column's first 64 words, the resident operands
   const uint32_t record = bwd_first_record(p, seq, lane);
   const int kbl = kb - seq.kb0;                      // in-sequence index of the k block
@@ -994,7 +994,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   const int kb = p.order_k != nullptr ? p.order_k[kb_at] : kb_at;
 
   const BwdSequence seq(p, kb, lane);
-  if (seq.qb0 < 0 || seq.qb0 >= p.nqb) return;
+  if (seq.qb0 < 0 || seq.qb0 > p.nqb) return;   // (== nqb: sequences without queries at the batch's end, whose keys get zeros)
   // Asked for together: the sequence's record, the mask column's first 64 words, the resident operand.  With one workgroup
   // per CU nothing covers the loads a workgroup begins with, and it has some eight tiles where 8K sequences keep a tenth.
   const uint32_t record = bwd_first_record(p, seq, lane);
