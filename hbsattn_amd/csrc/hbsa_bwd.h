@@ -199,7 +199,7 @@ __device__ __forceinline__ void bwd_store_rows(char *row_ptr, const f32x16 *acc,
 // The sequence a k block belongs to: what the dK/dV kernels need of it from the caller's arrays.  All three arrays are asked
 // for at once, a sequence per lane (one wait in place of one per sequence passed and two more behind it).
 struct BwdSequence {
-  int k0, k1, kb0, qb0, qb1;   // keys [k0, k1), first k block, q blocks [qb0, qb1)
+  int k0, k1, kb0, qb0, qb1;   // keys [k0, k1), first k block, q blocks [qb0, qb1), those that there are records and bit rows of
   __device__ __forceinline__ BwdSequence(const BwdParams &p, int kb, int lane) {
     if (p.batch < 64) {
       const int i = min(lane, p.batch);
@@ -221,6 +221,7 @@ struct BwdSequence {
       qb0 = p.cu_num_q_block[b];
       qb1 = p.cu_num_q_block[b + 1];
     }
+    qb1 = min(qb1, p.nqb);
   }
   // the sequence's keys lie inside the tensors, and the k block inside the sequence's numbering
   __device__ __forceinline__ bool fits(const BwdParams &p, int kb) const { return k0 >= 0 && k1 >= k0 && k1 <= p.total_k && kb >= kb0; }
@@ -228,6 +229,12 @@ struct BwdSequence {
 // The record of the sequence's first q block, a word per lane (nullptr words: no q blocks).
 __device__ __forceinline__ uint32_t bwd_first_record(const BwdParams &p, const BwdSequence &s, int lane) {
   return s.qb0 < s.qb1 && lane < 12 ? ((const uint32_t *)(p.info + s.qb0))[lane] : 0u;
+}
+// Whether that record is of the sequence's first q block and not flagged by the pre-pass.  With the keys and the position it
+// states, all rows of the sequence as the kernels count them lie inside the tensors (the pre-pass has checked the record's own).
+__device__ __forceinline__ bool bwd_record_holds(const BwdSequence &s, uint32_t record) {
+  auto word = [&](int i) { return __builtin_amdgcn_readlane((int)record, i); };   // 2: key_begin, 3: klen, 4: q_pos, 9: flags
+  return word(9) == 0 && word(2) == s.k0 && word(3) == s.k1 - s.k0 && word(4) == 0;
 }
 // A sequence the pre-pass found not to fit the tensors (flagged q block records, no bit rows) takes no part: its keys get zero
 // gradients where they lie inside dk and dv.
@@ -740,7 +747,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   QBlockInfo inf = {};
   int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
   if (qb_begin < qb_end) {
-    if (__builtin_amdgcn_readlane((int)record, 9) != 0) {   // flags
+    if (!bwd_record_holds(seq, record)) {
       bwd_zero_keys<D>(p, seq, kb, sub, hk);
       return;
     }
@@ -788,6 +795,10 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       inf.q_pos = (qb - qb_begin) * p.qbs;
       inf.row_begin = seq_row0 + inf.q_pos;
       inf.rows = min(p.qbs, seq_qlen - inf.q_pos);
+      if (inf.rows <= 0) {   // more q blocks than the sequence has rows for: none is written into such a block's bit row
+        qb = qb_begin - 1;
+        continue;
+      }
       r = PARTS && qb == qb_first ? r_first : 0;
       qoff = -64;   // the step above moves to the block's first tile
     }
@@ -1041,7 +1052,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   QBlockInfo inf = {};
   int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
   if (qb_begin < qb_end) {
-    if (__builtin_amdgcn_readlane((int)record, 9) != 0) {   // flags
+    if (!bwd_record_holds(seq, record)) {
       bwd_zero_keys<D>(p, seq, kb, sub, hk);
       return;
     }
@@ -1092,6 +1103,10 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       inf.q_pos = (qb - qb_begin) * p.qbs;
       inf.row_begin = seq_row0 + inf.q_pos;
       inf.rows = min(p.qbs, seq_qlen - inf.q_pos);
+      if (inf.rows <= 0) {   // more q blocks than the sequence has rows for: none is written into such a block's bit row
+        qb = qb_begin - 1;
+        continue;
+      }
       r = 0;
       if constexpr (PARTS) {
         if (qb == __builtin_amdgcn_readfirstlane(part_s->qb_first)) r = __builtin_amdgcn_readfirstlane(part_s->r_first);
