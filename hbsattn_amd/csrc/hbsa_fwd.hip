@@ -24,6 +24,8 @@
 //   O^T[d, query] += V^T[d, key] . P^T[key, query]  A = V^T (LDS, ds_read_b64_tr_b16)
 //                                                  B = P^T = the S^T accumulator
 //                                                      converted in place, no shuffle.
+#include <atomic>
+
 #include "hbsa_common.h"
 
 namespace hbsa {
@@ -768,8 +770,8 @@ int static_scratch(void **ptr) {
   return 0;
 }
 
-// The launch record and the arrival counters of `stream` on the current device; nullptr when there are none to give (no
-// device, the lookup failed, or kStreamSlots other streams of this device have taken them).
+// The launch record, the arrival counters and the room for an order of `stream` on the current device; nullptr when there are
+// none to give (no device, the lookup failed, kStreamSlots other streams of this device have taken them).
 struct StreamSlots {
   char *base;
   uint32_t *arrivals;
@@ -778,7 +780,15 @@ struct StreamSlots {
   hipStream_t stream[kStreamSlots];
 };
 StreamSlots g_stream_slots[kMaxDevices] = {};
+// hipStreamPerThread is one handle for every thread's own stream: two threads' launches would share what it is given.  An odd
+// number of the thread's own in its place, which no stream's address is and no later thread gets.
+hipStream_t this_threads_stream() {
+  static std::atomic<uintptr_t> threads{0x1000};
+  static thread_local const uintptr_t mine = threads.fetch_add(2) + 1;
+  return (hipStream_t)mine;
+}
 Sched *stream_sched_of(hipStream_t stream, uint32_t **arrivals = nullptr, OrderRoom **order = nullptr) {
+  if (stream == hipStreamPerThread) stream = this_threads_stream();
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
@@ -801,8 +811,7 @@ Sched *stream_sched_of(hipStream_t stream, uint32_t **arrivals = nullptr, OrderR
     if (t.used == kStreamSlots) return nullptr;
     t.stream[t.used++] = stream;
   }
-  // (hipStreamPerThread is one handle for every thread's own stream: two of them would share the room)
-  if (order != nullptr) *order = stream == hipStreamPerThread ? nullptr : t.order + i;
+  if (order != nullptr) *order = t.order + i;
   if (arrivals != nullptr) *arrivals = t.arrivals + (size_t)i * kMaxPartItems;
   return (Sched *)(t.base + (size_t)i * sizeof(Sched));
 }
