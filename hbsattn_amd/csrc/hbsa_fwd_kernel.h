@@ -1178,13 +1178,18 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           // Whether the reference was good enough for a half, and if not (rarely, or with a NaN) a better one.  No maximum
           // is formed: the exponentials are taken against the reference of the halves before, and only a sum (which
           // has to be formed anyway) above 2^kLazyRescaleLog2 can hide an exponential above it.  Then the maximum is looked
-          // for, the reference moved, O and l rescaled and the exponentials formed again.
+          // for, the reference of the rows that ask for it moved there, O and l rescaled and the exponentials formed again.
           // In place of a maximum of every half (eight v_max3 in a chain, an exchange between half wavefronts, a rescaled P),
-          // which the exponentials had to wait for.
+          // which the exponentials had to wait for.  (Sixteen exponentials reach that sum at 2^4 each, so the reference moves
+          // whenever this is entered: left where no exponential alone exceeds 2^8, a plateau of later scores that lie 2^4 to 2^8
+          // above the first tile's comes back here for every half: scores of deviation 0.3 with the first key block's 4 below the
+          // rest, 8 x 8192 tokens, 32 heads of 128, 1112 -> 929 us (918 without the step), 4 x 4096, 16 heads of 64, 164 -> 114
+          // (112).  A row whose own sums did not ask keeps its reference, so its bits do not depend on its neighbours.)
           auto settle_half = [&](const f32x16 &sh, float sum, short8v &p_lo, short8v &p_hi) {
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= kMostSum)) != 0, 0)) {
+            const uint64_t asked = __builtin_amdgcn_ballot_w64(!(sum <= kMostSum));
+            if (__builtin_expect(asked != 0, 0)) {
               const float mx = half_rowmax(sh);
-              const bool grow = mx > m_ref + kLazyRescaleLog2;
+              const bool grow = (((uint32_t)asked | (uint32_t)(asked >> 32)) >> l32 & 1u) != 0 && mx > m_ref;
               const float m_new = grow ? mx : m_ref;
               const float alpha = grow ? __builtin_amdgcn_exp2f(m_ref - m_new) : 1.f;
               l_run *= alpha;

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from hbsattn_amd import HBSAttention
+from hbsattn_amd import HBSAttention, set_onepass
 from hbsattn_amd.workloads import make_problem
 from helpers import assert_close_to_oracle, oracle_for
 
@@ -42,3 +42,56 @@ def test_rows_whose_first_tiles_are_hidden(d):
     out = HBSAttention(*w.args())
     assert_close_to_oracle(out, oracle_for(w), f"d={d}")
     assert (out[:50] == 0).all()   # q_len - k_len rows that see nothing
+
+
+def plateau(w, deviation, below):
+    """Scores of the given deviation, those of every sequence's first key block `below` natural-log units under the rest's;
+    every row's list begins with that block."""
+    d, kbs, block = w.q.shape[2], w.k_block_size, 0
+    w.q *= deviation
+    w.q[:, :, 0] = 4.
+    w.k[:, :, 0] = 0.
+    for b in range(len(w.cu_k) - 1):
+        a, z = int(w.cu_k[b]), int(w.cu_k[b + 1])
+        w.k[a:min(z, a + kbs), :, 0] = -below / (4. * d ** -0.5)
+        w.block_mask[:, :, block] = True
+        block += -(-(z - a) // kbs)
+    return w
+
+
+# a deviation of 0.3: all rows' references move in the same half tile; 1: every row's in another one, some rows' never
+@pytest.mark.parametrize("deviation,below", [(0.3, 4.), (1., 4.)])
+@pytest.mark.parametrize("d,kbs", [(32, 64), (64, 48), (128, 64), (128, 128), (256, 64)])
+def test_later_scores_a_little_above_the_first(d, kbs, deviation, below):
+    w = plateau(make_problem(seed=8, q_lens=[200, 333], k_lens=[900, 1400], hq=8, hk=2, d=d, qbs=80, kbs=kbs, keep=0.6, diag=True, causal=True,
+                             scale=None), deviation, below)
+    outs = []
+    for one in (True, False):   # rows packed with other rows' neighbours, and not: the same bits
+        previous = set_onepass(one)
+        try:
+            outs.append(HBSAttention(*w.args()))
+        finally:
+            set_onepass(previous)
+    assert_close_to_oracle(outs[0], oracle_for(w), f"d={d} kbs={kbs} deviation {deviation} {below} below")
+    assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_a_reference_that_lags_a_little_is_moved_once(d):
+    # Scores 2^4 to 2^8 above the first tile's: where the reference stays behind them, every half tile is worked on twice (1.47 times
+    # the time).  Moved once it is a half tile in sixty: 1.02.  The least of ten runs of each, taken in turn.
+    make = lambda below: plateau(make_problem(seed=9, q_lens=[4096] * 4, k_lens=[4096] * 4, hq=16, hk=16, d=d, qbs=64, kbs=64, keep=0.3,
+                                              diag=True, causal=True, scale=None, device="cuda", gen_device="device"), 0.3, below).args()
+    calls = [make(0.), make(4.)]
+    times = [[], []]
+    for _ in range(10):
+        for i, args in enumerate(calls):
+            HBSAttention(*args)
+            a, z = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                HBSAttention(*args)
+            z.record()
+            z.synchronize()
+            times[i].append(a.elapsed_time(z))
+    assert min(times[1]) <= 1.12 * min(times[0]), f"{min(times[1]) * 50:.1f} us against {min(times[0]) * 50:.1f}"
