@@ -212,9 +212,16 @@ struct BwdSequence {
       kb0 = __builtin_amdgcn_readlane(nkb, b);
       qb0 = __builtin_amdgcn_readlane(nqb, b);
       qb1 = __builtin_amdgcn_readlane(nqb, b + 1);
-    } else {
+    } else {   // 64 sequences at a time (dK/dV of 250 x 20 .. 128 tokens, 4 heads of 128: one at a time 127 us, so 60)
       int b = 0;
-      while (b + 1 < p.batch && p.cu_num_k_block[b + 1] <= kb) ++b;
+      for (;; b += 64) {
+        const int i = b + 1 + lane;
+        const uint64_t starts = __builtin_amdgcn_ballot_w64(i < p.batch && p.cu_num_k_block[min(i, p.batch)] <= kb);
+        if (~starts != 0) {
+          b += __builtin_ctzll(~starts);
+          break;
+        }
+      }
       k0 = p.cu_k[b];
       k1 = p.cu_k[b + 1];
       kb0 = p.cu_num_k_block[b];

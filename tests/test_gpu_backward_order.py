@@ -19,7 +19,9 @@ CASES = [
     ([200, 333], [1000, 333], 32, 32, 64, 128, 96, False),
     ([90, 260], [260, 90], 36, 36, 32, 16, 16, True),
     ([129, 400, 64], [129, 400, 64], 16, 8, 128, 64, 64, True),
-    # sequences of two rounds of a wavefront's lanes, the last of those that are ordered (256), one more; empty ones among them
+    # sequences of one, two and more rounds of a wavefront's lanes, the last of those that are ordered (256), one more; empty ones among them
+    ([i % 40 for i in range(63)], [i % 50 for i in range(63)], 4, 4, 64, 16, 16, True),
+    ([i % 40 for i in range(64)], [1 + i % 50 for i in range(64)], 4, 4, 64, 16, 16, False),
     ([i % 40 for i in range(65)], [i % 50 for i in range(65)], 4, 4, 64, 16, 16, True),
     ([i % 23 for i in range(256)], [i % 37 for i in range(256)], 4, 2, 32, 16, 16, True),
     ([1 + i % 23 for i in range(257)], [1 + i % 37 for i in range(257)], 2, 2, 32, 16, 16, False),
@@ -80,3 +82,33 @@ def test_gradients_on_the_workspace_of_a_forward_split_over_key_blocks():
     got = hbsa_backward(qd, kd, vd, out, dod, lse, prepared, None)
     for x, ref, name in zip(got, hbsa_oracle_grads(q, k, v, do, cu_q, cu_k, mask, qbs, kbs, causal, None), ("dq", "dk", "dv")):
         _check(x, ref, name)
+
+
+def test_a_backward_takes_no_longer_for_being_of_many_sequences():
+    # equal work in 60 sequences of 256 tokens and in 240 of 64: what a dK/dV workgroup does to find its sequence must not show
+    # (one sequence after the other, behind the order of the k blocks: 67 and 101 us; 64 at a time 67 and 70)
+    times = []
+    for n, length in ((60, 256), (240, 64)):
+        q, k, v, do, cu_q, cu_k, cq, ck, mask = _problem(14, [length] * n, [length] * n, 4, 4, 128, 64, 64, 0.0, torch.bfloat16)
+        for i in range(mask.shape[1]):
+            mask[:, i, i] = True
+        qd, kd, vd, dod = (t.cuda() for t in (q, k, v, do))
+        (nq, _, q2b, cu_nq), (nk, _, _, cu_nk) = calculate_blocks(cq, 64), calculate_blocks(ck, 64)
+        prepared = hbsa_prepare(cq, ck, mask.cuda(), 64, 64, True, nq, q2b, cu_nq, nk, cu_nk)
+        out, lse = hbsa_run(qd, kd, vd, prepared, None, return_lse=True)
+        graph = torch.cuda.CUDAGraph()
+        hbsa_backward(qd, kd, vd, out, dod, lse, prepared, None)
+        with torch.cuda.graph(graph):
+            hbsa_backward(qd, kd, vd, out, dod, lse, prepared, None)
+        best = float("inf")
+        for _ in range(10):
+            a, z = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(10):
+                graph.replay()
+            z.record()
+            z.synchronize()
+            best = min(best, a.elapsed_time(z) * 100)
+        times.append(best)
+    print("us of 60 and of 240 sequences", times)
+    assert times[1] <= 1.3 * times[0], times
