@@ -1,4 +1,4 @@
-"""dK/dV items taken in the order of the rows that can see them, and the form of the kernel for many of them."""
+"""dK/dV items taken in the order of the rows that can see them, and the form of the head dim 64 kernel for many of them."""
 import ctypes
 
 import pytest
@@ -7,11 +7,11 @@ import torch
 from hbsattn_amd import _lib, calculate_blocks
 from hbsattn_amd.interface import PreparedMask, hbsa_backward, hbsa_prepare, hbsa_run
 from oracle.grads import hbsa_oracle_grads
-from test_gpu_backward import _check, _problem
+from test_gpu_backward import _check, _gpu_grads, _problem
 
 pytestmark = pytest.mark.gpu
 
-# 512 items of two rounds and more on 256 CUs: 32 heads x 18 .. 40 k blocks; k blocks of one and two key slots, of a slot and a half
+# items of one to two rounds on 256 CUs, none cut into parts but in the last five; k blocks of one and two key slots, of a slot and a half
 CASES = [
     # q_lens, k_lens, hq, hk, d, qbs, kbs, causal
     ([70, 513, 0, 300], [70, 513, 90, 300], 32, 32, 64, 64, 32, True),      # an empty sequence; 31 blocks a head
@@ -112,3 +112,28 @@ def test_a_backward_takes_no_longer_for_being_of_many_sequences():
         times.append(best)
     print("us of 60 and of 240 sequences", times)
     assert times[1] <= 1.3 * times[0], times
+
+
+# The form for many items: more than 4.5 a CU at head dim 64, any number at 32.  Key blocks of up to four slots, a wavefront each: both
+# halves of a tile are one wavefront's.  Sequences with fewer and more queries than keys, last blocks of a few keys, several tiles of rows.
+MANY = [
+    ([300, 150, 700], [1400, 1300, 1390], 40, 40, 64, 64, 128, True),
+    ([300, 150, 700], [1400, 1300, 1390], 40, 40, 64, 128, 128, False),
+    ([200, 0, 900], [1000, 85, 1700], 36, 36, 64, 48, 80, True),
+    ([130, 333], [1601, 1630], 72, 36, 64, 80, 96, False),
+    ([90, 260, 500], [1600, 1600, 500], 40, 40, 64, 64, 64, True),
+    ([300, 150, 700], [1400, 1300, 1390], 40, 40, 32, 64, 128, True),
+    ([130, 333], [1601, 1630], 72, 36, 32, 80, 80, False),
+]
+
+
+@pytest.mark.parametrize("case", MANY, ids=[f"case{i}" for i in range(len(MANY))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_gradients_of_many_items(case, dtype):
+    q_lens, k_lens, hq, hk, d, qbs, kbs, causal = case
+    q, k, v, do, cu_q, cu_k, cq, ck, mask = _problem(13, q_lens, k_lens, hq, hk, d, qbs, kbs, 0.4, dtype)
+    assert 2 * mask.shape[2] * hk > 9 * torch.cuda.get_device_properties(0).multi_processor_count   # the rule for head dim 64
+    print(f"backward of many items {case} {dtype}", flush=True)
+    _, *got = _gpu_grads(q, k, v, do, cq, ck, mask, qbs, kbs, causal, None)
+    for x, ref, name in zip(got, hbsa_oracle_grads(q, k, v, do, cu_q, cu_k, mask, qbs, kbs, causal, None), ("dq", "dk", "dv")):
+        _check(x, ref, name)
