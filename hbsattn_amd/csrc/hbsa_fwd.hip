@@ -646,20 +646,34 @@ inline long long f32_items(int nhead_q, int nhead_k, int num_q_block, int q_bloc
 
 // Tiles of 16-key groups, for key block sizes that are no multiple of the tile: a tile of consecutive keys ends with its run of
 // kept blocks, and is then partly empty and masked.  The shorter the blocks, the more of that: 4 x 777 .. 5120 queries, 4100 ..
-// 8192 keys, 16 / 4 heads, half of the blocks kept, head dim 64, blocks of 16 / 48 / 112 / 208 keys 444 / 257 / 218 / 218 -> 177 /
-// 181 / 183 / 192 us; head dim 128, a fifth kept, 16 / 48 keys 420 / 209 -> 146 / 155; head dim 192 and 48 keys 273 -> 236; head dim
-// 256 1206 / 557 -> 391 / 405.  Whatever is kept the groups cost more address work a tile, and their list is longer: 464 and 976 keys
-// were even (239 -> 227, 261 -> 243, as much as runs gave), 2032 lost (151 -> 155 with a twentieth kept).
+// 8192 keys, 16 / 4 heads, half of the blocks kept, head dim 64, blocks of 16 / 48 / 112 keys 444 / 257 / 218 -> 177 / 181 / 183 us;
+// head dim 128, a fifth kept, 16 / 48 keys 420 / 209 -> 146 / 155; head dim 192 and 48 keys 273 -> 236; head dim 256 1206 / 557 ->
+// 391 / 405.  Whatever is kept the groups cost more address work a tile, and their list is longer: with little to be saved a tenth of the
+// time at head dim 128, a fifth at 96 and 256.  What is saved falls with the length of a run, so the largest block they are
+// for is the smaller the more a tile costs.  Groups against runs, per cent of the time, causal, a tenth / 0.3 / 0.6 kept, 3 x 2400 .. 5600
+// tokens, 16 / 4 heads in 128-row blocks, and 4 x 720 .. 1680, 8 heads in 64-row blocks:
+//   head dim 64:  112 keys -12 -14 -9 and -4 +1 +2, 160: -6 -10 -2 and +4 +2 +5, 208: -5 -8 -3 and -2 +4 +4; 176 (an eighth of a block's
+//                 tiles is not empty): -4 -6 -1 and -3 -2 +3, 240: +3 -4 0 and +5 +5 +6; 32 the same within 3
+//   128:          48: -19 -24 -15 and -13 -11 -8, 80: -23 -22 -10 and -8 -6 +4, 96: -14 -13 -1 and 0 +2 +10, 112: -6 -6 -4 and +4 +2 +8,
+//                 160: -9 -5 +1 and +6 +6 +11, 208: -3 0 +4 and +9 +11 +11
+//   96:           48: -15 -17 -8 and -3 -4 +3, 80: -17 -15 -5 and 0 +2 +12, 96: -7 -1 +7 and +9 +8 +19, 160: +3 +2 +11 and +18 +15 +20
+//   192 (160):    48: -10 -9 -3 and -3 -3 +10, 80: -2 -4 +6 and +3 +7 +12; 96 and 160 fill its tiles of 32 keys: +9 .. +16
+//   256:          48: -15 -14 -4 and +6 -2 0, 80: -10 -13 +1 and +1 +1 +7, 112: +5 +4 +8 and +19 +8 +15
 // An item's first tile is under way 0.2 to 0.8 us later, though, which is what shows where there is little to be saved: a kept block
 // leaves `empty` keys of its tiles, and a sequence has no more blocks than there are to each that ends in part of one (there are at
 // least that many sequences).  Up to four tiles saved a sequence, runs and groups: 13 x 92 .. 176 tokens, 8 heads of 128, 80-key blocks
 // 11.9 and 12.7 us; 4 x 200 .. 400, 8 of 64, 96-key blocks 13.2 and 13.9, but 48-key blocks 14.4 and 13.8; 9 x 135 .. 272, 2 of 128, 112-key
-// blocks 14.4 and 15.0.  Above: 8 x 40 .. 70, 8 / 2 heads of 64, 16-key blocks 10.2 and 9.2; 8 x 300 .. 500, 16 of 128, 80-key blocks 33.8 and 32.4.
-// A group is numbered in 16 bits.  The rule is the same for the one-launch and the prepared form, so they compute the same bits.
-constexpr int kMostGroupedBlock = 256;
-inline bool fwd_grouped(int total_k, int num_k_block, int k_block_size) {
+// blocks 14.4 and 15.0.  Above: 8 x 40 .. 70, 8 / 2 heads of 64, 16-key blocks 10.2 and 9.2.  Larger blocks need more: 8 x 120 .. 282, 8 / 1 heads of 64,
+// 80-key blocks, four saved, 12.3 and 12.6; at head dim 128 4 x 825, 2 / 1 heads, sixteen saved, 24.9 and 26.4 (few items, whose tiles follow
+// one another with nothing beside them).
+// A group is numbered in 16 bits.  The rule is the same for the one-launch and the prepared form, which pads head dims: they compute the same bits.
+inline bool fwd_grouped(long long pairs, int headdim, int total_k, int num_k_block, int k_block_size) {
+  const int tile = headdim > 128 && headdim <= 192 ? kTileKeys / 2 : kTileKeys, most = headdim <= 64 ? 208 : headdim <= 128 ? 96 : 48;
+  if (k_block_size % tile == 0 || k_block_size > most || (long long)num_k_block * k_block_size > 16 * 65535ll) return false;
   const long long empty = (kTileKeys - k_block_size % kTileKeys) % kTileKeys, parts = std::max<long long>(1, num_k_block - total_k / k_block_size);
-  return num_k_block * empty > 4 * kTileKeys * parts && k_block_size % kTileKeys != 0 && k_block_size < kMostGroupedBlock && (long long)num_k_block * k_block_size <= 16 * 65535ll;
+  if (8 * empty < k_block_size + empty) return false;
+  if (k_block_size > 48 && headdim > 64 && pairs < device_cus()) return false;
+  return num_k_block * empty > (k_block_size <= 48 ? 4 : headdim <= 64 ? 5 : 20) * kTileKeys * parts;
 }
 
 // The fields of FwdParams that follow from the call's shape and softmax_scale alone.
@@ -674,7 +688,7 @@ void fill_shape(FwdParams &fp, int total_q, int total_k, int nhead_q, int nhead_
   const FwdSplit split = fwd_split(slots, headdim, f32_exact, (long long)nhead_k * num_q_block, num_k_block, k_block_size,
                                    (long long)num_q_block * q_block_size, total_q);
   fp.nw = split.nw;
-  fp.grouped = fwd_grouped(total_k, num_k_block, k_block_size) ? 1 : 0;
+  fp.grouped = fwd_grouped((long long)nhead_k * num_q_block, headdim, total_k, num_k_block, k_block_size) ? 1 : 0;
   fp.split = split.parts;
   fp.ncol = headdim / 8;
   fp.max_parts = 1;
