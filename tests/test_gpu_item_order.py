@@ -1,8 +1,9 @@
-"""Items sorted by weight in the prepared form of the forward: the same results as in any other order."""
+"""Items sorted by weight in the prepared form of the forward: heaviest first, with the same results as in any other order."""
 import pytest
 import torch
 
-from hbsattn_amd import HBSAttention, set_onepass
+from hbsattn_amd import HBSAttention, _lib, set_onepass
+from hbsattn_amd.interface import hbsa_prepare
 from hbsattn_amd.workloads import make_problem
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,64 @@ def test_two_streams_prepare_at_once(two_launches):
                 got[i].append(HBSAttention(*w.args()))
     torch.cuda.synchronize()
     assert all(torch.equal(o, want[i]) for i in range(2) for o in got[i])
+
+
+def _orders(w):
+    """The two orders hbsa_prepare leaves at the end of its workspace: (q block << 16 | kv head) of every item, k block numbers."""
+    (nq, _, q2b, cu_nq), (nk, _, _, cu_nk) = w.q_meta, w.k_meta
+    prepared = hbsa_prepare(w.cu_q_seqlens, w.cu_k_seqlens, w.block_mask, w.q_block_size, w.k_block_size, w.causal, int(nq), q2b, cu_nq, int(nk),
+                            cu_nk, run_shape=(w.q.dtype, w.q.shape[0], w.k.shape[0], w.q.shape[1], w.q.shape[2]))
+    up = lambda x: -(-x // 256) * 256
+    pairs = w.block_mask.shape[0] * int(nq)
+    words = up(4 * pairs) // 4
+    at = _lib.load().hbsa_fwd_workspace_bytes(w.block_mask.shape[0], int(nq), int(nk)) - up(4 * pairs) - up(4 * int(nk))
+    ints = prepared.workspace[at:at + up(4 * pairs) + up(4 * int(nk))].view(torch.int32).cpu()
+    return ints[:pairs], ints[words:words + int(nk)]
+
+
+def _weights(w):
+    """Kept keys of every (q block, kv head), whole blocks, and the query rows that see a key of every k block."""
+    items, rows, qb, kb = {}, [], 0, 0
+    mask, shift = w.block_mask.cpu(), 4
+    while shift < 16 and (int(w.k_meta[0]) * w.k_block_size) >> shift >= 512:   # weights are told apart in units of 2^shift keys, 512 of them
+        shift += 1
+    for b in range(len(w.cu_q) - 1):
+        nq, nk = int(w.cu_q[b + 1] - w.cu_q[b]), int(w.cu_k[b + 1] - w.cu_k[b])
+        q_blocks, k_blocks = -(-nq // w.q_block_size), -(-nk // w.k_block_size)
+        for i in range(q_blocks):
+            sees = min(nk, min(nq, (i + 1) * w.q_block_size) + nk - nq) if w.causal else nk   # keys before this one
+            blocks = -(-max(0, sees) // w.k_block_size)
+            for h in range(mask.shape[0]):
+                kept = int(mask[h, qb + i, kb:kb + blocks].sum()) * w.k_block_size
+                items[(qb + i) << 16 | h] = min(511, (kept + (1 << shift) - 1) >> shift)
+        rows += [min(nq, nk - j * w.k_block_size) if w.causal else nq for j in range(k_blocks)]
+        qb, kb = qb + q_blocks, kb + k_blocks
+    return items, rows
+
+
+MANY = dict(hq=4, hk=4, d=64, qbs=16, kbs=16, keep=0.5)
+ORDERED = [SPECS[i] for i in (0, 1, 2, 4, 5, 6)] + [
+    dict(q_lens=[40 * (i % 3) for i in range(n)], k_lens=[384 + i % 50 for i in range(n)], causal=causal, **MANY)
+    for n, causal in ((63, True), (64, False), (65, True), (256, True))]
+
+
+@pytest.mark.parametrize("spec", ORDERED, ids=lambda s: f"{len(s['q_lens'])}x{s['q_lens'][0]}-h{s['hk']}-q{s['qbs']}-{s['causal']}")
+def test_items_and_k_blocks_come_heaviest_first(spec):
+    w = make_problem(seed=35, diag=spec["keep"] > 0, scale=None, **spec)
+    pairs = w.block_mask.shape[0] * w.block_mask.shape[1]
+    keys = int(w.cu_k[-1])
+    # what the preparation sorts: up to 4096 items, as many as CUs, of 384 keys a sequence on average
+    assert torch.cuda.get_device_properties(0).multi_processor_count <= pairs <= 4096 and keys >= 384 * (len(w.cu_k) - 1)
+    order, order_k = _orders(w)
+    items, rows = _weights(w)
+    assert sorted(order.tolist()) == sorted(items)
+    weights = [items[x] for x in order.tolist()]
+    assert weights == sorted(weights, reverse=True)
+    assert len(set(weights)) > 1 or spec["keep"] == 0.0
+    assert order_k.tolist() == sorted(range(len(rows)), key=lambda kb: -rows[kb])   # equals in their own order
+
+
+def test_k_blocks_of_more_sequences_than_are_ordered_keep_their_order():
+    n = 257
+    w = make_problem(seed=36, q_lens=[30] * n, k_lens=[384] * n, hq=2, hk=2, d=64, qbs=16, kbs=16, keep=0.5, diag=True, causal=True, scale=None)
+    assert _orders(w)[1].tolist() == list(range(w.block_mask.shape[2]))
