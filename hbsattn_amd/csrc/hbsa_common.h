@@ -117,7 +117,7 @@ struct FwdParams {
   int32_t nsub;   // workgroups per (kv head, q block) = ceil(ratio * wps / nw)
   uint32_t q_sign;  // 0x80008000 when softmax_scale < 0 (Q is negated, |scale| used)
   float c;        // |softmax_scale| * log2(e)
-  float lag;      // kLazyRescaleLog2 / c: how far the running max may lag, in raw score units
+  float lag;      // kLazyRescaleLog2 / c: how far the decode kernel's running max may lag, in raw score units
   FastDiv div_nsub, div_nqb, div_kbs;   // divisions on the scheduler's path
   int32_t f32;    // fp32 inputs staged as fp16: the softmax constants come from the launch record, where
                   // the setup kernel derived them from the tensors' maxima
@@ -226,7 +226,6 @@ struct ElemBF16 {
   }
   static __device__ __forceinline__ float lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
   static __device__ __forceinline__ float hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
-  static __device__ __forceinline__ uint32_t scale_packed(uint32_t w, float f) { return pack2(lo(w) * f, hi(w) * f); }
 };
 struct ElemF16 {
   static __device__ __forceinline__ f32x16 mfma(short8v a, short8v b, f32x16 c) {
@@ -238,7 +237,6 @@ struct ElemF16 {
   }
   static __device__ __forceinline__ float lo(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w).x; }
   static __device__ __forceinline__ float hi(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w).y; }
-  static __device__ __forceinline__ uint32_t scale_packed(uint32_t w, float f) { return pack2(lo(w) * f, hi(w) * f); }
 };
 
 // exchange-and-combine between lane i and lane i^32
@@ -338,7 +336,7 @@ struct BwdParams {
   float *parts;          // partial accumulators, shared by the two launches
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
   const int32_t *order_k;   // k blocks by falling number of query rows that can see them, nullptr: in their own order
-  int32_t many;          // host side only: more than two rounds of dK/dV items (head dim 64)
+  int32_t many;          // host side only: more than 4.5 dK/dV items a CU (head dim 64)
 };
 
 // ---- Items of the kernels without a scheduler: geometry and kept blocks straight from the caller's arrays (bits == nullptr)
@@ -427,13 +425,13 @@ __device__ __forceinline__ void parts_acquire() { __builtin_amdgcn_fence(__ATOMI
 // through the list) then gives every workgroup about the same.  One wavefront counts each pair, the workgroup that arrives last
 // sorts by counting; the order among equals is left to chance, and no result depends on it.
 // Measured, forward kernels: 6 x 300 .. 4000 tokens, 16 / 4 heads of 64, 1.8 items a place, 67 -> 48 us, the pre-pass 4.7 -> 7.7.
-// In the one-launch form, which has no pre-pass, a launch for the order alone (8 to 11 us) takes back what it gives: 8 x 2050
-// tokens, 16 heads of 192, not causal, 221 -> 199 + 11; C5's shape 276 -> 262 + 8.
+// The one-launch form has no pre-pass, and a launch for the order alone took 8 to 11 us: of what it gives, 8 x 2050 tokens, 16 heads of
+// 192, not causal, 221 -> 199, C5's shape 276 -> 262, 11 and 6 us would be left, and shorter calls lose.  That form takes no order.
 constexpr int kMaxOrderItems = 4096;   // pairs (of 8192, 4 x 8192 tokens with 32 heads, no launch takes the order, and sorting them costs 10 us)
 constexpr int kOrderBins = 2 * kThreads;   // weights told apart
 constexpr int kOrderCopies = 4;            // counters of one weight, by lane: equal weights otherwise queue at one word of LDS
 struct OrderRoom {   // a stream's
-  uint32_t order[kMaxOrderItems], weight[kMaxOrderItems];
+  uint32_t weight[kMaxOrderItems];
   uint32_t arrived, pad[63];   // zero before and after every launch
 };
 struct OrderLds {

@@ -1273,8 +1273,8 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
       fp.nparts = parts;
   }
   fp.div_nparts = make_fast_div((uint32_t)fp.nparts);
-  // the clocked walk: block sizes that are whole tiles, work that is not split, K/V of a head beyond what an L2 holds
   if (order_bytes(nhead_k, num_q_block, num_k_block) != 0) fp.order = (const uint32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
+  // the clocked walk: block sizes that are whole tiles, work that is not split, K/V of a head beyond what an L2 holds
   fp.walk = (!g_deterministic && fp.nparts == 1 && k_block_size % kTileKeys == 0 &&
              2ll * total_k * headdim * 2 >= g_walk_min_bytes) ? 1 : 0;
 

@@ -1095,7 +1095,8 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         if (compute) {
           // The tile is processed as two halves of 32 keys so that, inside one wavefront, the
           // matrix cores always have work queued while the vector ALU does the softmax of the
-          // other half:   S0, max(S0) | S1 + exp(S0) | PV0 + max(S1), exp(S1) | PV1.
+          // other half:   S0 | S1 + exp(S0) | PV0 + exp(S1) | PV1.   (A maximum, of S0, is formed for an item's first tile alone:
+          // see settle_half.)
           const bool first = chunk_base + t == 0;   // the item's first tile gives the reference
           // keys that are missing, or (causal) a last key that some lane's query does not see
           const bool edge = valid < KT || (p.causal && tile.pos(KT / 16 - 1) + 15 > wave_kvis_min);
