@@ -37,7 +37,7 @@ namespace hbsa {
 // backward.  That number falls along a sequence, so how many blocks of another sequence come before a block is a division.  A
 // wavefront works on one block at a time, a lane on a sequence in 64.  (A lane per block that went through the sequences took
 // 110 us with 250 of them and 40 with 64.)  Boundaries that do not fit each other, a long batch, a
-// call that no backward need follow (weigh_k 0): the blocks' own order.
+// call that no backward need follow and more k blocks than the wavefronts get done in time (weigh_k 0): the blocks' own order.
 constexpr int kWeighedSequences = 256;
 __device__ __forceinline__ void order_k_blocks(const PrepParams &p, int wave, int waves, int lane) {
   constexpr int N = kWeighedSequences / 64;
@@ -1108,6 +1108,10 @@ size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t 
 }  // extern "C"
 namespace {
 constexpr long long kWeighedKeys = 384;   // keys of a sequence, on average, from which on items are weighed
+// k blocks that a wavefront of the pre-pass puts in their place, one after the other at 0.4 us each: more of them (few q blocks and
+// heads, many keys) keep their own order.  2 x 45 .. 91 queries on 27883 .. 45509 keys, one head, 64-key blocks: 285 for each of four
+// wavefronts, pre-pass 4 -> 109 us.  Queries and keys of one length in equal blocks are one k block a wavefront at most.
+constexpr long long kOrderedKBlocks = 8;
 // weigh_items, weigh_k_blocks: the orders are made by weight.  Without, they are there, too (last q blocks first, k blocks in their
 // own order): a run or a backward may follow on the workspace.
 int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
@@ -1146,11 +1150,11 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
   pp.batch = batch; pp.nkb = num_k_block; pp.total_q = total_q; pp.total_k = total_k;
   pp.nhead_k = nhead_k;
   pp.weight_shift = weight_shift((long long)num_k_block * k_block_size);
-  pp.weigh_k = weigh_k_blocks ? 1 : 0;
   pp.order = nullptr;
   pp.order_k = nullptr;
   pp.room = nullptr;
   const dim3 grid((num_q_block + 3) / 4, nhead_k);
+  pp.weigh_k = weigh_k_blocks && num_k_block <= kOrderedKBlocks * (kThreads / 64) * grid.x * grid.y ? 1 : 0;
   if (order_bytes(nhead_k, num_q_block, num_k_block) != 0) {
     pp.order = (uint32_t *)((char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
     pp.order_k = (int32_t *)((char *)pp.order + order_bytes(nhead_k, num_q_block, num_k_block));

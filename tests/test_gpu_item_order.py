@@ -128,3 +128,13 @@ def test_k_blocks_of_more_sequences_than_are_ordered_keep_their_order():
     n = 257
     w = make_problem(seed=36, q_lens=[30] * n, k_lens=[384] * n, hq=2, hk=2, d=64, qbs=16, kbs=16, keep=0.5, diag=True, causal=True, scale=None)
     assert _orders(w)[1].tolist() == list(range(w.block_mask.shape[2]))
+
+
+@pytest.mark.parametrize("k_blocks", [32, 33])
+def test_k_blocks_are_ordered_by_enough_wavefronts_alone(k_blocks):
+    # two q blocks and one head are one workgroup of four wavefronts, of at most eight k blocks each: more would be put in their
+    # places one after the other for longer than it gives (285 for each wavefront took 109 us of the pre-pass, which takes 4)
+    w = make_problem(seed=37, q_lens=[16, 64], k_lens=[16 * 16, 16 * (k_blocks - 16)], hq=1, hk=1, d=64, qbs=64, kbs=16, keep=0.5, diag=True,
+                     causal=False, scale=None)
+    own = list(range(k_blocks))
+    assert _orders(w)[1].tolist() == (own[16:] + own[:16] if k_blocks == 32 else own)
