@@ -1107,7 +1107,16 @@ size_t hbsa_fwd_split_workspace_bytes(int32_t total_q, int32_t nhead_q, int32_t 
 
 }  // extern "C"
 namespace {
-constexpr long long kWeighedKeys = 384;   // keys of a sequence, on average, from which on items are weighed
+// Whether items are weighed.  Counting and sorting takes 3 us and 3 more for every thousand pairs, and gives what unequal items leave of a
+// launch's end: nothing where the device has no second round of them, little where they are a few tiles long or there are many rounds, and with
+// many kv heads neighbours in the order share no K and V.  Without and with the order, us: forward of 130 sequences, 64-row blocks, 300 .. 500
+// tokens, 4 heads of 64 (3508 pairs) 40.6 and 55.6, 1 .. 300 queries on 400 .. 900 keys (1680) 31.1 and 40.2, 50 on 1000, 16 heads
+// (2080) 43.0 and 52.0; training, 32 heads of 64, 8 x 500 .. 1500 tokens 153 and 168, 4 x 1000 103 and 113, of 128, 2 x 2000 .. 6000 580 and 602;
+// 1 x 2800, 8 heads (352 pairs) 77 and 80; 24 x 100 .. 900, 32 / 8 heads of 64, 237 and 248.  But 6 x 300 .. 4000, 8 heads (1416 pairs), of 64
+// 168 and 157, of 128 331 and 317, 2 x 2000 .. 6000, 8 of 128 (544), 345 and 335.
+inline bool items_weighed(long long pairs, int nhead_k, int batch, long long keys) {
+  return 2ll * device_cus() <= pairs && pairs <= 6ll * device_cus() && nhead_k <= 16 && batch < kSeqCap && keys >= 768ll * batch;
+}
 // k blocks that a wavefront of the pre-pass puts in their place, one after the other at 0.4 us each: more of them (few q blocks and
 // heads, many keys) keep their own order.  2 x 45 .. 91 queries on 27883 .. 45509 keys, one head, 64-key blocks: 285 for each of four
 // wavefronts, pre-pass 4 -> 109 us.  Queries and keys of one length in equal blocks are one k block a wavefront at most.
@@ -1158,12 +1167,9 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
   if (order_bytes(nhead_k, num_q_block, num_k_block) != 0) {
     pp.order = (uint32_t *)((char *)workspace + order_offset(nhead_k, num_q_block, num_k_block));
     pp.order_k = (int32_t *)((char *)pp.order + order_bytes(nhead_k, num_q_block, num_k_block));
-    // (a captured launch may be replayed on any stream, while the room belongs to this one)
-    // Counting and sorting takes 3 to 5 us, and gives what unequal items leave of a launch's end: nothing where the device has no
-    // second round of them, and too little where they are a few tiles long (250 x 20 .. 128 tokens, 16 / 4 heads of 64: 39.4 ->
-    // 44.6 us with the order, 2 x 700 tokens, 8 heads, in training 51.8 -> 55.0; 24 x 100 .. 900 in training 134 -> 114).
     const long long keys = std::min<long long>(total_k, (long long)num_k_block * k_block_size);
-    weigh_items = weigh_items && (long long)nhead_k * num_q_block >= device_cus() && keys >= kWeighedKeys * batch;
+    weigh_items = weigh_items && items_weighed((long long)nhead_k * num_q_block, nhead_k, batch, keys);
+    // (a captured launch may be replayed on any stream, while the room belongs to this one)
     if (weigh_items && !is_capturing((hipStream_t)stream)) (void)stream_sched_of((hipStream_t)stream, nullptr, &pp.room);
     hipLaunchKernelGGL((hbsa_prep_kernel<true>), grid, dim3(kThreads), 0, (hipStream_t)stream, pp);
   } else {
