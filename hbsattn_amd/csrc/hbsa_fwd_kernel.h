@@ -643,12 +643,16 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
 
   // ------------------------------------------------------------------ per-thread constants
   // tile loads: thread -> (row, 16-byte chunk) of the tile, same for every tile
-  // Where a round of the workgroup's loads is a whole number of rows after which the chunk placement repeats, the rounds
-  // differ in their scalar base only; elsewhere every load has its offset in a register.
-  constexpr bool UNIFORM = (64 * NW) % CPR == 0 && SW::POW2 && (64 * NW / CPR) % SW::PERIOD == 0;
-  constexpr int ROUND_ROWS = UNIFORM ? 64 * NW / CPR : 0, OFFSETS = UNIFORM ? 1 : LOADS;
+  // Rounds of the workgroup's loads that are a whole number of rows after which the chunk placement repeats apart differ in
+  // their scalar base only: load i takes offset i % OFFSETS, ahead_rows(i) rows on (at head dim 256, whose rounds are a quarter of
+  // the period, four offsets in place of eight: bytes of scratch a lane 184 -> 116 for head dims 200 to 248, 8 x 2050 tokens, 16 heads
+  // of 208, 412 -> 310 us).  Where rows are no power of two long every load has its offset in a register.
+  constexpr int ROUND_ROWS = SW::POW2 ? 64 * NW / CPR : 0;
+  constexpr int OFFSETS = !SW::POW2 ? LOADS : ROUND_ROWS >= SW::PERIOD ? 1 : SW::PERIOD / ROUND_ROWS < LOADS ? SW::PERIOD / ROUND_ROWS : LOADS;
+  static_assert(!SW::POW2 || (OFFSETS == LOADS || OFFSETS * ROUND_ROWS % SW::PERIOD == 0), "loads that share an offset share their chunk");
+  auto ahead_rows = [](int i) constexpr { return i / OFFSETS * OFFSETS * ROUND_ROWS; };
   uint32_t ld_koff[OFFSETS], ld_voff[OFFSETS];   // byte offset of the thread's chunk from the tile's (GROUPED: the group's) first row
-  bool ld_kin[LOADS], ld_vin[LOADS];             // COLS: the chunk is one of the row's
+  bool ld_kin[OFFSETS], ld_vin[OFFSETS];         // COLS: the chunk is one of the row's
   const uint32_t ks32 = (uint32_t)p.k_s, vs32 = (uint32_t)p.v_s;   // row strides in bytes (the host checks they fit)
   auto ld_place = [&](int i, int &r, uint32_t &kchunk, uint32_t &vchunk) {
     const int c = (i * NW + wave) * 64 + lane;
@@ -658,14 +662,12 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     vchunk = (uint32_t)((pc ^ SW::v(r)) * 16);
   };
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
+  for (int i = 0; i < OFFSETS; ++i) {
     int r; uint32_t kc, vc;
     ld_place(i, r, kc, vc);
-    if (i < OFFSETS) {
-      const uint32_t from = GROUPED ? (uint32_t)r & 15u : (uint32_t)r;
-      ld_koff[i] = from * ks32 + kc;
-      ld_voff[i] = from * vs32 + vc;
-    }
+    const uint32_t from = GROUPED ? (uint32_t)r & 15u : (uint32_t)r;
+    ld_koff[i] = from * ks32 + kc;
+    ld_voff[i] = from * vs32 + vc;
     ld_kin[i] = !COLS || kc < (uint32_t)p.ncol * 16u;
     ld_vin[i] = !COLS || vc < (uint32_t)p.ncol * 16u;
   }
@@ -751,7 +753,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         base += (uint64_t)(uint32_t)tile.pos(0) * (uint64_t)stride;
         static_for<0, LOADS>([&](auto i_) {
           constexpr int i = decltype(i_)::value;
-          uint32_t voff = (V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i]) +
+          uint32_t voff = (V_PART ? ld_voff[i % OFFSETS] : ld_koff[i % OFFSETS]) +
                           (lane >= 16 * CPR - (i * NW + wave_) * 64 ? apart : 0u);
           if (valid < KT) {
             const int row = ((i * NW + wave_) * 64 + lane) / CPR;
@@ -759,7 +761,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
             asm volatile("" : "+v"(step));
             voff += step;
           }
-          if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))
+          if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i % OFFSETS] : ld_kin[i % OFFSETS])))
             dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, voff, l0);
         });
         return;
@@ -770,7 +772,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         constexpr int ROUND = NW * 64 / CPR;   // rows between two loads
         const int row = ((i * NW + wave_) * 64 + lane) / CPR;
         int g = ONE ? ((wave_ * 64 / CPR) >> 4) + i * ROUND / 16 : ((i * NW + wave_) * 64 / CPR) >> 4;
-        uint32_t voff = V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i];
+        uint32_t voff = V_PART ? ld_voff[i % OFFSETS] : ld_koff[i % OFFSETS];
         if (valid < KT) {
           g = min(g, (valid - 1) >> 4);
           uint32_t step = (uint32_t)((min(row, valid - 1) & 15) - (row & 15)) * stride;
@@ -782,9 +784,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           const int second = 16 * (g + 1) * CPR - (i * NW + wave_) * 64;   // first lane of the second group, if one of them is
           voff += lane >= second ? (group_at(min(g + 1, (valid - 1) >> 4)) - pos) * stride : 0u;
         }
-        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))
+        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i % OFFSETS] : ld_kin[i % OFFSETS])))
           dma16(std::integral_constant<int, lds_off + i * NW * 1024>{},
-                base + (uint64_t)(pos + (UNIFORM ? (uint32_t)(i * ROUND) & 15u : 0u)) * (uint64_t)stride, voff, l0);
+                base + (uint64_t)(pos + ((uint32_t)ahead_rows(i) & 15u)) * (uint64_t)stride, voff, l0);
       });
       return;
     }
@@ -792,18 +794,18 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     if (valid == KT) {
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
-        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))   // (a lane that loads nothing leaves its 16 bytes of LDS alone)
-        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base + (uint64_t)(uint32_t)(i * ROUND_ROWS) * (V_PART ? vs32 : ks32),
-              V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i], l0);
+        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i % OFFSETS] : ld_kin[i % OFFSETS])))   // (a lane that loads nothing leaves its 16 bytes of LDS alone)
+        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base + (uint64_t)(uint32_t)ahead_rows(i) * (V_PART ? vs32 : ks32),
+              V_PART ? ld_voff[i % OFFSETS] : ld_koff[i % OFFSETS], l0);
       });
     } else {   // ragged tail of a run: rows past the end re-read the last valid row (masked later)
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
-        const int r0 = ((UNIFORM ? 0 : i * NW) * 64 + wave * 64 + lane) / CPR;
-        uint32_t step = (uint32_t)(min(r0 + i * ROUND_ROWS, valid - 1) - r0) * (V_PART ? vs32 : ks32);
+        const int r0 = (i % OFFSETS * NW * 64 + wave * 64 + lane) / CPR;
+        uint32_t step = (uint32_t)(min(r0 + ahead_rows(i), valid - 1) - r0) * (V_PART ? vs32 : ks32);
         asm volatile("" : "+v"(step));   // (or a 64-bit multiply-add is formed, and its 64-bit addend kept in registers)
-        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i] : ld_kin[i])))
-        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, (V_PART ? ld_voff[UNIFORM ? 0 : i] : ld_koff[UNIFORM ? 0 : i]) + step, l0);
+        if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i % OFFSETS] : ld_kin[i % OFFSETS])))
+        dma16(std::integral_constant<int, lds_off + i * NW * 1024>{}, base, (V_PART ? ld_voff[i % OFFSETS] : ld_koff[i % OFFSETS]) + step, l0);
       });
     }
   };

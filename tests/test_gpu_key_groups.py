@@ -89,4 +89,4 @@ def test_blocks_in_one_run_take_no_longer_than_whole_tiles(d, kbs):
             z.synchronize()
             times[i].append(a.elapsed_time(z))
     print(f"us {min(times[0]) * 100:.1f} {min(times[1]) * 100:.1f}")
-    assert min(times[1]) <= 1.07 * min(times[0]), f"{min(times[1]) * 100:.1f} us against {min(times[0]) * 100:.1f}"
+    assert min(times[1]) <= 1.09 * min(times[0]), f"{min(times[1]) * 100:.1f} us against {min(times[0]) * 100:.1f}"

@@ -94,4 +94,4 @@ def test_a_reference_that_lags_a_little_is_moved_once(d):
             z.record()
             z.synchronize()
             times[i].append(a.elapsed_time(z))
-    assert min(times[1]) <= 1.12 * min(times[0]), f"{min(times[1]) * 50:.1f} us against {min(times[0]) * 50:.1f}"
+    assert min(times[1]) <= 1.2 * min(times[0]), f"{min(times[1]) * 50:.1f} us against {min(times[0]) * 50:.1f}"
