@@ -672,7 +672,8 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
 // all keys and none for keys past the block's end (their columns are not stored).  Operand reads issued by hand as in the
 // dQ kernel were measured and are no faster.  dQ + dK/dV, 6 x 300 .. 4000 tokens, 16 / 4 heads, 64-key blocks, keep 0.4:
 // 250 -> 227 us with the loads two tiles ahead, 195 with the heads going round the grid (bwd_decode_grid).
-// MANY: the form with 165 registers a wavefront, three workgroups to a CU (head dim 32: 127, four), for many rounds of items.
+// MANY: the form with 165 registers a wavefront, three workgroups to a CU, for many rounds of items.  At head dim 32 (127 registers, 131
+// without) the two are even, 72 training calls of 75 .. 480 us within 2 %, and there is this one alone.
 // Two workgroups of 209 registers are better where there are few rounds and the longest item sets the time: dQ + dK/dV, 64-key blocks, at 1.4 rounds of two (6 x 300 ..
 // 4000 tokens, 16 / 4 heads) 205 and 215 us, at 2.0 (128-key blocks, 8 x 500 .. 3000, 32 / 8) 310 and 337, at 2.3 (2 x 600 .. 1500,
 // 32) 73 and 71, at 3.0 (6 x 4000, 16 / 4) 419 and 401, at 8 (4 x 8192, 16) 400 and 371.
@@ -1426,8 +1427,9 @@ int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t st
     return launch_bwd_parts<D, E, false, false>(bp, nhead_k, num_k_block, stream);
   } else {
     // (the kernel for smaller head dims decides for itself whether wavefronts share a slot)
-    if (D == 32 || bp.many) return launch_bwd_parts<D, E, false, true>(bp, nhead_k, num_k_block, stream);
-    return launch_bwd_parts<D, E, false, false>(bp, nhead_k, num_k_block, stream);
+    if constexpr (D == 32) return launch_bwd_parts<D, E, false, true>(bp, nhead_k, num_k_block, stream);
+    else if (bp.many) return launch_bwd_parts<D, E, false, true>(bp, nhead_k, num_k_block, stream);
+    else return launch_bwd_parts<D, E, false, false>(bp, nhead_k, num_k_block, stream);
   }
 }
 
