@@ -302,6 +302,23 @@ __device__ __forceinline__ void lds_wait(short4v &a, short4v &b, short4v &c, sho
   asm volatile("s_waitcnt lgkmcnt(%8)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f), "+v"(g), "+v"(h) : "n"(N));
 }
 
+// Placement of a K / V tile's rows in LDS: 16-byte chunk c of row r sits at chunk position c ^ k(r) (K), c ^ v(r) (V).
+// Rows by 16 consecutive ones (K, one chunk column at a time) then start at 16 different 16-byte slots of the 256-byte
+// bank sweep, and the 4 rows x 64 bytes of a transposing V read cover it once.  With a row of 4, 8, 16 or 32 chunks
+// that takes an exclusive or over all chunk bits; rows of 12, 20 and 24 chunks already step by 12, 4 and 8 slots, so
+// that the low two or three bits are enough (and the exchange stays inside the row).
+template <int D>
+struct FwdSwizzle {
+  static constexpr int CPR = D / 8;
+  static constexpr int RPG = 16 / CPR > 0 ? 16 / CPR : 1;   // rows per 256-byte bank sweep
+  static constexpr bool POW2 = (CPR & (CPR - 1)) == 0;
+  static constexpr int PERIOD = RPG * CPR;   // rows after which the placement repeats (POW2)
+  static __device__ __forceinline__ int k(int r) { return POW2 ? (r / RPG) % CPR : CPR % 8 == 0 ? (r >> 1) & 7 : (r >> 2) & 3; }
+  static __device__ __forceinline__ int v(int r) {
+    return POW2 ? (CPR >= 8 ? ((r / RPG) % (CPR / 4)) << 2 : 0) : CPR % 8 == 0 ? ((r >> 1) & 1) << 2 : 0;
+  }
+};
+
 template <int I, int N, typename F>
 __device__ __forceinline__ void static_for(F &&f) {
   if constexpr (I < N) {

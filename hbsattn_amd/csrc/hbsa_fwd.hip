@@ -535,16 +535,18 @@ inline size_t split_bytes(int parts, int total_q, int nhead_q, int nhead_k, int 
 // An odd number of parts (see decode_max_parts for why)
 inline int odd_parts(long long parts) { return parts < 2 ? 1 : parts % 2 ? (int)parts : (int)parts - 1; }
 // Parts an item of the fp32 kernel may be cut into, kPartKeys keys each at least.  With up to two items per CU (all resident
-// at once, the longest several times the average) enough parts for nine per CU, no more than all k blocks can fill, 32,
-// and kMaxPartBytes of partial results.  Measured, 4 sequences of 1279 .. 2697 tokens, 8 / 4 heads, keep 0.5: whole items
-// 153 us, parts of at least 512 / 256 / 128 keys 158 / 121 / 117 us at D = 64; 87 / 86 / 67 / 63 us at D = 32.
+// at once, the longest several times the average) enough parts for four per CU and five at least, no more than all k blocks can
+// fill, 32, and kMaxPartBytes of partial results.  Measured, four against nine per CU: 40 calls of 10 .. 120 us 4 % faster
+// (4 x 92 .. 298 tokens, 16 heads of 32, 18.7 -> 15.1 us; 5 x 169, 8 / 1 heads of 128, 31.6 -> 26.7; at worst 24.7 -> 25.9);
+// without the lower bound of five, 4 x 500 .. 3000 tokens, 8 / 4 heads of 64, 440 items: 79 -> 110.  Parts of at least 256
+// keys: 36.5 us in place of 27.7 (2 x 224 .. 324, 16 / 4 heads of 128).
 constexpr int kPartKeys = 128;
 constexpr size_t kMaxPartBytes = 96ull << 20;
 inline size_t f32_part_bytes(int headdim) { return (size_t)4 * (headdim / 2 + 2) * 64 * sizeof(float); }   // of one part
 int f32_max_parts(long long items, int headdim, int num_k_block) {
   const int cus = device_cus();
   if (items <= 0 || items > 2ll * cus || items > kMaxPartItems) return 1;
-  long long parts = std::min<long long>(32, 9ll * cus / items);
+  long long parts = std::min<long long>(32, std::max(5ll, 4ll * cus / items));
   parts = std::min<long long>(parts, num_k_block);
   parts = std::min<long long>(parts, (long long)(kMaxPartBytes / (f32_part_bytes(headdim) * (size_t)items)));
   return odd_parts(parts);

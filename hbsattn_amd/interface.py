@@ -24,9 +24,9 @@ _NATIVE_HEADDIMS = (32, 64, 128, 256)      # head dims every form of the forward
 _BWD_MAX_HEADDIM = 128                      # the backward kernels stop here
 _DTYPE_CODES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16, torch.float32: _lib.DTYPE_F32}
 
-# How fp32 q/k/v are multiplied: "exact" = fp32 matrix instructions, the arithmetic of the reference's
+# How fp32 q/k/v are multiplied: "exact" = unrounded operands, the arithmetic of the reference's
 # fp32 path (``tl.dot(..., allow_tf32=False)``, reference hbsattn/fwd_triton_auto_tile_size.py:205,225);
-# "fast" = scaled fp16 staging copies and the 16-bit kernel (11-bit operand significands, about ten
+# "fast" = scaled fp16 staging copies and the 16-bit kernel (11-bit operand significands, several
 # times faster).  The environment variable HBSATTN_AMD_FP32_MODE sets the initial mode.
 _fp32_mode = os.environ.get("HBSATTN_AMD_FP32_MODE", "exact")
 if _fp32_mode not in ("exact", "fast"):

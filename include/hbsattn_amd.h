@@ -37,7 +37,7 @@ extern "C" {
  * hbsattn/fwd_triton_auto_tile_size.py:272) */
 #define HBSA_DTYPE_BF16 0
 #define HBSA_DTYPE_F16 1
-#define HBSA_DTYPE_F32 2          /* fp32 tensors, fp32 matrix instructions: the reference's fp32 arithmetic */
+#define HBSA_DTYPE_F32 2          /* fp32 tensors, fp32 products and sums: the reference's fp32 arithmetic */
 #define HBSA_DTYPE_F32_STAGED16 3 /* fp32 tensors, 16-bit matrix instructions: see hbsa_fwd_workspace_bytes_dtype */
 
 #define HBSA_ERR_INVALID_ARGUMENT (-1)
@@ -135,10 +135,10 @@ size_t hbsa_fwd_workspace_bytes(int32_t nhead_k, int32_t num_q_block, int32_t nu
  * hbsa_fwd_workspace_bytes.
  *
  * fp32 q/k/v/out (the reference accepts them, its tests use them: reference
- * test/test_accuracy.py:24) come in two forms.  HBSA_DTYPE_F32 multiplies fp32 operands with fp32
- * matrix instructions, as the reference's fp32 path does (tl.dot(..., allow_tf32=False), reference
- * hbsattn/fwd_triton_auto_tile_size.py:205,225), at the fp32 matrix rate, a sixteenth of the bf16
- * one.  HBSA_DTYPE_F32_STAGED16 is the fast form: each tensor is multiplied by a power of two
+ * test/test_accuracy.py:24) come in two forms.  HBSA_DTYPE_F32 multiplies fp32 operands
+ * unrounded, as the reference's fp32 path does (tl.dot(..., allow_tf32=False), reference
+ * hbsattn/fwd_triton_auto_tile_size.py:205,225): each is the sum of three bf16 numbers, and six
+ * bf16 products, summed in fp32, stand for one.  HBSA_DTYPE_F32_STAGED16 is the fast form: each tensor is multiplied by a power of two
  * chosen from its largest magnitude (found on the device, no host synchronisation) and rounded to
  * fp16 staging copies in the workspace, the 16-bit kernel runs on those with fp32 accumulation and
  * softmax, and `out` is written as fp32.  Its operands carry 11-bit significands (fp32's range is
