@@ -20,7 +20,7 @@ API_SOURCE = os.path.join(CSRC, "hbsa_fwd.hip")     # the C ABI and the kernels 
 INST_SOURCE = os.path.join(CSRC, "hbsa_inst.hip")   # the attention kernels of one head dim and element type
 OUTPUT = os.path.join(_HERE, "libhbsattn_amd.so")
 # substrings of the mangled names of the kernels with hand-issued LDS reads ...
-HAND_ISSUED_READS = ("hbsa_fwd_kernel", "hbsa_bwd_dq_kernel", "hbsa_bwd_dkv8_kernel")
+HAND_ISSUED_READS = ("hbsa_fwd_kernel", "hbsa_bwd_dq_kernel", "hbsa_bwd_dkv")
 COMPILER_ISSUED = "hbsa_fwd_kernelILi256E"   # ... except the head dim 256 instantiations, whose reads the compiler issues
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32 out of scalar float code.

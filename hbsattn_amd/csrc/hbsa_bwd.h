@@ -26,11 +26,11 @@
 // Both recompute S.  The kept blocks of a mask row or column are found with one load per 32 or 64
 // blocks, not one per block.  Tiles go from global memory straight into LDS (global_load_lds_dwordx4),
 // two tiles ahead (V tiles of the dQ kernel one): tiles t + 1 and t + 2 travel while tile t is computed on, one barrier per
-// tile.  The dK/dV kernels walk the q blocks from the last to the first, so that the workgroups of a sequence, each of which
+// tile (per two tiles, one ahead, for k blocks of up to 64 keys at head dims up to 64).  The dK/dV kernels walk the q blocks from the last to the first, so that the workgroups of a sequence, each of which
 // a causal mask lets begin at another q block, start with the same tiles; the delta and the log-sum-exp of a tile's rows are
 // consecutive floats of one q head.  A tile that is
 // read both by rows and transposed is stored once, in a layout without bank conflicts for either
-// (BwdTile::swz_both).  In the dQ kernel and the D = 128 dK/dV kernel the operand reads from LDS are issued by
+// (BwdTile::swz_both).  The operand reads from LDS are issued by
 // hand, a fixed number ahead of the products that use them (BwdOperandOffsets).  The forward's persistent
 // scheduling is not applied here: the grids already start their heaviest workgroups first, and what bounds
 // both kernels at long sequences is the stream of tiles from memory next to the matrix work, not the tail.
@@ -131,41 +131,6 @@ __device__ __forceinline__ void bwd_transposed_products(const short4v *v, short8
 #pragma unroll
   for (int dt = 0; dt < BwdTile<D>::DT; ++dt) {
     const short8v va = __builtin_shufflevector(v[2 * dt], v[2 * dt + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-    acc[dt] = E::mfma(va, packed, acc[dt]);
-  }
-}
-
-// rows 32*h .. 32*h+31 of the tile . frag^T, the forward's S^T = K Q^T for one half of a tile
-template <int D, typename E>
-__device__ __forceinline__ f32x16 bwd_rows_times_frag(const char *tile, int h, const short8v *frag, int lane) {
-  using T = BwdTile<D>;
-  const int l32 = lane & 31, g32 = lane >> 5;
-  const int rd = l32 * T::RB + ((g32 ^ T::swz_both(l32)) << 4) + h * 32 * T::RB;
-  f32x16 a;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) a[i] = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < T::KSTEPS; ++ks) a = E::mfma(*(const short8v *)(tile + (rd ^ (ks * 32))), frag[ks], a);
-  return a;
-}
-
-// acc[dt] += tile^T (rows 16*g .. 16*g+15 of the tile as the contraction index) . packed, the forward's
-// O^T += V^T P^T for one group of 16 keys
-template <int D, typename E>
-__device__ __forceinline__ void bwd_transposed_times_packed(const char *tile, int g, short8v packed, int lane, f32x16 *acc) {
-  using T = BwdTile<D>;
-  const int g32 = lane >> 5;
-  const int key = 4 * g32 + ((lane & 15) >> 2);
-  const int lc = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-  const int rd = key * T::RB + ((lc ^ T::swz_both(key)) << 4) + 8 * (lane & 1);
-  const int rd8 = (key + 8) * T::RB + ((lc ^ T::swz_both(key + 8)) << 4) + 8 * (lane & 1);   // the row 8 further down
-#pragma unroll
-  for (int dt = 0; dt < T::DT; ++dt) {
-    const char *a = tile + (rd ^ (dt * 64)) + g * 16 * T::RB;
-    const char *a8 = tile + (rd8 ^ (dt * 64)) + g * 16 * T::RB;
-    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)HBSA_AS3(a));
-    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v *)HBSA_AS3(a8));
-    const short8v va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     acc[dt] = E::mfma(va, packed, acc[dt]);
   }
 }
@@ -530,7 +495,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
     }
     dlt = half_sum(dlt);
     if (g32 == 0 && l32 < nrows && (!PARTS || part == 0)) {
-      p.delta[(int64_t)hq * p.total_q + my_row] = dlt;
+      p.delta[(int64_t)hq * p.total_q + my_row] = -dlt;
       p.lse2[(int64_t)hq * p.total_q + my_row] = lse2;
     }
   }
@@ -661,34 +626,85 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
     bwd_store_rows<D, E>(p.dq + (int64_t)(inf.row_begin + row0 + l32) * p.dq_s + (int64_t)hq * p.dq_h, acc, p.scale, g32);
 }
 
+// ---- The tiles of a k block, for the dK/dV kernel of head dims up to 64: a list in LDS, made once by one wavefront.  (With every
+// wavefront walking the mask column tile by tile, a third of what it issued was that walk: 148 scalar instructions a tile.)
+constexpr int kBwdListCap = 256;   // entries: in-sequence position of the first row | q head of the group << 7, rows; a multiple of 64
+struct BwdTileRange {
+  int qb_begin;         // the sequence's first q block
+  int qb_low, qb_end;   // q blocks of the list
+  int row0, qlen;       // first query row and query count of the sequence
+  int r_last_end;       // q heads of the group below it are the last block's, ...
+  int r_first;          // ... those from it on the first one's (a part's share; the others' are all)
+  int first_row;        // in-sequence position of the first row that sees a key of the workgroup
+};
+// lane i: the word at bit row qb_end - 1 - i (by falling q block) of a mask column, zero outside of [low, end)
+__device__ __forceinline__ uint32_t bwd_column_word(const BwdParams &p, const uint32_t *column, int first, int low, int end, int lane) {
+  const int g = first + 63 - lane;
+  return g >= low && g < end ? column[(size_t)g * p.wpr] : 0u;
+}
+// Entries [chunk_base, chunk_base + kBwdListCap) of the tiles, last q block first, to `list`; returns how many there are in all.
+// first: the column's words of the last 64 q blocks, if they have been loaded.
+__device__ __forceinline__ int bwd_key_tiles(const BwdParams &p, const BwdTileRange &t, const uint32_t *column, int bit, const uint32_t *first,
+                                             int chunk_base, u32x2 *list, int lane) {
+  int total = 0;
+  for (int base = t.qb_end - 64; base + 63 >= t.qb_low; base -= 64) {
+    const uint32_t word = first != nullptr && base == t.qb_end - 64 ? *first : bwd_column_word(p, column, base, t.qb_low, t.qb_end, lane);
+    const int qb = base + 63 - lane, pos = (qb - t.qb_begin) * p.qbs;
+    const int rows = min(p.qbs, t.qlen - pos), skip = max(0, t.first_row - pos);   // rows of the block, and those before the first that sees a key
+    int heads = 0, tiles = 0, r0 = 0;
+    if (((word >> bit) & 1u) != 0 && skip < rows) {
+      r0 = qb == t.qb_low ? t.r_first : 0;
+      heads = (qb == t.qb_end - 1 ? t.r_last_end : p.ratio) - r0;
+      tiles = ((rows + 63) >> 6) - (skip >> 6);
+    }
+    const int mine = max(heads, 0) * tiles;
+    int incl = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int y = __shfl_up(incl, off);
+      if (lane >= off) incl += y;
+    }
+    int to = total + incl - mine - chunk_base;
+    for (int r = r0; r < r0 + heads; ++r)
+      for (int row = skip & ~63; row < rows; row += 64, ++to)
+        if (tiles > 0 && to >= 0 && to < kBwdListCap) list[to] = u32x2{(uint32_t)(pos + row), (uint32_t)r << 7 | (uint32_t)min(64, rows - row)};
+    total += __builtin_amdgcn_readlane(incl, 63);
+  }
+  return total;
+}
+
 // ---- dK, dV (head dims up to 64) ---------------------------------------------------------------------
 // Four wavefronts; K^T and V^T of a wavefront's 32 keys stay in registers.  The Q and dO tiles go straight
-// into LDS like the dQ kernel's (three buffers, one layout, one barrier per tile).  When the workgroup's keys
-// fill at most two 32-key slots (k blocks of up to 64 keys, or the narrow rest of a wider block), two
-// wavefronts share a slot and take the upper and lower 32 rows of every tile; their partial sums are added
-// through LDS at the end.
-// What bounds it: instruction issue, with two wavefronts per SIMD (226 registers when P, dS and both accumulators were in
-// flight together, 207 now; at three wavefronts, 168 registers, 50 of them spill).  Hence no comparisons where all rows see
-// all keys and none for keys past the block's end (their columns are not stored).  Operand reads issued by hand as in the
-// dQ kernel were measured and are no faster.  dQ + dK/dV, 6 x 300 .. 4000 tokens, 16 / 4 heads, 64-key blocks, keep 0.4:
-// 250 -> 227 us with the loads two tiles ahead, 195 with the heads going round the grid (bwd_decode_grid).
-// MANY: the form with 165 registers a wavefront, three workgroups to a CU, for many rounds of items.  At head dim 32 (127 registers, 131
-// without) the two are even, 72 training calls of 75 .. 480 us within 2 %, and there is this one alone.
-// Two workgroups of 209 registers are better where there are few rounds and the longest item sets the time: dQ + dK/dV, 64-key blocks, at 1.4 rounds of two (6 x 300 ..
-// 4000 tokens, 16 / 4 heads) 205 and 215 us, at 2.0 (128-key blocks, 8 x 500 .. 3000, 32 / 8) 310 and 337, at 2.3 (2 x 600 .. 1500,
-// 32) 73 and 71, at 3.0 (6 x 4000, 16 / 4) 419 and 401, at 8 (4 x 8192, 16) 400 and 371.
-template <int D, typename E, bool PARTS, bool MANY>
+// into LDS like the dQ kernel's (one layout, one barrier a step).  k blocks of up to 64 keys fill two 32-key slots (SPLIT):
+// two wavefronts work on one 64-row tile and the other two on the next one, a step is two tiles, and the two sums are added through
+// LDS at the end; two buffers, one step ahead.  Larger blocks fill four slots with one tile a step in three buffers, two
+// steps ahead; in the narrow rest of a block (at most two slots) two wavefronts share a slot and take the upper and lower 32
+// rows of every tile.
+// What bounds it: a tile is one chain from S to dK, and the wavefronts on the longest k blocks have a SIMD to themselves when the
+// others have ended, so that it is what one wavefront issues and waits for: of 3270 cycles a tile and wavefront 1530
+// were instructions (590 of them the walk over the mask, a tile at a time), 1120 waits for LDS and the barrier, one read after another.  Hence
+// the tile list (bwd_key_tiles), two tiles a barrier, operand reads issued by hand, dP started at -delta, both halves of a tile
+// unrolled, the second one's first reads before the first one's last products.  6 x 300 .. 4000 tokens, 16 / 4 heads, 64-key
+// blocks, keep 0.4: 141 us, with the list and two tiles a step by a workgroup of eight wavefronts 124, in this form 115, dP from
+// -delta and no refill of the list inside the loop 109, halves unrolled 100.  dQ + dK/dV + forward: 1 x 8000, 32 / 1 heads, 838 ->
+// 713; 6 x 4000, 16 / 4, 531 -> 497; 4 x 8192, 16 heads, 128-key blocks, 1537 -> 1521; head dim 32, 4 x 8192, 1008 -> 959.
+// (217 registers at head dim 64, two wavefronts a SIMD.  Three of 165 registers were the better form of the kernel before where there
+// were more than 4.5 items a CU; this one is faster there, too: 8 x 500 .. 3000, 32 / 8, 128-key blocks, 489 -> 466.)
+template <int D, typename E, bool PARTS, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) {
   static_assert(D <= 64, "head dim 128 has its own kernel");
   using T = BwdTile<D>;
+  // SPLIT (k blocks of up to 64 keys, two slots of 32): two wavefronts work on one tile and the other two on the next one
+  constexpr int TEAMS = SPLIT ? 2 : 1, WAVES = 4 / TEAMS, BUFS = SPLIT ? 2 : 3;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  // buffer s of the tiles (three of them): Q rows at s * 2 * TILE_BYTES, dO rows one tile further
-  float *rowv = (float *)(lds + 6 * T::TILE_BYTES);    // buffer s: [64] log2-domain log-sum-exp of the tile's rows, [64] their delta
+  // buffer s of a team's tiles (BUFS of them): Q rows at (s * TEAMS + team) * 2 * TILE_BYTES, dO rows one tile further
+  float *rowv = (float *)(lds + TEAMS * BUFS * 2 * T::TILE_BYTES);    // and of it: [64] log2-domain log-sum-exp of the tile's rows, [64] their -delta
+  u32x2 *list = (u32x2 *)(rowv + TEAMS * BUFS * 128);             // [kBwdListCap] tiles, see bwd_key_tiles
+  int *list_total = (int *)(list + kBwdListCap);
 
   const int lane = threadIdx.x & 63;
-  // ("& 3": the compiler then sees the two values rows_half can take, and does less of the loop over the halves at once.
-  // A launch bound of three workgroups in its place makes 46 registers spill.)
-  const int wave = __builtin_amdgcn_readfirstlane(MANY ? (threadIdx.x >> 6) & 3 : threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % WAVES;   // of the team
+  const int team = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / WAVES;
   const int g32 = lane >> 5, l32 = lane & 31;
   int hk, bx;
   bwd_decode_grid(p, (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u), hk, bx);
@@ -708,14 +724,10 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   const int kbl = kb - seq.kb0;                      // in-sequence index of the k block
   const int k0 = seq.k0, klen = seq.k1 - k0;
   const bool fits = seq.fits(p, kb);
-  auto column_word = [&](int first, int low, int end) -> uint32_t {   // lane i: the word of q block first + i, if low <= first + i < end
-    const int g = first + lane;
-    return g >= low && g < end ? p.bits[((size_t)hk * p.nqb + g) * p.wpr + (kbl >> 5)] : 0u;
-  };
-  const uint32_t first_word = !PARTS && fits ? column_word(seq.qb1 - 64, seq.qb0, seq.qb1) : 0u;
+  const uint32_t first_word = !PARTS && fits ? bwd_column_word(p, p.bits + (size_t)hk * p.nqb * p.wpr + (kbl >> 5), seq.qb1 - 64, seq.qb0, seq.qb1, lane) : 0u;
   const int krows = min(p.kbs, klen - kbl * p.kbs);  // keys in the block
   const int wg_keys = min(4 * kWaveRows, p.kbs - sub * 4 * kWaveRows);   // by the block size: the same for every k block
-  const bool shared_slots = wg_keys <= 2 * kWaveRows;                    // two wavefronts per 32-key slot
+  const bool shared_slots = !SPLIT && wg_keys <= 2 * kWaveRows;          // two wavefronts per 32-key slot
   const int slot = shared_slots ? (wave & 1) : wave;
   const int rows_half = shared_slots ? (wave >> 1) : 0;                  // which 32 rows of a tile (shared slots)
   const int row0 = (sub * 4 + slot) * kWaveRows;
@@ -747,148 +759,174 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   // the tile sequence: for every q block of the sequence that keeps this k block, for every q head of
   // the group, the block's rows in 64-row tiles (under a causal mask only those with a row that sees a
   // key of this workgroup)
-  const int qb_begin = seq.qb0;
-  int qb = qb_begin - 1, r = 0, qoff = 0, qb_end = seq.qb1;
-  int kept_base = qb_end;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
-  int qb_first = qb_begin, r_first = 0, r_last_end = p.ratio, nparts = 1;   // the part's share (BwdKeyPart)
-  uint64_t kept = 0;
-  QBlockInfo inf = {};
-  int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
-  if (qb_begin < qb_end) {
+  int shift = 0, nparts = 1, total = 0;
+  BwdTileRange range = {seq.qb0, seq.qb0, 0, 0, 0, p.ratio, 0, 0};
+  if (seq.qb0 < seq.qb1) {
     if (!bwd_record_holds(seq, record)) {
       bwd_zero_keys<D>(p, seq, kb, sub, hk);
       return;
     }
-    inf.shift = __builtin_amdgcn_readlane((int)record, 5);
-    seq_row0 = __builtin_amdgcn_readlane((int)record, 0);
-    seq_qlen = klen - inf.shift;
+    shift = __builtin_amdgcn_readlane((int)record, 5);
+    range.row0 = __builtin_amdgcn_readlane((int)record, 0);
+    range.qlen = klen - shift;
+    range.qb_end = seq.qb1;
+    range.first_row = p.causal ? wg_first_key - shift : 0;
   }
   if (!fits) return;   // (a sequence without queries that lies outside of the tensors)
+  int qb_low = seq.qb0;
   if constexpr (PARTS) {
-    const BwdKeyPart share(p, qb_begin, qb_end, inf.shift, wg_first_key, part);
+    const BwdKeyPart share(p, seq.qb0, range.qb_end, shift, wg_first_key, part);
     nparts = share.count;
     if (part >= nparts) return;
-    qb_first = share.qb_first;
-    r_first = share.r_first;
-    r_last_end = share.r_last_end;
-    qb_end = share.qb_last + 1;
-    kept_base = qb_end;
+    qb_low = share.qb_first;
+    range.r_first = share.r_first;
+    range.r_last_end = share.r_last_end;
+    range.qb_end = share.qb_last + 1;
   }
-  kept_base -= 64;
-  kept = __ballot(((PARTS ? column_word(kept_base, qb_first, qb_end) : first_word) >> (kbl & 31)) & 1u);
-  auto tile_reaches = [&]() {
-    return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
-  };
-  auto next_tile = [&]() -> bool {
-    for (;;) {
-      if (qb >= qb_begin) {   // inside a kept q block: next tile, then next head
-        qoff += 64;
-        if (qoff >= inf.rows) { qoff = 0; ++r; }
-        if (r < (PARTS && qb == qb_end - 1 ? r_last_end : p.ratio)) {
-          if (tile_reaches()) return true;
-          continue;
-        }
-      }
-      while (kept == 0) {   // one load per 64 q blocks: lane i looks at q block kept_base + i
-        kept_base -= 64;
-        if (kept_base + 63 < qb_first) return false;
-        const uint32_t word = column_word(kept_base, qb_first, qb_end);
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // (waited for here so that no other path waits)
-        kept = __ballot((word >> (kbl & 31)) & 1u);
-      }
-      const int at = 63 - __builtin_clzll(kept);
-      qb = kept_base + at;
-      kept &= ~(1ull << at);
-      // the q block's geometry follows from the sequence's (no load on this path)
-      inf.q_pos = (qb - qb_begin) * p.qbs;
-      inf.row_begin = seq_row0 + inf.q_pos;
-      inf.rows = min(p.qbs, seq_qlen - inf.q_pos);
-      if (inf.rows <= 0) {   // more q blocks than the sequence has rows for: none is written into such a block's bit row
-        qb = qb_begin - 1;
-        continue;
-      }
-      r = PARTS && qb == qb_first ? r_first : 0;
-      qoff = -64;   // the step above moves to the block's first tile
+  range.qb_low = qb_low;
+  const uint32_t *column = p.bits + (size_t)hk * p.nqb * p.wpr + (kbl >> 5);
+  if (range.qb_low < range.qb_end && range.qlen > 0) {
+    if (threadIdx.x < 64) {
+      const int n = bwd_key_tiles(p, range, column, kbl & 31, PARTS ? nullptr : &first_word, 0, list, lane);
+      if (lane == 0) *list_total = n;
     }
-  };
+    __syncthreads();
+    total = __builtin_amdgcn_readfirstlane(*list_total);
+  }
   // (placement of a tile's chunks over the four wavefronts: see hbsa_bwd_dq_kernel)
-  constexpr int RPL = 1024 / T::RB, LOADS = 64 / (4 * RPL);
+  constexpr int RPL = 1024 / T::RB, LOADS = 64 / (WAVES * RPL);
   const int ld_row = RPL * wave + lane / T::CPR;
   const uint32_t ld_chunk = (uint32_t)(((lane % T::CPR) ^ T::swz_both(ld_row)) * 16);
   const uint32_t q_s32 = (uint32_t)p.q_s, do_s32 = (uint32_t)p.do_s;   // the host checks that they fit
-  const uint32_t tiles_addr = (uint32_t)(uintptr_t)HBSA_AS3(lds) + (uint32_t)wave * 1024u;
-  const uint32_t row_addr = (uint32_t)(uintptr_t)HBSA_AS3(rowv);
+  const uint32_t q_voff = (uint32_t)ld_row * q_s32 + ld_chunk, do_voff = (uint32_t)ld_row * do_s32 + ld_chunk;   // of a full tile's first load
+  const char *q_base = p.q + (int64_t)range.row0 * p.q_s + (int64_t)hk * p.ratio * p.q_h, *g_base = p.dout + (int64_t)range.row0 * p.do_s + (int64_t)hk * p.ratio * p.do_h;
+  const int64_t row_base = (int64_t)hk * p.ratio * p.total_q + range.row0;
+  const uint32_t tiles_addr = (uint32_t)(uintptr_t)HBSA_AS3(lds) + (uint32_t)(team * 2 * T::TILE_BYTES + wave * 1024);
+  const uint32_t row_addr = (uint32_t)(uintptr_t)HBSA_AS3(rowv) + (uint32_t)team * 512u;
   // Loads of one tile per wavefront: LOADS of Q and of dO, and in wavefront 0 the two of the rows' values
-  auto fetch = [&](int buf) {   // the tile next_tile() has moved to
-    const int valid = min(64, inf.rows - qoff);
-    const int64_t row_first = inf.row_begin + qoff;
-    const int hq = hk * p.ratio + r;
-    const char *qsrc = p.q + row_first * p.q_s + (int64_t)hq * p.q_h;
-    const char *gsrc = p.dout + row_first * p.do_s + (int64_t)hq * p.do_h;
-    const uint32_t dst = tiles_addr + (uint32_t)(buf * 2 * T::TILE_BYTES);
+  auto fetch = [&](int buf, int pos, int valid, int r) {   // `valid` rows of q head r of the group, from in-sequence position pos on
+    const char *qsrc = q_base + (uint64_t)(uint32_t)pos * q_s32 + (int64_t)r * p.q_h;
+    const char *gsrc = g_base + (uint64_t)(uint32_t)pos * do_s32 + (int64_t)r * p.do_h;
+    const uint32_t dst = tiles_addr + (uint32_t)(buf * TEAMS * 2 * T::TILE_BYTES);
+    if (valid == 64) {   // a full tile: the loads differ in their scalar base only
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const uint32_t rr = (uint32_t)min(ld_row + 4 * RPL * i, valid - 1);   // rows past the block's end repeat its last row
-      bwd_dma16(dst + (uint32_t)(i * 4 * 1024), qsrc, rr * q_s32 + ld_chunk);
-      bwd_dma16(dst + (uint32_t)(T::TILE_BYTES + i * 4 * 1024), gsrc, rr * do_s32 + ld_chunk);
+      for (int i = 0; i < LOADS; ++i) {
+        bwd_dma16(dst + (uint32_t)(i * WAVES * 1024), qsrc + (uint64_t)(uint32_t)(WAVES * RPL * i) * q_s32, q_voff);
+        bwd_dma16(dst + (uint32_t)(T::TILE_BYTES + i * WAVES * 1024), gsrc + (uint64_t)(uint32_t)(WAVES * RPL * i) * do_s32, do_voff);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const uint32_t rr = (uint32_t)min(ld_row + WAVES * RPL * i, valid - 1);   // rows past the block's end repeat its last row
+        bwd_dma16(dst + (uint32_t)(i * WAVES * 1024), qsrc, rr * q_s32 + ld_chunk);
+        bwd_dma16(dst + (uint32_t)(T::TILE_BYTES + i * WAVES * 1024), gsrc, rr * do_s32 + ld_chunk);
+      }
     }
     if (wave == 0) {
       const uint32_t rvoff = (uint32_t)min(lane, valid - 1) * 4u;
-      bwd_dma4(row_addr + (uint32_t)(buf * 512), p.lse2 + (int64_t)hq * p.total_q + row_first, rvoff);
-      bwd_dma4(row_addr + (uint32_t)(buf * 512 + 256), p.delta + (int64_t)hq * p.total_q + row_first, rvoff);
+      const int64_t row_at = row_base + (int64_t)r * p.total_q + pos;
+      bwd_dma4(row_addr + (uint32_t)(buf * TEAMS * 512), p.lse2 + row_at, rvoff);
+      bwd_dma4(row_addr + (uint32_t)(buf * TEAMS * 512 + 256), p.delta + row_at, rvoff);
     }
   };
-  int n_ahead = 0;                               // tiles fetched and not computed on yet
-  int buf_f = 0, buf = 0;                        // buffer of the next fetch, and of the current tile
-  int fq_a = 0, fq_b = 0, va_a = 64, va_b = 64;  // first query position and row count of those tiles (a: the older)
-  bool more = next_tile();
-  auto issue = [&]() {   // fetches the tile next_tile() stands on and moves on
-    const int fq = inf.q_pos + qoff, va = min(64, inf.rows - qoff);
-    if (n_ahead == 0) { fq_a = fq; va_a = va; } else { fq_b = fq; va_b = va; }
-    fetch(buf_f);
-    buf_f = buf_f == 2 ? 0 : buf_f + 1;
-    ++n_ahead;
-    more = next_tile();
-  };
-  if (more) issue();
-  if (more) issue();
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the resident operands have arrived, and the tiles (see hbsa_bwd_dkv8_kernel)
-  const int shift = inf.shift;
+  BwdOperandOffsets<D> off;
+  off.init(lane);
+  const uint32_t lds_base = (uint32_t)(uintptr_t)HBSA_AS3(lds);
   const int h_begin = shared_slots ? rows_half : 0, h_end = shared_slots ? rows_half + 1 : 2;   // 32-row halves of a tile
+  for (int chunk_base = 0; chunk_base < total;) {   // ---- chunks of the tile list (usually one)
+  const int entries = min(total - chunk_base, kBwdListCap);
+  int n_ahead = 0;                               // tiles (of each team) fetched and not computed on yet
+  int buf_f = 0, buf = 0;                        // buffer of the next fetch, and of the current tile
+  int fq_a = 0, fq_b = 0, va_a = 64, va_b = 64;  // first query position and row count of those tiles (a: the older); no rows: there is none
+  int at = team;                                 // this team's next entry
+  u32x2 held = {0u, 0u};                         // lane i: entry i of the list's current 64
+  auto issue = [&]() {   // fetches the team's next tile
+    if (at - team < entries && ((at - team) & 63) == 0) {
+      held = list[min(at - team + lane, kBwdListCap - 1)];
+      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): here, not on every tile's path
+    }
+    int fq = 0, va = 0;
+    if (TEAMS == 1 || at < entries) {
+      const uint32_t y = (uint32_t)__builtin_amdgcn_readlane((int)held.y, at & 63);
+      fq = __builtin_amdgcn_readlane((int)held.x, at & 63);
+      va = (int)(y & 127u);
+      fetch(buf_f, fq, va, (int)(y >> 7));
+    }
+    if (n_ahead == 0) { fq_a = fq; va_a = va; } else { fq_b = fq; va_b = va; }
+    buf_f = buf_f == BUFS - 1 ? 0 : buf_f + 1;
+    ++n_ahead;
+    at += TEAMS;
+  };
+  auto more = [&]() { return at - team < entries; };
+  issue();
+  if (BUFS == 3 && more()) issue();
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the resident operands have arrived, and the tiles (see hbsa_bwd_dkv8_kernel)
   while (n_ahead > 0) {
     const int first_q_pos = fq_a, valid = va_a;
     // This wavefront's part of the tile has landed; the loads of the tile after it (a wavefront's loads return in
     // order) may still be under way.
-    if (n_ahead >= 2) {
+    if (n_ahead >= 2 && (TEAMS == 1 || va_b > 0)) {
       if (wave == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * LOADS + 2));
       else __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * LOADS));
     } else {
       __builtin_amdgcn_s_waitcnt(0x0F70);
     }
     __syncthreads();   // ... every wavefront's, and the buffer of the tile before has been read by all
-    const char *q_t = lds + buf * 2 * T::TILE_BYTES, *g_t = q_t + T::TILE_BYTES;
-    const float *lse_s = rowv + buf * 128, *dlt_s = lse_s + 64;
-    buf = buf == 2 ? 0 : buf + 1;
+    const uint32_t tile_lds = lds_base + (uint32_t)((buf * TEAMS + team) * 2 * T::TILE_BYTES);
+    const uint32_t rows_lds = lds_base + (uint32_t)(TEAMS * BUFS * 2 * T::TILE_BYTES + (buf * TEAMS + team) * 512);
+    buf = buf == BUFS - 1 ? 0 : buf + 1;
     fq_a = fq_b;
     va_a = va_b;
     --n_ahead;
-    if (more) issue();   // two tiles ahead
-    if (!active) continue;
+    if (more()) issue();   // ahead by one buffer less than there are
+    if (!active || (TEAMS > 1 && valid == 0)) continue;
     // rows first_vis .. valid - 1 of the tile see this lane's key (what lanes without a key sum up is not stored);
     // comparisons and selects are left out where all 64 rows see all of the wavefront's keys
     int first_vis = 0;
     if (p.causal) first_vis = max(0, key_pos - shift - first_q_pos);
     const bool diagonal = p.causal && wave_key_max - shift - first_q_pos > 0;
-#pragma unroll 1
-    for (int h = h_begin; h < h_end; ++h) {
-      // P first, its product with dO next, then dP: half as many values are alive at a time as with both at once
-      const f32x16 s = bwd_rows_times_frag<D, E>(q_t, h, kf, lane);
+    // Operand reads are issued by hand (BwdOperandOffsets), in the order the products need them and as far ahead as the counter
+    // (15 of them) and the registers allow: with a read next to every product, a tile was 16 round trips to LDS one after another.
+    const uint32_t q_t = tile_lds, g_t = q_t + (uint32_t)T::TILE_BYTES;
+    constexpr int KS = T::KSTEPS, DT = T::DT;
+    short8v qr[KS];
+    auto half = [&](auto h_) {
+      constexpr int h = decltype(h_)::value;
+      constexpr bool NEXT = SPLIT && h == 0;   // the other half follows: the first reads of it go out before this one's last products
+      const uint32_t h_rows = (uint32_t)h * (32 * T::RB), v_at = rows_lds + (uint32_t)(128 * h + 16 * g32);
+      short8v gr[KS], lv[4], dl[4];
+      short4v tg[2][2 * DT], tq[2][2 * DT];
+      if constexpr (!(SPLIT && h == 1))
+        static_for<0, KS>([&](auto i_) { qr[decltype(i_)::value] = lds_read_b128<0>(off.rows[decltype(i_)::value] + q_t + h_rows); });
+      static_for<0, 4>([&](auto i_) { lv[decltype(i_)::value] = lds_read_b128<32 * decltype(i_)::value>(v_at); });
+      static_for<0, KS>([&](auto i_) { gr[decltype(i_)::value] = lds_read_b128<0>(off.rows[decltype(i_)::value] + g_t + h_rows); });
+      f32x16 s, dp;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = 0.f;
+      static_for<0, KS>([&](auto i_) {
+        constexpr int i = decltype(i_)::value;
+        lds_wait1<(2 * KS + 3 - i)>(qr[i]);
+        s = E::mfma(qr[i], kf[i], s);
+      });
+      static_for<0, 4>([&](auto i_) { dl[decltype(i_)::value] = lds_read_b128<256 + 32 * decltype(i_)::value>(v_at); });
+      bwd_issue_transposed<D, 0>(off, g_t + h_rows, tg[0]);
+      asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(dl[0]), "+v"(dl[1]), "+v"(dl[2]), "+v"(dl[3]) : "n"(2 * DT));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dp[i] = __builtin_bit_cast(f32x4, dl[i >> 2])[i & 3];   // (dP starts at -delta)
+      static_for<0, KS>([&](auto i_) {
+        constexpr int i = decltype(i_)::value;
+        lds_wait1<(2 * DT)>(gr[i]);
+        dp = E::mfma(gr[i], vf[i], dp);
+      });
+      bwd_issue_transposed<D, 1>(off, g_t + h_rows, tg[1]);
+      asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(lv[0]), "+v"(lv[1]), "+v"(lv[2]), "+v"(lv[3]) : "n"(4 * DT));
+      // P and its product with dO, then dS and its product with Q
       float e[16];
       auto form_p = [&](auto short_, auto diagonal_) {
         const int left = valid - 32 * h - 4 * g32, before = first_vis - 32 * h - 4 * g32;
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
-          const f32x4 l4 = *(const f32x4 *)(lse_s + 32 * h + 8 * a + 4 * g32);
+          const f32x4 l4 = __builtin_bit_cast(f32x4, lv[a]);
 #pragma unroll
           for (int bq = 0; bq < 4; ++bq) {
             float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * a + bq], p.c, -l4[bq]));
@@ -903,41 +941,63 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       else form_p(std::false_type{}, std::false_type{});
       short8v lo, hi;
       bwd_pack<E>(e, lo, hi);
-      const f32x16 dp = bwd_rows_times_frag<D, E>(g_t, h, vf, lane);
-      bwd_transposed_times_packed<D, E>(g_t, 2 * h, lo, lane, acc_v);
-      bwd_transposed_times_packed<D, E>(g_t, 2 * h + 1, hi, lane, acc_v);
+      bwd_wait_transposed<D, 2 * DT>(tg[0]);
+      bwd_transposed_products<D, E>(tg[0], lo, acc_v);
+      bwd_issue_transposed<D, 0>(off, q_t + h_rows, tq[0]);
+      bwd_wait_transposed<D, 2 * DT>(tg[1]);
+      bwd_transposed_products<D, E>(tg[1], hi, acc_v);
+      bwd_issue_transposed<D, 1>(off, q_t + h_rows, tq[1]);
 #pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const f32x4 d4 = *(const f32x4 *)(dlt_s + 32 * h + 8 * a + 4 * g32);
-#pragma unroll
-        for (int bq = 0; bq < 4; ++bq) e[4 * a + bq] *= dp[4 * a + bq] - d4[bq];
-      }
+      for (int i = 0; i < 16; ++i) e[i] *= dp[i];
       bwd_pack<E>(e, lo, hi);
-      bwd_transposed_times_packed<D, E>(q_t, 2 * h, lo, lane, acc_k);
-      bwd_transposed_times_packed<D, E>(q_t, 2 * h + 1, hi, lane, acc_k);
-    }
+      if constexpr (NEXT)
+        static_for<0, KS>([&](auto i_) { qr[decltype(i_)::value] = lds_read_b128<0>(off.rows[decltype(i_)::value] + q_t + (uint32_t)(32 * T::RB)); });
+      bwd_wait_transposed<D, 2 * DT + (NEXT ? KS : 0)>(tq[0]);
+      bwd_transposed_products<D, E>(tq[0], lo, acc_k);
+      bwd_wait_transposed<D, NEXT ? KS : 0>(tq[1]);
+      bwd_transposed_products<D, E>(tq[1], hi, acc_k);
+    };
+    if (SPLIT || h_begin == 0) half(std::integral_constant<int, 0>{});
+    if (SPLIT || h_end == 2) half(std::integral_constant<int, 1>{});
   }
-  if (shared_slots) {   // the wavefronts of the lower rows hand their sums to those of the upper rows: [slot][register][lane] floats
+  chunk_base += kBwdListCap;
+  if (chunk_base < total) {
     __syncthreads();
-    float *xch = (float *)lds + (size_t)slot * (2 * T::DT * 16) * 64 + lane;
-    if (rows_half == 1) {
+    if (threadIdx.x < 64) (void)bwd_key_tiles(p, range, column, kbl & 31, nullptr, chunk_base, list, lane);
+    __syncthreads();
+  }
+  }
+  // the sums of the wavefronts that share a slot (the upper and lower rows' of a tile, the teams') go to the first of them
+  // through LDS: [wavefront][slot][register][lane] floats
+  const int sharers = TEAMS * (shared_slots ? 2 : 1), sharer = team * (shared_slots ? 2 : 1) + rows_half;
+  if (sharers > 1) {
+    constexpr int REGS = 2 * T::DT * 16;
+    const int slots = shared_slots ? 2 : 4;
+    __syncthreads();
+    float *xch = (float *)lds + (size_t)slot * REGS * 64 + lane;
+    if (sharer > 0) {
+      float *mine = xch + (size_t)(sharer - 1) * slots * REGS * 64;
 #pragma unroll
       for (int dt = 0; dt < T::DT; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          xch[(dt * 16 + i) * 64] = acc_k[dt][i];
-          xch[((T::DT + dt) * 16 + i) * 64] = acc_v[dt][i];
+          mine[(dt * 16 + i) * 64] = acc_k[dt][i];
+          mine[((T::DT + dt) * 16 + i) * 64] = acc_v[dt][i];
         }
     }
     __syncthreads();
-    if (rows_half == 0) {
+    if (sharer == 0) {
+#pragma unroll 1
+      for (int x = 1; x < sharers; ++x) {
+        const float *theirs = xch + (size_t)(x - 1) * slots * REGS * 64;
 #pragma unroll
-      for (int dt = 0; dt < T::DT; ++dt)
+        for (int dt = 0; dt < T::DT; ++dt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          acc_k[dt][i] += xch[(dt * 16 + i) * 64];
-          acc_v[dt][i] += xch[((T::DT + dt) * 16 + i) * 64];
-        }
+          for (int i = 0; i < 16; ++i) {
+            acc_k[dt][i] += theirs[(dt * 16 + i) * 64];
+            acc_v[dt][i] += theirs[((T::DT + dt) * 16 + i) * 64];
+          }
+      }
     }
   }
   if constexpr (PARTS) {
@@ -945,18 +1005,18 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       constexpr size_t kWaveFloats = (size_t)2 * T::DT * 1024;   // of one slot's accumulators
       const uint32_t item = (uint32_t)hk * (uint32_t)per_part + (uint32_t)bx;
       float *at = p.parts + ((size_t)item * p.parts_k * 4 + slot) * kWaveFloats + lane * 4;
-      if (rows_half == 0 && active) {
+      if (sharer == 0 && active) {
         bwd_leave_part<T::DT>(acc_k, at + (size_t)part * 4 * kWaveFloats);
         bwd_leave_part<T::DT>(acc_v, at + (size_t)part * 4 * kWaveFloats + kWaveFloats / 2);
       }
       if (!bwd_last_part(p.arrivals + item, nparts, (int *)lds)) return;
-      if (rows_half == 0 && active) {
+      if (sharer == 0 && active) {
         bwd_sum_parts<T::DT>(acc_k, at, 4 * kWaveFloats, nparts);
         bwd_sum_parts<T::DT>(acc_v, at + kWaveFloats / 2, 4 * kWaveFloats, nparts);
       }
     }
   }
-  if (rows_half == 0 && active && l32 < nrows) {
+  if (sharer == 0 && active && l32 < nrows) {
     const int64_t row = k0 + kbl * p.kbs + row0 + l32;
     bwd_store_rows<D, E>(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h, acc_k, p.scale, g32);
     bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, acc_v, 1.f, g32);
@@ -985,7 +1045,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   char *g_buf = lds + 4 * T::TILE_BYTES;               // [3] dO tiles
   char *p_buf = lds + 7 * T::TILE_BYTES;               // [2 tile parities][4 slots][2 halves][2][64 lanes] eight 16-bit values
   float *lse_s = (float *)(lds + 9 * T::TILE_BYTES);   // [3][64] log2-domain log-sum-exp of the tile's rows (index: the dO buffer's)
-  float *dlt_s = lse_s + 192;                          // [4][64] their delta (index: the Q buffer's)
+  float *dlt_s = lse_s + 192;                          // [4][64] their -delta (index: the Q buffer's)
   BwdPartRecord *part_s = (BwdPartRecord *)(dlt_s + 256);   // PARTS
 
   const int lane = threadIdx.x & 63;
@@ -1305,7 +1365,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
               for (int bq = 0; bq < 4; ++bq) {
                 const uint32_t w = pw[a >> 1][2 * (a & 1) + (bq >> 1)];
                 const float pv = (bq & 1) ? E::hi(w) : E::lo(w);
-                ed[4 * a + bq] = pv * (dp_prev[h][4 * a + bq] - d4[bq]);
+                ed[4 * a + bq] = pv * (dp_prev[h][4 * a + bq] + d4[bq]);
               }
             }
             short8v dlo, dhi;
@@ -1378,12 +1438,12 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   else run(std::integral_constant<int, 1>{});
 }
 
-// MANY: of the dK/dV kernel for head dims up to 64; SHARED: of the one for 128
-template <int D, typename E, bool PARTS_Q, bool PARTS_K, bool SHARED, bool MANY>
+// SHARED: k blocks of up to 64 keys (SPLIT of the dK/dV kernel for head dims up to 64)
+template <int D, typename E, bool PARTS_Q, bool PARTS_K, bool SHARED>
 int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   using T = BwdTile<D>;
   // LDS: the dQ kernel's three K and two V tiles; the dK/dV kernels' tile buffers, P records and row values
-  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? 9 * T::TILE_BYTES + 2048 : 6 * T::TILE_BYTES + 1536;
+  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? 9 * T::TILE_BYTES + 2048 : (SHARED ? 4 : 3) * (2 * T::TILE_BYTES + 512) + kBwdListCap * 8 + 16;
   if constexpr (lds_dkv > 48 * 1024) {
     static thread_local bool raised[kMaxDevices] = {};
     int dev = 0;
@@ -1392,7 +1452,7 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
     if (!raised[dev]) {
       const void *dkv = nullptr;
       if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>);
-      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K, MANY>);
+      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K, SHARED>);
       hipError_t e = hipFuncSetAttribute(dkv, hipFuncAttributeMaxDynamicSharedMemorySize, lds_dkv);
       if (e == hipSuccess)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&hbsa_bwd_dq_kernel<D, E, PARTS_Q>),
@@ -1407,30 +1467,23 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
   const dim3 kv_grid = bp.flat_grid ? dim3(k_wgs * (unsigned)nhead_k) : dim3(k_wgs, (unsigned)nhead_k);
   hipLaunchKernelGGL((hbsa_bwd_dq_kernel<D, E, PARTS_Q>), q_grid, dim3(kThreads), lds_dq, stream, bp);
   if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>), kv_grid, dim3(512), lds_dkv, stream, bp);
-  else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K, MANY>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
+  else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K, SHARED>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
 
-template <int D, typename E, bool SHARED, bool MANY>
+template <int D, typename E, bool SHARED>
 int launch_bwd_parts(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   const bool pq = bp.parts_q > 1, pk = bp.parts_k > 1;
-  if (pq && pk) return launch_bwd_kernels<D, E, true, true, SHARED, false>(bp, nhead_k, num_k_block, stream);
-  if (pk) return launch_bwd_kernels<D, E, false, true, SHARED, false>(bp, nhead_k, num_k_block, stream);
-  if (pq) return launch_bwd_kernels<D, E, true, false, SHARED, MANY>(bp, nhead_k, num_k_block, stream);
-  return launch_bwd_kernels<D, E, false, false, SHARED, MANY>(bp, nhead_k, num_k_block, stream);
+  if (pq && pk) return launch_bwd_kernels<D, E, true, true, SHARED>(bp, nhead_k, num_k_block, stream);
+  if (pk) return launch_bwd_kernels<D, E, false, true, SHARED>(bp, nhead_k, num_k_block, stream);
+  if (pq) return launch_bwd_kernels<D, E, true, false, SHARED>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_kernels<D, E, false, false, SHARED>(bp, nhead_k, num_k_block, stream);
 }
 template <int D, typename E>
 int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
-  if constexpr (D == 128) {
-    if (bp.kbs <= 2 * kWaveRows) return launch_bwd_parts<D, E, true, false>(bp, nhead_k, num_k_block, stream);
-    return launch_bwd_parts<D, E, false, false>(bp, nhead_k, num_k_block, stream);
-  } else {
-    // (the kernel for smaller head dims decides for itself whether wavefronts share a slot)
-    if constexpr (D == 32) return launch_bwd_parts<D, E, false, true>(bp, nhead_k, num_k_block, stream);
-    else if (bp.many) return launch_bwd_parts<D, E, false, true>(bp, nhead_k, num_k_block, stream);
-    else return launch_bwd_parts<D, E, false, false>(bp, nhead_k, num_k_block, stream);
-  }
+  if (bp.kbs <= 2 * kWaveRows) return launch_bwd_parts<D, E, true>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_parts<D, E, false>(bp, nhead_k, num_k_block, stream);
 }
 
 }  // namespace hbsa

@@ -333,7 +333,7 @@ struct BwdParams {
   char *dq, *dk, *dv;
   const float *lse;           // [total_q, nhead_q], contiguous
   // [nhead_q, total_q]: what the dQ kernel leaves for the dK/dV kernels, whose tiles are consecutive rows of one q head
-  float *delta;               // rowsum(dO * O)
+  float *delta;               // -rowsum(dO * O)
   float *lse2;                // lse * log2(e), +inf where lse is -inf
   const QBlockInfo *info;
   const uint32_t *bits;
@@ -353,7 +353,6 @@ struct BwdParams {
   float *parts;          // partial accumulators, shared by the two launches
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
   const int32_t *order_k;   // k blocks by falling number of query rows that can see them, nullptr: in their own order
-  int32_t many;          // host side only: more than 4.5 dK/dV items a CU (head dim 64)
 };
 
 // ---- Items of the kernels without a scheduler: geometry and kept blocks straight from the caller's arrays (bits == nullptr)

@@ -1550,7 +1550,6 @@ int hbsa_bwd(const void *q, const void *k, const void *v, const void *out, const
   bp.xcd_heads = bp.flat_grid && nhead_k % 8 == 0 ? 1 : 0;
   if (order_bytes(nhead_k, num_q_block, num_k_block) != 0)
     bp.order_k = (const int32_t *)((const char *)workspace + order_offset(nhead_k, num_q_block, num_k_block) + order_bytes(nhead_k, num_q_block, num_k_block));
-  bp.many = 2ll * num_k_block * bp.nsub_k * nhead_k > 9ll * device_cus();
   bp.c = softmax_scale * kLog2e;
   bp.scale = softmax_scale;
   hipStream_t st = (hipStream_t)stream;
