@@ -291,7 +291,7 @@ struct BwdCut {
 struct BwdPartRecord {
   float *first;        // partial accumulators of the item's first part
   uint32_t *counter;
-  int part, count, qb_first, r_first, r_last_end, unused;
+  int part, count;
 };
 // The dK/dV kernels' share of a k block: the (q block, q head of the group) pairs, q block by q block, from the first
 // q block with a row that sees a key of the workgroup (causal) to the sequence's last; one part's are [u0, u1) of them.
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
     bwd_store_rows<D, E>(p.dq + (int64_t)(inf.row_begin + row0 + l32) * p.dq_s + (int64_t)hq * p.dq_h, acc, p.scale, g32);
 }
 
-// ---- The tiles of a k block, for the dK/dV kernel of head dims up to 64: a list in LDS, made once by one wavefront.  (With every
+// ---- The tiles of a k block, for the dK/dV kernels: a list in LDS, made once by one wavefront.  (With every
 // wavefront walking the mask column tile by tile, a third of what it issued was that walk: 148 scalar instructions a tile.)
 constexpr int kBwdListCap = 256;   // entries: in-sequence position of the first row | q head of the group << 7, rows; a multiple of 64
 struct BwdTileRange {
@@ -1034,8 +1034,21 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
 // finishes tile t - 1 (whose dP it kept in registers) and forms dP of tile t, so one barrier per tile orders
 // everything.  Tiles go from global memory straight into LDS, stored once in the layout of BwdTile::swz_both,
 // and two tiles ahead (one workgroup per CU has nobody else to cover its waits for memory): four Q buffers
-// (tile t - 1 is still read while tile t + 2 arrives), three for dO, and with them three and four sets of the
+// (tile t - 1 is still read while tile t + 2 arrives), three for dO, and with them three sets of the
 // rows' log-sum-exp and delta, which wavefront 0 loads into LDS the same way.
+// What bounds it: the two roles' chains between two barriers, of which the matrix instructions are 2050 cycles a SIMD and tile, and what
+// a workgroup does before its first tile, which nothing covers (at 8192 tokens with a tenth kept 8.3 us of 28.5 for 8.3 tiles).  The tiles
+// come from a list (bwd_key_tiles; all eight wavefronts had walked the mask tile by tile), whose next entry is read while the barrier is waited for;
+// dP starts at -delta, and the rows' values and P are read by hand ahead of the transposed operands, behind which the compiler's own reads had
+// to wait for all of them.  Whole training calls, before and after: 1 x 32768 tokens, 8 heads, a tenth kept, 1255 -> 1211 us; 4 x 8192, 32
+// heads, 1858 -> 1825; 64-key blocks, 5 x 4491 .. 8593, 16 heads, 80-row blocks, 1418 -> 1315; 4 x 4096, 32 / 8 heads, 1080 -> 1029; 48-key blocks,
+// 5 x 823 .. 2209, 8 / 4 heads, 186 -> 173; few items, 6 x 1734, 2 heads, 128 -> 121.
+struct BwdListRecord {   // what a further chunk of the list is made from, kept in LDS: in registers over the tile loop it would spill
+  BwdTileRange range;
+  const uint32_t *column;
+  int bit, total;
+};
+constexpr int kBwdDkv8Lds = 9 * BwdTile<128>::TILE_BYTES + 1536 + kBwdListCap * 8 + sizeof(BwdListRecord) + sizeof(BwdPartRecord);
 template <typename E, bool PARTS, bool SHARED>
 __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   constexpr int D = 128;
@@ -1044,9 +1057,10 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   char *q_buf = lds;                                   // [4] Q tiles
   char *g_buf = lds + 4 * T::TILE_BYTES;               // [3] dO tiles
   char *p_buf = lds + 7 * T::TILE_BYTES;               // [2 tile parities][4 slots][2 halves][2][64 lanes] eight 16-bit values
-  float *lse_s = (float *)(lds + 9 * T::TILE_BYTES);   // [3][64] log2-domain log-sum-exp of the tile's rows (index: the dO buffer's)
-  float *dlt_s = lse_s + 192;                          // [4][64] their -delta (index: the Q buffer's)
-  BwdPartRecord *part_s = (BwdPartRecord *)(dlt_s + 256);   // PARTS
+  float *rows_s = (float *)(lds + 9 * T::TILE_BYTES);  // [3] of the dO buffer's rows: [64] log2-domain log-sum-exp, [64] -delta
+  u32x2 *list = (u32x2 *)(rows_s + 3 * 128);           // [kBwdListCap] tiles, see bwd_key_tiles
+  BwdListRecord *list_s = (BwdListRecord *)(list + kBwdListCap);
+  BwdPartRecord *part_s = (BwdPartRecord *)(list_s + 1);   // PARTS
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1080,11 +1094,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   const int kbl = kb - seq.kb0;
   const int k0 = seq.k0, klen = seq.k1 - k0;
   const bool fits = seq.fits(p, kb);
-  auto column_word = [&](int first, int low, int end) -> uint32_t {   // lane i: the word of q block first + i, if low <= first + i < end
-    const int g = first + lane;
-    return g >= low && g < end ? p.bits[((size_t)hk * p.nqb + g) * p.wpr + (kbl >> 5)] : 0u;
-  };
-  const uint32_t first_word = !PARTS && fits ? column_word(seq.qb1 - 64, seq.qb0, seq.qb1) : 0u;
+  const uint32_t *column = p.bits + (size_t)hk * p.nqb * p.wpr + (kbl >> 5);
+  const uint32_t first_word = !PARTS && fits ? bwd_column_word(p, column, seq.qb1 - 64, seq.qb0, seq.qb1, lane) : 0u;
   const int krows = min(p.kbs, klen - kbl * p.kbs);
   const int wg_row0 = sub * 4 * kWaveRows;                 // first key of the workgroup inside the block
   const int row0 = wg_row0 + key_slot * kWaveRows;
@@ -1112,77 +1123,40 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
 
-  const int qb_begin = seq.qb0;
-  int qb = qb_begin - 1, r = 0, qoff = 0, qb_end = seq.qb1;
-  int kept_base = qb_end;   // q blocks kept_base .. +63: those that keep this k block, not visited yet
-  int qb_low = qb_begin, r_end = p.ratio;   // the part's first q block, and the q block's heads that are the part's
-  uint64_t kept = 0;
-  QBlockInfo inf = {};
-  int seq_row0 = 0, seq_qlen = 0;   // first query row and query count of the sequence
-  if (qb_begin < qb_end) {
+  int shift = 0, total = 0;
+  BwdTileRange range = {seq.qb0, seq.qb0, seq.qb0, 0, 0, p.ratio, 0, 0};
+  if (seq.qb0 < seq.qb1) {
     if (!bwd_record_holds(seq, record)) {
       bwd_zero_keys<D>(p, seq, kb, sub, hk);
       return;
     }
-    inf.shift = __builtin_amdgcn_readlane((int)record, 5);
-    seq_row0 = __builtin_amdgcn_readlane((int)record, 0);
-    seq_qlen = klen - inf.shift;
+    shift = __builtin_amdgcn_readlane((int)record, 5);
+    range.row0 = __builtin_amdgcn_readlane((int)record, 0);
+    range.qlen = klen - shift;
+    range.qb_end = seq.qb1;
+    range.first_row = p.causal ? wg_first_key - shift : 0;
   }
   if (!fits) return;   // (a sequence without queries that lies outside of the tensors)
   if constexpr (PARTS) {
-    const BwdKeyPart share(p, qb_begin, qb_end, inf.shift, wg_first_key, part);
+    const BwdKeyPart share(p, seq.qb0, range.qb_end, shift, wg_first_key, part);
     if (part >= share.count) return;
     if (threadIdx.x == 0) {
       const size_t item = (size_t)hk * per_part + bx;
-      *part_s = BwdPartRecord{p.parts + item * p.parts_k * 8 * (T::DT * 1024), p.arrivals + item, part, share.count,
-                              share.qb_first, share.r_first, share.r_last_end, 0};
+      *part_s = BwdPartRecord{p.parts + item * p.parts_k * 8 * (T::DT * 1024), p.arrivals + item, part, share.count};
+    }
+    range.qb_low = share.qb_first;
+    range.r_first = share.r_first;
+    range.r_last_end = share.r_last_end;
+    range.qb_end = share.qb_last + 1;
+  }
+  if (PARTS || (range.qb_low < range.qb_end && range.qlen > 0)) {
+    if (threadIdx.x < 64) {
+      const int n = range.qlen > 0 ? bwd_key_tiles(p, range, column, kbl & 31, PARTS ? nullptr : &first_word, 0, list, lane) : 0;
+      if (lane == 0) *list_s = BwdListRecord{range, column, kbl & 31, n};
     }
     __syncthreads();
-    qb_low = share.qb_first;
-    qb_end = share.qb_last + 1;
-    kept_base = qb_end;
+    total = __builtin_amdgcn_readfirstlane(list_s->total);
   }
-  kept_base -= 64;
-  kept = __ballot(((PARTS ? column_word(kept_base, qb_low, qb_end) : first_word) >> (kbl & 31)) & 1u);
-  auto tile_reaches = [&]() {
-    return !p.causal || inf.q_pos + qoff + min(64, inf.rows - qoff) - 1 + inf.shift >= wg_first_key;
-  };
-  auto next_tile = [&]() -> bool {
-    for (;;) {
-      if (qb >= qb_begin) {
-        qoff += 64;
-        if (qoff >= inf.rows) { qoff = 0; ++r; }
-        if (r < (PARTS ? r_end : p.ratio)) {
-          if (tile_reaches()) return true;
-          continue;
-        }
-      }
-      while (kept == 0) {   // one load per 64 q blocks: lane i looks at q block kept_base + i; waited for here so that no other path waits
-        kept_base -= 64;
-        if (kept_base + 63 < qb_low) return false;
-        const uint32_t word = column_word(kept_base, qb_low, qb_end);
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        kept = __ballot((word >> (kbl & 31)) & 1u);
-      }
-      const int at = 63 - __builtin_clzll(kept);
-      qb = kept_base + at;
-      kept &= ~(1ull << at);
-      // the q block's geometry follows from the sequence's (no load on this path)
-      inf.q_pos = (qb - qb_begin) * p.qbs;
-      inf.row_begin = seq_row0 + inf.q_pos;
-      inf.rows = min(p.qbs, seq_qlen - inf.q_pos);
-      if (inf.rows <= 0) {   // more q blocks than the sequence has rows for: none is written into such a block's bit row
-        qb = qb_begin - 1;
-        continue;
-      }
-      r = 0;
-      if constexpr (PARTS) {
-        if (qb == __builtin_amdgcn_readfirstlane(part_s->qb_first)) r = __builtin_amdgcn_readfirstlane(part_s->r_first);
-        r_end = qb == qb_end - 1 ? __builtin_amdgcn_readfirstlane(part_s->r_last_end) : p.ratio;
-      }
-      qoff = -64;
-    }
-  };
   // A tile's 1024 chunks over eight wavefronts: wavefront w fills rows 4 * (8 * i + w) .. + 3 with load i
   // (i = 0, 1), lane l the 16 bytes at chunk position l % 16 of row l / 16 of those, which hold the
   // row's chunk (l % 16) ^ swz_both(row).
@@ -1192,19 +1166,18 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   const uint32_t q_addr = (uint32_t)(uintptr_t)HBSA_AS3(q_buf) + (uint32_t)wave * 1024u;
   const uint32_t g_addr = (uint32_t)(uintptr_t)HBSA_AS3(g_buf) + (uint32_t)wave * 1024u;
   const uint32_t q_voff = (uint32_t)ld_row * q_s32 + ld_chunk, g_voff = (uint32_t)ld_row * do_s32 + ld_chunk;   // of a full tile's first load
-  const uint32_t row_addr = (uint32_t)(uintptr_t)HBSA_AS3(lse_s);
+  const uint32_t row_addr = (uint32_t)(uintptr_t)HBSA_AS3(rows_s);
+  const char *q_base = p.q + (int64_t)range.row0 * p.q_s + (int64_t)hk * p.ratio * p.q_h, *g_base = p.dout + (int64_t)range.row0 * p.do_s + (int64_t)hk * p.ratio * p.do_h;
+  const int64_t row_base = (int64_t)hk * p.ratio * p.total_q + range.row0;
   // Loads of one tile per wavefront: two Q and two dO loads, and in wavefront 0 the two loads of the rows' values
-  auto fetch = [&](int qi, int gi) {   // the tile next_tile() has moved to, into Q buffer qi and dO buffer gi
-    const int valid = min(64, inf.rows - qoff);
-    const int64_t row_first = inf.row_begin + qoff;
-    const int hq = hk * p.ratio + r;
-    const char *qsrc = p.q + row_first * p.q_s + (int64_t)hq * p.q_h;
-    const char *gsrc = p.dout + row_first * p.do_s + (int64_t)hq * p.do_h;
+  auto fetch = [&](int qi, int gi, int pos, int valid, int r) {   // `valid` rows of q head r of the group, from in-sequence position pos on, into Q buffer qi and dO buffer gi
+    const char *qsrc = q_base + (uint64_t)(uint32_t)pos * q_s32 + (int64_t)r * p.q_h;
+    const char *gsrc = g_base + (uint64_t)(uint32_t)pos * do_s32 + (int64_t)r * p.do_h;
     if (valid == 64) {   // a full tile: the loads differ in their scalar base only
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        bwd_dma16(q_addr + (uint32_t)(qi * T::TILE_BYTES + i * 8 * 1024), qsrc + (int64_t)(32 * i) * p.q_s, q_voff);
-        bwd_dma16(g_addr + (uint32_t)(gi * T::TILE_BYTES + i * 8 * 1024), gsrc + (int64_t)(32 * i) * p.do_s, g_voff);
+        bwd_dma16(q_addr + (uint32_t)(qi * T::TILE_BYTES + i * 8 * 1024), qsrc + (uint64_t)(32u * i) * q_s32, q_voff);
+        bwd_dma16(g_addr + (uint32_t)(gi * T::TILE_BYTES + i * 8 * 1024), gsrc + (uint64_t)(32u * i) * do_s32, g_voff);
       }
     } else {
 #pragma unroll
@@ -1216,12 +1189,14 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     }
     if (wave == 0) {   // the rows' log-sum-exp and delta, one row per lane (rows past the block's end repeat its last row)
       const uint32_t rvoff = (uint32_t)min(lane, valid - 1) * 4u;
-      bwd_dma4(row_addr + (uint32_t)(gi * 256), p.lse2 + (int64_t)hq * p.total_q + row_first, rvoff);
-      bwd_dma4(row_addr + (uint32_t)(768 + qi * 256), p.delta + (int64_t)hq * p.total_q + row_first, rvoff);
+      const int64_t row_at = row_base + (int64_t)r * p.total_q + pos;
+      bwd_dma4(row_addr + (uint32_t)(gi * 512), p.lse2 + row_at, rvoff);
+      bwd_dma4(row_addr + (uint32_t)(gi * 512 + 256), p.delta + row_at, rvoff);
     }
   };
   // this lane's 2 x 16 bytes of a (tile parity, slot, half) record of P
   char *p_mine = p_buf + (size_t)slot * 4096 + lane * 16;
+  const uint32_t p_lds = (uint32_t)(uintptr_t)HBSA_AS3(p_mine);
 
   BwdOperandOffsets<D> off;
   off.init(lane);
@@ -1230,37 +1205,40 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   // register allocator keeps both roles' temporaries apart and spills.
   auto run = [&](auto role_) {
   constexpr int ROLE = decltype(role_)::value;
+  for (int chunk_base = 0; chunk_base < total;) {   // ---- chunks of the tile list (usually one)
+  const int entries = min(total - chunk_base, kBwdListCap);
   // Tiles are fetched two ahead: tile t lives in Q buffer t % 4 and dO buffer t % 3 (the dS wavefront still reads
   // Q of tile t - 1 in the iteration in which tile t + 2 arrives).
   int n_ahead = 0;                               // tiles fetched and not computed on yet
   int qi_f = 0, gi_f = 0;                        // buffers of the next fetch
   int fq_a = 0, fq_b = 0, va_a = 64, va_b = 64;  // first query position and row count of those tiles (a: the older)
-  bool more = next_tile();
-  auto issue = [&]() {   // fetches the tile next_tile() stands on and moves on
-    const int fq = inf.q_pos + qoff, va = min(64, inf.rows - qoff);
+  int at = 0;                                    // the next entry
+  auto issue = [&](u32x2 entry) {   // fetches the next tile, entry `at` of the list
+    const uint32_t y = (uint32_t)__builtin_amdgcn_readfirstlane((int)entry.y);
+    const int fq = __builtin_amdgcn_readfirstlane((int)entry.x), va = (int)(y & 127u);
     if (n_ahead == 0) { fq_a = fq; va_a = va; } else { fq_b = fq; va_b = va; }
-    fetch(qi_f, gi_f);
+    fetch(qi_f, gi_f, fq, va, (int)(y >> 7));
     qi_f = (qi_f + 1) & 3;
     gi_f = gi_f == 2 ? 0 : gi_f + 1;
     ++n_ahead;
-    more = next_tile();
+    ++at;
   };
-  if (more) issue();
-  if (more) issue();
+  issue(list[0]);
+  if (at < entries) issue(list[1]);
   // The resident operand has arrived before the loop begins (and with it the first two tiles, requested behind it): the
   // compiler counts only the loads it knows, and a wait of its own for it inside the loop would also wait for every tile under way.
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
   bool prev = false;        // the tile before the current one exists: its dK part is still due
   int qi = 0, gi = 0, par = 0;   // Q buffer, dO buffer and parity of the current tile
-  f32x16 dp_prev[NH];       // dS wavefront: dP of the previous tile
+  f32x16 dp_prev[NH];       // dS wavefront: dP - delta of the previous tile
 #pragma unroll
   for (int h = 0; h < NH; ++h)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dp_prev[h][i] = 0.f;
-  const int shift = inf.shift;
   while (n_ahead > 0 || prev) {
     const bool had = n_ahead > 0;
     const int first_q_pos = fq_a, valid = va_a;   // of the current tile (if any)
+    const u32x2 entry = list[min(at, kBwdListCap - 1)];   // (arrives while the barrier is waited for)
     // This wavefront's part of the current tile has landed; the loads of the tile after it (a wavefront's loads
     // return in order) may still be under way.
     if (n_ahead >= 2) {
@@ -1275,16 +1253,17 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       fq_a = fq_b;
       va_a = va_b;
       --n_ahead;
-      if (more) issue();   // two tiles ahead: the buffers it fills were last read an iteration ago
+      if (at < entries) issue(entry);   // two tiles ahead: the buffers it fills were last read an iteration ago
     }
     if (active) {
       // Operand reads are issued by hand (BwdOperandOffsets): PF reads of a pair of chains under way ahead of
       // their products, the transposing reads of a key group before the vector ALU work that precedes their
       // products.  The counts in the waits name only reads that every path issues.
-      constexpr int PF = 4, NC = NH * T::KSTEPS;
+      constexpr int PF = 4, NC = NH * T::KSTEPS, TR = 2 * T::DT;
       const uint32_t half_base = lds_base + (uint32_t)(first_row * T::RB);
+      const uint32_t v_at = row_addr + (uint32_t)(gi * 512 + first_row * 4 + 16 * g32);   // the rows' values
       short8v rb[PF];
-      short4v tb[2][2 * T::DT];
+      short4v tb[2][TR];
       if constexpr (ROLE == 0) {
         if (had) {   // ---- P wavefront, current tile
           const uint32_t q_t = half_base + (uint32_t)(q_now * T::TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
@@ -1306,20 +1285,26 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
             sv[i % NH] = E::mfma(rb[i % PF], frag[i / NH], sv[i % NH]);
             if constexpr (i + PF < NC) chain_read(std::integral_constant<int, i + PF>{});
           });
+          short8v lv[4];   // log-sum-exp of a half's rows
+          auto read_lse = [&](auto h_) {
+            static_for<0, 4>([&](auto a_) { lv[decltype(a_)::value] = lds_read_b128<128 * decltype(h_)::value + 32 * decltype(a_)::value>(v_at); });
+          };
+          read_lse(std::integral_constant<int, 0>{});
           bwd_issue_transposed<D, 0>(off, g_t, tb[0]);
-          bwd_issue_transposed<D, 1>(off, g_t, tb[1]);
           // edge: some row of the tile does not see some key of the wavefront (the causal diagonal, a slot with
           // fewer than 32 keys, a tile with fewer than 64 rows); elsewhere the per-element comparison and select
           // are left out.
           const bool edge = valid < 64 || (p.causal && wave_key_max - shift - first_q_pos > 0);
           auto half = [&](auto h_) {
             constexpr int h = decltype(h_)::value;
+            constexpr bool NEXT = h + 1 < NH;
+            asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(lv[0]), "+v"(lv[1]), "+v"(lv[2]), "+v"(lv[3]) : "n"(TR));
             float ep[16];
             auto form_p = [&](auto edge_) {
 #pragma unroll
               for (int a = 0; a < 4; ++a) {
                 const int rr0 = first_row + 32 * h + 8 * a + 4 * g32;
-                const f32x4 l4 = *(const f32x4 *)(lse_s + gi * 64 + rr0);
+                const f32x4 l4 = __builtin_bit_cast(f32x4, lv[a]);
 #pragma unroll
                 for (int bq = 0; bq < 4; ++bq) {
                   float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[h][4 * a + bq], p.c, -l4[bq]));
@@ -1330,16 +1315,17 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
             };
             if (edge) form_p(std::true_type{});
             else form_p(std::false_type{});
+            bwd_issue_transposed<D, 2 * h + 1>(off, g_t, tb[1]);
             short8v plo, phi;
             bwd_pack<E>(ep, plo, phi);
             *(short8v *)(p_mine + par * 16384 + h * 2048) = plo;
             *(short8v *)(p_mine + par * 16384 + h * 2048 + 1024) = phi;
-            bwd_wait_transposed<D, 2 * T::DT>(tb[0]);
+            if constexpr (NEXT) read_lse(std::integral_constant<int, h + 1>{});
+            bwd_wait_transposed<D, TR + (NEXT ? 4 : 0)>(tb[0]);
             bwd_transposed_products<D, E>(tb[0], plo, acc);
-            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 2>(off, g_t, tb[0]);
-            bwd_wait_transposed<D, (h + 1 < NH ? 2 * T::DT : 0)>(tb[1]);
+            if constexpr (NEXT) bwd_issue_transposed<D, 2>(off, g_t, tb[0]);
+            bwd_wait_transposed<D, (NEXT ? 4 + TR : 0)>(tb[1]);
             bwd_transposed_products<D, E>(tb[1], phi, acc);
-            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 3>(off, g_t, tb[1]);
           };
           static_for<0, NH>(half);
         }
@@ -1350,39 +1336,49 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
           rb[i % PF] = lds_read_b128<(i % NH) * 32 * T::RB>(off.rows[i / NH] + g_t);
         };
         if (prev) {   // ---- dS wavefront, the tile before: dS = P * (dP - delta), dK^T += Q^T dS
+          const uint32_t p_at = p_lds + (uint32_t)((par ^ 1) * 16384);
+          short8v pw[2];   // P of a half
+          auto read_p = [&](auto h_) {
+            pw[0] = lds_read_b128<2048 * decltype(h_)::value>(p_at);
+            pw[1] = lds_read_b128<2048 * decltype(h_)::value + 1024>(p_at);
+          };
+          read_p(std::integral_constant<int, 0>{});
           bwd_issue_transposed<D, 0>(off, q_t, tb[0]);
-          bwd_issue_transposed<D, 1>(off, q_t, tb[1]);
           auto half = [&](auto h_) {
             constexpr int h = decltype(h_)::value;
+            constexpr bool NEXT = h + 1 < NH;
+            asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(pw[0]), "+v"(pw[1]) : "n"(TR));
+            bwd_issue_transposed<D, 2 * h + 1>(off, q_t, tb[1]);
             float ed[16];
-            const u32x4 pw[2] = {*(const u32x4 *)(p_mine + (par ^ 1) * 16384 + h * 2048),
-                                 *(const u32x4 *)(p_mine + (par ^ 1) * 16384 + h * 2048 + 1024)};
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-              const int rr0 = first_row + 32 * h + 8 * a + 4 * g32;
-              const f32x4 d4 = *(const f32x4 *)(dlt_s + q_before * 64 + rr0);
-#pragma unroll
-              for (int bq = 0; bq < 4; ++bq) {
-                const uint32_t w = pw[a >> 1][2 * (a & 1) + (bq >> 1)];
-                const float pv = (bq & 1) ? E::hi(w) : E::lo(w);
-                ed[4 * a + bq] = pv * (dp_prev[h][4 * a + bq] + d4[bq]);
-              }
+            for (int i = 0; i < 16; ++i) {
+              const uint32_t w = __builtin_bit_cast(u32x4, pw[i >> 3])[(i & 7) >> 1];
+              ed[i] = ((i & 1) ? E::hi(w) : E::lo(w)) * dp_prev[h][i];
             }
             short8v dlo, dhi;
             bwd_pack<E>(ed, dlo, dhi);
-            bwd_wait_transposed<D, 2 * T::DT>(tb[0]);
+            if constexpr (NEXT) read_p(std::integral_constant<int, h + 1>{});
+            bwd_wait_transposed<D, TR + (NEXT ? 2 : 0)>(tb[0]);
             bwd_transposed_products<D, E>(tb[0], dlo, acc);
-            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 2>(off, q_t, tb[0]);
-            bwd_wait_transposed<D, (h + 1 < NH ? 2 * T::DT : 0)>(tb[1]);
+            if constexpr (NEXT) bwd_issue_transposed<D, 2>(off, q_t, tb[0]);
+            bwd_wait_transposed<D, (NEXT ? 2 + TR : 0)>(tb[1]);
             bwd_transposed_products<D, E>(tb[1], dhi, acc);
-            if constexpr (h + 1 < NH) bwd_issue_transposed<D, 3>(off, q_t, tb[1]);
           };
           static_for<0, NH>(half);
         }
-        if (had) {   // ---- dS wavefront, current tile: dP = dO V^T, kept for the next iteration
+        if (had) {   // ---- dS wavefront, current tile: dP - delta = dO V^T - delta, kept for the next iteration
+          short8v dl[NH][4];
+          static_for<0, 4 * NH>([&](auto i_) {
+            constexpr int i = decltype(i_)::value;
+            dl[i / 4][i % 4] = lds_read_b128<256 + 128 * (i / 4) + 32 * (i % 4)>(v_at);
+          });
           static_for<0, PF>(chain_read);
 #pragma unroll
-          for (int i = 0; i < 16; ++i) { dp_prev[0][i] = 0.f; dp_prev[NH - 1][i] = 0.f; }
+          for (int h = 0; h < NH; ++h) {
+            asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(dl[h][0]), "+v"(dl[h][1]), "+v"(dl[h][2]), "+v"(dl[h][3]) : "n"(PF));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dp_prev[h][i] = __builtin_bit_cast(f32x4, dl[h][i >> 2])[i & 3];
+          }
           static_for<0, NC>([&](auto i_) {
             constexpr int i = decltype(i_)::value;
             constexpr int ahead = (NC - 1 - i) < (PF - 1) ? (NC - 1 - i) : (PF - 1);
@@ -1397,6 +1393,18 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     qi = (qi + 1) & 3;
     gi = gi == 2 ? 0 : gi + 1;
     par ^= 1;
+  }
+  chunk_base += kBwdListCap;
+  if (chunk_base < total) {
+    __syncthreads();
+    if (wave == 0) {
+      int l = threadIdx.x;
+      asm volatile("" : "+v"(l));   // (nothing of this is to be prepared ahead of the tile loop)
+      const BwdListRecord rec = *list_s;
+      (void)bwd_key_tiles(p, rec.range, rec.column, rec.bit, nullptr, chunk_base, list, l);
+    }
+    __syncthreads();
+  }
   }
   if constexpr (SHARED) {   // the lower rows' sums go to the pair with the upper rows: [pair % 2][role][register][lane] floats
     // (the record of the part lies behind what this overwrites)
@@ -1443,7 +1451,7 @@ template <int D, typename E, bool PARTS_Q, bool PARTS_K, bool SHARED>
 int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   using T = BwdTile<D>;
   // LDS: the dQ kernel's three K and two V tiles; the dK/dV kernels' tile buffers, P records and row values
-  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? 9 * T::TILE_BYTES + 2048 : (SHARED ? 4 : 3) * (2 * T::TILE_BYTES + 512) + kBwdListCap * 8 + 16;
+  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? kBwdDkv8Lds : (SHARED ? 4 : 3) * (2 * T::TILE_BYTES + 512) + kBwdListCap * 8 + 16;
   if constexpr (lds_dkv > 48 * 1024) {
     static thread_local bool raised[kMaxDevices] = {};
     int dev = 0;

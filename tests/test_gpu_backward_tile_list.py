@@ -1,5 +1,5 @@
-"""The tile list of the dK/dV kernel for head dims up to 64: lists longer than a chunk of 256 tiles, odd numbers of tiles where
-two wavefronts take every other one (key blocks of up to 64 keys), tiles of fewer than 64 rows, key blocks whose last part is narrow."""
+"""The tile list of the dK/dV kernels: lists longer than a chunk of 256 tiles, odd numbers of tiles where
+two wavefronts take every other one (head dims up to 64, key blocks of up to 64 keys), tiles of fewer than 64 rows, key blocks whose last part is narrow."""
 import ctypes
 
 import pytest
@@ -45,7 +45,7 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("d", [32, 64, 128])
 @pytest.mark.parametrize("case", CASES, ids=[f"case{i}" for i in range(len(CASES))])
 def test_gradients_from_the_tile_list(case, d):
     q_lens, k_lens, hq, hk, qbs, kbs, keep, causal = case
