@@ -147,18 +147,66 @@ __device__ __forceinline__ void bwd_pack(const float *e, short8v &lo, short8v &h
   hi = __builtin_bit_cast(short8v, w[1]);
 }
 
-// accumulators [d, row = lane % 32] * f -> out row (16-bit), the forward's plain epilogue
-template <int D, typename E>
-__device__ __forceinline__ void bwd_store_rows(char *row_ptr, const f32x16 *acc, float f, int g32) {
+// ---- A wavefront's 32 rows, read and written four lanes to 64 contiguous bytes of a row (as the forward's q and output rows): the
+// operand layout has a lane on 16 bytes of every row of its own, the accumulators' on 8.  One instruction then covers 16 rows
+// in place of 32.  What it saves is a workgroup's beginning and end: of an item of eight tiles at D = 128 the stores alone were 3400 of 51000
+// cycles.  Training calls, one row a lane and as here: 4 x 8192 tokens, 32 heads of 128, a tenth kept, 1838 -> 1753 us; 64-key blocks, 5 x 4491 .. 8593,
+// 16 heads, 1309 -> 1263; 4 x 4096, 32 / 8, 1059 -> 1020; 7 x 2143, 32 / 4, 716 -> 693; head dim 64, 6 x 660, 32 heads, 111.5 -> 106.6.
+// Operand fragments of rows 0 .. 31 at `base` (those past `last` repeat it): lane i ends up with row i % 32, d = 16 * ks + 8 * (i / 32) .. + 7.
+// With h = bit 4 of the lane, load 2k takes row i % 16, load 2k + 1 row 16 + i % 16, both at bytes 64 * k + 32 * h + 16 * (i / 32);
+// then the h = 1 lanes of the first and the h = 0 lanes of the second trade places.
+template <int D>
+__device__ __forceinline__ void bwd_request_rows(const char *base, int64_t stride, int last, int lane, short8v *f) {
+  const int l16 = lane & 15, at = (lane & 16) * 2 + (lane >> 5) * 16;
+  const char *ra = base + min(l16, last) * stride + at, *rb = base + min(16 + l16, last) * stride + at;
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt)
+  for (int k = 0; k < BwdTile<D>::KSTEPS / 2; ++k) {
+    f[2 * k] = *(const short8v *)(ra + 64 * k);
+    f[2 * k + 1] = *(const short8v *)(rb + 64 * k);
+  }
+}
+template <int D>
+__device__ __forceinline__ void bwd_place_rows(short8v *f) {
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      u32x2 w;
-      w.x = E::pack2(acc[dt][4 * i4 + 0] * f, acc[dt][4 * i4 + 1] * f);
-      w.y = E::pack2(acc[dt][4 * i4 + 2] * f, acc[dt][4 * i4 + 3] * f);
-      *(u32x2 *)(row_ptr + (dt * 32 + 8 * i4 + 4 * g32) * 2) = w;
+  for (int k = 0; k < BwdTile<D>::KSTEPS / 2; ++k) {
+    u32x4 a = __builtin_bit_cast(u32x4, f[2 * k]), b = __builtin_bit_cast(u32x4, f[2 * k + 1]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const auto r = __builtin_amdgcn_permlane16_swap(a[j], b[j], false, false);
+      a[j] = r[0];
+      b[j] = r[1];
     }
+    f[2 * k] = __builtin_bit_cast(short8v, a);
+    f[2 * k + 1] = __builtin_bit_cast(short8v, b);
+  }
+}
+// accumulators [d, row = lane % 32] * f -> rows 0 .. n - 1 at `base` (16-bit): lanes i and i + 32 (one row) trade halves, then
+// lanes i and i + 16 the two 16-dim halves of a block
+template <int D, typename E>
+__device__ __forceinline__ void bwd_store_rows(char *base, int64_t stride, int n, const f32x16 *acc, float f, int lane) {
+  const int l16 = lane & 15;
+  char *row_x = base + l16 * stride + (lane & 16) * 2 + (lane >> 5) * 16, *row_y = row_x + 16 * stride;   // (a row past the end is not stored)
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt) {
+    u32x4 w[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      uint32_t x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = E::pack2(acc[dt][8 * m + 2 * j] * f, acc[dt][8 * m + 2 * j + 1] * f);
+      const auto r0 = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
+      const auto r1 = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
+      w[m] = u32x4{(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]};
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const auto r = __builtin_amdgcn_permlane16_swap(w[0][j], w[1][j], false, false);
+      w[0][j] = r[0];
+      w[1][j] = r[1];
+    }
+    if (l16 < n) *(u32x4 *)(row_x + dt * 64) = w[0];
+    if (16 + l16 < n) *(u32x4 *)(row_y + dt * 64) = w[1];
+  }
 }
 
 // The sequence a k block belongs to: what the dK/dV kernels need of it from the caller's arrays.  All three arrays are asked
@@ -381,16 +429,11 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   float row_lse = 0.f;
   const int my_row = inf.row_begin + min(row0 + l32, inf.rows - 1);
   if (active) {
-    const char *qrow = p.q + (int64_t)my_row * p.q_s + (int64_t)hq * p.q_h + g32 * 16;
-    const char *grow = p.dout + (int64_t)my_row * p.do_s + (int64_t)hq * p.do_h + g32 * 16;
-    const char *orow = p.out + (int64_t)my_row * p.o_s + (int64_t)hq * p.o_h + g32 * 16;
+    const int64_t first = inf.row_begin + row0;
     row_lse = p.lse[(int64_t)my_row * p.nhead_q + hq];
-#pragma unroll
-    for (int ks = 0; ks < T::KSTEPS; ++ks) {
-      dof[ks] = *(const short8v *)(grow + ks * 32);
-      of[ks] = *(const short8v *)(orow + ks * 32);
-      qf[ks] = *(const short8v *)(qrow + ks * 32);
-    }
+    bwd_request_rows<D>(p.dout + first * p.do_s + (int64_t)hq * p.do_h, p.do_s, nrows - 1, lane, dof);
+    bwd_request_rows<D>(p.out + first * p.o_s + (int64_t)hq * p.o_h, p.o_s, nrows - 1, lane, of);
+    bwd_request_rows<D>(p.q + first * p.q_s + (int64_t)hq * p.q_h, p.q_s, nrows - 1, lane, qf);
   } else {
 #pragma unroll
     for (int ks = 0; ks < T::KSTEPS; ++ks) { qf[ks] = short8v{0, 0, 0, 0, 0, 0, 0, 0}; dof[ks] = of[ks] = qf[ks]; }
@@ -482,6 +525,9 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
   float lse2 = INFINITY, dlt = 0.f;         // a row that takes no part gets P = exp2(-inf) = 0
   if (active) {
     lse2 = row_lse == -INFINITY ? INFINITY : row_lse * kLog2e;
+    bwd_place_rows<D>(dof);
+    bwd_place_rows<D>(of);
+    bwd_place_rows<D>(qf);
     // delta = sum over d of dO * O of the row: this lane's half of the head dim, then the other half's from lane + 32.
     // Every (row, q head) belongs to exactly one wavefront of this grid, which also leaves it for the dK/dV kernel.
 #pragma unroll
@@ -622,8 +668,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dq_kernel(BwdParams p) {
       if (active) bwd_sum_parts<T::DT>(acc, first, 4 * kWaveFloats, nparts);
     }
   }
-  if (active && l32 < nrows)
-    bwd_store_rows<D, E>(p.dq + (int64_t)(inf.row_begin + row0 + l32) * p.dq_s + (int64_t)hq * p.dq_h, acc, p.scale, g32);
+  if (active) bwd_store_rows<D, E>(p.dq + (int64_t)(inf.row_begin + row0) * p.dq_s + (int64_t)hq * p.dq_h, p.dq_s, nrows, acc, p.scale, lane);
 }
 
 // ---- The tiles of a k block, for the dK/dV kernels: a list in LDS, made once by one wavefront.  (With every
@@ -739,13 +784,9 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
 
   short8v kf[T::KSTEPS], vf[T::KSTEPS];   // K^T and V^T fragments: lane holds key l32, d = 16*ks + 8*g32 .. +7
   if (active && fits) {
-    const char *krow = p.k + (int64_t)(k0 + key_pos) * p.k_s + (int64_t)hk * p.k_h + g32 * 16;
-    const char *vrow = p.v + (int64_t)(k0 + key_pos) * p.v_s + (int64_t)hk * p.v_h + g32 * 16;
-#pragma unroll
-    for (int ks = 0; ks < T::KSTEPS; ++ks) {
-      kf[ks] = *(const short8v *)(krow + ks * 32);
-      vf[ks] = *(const short8v *)(vrow + ks * 32);
-    }
+    const int64_t first = k0 + kbl * p.kbs + row0;
+    bwd_request_rows<D>(p.k + first * p.k_s + (int64_t)hk * p.k_h, p.k_s, nrows - 1, lane, kf);
+    bwd_request_rows<D>(p.v + first * p.v_s + (int64_t)hk * p.v_h, p.v_s, nrows - 1, lane, vf);
   } else {
 #pragma unroll
     for (int ks = 0; ks < T::KSTEPS; ++ks) { kf[ks] = short8v{0, 0, 0, 0, 0, 0, 0, 0}; vf[ks] = kf[ks]; }
@@ -861,6 +902,10 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   issue();
   if (BUFS == 3 && more()) issue();
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the resident operands have arrived, and the tiles (see hbsa_bwd_dkv8_kernel)
+  if (chunk_base == 0) {
+    bwd_place_rows<D>(kf);
+    bwd_place_rows<D>(vf);
+  }
   while (n_ahead > 0) {
     const int first_q_pos = fq_a, valid = va_a;
     // This wavefront's part of the tile has landed; the loads of the tile after it (a wavefront's loads return in
@@ -1016,10 +1061,10 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
       }
     }
   }
-  if (sharer == 0 && active && l32 < nrows) {
-    const int64_t row = k0 + kbl * p.kbs + row0 + l32;
-    bwd_store_rows<D, E>(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h, acc_k, p.scale, g32);
-    bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, acc_v, 1.f, g32);
+  if (sharer == 0 && active) {
+    const int64_t row = k0 + kbl * p.kbs + row0;
+    bwd_store_rows<D, E>(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h, p.dk_s, nrows, acc_k, p.scale, lane);
+    bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, p.dv_s, nrows, acc_v, 1.f, lane);
   }
 }
 
@@ -1109,10 +1154,9 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   // key l32, d = 16 * ks + 8 * g32 .. + 7
   short8v frag[T::KSTEPS];
   if (active && fits) {
-    const char *src = role == 0 ? p.k + (int64_t)(k0 + key_pos) * p.k_s + (int64_t)hk * p.k_h
-                                : p.v + (int64_t)(k0 + key_pos) * p.v_s + (int64_t)hk * p.v_h;
-#pragma unroll
-    for (int ks = 0; ks < T::KSTEPS; ++ks) frag[ks] = *(const short8v *)(src + g32 * 16 + ks * 32);
+    const int64_t first = k0 + kbl * p.kbs + row0;
+    const int64_t stride = role == 0 ? p.k_s : p.v_s;
+    bwd_request_rows<D>((role == 0 ? p.k + (int64_t)hk * p.k_h : p.v + (int64_t)hk * p.v_h) + first * stride, stride, nrows - 1, lane, frag);
   } else {
 #pragma unroll
     for (int ks = 0; ks < T::KSTEPS; ++ks) frag[ks] = short8v{0, 0, 0, 0, 0, 0, 0, 0};
@@ -1228,6 +1272,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   // The resident operand has arrived before the loop begins (and with it the first two tiles, requested behind it): the
   // compiler counts only the loads it knows, and a wait of its own for it inside the loop would also wait for every tile under way.
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+  if (chunk_base == 0) bwd_place_rows<D>(frag);
   bool prev = false;        // the tile before the current one exists: its dK part is still due
   int qi = 0, gi = 0, par = 0;   // Q buffer, dO buffer and parity of the current tile
   f32x16 dp_prev[NH];       // dS wavefront: dP - delta of the previous tile
@@ -1267,8 +1312,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       if constexpr (ROLE == 0) {
         if (had) {   // ---- P wavefront, current tile
           const uint32_t q_t = half_base + (uint32_t)(q_now * T::TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
-          int first_vis = 0;   // rows of the tile from first_vis on see this lane's key (causal)
-          if (p.causal) first_vis = max(0, key_pos - shift - first_q_pos);
+          // rows first_vis .. left - 1 of the tile, counted from the lane's first, see its key
+          const int lane_row = first_row + 4 * g32, left = valid - lane_row, first_vis = p.causal ? key_pos - shift - first_q_pos - lane_row : -64;
           // S = Q K^T, the steps of the halves in turn (read i: half i % NH, step i / NH)
           auto chain_read = [&](auto i_) {
             constexpr int i = decltype(i_)::value;
@@ -1303,12 +1348,11 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
             auto form_p = [&](auto edge_) {
 #pragma unroll
               for (int a = 0; a < 4; ++a) {
-                const int rr0 = first_row + 32 * h + 8 * a + 4 * g32;
                 const f32x4 l4 = __builtin_bit_cast(f32x4, lv[a]);
 #pragma unroll
                 for (int bq = 0; bq < 4; ++bq) {
                   float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[h][4 * a + bq], p.c, -l4[bq]));
-                  if constexpr (decltype(edge_)::value) pv = (rr0 + bq >= first_vis && rr0 + bq < valid) ? pv : 0.f;   // rows past the block's end repeat its last row
+                  if constexpr (decltype(edge_)::value) pv = (32 * h + 8 * a + bq >= first_vis && 32 * h + 8 * a + bq < left) ? pv : 0.f;   // rows past the block's end repeat its last row
                   ep[4 * a + bq] = pv;
                 }
               }
@@ -1436,10 +1480,10 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       if (owner) bwd_sum_parts<T::DT>(acc, at, 8 * kWaveFloats, count);
     }
   }
-  if (owner && l32 < nrows) {
-    const int64_t row = k0 + kbl * p.kbs + row0 + l32;
-    if constexpr (ROLE == 0) bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, acc, 1.f, g32);
-    else bwd_store_rows<D, E>(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h, acc, p.scale, g32);
+  if (owner) {
+    const int64_t row = k0 + kbl * p.kbs + row0;
+    if constexpr (ROLE == 0) bwd_store_rows<D, E>(p.dv + row * p.dv_s + (int64_t)hk * p.dv_h, p.dv_s, nrows, acc, 1.f, lane);
+    else bwd_store_rows<D, E>(p.dk + row * p.dk_s + (int64_t)hk * p.dk_h, p.dk_s, nrows, acc, p.scale, lane);
   }
   };
   if (role == 0) run(std::integral_constant<int, 0>{});
