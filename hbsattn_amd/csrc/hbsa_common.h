@@ -84,6 +84,8 @@ struct PrepParams {
   int32_t nhead_k, weight_shift;
   int32_t *order_k;        // [nkb]: the k blocks by falling number of query rows that can see them
   int32_t weigh_k;         // 0: in their own order
+  uint32_t *copies;        // bit row copies of a split into nparts parts (at most 32), one array of bit rows after another; nparts 0: not split
+  int32_t nparts;
 };
 
 // Division by a launch constant d, exact for 0 <= n < 2^31: n / d == (n * m) >> s with

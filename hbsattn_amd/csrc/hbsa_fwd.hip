@@ -30,6 +30,18 @@
 
 namespace hbsa {
 
+// The k blocks [lo, hi) of a q block's own sequence (of n) that part `part` of nparts of a split sees
+struct PartRange {
+  int lo, hi;
+  __device__ __forceinline__ uint32_t word_mask(int j0) const {   // of blocks j0 .. j0 + 31
+    const int a = max(lo - j0, 0), b = min(hi - j0, 32);
+    return a < b ? (~0u << a) & (~0u >> (32 - b)) : 0u;
+  }
+};
+__device__ __forceinline__ PartRange part_range(int part, int nparts, int n) {
+  return {(int)((int64_t)part * n / nparts), (int)((int64_t)(part + 1) * n / nparts)};
+}
+
 // --------------------------------------------------------------------------------------
 // Pre-pass: one wavefront per (kv head, q block).
 // --------------------------------------------------------------------------------------
@@ -130,11 +142,18 @@ __global__ __launch_bounds__(kThreads) void hbsa_prep_kernel(PrepParams p) {
   uint32_t *row = p.bits + ((size_t)hk * p.nqb + g) * p.wpr;
   const uint8_t *m = p.mask + hk * p.ms_h + g * p.ms_q + kb0 * p.ms_k;
   const int nw64 = (nkb + 63) >> 6;
+  // (the copies of a split's parts: lane 2 * part + half has a word's share of the part)
+  const int part = lane >> 1, half = lane & 1;
+  PartRange mine = {0, 0};
+  if (part < p.nparts) mine = part_range(part, p.nparts, nkb);
+  uint32_t *copy = p.copies + ((size_t)part * p.nhead_k * p.nqb + (size_t)hk * p.nqb + g) * p.wpr + half;
   for (int w = 0; w < nw64; ++w) {
     const int j = w * 64 + lane;
     const bool keep = j < nvis && m[j * p.ms_k] != 0;
     const uint64_t bal = __ballot(keep);
-    if (lane < 2) row[2 * w + lane] = lane ? (uint32_t)(bal >> 32) : (uint32_t)bal;
+    const uint32_t word = half ? (uint32_t)(bal >> 32) : (uint32_t)bal;
+    if (lane < 2) row[2 * w + lane] = word;
+    if (part < p.nparts) copy[2 * w] = word & mine.word_mask(w * 64 + half * 32);
     kept_keys += __builtin_popcountll(bal) * p.kbs;
   }
   if (ORDER && lane == 0) {
@@ -302,8 +321,8 @@ __global__ __launch_bounds__(256) void hbsa_f32_stage_kernel(F32Tensor t, const 
   }
 }
 
-// Split over key blocks: bit row copy `part` keeps the k blocks [part * n / nparts, (part + 1) * n / nparts)
-// of a q block's own sequence (n = its k blocks).
+// Split over key blocks of a prepared mask: bit row copy `part` keeps its part_range.  A call that runs its own pre-pass has the
+// copies from that (a launch less: 2 us, 28.7 -> 26.4 and 252.8 -> 250.5 of two chunks of 2 and 4 heads).
 __global__ __launch_bounds__(256) void hbsa_split_bits_kernel(const uint32_t *bits, uint32_t *out, const QBlockInfo *info,
                                                               int nhead_k, int nqb, int wpr, int nparts) {
   const int64_t per_part = (int64_t)nhead_k * nqb * wpr;
@@ -312,14 +331,7 @@ __global__ __launch_bounds__(256) void hbsa_split_bits_kernel(const uint32_t *bi
   const int part = (int)(i / per_part);
   const int64_t r = i % per_part;
   const int w = (int)(r % wpr), qb = (int)((r / wpr) % nqb);
-  const int n = info[qb].nkblk;
-  const int lo = (int)((int64_t)part * n / nparts), hi = (int)((int64_t)(part + 1) * n / nparts);
-  uint32_t m = 0;
-  for (int b = 0; b < 32; ++b) {
-    const int j = w * 32 + b;
-    if (j >= lo && j < hi) m |= 1u << b;
-  }
-  out[i] = bits[r] & m;
+  out[i] = bits[r] & part_range(part, nparts, info[qb].nkblk).word_mask(w * 32);
 }
 
 // out[row, head, :] = sum over parts of exp(lse_part - lse) * partial, lse = log sum exp(lse_part);
@@ -742,13 +754,13 @@ void fill_shape(FwdParams &fp, int total_q, int total_k, int nhead_q, int nhead_
 
 template <int D, typename E, bool OUT32>
 int launch_fwd_split(FwdParams &fp, long long items, hipStream_t stream, char *area, int num_k_block, int total_q,
-                     int nhead_q) {
+                     int nhead_q, bool copies_made) {
   const int parts = fp.nparts;
   uint32_t *bit_copies = (uint32_t *)area;
   char *after_bits = area + split_bits_bytes(parts, fp.nhead_k, fp.nqb, num_k_block);
   fp.part_out = (float *)after_bits;
   fp.part_lse = (float *)(after_bits + split_out_bytes(parts, total_q, nhead_q, D));
-  {
+  if (!copies_made) {
     const int64_t n = (int64_t)fp.nhead_k * fp.nqb * fp.wpr * parts;
     hipLaunchKernelGGL(hbsa_split_bits_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, fp.bits,
                        bit_copies, fp.info, fp.nhead_k, fp.nqb, fp.wpr, parts);
@@ -770,8 +782,8 @@ int launch_fwd_split(FwdParams &fp, long long items, hipStream_t stream, char *a
 }
 
 template <int D, typename E, bool OUT32>
-int run_fwd(FwdParams &fp, long long items, hipStream_t stream, char *split_area, int num_k_block) {
-  if (fp.nparts > 1) return launch_fwd_split<D, E, OUT32>(fp, items, stream, split_area, num_k_block, fp.total_q, fp.nhead_q);
+int run_fwd(FwdParams &fp, long long items, hipStream_t stream, char *split_area, int num_k_block, bool copies_made) {
+  if (fp.nparts > 1) return launch_fwd_split<D, E, OUT32>(fp, items, stream, split_area, num_k_block, fp.total_q, fp.nhead_q, copies_made);
   return launch_fwd<D, E, OUT32>(fp, items, stream);
 }
 
@@ -1152,11 +1164,13 @@ inline bool items_weighed(long long pairs, int nhead_k, int batch, long long key
 constexpr long long kOrderedKBlocks = 8;
 // weigh_items, weigh_k_blocks: the orders are made by weight.  Without, they are there, too (last q blocks first, k blocks in their
 // own order): a run or a backward may follow on the workspace.
+// copies: where the bit row copies of a split into nparts go, or nullptr
 int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint8_t *block_mask,
                      const int32_t *q_block_to_batch, const int32_t *cu_num_q_block, const int32_t *cu_num_k_block,
                      void *workspace, size_t workspace_bytes, int32_t batch, int32_t nhead_k, int32_t num_q_block,
                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size, int32_t causal,
-                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream, bool weigh_items, bool weigh_k_blocks) {
+                     int32_t total_q, int32_t total_k, const int64_t *mask_strides, void *stream, bool weigh_items, bool weigh_k_blocks,
+                     uint32_t *copies = nullptr, int nparts = 0) {
   g_err[0] = 0;
   if (batch < 0 || num_q_block < 0 || num_k_block < 0 || total_q < 0 || total_k < 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
@@ -1187,6 +1201,8 @@ int prepare(const int32_t *cu_q_seqlens, const int32_t *cu_k_seqlens, const uint
   pp.causal = causal ? 1 : 0;
   pp.batch = batch; pp.nkb = num_k_block; pp.total_q = total_q; pp.total_k = total_k;
   pp.nhead_k = nhead_k;
+  pp.copies = copies;
+  pp.nparts = nparts;
   pp.weight_shift = weight_shift((long long)num_k_block * k_block_size);
   pp.order = nullptr;
   pp.order_k = nullptr;
@@ -1230,11 +1246,14 @@ int hbsa_fwd_run(const void *q, const void *k, const void *v, void *out, void *w
                           strides, stream);
 }
 
-int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, float *lse, const int64_t *lse_strides,
-                     void *workspace, size_t workspace_bytes, int32_t dtype, int32_t total_q, int32_t total_k,
-                     int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block, int32_t num_k_block,
-                     int32_t q_block_size, int32_t k_block_size, int32_t causal, float softmax_scale,
-                     const int64_t *strides, void *stream) {
+}  // extern "C"
+namespace {
+// hbsa_fwd_run_lse; copies_made: the pre-pass of the same call has left the bit row copies of a split
+int run_prepared(const void *q, const void *k, const void *v, void *out, float *lse, const int64_t *lse_strides,
+                 void *workspace, size_t workspace_bytes, int32_t dtype, int32_t total_q, int32_t total_k,
+                 int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block, int32_t num_k_block,
+                 int32_t q_block_size, int32_t k_block_size, int32_t causal, float softmax_scale,
+                 const int64_t *strides, void *stream, bool copies_made) {
   g_err[0] = 0;
   if (lse != nullptr && lse_strides == nullptr) return fail(HBSA_ERR_INVALID_ARGUMENT, "lse without lse_strides");
   if (total_q < 0 || total_k < 0) return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
@@ -1332,27 +1351,25 @@ int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, flo
       hipLaunchKernelGGL(hbsa_f32_stage_kernel, dim3(nb), dim3(256), 0, st, t, &fp.sched->in_mul[i], (uint32_t *)dst[i]);
     }
     switch (headdim) {
-      case 32: return run_fwd<32, ElemF16, true>(fp, items, st, split_area, num_k_block);
-      case 64: return run_fwd<64, ElemF16, true>(fp, items, st, split_area, num_k_block);
-      case 128: return run_fwd<128, ElemF16, true>(fp, items, st, split_area, num_k_block);
-      default: return run_fwd<256, ElemF16, true>(fp, items, st, split_area, num_k_block);
+      case 32: return run_fwd<32, ElemF16, true>(fp, items, st, split_area, num_k_block, copies_made);
+      case 64: return run_fwd<64, ElemF16, true>(fp, items, st, split_area, num_k_block, copies_made);
+      case 128: return run_fwd<128, ElemF16, true>(fp, items, st, split_area, num_k_block, copies_made);
+      default: return run_fwd<256, ElemF16, true>(fp, items, st, split_area, num_k_block, copies_made);
     }
   }
   const bool bf = dtype == HBSA_DTYPE_BF16;
   switch (headdim) {
-    case 32: return bf ? run_fwd<32, ElemBF16, false>(fp, items, st, split_area, num_k_block)
-                       : run_fwd<32, ElemF16, false>(fp, items, st, split_area, num_k_block);
-    case 64: return bf ? run_fwd<64, ElemBF16, false>(fp, items, st, split_area, num_k_block)
-                       : run_fwd<64, ElemF16, false>(fp, items, st, split_area, num_k_block);
-    case 128: return bf ? run_fwd<128, ElemBF16, false>(fp, items, st, split_area, num_k_block)
-                        : run_fwd<128, ElemF16, false>(fp, items, st, split_area, num_k_block);
-    default: return bf ? run_fwd<256, ElemBF16, false>(fp, items, st, split_area, num_k_block)
-                       : run_fwd<256, ElemF16, false>(fp, items, st, split_area, num_k_block);
+    case 32: return bf ? run_fwd<32, ElemBF16, false>(fp, items, st, split_area, num_k_block, copies_made)
+                       : run_fwd<32, ElemF16, false>(fp, items, st, split_area, num_k_block, copies_made);
+    case 64: return bf ? run_fwd<64, ElemBF16, false>(fp, items, st, split_area, num_k_block, copies_made)
+                       : run_fwd<64, ElemF16, false>(fp, items, st, split_area, num_k_block, copies_made);
+    case 128: return bf ? run_fwd<128, ElemBF16, false>(fp, items, st, split_area, num_k_block, copies_made)
+                        : run_fwd<128, ElemF16, false>(fp, items, st, split_area, num_k_block, copies_made);
+    default: return bf ? run_fwd<256, ElemBF16, false>(fp, items, st, split_area, num_k_block, copies_made)
+                       : run_fwd<256, ElemF16, false>(fp, items, st, split_area, num_k_block, copies_made);
   }
 }
 
-}  // extern "C"
-namespace {
 // hbsa_fwd, with the one-launch form allowed or not
 int fwd_call(const void *q, const void *k, const void *v, void *out, const int32_t *cu_q_seqlens,
              const int32_t *cu_k_seqlens, const uint8_t *block_mask, const int32_t *q_block_to_batch,
@@ -1429,13 +1446,23 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   const long long places = (long long)device_cus() * (shape.nw == 8 || headdim > 192 ? 1 : 2), items = (long long)nhead_k * num_q_block * shape.nsub;
   int rc = prepare(cu_q_seqlens, cu_k_seqlens, block_mask, q_block_to_batch, cu_num_q_block, cu_num_k_block, workspace, workspace_bytes,
                    batch, nhead_k, num_q_block, num_k_block, q_block_size, k_block_size, causal, total_q, total_k, strides + 8, stream,
-                   !split && !f32_exact && items > places && items <= 2ll * kStaticShare * places, false);
+                   !split && !f32_exact && items > places && items <= 2ll * kStaticShare * places, false,
+                   split && !f32_exact ? (uint32_t *)((char *)workspace + need) : nullptr, split && !f32_exact ? shape.split : 0);
   if (rc != 0) return rc;
-  return hbsa_fwd_run(q, k, v, out, workspace, workspace_bytes, dtype, total_q, total_k, nhead_q, nhead_k, headdim,
-                      num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, strides, stream);
+  return run_prepared(q, k, v, out, nullptr, nullptr, workspace, workspace_bytes, dtype, total_q, total_k, nhead_q, nhead_k, headdim,
+                      num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, strides, stream, split && !f32_exact);
 }
 }  // namespace
 extern "C" {
+
+int hbsa_fwd_run_lse(const void *q, const void *k, const void *v, void *out, float *lse, const int64_t *lse_strides,
+                     void *workspace, size_t workspace_bytes, int32_t dtype, int32_t total_q, int32_t total_k,
+                     int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block, int32_t num_k_block,
+                     int32_t q_block_size, int32_t k_block_size, int32_t causal, float softmax_scale,
+                     const int64_t *strides, void *stream) {
+  return run_prepared(q, k, v, out, lse, lse_strides, workspace, workspace_bytes, dtype, total_q, total_k, nhead_q, nhead_k, headdim,
+                      num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, strides, stream, false);
+}
 
 int hbsa_fwd(const void *q, const void *k, const void *v, void *out, const int32_t *cu_q_seqlens,
              const int32_t *cu_k_seqlens, const uint8_t *block_mask, const int32_t *q_block_to_batch,
