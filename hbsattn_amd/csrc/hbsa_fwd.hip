@@ -497,7 +497,7 @@ int device_cus() {
 // Split of `items` items over key blocks where `places` workgroups run at once: the number of parts with the fewest
 // rounds of the device, counted in whole items, plus what a part costs (its fp32 partial results are written and merged;
 // and the split is four launches in place of one).  A problem of chunks, its keys many times its queries, has items of
-// about one weight, so the count is right and parts of kChunkPartTiles tiles pay; elsewhere the causal order evens the rounds out and
+// about one weight, so the count is right and parts of kChunkPartTiles tiles pay from kChunkTiles on; elsewhere the causal order evens the rounds out and
 // only a problem that leaves places empty is split, into parts of kPartTiles.  (Tiles and not keys: a k block smaller than a
 // tile has one to itself.  All tiles of the problem stand in for an item's.)
 // Measured, us, before any of this (2 * CUs / items parts) and as here: chunks of 512 on 32000 keys, 32 / 8 heads of 128, one 113 ->
@@ -511,11 +511,15 @@ int device_cus() {
 // 80000 keys, 32 / 8 heads, 260 and 278), it is left alone.
 // (At most five items for eight places of workgroups of four: beyond that they stay one launch.  10 x 32 items of 256 dims on
 // 21000 keys, a place for 256 of them: split 1428, whole 932.)
-constexpr int kChunkPartTiles = 32, kPartTiles = 96, kLongPartTiles = 128;
+// Parts of 16 tiles in place of 32, once the merge and the copies cost what they do here: 100 drawn chunks of 23 .. 700 us 1.024 times as
+// fast (1 x 414 .. 829 on 7800 .. 9400 keys, 4 / 2 heads of 64, 39.6 -> 28.7; 1 x 92 .. 184 on 9000, 16 / 8 of 128, 57 -> 43; at worst
+// 27.7 -> 30.5, which had been 35.6 before those; 12 tiles: 1.027).  Below 64 tiles in all one launch is the faster (23.1 against 25.8).
+constexpr int kChunkTiles = 64, kChunkPartTiles = 16, kPartTiles = 96, kLongPartTiles = 128;
 int split_parts(long long items, int nw, int headdim, int num_k_block, int k_block_size, long long queries) {
   const long long tiles = (long long)num_k_block * ((k_block_size + kTileKeys - 1) / kTileKeys);
   const bool chunks = (long long)num_k_block * k_block_size >= 4 * queries;
   const long long cus = device_cus(), places = nw == 8 || headdim > 192 ? cus : 2 * cus;
+  if (chunks && tiles < kChunkTiles) return 1;
   if (items <= 0 || cus <= 0 || items > (nw == 8 ? (chunks ? 2 * cus : cus) : 5 * places / 8)) return 1;
   const long long most = std::min<long long>(std::min<long long>(32, num_k_block / 8), tiles / (chunks ? kChunkPartTiles : kPartTiles));
   const double part = 0.05 * std::max<double>((double)items, 1.0) / (double)places;
