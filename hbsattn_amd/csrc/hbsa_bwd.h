@@ -258,15 +258,15 @@ __device__ __forceinline__ bool bwd_record_holds(const BwdSequence &s, uint32_t 
 }
 // A sequence the pre-pass found not to fit the tensors (flagged q block records, no bit rows) takes no part: its keys get zero
 // gradients where they lie inside dk and dv.
-template <int D>
+template <int D, int KEYS>   // of a workgroup
 __device__ __forceinline__ void bwd_zero_keys(const BwdParams &p, const BwdSequence &s, int kb, int sub, int hk) {
   const int64_t k0 = s.k0, k1 = s.k1;
   const int kbl = kb - s.kb0;
   if (k0 < 0 || k1 <= k0 || kbl < 0) return;
-  const int64_t first = k0 + (int64_t)kbl * p.kbs + (int64_t)sub * 4 * kWaveRows;
+  const int64_t first = k0 + (int64_t)kbl * p.kbs + (int64_t)sub * KEYS;
   int64_t stop = k0 + (int64_t)(kbl + 1) * p.kbs;
   stop = stop < k1 ? stop : k1;
-  stop = stop < first + 4 * kWaveRows ? stop : first + 4 * kWaveRows;
+  stop = stop < first + KEYS ? stop : first + KEYS;
   stop = stop < p.total_k ? stop : (int64_t)p.total_k;
   const u32x4 zero = {0u, 0u, 0u, 0u};
   for (int64_t i = threadIdx.x; i < (stop - first) * (D / 8); i += blockDim.x) {
@@ -689,6 +689,7 @@ __device__ __forceinline__ uint32_t bwd_column_word(const BwdParams &p, const ui
 }
 // Entries [chunk_base, chunk_base + kBwdListCap) of the tiles, last q block first, to `list`; returns how many there are in all.
 // first: the column's words of the last 64 q blocks, if they have been loaded.
+template <int ROWS>   // of a tile
 __device__ __forceinline__ int bwd_key_tiles(const BwdParams &p, const BwdTileRange &t, const uint32_t *column, int bit, const uint32_t *first,
                                              int chunk_base, u32x2 *list, int lane) {
   int total = 0;
@@ -700,7 +701,7 @@ __device__ __forceinline__ int bwd_key_tiles(const BwdParams &p, const BwdTileRa
     if (((word >> bit) & 1u) != 0 && skip < rows) {
       r0 = qb == t.qb_low ? t.r_first : 0;
       heads = (qb == t.qb_end - 1 ? t.r_last_end : p.ratio) - r0;
-      tiles = ((rows + 63) >> 6) - (skip >> 6);
+      tiles = (rows + ROWS - 1) / ROWS - skip / ROWS;
     }
     const int mine = max(heads, 0) * tiles;
     int incl = mine;
@@ -711,8 +712,8 @@ __device__ __forceinline__ int bwd_key_tiles(const BwdParams &p, const BwdTileRa
     }
     int to = total + incl - mine - chunk_base;
     for (int r = r0; r < r0 + heads; ++r)
-      for (int row = skip & ~63; row < rows; row += 64, ++to)
-        if (tiles > 0 && to >= 0 && to < kBwdListCap) list[to] = u32x2{(uint32_t)(pos + row), (uint32_t)r << 7 | (uint32_t)min(64, rows - row)};
+      for (int row = skip & ~(ROWS - 1); row < rows; row += ROWS, ++to)
+        if (tiles > 0 && to >= 0 && to < kBwdListCap) list[to] = u32x2{(uint32_t)(pos + row), (uint32_t)r << 7 | (uint32_t)min(ROWS, rows - row)};
     total += __builtin_amdgcn_readlane(incl, 63);
   }
   return total;
@@ -804,7 +805,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   BwdTileRange range = {seq.qb0, seq.qb0, 0, 0, 0, p.ratio, 0, 0};
   if (seq.qb0 < seq.qb1) {
     if (!bwd_record_holds(seq, record)) {
-      bwd_zero_keys<D>(p, seq, kb, sub, hk);
+      bwd_zero_keys<D, 4 * kWaveRows>(p, seq, kb, sub, hk);
       return;
     }
     shift = __builtin_amdgcn_readlane((int)record, 5);
@@ -828,7 +829,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   const uint32_t *column = p.bits + (size_t)hk * p.nqb * p.wpr + (kbl >> 5);
   if (range.qb_low < range.qb_end && range.qlen > 0) {
     if (threadIdx.x < 64) {
-      const int n = bwd_key_tiles(p, range, column, kbl & 31, PARTS ? nullptr : &first_word, 0, list, lane);
+      const int n = bwd_key_tiles<64>(p, range, column, kbl & 31, PARTS ? nullptr : &first_word, 0, list, lane);
       if (lane == 0) *list_total = n;
     }
     __syncthreads();
@@ -1008,7 +1009,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   chunk_base += kBwdListCap;
   if (chunk_base < total) {
     __syncthreads();
-    if (threadIdx.x < 64) (void)bwd_key_tiles(p, range, column, kbl & 31, nullptr, chunk_base, list, lane);
+    if (threadIdx.x < 64) (void)bwd_key_tiles<64>(p, range, column, kbl & 31, nullptr, chunk_base, list, lane);
     __syncthreads();
   }
   }
@@ -1068,7 +1069,7 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
   }
 }
 
-// ---- dK, dV at D = 128: eight wavefronts in two roles -------------------------------------------------
+// ---- dK, dV at D = 128: wavefronts in two roles ---------------------------------------------------------
 // The kernel above would hold K^T, V^T and both accumulators of a wavefront in registers: 256 + 238 at
 // D = 128, one wavefront per SIMD.  Here two wavefronts share a 32-key slot (and a SIMD) and split the four
 // products between them, each with one operand and one accumulator in registers:
@@ -1086,39 +1087,45 @@ __global__ __launch_bounds__(kThreads, 2) void hbsa_bwd_dkv_kernel(BwdParams p) 
 // come from a list (bwd_key_tiles; all eight wavefronts had walked the mask tile by tile), whose next entry is read while the barrier is waited for;
 // dP starts at -delta, and the rows' values and P are read by hand ahead of the transposed operands, behind which the compiler's own reads had
 // to wait for all of them.  Whole training calls, before and after: 1 x 32768 tokens, 8 heads, a tenth kept, 1255 -> 1211 us; 4 x 8192, 32
-// heads, 1858 -> 1825; 64-key blocks, 5 x 4491 .. 8593, 16 heads, 80-row blocks, 1418 -> 1315; 4 x 4096, 32 / 8 heads, 1080 -> 1029; 48-key blocks,
+// heads, 1858 -> 1825; 64-key blocks (the shared form), 5 x 4491 .. 8593, 16 heads, 80-row blocks, 1418 -> 1315; 4 x 4096, 32 / 8 heads, 1080 -> 1029; 48-key blocks,
 // 5 x 823 .. 2209, 8 / 4 heads, 186 -> 173; few items, 6 x 1734, 2 heads, 128 -> 121.
+// Of the forms (which of them when, with figures: bwd_form) the narrow one has two workgroups a CU, of four wavefronts on 64 keys and tiles of 32
+// rows: 66 KB of LDS and 222 registers.  In the shared one eight wavefronts do as little between two barriers, 16 products each, and all wait.
 struct BwdListRecord {   // what a further chunk of the list is made from, kept in LDS: in registers over the tile loop it would spill
   BwdTileRange range;
   const uint32_t *column;
   int bit, total;
 };
-constexpr int kBwdDkv8Lds = 9 * BwdTile<128>::TILE_BYTES + 1536 + kBwdListCap * 8 + sizeof(BwdListRecord) + sizeof(BwdPartRecord);
-template <typename E, bool PARTS, bool SHARED>
-__global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
+// Its three forms (bwd_form): rows of a tile, wavefronts and keys of a workgroup
+constexpr int bwd_dkv8_rows(int form) { return form == kBwdNarrow ? 32 : 64; }
+constexpr int bwd_dkv8_threads(int form) { return form == kBwdNarrow ? 256 : 512; }
+constexpr int bwd_dkv8_lds(int form) {   // tiles, P records (two parities), the rows' values, the list
+  return 7 * bwd_dkv8_rows(form) * 256 + 2 * (bwd_dkv8_threads(form) / 128) * (form == kBwdWide ? 2 : 1) * 2048 + 1536 + kBwdListCap * 8 +
+         (int)sizeof(BwdListRecord) + (int)sizeof(BwdPartRecord);
+}
+template <typename E, bool PARTS, int FORM>
+__global__ __launch_bounds__(bwd_dkv8_threads(FORM), FORM == kBwdNarrow ? 2 : 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   constexpr int D = 128;
   using T = BwdTile<D>;
+  constexpr int ROWS = bwd_dkv8_rows(FORM), WAVES = bwd_dkv8_threads(FORM) / 64, SLOTS = WAVES / 2;
+  constexpr int NH = FORM == kBwdWide ? 2 : 1;       // 32-row halves of a tile a wavefront works on
+  constexpr int KEY_SLOTS = FORM == kBwdWide ? 4 : 2;
+  constexpr int TILE_BYTES = ROWS * T::RB, P_BYTES = SLOTS * NH * 2048;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   char *q_buf = lds;                                   // [4] Q tiles
-  char *g_buf = lds + 4 * T::TILE_BYTES;               // [3] dO tiles
-  char *p_buf = lds + 7 * T::TILE_BYTES;               // [2 tile parities][4 slots][2 halves][2][64 lanes] eight 16-bit values
-  float *rows_s = (float *)(lds + 9 * T::TILE_BYTES);  // [3] of the dO buffer's rows: [64] log2-domain log-sum-exp, [64] -delta
+  char *g_buf = lds + 4 * TILE_BYTES;                  // [3] dO tiles
+  char *p_buf = lds + 7 * TILE_BYTES;                  // [2 tile parities][SLOTS][NH][2][64 lanes] eight 16-bit values
+  float *rows_s = (float *)(p_buf + 2 * P_BYTES);      // [3] of the dO buffer's rows: [64] log2-domain log-sum-exp, [64] -delta
   u32x2 *list = (u32x2 *)(rows_s + 3 * 128);           // [kBwdListCap] tiles, see bwd_key_tiles
   BwdListRecord *list_s = (BwdListRecord *)(list + kBwdListCap);
   BwdPartRecord *part_s = (BwdPartRecord *)(list_s + 1);   // PARTS
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int slot = wave & 3, role = wave >> 2;   // pair of wavefronts; 0: the P wavefront, 1: the dS wavefront
-  // SHARED (k blocks of up to 64 keys): pairs 0 and 2, 1 and 3 work on the same 32 keys, the first ones on the upper 32 rows
-  // of every tile and the others on the lower ones, whose sums are added through LDS at the end.  Otherwise pair i has keys
-  // 32 i .. 32 i + 31 and both halves of the tile.
-  // (with four of eight wavefronts idle, dQ + dK/dV, 64-key blocks: 6 x 1500 .. 4000 tokens, 32 / 8 heads, 801 -> 678 us;
-  // 4 x 4096, 32 heads, 1013 -> 954; 48-key blocks, 4 x 2000 .. 6000, 16 heads, 848 -> 770.  With the chain in two accumulators
-  // 692, 971 and 785.)
-  constexpr int NH = SHARED ? 1 : 2;                 // halves of a tile a wavefront works on
-  const int key_slot = SHARED ? slot & 1 : slot;
-  const int first_row = SHARED ? 32 * (slot >> 1) : 0;   // ... from this row on
+  const int slot = wave % SLOTS, role = wave / SLOTS;   // pair of wavefronts; 0: the P wavefront, 1: the dS wavefront
+  // Pair i has keys 32 i .. 32 i + 31; in the shared form pairs 0 and 2, 1 and 3 have the same 32 keys, the first ones the upper 32 rows of
+  // every tile and the others the lower ones, whose sums are added through LDS at the end.
+  const int key_slot = slot % KEY_SLOTS, first_row = FORM == kBwdShared ? 32 * (slot / KEY_SLOTS) : 0;
   const int g32 = lane >> 5, l32 = lane & 31;
   int hk, bx;
   bwd_decode_grid(p, (unsigned)(p.nkb * p.nsub_k) * (PARTS ? (unsigned)p.parts_k : 1u), hk, bx);
@@ -1142,7 +1149,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   const uint32_t *column = p.bits + (size_t)hk * p.nqb * p.wpr + (kbl >> 5);
   const uint32_t first_word = !PARTS && fits ? bwd_column_word(p, column, seq.qb1 - 64, seq.qb0, seq.qb1, lane) : 0u;
   const int krows = min(p.kbs, klen - kbl * p.kbs);
-  const int wg_row0 = sub * 4 * kWaveRows;                 // first key of the workgroup inside the block
+  const int wg_row0 = sub * KEY_SLOTS * kWaveRows;             // first key of the workgroup inside the block
   const int row0 = wg_row0 + key_slot * kWaveRows;
   const int nrows = min(kWaveRows, krows - row0);
   const bool active = nrows > 0;
@@ -1171,7 +1178,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   BwdTileRange range = {seq.qb0, seq.qb0, seq.qb0, 0, 0, p.ratio, 0, 0};
   if (seq.qb0 < seq.qb1) {
     if (!bwd_record_holds(seq, record)) {
-      bwd_zero_keys<D>(p, seq, kb, sub, hk);
+      bwd_zero_keys<D, KEY_SLOTS * kWaveRows>(p, seq, kb, sub, hk);
       return;
     }
     shift = __builtin_amdgcn_readlane((int)record, 5);
@@ -1186,7 +1193,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     if (part >= share.count) return;
     if (threadIdx.x == 0) {
       const size_t item = (size_t)hk * per_part + bx;
-      *part_s = BwdPartRecord{p.parts + item * p.parts_k * 8 * (T::DT * 1024), p.arrivals + item, part, share.count};
+      *part_s = BwdPartRecord{p.parts + item * p.parts_k * WAVES * (T::DT * 1024), p.arrivals + item, part, share.count};
     }
     range.qb_low = share.qb_first;
     range.r_first = share.r_first;
@@ -1195,16 +1202,16 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   }
   if (PARTS || (range.qb_low < range.qb_end && range.qlen > 0)) {
     if (threadIdx.x < 64) {
-      const int n = range.qlen > 0 ? bwd_key_tiles(p, range, column, kbl & 31, PARTS ? nullptr : &first_word, 0, list, lane) : 0;
+      const int n = range.qlen > 0 ? bwd_key_tiles<ROWS>(p, range, column, kbl & 31, PARTS ? nullptr : &first_word, 0, list, lane) : 0;
       if (lane == 0) *list_s = BwdListRecord{range, column, kbl & 31, n};
     }
     __syncthreads();
     total = __builtin_amdgcn_readfirstlane(list_s->total);
   }
-  // A tile's 1024 chunks over eight wavefronts: wavefront w fills rows 4 * (8 * i + w) .. + 3 with load i
+  // A tile's chunks over the wavefronts: wavefront w fills rows 4 * (WAVES * i + w) .. + 3 with load i
   // (i = 0, 1), lane l the 16 bytes at chunk position l % 16 of row l / 16 of those, which hold the
   // row's chunk (l % 16) ^ swz_both(row).
-  const int ld_row = 4 * wave + (lane >> 4);                              // + 32 * i
+  const int ld_row = 4 * wave + (lane >> 4);                              // + 4 * WAVES * i
   const uint32_t ld_chunk = (uint32_t)(((lane & 15) ^ T::swz_both(ld_row & 15)) * 16);
   const uint32_t q_s32 = (uint32_t)p.q_s, do_s32 = (uint32_t)p.do_s;      // the host checks that they fit
   const uint32_t q_addr = (uint32_t)(uintptr_t)HBSA_AS3(q_buf) + (uint32_t)wave * 1024u;
@@ -1217,18 +1224,18 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   auto fetch = [&](int qi, int gi, int pos, int valid, int r) {   // `valid` rows of q head r of the group, from in-sequence position pos on, into Q buffer qi and dO buffer gi
     const char *qsrc = q_base + (uint64_t)(uint32_t)pos * q_s32 + (int64_t)r * p.q_h;
     const char *gsrc = g_base + (uint64_t)(uint32_t)pos * do_s32 + (int64_t)r * p.do_h;
-    if (valid == 64) {   // a full tile: the loads differ in their scalar base only
+    if (valid == ROWS) {   // a full tile: the loads differ in their scalar base only
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        bwd_dma16(q_addr + (uint32_t)(qi * T::TILE_BYTES + i * 8 * 1024), qsrc + (uint64_t)(32u * i) * q_s32, q_voff);
-        bwd_dma16(g_addr + (uint32_t)(gi * T::TILE_BYTES + i * 8 * 1024), gsrc + (uint64_t)(32u * i) * do_s32, g_voff);
+        bwd_dma16(q_addr + (uint32_t)(qi * TILE_BYTES + i * WAVES * 1024), qsrc + (uint64_t)(4u * WAVES * i) * q_s32, q_voff);
+        bwd_dma16(g_addr + (uint32_t)(gi * TILE_BYTES + i * WAVES * 1024), gsrc + (uint64_t)(4u * WAVES * i) * do_s32, g_voff);
       }
     } else {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const uint32_t rr = (uint32_t)min(ld_row + 32 * i, valid - 1);   // rows past the block's end repeat its last row
-        bwd_dma16(q_addr + (uint32_t)(qi * T::TILE_BYTES + i * 8 * 1024), qsrc, rr * q_s32 + ld_chunk);
-        bwd_dma16(g_addr + (uint32_t)(gi * T::TILE_BYTES + i * 8 * 1024), gsrc, rr * do_s32 + ld_chunk);
+        const uint32_t rr = (uint32_t)min(ld_row + 4 * WAVES * i, valid - 1);   // rows past the block's end repeat its last row
+        bwd_dma16(q_addr + (uint32_t)(qi * TILE_BYTES + i * WAVES * 1024), qsrc, rr * q_s32 + ld_chunk);
+        bwd_dma16(g_addr + (uint32_t)(gi * TILE_BYTES + i * WAVES * 1024), gsrc, rr * do_s32 + ld_chunk);
       }
     }
     if (wave == 0) {   // the rows' log-sum-exp and delta, one row per lane (rows past the block's end repeat its last row)
@@ -1239,7 +1246,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
     }
   };
   // this lane's 2 x 16 bytes of a (tile parity, slot, half) record of P
-  char *p_mine = p_buf + (size_t)slot * 4096 + lane * 16;
+  char *p_mine = p_buf + (size_t)slot * (NH * 2048) + lane * 16;
   const uint32_t p_lds = (uint32_t)(uintptr_t)HBSA_AS3(p_mine);
 
   BwdOperandOffsets<D> off;
@@ -1255,7 +1262,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   // Q of tile t - 1 in the iteration in which tile t + 2 arrives).
   int n_ahead = 0;                               // tiles fetched and not computed on yet
   int qi_f = 0, gi_f = 0;                        // buffers of the next fetch
-  int fq_a = 0, fq_b = 0, va_a = 64, va_b = 64;  // first query position and row count of those tiles (a: the older)
+  int fq_a = 0, fq_b = 0, va_a = ROWS, va_b = ROWS;  // first query position and row count of those tiles (a: the older)
   int at = 0;                                    // the next entry
   auto issue = [&](u32x2 entry) {   // fetches the next tile, entry `at` of the list
     const uint32_t y = (uint32_t)__builtin_amdgcn_readfirstlane((int)entry.y);
@@ -1311,7 +1318,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       short4v tb[2][TR];
       if constexpr (ROLE == 0) {
         if (had) {   // ---- P wavefront, current tile
-          const uint32_t q_t = half_base + (uint32_t)(q_now * T::TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
+          const uint32_t q_t = half_base + (uint32_t)(q_now * TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * TILE_BYTES);
           // rows first_vis .. left - 1 of the tile, counted from the lane's first, see its key
           const int lane_row = first_row + 4 * g32, left = valid - lane_row, first_vis = p.causal ? key_pos - shift - first_q_pos - lane_row : -64;
           // S = Q K^T, the steps of the halves in turn (read i: half i % NH, step i / NH)
@@ -1339,7 +1346,7 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
           // edge: some row of the tile does not see some key of the wavefront (the causal diagonal, a slot with
           // fewer than 32 keys, a tile with fewer than 64 rows); elsewhere the per-element comparison and select
           // are left out.
-          const bool edge = valid < 64 || (p.causal && wave_key_max - shift - first_q_pos > 0);
+          const bool edge = valid < ROWS || (p.causal && wave_key_max - shift - first_q_pos > 0);
           auto half = [&](auto h_) {
             constexpr int h = decltype(h_)::value;
             constexpr bool NEXT = h + 1 < NH;
@@ -1362,8 +1369,8 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
             bwd_issue_transposed<D, 2 * h + 1>(off, g_t, tb[1]);
             short8v plo, phi;
             bwd_pack<E>(ep, plo, phi);
-            *(short8v *)(p_mine + par * 16384 + h * 2048) = plo;
-            *(short8v *)(p_mine + par * 16384 + h * 2048 + 1024) = phi;
+            *(short8v *)(p_mine + par * P_BYTES + h * 2048) = plo;
+            *(short8v *)(p_mine + par * P_BYTES + h * 2048 + 1024) = phi;
             if constexpr (NEXT) read_lse(std::integral_constant<int, h + 1>{});
             bwd_wait_transposed<D, TR + (NEXT ? 4 : 0)>(tb[0]);
             bwd_transposed_products<D, E>(tb[0], plo, acc);
@@ -1374,13 +1381,13 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
           static_for<0, NH>(half);
         }
       } else {
-        const uint32_t q_t = half_base + (uint32_t)(q_before * T::TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * T::TILE_BYTES);
+        const uint32_t q_t = half_base + (uint32_t)(q_before * TILE_BYTES), g_t = half_base + (uint32_t)((4 + gi) * TILE_BYTES);
         auto chain_read = [&](auto i_) {   // dP = dO V^T of both halves of the current tile, as above
           constexpr int i = decltype(i_)::value;
           rb[i % PF] = lds_read_b128<(i % NH) * 32 * T::RB>(off.rows[i / NH] + g_t);
         };
         if (prev) {   // ---- dS wavefront, the tile before: dS = P * (dP - delta), dK^T += Q^T dS
-          const uint32_t p_at = p_lds + (uint32_t)((par ^ 1) * 16384);
+          const uint32_t p_at = p_lds + (uint32_t)((par ^ 1) * P_BYTES);
           short8v pw[2];   // P of a half
           auto read_p = [&](auto h_) {
             pw[0] = lds_read_b128<2048 * decltype(h_)::value>(p_at);
@@ -1445,12 +1452,12 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
       int l = threadIdx.x;
       asm volatile("" : "+v"(l));   // (nothing of this is to be prepared ahead of the tile loop)
       const BwdListRecord rec = *list_s;
-      (void)bwd_key_tiles(p, rec.range, rec.column, rec.bit, nullptr, chunk_base, list, l);
+      (void)bwd_key_tiles<ROWS>(p, rec.range, rec.column, rec.bit, nullptr, chunk_base, list, l);
     }
     __syncthreads();
   }
   }
-  if constexpr (SHARED) {   // the lower rows' sums go to the pair with the upper rows: [pair % 2][role][register][lane] floats
+  if constexpr (FORM == kBwdShared) {   // the lower rows' sums go to the pair with the upper rows: [pair % 2][role][register][lane] floats
     // (the record of the part lies behind what this overwrites)
     __syncthreads();
     float *xch = (float *)lds + (size_t)(key_slot * 2 + ROLE) * (T::DT * 16) * 64 + lane;
@@ -1468,16 +1475,16 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
         for (int i = 0; i < 16; ++i) acc[dt][i] += xch[(dt * 16 + i) * 64];
     }
   }
-  const bool owner = active && (!SHARED || slot < 2);   // of the sums of 32 keys
+  const bool owner = active && slot < KEY_SLOTS;   // of the sums of 32 keys
   if constexpr (PARTS) {
     const BwdPartRecord rec = *part_s;
     const int count = __builtin_amdgcn_readfirstlane(rec.count);
     if (count > 1) {
       constexpr size_t kWaveFloats = (size_t)T::DT * 1024;   // of one wavefront's accumulators
       float *at = rec.first + (size_t)wave * kWaveFloats + lane * 4;
-      if (owner) bwd_leave_part<T::DT>(acc, at + (size_t)rec.part * 8 * kWaveFloats);
+      if (owner) bwd_leave_part<T::DT>(acc, at + (size_t)rec.part * WAVES * kWaveFloats);
       if (!bwd_last_part(rec.counter, count, (int *)lds)) return;
-      if (owner) bwd_sum_parts<T::DT>(acc, at, 8 * kWaveFloats, count);
+      if (owner) bwd_sum_parts<T::DT>(acc, at, WAVES * kWaveFloats, count);
     }
   }
   if (owner) {
@@ -1490,12 +1497,12 @@ __global__ __launch_bounds__(512, 1) void hbsa_bwd_dkv8_kernel(BwdParams p) {
   else run(std::integral_constant<int, 1>{});
 }
 
-// SHARED: k blocks of up to 64 keys (SPLIT of the dK/dV kernel for head dims up to 64)
-template <int D, typename E, bool PARTS_Q, bool PARTS_K, bool SHARED>
+// FORM: of the dK/dV kernel (kBwdShared is SPLIT at head dims up to 64)
+template <int D, typename E, bool PARTS_Q, bool PARTS_K, int FORM>
 int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   using T = BwdTile<D>;
   // LDS: the dQ kernel's three K and two V tiles; the dK/dV kernels' tile buffers, P records and row values
-  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? kBwdDkv8Lds : (SHARED ? 4 : 3) * (2 * T::TILE_BYTES + 512) + kBwdListCap * 8 + 16;
+  constexpr int lds_dq = 5 * T::TILE_BYTES, lds_dkv = D == 128 ? bwd_dkv8_lds(FORM) : (FORM == kBwdShared ? 4 : 3) * (2 * T::TILE_BYTES + 512) + kBwdListCap * 8 + 16;
   if constexpr (lds_dkv > 48 * 1024) {
     static thread_local bool raised[kMaxDevices] = {};
     int dev = 0;
@@ -1503,8 +1510,8 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
       return fail(HBSA_ERR_UNSUPPORTED, "no current device, or device index above %d", kMaxDevices - 1);
     if (!raised[dev]) {
       const void *dkv = nullptr;
-      if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>);
-      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K, SHARED>);
+      if constexpr (D == 128) dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv8_kernel<E, PARTS_K, FORM>);
+      else dkv = reinterpret_cast<const void *>(&hbsa_bwd_dkv_kernel<D, E, PARTS_K, FORM == kBwdShared>);
       hipError_t e = hipFuncSetAttribute(dkv, hipFuncAttributeMaxDynamicSharedMemorySize, lds_dkv);
       if (e == hipSuccess)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&hbsa_bwd_dq_kernel<D, E, PARTS_Q>),
@@ -1518,24 +1525,26 @@ int launch_bwd_kernels(const BwdParams &bp, int nhead_k, int num_k_block, hipStr
   const dim3 q_grid = bp.flat_grid ? dim3(q_wgs * (unsigned)nhead_k) : dim3(q_wgs, (unsigned)nhead_k);
   const dim3 kv_grid = bp.flat_grid ? dim3(k_wgs * (unsigned)nhead_k) : dim3(k_wgs, (unsigned)nhead_k);
   hipLaunchKernelGGL((hbsa_bwd_dq_kernel<D, E, PARTS_Q>), q_grid, dim3(kThreads), lds_dq, stream, bp);
-  if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K, SHARED>), kv_grid, dim3(512), lds_dkv, stream, bp);
-  else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K, SHARED>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
+  if constexpr (D == 128) hipLaunchKernelGGL((hbsa_bwd_dkv8_kernel<E, PARTS_K, FORM>), kv_grid, dim3(bwd_dkv8_threads(FORM)), lds_dkv, stream, bp);
+  else hipLaunchKernelGGL((hbsa_bwd_dkv_kernel<D, E, PARTS_K, FORM == kBwdShared>), kv_grid, dim3(kThreads), lds_dkv, stream, bp);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
 
-template <int D, typename E, bool SHARED>
+template <int D, typename E, int FORM>
 int launch_bwd_parts(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
   const bool pq = bp.parts_q > 1, pk = bp.parts_k > 1;
-  if (pq && pk) return launch_bwd_kernels<D, E, true, true, SHARED>(bp, nhead_k, num_k_block, stream);
-  if (pk) return launch_bwd_kernels<D, E, false, true, SHARED>(bp, nhead_k, num_k_block, stream);
-  if (pq) return launch_bwd_kernels<D, E, true, false, SHARED>(bp, nhead_k, num_k_block, stream);
-  return launch_bwd_kernels<D, E, false, false, SHARED>(bp, nhead_k, num_k_block, stream);
+  if (pq && pk) return launch_bwd_kernels<D, E, true, true, FORM>(bp, nhead_k, num_k_block, stream);
+  if (pk) return launch_bwd_kernels<D, E, false, true, FORM>(bp, nhead_k, num_k_block, stream);
+  if (pq) return launch_bwd_kernels<D, E, true, false, FORM>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_kernels<D, E, false, false, FORM>(bp, nhead_k, num_k_block, stream);
 }
 template <int D, typename E>
 int launch_bwd(const BwdParams &bp, int nhead_k, int num_k_block, hipStream_t stream) {
-  if (bp.kbs <= 2 * kWaveRows) return launch_bwd_parts<D, E, true>(bp, nhead_k, num_k_block, stream);
-  return launch_bwd_parts<D, E, false>(bp, nhead_k, num_k_block, stream);
+  if constexpr (D == 128)
+    if (bp.form_k == kBwdNarrow) return launch_bwd_parts<D, E, kBwdNarrow>(bp, nhead_k, num_k_block, stream);
+  if (bp.form_k == kBwdShared) return launch_bwd_parts<D, E, kBwdShared>(bp, nhead_k, num_k_block, stream);
+  return launch_bwd_parts<D, E, kBwdWide>(bp, nhead_k, num_k_block, stream);
 }
 
 }  // namespace hbsa

@@ -344,7 +344,7 @@ struct BwdParams {
   int32_t nqb, nkb, xcd_heads, batch, ratio, nhead_q, qbs, kbs, wpr, causal;   // xcd_heads: see the dK/dV kernels
   int32_t total_k;
   int32_t wps, nsub;     // q side: wave slots per q head and workgroups per (kv head, q block), as in the forward
-  int32_t nsub_k;        // k side: workgroups per (kv head, k block) = ceil(k_block_size / 128)
+  int32_t nsub_k;        // k side: workgroups per (kv head, k block), of 128 keys or (form_k == kBwdNarrow) 64
   float c;               // softmax_scale * log2(e), signed
   float scale;
   // Items cut into parts (see BwdCut): at most parts_q k block ranges a dQ item, of min_blocks_q k blocks at least, and parts_k
@@ -355,7 +355,9 @@ struct BwdParams {
   float *parts;          // partial accumulators, shared by the two launches
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
   const int32_t *order_k;   // k blocks by falling number of query rows that can see them, nullptr: in their own order
+  int32_t form_k;         // of the dK/dV kernel (bwd_form)
 };
+constexpr int kBwdWide = 0, kBwdShared = 1, kBwdNarrow = 2;
 
 // ---- Items of the kernels without a scheduler: geometry and kept blocks straight from the caller's arrays (bits == nullptr)
 // or from a prepared workspace.  Everything here is uniform over the calling wavefront.

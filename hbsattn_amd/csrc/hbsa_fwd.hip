@@ -672,14 +672,32 @@ inline int bwd_parts(long long items, int resident, int rounds, int pieces, size
   parts = std::min<long long>(parts, (long long)(kMaxPartBytes / (item_bytes * (size_t)items)));
   return parts < 2 ? 1 : (int)parts;
 }
+// The D = 128 dK/dV kernel has three forms: wide, eight wavefronts on 128 keys and tiles of 64 rows, one workgroup a CU; shared, the
+// same on 64 keys, two wavefronts' sums each put together at the end; and narrow, four on 64 keys and tiles of 32 rows, two workgroups a CU.
+// Those two cover each other's waits, and a tile of 32 rows leaves less of a block's end empty, but each is slower by itself, and a block
+// of more than 64 keys has its tiles loaded by two of them.  Measured, us, whole training calls:
+// - blocks of up to 64 keys, shared and narrow: 5 x 4491 .. 8593 tokens, 16 heads, 7776 items, 1266 and 1052, 4 x 4096, 32 / 8, 2048 items, 1030 and
+//   985; but below four items a CU 6 x 1181 .. 2120, 32 / 4, 824 items, 406 and 436, 3 x 5431, 4 / 2, 510, 305 and 358, 6 x 1734, 2 heads, 444, 119 and 126
+//   (short ones gain there, too: 6 x 181 .. 458, 16 heads, 670 items, 88 and 81);
+// - blocks of 128 keys, wide and narrow, where 64-row tiles hold an eighth more rows than 32-row ones: 4 x 2000 .. 4000, 8 / 2 heads, 32-row
+//   blocks 470 and 316, 16-row ones 309 and 276, 80-row ones 5 x 1249, 16 / 8, 198 and 182, 4 x 3000 .. 6000, 16 heads, 1336 and 1261, 208-row ones 655 and
+//   639; elsewhere 7 x 2143, 32 / 4, 64-row blocks, 690 and 719, 1 x 32768, 8 heads, 1180 and 1218.
+int bwd_form(int headdim, int nhead_k, int num_k_block, int q_block_size, int k_block_size) {
+  if (headdim != 128) return k_block_size <= 2 * kWaveRows ? kBwdShared : kBwdWide;
+  if (k_block_size <= 2 * kWaveRows) return (long long)nhead_k * num_k_block >= 4ll * device_cus() ? kBwdNarrow : kBwdShared;
+  const int in64 = (q_block_size + 63) / 64 * 64, in32 = (q_block_size + 31) / 32 * 32;
+  return 8 * in64 >= 9 * in32 ? kBwdNarrow : kBwdWide;
+}
+inline int bwd_wg_keys(int form) { return (form == kBwdNarrow ? 2 : 4) * kWaveRows; }
 BwdPartPlan bwd_part_plan(int nhead_q, int nhead_k, int headdim, int num_q_block, int num_k_block, int q_block_size, int k_block_size) {
   const int ratio = nhead_q / nhead_k, wps = (q_block_size + kWaveRows - 1) / kWaveRows;
   BwdPartPlan r;
   r.q_items = (long long)nhead_k * num_q_block * ((ratio * wps + 3) / 4);
-  r.k_items = (long long)nhead_k * num_k_block * ((k_block_size + 4 * kWaveRows - 1) / (4 * kWaveRows));
-  const size_t q_bytes = (size_t)4 * kWaveRows * headdim * sizeof(float), k_bytes = 2 * q_bytes;
+  const int form = bwd_form(headdim, nhead_k, num_k_block, q_block_size, k_block_size);
+  r.k_items = (long long)nhead_k * num_k_block * ((k_block_size + bwd_wg_keys(form) - 1) / bwd_wg_keys(form));
+  const size_t q_bytes = (size_t)4 * kWaveRows * headdim * sizeof(float), k_bytes = form == kBwdNarrow ? q_bytes : 2 * q_bytes;
   r.parts_q = bwd_parts(r.q_items, headdim == 128 ? 2 : 3, 1, num_k_block, q_bytes);
-  r.parts_k = bwd_parts(r.k_items, headdim == 128 ? 1 : 3, headdim == 128 ? 1 : 2, (int)std::min<long long>((long long)num_q_block * ratio, 1 << 20), k_bytes);
+  r.parts_k = bwd_parts(r.k_items, headdim != 128 ? 3 : form == kBwdNarrow ? 2 : 1, headdim == 128 ? 1 : 2, (int)std::min<long long>((long long)num_q_block * ratio, 1 << 20), k_bytes);
   const size_t bq = r.parts_q > 1 ? q_bytes * r.parts_q * (size_t)r.q_items : 0, bk = r.parts_k > 1 ? k_bytes * r.parts_k * (size_t)r.k_items : 0;
   r.bytes = align_up(std::max(bq, bk), 256);
   return r;
@@ -1608,7 +1626,8 @@ int hbsa_bwd(const void *q, const void *k, const void *v, const void *out, const
   bp.wpr = words_per_row(num_k_block); bp.causal = causal ? 1 : 0;
   bp.wps = (q_block_size + kWaveRows - 1) / kWaveRows;
   bp.nsub = (bp.ratio * bp.wps + 3) / 4;
-  bp.nsub_k = (k_block_size + 4 * kWaveRows - 1) / (4 * kWaveRows);
+  bp.form_k = bwd_form(headdim, nhead_k, num_k_block, q_block_size, k_block_size);
+  bp.nsub_k = (k_block_size + bwd_wg_keys(bp.form_k) - 1) / bwd_wg_keys(bp.form_k);
   bp.flat_grid = ((long long)num_k_block * bp.nsub_k * nhead_k < (1LL << 31) && (long long)num_q_block * bp.nsub * nhead_k < (1LL << 31)) ? 1 : 0;
   bp.xcd_heads = bp.flat_grid && nhead_k % 8 == 0 ? 1 : 0;
   if (order_bytes(nhead_k, num_q_block, num_k_block) != 0)
