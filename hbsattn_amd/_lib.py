@@ -66,6 +66,8 @@ def load() -> ctypes.CDLL:
     lib.hbsa_fwd_v_locked.argtypes = [vp, ctypes.c_size_t, vp, ctypes.c_float, vp, vp]
     lib.hbsa_fwd_one.restype = ctypes.c_int
     lib.hbsa_fwd_one.argtypes = [vp, vp, ctypes.c_float, vp, vp]
+    lib.hbsa_fwd_counted.restype = ctypes.c_int
+    lib.hbsa_fwd_counted.argtypes = [vp, vp, ctypes.c_float, vp, vp, ctypes.c_int32, vp]
     lib.hbsa_fwd_static.restype = ctypes.c_int
     lib.hbsa_fwd_static.argtypes = [vp] * 10 + [ctypes.c_int32] * 12 + [ctypes.c_float, i64p, vp]
     lib.hbsa_fwd_prepare.restype = ctypes.c_int

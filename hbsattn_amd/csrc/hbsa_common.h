@@ -163,6 +163,11 @@ struct FwdParams {
   int32_t grouped;       // host side only: tiles of 16-key groups (the GROUPED form of the kernel)
   // Items handed out without queues in the order of their weights (see OrderRoom), nullptr: last q blocks first
   const uint32_t *order;         // [num_q_block * nhead_k]: q block << 16 | kv head, heaviest first
+  // One-launch form whose caller has not counted the blocks (counts != nullptr): the sides of count_sides (1: queries, 2: keys; cu_nqb, cu_nkb
+  // then point to something that can be read) are counted by every workgroup for itself, and the first writes counts[2] = whether the
+  // totals are nqb and nkb_total, counts[3] = ticket, in one 8-byte store
+  int32_t *counts;
+  int32_t ticket, count_sides;
 };
 
 // Boundaries of one sequence of the packed batch, as read from the caller's device arrays.
@@ -530,6 +535,8 @@ template <int D, typename E, bool OUT32>
 int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
+int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>

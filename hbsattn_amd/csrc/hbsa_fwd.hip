@@ -929,7 +929,7 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
                 const int32_t *cu_k_seqlens, const uint8_t *block_mask, const int32_t *cu_num_q_block,
                 const int32_t *cu_num_k_block, int32_t dtype, int32_t batch, int32_t total_q, int32_t total_k, int32_t nhead_q,
                 int32_t nhead_k, int32_t headdim, int32_t num_q_block, int32_t num_k_block, int32_t q_block_size,
-                int32_t k_block_size, int32_t causal, float softmax_scale, const int64_t *strides, hipStream_t st) {
+                int32_t k_block_size, int32_t causal, float softmax_scale, const int64_t *strides, hipStream_t st, int32_t *counts, int32_t ticket) {
   FwdParams fp;
   std::memset(&fp, 0, sizeof(fp));
   const bool cols = headdim != 32 && headdim != 64 && headdim != 128 && headdim != 256;
@@ -954,7 +954,17 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   fp.cu_q = cu_q_seqlens; fp.cu_k = cu_k_seqlens; fp.cu_nqb = cu_num_q_block; fp.cu_nkb = cu_num_k_block;
   fp.mask = block_mask; fp.ms_h = strides[8]; fp.ms_q = strides[9];
   fp.batch = batch; fp.nkb_total = num_k_block; fp.total_k = total_k; fp.qbs = q_block_size;
+  fp.counts = counts; fp.ticket = ticket;
+  fp.count_sides = (cu_num_q_block == nullptr ? 1 : 0) | (cu_num_k_block == nullptr ? 2 : 0);
+  if (cu_num_q_block == nullptr) fp.cu_nqb = cu_q_seqlens;
+  if (cu_num_k_block == nullptr) fp.cu_nkb = cu_k_seqlens;
   const bool bf = dtype == HBSA_DTYPE_BF16;
+  if (counts != nullptr) {   // (eight wavefronts and the other head dims are for larger calls, or rarer ones)
+    if (cols || headdim > 128 || fp.nw != 4) return kNotOnePass;
+    if (headdim == 32) return bf ? launch_fwd_counted<32, ElemBF16>(fp, items, st) : launch_fwd_counted<32, ElemF16>(fp, items, st);
+    if (headdim == 64) return bf ? launch_fwd_counted<64, ElemBF16>(fp, items, st) : launch_fwd_counted<64, ElemF16>(fp, items, st);
+    return bf ? launch_fwd_counted<128, ElemBF16>(fp, items, st) : launch_fwd_counted<128, ElemF16>(fp, items, st);
+  }
   if (cols) {   // a head dim without a kernel of its own runs in the next one up, its missing columns zero on the chip
     if (headdim < 32) return bf ? launch_fwd_cols<32, ElemBF16>(fp, items, st) : launch_fwd_cols<32, ElemF16>(fp, items, st);
     if (headdim < 64) return bf ? launch_fwd_cols<64, ElemBF16>(fp, items, st) : launch_fwd_cols<64, ElemF16>(fp, items, st);
@@ -1404,7 +1414,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
              size_t workspace_bytes, int32_t dtype, int32_t batch, int32_t total_q, int32_t total_k,
              int32_t nhead_q, int32_t nhead_k, int32_t headdim, int32_t num_q_block, int32_t num_k_block,
              int32_t q_block_size, int32_t k_block_size, int32_t causal, float softmax_scale,
-             const int64_t *strides, void *stream, bool allow_onepass, bool any_dim = false) {
+             const int64_t *strides, void *stream, bool allow_onepass, bool any_dim = false, int32_t *counts = nullptr, int32_t ticket = 0) {
   g_err[0] = 0;
   if (total_q == 0 || num_q_block == 0 || nhead_q == 0) return 0;
   if (!strides) return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
@@ -1422,7 +1432,7 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   if (int rc = check_strides(strides, dtype == HBSA_DTYPE_F32 || dtype == HBSA_DTYPE_F32_STAGED16)) return rc;
   if (batch < 0 || num_q_block < 0 || num_k_block < 0 || total_q < 0 || total_k < 0)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "negative size");
-  if (!cu_q_seqlens || !cu_k_seqlens || !block_mask || !cu_num_q_block || !cu_num_k_block)
+  if (!cu_q_seqlens || !cu_k_seqlens || !block_mask || (!counts && (!cu_num_q_block || !cu_num_k_block)))
     return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
   if (q_block_size <= 0 || k_block_size <= 0 || q_block_size % 16 || k_block_size % 16)
     return fail(HBSA_ERR_INVALID_ARGUMENT, "q_block_size (%d) and k_block_size (%d) must be positive multiples of 16",
@@ -1431,12 +1441,12 @@ int fwd_call(const void *q, const void *k, const void *v, void *out, const int32
   if (nhead_k > 65535) return fail(HBSA_ERR_UNSUPPORTED, "nhead_k %d > 65535", nhead_k);
   const bool f32_exact = dtype == HBSA_DTYPE_F32;
   const DecodePlan plan = decode_plan(dtype, nhead_q, nhead_k, num_q_block, total_q, q_block_size, num_k_block, k_block_size);
-  const bool decode = !any_dim && plan.use;
+  const bool decode = (!any_dim || counts != nullptr) && plan.use;
   const bool direct = allow_onepass && g_onepass && (f32_exact || decode);   // a kernel that reads boundaries and mask itself
   if (allow_onepass && !direct) {
     const int one = try_onepass(q, k, v, out, cu_q_seqlens, cu_k_seqlens, block_mask, cu_num_q_block, cu_num_k_block, dtype,
                                 batch, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size,
-                                k_block_size, causal, softmax_scale, strides, (hipStream_t)stream);
+                                k_block_size, causal, softmax_scale, strides, (hipStream_t)stream, counts, ticket);
     if (one != kNotOnePass) return one;
   }
   if (any_dim) return fail(HBSA_ERR_WORKSPACE_TOO_SMALL, "the call is not one launch: use hbsa_fwd with a workspace");
@@ -1524,6 +1534,19 @@ int hbsa_fwd_one(const void *const *ptrs, const int32_t *sizes, float softmax_sc
                   (const uint8_t *)ptrs[6], (const int32_t *)ptrs[7], (const int32_t *)ptrs[8], (const int32_t *)ptrs[9],
                   nullptr, 0, sizes[0], sizes[1], sizes[2], sizes[3], sizes[4], sizes[5], sizes[6], sizes[7],
                   sizes[8], sizes[9], sizes[10], sizes[11], softmax_scale, strides, stream, true, true);
+}
+
+int hbsa_fwd_counted(const void *const *ptrs, const int32_t *sizes, float softmax_scale, const int64_t *strides, int32_t *counts,
+                     int32_t ticket, void *stream) {
+  g_err[0] = 0;
+  if (!ptrs || !sizes || !counts) return fail(HBSA_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if ((uintptr_t)counts & 15) return fail(HBSA_ERR_INVALID_ARGUMENT, "counts must be 16-byte aligned");
+  if (sizes[1] < 1) return fail(HBSA_ERR_INVALID_ARGUMENT, "no sequences");
+  if (sizes[2] == 0 || sizes[7] == 0 || sizes[4] == 0) return fail(HBSA_ERR_INVALID_ARGUMENT, "nothing to launch: no counts would be written");
+  return fwd_call(ptrs[0], ptrs[1], ptrs[2], (void *)ptrs[3], (const int32_t *)ptrs[4], (const int32_t *)ptrs[5],
+                  (const uint8_t *)ptrs[6], (const int32_t *)ptrs[7], (const int32_t *)ptrs[8], (const int32_t *)ptrs[9],
+                  nullptr, 0, sizes[0], sizes[1], sizes[2], sizes[3], sizes[4], sizes[5], sizes[6], sizes[7],
+                  sizes[8], sizes[9], sizes[10], sizes[11], softmax_scale, strides, stream, true, true, counts, ticket);
 }
 
 int hbsa_fwd_static(const void *q, const void *k, const void *v, void *out, const int32_t *cu_q_seqlens,

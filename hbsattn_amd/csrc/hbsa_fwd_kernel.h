@@ -183,7 +183,7 @@ __device__ __forceinline__ int build_group_list(uint16_t *list, int chunk_base, 
   return total;
 }
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED>
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED, bool COUNTED>
 __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3 : 4) void hbsa_fwd_kernel(FwdParams p) {
   // OUT32: fp32 output (the fp32-input path; q/k/v are then fp16 staging copies)
   // EXTRAS: the clocked walk, the split over key blocks and the log-sum-exp output are compiled in.  The
@@ -200,6 +200,8 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   // GROUPED: tiles are made of groups of 16 keys from any places, for block sizes that are no multiple of the tile.  Otherwise a
   // tile is consecutive keys of one run of kept blocks, and the end of every run is a tile that is partly empty and has to be
   // masked (blocks of 48 keys, half of them kept: 120 keys' worth of tiles for 96, half of the tiles masked).
+  // COUNTED: (FUSED) the caller has not counted the blocks; see FwdParams::counts.  Kernels of their own: compiled in everywhere, the
+  // counting cost calls that do not use it 1 % (16 x 40 .. 500 tokens, 32 / 8 heads, 37.7 -> 38.0 us; 8 x 2050, 16 of 192, 227.6 -> 229.7).
   // NW: wavefronts (wave slots) of a workgroup, 4 or 8.  Eight are used when the q heads of a GQA group
   // and the 32-row slices of a q block give an item more than four wave slots: one workgroup per CU then
   // stages every K/V tile once for all of them instead of two workgroups staging it each (D = 128 only, and
@@ -606,8 +608,45 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       for (int i = lane; i <= p.batch; i += 64) {
         lds_seq[i] = p.cu_q[i];
         lds_seq[kSeqCap + i] = p.cu_k[i];
-        lds_seq[2 * kSeqCap + i] = p.cu_nqb[i];
+        lds_seq[2 * kSeqCap + i] = p.cu_nqb[i];   // (either array where the caller has not counted: replaced below)
         lds_seq[3 * kSeqCap + i] = p.cu_nkb[i];
+      }
+      if constexpr (COUNTED) {   // as hbsa_block_counts_kernel, whose launch was 2.6 us of a call's 13.5 (5 x 32 tokens, 8 / 2 heads of 32)
+        const int l = lane;
+        bool bad = false;
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+          if (!((p.count_sides >> side) & 1)) continue;
+          const int *cu = lds_seq + side * kSeqCap;
+          int *first = lds_seq + (2 + side) * kSeqCap, before = 0;
+          const uint32_t size = (uint32_t)(side == 0 ? p.qbs : p.kbs);
+          for (int base = 0; base <= p.batch; base += 64) {
+            const int i = base + l;
+            int n = 0;
+            if (i < p.batch) {
+              const int64_t len = (int64_t)cu[i + 1] - cu[i];
+              if (len < 0) bad = true;
+              else n = (int)((uint32_t)(len + size - 1) / size);
+            }
+            int incl = n;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+              const int x = __shfl_up(incl, off);
+              if (l >= off) incl += x;
+            }
+            if (i <= p.batch) first[i] = before + incl - n;
+            before += __builtin_amdgcn_readlane(incl, 63);
+          }
+          if (before != (side == 0 ? p.nqb : p.nkb_total)) bad = true;
+        }
+        bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+        if (bad)   // the mask does not fit: sequences without blocks, nothing is read for them
+          for (int i = l; i <= p.batch; i += 64) {
+            if (p.count_sides & 1) lds_seq[2 * kSeqCap + i] = 0;
+            if (p.count_sides & 2) lds_seq[3 * kSeqCap + i] = 0;
+          }
+        if (blockIdx.x == 0 && l == 0)
+          __hip_atomic_store((uint64_t *)(p.counts + 2), (uint64_t)(uint32_t)p.ticket << 32 | (bad ? 0u : 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
     pending = claim();
@@ -1424,10 +1463,11 @@ inline int persistent_grid(const void *kernel, int lds_bytes, int threads) {
   return cus * per_cu;
 }
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false, bool COLS = false, bool GROUPED = false>
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false, bool COLS = false, bool GROUPED = false,
+          bool COUNTED = false>
 int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   constexpr int lds_bytes = 4 * (D > 128 && D <= 192 ? 32 : 64) * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
-  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED>);
+  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED>);
   // workgroups that fit the current device at once; the attribute and the occupancy are per device
   static thread_local int resident_of[kMaxDevices] = {};
   int dev = 0;
@@ -1446,7 +1486,7 @@ int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   // heads, the crowd at few counters) would be a good part of such a launch.
   launch.one_each = items <= (long long)kStaticShare * resident ? (int)items : 0;
   if (launch.one_each == 0 || launch.nparts != 1 || items <= resident) launch.order = nullptr;
-  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
+  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, "hbsa_fwd_kernel launch: %s", hipGetErrorString(e));
   return 0;
@@ -1480,6 +1520,16 @@ int launch_fused_tiles(const FwdParams &fp, long long items, hipStream_t stream)
 template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream) {
   return fp.grouped ? launch_fused_tiles<D, E, true>(fp, items, stream) : launch_fused_tiles<D, E, false>(fp, items, stream);
+}
+
+// the one-launch form that counts the blocks itself, workgroups of four wavefronts
+template <int D, typename E>
+int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream) {
+  if (fp.grouped)
+    return fp.pack ? launch_fwd_nw<D, E, false, 4, false, true, true, false, true, true>(fp, items, stream)
+                   : launch_fwd_nw<D, E, false, 4, false, true, false, false, true, true>(fp, items, stream);
+  return fp.pack ? launch_fwd_nw<D, E, false, 4, false, true, true, false, false, true>(fp, items, stream)
+                 : launch_fwd_nw<D, E, false, 4, false, true, false, false, false, true>(fp, items, stream);
 }
 
 // the one-launch form for tensors whose head dim (fp.ncol chunks of eight elements) is D or less

@@ -3,7 +3,7 @@
 //   1  forward with 16-bit output (both forms)     2  forward with fp32 output (fp32 tensors staged as fp16)
 //   3  backward                                    4  forward on fp32 operands
 //   5  forward, head dims up to HBSA_D (also 96, 160 and 192)
-//   6  forward, few queries per item
+//   6  forward, few queries per item                 7  forward that counts the blocks itself
 #if HBSA_PART == 1
 #include "hbsa_fwd_kernel.h"
 template int hbsa::launch_fwd<HBSA_D, hbsa::HBSA_E, false>(const FwdParams &, long long, hipStream_t);
@@ -23,6 +23,9 @@ template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long
 #elif HBSA_PART == 6
 #include "hbsa_fwd_decode.h"
 template int hbsa::launch_fwd_decode<HBSA_D, hbsa::HBSA_E>(const FwdParams &, int, long long, hipStream_t);
+#elif HBSA_PART == 7
+#include "hbsa_fwd_kernel.h"
+template int hbsa::launch_fwd_counted<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
 #else
-#error "HBSA_PART is 1 to 6"
+#error "HBSA_PART is 1 to 7"
 #endif

@@ -110,8 +110,9 @@ at::Tensor bytes_like(const at::Tensor &t, size_t n) { return at::empty({(int64_
 
 bool native_dim(int64_t d) { return d == 32 || d == 64 || d == 128 || d == 256; }
 
-// The output; undefined when the head dim has to be padded first.
-at::Tensor plain_forward(const Problem &p, hipStream_t stream) {
+// The output; undefined when the head dim has to be padded first, or (with a slot for the block counts) when the call is not one
+// launch that counts the blocks itself; nothing has been launched then.
+at::Tensor plain_forward(const Problem &p, hipStream_t stream, int32_t *slot = nullptr, int32_t ticket = 0) {
   at::Tensor out = at::empty(p.q.sizes(), p.q.options());
   const int64_t strides[11] = {tok_stride(p.q), head_stride(p.q), tok_stride(p.k), head_stride(p.k), tok_stride(p.v), head_stride(p.v),
                                tok_stride(out), head_stride(out), p.mask.stride(0), p.mask.stride(1),
@@ -121,8 +122,14 @@ at::Tensor plain_forward(const Problem &p, hipStream_t stream) {
                              (int32_t)p.qbs, (int32_t)p.kbs, p.causal ? 1 : 0};
   const void *ptrs[11] = {p.q.const_data_ptr(), p.k.const_data_ptr(), p.v.const_data_ptr(), out.mutable_data_ptr(),
                           p.cu_q.const_data_ptr(), p.cu_k.const_data_ptr(), p.mask.const_data_ptr(),
-                          p.qb2b.defined() ? p.qb2b.const_data_ptr() : nullptr, p.cu_nqb.const_data_ptr(), p.cu_nkb.const_data_ptr(),
-                          nullptr};
+                          p.qb2b.defined() ? p.qb2b.const_data_ptr() : nullptr, p.cu_nqb.defined() ? p.cu_nqb.const_data_ptr() : nullptr,
+                          p.cu_nkb.defined() ? p.cu_nkb.const_data_ptr() : nullptr, nullptr};
+  if (slot != nullptr) {
+    const int rc = hbsa_fwd_counted(ptrs, sizes, (float)p.scale, strides, slot, ticket, stream);
+    if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) return at::Tensor();
+    if (rc != 0) raise("hbsa_fwd_counted", rc);
+    return out;
+  }
   if (!native_dim(p.q.size(2))) {
     const int rc = hbsa_fwd_one(ptrs, sizes, (float)p.scale, strides, stream);
     if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) return at::Tensor();   // no single launch: the caller pads
@@ -307,12 +314,20 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     }
   }
   CountTicket counts(g_slots, counting ? g_slots.take(count_page) : nullptr, StateOf{stream});
+  at::Tensor out;
   if (counting) {
-    // Counts and first blocks of the sequences in one small launch.  The device checks the counts against the mask's
+    // One launch that counts the blocks itself, or counts and first blocks of the sequences in one small launch.  The device checks the counts against the mask's
     // shape and leaves empty sequences when they differ, so the attention launch can follow at once; the host reads
     // the counts while it runs, and a call whose mask does not fit is reported by the caller.
     if (counts.slot == nullptr) Py_RETURN_NONE;
     counts.ticket = g_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
+    p.nqb = p.mask.size(1);
+    p.nkb = p.mask.size(2);
+    counts.launched = true;
+    if (!wants_grad && st != at::kFloat) out = plain_forward(p, stream, counts.slot, counts.ticket);
+    counts.launched = out.defined();
+  }
+  if (counting && !out.defined()) {
     at::Tensor firsts = at::empty({2, n_seq}, p.cu_q.options());
     int32_t *first = firsts.mutable_data_ptr<int32_t>();
     counts.launched = true;
@@ -320,17 +335,11 @@ PyObject *call(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
                                      k_given ? nullptr : p.cu_k.const_data_ptr<int32_t>(), (int)p.kbs, (int)p.mask.size(2),
                                      first + n_seq, (int)n_seq - 1, counts.slot, counts.ticket, stream);
     if (rc != 0) Py_RETURN_NONE;
-    if (!q_given) {
-      p.cu_nqb = firsts.select(0, 0);
-      p.nqb = p.mask.size(1);
-    }
-    if (!k_given) {
-      p.cu_nkb = firsts.select(0, 1);
-      p.nkb = p.mask.size(2);
-    }
+    if (!q_given) p.cu_nqb = firsts.select(0, 0);
+    if (!k_given) p.cu_nkb = firsts.select(0, 1);
   }
 
-  const at::Tensor out = wants_grad ? Attention::apply(p.q, p.k, p.v, p) : plain_forward(p, stream);
+  if (!out.defined()) out = wants_grad ? Attention::apply(p.q, p.k, p.v, p) : plain_forward(p, stream);
   bool counts_fit = true;
   if (counting) {
     Py_BEGIN_ALLOW_THREADS

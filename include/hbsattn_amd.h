@@ -249,6 +249,14 @@ int hbsa_fwd_v(const void *const *ptrs, size_t workspace_bytes, const int32_t *s
  */
 int hbsa_fwd_one(const void *const *ptrs, const int32_t *sizes, float softmax_scale, const int64_t *strides, void *stream);
 
+/* hbsa_fwd_one for a caller that has not counted the blocks: cu_num_q_block, cu_num_k_block or both may be NULL in `ptrs`, and are then
+ * counted by the launch itself.  `counts` is as in hbsa_block_counts, 16-byte aligned; the launch writes counts[2] = 1 when no length is
+ * negative and the totals are sizes' num_q_block and num_k_block, else 0 (the output is then undefined, nothing out of range is touched), and
+ * counts[3] = ticket, both at once when it begins.  HBSA_ERR_WORKSPACE_TOO_SMALL: no such launch for this call (fp32 tensors, other
+ * head dims than 32, 64 and 128, few queries per q block, a split, workgroups of eight wavefronts, a captured stream ..), nothing was launched and nothing will be written. */
+int hbsa_fwd_counted(const void *const *ptrs, const int32_t *sizes, float softmax_scale, const int64_t *strides, int32_t *counts,
+                     int32_t ticket, void *stream);
+
 /*
  * hbsa_fwd for callers that cannot allocate device memory or pass a workspace: code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
