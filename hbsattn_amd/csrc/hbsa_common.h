@@ -139,8 +139,18 @@ struct FwdParams {
   // normalised fp32 partial result and its log-sum-exp; hbsa_merge_kernel combines them.
   int32_t nparts;         // 1: no split
   FastDiv div_nparts;
-  float *part_out;        // [nparts, total_q, nhead_q, D]
-  float *part_lse;        // [nparts, total_q, nhead_q]
+  // One-launch form whose caller has not counted the blocks (the COUNTED kernels, in the place of what a split needs: 16 bytes more of
+  // arguments cost every short call 0.2 us): the sides of count_info[1] (1: queries, 2: keys; cu_nqb, cu_nkb then point to something that
+  // can be read) are counted by every workgroup for itself, and the first writes counts[2] = whether the totals are nqb and
+  // nkb_total, counts[3] = count_info[0], the caller's ticket, in one 8-byte store.
+  union {
+    float *part_out;        // [nparts, total_q, nhead_q, D]
+    int32_t *counts;
+  };
+  union {
+    float *part_lse;        // [nparts, total_q, nhead_q]
+    int32_t count_info[2];
+  };
   int32_t total_q, nhead_q;
   // One-launch form (the kernel instantiated with FUSED): no pre-pass has run, `info` and `bits` are unused,
   // and the scheduler derives every item's geometry and bit row itself from the caller's arrays.
@@ -163,11 +173,6 @@ struct FwdParams {
   int32_t grouped;       // host side only: tiles of 16-key groups (the GROUPED form of the kernel)
   // Items handed out without queues in the order of their weights (see OrderRoom), nullptr: last q blocks first
   const uint32_t *order;         // [num_q_block * nhead_k]: q block << 16 | kv head, heaviest first
-  // One-launch form whose caller has not counted the blocks (counts != nullptr): the sides of count_sides (1: queries, 2: keys; cu_nqb, cu_nkb
-  // then point to something that can be read) are counted by every workgroup for itself, and the first writes counts[2] = whether the
-  // totals are nqb and nkb_total, counts[3] = ticket, in one 8-byte store
-  int32_t *counts;
-  int32_t ticket, count_sides;
 };
 
 // Boundaries of one sequence of the packed batch, as read from the caller's device arrays.

@@ -954,8 +954,9 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   fp.cu_q = cu_q_seqlens; fp.cu_k = cu_k_seqlens; fp.cu_nqb = cu_num_q_block; fp.cu_nkb = cu_num_k_block;
   fp.mask = block_mask; fp.ms_h = strides[8]; fp.ms_q = strides[9];
   fp.batch = batch; fp.nkb_total = num_k_block; fp.total_k = total_k; fp.qbs = q_block_size;
-  fp.counts = counts; fp.ticket = ticket;
-  fp.count_sides = (cu_num_q_block == nullptr ? 1 : 0) | (cu_num_k_block == nullptr ? 2 : 0);
+  fp.counts = counts;
+  fp.count_info[0] = ticket;
+  fp.count_info[1] = (cu_num_q_block == nullptr ? 1 : 0) | (cu_num_k_block == nullptr ? 2 : 0);
   if (cu_num_q_block == nullptr) fp.cu_nqb = cu_q_seqlens;
   if (cu_num_k_block == nullptr) fp.cu_nkb = cu_k_seqlens;
   const bool bf = dtype == HBSA_DTYPE_BF16;

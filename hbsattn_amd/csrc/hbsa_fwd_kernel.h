@@ -616,7 +616,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         bool bad = false;
 #pragma unroll
         for (int side = 0; side < 2; ++side) {
-          if (!((p.count_sides >> side) & 1)) continue;
+          if (!((p.count_info[1] >> side) & 1)) continue;
           const int *cu = lds_seq + side * kSeqCap;
           int *first = lds_seq + (2 + side) * kSeqCap, before = 0;
           const uint32_t size = (uint32_t)(side == 0 ? p.qbs : p.kbs);
@@ -642,11 +642,11 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         bad = __builtin_amdgcn_ballot_w64(bad) != 0;
         if (bad)   // the mask does not fit: sequences without blocks, nothing is read for them
           for (int i = l; i <= p.batch; i += 64) {
-            if (p.count_sides & 1) lds_seq[2 * kSeqCap + i] = 0;
-            if (p.count_sides & 2) lds_seq[3 * kSeqCap + i] = 0;
+            if (p.count_info[1] & 1) lds_seq[2 * kSeqCap + i] = 0;
+            if (p.count_info[1] & 2) lds_seq[3 * kSeqCap + i] = 0;
           }
         if (blockIdx.x == 0 && l == 0)
-          __hip_atomic_store((uint64_t *)(p.counts + 2), (uint64_t)(uint32_t)p.ticket << 32 | (bad ? 0u : 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          __hip_atomic_store((uint64_t *)(p.counts + 2), (uint64_t)(uint32_t)p.count_info[0] << 32 | (bad ? 0u : 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
     pending = claim();
