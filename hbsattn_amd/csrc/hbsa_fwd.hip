@@ -936,12 +936,7 @@ int try_onepass(const void *q, const void *k, const void *v, void *out, const in
   fill_shape(fp, total_q, total_k, nhead_q, nhead_k, headdim, num_q_block, num_k_block, q_block_size, k_block_size, causal, softmax_scale, false,
              true, cols);
   const long long items = (long long)nhead_k * num_q_block * fp.nsub;
-  // A head dim without a kernel of its own has no split form: its tensors are copied and padded first, 27 us of 93.  Sequences of which none
-  // by itself would be split are the faster as one launch: 7 x 2138 tokens, 2 / 1 heads of 48, 96 and 192, 94 -> 26, 93 -> 29 and 100 -> 50;
-  // 7 x 2023 .. 3666, one head of 80, 98 -> 48.  Chunks and longer sequences stay split.
-  const long long tiles = (long long)num_k_block * ((k_block_size + kTileKeys - 1) / kTileKeys);
-  const bool whole = cols && (long long)num_k_block * k_block_size < 4ll * num_q_block * q_block_size && tiles < 2ll * kPartTiles * batch;
-  Sched *sched = onepass_record(dtype, batch, total_k, headdim, k_block_size, strides[10], items, whole ? 1 : fp.split, st);
+  Sched *sched = onepass_record(dtype, batch, total_k, headdim, k_block_size, strides[10], items, fp.split, st);
   if (sched == nullptr) return kNotOnePass;
 
   fp.q = (const char *)q; fp.k = (const char *)k; fp.v = (const char *)v; fp.out = (char *)out;

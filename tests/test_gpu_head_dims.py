@@ -26,15 +26,6 @@ def test_columns_past_the_head_dim_take_no_part(d, dtype, qbs, kbs, causal, hq, 
     assert _lib.host().call(*w.args(), _lib.DTYPE_F32) is not None
 
 
-@pytest.mark.parametrize("d", [48, 96, 160, 192])
-def test_few_items_of_several_sequences_are_one_launch(d, monkeypatch):
-    # at a head dim of a kernel's own these would be split over key blocks: 74 items, 294 key blocks
-    w = make_problem(seed=d, q_lens=[1600, 1500, 1590], k_lens=[1600, 1500, 1590], hq=2, hk=1, d=d, qbs=64, kbs=16, keep=0.3, diag=True,
-                     causal=True, scale=None)
-    monkeypatch.setattr("hbsattn_amd.interface.hbsa_forward", lambda *a, **k: pytest.fail("the call left the compiled host path"))
-    assert_close_to_oracle(HBSAttention(*w.args()), oracle_for(w), f"head dim {d}")
-
-
 def test_missing_columns_cost_little():
     # The work and the kernel are head dim 256's.  With an offset and a column mask in registers for each of a wavefront's sixteen loads it
     # spilled in the tile loop: 1.53 times the time; with the eight that differ 1.15.  The least of ten runs of each, taken in turn.
