@@ -816,7 +816,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       return;
     }
     base = tile_ptr(base, tile.first, stride);
-    if (valid == KT) {
+    if (__builtin_expect(valid == KT, 1)) {
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
         if ((!LAST_PART || i < LOADS - 1 || (i * NW + wave) * 64 < CPR * KT) && (!COLS || (V_PART ? ld_vin[i % OFFSETS] : ld_kin[i % OFFSETS])))   // (a lane that loads nothing leaves its 16 bytes of LDS alone)
@@ -1080,15 +1080,29 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         return tile_ref((uint32_t)__builtin_amdgcn_readlane((int)from.x, lane_at),
                         GROUPED ? (uint32_t)__builtin_amdgcn_readlane((int)from.y, lane_at) : 0u, c, chunk_base + x, total);
       };
+      held = entry_of(0);
+      TileRef nx_tile = held_tile(held, 0, 0);
       for (int t = 0; t < n; ++t) {   // ---------------------------------- one iteration per 64-key tile
-        if ((t & 63) == 0) held = entry_of(t);
-        const TileRef tile = held_tile(held, t & 63, t);
+        const TileRef tile = nx_tile;
         const int kpos = tile.first, valid = tile.valid;
+        const bool more = t + 1 < n, last = chunk_base + t + 1 == total;
+        // The next tile is looked up before the wait, and what is rare stands out of line: between the barrier and the tile's first
+        // products none of the workgroup's wavefronts has work for the matrix cores, and scalar code there, taken branches above
+        // all, is paid by every one of them (some 70 scalar instructions and six taken branches before, 30 and one here: 16 x 40 .. 500
+        // tokens, 32 / 8 heads of 128, 35.4 -> 34.7 us; two chunks on 65000 keys 268 -> 262; 8 x 2050, 16 heads of 192, 215 -> 211).
+        TileRef nx = {0, 0, 0u, 0u};      // valid > 0: a next tile exists and its loads go out during this tile
+        if (__builtin_expect(more, 1)) {
+          if (__builtin_expect(((t + 1) & 63) == 0, 0)) held = entry_of(t + 1);
+          nx = held_tile(held, (t + 1) & 63, t + 1);
+        }
+        const char *nx_k = kg, *nx_v = vg;
+        const bool compute = active && (!p.causal || kpos <= wave_kvis_max);
+        // keys that are missing, or (causal) a last key that some lane's query does not see
+        const bool edge = valid < KT || (p.causal && tile.pos(KT / 16 - 1) + 15 > wave_kvis_min);
 
         if (t > 0 || chunk_base > 0 || !active) settle();   // the current tile has landed in LDS
         __syncthreads();                     // ... for every wave, and the other buffers are free
 
-        const bool last = chunk_base + t + 1 == total;
         // The clock is dealt with on few tiles only (wavefront 0; any work it does alone on every tile
         // makes the other three wait at the next barrier): the item's first tile, every eighth, and
         // the last three.
@@ -1098,12 +1112,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           if (chunk_base + t + 2 == total) next_start(c ^ 1);
           if (last) leave_clock();
         }
-        TileRef nx = {0, 0, 0u, 0u};      // valid > 0: a next tile exists and its loads go out during this tile
-        const char *nx_k = kg, *nx_v = vg;
-        if (t + 1 < n) {
-          if (((t + 1) & 63) == 0) nx = held_tile(entry_of(t + 1), 0, t + 1);
-          else nx = held_tile(held, (t + 1) & 63, t + 1);
-        } else if (last) {
+        if (__builtin_expect(last, 0)) {
           nxt_hk = hdr_word(c ^ 1, H_HK);
           if (nxt_hk >= 0 && hdr_word(c ^ 1, H_TOTAL) > 0) {
             nx = listed_tile(c ^ 1, GROUPED ? 0 : hdr_word(c ^ 1, H_T0), 0);
@@ -1111,10 +1120,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
             nx_v = item_v(c ^ 1);
           }
         }
+        nx_tile = nx;
         // The next tile's K is requested right after this tile's first operand reads, its V only after
         // the first MFMA block: the wavefronts then do not all queue at the load unit at once.
 
-        const bool compute = active && (!p.causal || kpos <= wave_kvis_max);
         if (!compute && nx.valid > 0) {
           issue_k(buf ^ 1, nx_k, nx);
           issue_v(buf ^ 1, nx_v, nx);
@@ -1125,10 +1134,6 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           // other half:   S0 | S1 + exp(S0) | PV0 + exp(S1) | PV1.   (A maximum, of S0, is formed for an item's first tile alone:
           // see settle_half.)
           const bool first = chunk_base + t == 0;   // the item's first tile gives the reference
-          // keys that are missing, or (causal) a last key that some lane's query does not see
-          const bool edge = valid < KT || (p.causal && tile.pos(KT / 16 - 1) + 15 > wave_kvis_min);
-
-
           f32x16 s0, s1;
 #pragma unroll
           for (int i = 0; i < 16; ++i) { s0[i] = 0.f; s1[i] = 0.f; }
