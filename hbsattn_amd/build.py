@@ -21,7 +21,7 @@ INST_SOURCE = os.path.join(CSRC, "hbsa_inst.hip")   # the attention kernels of o
 OUTPUT = os.path.join(_HERE, "libhbsattn_amd.so")
 # substrings of the mangled names of the kernels with hand-issued LDS reads ...
 HAND_ISSUED_READS = ("hbsa_fwd_kernel", "hbsa_bwd_dq_kernel", "hbsa_bwd_dkv")
-COMPILER_ISSUED = "hbsa_fwd_kernelILi256E"   # ... except the head dim 256 instantiations, whose reads the compiler issues
+COMPILER_ISSUED = "hbsa_fwd_kernelILi256E"   # ... except the head dim 256 instantiations, whose reads the compiler issues (it may move such a register to the other half at any time)
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32 out of scalar float code.
 HIPCC_FLAGS = [
@@ -30,11 +30,20 @@ HIPCC_FLAGS = [
     "-I" + os.path.join(_ROOT, "include"), "-I" + CSRC,
 ]
 
+# At head dim 256 a wavefront has the 512 registers of a SIMD, half of them accumulation registers, which the vector ALU cannot
+# read.  Left to itself the compiler writes every matrix product there, the scores among them, moves them over one by one (1133
+# moves in the plain kernel, 313 with the flag) and spills 37 to 135 registers beside that (none with it); told to write products
+# to vector registers it keeps the output and Q operand in the other half.  8 x 2050 tokens, 16 heads, 260 -> 209 us;
+# 8 x 8192 975 -> 826; head dim 208, 307 -> 225; fp32 tensors 261 -> 220; the bits are the same.  At the other head dims all
+# products stand in vector registers anyway.
+MFMA_IN_VGPRS = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+
 
 def units() -> list:
     """``(name, source, extra flags)`` of every translation unit of the library, the ones that take longest first."""
     def inst(d, elem, part):
-        return (f"{elem}_{d}_{part}", INST_SOURCE, [f"-DHBSA_D={d}", f"-DHBSA_E={elem}", f"-DHBSA_PART={part}"])
+        flags = [f"-DHBSA_D={d}", f"-DHBSA_E={elem}", f"-DHBSA_PART={part}"]
+        return (f"{elem}_{d}_{part}", INST_SOURCE, flags + (MFMA_IN_VGPRS if d == 256 else []))
 
     out = [inst(d, e, 1) for d in (128, 64, 256, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 3) for d in (128, 64, 32) for e in ("ElemBF16", "ElemF16")]

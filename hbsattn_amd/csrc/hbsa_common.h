@@ -282,8 +282,8 @@ static_assert(sizeof(Sched) == 256, "Sched is one 256-byte slot of the workspace
 // (The transposing read is issued this way because the compiler otherwise waits for every
 // outstanding global->LDS load before it; the K reads so that their issue distance is fixed.)
 // HAND = false gives the same reads as ordinary loads the compiler schedules and waits for itself (the
-// lds_wait calls then do nothing): the form for instantiations that spill registers, where a register with
-// a hand-issued read in flight could be saved before its data arrives.
+// lds_wait calls then do nothing): the form for instantiations that move registers to the accumulation half, where a
+// register with a hand-issued read in flight could be moved before its data arrives.
 template <int OFF, bool HAND = true>
 __device__ __forceinline__ short8v lds_read_b128(uint32_t addr) {
   if constexpr (HAND) {

@@ -8,7 +8,7 @@ namespace hbsa {
 // --------------------------------------------------------------------------------------
 // Main kernel (persistent).  D = head dim (32, 64, 128 or 256); rows of K/V tiles are D*2 bytes.  At D = 256 a
 // wavefront's output accumulator and query operand alone are 192 registers, so a CU runs one workgroup of four
-// wavefronts, each with the 512 registers of a SIMD (accumulators in the AGPR half), and its two 128 KB of K/V
+// wavefronts, each with the 512 registers of a SIMD (the output in the AGPR half; hbsattn_amd/build.py), and its two 128 KB of K/V
 // tile buffers take most of the LDS.
 //
 // Scheduling.  The grid is as many workgroups as fit the device at once and every workgroup
@@ -670,8 +670,8 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   // tile loads: thread -> (row, 16-byte chunk) of the tile, same for every tile
   // Rounds of the workgroup's loads that are a whole number of rows after which the chunk placement repeats apart differ in
   // their scalar base only: load i takes offset i % OFFSETS, ahead_rows(i) rows on (at head dim 256, whose rounds are a quarter of
-  // the period, four offsets in place of eight: bytes of scratch a lane 184 -> 116 for head dims 200 to 248, 8 x 2050 tokens, 16 heads
-  // of 208, 412 -> 310 us).  Where rows are no power of two long every load has its offset in a register.
+  // the period, four offsets in place of eight: 8 x 2050 tokens, 16 heads of 208, 412 -> 310 us when the kernel still spilled, 225
+  // now).  Where rows are no power of two long every load has its offset in a register.
   constexpr int ROUND_ROWS = SW::POW2 ? 64 * NW / CPR : 0;
   constexpr int OFFSETS = !SW::POW2 ? LOADS : ROUND_ROWS >= SW::PERIOD ? 1 : SW::PERIOD / ROUND_ROWS < LOADS ? SW::PERIOD / ROUND_ROWS : LOADS;
   static_assert(!SW::POW2 || (OFFSETS == LOADS || OFFSETS * ROUND_ROWS % SW::PERIOD == 0), "loads that share an offset share their chunk");
