@@ -84,8 +84,6 @@ struct PrepParams {
   int32_t nhead_k, weight_shift;
   int32_t *order_k;        // [nkb]: the k blocks by falling number of query rows that can see them
   int32_t weigh_k;         // 0: in their own order
-  uint32_t *copies;        // bit row copies of a split into nparts parts (at most 32), one array of bit rows after another; nparts 0: not split
-  int32_t nparts;
 };
 
 // Division by a launch constant d, exact for 0 <= n < 2^31: n / d == (n * m) >> s with
@@ -135,8 +133,9 @@ struct FwdParams {
   float *lse;             // optional [total_q, nhead_q] log-sum-exp output (nullptr: none)
   int64_t lse_s, lse_h;   // its strides in elements
   // Split over key blocks (few, long work items): every (kv head, q block, slot group) becomes
-  // nparts items, part i sees the bit row copy i (its share of the k blocks) and stores a
-  // normalised fp32 partial result and its log-sum-exp; hbsa_merge_kernel combines them.
+  // nparts items.  Part i sees its share of the kept k blocks and stores a normalised fp32 partial result and its log-sum-exp;
+  // hbsa_merge_kernel combines them.  An item of few keys has fewer parts (the others find nothing to do), or one, which
+  // writes the output itself.
   int32_t nparts;         // 1: no split
   FastDiv div_nparts;
   // One-launch form whose caller has not counted the blocks (the COUNTED kernels, in the place of what a split needs: 16 bytes more of
@@ -148,7 +147,7 @@ struct FwdParams {
     int32_t *counts;
   };
   union {
-    float *part_lse;        // [nparts, total_q, nhead_q]
+    float *part_lse;        // [nparts, total_q, nhead_q], and behind them int32 [total_q, nhead_q], the rows' numbers of parts
     int32_t count_info[2];
   };
   int32_t total_q, nhead_q;
@@ -430,6 +429,10 @@ struct ItemParts {
     count = (nvis + per - 1) / per;
     if (count < 1) count = 1;
   }
+  __device__ __forceinline__ uint32_t word_mask(int part, int j0) const {   // of a part's blocks among j0 .. j0 + 31
+    const int a = max(part * per - j0, 0), b = min((part + 1) * per - j0, 32);
+    return a < b ? (~0u << a) & (~0u >> (32 - b)) : 0u;
+  }
 };
 
 // Partial results travel between workgroups, and so between the chip's eight dies, whose L2 caches know nothing of each
@@ -542,8 +545,10 @@ template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream);
-template <int D, typename E>
+template <int D, typename E, bool PARTS>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
+int launch_fwd_parts(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_decode(const FwdParams &fp, int most, long long items, hipStream_t stream);
 template <int D>

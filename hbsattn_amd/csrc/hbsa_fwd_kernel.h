@@ -186,7 +186,7 @@ __device__ __forceinline__ int build_group_list(uint16_t *list, int chunk_base, 
 template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED, bool COUNTED>
 __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3 : 4) void hbsa_fwd_kernel(FwdParams p) {
   // OUT32: fp32 output (the fp32-input path; q/k/v are then fp16 staging copies)
-  // EXTRAS: the clocked walk, the split over key blocks and the log-sum-exp output are compiled in.  The
+  // EXTRAS: the split over key blocks is compiled in, and (not FUSED) the clocked walk and the log-sum-exp output.  The
   // plain call uses none of them, and its kernel is a tenth shorter without them (1-2 % faster: eight
   // wavefronts in different parts of a long kernel share one instruction cache).
   // FUSED: the one-launch form.  No pre-pass has run: wavefront 0 derives an item's geometry from the
@@ -218,6 +218,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   using SW = FwdSwizzle<D>;
   constexpr int KSTEPS = D / 16;       // MFMA k-steps of Q.K^T
   constexpr int DT = D / 32;           // 32-row tiles of O^T
+  constexpr bool WALK = EXTRAS && !FUSED;
   constexpr bool HAND = D <= 192;      // operand reads from LDS issued and waited for by hand (see lds_read_b128)
 
   extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -387,24 +388,33 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     return words;
   };
   // words of a later window of a row (rows longer than kMaskWindow blocks): fetched and waited for on the spot
-  auto fused_more_words = [&](const uint8_t *mrow, int nvis) {
-    return [&, mrow, nvis](int window) -> uint32_t {
+  auto fused_more_words = [&](const uint8_t *mrow, int nvis, int part) {
+    return [&, mrow, nvis, part](int window) -> uint32_t {
       const int first = window * kMaskWindow;
       const int count = min(kMaskWindow, nvis - first);
       if (count <= 0) return 0u;
       const int sh = mask_dma(mrow, first, count);
       __builtin_amdgcn_s_waitcnt(0x0F70);
       asm volatile("" : : : "memory");
-      return staged_words(sh, count);
+      uint32_t words = staged_words(sh, count);
+      if constexpr (EXTRAS) {   // (a row of several windows: cut by position)
+        if (nvis > kMaskWindow) words &= ItemParts(fresh_args(), nvis).word_mask(part, 32 * (window * 64 + lane));
+      }
+      return words;
     };
   };
   // the same for a prepared bit row in the workspace
-  auto prepared_more_words = [&](const uint32_t *row, int nwords) {
+  auto prepared_more_words = [&](const uint32_t *row, int nwords, int part, int kmax, int nkblk) {
     return [=](int window) -> uint32_t {
       const int i = window * 64 + lane;
       uint32_t held = i < nwords ? row[i] : 0u;
       __builtin_amdgcn_s_waitcnt(0x0F70);   // wait here, not (for everything in flight) on the common path
       asm volatile("" : "+v"(held));
+      if constexpr (EXTRAS) {
+        const FwdParams &p = fresh_args();
+        const int nvis = min(nkblk, (int)fast_div((uint32_t)(kmax + p.kbs - 1), p.div_kbs));
+        if (p.nparts > 1 && nvis > kMaskWindow) held &= ItemParts(p, nvis).word_mask(part, 32 * i);
+      }
       return held;
     };
   };
@@ -466,7 +476,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         st_ms = st_nvis > 0 ? mask_dma(st_mrow, 0, min(st_nvis, kMaskWindow)) : 0;
       } else {
         st_info = lane < 12 ? ((const uint32_t *)(p.info + st_qb))[lane] : 0u;
-        st_bits = lane < p.wpr ? p.bits[(((size_t)st_part * p.nhead_k + st_hk) * p.nqb + st_qb) * p.wpr + lane] : 0u;
+        st_bits = lane < p.wpr ? p.bits[((size_t)st_hk * p.nqb + st_qb) * p.wpr + lane] : 0u;
       }
     }
   };
@@ -478,26 +488,60 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     else
       return build_tile_list<KT>(lds_list + c * kListCap, chunk_base, more_words, nwords, p.kbs, p.div_kbs, kmax, first_words, lane);
   };
+  // Split over key blocks: part `part` sees a share of the item's kept k blocks, counted from the bit row, so that parts are of one
+  // length and an item of few keys is whole; a row of several windows of words is cut by position.
+  // words: lane i's word i of the row (of blocks below nvis); returns the part's, and how many parts the item has.
+  auto part_words = [&](uint32_t words, int nvis, int part, int &parts) -> uint32_t {
+    const FwdParams &p = fresh_args();
+    if (32 * lane >= nvis) words = 0u;   // (a prepared row is written as far as its sequence goes)
+    if (nvis > kMaskWindow) {
+      const ItemParts cut(p, nvis);
+      parts = cut.count;
+      return words & cut.word_mask(part, 32 * lane);
+    }
+    const int mine = __builtin_popcount(words);
+    int upto = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int x = __shfl_up(upto, off);
+      if (lane >= off) upto += x;
+    }
+    const ItemParts cut(p, __builtin_amdgcn_readlane(upto, 63));
+    parts = cut.count;
+    // kept blocks of this word before and after the part
+    int skip = min(max(part * cut.per - (upto - mine), 0), mine), drop = min(max(upto - (part + 1) * cut.per, 0), mine);
+    if (part >= parts || skip + drop >= mine) return 0u;
+    for (; skip > 0; --skip) words &= words - 1u;
+    for (; drop > 0; --drop) words &= ~(0x80000000u >> __builtin_clz(words));
+    return words;
+  };
   // expand the staged item into list `c` and write its header
   auto build = [&](int c) {
     const FwdParams &p = fresh_args();
     int *hdr = lds_hdr + c * H_WORDS;
-    int total = 0;
+    int total = 0, parts = 1;
     if (st_hk >= 0) {
       const int nkblk = __builtin_amdgcn_readlane((int)st_info, 6);
       const int kmax = __builtin_amdgcn_readlane((int)st_info, 7);
       if constexpr (FUSED) {
         // the staged bytes arrived with the wait of a tile, or one of the waits before the first item, since stage()
         st_bits = st_nvis > 0 ? staged_words(st_ms, min(st_nvis, kMaskWindow)) : 0u;
-        total = list_of(c, 0, fused_more_words(st_mrow, st_nvis), 2 * ((st_nvis + 63) >> 6), kmax, st_bits);
+        if constexpr (EXTRAS) {
+          st_bits = part_words(st_bits, st_nvis, st_part, parts);
+          if (st_sub * NW * kWaveRows >= p.ratio * __builtin_amdgcn_readlane((int)st_info, 1)) parts = 0;   // no rows, so no tiles
+        }
+        if (!EXTRAS || st_part < parts)
+          total = list_of(c, 0, fused_more_words(st_mrow, st_nvis, st_part), 2 * ((st_nvis + 63) >> 6), kmax, st_bits);
       } else {
         const int nwords = 2 * ((nkblk + 63) >> 6);
-        total = list_of(c, 0, prepared_more_words(p.bits + (((size_t)st_part * p.nhead_k + st_hk) * p.nqb + st_qb) * p.wpr, nwords),
-                        nwords, kmax, st_bits);
+        if (EXTRAS && p.nparts > 1) st_bits = part_words(st_bits, min(nkblk, (int)fast_div((uint32_t)(kmax + p.kbs - 1), p.div_kbs)), st_part, parts);
+        if (!EXTRAS || st_part < parts)
+          total = list_of(c, 0, prepared_more_words(p.bits + ((size_t)st_hk * p.nqb + st_qb) * p.wpr, nwords, st_part, kmax, nkblk), nwords, kmax, st_bits);
       }
     }
     if (lane == 0) {
-      hdr[H_HK] = st_hk; hdr[H_QB] = st_qb; hdr[H_SUB] = st_sub; hdr[H_PART] = st_part;
+      hdr[H_HK] = st_hk; hdr[H_QB] = st_qb; hdr[H_SUB] = st_sub;
+      hdr[H_PART] = EXTRAS ? st_part | parts << 8 : 0;
       hdr[H_TOTAL] = GROUPED ? (total + KT / 16 - 1) / (KT / 16) : total;
       if (GROUPED) hdr[H_GROUPS] = total;
       hdr[H_T0] = 0;   // the item's walk starts at its first tile unless next_start() decides otherwise
@@ -534,7 +578,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     const FwdParams &p = fresh_args();
     const int nkblk = __builtin_amdgcn_readlane((int)st_info, 6);
     const int seq = __builtin_amdgcn_readlane((int)st_info, 8);
-    w_part_of[c_] = EXTRAS && p.walk != 0 && st_hk >= 0 && total_ >= 3 && total_ <= kListCap;
+    w_part_of[c_] = WALK && p.walk != 0 && st_hk >= 0 && total_ >= 3 && total_ <= kListCap;
     w_clock_of[c_] = p.clock + (size_t)(st_hk < 0 ? 0 : st_hk) * p.nqb + seq;
     w_tiles_of[c_] = (nkblk * p.kbs + kTileKeys - 1) >> 6;
   };
@@ -1011,7 +1055,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   for (;;) {   // ------------------------------------------------------ one iteration per work item
     const int cur_hk = hdr_word(c, H_HK);
     const int cur_sub = hdr_word(c, H_SUB);
-    const int cur_part = hdr_word(c, H_PART);   // read now: wavefront 0 rewrites the header while others finish this item
+    const int cur_part = EXTRAS ? hdr_word(c, H_PART) & 255 : 0, cur_parts = EXTRAS ? hdr_word(c, H_PART) >> 8 : 1;   // read now: wavefront 0 rewrites the header while others finish this item
     const int total = hdr_word(c, H_TOTAL);
     const int row_begin = hdr_word(c, H_ROW_BEGIN);
     const int rows = hdr_word(c, H_ROWS);
@@ -1026,7 +1070,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     if (wave == 0) {   // stay one item ahead: expand the staged item, stage the one after it
       if (!settled) settle();   // (the staged item's mask bytes among what it waits for: no tile of the item before may have been waited for)
       build(c ^ 1);
-      if (EXTRAS && p.walk) note_item(c ^ 1, hdr_word(c ^ 1, H_TOTAL));
+      if (WALK && p.walk) note_item(c ^ 1, hdr_word(c ^ 1, H_TOTAL));
       stage();
       pending = claim();
       settled = false;
@@ -1106,7 +1150,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         // The clock is dealt with on few tiles only (wavefront 0; any work it does alone on every tile
         // makes the other three wait at the next barrier): the item's first tile, every eighth, and
         // the last three.
-        if (EXTRAS && p.walk && wave == 0 && ((t & (kWalkReportTiles - 1)) == 0 || chunk_base + t + 3 >= total)) {
+        if (WALK && p.walk && wave == 0 && ((t & (kWalkReportTiles - 1)) == 0 || chunk_base + t + 3 >= total)) {
           report(c, kpos, chunk_base + t == 0, t + t0 >= n ? 1 : 0);
           if (chunk_base + t + 3 == total) peek_next(c ^ 1);
           if (chunk_base + t + 2 == total) next_start(c ^ 1);
@@ -1335,16 +1379,25 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           int kb0;
           const QBlockInfo inf = fused_geometry(qb, kb0);
           const int nvis = min(inf.nkblk, (int)fast_div((uint32_t)(inf.kmax + p.kbs - 1), p.div_kbs));
-          auto more = fused_more_words(p.mask + (int64_t)cur_hk * p.ms_h + (int64_t)qb * p.ms_q + kb0, nvis);
-          const uint32_t first = more(0);
+          auto more = fused_more_words(p.mask + (int64_t)cur_hk * p.ms_h + (int64_t)qb * p.ms_q + kb0, nvis, cur_part);
+          uint32_t first = more(0);
+          if constexpr (EXTRAS) {
+            int parts;
+            first = part_words(first, nvis, cur_part, parts);
+          }
           (void)list_of(c, chunk_base, more, 2 * ((nvis + 63) >> 6), inf.kmax, first);
           // the staging area held the staged item's bytes: request them again (they arrive with the next tile's wait)
           if (st_hk >= 0 && st_nvis > 0) st_ms = mask_dma(st_mrow, 0, min(st_nvis, kMaskWindow));
         } else {
           const QBlockInfo inf = p.info[qb];
-          const uint32_t *row = p.bits + (((size_t)cur_part * p.nhead_k + cur_hk) * p.nqb + qb) * p.wpr;
+          const uint32_t *row = p.bits + ((size_t)cur_hk * p.nqb + qb) * p.wpr;
           const int nwords = 2 * ((inf.nkblk + 63) >> 6);
-          (void)list_of(c, chunk_base, prepared_more_words(row, nwords), nwords, inf.kmax, lane < nwords ? row[lane] : 0u);
+          uint32_t first = lane < nwords ? row[lane] : 0u;
+          if (EXTRAS && p.nparts > 1) {
+            int parts;
+            first = part_words(first, min(inf.nkblk, (int)fast_div((uint32_t)(inf.kmax + p.kbs - 1), p.div_kbs)), cur_part, parts);
+          }
+          (void)list_of(c, chunk_base, prepared_more_words(row, nwords, cur_part, inf.kmax, inf.nkblk), nwords, inf.kmax, first);
         }
       }
       __syncthreads();
@@ -1360,29 +1413,31 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     if (nxt_hk >= 0) request_q(nxt_hk, hdr_word(c ^ 1, H_SUB), hdr_word(c ^ 1, H_ROW_BEGIN), hdr_word(c ^ 1, H_ROWS));
 
     // ---- epilogue: normalise, convert, store (rows with no visible key store exact zeros)
-    if (active) {
+    if (active && (!EXTRAS || cur_part < cur_parts)) {
       const FwdParams &p = fresh_args();
       int hq, my_r;   // this lane's query (lanes l32 >= nrows repeat the last one and store nothing)
       slot_entry(slot, l32, rows, hq, my_r);
       const float l_tot = half_sum(l_run);
       const float inv = l_tot > 0.f ? __builtin_amdgcn_rcpf(l_tot) : 0.f;   // 1 ulp; a full division is ten instructions
-      if (EXTRAS && p.nparts > 1) {
+      if (EXTRAS && p.nparts > 1 && cur_part == 0 && g32 == 0 && l32 < nrows)   // the row's number of parts, behind the log-sum-exps
+        ((int32_t *)p.part_lse)[((int64_t)p.nparts * p.total_q + (row_begin + my_r)) * p.nhead_q + hq] = cur_parts;
+      if (EXTRAS && cur_parts > 1) {
         // split over key blocks: this part's normalised result and log-sum-exp, for the merge kernel
         if (l32 < nrows) {
           const int64_t rh = ((int64_t)cur_part * p.total_q + (row_begin + my_r)) * p.nhead_q + hq;
           if (g32 == 0)
             p.part_lse[rh] = l_tot > 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
-          float *dst = p.part_out + rh * D;
+          float *dst = p.part_out + rh * (COLS ? 8 * p.ncol : D);
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int i4 = 0; i4 < 4; ++i4) {
               f32x4 w = {o[dt][4 * i4 + 0] * inv, o[dt][4 * i4 + 1] * inv, o[dt][4 * i4 + 2] * inv, o[dt][4 * i4 + 3] * inv};
-              *(f32x4 *)(dst + dt * 32 + 8 * i4 + 4 * g32) = w;
+              if (!COLS || 4 * dt + i4 < p.ncol) *(f32x4 *)(dst + dt * 32 + 8 * i4 + 4 * g32) = w;
             }
         }
       } else {
-      if (EXTRAS && p.lse != nullptr && g32 == 0 && l32 < nrows) {
+      if (WALK && p.lse != nullptr && g32 == 0 && l32 < nrows) {
         // natural-log sum over the row's visible keys of exp(scale * q.k); m_ref is the (possibly
         // lagging) reference maximum the row sum was accumulated under, which makes this exact
         const float lse = l_tot > 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
@@ -1530,6 +1585,22 @@ int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream) {
   return fp.grouped ? launch_fused_tiles<D, E, true>(fp, items, stream) : launch_fused_tiles<D, E, false>(fp, items, stream);
 }
 
+// The one-launch form cut over key blocks: fp.nparts parts an item at most, put together by hbsa_merge_kernel.  In place of pre-pass, a bit row
+// copy for each part, attention and merge: three launches, and the mask read and written once more.  Slots are packed here, which leaves
+// whole workgroups of ragged q blocks without rows and so without tiles.  us, before and after, one job: 2 x 300 .. 512 queries on 65000
+// keys, 32 / 8 heads of 128, 267 -> 234 (q blocks of 4 and 70 rows among them); 512 on 32000 93 -> 79; 2 x 146 .. 292 on 9000 .. 17000, 32 / 8 of
+// 64, 35.5 -> 27.2; 40 .. 80 on 8000, 8 / 1 of 64, 19.3 -> 15.8; head dim 80, 4 x 2700 .. 3900 tokens, one head, 84 -> 27.
+template <int D, typename E>
+int launch_fwd_parts(const FwdParams &fp, long long items, hipStream_t stream) {
+  if constexpr (D == 128) {
+    if (fp.nw == 8)
+      return fp.grouped ? launch_fwd_nw<D, E, false, 8, true, true, true, false, true>(fp, items, stream)
+                        : launch_fwd_nw<D, E, false, 8, true, true, true>(fp, items, stream);
+  }
+  return fp.grouped ? launch_fwd_nw<D, E, false, 4, true, true, true, false, true>(fp, items, stream)
+                    : launch_fwd_nw<D, E, false, 4, true, true, true>(fp, items, stream);
+}
+
 // the one-launch form that counts the blocks itself, workgroups of four wavefronts
 template <int D, typename E>
 int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream) {
@@ -1541,12 +1612,12 @@ int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream)
 }
 
 // the one-launch form for tensors whose head dim (fp.ncol chunks of eight elements) is D or less
-template <int D, typename E>
+template <int D, typename E, bool PARTS>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream) {
   // (a load of rows whose length is no power of two can span two groups: the lanes' offsets have to reach from one to the other)
   const bool reaches = 1024 % (2 * D) == 0 || (uint64_t)fp.wpr * 32u * (uint64_t)fp.kbs * (uint64_t)std::max(fp.k_s, fp.v_s) < (1ull << 32);
-  if (fp.grouped && reaches) return launch_fwd_nw<D, E, false, 4, false, true, true, true, true>(fp, items, stream);
-  return launch_fwd_nw<D, E, false, 4, false, true, true, true>(fp, items, stream);
+  if (fp.grouped && reaches) return launch_fwd_nw<D, E, false, 4, PARTS, true, true, true, true>(fp, items, stream);
+  return launch_fwd_nw<D, E, false, 4, PARTS, true, true, true>(fp, items, stream);
 }
 
 }  // namespace hbsa

@@ -131,9 +131,15 @@ bool plain_forward(const Problem &p, hipStream_t stream, at::Tensor &out, CountT
     return true;
   }
   if (!native_dim(p.q.size(2))) {
-    const int rc = hbsa_fwd_one(ptrs, sizes, (float)p.scale, strides, stream);
-    if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) return false;   // no single launch: the caller pads
-    if (rc != 0) raise("hbsa_fwd_one", rc);
+    const size_t n = parts_bytes(p) == 0 ? 0 : workspace_bytes(p);
+    at::Tensor ws;
+    if (n != 0) {
+      ws = bytes_like(p.q, n);
+      ptrs[10] = ws.mutable_data_ptr();
+    }
+    const int rc = hbsa_fwd_any(ptrs, n, sizes, (float)p.scale, strides, stream);
+    if (rc == HBSA_ERR_WORKSPACE_TOO_SMALL) return false;   // neither form that reads such rows: the caller pads
+    if (rc != 0) raise("hbsa_fwd_any", rc);
     return true;
   }
   int rc = HBSA_ERR_WORKSPACE_TOO_SMALL;
@@ -142,7 +148,7 @@ bool plain_forward(const Problem &p, hipStream_t stream, at::Tensor &out, CountT
     const size_t n = workspace_bytes(p);
     at::Tensor ws = bytes_like(p.q, n);
     ptrs[10] = ws.mutable_data_ptr();
-    rc = hbsa_fwd_v(ptrs, n, sizes, (float)p.scale, strides, stream);
+    rc = hbsa_fwd_any(ptrs, n, sizes, (float)p.scale, strides, stream);
   }
   if (rc != 0) raise("hbsa_fwd", rc);
   return true;

@@ -249,6 +249,11 @@ int hbsa_fwd_v(const void *const *ptrs, size_t workspace_bytes, const int32_t *s
  */
 int hbsa_fwd_one(const void *const *ptrs, const int32_t *sizes, float softmax_scale, const int64_t *strides, void *stream);
 
+/* hbsa_fwd_v for a caller that looks for nothing in the workspace afterwards (0 bytes: none), for any head dim that hbsa_fwd_one takes: a
+ * call whose work is cut over its key blocks then has no pre-pass, only the attention launch and the merge.  HBSA_ERR_WORKSPACE_TOO_SMALL, and
+ * nothing launched, also where another head dim than 32, 64, 128 and 256 needs the two-launch form. */
+int hbsa_fwd_any(const void *const *ptrs, size_t workspace_bytes, const int32_t *sizes, float softmax_scale, const int64_t *strides, void *stream);
+
 /* hbsa_fwd_one for a caller that has not counted the blocks: cu_num_q_block, cu_num_k_block or both may be NULL in `ptrs`, and are then
  * counted by the launch itself.  `counts` is as in hbsa_block_counts, 16-byte aligned; the launch writes counts[2] = 1 when no length is
  * negative and the totals are sizes' num_q_block and num_k_block, else 0 (the output is then undefined, nothing out of range is touched), and
