@@ -183,7 +183,7 @@ __device__ __forceinline__ int build_group_list(uint16_t *list, int chunk_base, 
   return total;
 }
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED, bool COUNTED>
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED, bool COUNTED, bool ONE>
 __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3 : 4) void hbsa_fwd_kernel(FwdParams p) {
   // OUT32: fp32 output (the fp32-input path; q/k/v are then fp16 staging copies)
   // EXTRAS: the split over key blocks is compiled in, and (not FUSED) the clocked walk and the log-sum-exp output.  The
@@ -202,6 +202,12 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   // masked (blocks of 48 keys, half of them kept: 120 keys' worth of tiles for 96, half of the tiles masked).
   // COUNTED: (FUSED) the caller has not counted the blocks; see FwdParams::counts.  Kernels of their own: compiled in everywhere, the
   // counting cost calls that do not use it 1 % (16 x 40 .. 500 tokens, 32 / 8 heads, 37.7 -> 38.0 us; 8 x 2050, 16 of 192, 227.6 -> 229.7).
+  // ONE: (FUSED) no workgroup has a second item: nothing is staged, listed or claimed for one, and there is that much less code to fetch
+  // before the first tile, at 0.1 us a cold line.  A third of a call of a few tiles is the scheduler's code: us, before and after, 2 x 27 tokens, 16 / 8
+  // heads of 32, 8.0 -> 7.2; 2 x 54 .. 72, 32 / 16, 9.3 -> 8.4; 8 x 149 .. 240, 2 heads, 10.6 -> 9.7; 1 x 204 .. 512, 32 / 16 of 128, 15.2 -> 14.5.
+  // (A kernel of its own, with packed slots, which give the same bits: as a branch it cost launches of two and more items 0.7 % at head dim
+  // 128, 35.0 -> 35.3 and 64.0 -> 64.5; the COUNTED and COLS kernels and the split ones of four wavefronts,
+  // where nothing got slower, have the branch; split ones of eight, whose items are long, lost 1 % with it.)
   // NW: wavefronts (wave slots) of a workgroup, 4 or 8.  Eight are used when the q heads of a GQA group
   // and the 32-row slices of a q block give an item more than four wave slots: one workgroup per CU then
   // stages every K/V tile once for all of them instead of two workgroups staging it each (D = 128 only, and
@@ -644,6 +650,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     w_ptr = nullptr;
   };
 
+  constexpr bool MAY_ONE = COUNTED || COLS || (FUSED && EXTRAS && NW == 4);
+  const bool one = ONE || (MAY_ONE && p.one_each != 0 && p.one_each <= (int)gridDim.x);
+  const bool schedules = wave == 0 && !one;
   if constexpr (COLS) {
     for (int i = threadIdx.x; i < 4 * TILE_BYTES / 16; i += NW * 64) *(u32x4 *)(lds_k + i * 16) = u32x4{0u, 0u, 0u, 0u};
   }
@@ -704,11 +713,14 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     }
     build(0);
     note_item(0, hdr_word(0, H_TOTAL));
-    pending = claim();
-    stage();
-    pending = claim();
+    if (schedules) {
+      pending = claim();
+      stage();
+      pending = claim();
+    } else if (lane == 0) {
+      lds_hdr[H_WORDS + H_HK] = -1;
+    }
   }
-  __syncthreads();
 
   // ------------------------------------------------------------------ per-thread constants
   // tile loads: thread -> (row, 16-byte chunk) of the tile, same for every tile
@@ -837,10 +849,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       }
       static_for<0, LOADS>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
-        constexpr bool ONE = 1024 % RB == 0;
+        constexpr bool WHOLE = 1024 % RB == 0;
         constexpr int ROUND = NW * 64 / CPR;   // rows between two loads
         const int row = ((i * NW + wave_) * 64 + lane) / CPR;
-        int g = ONE ? ((wave_ * 64 / CPR) >> 4) + i * ROUND / 16 : ((i * NW + wave_) * 64 / CPR) >> 4;
+        int g = WHOLE ? ((wave_ * 64 / CPR) >> 4) + i * ROUND / 16 : ((i * NW + wave_) * 64 / CPR) >> 4;
         uint32_t voff = V_PART ? ld_voff[i % OFFSETS] : ld_koff[i % OFFSETS];
         if (valid < KT) {
           g = min(g, (valid - 1) >> 4);
@@ -849,7 +861,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           voff += step;
         }
         const uint32_t pos = group_at(g);
-        if constexpr (!ONE) {
+        if constexpr (!WHOLE) {
           const int second = 16 * (g + 1) * CPR - (i * NW + wave_) * 64;   // first lane of the second group, if one of them is
           voff += lane >= second ? (group_at(min(g + 1, (valid - 1) >> 4)) - pos) * stride : 0u;
         }
@@ -1036,9 +1048,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   };
 
   // ------------------------------------------------------------------ first item
+  __syncthreads();   // (the other wavefronts have done what is above while wavefront 0 made the list, and its code is there)
   int c = 0;   // list / header of the current item
   if (hdr_word(0, H_HK) < 0) {
-    leave();
+    if (!ONE) leave();
     return;
   }
   if (hdr_word(0, H_TOTAL) > 0) issue_first(0, 0);
@@ -1067,7 +1080,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     // place its part of that tile is there as well.  What the scheduler asks for below then has the first tile's time to arrive.
     // (In every wavefront: the compiler then knows that these loads have arrived.)
     place_q();
-    if (wave == 0) {   // stay one item ahead: expand the staged item, stage the one after it
+    if (schedules) {   // stay one item ahead: expand the staged item, stage the one after it
       if (!settled) settle();   // (the staged item's mask bytes among what it waits for: no tile of the item before may have been waited for)
       build(c ^ 1);
       if (WALK && p.walk) note_item(c ^ 1, hdr_word(c ^ 1, H_TOTAL));
@@ -1156,7 +1169,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           if (chunk_base + t + 2 == total) next_start(c ^ 1);
           if (last) leave_clock();
         }
-        if (__builtin_expect(last, 0)) {
+        if (!ONE && __builtin_expect(last, 0)) {
           nxt_hk = hdr_word(c ^ 1, H_HK);
           if (nxt_hk >= 0 && hdr_word(c ^ 1, H_TOTAL) > 0) {
             nx = listed_tile(c ^ 1, GROUPED ? 0 : hdr_word(c ^ 1, H_T0), 0);
@@ -1387,7 +1400,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
           }
           (void)list_of(c, chunk_base, more, 2 * ((nvis + 63) >> 6), inf.kmax, first);
           // the staging area held the staged item's bytes: request them again (they arrive with the next tile's wait)
-          if (st_hk >= 0 && st_nvis > 0) st_ms = mask_dma(st_mrow, 0, min(st_nvis, kMaskWindow));
+          if (!ONE && st_hk >= 0 && st_nvis > 0) st_ms = mask_dma(st_mrow, 0, min(st_nvis, kMaskWindow));
         } else {
           const QBlockInfo inf = p.info[qb];
           const uint32_t *row = p.bits + ((size_t)cur_hk * p.nqb + qb) * p.wpr;
@@ -1497,7 +1510,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     }
 
     // ---- move on to the next item
-    if (total == 0) {
+    if (!ONE && total == 0) {
       // No tile, hence no barrier since this item began: the next list may still be being written,
       // and nothing of the next item has been requested yet.
       w_next_lap = -1;   // (nor has its walk been given a start: it takes no part in the clock)
@@ -1510,10 +1523,10 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       }
       __syncthreads();   // wave 0 rewrites this item's list next; every wave has read its header by now
     }
-    if (nxt_hk < 0) break;
+    if (ONE || nxt_hk < 0) break;
     c ^= 1;
   }
-  leave();
+  if (!ONE) leave();
 }
 
 inline int persistent_grid(const void *kernel, int lds_bytes, int threads) {
@@ -1527,10 +1540,10 @@ inline int persistent_grid(const void *kernel, int lds_bytes, int threads) {
 }
 
 template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false, bool COLS = false, bool GROUPED = false,
-          bool COUNTED = false>
+          bool COUNTED = false, bool ONE = false>
 int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   constexpr int lds_bytes = 4 * (D > 128 && D <= 192 ? 32 : 64) * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
-  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED>);
+  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED, ONE>);
   // workgroups that fit the current device at once; the attribute and the occupancy are per device
   static thread_local int resident_of[kMaxDevices] = {};
   int dev = 0;
@@ -1543,13 +1556,16 @@ int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
     resident = persistent_grid(kernel, lds_bytes, NW * 64);
     if (resident <= 0) return fail(HBSA_ERR_UNSUPPORTED, "could not size the persistent grid");
   }
+  if constexpr (FUSED && NW == 4 && !EXTRAS && !COLS && !COUNTED && !ONE) {
+    if (items <= resident) return launch_fwd_nw<D, E, false, 4, false, true, true, false, GROUPED, false, true>(fp, items, stream);
+  }
   const int grid = (int)(items < resident ? items : resident);
   FwdParams launch = fp;
   // Few items per workgroup: a fixed order instead of the per-XCD queues, whose round trips (and, with few kv
   // heads, the crowd at few counters) would be a good part of such a launch.
   launch.one_each = items <= (long long)kStaticShare * resident ? (int)items : 0;
   if (launch.one_each == 0 || launch.nparts != 1 || items <= resident) launch.order = nullptr;
-  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
+  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED, ONE>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, "hbsa_fwd_kernel launch: %s", hipGetErrorString(e));
   return 0;
