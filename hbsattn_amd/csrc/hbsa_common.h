@@ -84,6 +84,7 @@ struct PrepParams {
   int32_t nhead_k, weight_shift;
   int32_t *order_k;        // [nkb]: the k blocks by falling number of query rows that can see them
   int32_t weigh_k;         // 0: in their own order
+  int32_t shared_tiles;    // for the launch record
 };
 
 // Division by a launch constant d, exact for 0 <= n < 2^31: n / d == (n * m) >> s with
@@ -169,6 +170,7 @@ struct FwdParams {
   int32_t parts_last;    // workgroups are numbered by part first (else: the parts of an item are neighbours)
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
   int32_t split;         // host side only: parts of the split over key blocks that pay (fwd_split)
+  int32_t teams;         // host side only: two teams for the tiles of every item (fwd_teams)
   int32_t grouped;       // host side only: tiles of 16-key groups (the GROUPED form of the kernel)
   // Items handed out without queues in the order of their weights (see OrderRoom), nullptr: last q blocks first
   const uint32_t *order;         // [num_q_block * nhead_k]: q block << 16 | kv head, heaviest first
@@ -271,7 +273,8 @@ struct Sched {
   // bit patterns of max|x| over q, k, v and the power-of-two staging multipliers
   uint32_t amax[3];
   float in_mul[3];
-  uint32_t pad[47];
+  uint32_t shared_tiles;   // prepared masks: teams may share an item's tiles (team_sequences)
+  uint32_t pad[46];
 };
 static_assert(sizeof(Sched) == 256, "Sched is one 256-byte slot of the workspace");
 
@@ -545,8 +548,10 @@ template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream);
-template <int D, typename E, bool PARTS>
+template <int D, typename E, bool PARTS, int TEAMS>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
+int launch_fwd_teams(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_parts(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>

@@ -43,6 +43,7 @@ constexpr int kGroupCap = 2 * kListCap;   // GROUPED: 16-bit entries of a list, 
 // Bytes of the one-launch form's staging area for one row of block_mask bytes (2048 blocks and the alignment slack)
 constexpr int kMaskWindow = 2048;
 constexpr int kMaskStage = kMaskWindow + 256;
+constexpr int kTeamTiles = 6;   // tiles of an item that teams share, at least
 constexpr float kMostSum = 256.f;   // 2^kLazyRescaleLog2
 static_assert(kLazyRescaleLog2 == 8.0f, "kMostSum");
 
@@ -183,8 +184,8 @@ __device__ __forceinline__ int build_group_list(uint16_t *list, int chunk_base, 
   return total;
 }
 
-template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED, bool COUNTED, bool ONE>
-__global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3 : 4) void hbsa_fwd_kernel(FwdParams p) {
+template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED, bool PACK, bool COLS, bool GROUPED, bool COUNTED, bool ONE, int TEAMS>
+__global__ __launch_bounds__(NW * TEAMS * 64, TEAMS > 1 || D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3 : 4) void hbsa_fwd_kernel(FwdParams p) {
   // OUT32: fp32 output (the fp32-input path; q/k/v are then fp16 staging copies)
   // EXTRAS: the split over key blocks is compiled in, and (not FUSED) the clocked walk and the log-sum-exp output.  The
   // plain call uses none of them, and its kernel is a tenth shorter without them (1-2 % faster: eight
@@ -208,6 +209,9 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   // (A kernel of its own, with packed slots, which give the same bits: as a branch it cost launches of two and more items 0.7 % at head dim
   // 128, 35.0 -> 35.3 and 64.0 -> 64.5; the COUNTED and COLS kernels and the split ones of four wavefronts,
   // where nothing got slower, have the branch; split ones of eight, whose items are long, lost 1 % with it.)
+  // TEAMS: (ONE) the item's tiles are shared out among this many teams of NW wavefronts, each with tile buffers of its own, tile i to team
+  // i % TEAMS; their sums are put together through LDS at the end.  For launches that leave SIMDs with one wavefront: alone there, its tile is a
+  // chain of matrix products, exponentials and LDS reads with nothing beside them (see fwd_teams).
   // NW: wavefronts (wave slots) of a workgroup, 4 or 8.  Eight are used when the q heads of a GQA group
   // and the 32-row slices of a q block give an item more than four wave slots: one workgroup per CU then
   // stages every K/V tile once for all of them instead of two workgroups staging it each (D = 128 only, and
@@ -224,19 +228,21 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
   using SW = FwdSwizzle<D>;
   constexpr int KSTEPS = D / 16;       // MFMA k-steps of Q.K^T
   constexpr int DT = D / 32;           // 32-row tiles of O^T
-  constexpr bool WALK = EXTRAS && !FUSED;
+  constexpr bool WALK = EXTRAS && !FUSED && !ONE, LSE = EXTRAS && !FUSED;
+  static_assert(TEAMS == 1 || ONE, "the tiles of one item");
   constexpr bool HAND = D <= 192;      // operand reads from LDS issued and waited for by hand (see lds_read_b128)
 
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  char *lds_k = lds;
-  int *lds_hdr = (int *)(lds + 4 * TILE_BYTES);     // [2][H_WORDS]
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int team = TEAMS > 1 ? wave_all / NW : 0, wave = TEAMS > 1 ? wave_all % NW : wave_all;
+  char *lds_k = lds + team * 4 * TILE_BYTES;
+  int *lds_hdr = (int *)(lds + TEAMS * 4 * TILE_BYTES);     // [2][H_WORDS]
   int *lds_list = lds_hdr + 2 * H_WORDS;            // [2][kListCap]
   int *lds_seq = lds_list + 2 * kListCap;           // FUSED: [4][kSeqCap] cu_q, cu_k, cu_num_q_block, cu_num_k_block
   uint8_t *lds_mask = (uint8_t *)(lds_seq + 4 * kSeqCap);   // FUSED: [kMaskStage] block_mask bytes of the staged item
   auto hdr_word = [&](int c_, int i) { return __builtin_amdgcn_readfirstlane(lds_hdr[c_ * H_WORDS + i]); };
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g32 = lane >> 5;   // which half of the wavefront
   const int l32 = lane & 31;   // query within the wave slot / key row within a sub-tile
 
@@ -652,11 +658,11 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
 
   constexpr bool MAY_ONE = COUNTED || COLS || (FUSED && EXTRAS && NW == 4);
   const bool one = ONE || (MAY_ONE && p.one_each != 0 && p.one_each <= (int)gridDim.x);
-  const bool schedules = wave == 0 && !one;
+  const bool schedules = wave_all == 0 && !one;
   if constexpr (COLS) {
-    for (int i = threadIdx.x; i < 4 * TILE_BYTES / 16; i += NW * 64) *(u32x4 *)(lds_k + i * 16) = u32x4{0u, 0u, 0u, 0u};
+    for (int i = threadIdx.x; i < TEAMS * 4 * TILE_BYTES / 16; i += NW * TEAMS * 64) *(u32x4 *)(lds + i * 16) = u32x4{0u, 0u, 0u, 0u};
   }
-  if (wave == 0) {
+  if (wave_all == 0) {
     if constexpr (FUSED) {   // the sequences' boundaries, for fused_geometry()
       for (int i = lane; i <= p.batch; i += 64) {
         lds_seq[i] = p.cu_q[i];
@@ -1054,8 +1060,19 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     if (!ONE) leave();
     return;
   }
-  if (hdr_word(0, H_TOTAL) > 0) issue_first(0, 0);
-  request_q(hdr_word(0, H_HK), hdr_word(0, H_SUB), hdr_word(0, H_ROW_BEGIN), hdr_word(0, H_ROWS));
+  // tiles of a step of all teams; a short list is the first team's alone
+  const int step = TEAMS > 1 && hdr_word(0, H_TOTAL) >= kTeamTiles && (FUSED || p.sched->shared_tiles != 0) ? TEAMS : 1;
+  const int off = step > 1 ? team : team > 0 ? 0x3fffffff : 0;   // the team's first tile
+  if constexpr (TEAMS > 1) {
+    if (off < hdr_word(0, H_TOTAL)) {
+      const TileRef tile = listed_tile(0, off, 0);
+      issue_k(0, item_k(0), tile);
+      issue_v(0, item_v(0), tile);
+    }
+  } else if (hdr_word(0, H_TOTAL) > 0) {
+    issue_first(0, 0);
+  }
+  if (TEAMS == 1 || team == 0 || step > 1) request_q(hdr_word(0, H_HK), hdr_word(0, H_SUB), hdr_word(0, H_ROW_BEGIN), hdr_word(0, H_ROWS));
   // What this wavefront asked for so far has arrived, the scheduler's records included: the compiler is told here, or it
   // waits for ALL outstanding memory traffic where they are first read.
   bool settled = false;   // ... since the scheduler last asked for something
@@ -1102,7 +1119,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     }
     const int wave_kvis_min = q_pos + slot.min_r + shift;
     const int wave_kvis_max = q_pos + slot.max_r + shift;
-    const bool active = nrows > 0;
+    const bool active = nrows > 0 && (TEAMS == 1 || team == 0 || step > 1);
 
     f32x16 o[DT];
 #pragma unroll
@@ -1138,22 +1155,24 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
                         GROUPED ? (uint32_t)__builtin_amdgcn_readlane((int)from.y, lane_at) : 0u, c, chunk_base + x, total);
       };
       held = entry_of(0);
-      TileRef nx_tile = held_tile(held, 0, 0);
-      for (int t = 0; t < n; ++t) {   // ---------------------------------- one iteration per 64-key tile
+      TileRef nx_tile = {0, 0, 0u, 0u};
+      if (TEAMS == 1 || off < n) nx_tile = held_tile(held, TEAMS > 1 ? off : 0, TEAMS > 1 ? off : 0);
+      for (int t = 0; t < n; t += TEAMS > 1 ? step : 1) {   // ---------------------------------- one iteration per 64-key tile
         const TileRef tile = nx_tile;
         const int kpos = tile.first, valid = tile.valid;
-        const bool more = t + 1 < n, last = chunk_base + t + 1 == total;
+        const int t_next = TEAMS > 1 ? t + off + step : t + 1;
+        const bool more = t_next < n, last = chunk_base + t + 1 == total;
         // The next tile is looked up before the wait, and what is rare stands out of line: between the barrier and the tile's first
         // products none of the workgroup's wavefronts has work for the matrix cores, and scalar code there, taken branches above
         // all, is paid by every one of them (some 70 scalar instructions and six taken branches before, 30 and one here: 16 x 40 .. 500
         // tokens, 32 / 8 heads of 128, 35.4 -> 34.7 us; two chunks on 65000 keys 268 -> 262; 8 x 2050, 16 heads of 192, 215 -> 211).
         TileRef nx = {0, 0, 0u, 0u};      // valid > 0: a next tile exists and its loads go out during this tile
         if (__builtin_expect(more, 1)) {
-          if (__builtin_expect(((t + 1) & 63) == 0, 0)) held = entry_of(t + 1);
-          nx = held_tile(held, (t + 1) & 63, t + 1);
+          if (__builtin_expect((t_next & 63) < (TEAMS > 1 ? step : 1), 0)) held = entry_of(t_next & ~63);
+          nx = held_tile(held, t_next & 63, t_next);
         }
         const char *nx_k = kg, *nx_v = vg;
-        const bool compute = active && (!p.causal || kpos <= wave_kvis_max);
+        const bool compute = active && (TEAMS == 1 || t + off < n) && (!p.causal || kpos <= wave_kvis_max);
         // keys that are missing, or (causal) a last key that some lane's query does not see
         const bool edge = valid < KT || (p.causal && tile.pos(KT / 16 - 1) + 15 > wave_kvis_min);
 
@@ -1384,7 +1403,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
       if (chunk_base >= total) break;
       // a longer item: expand the next chunk of its tile list in place
       __syncthreads();
-      if (wave == 0) {
+      if (wave_all == 0) {
         // (the staged records now belong to a later item, so this item's are fetched again)
         const FwdParams &p = fresh_args();
         const int qb = hdr_word(c, H_QB);
@@ -1414,8 +1433,8 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
         }
       }
       __syncthreads();
-      {   // nothing is in flight here: fetch the chunk's first tile
-        const TileRef tile = listed_tile(c, 0, chunk_base);
+      if (TEAMS == 1 || off < total - chunk_base) {   // nothing is in flight here: fetch the chunk's first tile
+        const TileRef tile = listed_tile(c, TEAMS > 1 ? off : 0, chunk_base);
         issue_k(buf, kg, tile);
         issue_v(buf, vg, tile);
       }
@@ -1425,8 +1444,39 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
     // (outside of the tile loop, or the compiler waits for them inside it)
     if (nxt_hk >= 0) request_q(nxt_hk, hdr_word(c ^ 1, H_SUB), hdr_word(c ^ 1, H_ROW_BEGIN), hdr_word(c ^ 1, H_ROWS));
 
+    if constexpr (TEAMS > 1) {   // the teams' sums: to the larger of their references, in the order of the teams
+      static_assert((DT * 4 + 1) * 1024 <= 8 * TILE_BYTES / (TEAMS > 1 ? NW : 1), "the sums of a team fit its and the first team's tile buffers");
+      if (step > 1) {
+        f32x4 *sums = (f32x4 *)lds + wave * (DT * 4 + 1) * 64 + lane;
+        __syncthreads();   // no tile is read any more
+        if (team > 0 && active) {
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sums[(dt * 4 + i) * 64] = f32x4{o[dt][4 * i], o[dt][4 * i + 1], o[dt][4 * i + 2], o[dt][4 * i + 3]};
+          sums[DT * 4 * 64] = f32x4{m_ref, l_run, 0.f, 0.f};
+        }
+        __syncthreads();
+        if (team == 0 && active) {
+          const f32x4 ml = sums[DT * 4 * 64];
+          const float m = fmaxf(m_ref, ml[0]);
+          const float mine = m_ref == m ? 1.f : __builtin_amdgcn_exp2f(m_ref - m), other = ml[0] == m ? 1.f : __builtin_amdgcn_exp2f(ml[0] - m);
+          m_ref = m;
+          l_run = l_run * mine + ml[1] * other;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const f32x4 x = sums[(dt * 4 + i) * 64];
+#pragma unroll
+              for (int j = 0; j < 4; ++j) o[dt][4 * i + j] = o[dt][4 * i + j] * mine + x[j] * other;
+            }
+        }
+      }
+    }
+
     // ---- epilogue: normalise, convert, store (rows with no visible key store exact zeros)
-    if (active && (!EXTRAS || cur_part < cur_parts)) {
+    if (active && (TEAMS == 1 || team == 0) && (!EXTRAS || cur_part < cur_parts)) {
       const FwdParams &p = fresh_args();
       int hq, my_r;   // this lane's query (lanes l32 >= nrows repeat the last one and store nothing)
       slot_entry(slot, l32, rows, hq, my_r);
@@ -1450,7 +1500,7 @@ __global__ __launch_bounds__(NW * 64, D > 192 ? 1 : D > 64 ? 8 / NW : D > 32 ? 3
             }
         }
       } else {
-      if (WALK && p.lse != nullptr && g32 == 0 && l32 < nrows) {
+      if (LSE && p.lse != nullptr && g32 == 0 && l32 < nrows) {
         // natural-log sum over the row's visible keys of exp(scale * q.k); m_ref is the (possibly
         // lagging) reference maximum the row sum was accumulated under, which makes this exact
         const float lse = l_tot > 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
@@ -1540,10 +1590,10 @@ inline int persistent_grid(const void *kernel, int lds_bytes, int threads) {
 }
 
 template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false, bool PACK = false, bool COLS = false, bool GROUPED = false,
-          bool COUNTED = false, bool ONE = false>
+          bool COUNTED = false, bool ONE = false, int TEAMS = 1>
 int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
-  constexpr int lds_bytes = 4 * (D > 128 && D <= 192 ? 32 : 64) * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
-  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED, ONE>);
+  constexpr int lds_bytes = TEAMS * 4 * (D > 128 && D <= 192 ? 32 : 64) * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
+  const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED, ONE, TEAMS>);
   // workgroups that fit the current device at once; the attribute and the occupancy are per device
   static thread_local int resident_of[kMaxDevices] = {};
   int dev = 0;
@@ -1553,19 +1603,19 @@ int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   if (resident == 0) {
     hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (e != hipSuccess) return fail((int)e, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-    resident = persistent_grid(kernel, lds_bytes, NW * 64);
+    resident = persistent_grid(kernel, lds_bytes, NW * TEAMS * 64);
     if (resident <= 0) return fail(HBSA_ERR_UNSUPPORTED, "could not size the persistent grid");
   }
   if constexpr (FUSED && NW == 4 && !EXTRAS && !COLS && !COUNTED && !ONE) {
     if (items <= resident) return launch_fwd_nw<D, E, false, 4, false, true, true, false, GROUPED, false, true>(fp, items, stream);
   }
-  const int grid = (int)(items < resident ? items : resident);
+  const int grid = (int)(ONE || items < resident ? items : resident);
   FwdParams launch = fp;
   // Few items per workgroup: a fixed order instead of the per-XCD queues, whose round trips (and, with few kv
   // heads, the crowd at few counters) would be a good part of such a launch.
-  launch.one_each = items <= (long long)kStaticShare * resident ? (int)items : 0;
+  launch.one_each = ONE || items <= (long long)kStaticShare * resident ? (int)items : 0;
   if (launch.one_each == 0 || launch.nparts != 1 || items <= resident) launch.order = nullptr;
-  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED, ONE>), dim3(grid), dim3(NW * 64), lds_bytes, stream, launch);
+  hipLaunchKernelGGL((hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED, ONE, TEAMS>), dim3(grid), dim3(NW * TEAMS * 64), lds_bytes, stream, launch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail((int)e, "hbsa_fwd_kernel launch: %s", hipGetErrorString(e));
   return 0;
@@ -1627,13 +1677,26 @@ int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream)
                  : launch_fwd_nw<D, E, false, 4, false, true, false, false, false, true>(fp, items, stream);
 }
 
+// Two teams for the tiles of an item (see fwd_teams): the one-launch form, that counts the blocks or not, and the prepared form
+template <int D, typename E>
+int launch_fwd_teams(const FwdParams &fp, long long items, hipStream_t stream) {
+  if (fp.info != nullptr)
+    return fp.grouped ? launch_fwd_nw<D, E, false, 4, true, false, false, false, true, false, true, 2>(fp, items, stream)
+                      : launch_fwd_nw<D, E, false, 4, true, false, false, false, false, false, true, 2>(fp, items, stream);
+  if (fp.counts != nullptr)
+    return fp.grouped ? launch_fwd_nw<D, E, false, 4, false, true, true, false, true, true, true, 2>(fp, items, stream)
+                      : launch_fwd_nw<D, E, false, 4, false, true, true, false, false, true, true, 2>(fp, items, stream);
+  return fp.grouped ? launch_fwd_nw<D, E, false, 4, false, true, true, false, true, false, true, 2>(fp, items, stream)
+                    : launch_fwd_nw<D, E, false, 4, false, true, true, false, false, false, true, 2>(fp, items, stream);
+}
+
 // the one-launch form for tensors whose head dim (fp.ncol chunks of eight elements) is D or less
-template <int D, typename E, bool PARTS>
+template <int D, typename E, bool PARTS, int TEAMS>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream) {
   // (a load of rows whose length is no power of two can span two groups: the lanes' offsets have to reach from one to the other)
   const bool reaches = 1024 % (2 * D) == 0 || (uint64_t)fp.wpr * 32u * (uint64_t)fp.kbs * (uint64_t)std::max(fp.k_s, fp.v_s) < (1ull << 32);
-  if (fp.grouped && reaches) return launch_fwd_nw<D, E, false, 4, PARTS, true, true, true, true>(fp, items, stream);
-  return launch_fwd_nw<D, E, false, 4, PARTS, true, true, true>(fp, items, stream);
+  if (fp.grouped && reaches) return launch_fwd_nw<D, E, false, 4, PARTS, true, true, true, true, false, (TEAMS > 1), TEAMS>(fp, items, stream);
+  return launch_fwd_nw<D, E, false, 4, PARTS, true, true, true, false, false, (TEAMS > 1), TEAMS>(fp, items, stream);
 }
 
 }  // namespace hbsa

@@ -5,6 +5,7 @@
 //   5  forward, head dims up to HBSA_D (also 96, 160 and 192)
 //   6  forward, few queries per item                 7  forward that counts the blocks itself
 //   8, 9  forms 1 (one launch) and 5 cut over key blocks
+//   10, 11  forms 1 and 7, and 5, with two teams for the tiles of an item
 #if HBSA_PART == 1
 #include "hbsa_fwd_kernel.h"
 template int hbsa::launch_fwd<HBSA_D, hbsa::HBSA_E, false>(const FwdParams &, long long, hipStream_t);
@@ -20,7 +21,7 @@ template int hbsa::launch_bwd<HBSA_D, hbsa::HBSA_E>(const BwdParams &, int, int,
 template int hbsa::launch_fwd_f32<HBSA_D>(const FwdParams &, float, long long, hipStream_t);
 #elif HBSA_PART == 5
 #include "hbsa_fwd_kernel.h"
-template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E, false>(const FwdParams &, long long, hipStream_t);
+template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E, false, 1>(const FwdParams &, long long, hipStream_t);
 #elif HBSA_PART == 6
 #include "hbsa_fwd_decode.h"
 template int hbsa::launch_fwd_decode<HBSA_D, hbsa::HBSA_E>(const FwdParams &, int, long long, hipStream_t);
@@ -32,7 +33,13 @@ template int hbsa::launch_fwd_counted<HBSA_D, hbsa::HBSA_E>(const FwdParams &, l
 template int hbsa::launch_fwd_parts<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
 #elif HBSA_PART == 9
 #include "hbsa_fwd_kernel.h"
-template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E, true>(const FwdParams &, long long, hipStream_t);
+template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E, true, 1>(const FwdParams &, long long, hipStream_t);
+#elif HBSA_PART == 10
+#include "hbsa_fwd_kernel.h"
+template int hbsa::launch_fwd_teams<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
+#elif HBSA_PART == 11
+#include "hbsa_fwd_kernel.h"
+template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E, false, 2>(const FwdParams &, long long, hipStream_t);
 #else
-#error "HBSA_PART is 1 to 9"
+#error "HBSA_PART is 1 to 11"
 #endif
