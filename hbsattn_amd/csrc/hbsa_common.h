@@ -170,8 +170,9 @@ struct FwdParams {
   int32_t parts_last;    // workgroups are numbered by part first (else: the parts of an item are neighbours)
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
   int32_t split;         // host side only: parts of the split over key blocks that pay (fwd_split)
-  int32_t teams;         // host side only: two teams for the tiles of every item (fwd_teams)
-  int32_t grouped;       // host side only: tiles of 16-key groups (the GROUPED form of the kernel)
+  // host side only, 16 bits each (the arguments grow by nothing): two teams for the tiles of every item (fwd_teams); tiles of 16-key groups (the
+  // GROUPED form of the kernel)
+  int16_t teams, grouped;
   // Items handed out without queues in the order of their weights (see OrderRoom), nullptr: last q blocks first
   const uint32_t *order;         // [num_q_block * nhead_k]: q block << 16 | kv head, heaviest first
 };
