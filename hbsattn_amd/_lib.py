@@ -45,6 +45,8 @@ def load() -> ctypes.CDLL:
     lib.hbsa_fwd_launches.argtypes = [ctypes.c_int32] * 10 + [ctypes.c_int64, ctypes.c_void_p]
     lib.hbsa_fwd_decodes.restype = ctypes.c_int
     lib.hbsa_fwd_decodes.argtypes = [ctypes.c_int32] * 8
+    lib.hbsa_fwd_plan.restype = ctypes.c_int
+    lib.hbsa_fwd_plan.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p]
     lib.hbsa_set_onepass.restype = ctypes.c_int
     lib.hbsa_set_onepass.argtypes = [ctypes.c_int]
     lib.hbsa_set_walk_min_bytes.restype = ctypes.c_longlong

@@ -87,6 +87,12 @@ int hbsa_fwd_launches(int32_t dtype, int32_t batch, int32_t total_k, int32_t nhe
 int hbsa_fwd_decodes(int32_t dtype, int32_t total_q, int32_t nhead_q, int32_t nhead_k, int32_t num_q_block,
                      int32_t num_k_block, int32_t q_block_size, int32_t k_block_size);
 
+/* What the attention launch of a call is made of, where hbsa_fwd_decodes says 0 and the tensors are not HBSA_DTYPE_F32: `sizes` as in
+ * hbsa_fwd_v, prepared 0 for the one-launch form and others for a run of a prepared mask (HBSA_DTYPE_F32_STAGED16, and not head dims other than
+ * 32, 64, 128 and 256).  plan[4] = { wavefronts of a team, teams of a workgroup (2: they share the tiles of items that have six or more; a prepared mask of
+ * short sequences leaves all to the first), parts of an item at most (with a workspace that has the room), work items, of one part each }.  Host-side only. */
+int hbsa_fwd_plan(const int32_t *sizes, int32_t prepared, int32_t *plan);
+
 /* Size (K + V bytes of one kv head) from which the clocked walk above is used; a negative value only
  * reads the setting.  Returns the previous value. */
 long long hbsa_set_walk_min_bytes(long long bytes);

@@ -1,0 +1,33 @@
+"""Wavefronts, teams and parts of the attention launch: a form without kernels of two teams keeps the workgroups that suit it."""
+import ctypes
+
+import pytest
+
+from hbsattn_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def plan_of(prepared, dtype=_lib.DTYPE_BF16, *, batch, total_q, total_k, hq, hk, d, nqb, nkb, qbs, kbs):
+    """(wavefronts of a team, teams, parts, items)"""
+    sizes = (ctypes.c_int32 * 12)(dtype, batch, total_q, total_k, hq, hk, d, nqb, nkb, qbs, kbs, 1)
+    plan = (ctypes.c_int32 * 4)()
+    lib = _lib.load()
+    assert lib.hbsa_fwd_plan(ctypes.addressof(sizes), int(prepared), ctypes.addressof(plan)) == 0, _lib.last_error()
+    return tuple(plan)
+
+
+def test_forms_without_teams_keep_their_wavefronts():
+    # eight q heads on one, 48-row blocks of 20 rows: 16 plain slots, twos of eight wavefronts; 12 packed ones, threes of four
+    size = dict(batch=40, total_q=800, total_k=1600, hq=8, hk=1, d=128, nqb=40, nkb=40, qbs=48, kbs=64)
+    lib = _lib.load()
+    assert plan_of(True, **size) == (4, 2, 1, 160)
+    assert plan_of(True, _lib.DTYPE_F32_STAGED16, **size) == (8, 1, 1, 80)
+    deterministic, least = lib.hbsa_set_deterministic(0), lib.hbsa_set_walk_min_bytes(0)
+    try:
+        assert plan_of(True, **size) == (8, 1, 1, 80)   # the clocked walk
+    finally:
+        lib.hbsa_set_deterministic(deterministic)
+        lib.hbsa_set_walk_min_bytes(least)
+    # sequences of one block each: one launch leaves them to one team of packed slots
+    assert plan_of(False, **size) == (4, 1, 1, 120)
