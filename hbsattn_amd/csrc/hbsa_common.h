@@ -170,12 +170,36 @@ struct FwdParams {
   int32_t parts_last;    // workgroups are numbered by part first (else: the parts of an item are neighbours)
   uint32_t *arrivals;    // one counter per item, zero before and after every launch
   int32_t split;         // host side only: parts of the split over key blocks that pay (fwd_split)
-  // host side only, 16 bits each (the arguments grow by nothing): two teams for the tiles of every item (fwd_teams); tiles of 16-key groups (the
-  // GROUPED form of the kernel)
-  int16_t teams, grouped;
+  // host side only, 32 bits in all (the arguments grow by nothing): two teams for the tiles of every item (fwd_teams); what the two unions hold (put_parts,
+  // put_counts); tiles of 16-key groups (the GROUPED form of the kernel)
+  int8_t teams, unions;
+  int16_t grouped;
   // Items handed out without queues in the order of their weights (see OrderRoom), nullptr: last q blocks first
   const uint32_t *order;         // [num_q_block * nhead_k]: q block << 16 | kv head, heaviest first
 };
+
+// The only writers of the unions of FwdParams; false where the other one has been there (once a split's pointers were written over, and its kernel
+// stored its results at address zero and up).  Every launch asks unions_fit first.
+enum : int8_t { kUnionsEmpty, kUnionsParts, kUnionsCounts };
+inline bool put_parts(FwdParams &fp, float *out, float *lse) {
+  if (fp.unions == kUnionsCounts) return false;
+  fp.unions = kUnionsParts;
+  fp.part_out = out;
+  fp.part_lse = lse;
+  return true;
+}
+inline bool put_counts(FwdParams &fp, int32_t *counts, int32_t ticket, int32_t sides) {
+  if (fp.unions == kUnionsParts) return false;
+  fp.unions = kUnionsCounts;
+  fp.counts = counts;
+  fp.count_info[0] = ticket;
+  fp.count_info[1] = sides;
+  return true;
+}
+// counted: the kernel counts blocks.  (nparts > 1: it writes partial results)
+inline bool unions_fit(const FwdParams &fp, bool counted) {
+  return counted ? fp.unions == kUnionsCounts && fp.nparts == 1 : fp.unions == (fp.nparts > 1 ? kUnionsParts : kUnionsEmpty);
+}
 
 // Boundaries of one sequence of the packed batch, as read from the caller's device arrays.
 struct SeqBounds {

@@ -1594,6 +1594,7 @@ template <int D, typename E, bool OUT32, int NW, bool EXTRAS, bool FUSED = false
 int launch_fwd_nw(const FwdParams &fp, long long items, hipStream_t stream) {
   constexpr int lds_bytes = TEAMS * 4 * (D > 128 && D <= 192 ? 32 : 64) * D * 2 + 2 * H_WORDS * 4 + 2 * kListCap * 4 + (FUSED ? 4 * kSeqCap * 4 + kMaskStage : 0);
   const void *kernel = reinterpret_cast<const void *>(&hbsa_fwd_kernel<D, E, OUT32, NW, EXTRAS, FUSED, PACK, COLS, GROUPED, COUNTED, ONE, TEAMS>);
+  if (!unions_fit(fp, COUNTED) || (!EXTRAS && fp.nparts > 1)) return fail(HBSA_ERR_UNSUPPORTED, "partial results or counts that the kernel has no place for");
   // workgroups that fit the current device at once; the attribute and the occupancy are per device
   static thread_local int resident_of[kMaxDevices] = {};
   int dev = 0;
@@ -1683,7 +1684,7 @@ int launch_fwd_teams(const FwdParams &fp, long long items, hipStream_t stream) {
   if (fp.info != nullptr)
     return fp.grouped ? launch_fwd_nw<D, E, false, 4, true, false, false, false, true, false, true, 2>(fp, items, stream)
                       : launch_fwd_nw<D, E, false, 4, true, false, false, false, false, false, true, 2>(fp, items, stream);
-  if (fp.counts != nullptr)
+  if (fp.unions == kUnionsCounts)
     return fp.grouped ? launch_fwd_nw<D, E, false, 4, false, true, true, false, true, true, true, 2>(fp, items, stream)
                       : launch_fwd_nw<D, E, false, 4, false, true, true, false, false, true, true, 2>(fp, items, stream);
   return fp.grouped ? launch_fwd_nw<D, E, false, 4, false, true, true, false, true, false, true, 2>(fp, items, stream)
