@@ -59,17 +59,17 @@ def units() -> list:
     return out + [("api", API_SOURCE, [])]
 
 
-def _vgpr_spills(remarks: str) -> dict:
-    """Kernels with vector-register spills, from the compiler's resource-usage remarks."""
-    spills, name = {}, None
+def _kernels_with(what: str, remarks: str) -> dict:
+    """Kernels whose count of ``what`` is not zero, from the compiler's resource-usage remarks."""
+    counts, name = {}, None
     for line in remarks.splitlines():
         m = re.search(r"remark:\s+Function Name: (\S+)", line)
         if m:
             name = m.group(1)
-        m = re.search(r"remark:\s+VGPRs Spill: (\d+)", line)
+        m = re.search(r"remark:\s+" + what + r": (\d+)", line)
         if m and name is not None and int(m.group(1)) > 0:
-            spills[name] = int(m.group(1))
-    return spills
+            counts[name] = int(m.group(1))
+    return counts
 
 
 def compile_unit(unit, objdir: str):
@@ -97,7 +97,7 @@ def build(verbose: bool = False) -> str:
     with tempfile.TemporaryDirectory() as objdir, concurrent.futures.ThreadPoolExecutor(jobs) as pool:
         host = pool.submit(compile_host, objdir)
         done = list(pool.map(lambda u: compile_unit(u, objdir), units()))
-        check_spills("".join(remarks for _, remarks in done), verbose)
+        check_registers("".join(remarks for _, remarks in done), verbose)
         link([obj for obj, _ in done], OUTPUT)
         link_host(host.result())
     if verbose:
@@ -138,18 +138,20 @@ def link_host(obj: str) -> None:
         raise RuntimeError("g++ failed: " + " ".join(cmd) + "\n" + res.stdout + res.stderr)
 
 
-def check_spills(remarks: str, verbose: bool = False) -> None:
+def check_registers(remarks: str, verbose: bool = False) -> None:
     # The attention kernels named above issue their LDS reads by hand and wait for them by count.  The
-    # compiler does not know that such a register has a read in flight; if it spills one, it saves the
-    # register before the data has arrived and the result is wrong now and then.  So a build in which
-    # such a kernel spills vector registers is refused.  (The other kernels leave every wait to the
-    # compiler; a spill there only costs time and is reported.)
-    spills = _vgpr_spills(remarks)
-    fatal = {k: v for k, v in spills.items() if any(n in k for n in HAND_ISSUED_READS) and COMPILER_ISSUED not in k}
-    if fatal:
-        raise RuntimeError(f"vector-register spills in {fatal}: reduce register pressure (see the comment here)")
-    if spills and verbose:
-        print(f"note: vector-register spills in {spills}")
+    # compiler does not know that such a register has a read in flight; if it spills one, or moves it to an
+    # accumulation register, it saves the register before the data has arrived and the result is wrong now
+    # and then.  So a build in which such a kernel spills vector registers or has accumulation registers
+    # (which it needs for nothing else: its products stand in vector registers) is refused.  (The other
+    # kernels leave every wait to the compiler; a spill there only costs time and is reported.)
+    for what in ("VGPRs Spill", "AGPRs"):
+        found = _kernels_with(what, remarks)
+        fatal = {k: v for k, v in found.items() if any(n in k for n in HAND_ISSUED_READS) and COMPILER_ISSUED not in k}
+        if fatal:
+            raise RuntimeError(f"{what} of {fatal}: reduce register pressure (see the comment here)")
+        if found and verbose and what == "VGPRs Spill":
+            print(f"note: vector-register spills in {found}")
 
 
 EXAMPLE_SOURCE = os.path.join(_HERE, "csrc", "cabi_example.cpp")
