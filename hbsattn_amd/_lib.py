@@ -68,6 +68,8 @@ def load() -> ctypes.CDLL:
     lib.hbsa_fwd_v_locked.argtypes = [vp, ctypes.c_size_t, vp, ctypes.c_float, vp, vp]
     lib.hbsa_fwd_one.restype = ctypes.c_int
     lib.hbsa_fwd_one.argtypes = [vp, vp, ctypes.c_float, vp, vp]
+    lib.hbsa_fwd_any.restype = ctypes.c_int
+    lib.hbsa_fwd_any.argtypes = [vp, ctypes.c_size_t, vp, ctypes.c_float, vp, vp]
     lib.hbsa_fwd_counted.restype = ctypes.c_int
     lib.hbsa_fwd_counted.argtypes = [vp, vp, ctypes.c_float, vp, vp, ctypes.c_int32, vp]
     lib.hbsa_fwd_static.restype = ctypes.c_int

@@ -251,13 +251,16 @@ int hbsa_fwd_v(const void *const *ptrs, size_t workspace_bytes, const int32_t *s
  * hbsa_fwd_v without a workspace: the one-launch form alone, for any head dim that is a multiple of 8 up to 256 (a
  * head dim other than 32, 64, 128 and 256 runs in the next larger kernel with its missing columns zero on the chip;
  * 96, 160 and 192 have kernels of their own).  ptrs[10] is not looked at.  HBSA_ERR_WORKSPACE_TOO_SMALL, and nothing
- * launched, when the one-launch form does not apply to the call.
+ * launched, when the one-launch form does not apply to the call.  (hbsa_fwd_any without a workspace is the same for those
+ * other head dims; for 32, 64, 128 and 256 it sends few queries per q block to the kernel of hbsa_fwd_decodes, and this entry does not.)
  */
 int hbsa_fwd_one(const void *const *ptrs, const int32_t *sizes, float softmax_scale, const int64_t *strides, void *stream);
 
 /* hbsa_fwd_v for a caller that looks for nothing in the workspace afterwards (0 bytes: none), for any head dim that hbsa_fwd_one takes: a
- * call whose work is cut over its key blocks then has no pre-pass, only the attention launch and the merge.  HBSA_ERR_WORKSPACE_TOO_SMALL, and
- * nothing launched, also where another head dim than 32, 64, 128 and 256 needs the two-launch form. */
+ * call whose work is cut over its key blocks then has no pre-pass, only the attention launch and the merge.  The parts' room lies behind the first
+ * hbsa_fwd_workspace_bytes_dtype(...) bytes, as in hbsa_fwd; where the workspace ends before it, head dims 32, 64, 128 and 256 run uncut, pre-pass and
+ * attention, and others are refused.  HBSA_ERR_WORKSPACE_TOO_SMALL, and nothing launched, also where another head dim than 32, 64, 128 and 256 needs the
+ * pre-pass. */
 int hbsa_fwd_any(const void *const *ptrs, size_t workspace_bytes, const int32_t *sizes, float softmax_scale, const int64_t *strides, void *stream);
 
 /* hbsa_fwd_one for a caller that has not counted the blocks: cu_num_q_block, cu_num_k_block or both may be NULL in `ptrs`, and are then

@@ -223,3 +223,58 @@ def test_a_call_without_a_device_reports_two_launches_and_asks_for_its_workspace
     import torch
     if not torch.cuda.is_available():
         assert _call_fwd(lib, ws=None, ws_bytes=0) == -3 and "workspace" in _lib.last_error()
+
+
+@pytest.mark.parametrize("over,ws_bytes,code,needle", [
+    ({4: 30, 5: 4}, 1 << 30, -1, "divisible"),
+    ({6: 12}, 1 << 30, -2, "headdim"),      # no multiple of 8
+    ({6: 0}, 1 << 30, -2, "headdim"),
+    ({6: 264}, 1 << 30, -2, "headdim"),
+    ({9: 100}, 1 << 30, -1, "multiples of 16"),
+    ({6: 80}, 1 << 30, -3, "workspace"),    # the one-launch form is off: such rows have no other
+    ({6: 128}, 16, -3, "workspace"),
+    ({6: 128}, 0, -3, "workspace"),
+    ({2: 0}, 0, 0, ""),
+])
+@pytest.mark.parametrize("entry", ["hbsa_fwd_any", "hbsa_fwd_one"])
+def test_entries_for_any_head_dim_refuse_without_touching_the_gpu(entry, over, ws_bytes, code, needle):
+    lib = _lib.load()
+    if entry == "hbsa_fwd_one" and ws_bytes == 16:
+        pytest.skip("takes no workspace")
+    strides = (ctypes.c_int64 * 11)(4096, 128, 4096, 128, 4096, 128, 4096, 128, 1, 1, 1)
+    ptrs = (ctypes.c_void_p * 11)(*([256] * 11))
+    sizes = (ctypes.c_int32 * 12)(0, 1, 128, 128, 32, 32, 128, 1, 1, 128, 128, 1)
+    for i, v in over.items():
+        sizes[i] = v
+    a = lambda x: ctypes.addressof(x)
+    one = lib.hbsa_set_onepass(0)
+    try:
+        rc = (lib.hbsa_fwd_any(a(ptrs), ws_bytes, a(sizes), 0.1, a(strides), None) if entry == "hbsa_fwd_any"
+              else lib.hbsa_fwd_one(a(ptrs), a(sizes), 0.1, a(strides), None))
+    finally:
+        lib.hbsa_set_onepass(one)
+    assert rc == code and needle in _lib.last_error()
+
+
+def test_entries_for_any_head_dim_refuse_null_arrays():
+    lib = _lib.load()
+    assert lib.hbsa_fwd_any(None, 0, None, 0.1, None, None) == -1 and "null" in _lib.last_error()
+    assert lib.hbsa_fwd_one(None, None, 0.1, None, None) == -1 and "null" in _lib.last_error()
+    assert lib.hbsa_fwd_plan(None, 0, None) == -1 and "null" in _lib.last_error()
+
+
+def test_plan_refuses_what_other_kernels_compute():
+    lib = _lib.load()
+    plan = (ctypes.c_int32 * 4)()
+
+    def rc(prepared, **over):
+        v = dict(dtype=0, batch=1, total_q=128, total_k=128, hq=4, hk=4, d=128, nqb=1, nkb=1, qbs=128, kbs=128, causal=1)
+        v.update(over)
+        sizes = (ctypes.c_int32 * 12)(*v.values())
+        return lib.hbsa_fwd_plan(ctypes.addressof(sizes), prepared, ctypes.addressof(plan))
+
+    assert rc(0) == 0 and rc(1) == 0 and rc(0, d=80) == 0 and rc(1, dtype=_lib.DTYPE_F32_STAGED16) == 0
+    for prepared, over in ((0, dict(dtype=_lib.DTYPE_F32)), (0, dict(dtype=_lib.DTYPE_F32_STAGED16)), (1, dict(d=80)), (0, dict(d=12)),
+                           (0, dict(total_q=1, nqb=1, qbs=16))):   # (a decode step)
+        assert rc(prepared, **over) == -2, (prepared, over)
+    assert rc(0, hk=3) == -1 and rc(0, total_q=0) == -1
