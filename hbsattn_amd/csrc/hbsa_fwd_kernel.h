@@ -961,7 +961,9 @@ __global__ __launch_bounds__(NW * TEAMS * 64, TEAMS > 1 || D > 192 ? 1 : D > 64 
     int min_r, max_r;   // smallest and largest query row among them
     int hq;             // plain form: the slot's q head; packed form: the group's first q head
   };
-  auto quotient = [](int a, int b) {   // a / b for 0 <= a < 2^20, 0 < b < 2^12
+  // a / b for 0 <= a < 2^20 (kPackedEntries), b > 0.  Exact: (a + 0.5) / b is 0.5 / b or more from the whole numbers, a relative distance of 2^-21 of
+  // what is at most 2^20 / b, and the reciprocal (1 ulp) and the product (half of one) are off by 1.5 * 2^-23 of it.  (Above 2^22 it is not exact.)
+  auto quotient = [](int a, int b) {
     return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
   };
   auto slot_of = [&](int hk, int sub, int rows) -> Slot {
