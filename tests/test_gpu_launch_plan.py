@@ -2,6 +2,7 @@
 import ctypes
 
 import pytest
+import torch
 
 from hbsattn_amd import _lib
 
@@ -15,6 +16,12 @@ def plan_of(prepared, dtype=_lib.DTYPE_BF16, *, batch, total_q, total_k, hq, hk,
     lib = _lib.load()
     assert lib.hbsa_fwd_plan(ctypes.addressof(sizes), int(prepared), ctypes.addressof(plan)) == 0, _lib.last_error()
     return tuple(plan)
+
+
+def plan_for(w, prepared=False):
+    code = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}[w.q.dtype]
+    return plan_of(prepared, code, batch=len(w.cu_q) - 1, total_q=w.q.shape[0], total_k=w.k.shape[0], hq=w.q.shape[1], hk=w.k.shape[1], d=w.q.shape[2],
+                   nqb=w.q_meta[0], nkb=w.k_meta[0], qbs=w.q_block_size, kbs=w.k_block_size)
 
 
 def test_forms_without_teams_keep_their_wavefronts():

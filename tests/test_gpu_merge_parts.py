@@ -28,8 +28,7 @@ def test_merged_parts(k_blocks, d):
     out, lse = hbsa_run(w.q, w.k, w.v, prepared, None, return_lse=True)
     assert_close_to_oracle(out, oracle_for(w), f"{k_blocks} key blocks")
     assert out[40:, :2].abs().max() == 0 and torch.isinf(lse[40:, :2]).all() and torch.isfinite(lse[:40]).all()
-    # the prepared mask's bit rows were copied for the parts by a launch of their own; a call that makes its bit rows itself has the
-    # pre-pass write the copies, and runs the same parts
+    # the prepared form and the one-launch form cut the items by themselves, and make the same parts
     assert _lib.load().hbsa_fwd_launches(_lib.DTYPE_BF16, 2, w.k.shape[0], 4, 2, d, int(nq), int(nk), 64, 64, 0, None) > 1
     assert torch.equal(HBSAttention(*a), out)
     again, lse2 = hbsa_run(w.q, w.k, w.v, prepared, None, return_lse=True)
