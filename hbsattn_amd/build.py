@@ -50,6 +50,7 @@ def units() -> list:
     out += [inst(d, e, 5) for d in (192, 160, 256, 128, 96, 64, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 7) for d in (128, 64, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 8) for d in (128, 64, 256, 32) for e in ("ElemBF16", "ElemF16")]
+    out += [inst(d, e, 12) for d in (128, 64, 256, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 9) for d in (192, 160, 256, 128, 96, 64, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 10) for d in (128, 64, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 11) for d in (128, 96, 64, 32) for e in ("ElemBF16", "ElemF16")]

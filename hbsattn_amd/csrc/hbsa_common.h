@@ -580,6 +580,8 @@ int launch_fwd_teams(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_parts(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
+int launch_fwd_prepared_parts(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
 int launch_fwd_decode(const FwdParams &fp, int most, long long items, hipStream_t stream);
 template <int D>
 int launch_fwd_f32(const FwdParams &fp, float c_signed, long long items, hipStream_t stream);

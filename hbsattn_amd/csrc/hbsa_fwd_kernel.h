@@ -535,18 +535,21 @@ __global__ __launch_bounds__(NW * TEAMS * 64, TEAMS > 1 || D > 192 ? 1 : D > 64 
     if (st_hk >= 0) {
       const int nkblk = __builtin_amdgcn_readlane((int)st_info, 6);
       const int kmax = __builtin_amdgcn_readlane((int)st_info, 7);
+      // packed slots behind the q block's entries: no rows, so no tiles
+      auto rowless = [&]() { return st_sub * NW * kWaveRows >= p.ratio * __builtin_amdgcn_readlane((int)st_info, 1); };
       if constexpr (FUSED) {
         // the staged bytes arrived with the wait of a tile, or one of the waits before the first item, since stage()
         st_bits = st_nvis > 0 ? staged_words(st_ms, min(st_nvis, kMaskWindow)) : 0u;
         if constexpr (EXTRAS) {
           st_bits = part_words(st_bits, st_nvis, st_part, parts);
-          if (st_sub * NW * kWaveRows >= p.ratio * __builtin_amdgcn_readlane((int)st_info, 1)) parts = 0;   // no rows, so no tiles
+          if (rowless()) parts = 0;
         }
         if (!EXTRAS || st_part < parts)
           total = list_of(c, 0, fused_more_words(st_mrow, st_nvis, st_part), 2 * ((st_nvis + 63) >> 6), kmax, st_bits);
       } else {
         const int nwords = 2 * ((nkblk + 63) >> 6);
         if (EXTRAS && p.nparts > 1) st_bits = part_words(st_bits, min(nkblk, (int)fast_div((uint32_t)(kmax + p.kbs - 1), p.div_kbs)), st_part, parts);
+        if (EXTRAS && PACK && rowless()) parts = 0;
         if (!EXTRAS || st_part < parts)
           total = list_of(c, 0, prepared_more_words(p.bits + ((size_t)st_hk * p.nqb + st_qb) * p.wpr, nwords, st_part, kmax, nkblk), nwords, kmax, st_bits);
       }
@@ -1670,6 +1673,18 @@ int launch_fwd_parts(const FwdParams &fp, long long items, hipStream_t stream) {
                     : launch_fwd_nw<D, E, false, 4, true, true, true>(fp, items, stream);
 }
 
+// The same on a prepared mask, where the slots are packed (plain ones: launch_fwd)
+template <int D, typename E>
+int launch_fwd_prepared_parts(const FwdParams &fp, long long items, hipStream_t stream) {
+  if constexpr (D == 128) {
+    if (fp.nw == 8)
+      return fp.grouped ? launch_fwd_nw<D, E, false, 8, true, false, true, false, true>(fp, items, stream)
+                        : launch_fwd_nw<D, E, false, 8, true, false, true>(fp, items, stream);
+  }
+  return fp.grouped ? launch_fwd_nw<D, E, false, 4, true, false, true, false, true>(fp, items, stream)
+                    : launch_fwd_nw<D, E, false, 4, true, false, true>(fp, items, stream);
+}
+
 // the one-launch form that counts the blocks itself, workgroups of four wavefronts
 template <int D, typename E>
 int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream) {
@@ -1681,11 +1696,15 @@ int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream)
 }
 
 // Two teams for the tiles of an item (see fwd_teams): the one-launch form, that counts the blocks or not, and the prepared form
+template <int D, typename E, bool GROUPED>
+int launch_prepared_teams(const FwdParams &fp, long long items, hipStream_t stream) {
+  return fp.pack ? launch_fwd_nw<D, E, false, 4, true, false, true, false, GROUPED, false, true, 2>(fp, items, stream)
+                 : launch_fwd_nw<D, E, false, 4, true, false, false, false, GROUPED, false, true, 2>(fp, items, stream);
+}
 template <int D, typename E>
 int launch_fwd_teams(const FwdParams &fp, long long items, hipStream_t stream) {
   if (fp.info != nullptr)
-    return fp.grouped ? launch_fwd_nw<D, E, false, 4, true, false, false, false, true, false, true, 2>(fp, items, stream)
-                      : launch_fwd_nw<D, E, false, 4, true, false, false, false, false, false, true, 2>(fp, items, stream);
+    return fp.grouped ? launch_prepared_teams<D, E, true>(fp, items, stream) : launch_prepared_teams<D, E, false>(fp, items, stream);
   if (fp.unions == kUnionsCounts)
     return fp.grouped ? launch_fwd_nw<D, E, false, 4, false, true, true, false, true, true, true, 2>(fp, items, stream)
                       : launch_fwd_nw<D, E, false, 4, false, true, true, false, false, true, true, 2>(fp, items, stream);

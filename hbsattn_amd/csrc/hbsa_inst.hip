@@ -6,6 +6,7 @@
 //   6  forward, few queries per item                 7  forward that counts the blocks itself
 //   8, 9  forms 1 (one launch) and 5 cut over key blocks
 //   10, 11  forms 1 and 7, and 5, with two teams for the tiles of an item
+//   12  form 1 on a prepared mask, packed slots, cut over key blocks
 #if HBSA_PART == 1
 #include "hbsa_fwd_kernel.h"
 template int hbsa::launch_fwd<HBSA_D, hbsa::HBSA_E, false>(const FwdParams &, long long, hipStream_t);
@@ -40,6 +41,9 @@ template int hbsa::launch_fwd_teams<HBSA_D, hbsa::HBSA_E>(const FwdParams &, lon
 #elif HBSA_PART == 11
 #include "hbsa_fwd_kernel.h"
 template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E, false, 2>(const FwdParams &, long long, hipStream_t);
+#elif HBSA_PART == 12
+#include "hbsa_fwd_kernel.h"
+template int hbsa::launch_fwd_prepared_parts<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
 #else
-#error "HBSA_PART is 1 to 11"
+#error "HBSA_PART is 1 to 12"
 #endif

@@ -23,6 +23,8 @@ FORMS = {
     "teams 96": (dict(q_lens=[1300], k_lens=[1300], hq=2, hk=1, d=96, qbs=64, kbs=64, keep=0.4), (4, 2, False)),
     "split": (dict(q_lens=[70, 4], k_lens=[6000, 5000], hq=4, hk=2, d=64, qbs=64, kbs=64, keep=0.3), (4, 1, True)),
     "split 128": (dict(q_lens=[70, 4], k_lens=[6000, 5000], hq=8, hk=2, d=128, qbs=128, kbs=64, keep=0.3), (8, 1, True)),
+    "split packed": (dict(q_lens=[70, 4], k_lens=[6000, 5000], hq=8, hk=1, d=64, qbs=48, kbs=64, keep=0.3), (4, 1, True)),
+    "teams packed": (dict(q_lens=[700, 300], k_lens=[700, 300], hq=8, hk=1, d=128, qbs=16, kbs=48, keep=0.6), (4, 2, False)),
     "split 80": (dict(q_lens=[70, 4], k_lens=[6000, 5000], hq=4, hk=2, d=80, qbs=64, kbs=48, keep=0.3), (4, 1, True)),
     "split 256": (dict(q_lens=[70, 4], k_lens=[6000, 5000], hq=4, hk=2, d=256, qbs=64, kbs=64, keep=0.3), (4, 1, True)),
 }
@@ -94,7 +96,7 @@ def test_two_streams_at_once(form):
     assert all(torch.equal(o, want[i]) for i in range(2) for o in outs[i])
 
 
-@pytest.mark.parametrize("form", ["sole", "teams", "teams 128", "split", "split 128"])
+@pytest.mark.parametrize("form", ["sole", "teams", "teams 128", "teams packed", "split", "split 128", "split packed"])
 def test_gradients(form):
     w = _problem(form)
     plain = HBSAttention(*w.args())
@@ -110,7 +112,7 @@ def test_gradients(form):
         assert err.mean() <= max(2e-3, 1e-2 * ref.abs().mean().item()), (name, err.mean())
 
 
-@pytest.mark.parametrize("form", ["sole", "teams", "teams 128", "split", "split 128", "split 256"])
+@pytest.mark.parametrize("form", ["sole", "teams", "teams 128", "teams packed", "split", "split 128", "split 256", "split packed"])
 def test_log_sum_exp(form):
     w = _problem(form, causal=False)
     w.block_mask[0, -1] = False   # rows that see no key

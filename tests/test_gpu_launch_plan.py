@@ -28,7 +28,7 @@ def test_forms_without_teams_keep_their_wavefronts():
     # eight q heads on one, 48-row blocks of 20 rows: 16 plain slots, twos of eight wavefronts; 12 packed ones, threes of four
     size = dict(batch=40, total_q=800, total_k=1600, hq=8, hk=1, d=128, nqb=40, nkb=40, qbs=48, kbs=64)
     lib = _lib.load()
-    assert plan_of(True, **size) == (4, 2, 1, 160)
+    assert plan_of(True, **size) == (4, 2, 1, 120)
     assert plan_of(True, _lib.DTYPE_F32_STAGED16, **size) == (8, 1, 1, 80)
     deterministic, least = lib.hbsa_set_deterministic(0), lib.hbsa_set_walk_min_bytes(0)
     try:
