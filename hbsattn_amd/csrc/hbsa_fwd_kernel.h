@@ -1493,8 +1493,8 @@ __global__ __launch_bounds__(NW * TEAMS * 64, TEAMS > 1 || D > 192 ? 1 : D > 64 
         // split over key blocks: this part's normalised result and log-sum-exp, for the merge kernel
         if (l32 < nrows) {
           const int64_t rh = ((int64_t)cur_part * p.total_q + (row_begin + my_r)) * p.nhead_q + hq;
-          if (g32 == 0)   // (-inf: no key.  A NaN stays one: the part is not to be left out)
-            p.part_lse[rh] = l_tot != 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : -INFINITY;
+          if (g32 == 0)   // (-inf: no key; inf: NaN, which would be left out of the merge's maximum.  Its weight there is exp(inf - inf))
+            p.part_lse[rh] = l_tot > 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718055994531f : l_tot == 0.f ? -INFINITY : INFINITY;
           float *dst = p.part_out + rh * (COLS ? 8 * p.ncol : D);
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
