@@ -38,3 +38,17 @@ def test_forms_without_teams_keep_their_wavefronts():
         lib.hbsa_set_walk_min_bytes(least)
     # sequences of one block each: one launch leaves them to one team of packed slots
     assert plan_of(False, **size) == (4, 1, 1, 120)
+
+
+@pytest.mark.parametrize("batch,q,k,hq,hk,qbs,kbs,plan", [
+    (8, 342, 2919, 32, 2, 80, 16, (4, 1, 1, 800)),      # plain slots are too many to be cut, and the sequences too short for packed eights to be
+    (9, 21, 856, 32, 2, 176, 48, (8, 1, 1, 198)),
+    (3, 130, 2843, 64, 4, 16, 48, (4, 1, 2, 216)),      # ... which are cut as fours
+    (13, 9, 4407, 32, 2, 112, 64, (8, 1, 4, 182)),      # long ones
+])
+def test_packed_eights_are_cut_where_sequences_are_long(batch, q, k, hq, hk, qbs, kbs, plan):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the numbers of items are for 256 compute units")
+    size = dict(batch=batch, total_q=batch * q, total_k=batch * k, hq=hq, hk=hk, d=128, nqb=batch * -(-q // qbs), nkb=batch * -(-k // kbs), qbs=qbs, kbs=kbs)
+    assert plan_of(False, **size) == plan
+    assert plan_of(True, **size)[1:3] == plan[1:3]
