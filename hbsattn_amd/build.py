@@ -38,6 +38,14 @@ HIPCC_FLAGS = [
 # products stand in vector registers anyway.
 MFMA_IN_VGPRS = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 
+# The one-launch kernels of eight wavefronts with packed slots: what is only jumped to begins on a line of 64 bytes.  Their tile loop is instruction for
+# instruction the plain slots' one, which got 2 % faster when the next tile's look-up moved before the barrier, but where it came to lie it got slower.
+# us, before that, since then, aligned (4 x 6000 tokens, 64-key blocks, 15 % kept, slots of eight in use): 32 / 16 heads, 80 rows, 5 of 8, 552, 566, 560; 32 / 8,
+# 48 rows, 6, 479, 490, 483; 32 / 16, 112 rows, 7, 446, 451, 449; 32 / 2, 16 rows, 8, 409, 416, 411; 48-key blocks, 5, 616, 604, 601.  Not for all kernels: 16 x 40 .. 500
+# tokens, 32 / 8 heads of 128, whose code is mostly fetched for the first time, 35.0 -> 35.7.  (Lines of 32 or 128 bytes, aligned loops, the look-up
+# behind the barrier in these kernels alone: 558 to 570 for the first of them.)
+ALIGNED = ["-mllvm", "-align-all-nofallthru-blocks=6"]
+
 
 def units() -> list:
     """``(name, source, extra flags)`` of every translation unit of the library, the ones that take longest first."""
@@ -46,6 +54,7 @@ def units() -> list:
         return (f"{elem}_{d}_{part}", INST_SOURCE, flags + (MFMA_IN_VGPRS if d == 256 else []))
 
     out = [inst(d, e, 1) for d in (128, 64, 256, 32) for e in ("ElemBF16", "ElemF16")]
+    out += [(n, f, flags + ALIGNED) for n, f, flags in (inst(128, e, 13) for e in ("ElemBF16", "ElemF16"))]
     out += [inst(d, e, 3) for d in (128, 64, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 5) for d in (192, 160, 256, 128, 96, 64, 32) for e in ("ElemBF16", "ElemF16")]
     out += [inst(d, e, 7) for d in (128, 64, 32) for e in ("ElemBF16", "ElemF16")]

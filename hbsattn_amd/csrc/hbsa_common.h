@@ -572,6 +572,8 @@ int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
 int launch_fwd_fused(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E>
+int launch_packed_eights(const FwdParams &fp, long long items, hipStream_t stream);
+template <int D, typename E>
 int launch_fwd_counted(const FwdParams &fp, long long items, hipStream_t stream);
 template <int D, typename E, bool PARTS, int TEAMS>
 int launch_fwd_cols(const FwdParams &fp, long long items, hipStream_t stream);

@@ -1641,13 +1641,11 @@ template <int D, typename E, bool OUT32>
 int launch_fwd(const FwdParams &fp, long long items, hipStream_t stream) {
   return fp.grouped ? launch_fwd_tiles<D, E, OUT32, true>(fp, items, stream) : launch_fwd_tiles<D, E, OUT32, false>(fp, items, stream);
 }
-// the one-launch form (16-bit tensors, none of the extras)
+// the one-launch form (16-bit tensors, none of the extras; eight wavefronts and packed slots: launch_packed_eights)
 template <int D, typename E, bool GROUPED>
 int launch_fused_tiles(const FwdParams &fp, long long items, hipStream_t stream) {
   if constexpr (D == 128) {
-    if (fp.nw == 8)
-      return fp.pack ? launch_fwd_nw<D, E, false, 8, false, true, true, false, GROUPED>(fp, items, stream)
-                     : launch_fwd_nw<D, E, false, 8, false, true, false, false, GROUPED>(fp, items, stream);
+    if (fp.nw == 8) return launch_fwd_nw<D, E, false, 8, false, true, false, false, GROUPED>(fp, items, stream);
   }
   return fp.pack ? launch_fwd_nw<D, E, false, 4, false, true, true, false, GROUPED>(fp, items, stream)
                  : launch_fwd_nw<D, E, false, 4, false, true, false, false, GROUPED>(fp, items, stream);
@@ -1683,6 +1681,13 @@ int launch_fwd_prepared_parts(const FwdParams &fp, long long items, hipStream_t 
   }
   return fp.grouped ? launch_fwd_nw<D, E, false, 4, true, false, true, false, true>(fp, items, stream)
                     : launch_fwd_nw<D, E, false, 4, true, false, true>(fp, items, stream);
+}
+
+// The one-launch form, packed slots, eight wavefronts (a unit of its own: see ALIGNED in hbsattn_amd/build.py)
+template <int D, typename E>
+int launch_packed_eights(const FwdParams &fp, long long items, hipStream_t stream) {
+  return fp.grouped ? launch_fwd_nw<D, E, false, 8, false, true, true, false, true>(fp, items, stream)
+                    : launch_fwd_nw<D, E, false, 8, false, true, true>(fp, items, stream);
 }
 
 // the one-launch form that counts the blocks itself, workgroups of four wavefronts

@@ -7,6 +7,7 @@
 //   8, 9  forms 1 (one launch) and 5 cut over key blocks
 //   10, 11  forms 1 and 7, and 5, with two teams for the tiles of an item
 //   12  form 1 on a prepared mask, packed slots, cut over key blocks
+//   13  the one-launch form of 1, packed slots, eight wavefronts
 #if HBSA_PART == 1
 #include "hbsa_fwd_kernel.h"
 template int hbsa::launch_fwd<HBSA_D, hbsa::HBSA_E, false>(const FwdParams &, long long, hipStream_t);
@@ -44,6 +45,9 @@ template int hbsa::launch_fwd_cols<HBSA_D, hbsa::HBSA_E, false, 2>(const FwdPara
 #elif HBSA_PART == 12
 #include "hbsa_fwd_kernel.h"
 template int hbsa::launch_fwd_prepared_parts<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
+#elif HBSA_PART == 13
+#include "hbsa_fwd_kernel.h"
+template int hbsa::launch_packed_eights<HBSA_D, hbsa::HBSA_E>(const FwdParams &, long long, hipStream_t);
 #else
-#error "HBSA_PART is 1 to 12"
+#error "HBSA_PART is 1 to 13"
 #endif
