@@ -193,8 +193,8 @@ __global__ __launch_bounds__(NW * TEAMS * 64, TEAMS > 1 || D > 192 ? 1 : D > 64 
   // FUSED: the one-launch form.  No pre-pass has run: wavefront 0 derives an item's geometry from the
   // sequence boundaries (kept in LDS) and its bit row from the item's own block_mask bytes, which it
   // fetches into an LDS staging area one item ahead, where the other form fetches the prepared records.
-  // PACK: wave slots packed across the q heads of a GQA group (see slot_of below); instantiated for the
-  // one-launch form only, since either placement of the queries gives the same results bit for bit.
+  // PACK: wave slots packed across the q heads of a GQA group (see slot_of below).  Either placement of the queries gives the
+  // same results bit for bit; a prepared mask's launch has packed ones where it is cut over key blocks or has teams.
   // COLS: the tensors' rows hold p.ncol <= D / 8 chunks of eight elements (a head dim that is no D of its own).  The
   // columns past them are zero in LDS (cleared once, never loaded) and in the Q operand, and not stored: in place of
   // zero-padded copies of q, k, v and a copy of the output.

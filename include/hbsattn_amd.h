@@ -201,7 +201,9 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
  * boundaries -> a compact work description in `workspace`) and the attention kernel.  A call on bf16 or
  * fp16 tensors is ONE launch, and does not touch `workspace`, when the attention kernel's scheduler can
  * read the boundaries and the mask bytes itself: mask_kblk stride 1, at most 127 sequences, work that
- * would neither be split over key blocks (hbsa_fwd_split_workspace_bytes) nor use the clocked walk,
+ * would neither be split over key blocks (hbsa_fwd_split_workspace_bytes; hbsa_fwd_any cuts the one-launch form itself,
+ * attention and merge, where this call adds the pre-pass) nor use the clocked walk, at most 2^20 (q head of a group, row)
+ * entries a q block where nhead_q > nhead_k and q_block_size is no multiple of 32,
  * `stream` not being captured into a graph, and fewer than 64 other streams of the device having made such
  * calls.  (A call with few queries per q block, see hbsa_fwd_decodes, goes to a kernel of its own that reads boundaries and
  * mask itself under none of these conditions, and writes partial results to `workspace` where it is large enough.)  The
@@ -218,7 +220,7 @@ size_t hbsa_fwd_parts_bytes(int32_t dtype, int32_t total_q, int32_t nhead_q, int
  * reference hbsattn/fwd_triton_auto_tile_size.py:269; callers do the same with zero columns up to one of
  * these); q_block_size, k_block_size positive multiples of 16; nhead_q % nhead_k == 0; every sequence
  * length >= 1; hbsa_fwd_one takes other head dims too.  At headdim 256 a CU runs one workgroup of four wavefronts whose
- * operand reads the compiler schedules: it works, at about two thirds of the efficiency of headdim 128.  Query rows with no
+ * operand reads the compiler schedules: 0.93 to 0.98 of the efficiency of headdim 128 (8 x 2050 and 8 x 8192 tokens, 16 heads).  Query rows with no
  * visible key produce exactly 0 (reference hbsattn/reference.py:97-98).
  */
 int hbsa_fwd(const void *q, const void *k, const void *v, void *out,
