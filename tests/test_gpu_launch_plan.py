@@ -43,7 +43,8 @@ def test_forms_without_teams_keep_their_wavefronts():
 @pytest.mark.parametrize("batch,q,k,hq,hk,qbs,kbs,plan", [
     (8, 342, 2919, 32, 2, 80, 16, (4, 1, 1, 800)),      # plain slots are too many to be cut, and the sequences too short for packed eights to be
     (9, 21, 856, 32, 2, 176, 48, (8, 1, 1, 198)),
-    (3, 130, 2843, 64, 4, 16, 48, (4, 1, 2, 216)),      # ... which are cut as fours
+    (4, 15, 1097, 64, 4, 48, 64, (4, 1, 4, 96)),        # ... which are cut as fours
+    (3, 130, 2843, 64, 4, 16, 48, (4, 2, 1, 216)),      # many rows on short sequences
     (13, 9, 4407, 32, 2, 112, 64, (8, 1, 4, 182)),      # long ones
 ])
 def test_packed_eights_are_cut_where_sequences_are_long(batch, q, k, hq, hk, qbs, kbs, plan):
@@ -52,3 +53,20 @@ def test_packed_eights_are_cut_where_sequences_are_long(batch, q, k, hq, hk, qbs
     size = dict(batch=batch, total_q=batch * q, total_k=batch * k, hq=hq, hk=hk, d=128, nqb=batch * -(-q // qbs), nkb=batch * -(-k // kbs), qbs=qbs, kbs=kbs)
     assert plan_of(False, **size) == plan
     assert plan_of(True, **size)[1:3] == plan[1:3]
+
+
+@pytest.mark.parametrize("nqb,total_q,total_k,nkb,cut", [
+    (16, 1016, 10264, 168, False),    # 8 x 127 queries on 1283 keys: 320 workgroups of four
+    (16, 1016, 20480, 320, True),     # 64 keys to one of them
+    (16, 1016, 20416, 319, False),
+    (8, 243, 9728, 152, True),        # 0.8 rows of all heads to a key
+    (8, 244, 9728, 152, False),
+    (6, 381, 4200, 66, False),        # 120 workgroups
+    (5, 381, 4200, 66, True),
+])
+@pytest.mark.parametrize("prepared", [False, True])
+def test_many_rows_on_short_sequences_are_left_whole(nqb, total_q, total_k, nkb, cut, prepared):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the numbers of items are for 256 compute units")
+    plan = plan_of(prepared, batch=3, total_q=total_q, total_k=total_k, hq=32, hk=4, d=64, nqb=nqb, nkb=nkb, qbs=80, kbs=64)
+    assert (plan[2] > 1) == cut

@@ -21,7 +21,9 @@ pytestmark = pytest.mark.gpu
     ([900], [900], 16, 2, 64, 16, 128, (4, 2, 1, 114)),
     ([2] * 9, [2879] * 9, 128, 8, 128, 48, 80, (8, 1, 1, 216)),         # plain slots would be cut, packed ones are not
     ([21] * 9, [856] * 9, 32, 2, 128, 176, 48, (8, 1, 1, 198)),         # packed eights, not cut
-    ([130] * 3, [2843] * 3, 64, 4, 128, 16, 48, (4, 1, 2, 216)),        # ... cut as fours
+    ([15] * 4, [1097] * 4, 64, 4, 128, 48, 64, (4, 1, 4, 96)),          # ... cut as fours
+    ([130] * 3, [2843] * 3, 64, 4, 128, 16, 48, (4, 2, 1, 216)),        # many rows on short sequences: whole
+    ([127] * 8, [1283] * 8, 32, 4, 64, 80, 64, (4, 1, 1, 320)),
     ([9] * 13, [4407] * 13, 32, 2, 128, 112, 64, (8, 1, 4, 182)),       # ... cut
 ])
 @pytest.mark.parametrize("causal", [True, False])
