@@ -57,8 +57,8 @@ def test_packed_eights_are_cut_where_sequences_are_long(batch, q, k, hq, hk, qbs
 
 @pytest.mark.parametrize("nqb,total_q,total_k,nkb,cut", [
     (16, 1016, 10264, 168, False),    # 8 x 127 queries on 1283 keys: 320 workgroups of four
-    (16, 1016, 20480, 320, True),     # 64 keys to one of them
-    (16, 1016, 20416, 319, False),
+    (16, 1016, 28160, 440, True),     # 88 keys to one of them
+    (16, 1016, 28096, 439, False),
     (8, 243, 9728, 152, True),        # 0.8 rows of all heads to a key
     (8, 244, 9728, 152, False),
     (6, 381, 4200, 66, False),        # 120 workgroups
